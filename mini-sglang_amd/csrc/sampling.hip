@@ -212,35 +212,77 @@ struct Philox {
 
 constexpr int kBins = 2048;  // 11-bit digits; thread t owns bins 2047-2t and 2046-2t (descending)
 constexpr uint32_t kNoDigit = 0xffffffffu;
+constexpr int kStrip = 8;    // loads of a row in flight per thread: a pass is bound by their latency, not by bytes
+
+// What a row's probabilities come from.  raw(i): the stored number; weight(x): a number in the order of the probabilities
+// (the probability itself, or e = 2^((x - max) k)); prob(w): the probability of that weight.
+struct ProbRow {
+  static constexpr bool kSoftmax = false;
+  const float* row;
+  __device__ __forceinline__ float raw(int64_t i) const { return row[i]; }
+  __device__ __forceinline__ float weight(float x) const { return x; }
+  __device__ __forceinline__ float prob(float w) const { return w; }
+};
+// the same numbers softmax_kernel stores, recomputed from the logits: same maximum, same order of the sum, same rounding
+template <int DT>
+struct LogitRow {
+  static constexpr bool kSoftmax = true;
+  const void* row;
+  float mx, k, inv;
+  __device__ __forceinline__ float raw(int64_t i) const { return load_logit<DT>(row, i); }
+  __device__ __forceinline__ float weight(float x) const { return __builtin_amdgcn_exp2f((x - mx) * k); }
+  __device__ __forceinline__ float prob(float w) const { return w * inv; }
+};
+
+// Calls f(index, raw value) for the row elements tid, tid + 1024, ... in order, kStrip loads in flight; `in` is false past the end
+// (the calls are uniform over the workgroup, so f may use ballots).
+template <class Src, class F>
+__device__ __forceinline__ void walk_row(const Src& src, int64_t vocab, F f) {
+  const int tid = threadIdx.x;
+  int64_t base = 0;
+  for (; base + (int64_t)kStrip * kRowThreads <= vocab; base += (int64_t)kStrip * kRowThreads) {
+    float x[kStrip];
+#pragma unroll
+    for (int u = 0; u < kStrip; ++u) x[u] = src.raw(base + u * kRowThreads + tid);
+#pragma unroll
+    for (int u = 0; u < kStrip; ++u) f(base + u * kRowThreads + tid, x[u], true);
+  }
+  for (; base < vocab; base += kRowThreads) {
+    const int64_t i = base + tid;
+    const bool in = i < vocab;
+    f(i, in ? src.raw(i) : 0.f, in);
+  }
+}
 
 // One radix-select level.  Elements taking part: bits >= floor_bits and (bits & mask) == prefix.
 // BY_MASS = false: find the digit where the descending element COUNT reaches `target`;
 // BY_MASS = true : where the descending fixed-point MASS reaches `target`.
-// Returns the digit; `target` is reduced by what lies above it, `mass_above` accumulates the
-// mass of everything strictly above the chosen digit, `digit_mass` = mass inside the digit.
-template <bool BY_MASS>
-__device__ __forceinline__ uint32_t select_level(const float* __restrict__ row, int64_t vocab,
-                                                 uint32_t floor_bits, uint32_t mask, uint32_t prefix,
-                                                 int shift, int nbits, u64& target, u64& mass_above,
-                                                 u64& digit_mass, uint32_t* h_cnt, u64* h_mass, u64* lds_w,
+// Returns the digit; `target` is reduced by what lies above it.
+template <bool BY_MASS, class Src>
+__device__ __forceinline__ uint32_t select_level(const Src& src, int64_t vocab, uint32_t floor_bits, uint32_t mask, uint32_t prefix,
+                                                 int shift, int nbits, u64& target, uint32_t* h_cnt, u64* h_mass, u64* lds_w,
                                                  uint32_t* s_digit) {
   const int tid = threadIdx.x;
   const uint32_t dmask = (1u << nbits) - 1u;
   for (int b = tid; b < kBins; b += kRowThreads) {
-    h_cnt[b] = 0u;
-    h_mass[b] = 0ull;
+    if (BY_MASS) h_mass[b] = 0ull;
+    else h_cnt[b] = 0u;
   }
   if (tid == 0) *s_digit = kNoDigit;  // stays if the row holds less than `target` (fewer than k positive entries)
   __syncthreads();
-  for (int64_t i = tid; i < vocab; i += kRowThreads) {
-    const float p = row[i];
+  walk_row(src, vocab, [&](int64_t, float x, bool in) {
+    const float p = src.prob(src.weight(x));
     const uint32_t bits = __float_as_uint(p);
-    if (bits >= floor_bits && (bits & mask) == prefix && p > 0.f) {
+    if (in && bits >= floor_bits && (bits & mask) == prefix && p > 0.f) {
       const uint32_t d = (bits >> shift) & dmask;
-      atomicAdd(&h_cnt[d], 1u);
-      atomicAdd(&h_mass[d], fixed_mass(p));
+      if (BY_MASS) {
+        const u64 m = fixed_mass(p);
+        if (m) atomicAdd(&h_mass[d], m);
+      } else {
+        atomicAdd(&h_cnt[d], 1u);
+      }
     }
-  }
+  });
   __syncthreads();
   const int b_hi = kBins - 1 - 2 * tid, b_lo = b_hi - 1;  // descending ownership
   const u64 q_hi = BY_MASS ? h_mass[b_hi] : (u64)h_cnt[b_hi];
@@ -256,86 +298,248 @@ __device__ __forceinline__ uint32_t select_level(const float* __restrict__ row, 
     __syncthreads();
     return kNoDigit;
   }
-  // mass strictly above the digit, and quantity strictly above (to reduce the target)
-  u64 m_above = 0, q_above = 0;
-  if ((uint32_t)b_hi > digit) { m_above += h_mass[b_hi]; q_above += q_hi; }
-  if ((uint32_t)b_lo > digit) { m_above += h_mass[b_lo]; q_above += q_lo; }
-  m_above = block_sum_u64(m_above, lds_w);
-  q_above = block_sum_u64(q_above, lds_w);
-  mass_above += m_above;
-  target -= q_above;
-  digit_mass = h_mass[digit];
-  __syncthreads();
+  u64 q_above = 0;  // quantity strictly above the digit, to reduce the target
+  if ((uint32_t)b_hi > digit) q_above += q_hi;
+  if ((uint32_t)b_lo > digit) q_above += q_lo;
+  target -= block_sum_u64(q_above, lds_w);
   return digit;
 }
 
-__global__ __launch_bounds__(kRowThreads) void sample_kernel(int* __restrict__ out,
-                                                             const float* __restrict__ probs,
-                                                             const int* __restrict__ top_k,
-                                                             const float* __restrict__ top_p, int64_t vocab,
-                                                             int64_t stride, u64 seed, u64 offset) {
-  __shared__ uint32_t h_cnt[kBins];
-  __shared__ u64 h_mass[kBins];
+// bits of the value where the descending count / mass reaches `target`, or kNoDigit (no finite number has these bits)
+template <bool BY_MASS, class Src>
+__device__ __forceinline__ uint32_t select_bits(const Src& src, int64_t vocab, uint32_t floor_bits, u64 target, uint32_t* h_cnt, u64* h_mass,
+                                                u64* lds_w, uint32_t* s_digit) {
+  uint32_t prefix = 0u, mask = 0u;
+#pragma unroll 1
+  for (int level = 0; level < 3; ++level) {
+    const int shift = level == 0 ? 21 : level == 1 ? 10 : 0, nbits = level == 2 ? 10 : 11;
+    const uint32_t d = select_level<BY_MASS>(src, vocab, floor_bits, mask, prefix, shift, nbits, target, h_cnt, h_mass, lds_w, s_digit);
+    if (d == kNoDigit) return kNoDigit;
+    prefix |= d << shift;
+    mask |= ((1u << nbits) - 1u) << shift;
+  }
+  return prefix;
+}
+
+// the `target`-th largest (1-based) of the workgroup's 1024 non-negative numbers, one per thread
+__device__ __forceinline__ uint32_t kth_largest(uint32_t bits, int target, uint32_t* hist, uint32_t* s_two) {
+  const int tid = threadIdx.x;
+  uint32_t prefix = 0u, mask = 0u;
+#pragma unroll 1
+  for (int shift = 24; shift >= 0; shift -= 8) {
+    if (tid < 256) hist[tid] = 0u;
+    __syncthreads();
+    if ((bits & mask) == prefix) atomicAdd(&hist[(bits >> shift) & 255u], 1u);
+    __syncthreads();
+    if (tid < 64) {  // lane l owns the bins 255 - 4 l ... 252 - 4 l
+      int c[4], s = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s += c[q] = (int)hist[255 - 4 * tid - q];
+      int above = s;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(above, d, 64);
+        if (tid >= d) above += o;
+      }
+      above -= s;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (above < target && target <= above + c[q]) {
+          s_two[0] = (uint32_t)(255 - 4 * tid - q);
+          s_two[1] = (uint32_t)above;
+        }
+        above += c[q];
+      }
+    }
+    __syncthreads();
+    prefix |= s_two[0] << shift;
+    mask |= 255u << shift;
+    target -= (int)s_two[1];
+  }
+  __syncthreads();
+  return prefix;
+}
+
+constexpr int kList = 2048;          // candidates of a row that the short path holds (= kBins: it reuses the histograms)
+constexpr int kListTopK = 1024;      // largest top-k it is tried for: one column maximum per thread bounds the k-th largest from below
+constexpr int kListTopP = 512;       // candidates asked for when only a mass is given
+constexpr uint32_t kTinyWeight = 0x17800000u;  // 2^-80: below it two weights apart may be one probability (denormal)
+
+// One 1024-thread workgroup per row.
+//
+// Short path (any top-k up to 1024, or a top-p whose nucleus is small): thread t's largest number over the columns t, t + 1024, ...
+// is known after one pass; the k-th largest of these 1024 maxima has at least k numbers at or above it, so the second pass collects
+// only what reaches it -- some k numbers out of a 152 k vocabulary -- and both thresholds and the draw are integer sums over that
+// list.  The general path finds the same thresholds by three radix levels over the whole row; it stays for wide nuclei, top-k above
+// 1024 and rows whose largest numbers share a column.
+//
+// Bound: one CU walks one row (304 KB of bf16 logits) twice, an exponential and ~10 VALU operations per element in the second pass.
+// 64 rows x 151936 bf16 logits, top-k and top-p: softmax_kernel + radix levels over the stored fp32 probabilities (ten passes, u64 LDS
+// atomics for every element of a first level) 551 us; this kernel from the logits 48.7 us.
+template <class Src>
+__device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64_t k, float pp, int64_t vocab, float inv_t, u64 seed, u64 offset) {
+  __shared__ uint32_t h_cnt[kBins];  // histogram | candidates' probability bits
+  __shared__ u64 h_mass[kBins];      // histogram | candidates' masses
+  __shared__ int s_index[kList];
   __shared__ u64 lds_w[kRowThreads / 64];
-  __shared__ uint32_t s_digit;
-  __shared__ int s_pick;
+  __shared__ float lds_f[kRowThreads / 64];
+  __shared__ uint32_t s_digit, s_two[2];
+  __shared__ int s_pick, s_n;
   const int tid = threadIdx.x;
   const int64_t r = blockIdx.x;
-  const float* row = probs + r * stride;
+  const bool has_k = k >= 1 && k < vocab;
+  const bool by_count = has_k && k <= kListTopK, by_mass = !has_k && pp < 1.0f;
 
   uint32_t thr_bits = 0u;  // keep set = { bits >= thr_bits, p > 0 }
   u64 kept_mass = 0;
-  bool have_mass = false;
+  bool done = false;       // uniform: the threshold is known and every number that reaches it is in the list
+  int n = 0;
 
-  const int64_t k = top_k ? (int64_t)top_k[r] : vocab;
-  if (k >= 1 && k < vocab) {
-    u64 target = (u64)k, above = 0, dm = 0;
-    uint32_t prefix = 0u, mask = 0u;
-    const uint32_t d1 = select_level<false>(row, vocab, 0u, mask, prefix, 21, 11, target, above, dm, h_cnt,
-                                            h_mass, lds_w, &s_digit);
-    // fewer than k positive probabilities (a low temperature underflows the tail to 0): top-k keeps all of them,
-    // as flashinfer does -- no threshold, mass computed below if top-p needs it
-    if (d1 != kNoDigit) {
-      prefix |= d1 << 21; mask |= 0x7ffu << 21;
-      const uint32_t d2 = select_level<false>(row, vocab, 0u, mask, prefix, 10, 11, target, above, dm, h_cnt,
-                                              h_mass, lds_w, &s_digit);
-      prefix |= d2 << 10; mask |= 0x7ffu << 10;
-      const uint32_t d3 = select_level<false>(row, vocab, 0u, mask, prefix, 0, 10, target, above, dm, h_cnt,
-                                              h_mass, lds_w, &s_digit);
-      prefix |= d3;
-      thr_bits = prefix;  // the k-th largest value; ties at it stay in the keep set
-      kept_mass = above + dm;
-      have_mass = true;
+  float col = Src::kSoftmax ? -INFINITY : 0.f;
+  if (Src::kSoftmax || by_count || by_mass)
+    walk_row(src, vocab, [&](int64_t, float x, bool in) { col = in ? fmaxf(col, x) : col; });
+  if constexpr (Src::kSoftmax) {
+    src.mx = block_reduce_max(col, lds_f);
+    src.k = inv_t * 1.4426950408889634f;
+  }
+  uint32_t floor_bits = 0u, list_bits = kNoDigit;  // list_bits: what a weight has to reach to be listed
+  if (by_count || by_mass) {
+    const float w = src.weight(col);
+    const int want = (int)(by_count ? k : (int64_t)kListTopP);
+    floor_bits = kth_largest(w > 0.f ? __float_as_uint(w) : 0u, want, h_cnt, s_two);  // NaN counts as nothing here
+    // weights up to some units in the last place apart can be the same probability: the list starts a little below
+    if (floor_bits > (Src::kSoftmax ? kTinyWeight : 0u)) list_bits = floor_bits - (Src::kSoftmax ? 8u : 0u);
+  }
+  if (tid == 0) { s_n = 0; s_pick = -1; }
+  __syncthreads();
+  if (Src::kSoftmax || list_bits != kNoDigit) {
+    float sum = 0.f;
+    walk_row(src, vocab, [&](int64_t i, float x, bool in) {
+      const float w = src.weight(x);
+      if (in) sum += w;
+      const bool hit = in && w > 0.f && __float_as_uint(w) >= list_bits;
+      const u64 votes = __ballot(hit);
+      if (votes) {
+        const int lane = tid & 63;
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&s_n, __popcll(votes));
+        at = __shfl(at, 0, 64) + __popcll(votes & ((1ull << lane) - 1ull));
+        if (hit && at < kList) {
+          s_index[at] = (int)i;
+          h_cnt[at] = __float_as_uint(w);
+        }
+      }
+    });
+    if constexpr (Src::kSoftmax) src.inv = 1.0f / block_reduce_sum(sum, lds_f);
+    __syncthreads();
+    n = s_n;
+  }
+  if (list_bits != kNoDigit && n <= kList) {
+    uint32_t mine[kList / kRowThreads];
+    bool sure[kList / kRowThreads];  // not among the few below the floor, of whose equals some may be missing
+#pragma unroll
+    for (int e = 0; e < kList / kRowThreads; ++e) {
+      const int c = tid + e * kRowThreads;
+      sure[e] = c < n && h_cnt[c] >= floor_bits;
+      const float p = c < n ? src.prob(__uint_as_float(h_cnt[c])) : 0.f;
+      mine[e] = __float_as_uint(p);
+      if (c < n) {
+        h_cnt[c] = mine[e];
+        h_mass[c] = fixed_mass(p);
+      }
+    }
+    u64 target = 0;
+    if (by_mass) {
+      u64 loc = 0;
+      walk_row(src, vocab, [&](int64_t, float x, bool in) {
+        const u64 m = fixed_mass(src.prob(src.weight(x)));
+        loc += in ? m : 0ull;
+      });
+      kept_mass = block_sum_u64(loc, lds_w);
+      target = (u64)((double)pp * (double)kept_mass);
+      if (target < 1) target = 1;
+      if (target > kept_mass) target = kept_mass;
+    }
+    if (tid == 0) s_digit = kNoDigit;
+    __syncthreads();
+    u64 m_above[kList / kRowThreads], m_same[kList / kRowThreads];
+#pragma unroll
+    for (int e = 0; e < kList / kRowThreads; ++e) {
+      m_above[e] = m_same[e] = 0;
+      if (tid + e * kRowThreads >= n) continue;
+      int c_above = 0, c_same = 0;
+      for (int j = 0; j < n; ++j) {
+        const uint32_t b = h_cnt[j];
+        const u64 m = h_mass[j];
+        if (b > mine[e]) { ++c_above; m_above[e] += m; }
+        else if (b == mine[e]) { ++c_same; m_same[e] += m; }
+      }
+      const bool here = by_count ? c_above < k && k <= c_above + c_same : m_above[e] < target && target <= m_above[e] + m_same[e];
+      if (sure[e] && here) {  // equal candidates write equal words
+        s_digit = mine[e];
+        lds_w[0] = m_above[e] + m_same[e];
+      }
+    }
+    __syncthreads();
+    if (s_digit != kNoDigit && (by_count || kept_mass > 0)) {
+      thr_bits = s_digit;
+      kept_mass = lds_w[0];
+      done = true;
+    }
+    __syncthreads();
+    if (done && by_count && pp < 1.0f && kept_mass > 0) {
+      target = (u64)((double)pp * (double)kept_mass);
+      if (target < 1) target = 1;
+      if (target > kept_mass) target = kept_mass;
+#pragma unroll
+      for (int e = 0; e < kList / kRowThreads; ++e)
+        if (mine[e] >= thr_bits && tid + e * kRowThreads < n && m_above[e] < target && target <= m_above[e] + m_same[e]) s_digit = mine[e];
+      __syncthreads();
+      thr_bits = s_digit;
+    }
+    if (done) {  // the draw over the list, in index order
+      u64 loc = 0;
+#pragma unroll
+      for (int e = 0; e < kList / kRowThreads; ++e)
+        if (tid + e * kRowThreads < n && mine[e] >= thr_bits) loc += h_mass[tid + e * kRowThreads];
+      const u64 total = block_sum_u64(loc, lds_w);
+      const uint32_t x = Philox::draw(seed, offset + (u64)r);
+      const u64 u = (total >> 32) * (u64)x + (((total & 0xffffffffull) * (u64)x) >> 32);
+#pragma unroll
+      for (int e = 0; e < kList / kRowThreads; ++e) {
+        const int c = tid + e * kRowThreads;
+        if (c >= n || mine[e] < thr_bits) continue;
+        const int idx = s_index[c];
+        u64 before = 0;
+        for (int j = 0; j < n; ++j)
+          if (h_cnt[j] >= thr_bits && s_index[j] < idx) before += h_mass[j];
+        if (u >= before && u < before + h_mass[c]) s_pick = idx;
+      }
+      __syncthreads();
+      if (tid == 0) out[r] = s_pick < 0 ? 0 : s_pick;
+      return;
     }
   }
-  const float pp = top_p ? top_p[r] : 1.0f;
+
+  if (has_k) {
+    // fewer than k positive probabilities (a low temperature underflows the tail to 0): top-k keeps all of them,
+    // as flashinfer does -- no threshold; ties at the k-th largest value stay in the keep set
+    const uint32_t v = select_bits<false>(src, vocab, 0u, (u64)k, h_cnt, h_mass, lds_w, &s_digit);
+    if (v != kNoDigit) thr_bits = v;
+  }
   if (pp < 1.0f) {
-    if (!have_mass) {
-      u64 loc = 0;
-      for (int64_t i = tid; i < vocab; i += kRowThreads) loc += fixed_mass(row[i]);
-      kept_mass = block_sum_u64(loc, lds_w);
-    }
+    u64 loc = 0;
+    walk_row(src, vocab, [&](int64_t, float x, bool in) {
+      const float p = src.prob(src.weight(x));
+      if (in && __float_as_uint(p) >= thr_bits) loc += fixed_mass(p);
+    });
+    kept_mass = block_sum_u64(loc, lds_w);
     u64 target = (u64)((double)pp * (double)kept_mass);
     if (target < 1) target = 1;
     if (target > kept_mass) target = kept_mass;
     if (kept_mass > 0) {
-      u64 above = 0, dm = 0;
-      uint32_t prefix = 0u, mask = 0u;
-      const uint32_t floor_bits = thr_bits;
-      const uint32_t d1 = select_level<true>(row, vocab, floor_bits, mask, prefix, 21, 11, target, above, dm,
-                                             h_cnt, h_mass, lds_w, &s_digit);
-      if (d1 != kNoDigit) {  // (target <= kept_mass, so a digit exists; the guard keeps a bad row from indexing out of range)
-        prefix |= d1 << 21; mask |= 0x7ffu << 21;
-        const uint32_t d2 = select_level<true>(row, vocab, floor_bits, mask, prefix, 10, 11, target, above, dm,
-                                               h_cnt, h_mass, lds_w, &s_digit);
-        prefix |= d2 << 10; mask |= 0x7ffu << 10;
-        const uint32_t d3 = select_level<true>(row, vocab, floor_bits, mask, prefix, 0, 10, target, above, dm,
-                                               h_cnt, h_mass, lds_w, &s_digit);
-        prefix |= d3;
-        thr_bits = prefix > thr_bits ? prefix : thr_bits;
-        kept_mass = above + dm;
-        have_mass = true;
-      }
+      const uint32_t v = select_bits<true>(src, vocab, thr_bits, target, h_cnt, h_mass, lds_w, &s_digit);
+      if (v != kNoDigit) thr_bits = v > thr_bits ? v : thr_bits;  // (target <= kept_mass, so a value exists)
     }
   }
 
@@ -345,19 +549,28 @@ __global__ __launch_bounds__(kRowThreads) void sample_kernel(int* __restrict__ o
   constexpr int kWaves = kRowThreads / 64;
   const int64_t seg = ((vocab + kWaves - 1) / kWaves + 63) / 64 * 64;
   const int64_t lo = (int64_t)w * seg, hi = min(vocab, lo + seg);
+  auto mass_at = [&](float x) {
+    const float p = src.prob(src.weight(x));
+    return __float_as_uint(p) >= thr_bits ? fixed_mass(p) : 0ull;
+  };
   u64 wave_mass = 0;
-  for (int64_t i = lo + lane; i < hi; i += 64) {
-    const float p = row[i];
-    if (__float_as_uint(p) >= thr_bits) wave_mass += fixed_mass(p);
+  int64_t at = lo + lane;
+  for (; at + (kStrip - 1) * 64 < hi; at += kStrip * 64) {
+    float x[kStrip];
+#pragma unroll
+    for (int u = 0; u < kStrip; ++u) x[u] = src.raw(at + u * 64);
+#pragma unroll
+    for (int u = 0; u < kStrip; ++u) wave_mass += mass_at(x[u]);
   }
+  for (; at < hi; at += 64) wave_mass += mass_at(src.raw(at));
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
     const uint32_t l = __shfl_xor((uint32_t)wave_mass, d, 64);
     const uint32_t h = __shfl_xor((uint32_t)(wave_mass >> 32), d, 64);
     wave_mass += ((u64)h << 32) | l;
   }
+  __syncthreads();
   if (lane == 0) lds_w[w] = wave_mass;
-  if (tid == 0) s_pick = -1;
   __syncthreads();
   u64 total = 0, before = 0;
   for (int i = 0; i < kWaves; ++i) {
@@ -369,36 +582,58 @@ __global__ __launch_bounds__(kRowThreads) void sample_kernel(int* __restrict__ o
   const u64 u = (total >> 32) * (u64)x + (((total & 0xffffffffull) * (u64)x) >> 32);
   if (total > 0 && u >= before && u < before + wave_mass) {  // exactly one wave
     u64 run = before;
-    for (int64_t base = lo; base < hi; base += 64) {
-      const int64_t i = base + lane;
-      u64 m = 0;
-      if (i < hi) {
-        const float p = row[i];
-        if (__float_as_uint(p) >= thr_bits) m = fixed_mass(p);
-      }
-      u64 incl = m;
+    // strips of 8 x 64 indices: their sum first, the indices one by one only in the strip that holds u
+    for (int64_t base = lo; base < hi; base += kStrip * 64) {
+      u64 m[kStrip], strip = 0;
 #pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const u64 o = shfl_up_u64(incl, d);
-        if (lane >= d) incl += o;
+      for (int e = 0; e < kStrip; ++e) {
+        const int64_t i = base + e * 64 + lane;
+        m[e] = i < hi ? mass_at(src.raw(i)) : 0ull;
+        strip += m[e];
       }
-      const u64 chunk = shfl_u64(incl, 63);
-      if (u < run + chunk) {
-        const bool mine = m > 0 && u >= run + incl - m && u < run + incl;
-        if (mine) s_pick = (int)i;
-        break;
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) {
+        const uint32_t l = __shfl_xor((uint32_t)strip, d, 64);
+        const uint32_t h = __shfl_xor((uint32_t)(strip >> 32), d, 64);
+        strip += ((u64)h << 32) | l;
       }
-      run += chunk;
+      if (u >= run + strip) {
+        run += strip;
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < kStrip; ++e) {
+        u64 incl = m[e];
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const u64 o = shfl_up_u64(incl, d);
+          if (lane >= d) incl += o;
+        }
+        if (m[e] > 0 && u >= run + incl - m[e] && u < run + incl) s_pick = (int)(base + e * 64 + lane);
+        run += shfl_u64(incl, 63);
+      }
+      break;
     }
   }
   __syncthreads();
-  if (tid == 0) {
-    int pick = s_pick;
-    if (pick < 0) {  // degenerate row (all-zero mass): fall back to the first index
-      pick = 0;
-    }
-    out[r] = pick;
-  }
+  if (tid == 0) out[r] = s_pick < 0 ? 0 : s_pick;  // degenerate row (all-zero mass): fall back to the first index
+}
+
+__global__ __launch_bounds__(kRowThreads) void sample_kernel(int* __restrict__ out, const float* __restrict__ probs,
+                                                             const int* __restrict__ top_k, const float* __restrict__ top_p, int64_t vocab,
+                                                             int64_t stride, u64 seed, u64 offset) {
+  const int64_t r = blockIdx.x;
+  sample_row(ProbRow{probs + r * stride}, out, top_k ? (int64_t)top_k[r] : vocab, top_p ? top_p[r] : 1.0f, vocab, 0.f, seed, offset);
+}
+
+template <int DT>
+__global__ __launch_bounds__(kRowThreads) void sample_filtered_logits_kernel(int* __restrict__ out, const char* __restrict__ logits,
+                                                                             const float* __restrict__ temperatures,
+                                                                             const int* __restrict__ top_k, const float* __restrict__ top_p,
+                                                                             int64_t vocab, int64_t row_stride_bytes, u64 seed, u64 offset) {
+  const int64_t r = blockIdx.x;
+  sample_row(LogitRow<DT>{logits + r * row_stride_bytes, 0.f, 0.f, 0.f}, out, top_k ? (int64_t)top_k[r] : vocab, top_p ? top_p[r] : 1.0f,
+             vocab, 1.0f / temperatures[r], seed, offset);
 }
 
 
@@ -578,6 +813,31 @@ extern "C" int msgl_sample_top_k_top_p(int32_t* out, const float* probs, const i
   sample_kernel<<<dim3((unsigned)rows), dim3(kRowThreads), 0, static_cast<hipStream_t>(stream)>>>(
       out, probs, top_k, top_p, vocab, probs_stride, (u64)seed, (u64)offset);
   MSGL_CHECK_LAUNCH("sample_top_k_top_p");
+  return MSGL_OK;
+}
+
+// probs path's draw without the probs: same thresholds, same masses, same pick as softmax_temperature + sample_top_k_top_p
+extern "C" int msgl_sample_filtered_logits(int32_t* out, const void* logits, const float* temperatures, const int32_t* top_k,
+                                           const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride, int logits_dtype,
+                                           uint64_t seed, uint64_t offset, void* stream) {
+  MSGL_REQUIRE(rows >= 0, "sample_filtered_logits: negative rows");
+  if (rows == 0) return MSGL_OK;
+  MSGL_REQUIRE(out && logits && temperatures, "sample_filtered_logits: null pointer");
+  MSGL_REQUIRE(vocab >= 1 && vocab < (1ll << 31) && rows < (1ll << 31), "sample_filtered_logits: bad shape");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const dim3 g((unsigned)rows), b(kRowThreads);
+#define MSGL_SAMPLE(DT, ESZ)                                                                                                       \
+  sample_filtered_logits_kernel<DT><<<g, b, 0, s>>>(out, (const char*)logits, temperatures, top_k, top_p, vocab, logits_stride * ESZ, \
+                                                    (u64)seed, (u64)offset)
+  if (logits_dtype == MSGL_F32) MSGL_SAMPLE(MSGL_F32, 4);
+  else if (logits_dtype == MSGL_BF16) MSGL_SAMPLE(MSGL_BF16, 2);
+  else if (logits_dtype == MSGL_FP16) MSGL_SAMPLE(MSGL_FP16, 2);
+  else {
+    set_error("sample_filtered_logits: unsupported dtype code %d", logits_dtype);
+    return MSGL_EINVAL;
+  }
+#undef MSGL_SAMPLE
+  MSGL_CHECK_LAUNCH("sample_filtered_logits");
   return MSGL_OK;
 }
 

@@ -123,8 +123,8 @@ def gelu_and_mul(input: torch.Tensor, out: Optional[torch.Tensor] = None,
 class _DeferredProbs:
     """What `softmax(logits, T)` hands back: the reference's `sample_impl` (P/engine/sample.py:24-45) passes it
     straight to one of the sampling functions and never looks inside.  Temperature-only batches are then drawn
-    by ONE fused kernel from the logits (no [B, V] fp32 probabilities tensor); the top-k / top-p functions
-    materialise the probabilities and run the radix-select kernel.  Anything else that treats the object as a
+    by ONE fused kernel from the logits (no [B, V] fp32 probabilities tensor), and so are the
+    top-k / top-p functions, through the exact values that the probabilities would have.  Anything else that treats the object as a
     tensor gets the materialised tensor through `__torch_function__`-free explicit conversion (`.probs()`)."""
 
     __slots__ = ("logits", "temperature", "_probs")
@@ -174,13 +174,16 @@ class _SamplingNamespace:
         return d if deferred else d.probs()
 
     def _sample(self, probs, top_k, top_p):
-        probs = _as_probs(probs)
         dev = probs.device
         if isinstance(top_k, int):
             top_k = torch.full((probs.shape[0],), top_k, dtype=torch.int32, device=dev)
         if isinstance(top_p, float):
             top_p = torch.full((probs.shape[0],), top_p, dtype=torch.float32, device=dev)
         # every TP rank seeds identically (P/engine/engine.py:37) => identical draws on all ranks
+        if isinstance(probs, _DeferredProbs) and probs._probs is None:  # nobody has asked for the probabilities: straight from the logits
+            return ops.sample_filtered_logits(probs.logits, probs.temperature, top_k, top_p, torch.initial_seed(),
+                                              self._next_offset(probs.shape[0]))
+        probs = _as_probs(probs)
         return ops.sample_top_k_top_p(probs, top_k, top_p, torch.initial_seed(), self._next_offset(probs.shape[0]))
 
     def sampling_from_probs(self, probs, **_kw):

@@ -446,6 +446,28 @@ def sample_top_k_top_p(probs: torch.Tensor, top_k: Optional[torch.Tensor], top_p
     return out
 
 
+def sample_filtered_logits(logits: torch.Tensor, temperatures: torch.Tensor, top_k: Optional[torch.Tensor], top_p: Optional[torch.Tensor],
+                           seed: int, offset: int) -> torch.Tensor:
+    """sample_top_k_top_p(softmax_temperature(logits, temperatures), ...) in one launch, without the probabilities: the same picks."""
+    _need_cuda(logits, temperatures)
+    assert logits.dim() == 2 and logits.stride(1) == 1 and temperatures.dtype == torch.float32
+    rows = logits.shape[0]
+    out = torch.empty(rows, dtype=torch.int32, device=logits.device)
+    if top_k is not None:
+        assert top_k.dtype == torch.int32 and top_k.is_cuda and top_k.numel() == rows
+    if top_p is not None:
+        assert top_p.dtype == torch.float32 and top_p.is_cuda and top_p.numel() == rows
+    check(
+        lib().msgl_sample_filtered_logits(
+            out.data_ptr(), logits.data_ptr(), temperatures.data_ptr(), top_k.data_ptr() if top_k is not None else None,
+            top_p.data_ptr() if top_p is not None else None, rows, logits.shape[1], logits.stride(0), _logits_dt(logits),
+            seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF, _stream(),
+        ),
+        "sample_filtered_logits",
+    )
+    return out
+
+
 def sample_from_logits(logits: torch.Tensor, temperatures: torch.Tensor, seed: int, offset: int) -> torch.Tensor:
     """index ~ softmax(logits / T) per row, fused (no probs tensor); rows must be 16-byte aligned."""
     _need_cuda(logits, temperatures)

@@ -214,3 +214,63 @@ def test_top_k_larger_than_the_number_of_positive_probabilities(ops, dev):
     outs = [ops.sample_top_k_top_p(pd, k, p, seed=3, offset=i * 6).cpu().tolist()[3] for i in range(30)]
     assert set(outs) == {hot[3]}
     assert len(seen[5]) >= 2
+
+
+def _philox(seed, ctr):
+    """First word of Philox4x32-10 of counter (ctr, 0) under key `seed`."""
+    c, k = [ctr & 0xFFFFFFFF, ctr >> 32, 0, 0], [seed & 0xFFFFFFFF, seed >> 32]
+    for _ in range(10):
+        a, b = 0xD2511F53 * c[0], 0xCD9E8D57 * c[2]
+        c = [(b >> 32) ^ c[1] ^ k[0], b & 0xFFFFFFFF, (a >> 32) ^ c[3] ^ k[1], a & 0xFFFFFFFF]
+        k = [(k[0] + 0x9E3779B9) & 0xFFFFFFFF, (k[1] + 0xBB67AE85) & 0xFFFFFFFF]
+    return c[0]
+
+
+def _filtered_pick(p, k, pp, seed, ctr):
+    """The pick over one row of fp32 probabilities in whole numbers of 2^-40: k-th largest value, then the value where the descending
+    mass reaches pp of what is kept (ties stay), then the inverse CDF in index order."""
+    import numpy as np
+
+    mass = np.floor(np.where(p > 0, p, 0).astype(np.float64) * 2.0 ** 40).astype(np.int64)
+    keep = p > 0
+    if 1 <= k < p.size and keep.sum() >= k:
+        keep &= p >= np.sort(p[keep])[-k]
+    total = int(mass[keep].sum())
+    if pp < 1.0 and total > 0:
+        target = min(max(int(float(np.float32(pp)) * float(total)), 1), total)
+        order = np.argsort(-p[keep], kind="stable")
+        v = p[keep][order][int(np.searchsorted(np.cumsum(mass[keep][order]), target))]
+        keep &= p >= v
+        total = int(mass[keep].sum())
+    u = (total * _philox(seed, ctr)) >> 32
+    idx = np.nonzero(keep)[0]
+    run = np.cumsum(mass[idx])
+    return int(idx[np.searchsorted(run, u, side="right")]) if total else 0
+
+
+# vocabularies around the 1024 columns and the strips of 8 loads; rows whose largest numbers share one column (the candidate list
+# overflows or asks for more than its column maxima give), plain rows, ties, few positive probabilities
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("vocab", [1, 7, 1023, 1025, 8192 + 5, 33333, 151936])
+def test_filtered_draw_is_the_integer_rule(ops, dev, dtype, vocab):
+    g = torch.Generator().manual_seed(vocab)
+    rows = [(k, p, t, kind) for kind in ("plain", "column", "ties", "cold")
+            for k, p, t in ((1, 1.0, 1.0), (50, 0.9, 0.7), (0, 0.8, 0.5), (0, 0.99, 1.0), (1024, 0.95, 1.0), (1500, 0.9, 1.0), (20, 1.0, 0.4), (0, 1.0, 1.0))]
+    logits = torch.randn((len(rows), vocab), generator=g) * 2.5
+    for r, (_, _, _, kind) in enumerate(rows):
+        if kind == "column":
+            logits[r, 3::1024] += 9.0
+        elif kind == "ties":
+            logits[r] = torch.round(logits[r] * 2) / 2
+        elif kind == "cold":
+            logits[r, 5:] -= 300.0
+    logits = logits.to(dtype).to(dev)
+    k = torch.tensor([x[0] for x in rows], dtype=torch.int32, device=dev)
+    p = torch.tensor([x[1] for x in rows], dtype=torch.float32, device=dev)
+    t = torch.tensor([x[2] for x in rows], dtype=torch.float32, device=dev)
+    probs = ops.softmax_temperature(logits, t)
+    host = probs.cpu().numpy()
+    for off in (0, 1000):
+        want = [_filtered_pick(host[r], rows[r][0], rows[r][1], 77, off + r) for r in range(len(rows))]
+        assert ops.sample_top_k_top_p(probs, k, p, 77, off).cpu().tolist() == want
+        assert ops.sample_filtered_logits(logits, t, k, p, 77, off).cpu().tolist() == want
