@@ -180,6 +180,69 @@ __device__ __forceinline__ void find_group(const int* __restrict__ cu_q, int B, 
   __syncthreads();
 }
 
+// The same question answered by one wave without LDS, groups of the batch in the order of their last key position, farthest first (what
+// comes last in a launch should be short).  Up to 64 requests: the position x with #groups ending at or past x > index >= #groups ending past
+// x by bisection, then the rank among the groups that end at x.  More requests: last group first, in the order of the batch.
+// -> request (-1: past the last group), first token of the group.
+__device__ __forceinline__ int find_group_by_keys(const int* __restrict__ cu_q, const int* __restrict__ seq_lens, int B, int QT, int index,
+                                                  int total_groups, int* tok0) {
+  const int lane = threadIdx.x & 63;
+  if (B <= 64) {
+    int n = 0, start = 0;
+    if (lane < B) {
+      const int q = cu_q[lane + 1] - cu_q[lane];
+      n = (q + QT - 1) / QT;
+      start = seq_lens[lane] - q;
+    }
+    // groups of this lane's request that end at position x or later (the end of group p is start + QT (p + 1), the last one's rounded up)
+    auto past = [&](int x) { return max(0, n - max(0, (x - start + QT - 1) / QT - 1)); };
+    auto total = [&](int v) {
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+      return __builtin_amdgcn_readfirstlane(v);
+    };
+    int hi = start + n * QT;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) hi = max(hi, __shfl_xor(hi, o, 64));
+    hi = __builtin_amdgcn_readfirstlane(hi) + 1;  // nothing ends here
+    int lo = 0, above = 0;                        // everything ends past 0
+    if (total(n) <= index) return -1;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1, c = total(past(mid));
+      if (c > index) {
+        lo = mid;
+      } else {
+        hi = mid;
+        above = c;
+      }
+    }
+    const int here = past(lo) - past(lo + 1), rank = index - above;
+    const uint64_t votes = __builtin_amdgcn_ballot_w64(here > 0);
+    const bool mine = here > 0 && __popcll(votes & ((1ull << lane) - 1ull)) == rank;
+    const int b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(mine));
+    *tok0 = ((lo - __builtin_amdgcn_readlane(start, b)) / QT - 1) * QT;
+    return b;
+  }
+  index = total_groups - 1 - index;
+  for (int c0 = 0; c0 < B; c0 += 64) {
+    const int n = c0 + lane < B ? (cu_q[c0 + lane + 1] - cu_q[c0 + lane] + QT - 1) / QT : 0;
+    int incl = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += v;
+    }
+    const uint64_t votes = __builtin_amdgcn_ballot_w64(incl > index);
+    if (votes) {
+      const int l = __builtin_ctzll(votes);
+      *tok0 = (index - __builtin_amdgcn_readlane(incl - n, l)) * QT;
+      return c0 + l;
+    }
+    index -= __builtin_amdgcn_readlane(incl, 63);
+  }
+  return -1;
+}
+
 bool dtype_ok(int dt) { return dt == MSGL_MIX_BF16 || dt == MSGL_MIX_F32; }
 
 int ensure_lds(const void* fn, size_t bytes) {

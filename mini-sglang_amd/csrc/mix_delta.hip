@@ -13,7 +13,7 @@
 //   poly_act_kernel          a N(z) + b N(z^2) + c N(z^3) + e,  N = divide a row by its root mean square
 //   route_top_kernel         stand-alone router on given fp32 logits (long batches)
 //   kv_store_kernel          k and the (blended) v of a token -> cache rows at out_loc
-//   window_attn_kernel       sliding-window attention over the paged rows: raw scores of all heads, mixed by the H x H table,
+//   window_attn_kernel       (what mix_window.hip does not take:) sliding-window attention over the paged rows: raw scores of all heads, mixed by the H x H table,
 //                            fp32 online softmax, per-head sigmoid output gate; one workgroup per query token
 //   short_conv_kernel        causal per-channel convolution over time + SiLU, inputs before the portion from the request's
 //                            conv state; q / k heads made unit vectors (q also * d^-1/2);  conv_state_kernel shifts the state
@@ -793,6 +793,12 @@ __global__ __launch_bounds__(256) void head_gated_norm_kernel(T* __restrict__ ou
 
 }  // namespace
 
+// mix_window.hip: the matrix-core form of window_attn (1 launched, 0 not its sizes, < 0 error)
+extern "C" int mix_window_attn_mfma(void* out, float* part_o, float* part_ml, const void* src, int64_t ld_src, int g_off, const void* k_cache,
+                                    const void* v_cache, const int* table, int64_t table_stride, const int* req_rows, const int* seq_lens,
+                                    const int* cu_q, int batch, int total_q, int H, int G, int d, int dv, int window, float scale,
+                                    const float* talk, int splits, hipStream_t s);
+
 extern "C" {
 
 int msgl_mix_embed_norm(float* x32, const void* table, const int* ids, const void* w, float eps, int tokens, int W, int dtype,
@@ -889,6 +895,15 @@ int msgl_mix_window_attn(void* out, const void* src, int64_t ld_src, int g_off, 
   const size_t es = dtype == MSGL_MIX_BF16 ? 2 : 4;
   float* part_o = workspace;
   float* part_ml = workspace ? workspace + (size_t)splits * total_q * H * dv : nullptr;
+  // bf16 caches of 8 or 16 heads up to 128 wide: the matrix cores, down to one new token per request, where 15 of a group's 16 rows are
+  // empty (16 heads, 2000 cached keys, this kernel -> that one: 4 requests x 1 token 102 -> 47 us, x 4 240 -> 52, x 32 581 -> 77;
+  // 32 x 1 153 -> 80; 4 requests of 1500 - 2548 new tokens 5198 -> 277).  Other sizes and fp32 stay here.
+  int done = 0;
+  if (dtype == MSGL_MIX_BF16) {
+    done = mix_window_attn_mfma(out, part_o, part_ml, src, ld_src, g_off, k_cache, v_cache, table, table_stride, req_rows, seq_lens, cu_q, batch,
+                                total_q, H, G, d, dv, window, scale, talk, splits, s);
+    if (done < 0) return done;
+  }
   // query tokens per workgroup: 8 where portions are long and the tile fits half the LDS (two workgroups per CU), else 4, else 1
 #define WA_LAUNCH(QT)                                                                                                                  \
   {                                                                                                                                    \
@@ -900,7 +915,8 @@ int msgl_mix_window_attn(void* out, const void* src, int64_t ld_src, int g_off, 
                                   cu_q, batch, total_q, H, G, d, dv, window, scale, talk, splits);)                                     \
   }
   const auto lds_of = [&](int qt) { return (size_t)(H * H + 2 * H * qt * 64 + 3 * H * qt + 64 + 3) * 4 + (size_t)qt * H * d * es; };
-  if (total_q >= 8 * batch && lds_of(8) <= 80 * 1024) {
+  if (done) {
+  } else if (total_q >= 8 * batch && lds_of(8) <= 80 * 1024) {
     WA_LAUNCH(8)
   } else if (total_q >= 4 * batch && lds_of(4) <= 80 * 1024) {
     WA_LAUNCH(4)

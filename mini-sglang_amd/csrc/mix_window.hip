@@ -1,0 +1,313 @@
+// Sliding-window attention with mixed heads on the matrix cores (bf16 caches): the form of window_attn_kernel (mix_delta.hip) for
+// portions of query tokens.  Same C entry, msgl_mix_window_attn; this file holds one kernel and the function that launches it.
+//
+// What bounds it: per visible (query, key) pair and H heads the two products are 2 H (d + 2 dv) flops for the bf16 matrix cores, the
+// mixing of the scores 2 H^2 flops in fp32 and the softmax about fifteen vector operations per head; at H = 16, d = dv = 128 each of the
+// three takes about the same time, so they have to run beside each other.  The mixing is itself a product, table x scores with the heads
+// as contraction: it goes to the fp32 matrix instructions (on vector FMAs it was 256 of them a pair, and every wave read every head's
+// scores back from LDS).
+//
+// 4 requests of 1500 - 2548 new tokens, 16 heads of 128 over 4 key heads, window 2048: 5198 us on the vector units, 453 us with both
+// products on the matrix cores and the mixing on vector FMAs in step with them, 277 us as below (264 TFLOP/s of useful products; the
+// softmax and the LDS round trip of the scores are what is left).
+//
+// Precision: scores are bf16 x bf16 products with fp32 sums, mixed and exponentiated in fp32; a probability enters the second product
+// as the sum of two bf16 numbers (its rounding and what the rounding left, 16 bits in all), so nothing held in 32 bits drops to 16.
+#include "mix_common.h"
+
+namespace {
+
+constexpr int kWinTile = 32;           // keys per tile
+constexpr int kWinKC = 4, kWinVC = 8;  // head sizes up to 128
+constexpr int kWinRow = 36;            // floats of a mixed (head, query) row in LDS: 32 keys, padded so that 16 rows cover all banks
+template <int NH>
+constexpr int kWinRaw = kWinTile * NH + 4;  // floats of a query's raw scores in LDS: [32 keys][NH], padded the same way
+
+// Workgroup = 16 query tokens of one request x all NH heads (x one of `splits` key ranges), NH / 2 waves of two heads each, which share
+// a key / value head.  Two phases per tile of 32 keys, a barrier behind each:
+//   C(t)  the waves share the tile's keys: mixed scores = talk x raw, a product over the heads per key; the next tile's K rows and this
+//         tile's V rows, requested a phase before, go to LDS
+//   D(t)  the waves share the heads: S^T = K Q^T of tile t + 1 (Q held in registers) -> raw scores to LDS, which the vector work of
+//         tile t covers: mask, online softmax, O^T += V^T P^T (a lane reads four consecutive keys of its query, the layout the product
+//         takes; V through transposing LDS reads)
+template <int NH>
+__global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
+                                                                  const bf16_t* __restrict__ src, int64_t ld_src, int g_off,
+                                                                  const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
+                                                                  const int* __restrict__ table, int64_t table_stride,
+                                                                  const int* __restrict__ req_rows, const int* __restrict__ seq_lens,
+                                                                  const int* __restrict__ cu_q, int B, int total_q, int G, int d, int dv,
+                                                                  int window, float scale, const float* __restrict__ talk, int splits, int qvec) {
+  constexpr int HPW = 2, NT = NH * 32, NW = NH / 2, KC = kWinKC, VC = kWinVC, KS = kWinTile / 16, GS = NH / 4, RAW = kWinRaw<NH>;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const int VS = G * VC * 16 + 8, KSR = G * KC * 32 + 8;
+  float* raw = smem;                                                      // [16 queries][32 keys][NH]
+  float* mixed = raw + 16 * RAW;                                          // [NH][16 queries][kWinRow]
+  uint16_t* sv = reinterpret_cast<uint16_t*>(mixed + NH * 16 * kWinRow);  // [32][VS]
+  uint16_t* sk = sv + kWinTile * VS;                                      // [32][KSR]
+  __shared__ int s_slot[4][kWinTile];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  int tok0 = 0;
+  const int b = find_group_by_keys(cu_q, seq_lens, B, 16, (int)blockIdx.x, (int)gridDim.x, &tok0);
+  if (b < 0) return;
+  const int q_len = cu_q[b + 1] - cu_q[b], start = seq_lens[b] - q_len;
+  const int last_tok = min(tok0 + 16, q_len) - 1;
+  const bool valid = tok0 + lr < q_len;
+  const size_t tok = (size_t)cu_q[b] + (valid ? tok0 + lr : tok0);
+  const int limit = valid ? start + tok0 + lr : -1;
+  const int lo_row = window > 0 ? max(0, limit - window + 1) : 0;
+  const int n_keys = start + last_tok + 1, lo_blk = window > 0 ? max(0, start + tok0 - window + 1) : 0;
+  const int per = ((n_keys - lo_blk + splits - 1) / splits + kWinTile - 1) / kWinTile * kWinTile;
+  const int k_begin = lo_blk + (int)blockIdx.y * per, k_end = min(n_keys, k_begin + per);
+  const int all_hi = start + tok0, all_lo = window > 0 ? max(0, start + last_tok - window + 1) : 0;  // keys that every row sees
+  const int h0 = wave * HPW, rep = NH / G, grp = h0 / rep;
+  const float scale2 = scale * 1.4426950408889634f;
+  // the table as first operand: row = head, contraction index 4 steps (NH = 16) of g = GS lg + step, which is what a lane reads at once
+  float tk[GS];
+#pragma unroll
+  for (int u = 0; u < GS; ++u) tk[u] = lr < NH ? talk[lr * NH + GS * lg + u] * scale2 : 0.f;
+  bf16x8_t qf[HPW][KC];
+  f32x4_t o[HPW][VC];
+  float m[HPW], lsum[HPW];
+#pragma unroll
+  for (int hh = 0; hh < HPW; ++hh) {
+    const bf16_t* qrow = src + tok * (size_t)ld_src + (size_t)(h0 + hh) * d;
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) {
+      const int k = kc * 32 + lg * 8;
+      Q4 f{0u, 0u, 0u, 0u};
+      if (valid && k < d) f = load8(qrow + k, d - k, qvec != 0);
+      qf[hh][kc] = __builtin_bit_cast(bf16x8_t, f);
+    }
+#pragma unroll
+    for (int vt = 0; vt < VC; ++vt) o[hh][vt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    m[hh] = -INFINITY;
+    lsum[hh] = 0.f;
+  }
+  const int* trow = table + (size_t)req_rows[b] * table_stride;
+  const size_t nk = (size_t)G * d, nv = (size_t)G * dv;
+  // 16-byte pieces of a tile's key and value rows (both 128 wide per head in LDS, zeros past the head); at most NH / 4 key heads
+  static_assert(KC * 4 == VC * 2, "keys and values share the piece map");
+  const int chunks = G * VC * 2;
+  constexpr int NP = kWinTile * (NH / 4) * VC * 2 / NT;  // pieces per thread
+  Q4 pre_k[NP], pre_v[NP];
+  // the rows of tile j0 (its slots in s_slot[buf]) into registers, and from there to LDS
+  auto request = [&](Q4 (&pre)[NP], const bf16_t* cache, size_t ld_row, int dh, int j0, int buf) {
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int e = u * NT + (int)threadIdx.x;
+      const int key = e / chunks, ch = e - key * chunks, hv = ch / (VC * 2), c = (ch - hv * (VC * 2)) * 8;
+      pre[u] = Q4{0u, 0u, 0u, 0u};
+      if (key < kWinTile && j0 + key < k_end && c < dh)
+        pre[u] = *reinterpret_cast<const Q4*>(cache + (size_t)s_slot[buf][key] * ld_row + (size_t)hv * dh + c);
+    }
+  };
+  auto stage = [&](const Q4 (&pre)[NP], uint16_t* dst, int ld_row) {
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int e = u * NT + (int)threadIdx.x;
+      const int key = e / chunks, ch = e - key * chunks;
+      if (key < kWinTile) *reinterpret_cast<Q4*>(&dst[key * ld_row + ch * 8]) = pre[u];
+    }
+  };
+  auto slots_of = [&](int j0, int buf) {
+    if (threadIdx.x < kWinTile && j0 + (int)threadIdx.x < k_end) s_slot[buf][threadIdx.x] = trow[j0 + threadIdx.x];
+  };
+  f32x4_t sc[HPW][KS];
+  auto scores = [&]() {  // raw scores of the tile in sk
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+      for (int hh = 0; hh < HPW; ++hh) sc[hh][ks] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) {
+        const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(&sk[(ks * 16 + lr) * KSR + grp * KC * 32 + kc * 32 + lg * 8]);
+#pragma unroll
+        for (int hh = 0; hh < HPW; ++hh) sc[hh][ks] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[hh][kc], sc[hh][ks], 0, 0, 0);
+      }
+    }
+  };
+  auto store_raw = [&]() {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        *reinterpret_cast<float2*>(raw + lr * RAW + (ks * 16 + 4 * lg + c) * NH + h0) = float2{sc[0][ks][c], sc[1][ks][c]};
+  };
+  constexpr int TW = kWinTile;
+  slots_of(k_begin, 0);
+  slots_of(k_begin + TW, 1);
+  slots_of(k_begin + 2 * TW, 2);
+  __syncthreads();
+  request(pre_k, k_cache, nk, d, k_begin, 0);
+  stage(pre_k, sk, KSR);
+  request(pre_v, v_cache, nv, dv, k_begin, 0);
+  request(pre_k, k_cache, nk, d, k_begin + TW, 1);
+  __syncthreads();
+  scores();
+  store_raw();
+  __syncthreads();
+  int buf = 0;
+  for (int j0 = k_begin; j0 < k_end; j0 += TW, buf = (buf + 1) & 3) {
+    const int nj = j0 + TW;
+    // ---- C(t)
+    {
+      constexpr int KPW = kWinTile / NW;  // keys of this wave
+#pragma unroll
+      for (int k0 = 0; k0 < KPW; k0 += 4) {
+        f32x4_t mx[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float* x = raw + lr * RAW + (wave * KPW + k0 + i) * NH + GS * lg;
+          mx[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int u = 0; u < GS; ++u) mx[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(tk[u], x[u], mx[i], 0, 0, 0);
+        }
+        if (4 * lg < NH) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            *reinterpret_cast<f32x4_t*>(mixed + ((4 * lg + c) * 16 + lr) * kWinRow + wave * KPW + k0) = f32x4_t{mx[0][c], mx[1][c], mx[2][c], mx[3][c]};
+        }
+      }
+    }
+    stage(pre_v, sv, VS);
+    stage(pre_k, sk, KSR);
+    slots_of(j0 + 3 * TW, (buf + 3) & 3);
+    __syncthreads();
+    // ---- D(t)
+    request(pre_v, v_cache, nv, dv, nj, (buf + 1) & 3);
+    request(pre_k, k_cache, nk, d, nj + TW, (buf + 2) & 3);
+    scores();  // of tile t + 1 (zeros past the last)
+    f32x4_t s[HPW][KS];
+#pragma unroll
+    for (int hh = 0; hh < HPW; ++hh)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) s[hh][ks] = *reinterpret_cast<const f32x4_t*>(mixed + ((h0 + hh) * 16 + lr) * kWinRow + ks * 16 + 4 * lg);
+    const bool whole = nj <= k_end && nj - 1 <= all_hi && j0 >= all_lo;
+    uint2 hi[HPW][KS], lo[HPW][KS];
+#pragma unroll
+    for (int hh = 0; hh < HPW; ++hh) {
+      float tmax = -INFINITY;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        if (!whole) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const int j = j0 + ks * 16 + 4 * lg + c;
+            if (!(j <= limit && j >= lo_row && j < k_end)) s[hh][ks][c] = -INFINITY;
+          }
+        }
+        tmax = fmaxf(tmax, fmaxf(fmaxf(s[hh][ks][0], s[hh][ks][1]), fmaxf(s[hh][ks][2], s[hh][ks][3])));
+      }
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+      const float m_new = fmaxf(m[hh], tmax);
+      const float base = m_new == -INFINITY ? 0.f : m_new;  // no visible key yet: every weight below is exp2(-inf) = 0
+      const float alpha = __builtin_amdgcn_exp2f(m[hh] - base);
+      float psum = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        float p[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          p[c] = __builtin_amdgcn_exp2f(s[hh][ks][c] - base);
+          psum += p[c];
+        }
+        hi[hh][ks] = uint2{pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3])};
+        lo[hh][ks] = uint2{pack_bf16(p[0] - __uint_as_float(hi[hh][ks].x << 16), p[1] - __uint_as_float(hi[hh][ks].x & 0xffff0000u)),
+                           pack_bf16(p[2] - __uint_as_float(hi[hh][ks].y << 16), p[3] - __uint_as_float(hi[hh][ks].y & 0xffff0000u))};
+      }
+      lsum[hh] = fmaf(lsum[hh], alpha, psum);
+      if (__builtin_amdgcn_ballot_w64(m_new > m[hh]) != 0) {
+#pragma unroll
+        for (int vt = 0; vt < VC; ++vt)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) o[hh][vt][c] *= alpha;
+      }
+      m[hh] = m_new;
+    }
+    store_raw();
+    const uint16_t* vbase = &sv[(4 * lg + (lr >> 2)) * VS + grp * VC * 16 + 4 * (lr & 3)];
+#pragma unroll
+    for (int kp = 0; kp < KS / 2; ++kp) {
+      if (j0 + kp * 32 >= k_end) break;
+#pragma unroll
+      for (int vt = 0; vt < VC; ++vt) {
+        const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vbase + kp * 32 * VS + vt * 16));
+        const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vbase + (kp * 32 + 16) * VS + vt * 16));
+        const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+        for (int hh = 0; hh < HPW; ++hh) {
+          const Q4 ph{hi[hh][2 * kp].x, hi[hh][2 * kp].y, hi[hh][2 * kp + 1].x, hi[hh][2 * kp + 1].y};
+          const Q4 pl{lo[hh][2 * kp].x, lo[hh][2 * kp].y, lo[hh][2 * kp + 1].x, lo[hh][2 * kp + 1].y};
+          o[hh][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, pl), o[hh][vt], 0, 0, 0);
+          o[hh][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, ph), o[hh][vt], 0, 0, 0);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (!valid) return;
+#pragma unroll
+  for (int hh = 0; hh < HPW; ++hh) {
+    float l = lsum[hh];
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    const int h = h0 + hh;
+    if (splits == 1) {
+      const float gz = ld(src + tok * (size_t)ld_src + g_off + h);
+      const float f = 1.0f / (l * (1.0f + __expf(-gz)));
+#pragma unroll
+      for (int vt = 0; vt < VC; ++vt) {
+        const int e = vt * 16 + 4 * lg;
+        if (e < dv)
+          *reinterpret_cast<uint2*>(out + tok * (size_t)(NH * dv) + (size_t)h * dv + e) =
+              uint2{pack_bf16(o[hh][vt][0] * f, o[hh][vt][1] * f), pack_bf16(o[hh][vt][2] * f, o[hh][vt][3] * f)};
+      }
+    } else {
+      const size_t row = ((size_t)blockIdx.y * total_q + tok) * NH + h;
+#pragma unroll
+      for (int vt = 0; vt < VC; ++vt) {
+        const int e = vt * 16 + 4 * lg;
+        if (e < dv) *reinterpret_cast<f32x4_t*>(part_o + row * dv + e) = o[hh][vt];
+      }
+      if (lg == 0) {
+        part_ml[row * 2] = m[hh] * 0.6931471805599453f;  // the maxima leave in natural units
+        part_ml[row * 2 + 1] = l;
+      }
+    }
+  }
+}
+
+template <int NH>
+size_t window_lds(int G) {
+  return (size_t)(NH * 16 * kWinRow + 16 * kWinRaw<NH>) * sizeof(float) + (size_t)kWinTile * (G * (kWinVC * 16 + kWinKC * 32) + 16) * sizeof(uint16_t);
+}
+
+}  // namespace
+
+// 1: launched; 0: these sizes are not this kernel's (the caller takes the other one); < 0: an error code.
+extern "C" __attribute__((visibility("hidden"))) int mix_window_attn_mfma(
+    void* out, float* part_o, float* part_ml, const void* src, int64_t ld_src, int g_off, const void* k_cache, const void* v_cache, const int* table,
+    int64_t table_stride, const int* req_rows, const int* seq_lens, const int* cu_q, int batch, int total_q, int H, int G, int d, int dv, int window,
+    float scale, const float* talk, int splits, hipStream_t s) {
+  const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  // heads of 8 | 16 so that a wave's heads share a value head; rows that 16-byte loads and 8-byte stores may walk
+  if (!(H == 8 || H == 16) || G > H / 4 || (H / 2) % G || d > 128 || dv > 128 || d % 8 || dv % 8) return 0;
+  if (!al(k_cache) || !al(v_cache) || !al(out) || (part_o && !al(part_o))) return 0;
+  const int qvec = al(src) && ld_src % 8 == 0;
+  const dim3 grid(total_q / 16 + batch, splits);
+#define WIN_LAUNCH(NH)                                                                                                                        \
+  {                                                                                                                                           \
+    const size_t lds = window_lds<NH>(G);                                                                                                     \
+    MIX_REQUIRE(ensure_lds((const void*)window_attn_mfma_kernel<NH>, lds) == 0, "window_attn: %zu bytes of LDS", lds);                        \
+    hipLaunchKernelGGL((window_attn_mfma_kernel<NH>), grid, dim3(NH * 32), lds, s, mp<bf16_t>(out), part_o, part_ml, cp<bf16_t>(src), ld_src,     \
+                       g_off, cp<bf16_t>(k_cache), cp<bf16_t>(v_cache), table, table_stride, req_rows, seq_lens, cu_q, batch, total_q, G, d,  \
+                       dv, window, scale, talk, splits, qvec);                                                                                \
+  }
+  if (H == 16) WIN_LAUNCH(16) else WIN_LAUNCH(8)
+#undef WIN_LAUNCH
+  MIX_LAUNCHED("window_attn");
+  return 1;
+}

@@ -378,6 +378,12 @@ def window_attn(out: torch.Tensor, src: torch.Tensor, g_off: int, k_cache: torch
     assert k_cache.dtype == src.dtype == v_cache.dtype and talk.dtype == torch.float32 and talk.is_contiguous() and talk.shape == (H, H)
     assert table.dtype == torch.int32 and table.stride(1) == 1
     assert req_rows.numel() >= batch and seq_lens.numel() >= batch and cu_q.numel() >= batch + 1
+    if splits == 1:
+        # a few short portions are some tens of 16-token groups for 256 compute units: cut their keys as well (32 portions of 8 - 32
+        # tokens over 2000 keys, 16 heads: 226 -> 72 us); from static sizes only, so a captured graph keeps its grid
+        groups, keys = T // 16 + batch, min(window, table.shape[1]) if window > 0 else table.shape[1]
+        if groups <= 128:
+            splits = max(1, min(256 // groups, keys // 256, 8))
     ws = None
     if splits > 1:
         ws = torch.empty(mix_lib().msgl_mix_window_attn_workspace_floats(T, H, dv, splits), dtype=torch.float32, device=out.device)

@@ -215,6 +215,47 @@ def test_window_edges_one_key_stands_out(dev, dtype, window, splits):
                 assert float((got[outside] - want).abs().max()) > 0.05 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("splits", [1, 3], ids=["one-range", "three-ranges"])
+@pytest.mark.parametrize("H,G,d,dv", [(16, 4, 128, 128), (16, 1, 128, 72), (16, 2, 64, 128), (8, 2, 128, 128), (8, 1, 40, 16)])
+def test_window_matrix_cores(dev, H, G, d, dv, splits):
+    """The matrix-core form at the edges of its 16-token groups and 32-key tiles: portions of 1 - 100 new tokens after 0 - 100 cached
+    ones in one launch, windows around the tile, against float64.  Bound: the bf16 result (2^-9 of the value) and weights of 16 bits
+    whose errors do not cancel (2^-16 of the largest value, twice, with room for fp32 sums)."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(H * 1000 + d + dv)
+    new, old = [33, 1, 100, 16, 17, 5], [0, 64, 100, 31, 0, 3]
+    for window in (0, 1, 31, 32, 33, 70):
+        B, T = len(new), sum(new)
+        slots = torch.randperm(1024, generator=g)
+        table, at = torch.zeros((B, 256), dtype=torch.int32), 0
+        kc, vc = torch.zeros((1024, G * d)), torch.zeros((1024, G * dv))
+        src = torch.randn(T, H * d + H, generator=g).bfloat16()
+        talk = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)
+        refs, row = [], 0
+        for b, (n, c) in enumerate(zip(new, old)):
+            k, v = torch.randn(n + c, G, d, generator=g).bfloat16(), torch.randn(n + c, G, dv, generator=g).bfloat16()
+            mine = slots[at: at + n + c]
+            at += n + c
+            table[b, : n + c] = mine.int()
+            kc[mine], vc[mine] = k.reshape(n + c, -1).float(), v.reshape(n + c, -1).float()
+            part = src[row: row + n].double()
+            q = torch.cat([torch.zeros(c, H, d, dtype=torch.float64), part[:, : H * d].view(n, H, d)])
+            gate = torch.cat([torch.zeros(c, H, dtype=torch.float64), part[:, H * d:]])
+            refs.append(_window_reference(q, k.double(), v.double(), gate, talk.double(), d ** -0.5, window, H // G)[c:].reshape(n, -1))
+            row += n
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+        out = torch.empty((T, H * dv), dtype=torch.bfloat16, device=dev)
+        cu = [0]
+        for n in new:
+            cu.append(cu[-1] + n)
+        mixops.window_attn(out, src.to(dev), H * d, kc.bfloat16().to(dev), vc.bfloat16().to(dev), table.to(dev), i32(range(B)),
+                           i32([n + c for n, c in zip(new, old)]), i32(cu), B, H, G, d, dv, window, d ** -0.5, talk.to(dev), splits=splits)
+        ref = torch.cat(refs)
+        diff = (out.double().cpu() - ref).abs()
+        assert bool((diff <= 2.0 ** -8 * ref.abs() + 2.0 ** -14 * ref.abs().max()).all()), (window, float(diff.max()))
+
+
 @pytest.mark.parametrize("chunk", [0, 1, 5], ids=["whole", "chunks-of-1", "chunks-of-5"])
 def test_delta_rule_state_slots_and_cuts(dev, chunk):
     """The recurrence kernel alone: two requests in one launch on state rows that hold garbage, then continued in a second
