@@ -180,7 +180,29 @@ __device__ __forceinline__ void find_group(const int* __restrict__ cu_q, int B, 
   __syncthreads();
 }
 
-// The same question answered by one wave without LDS, groups of the batch in the order of their last key position, farthest first (what
+// The same question answered by every wave for itself, without LDS or barriers. -> request (-1: past the last group), first token of the group.
+__device__ __forceinline__ int find_group_wave(const int* __restrict__ cu_q, int B, int QT, int index, int* tok0) {
+  const int lane = threadIdx.x & 63;
+  for (int c0 = 0; c0 < B; c0 += 64) {
+    const int n = c0 + lane < B ? (cu_q[c0 + lane + 1] - cu_q[c0 + lane] + QT - 1) / QT : 0;
+    int incl = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += v;
+    }
+    const uint64_t votes = __builtin_amdgcn_ballot_w64(incl > index);
+    if (votes) {
+      const int l = __builtin_ctzll(votes);
+      *tok0 = (index - __builtin_amdgcn_readlane(incl - n, l)) * QT;
+      return c0 + l;
+    }
+    index -= __builtin_amdgcn_readlane(incl, 63);
+  }
+  return -1;
+}
+
+// The same again with the batch's groups in the order of their last key position, farthest first (what
 // comes last in a launch should be short).  Up to 64 requests: the position x with #groups ending at or past x > index >= #groups ending past
 // x by bisection, then the rank among the groups that end at x.  More requests: last group first, in the order of the batch.
 // -> request (-1: past the last group), first token of the group.
@@ -223,24 +245,7 @@ __device__ __forceinline__ int find_group_by_keys(const int* __restrict__ cu_q, 
     *tok0 = ((lo - __builtin_amdgcn_readlane(start, b)) / QT - 1) * QT;
     return b;
   }
-  index = total_groups - 1 - index;
-  for (int c0 = 0; c0 < B; c0 += 64) {
-    const int n = c0 + lane < B ? (cu_q[c0 + lane + 1] - cu_q[c0 + lane] + QT - 1) / QT : 0;
-    int incl = n;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int v = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += v;
-    }
-    const uint64_t votes = __builtin_amdgcn_ballot_w64(incl > index);
-    if (votes) {
-      const int l = __builtin_ctzll(votes);
-      *tok0 = (index - __builtin_amdgcn_readlane(incl - n, l)) * QT;
-      return c0 + l;
-    }
-    index -= __builtin_amdgcn_readlane(incl, 63);
-  }
-  return -1;
+  return find_group_wave(cu_q, B, QT, total_groups - 1 - index, tok0);
 }
 
 bool dtype_ok(int dt) { return dt == MSGL_MIX_BF16 || dt == MSGL_MIX_F32; }

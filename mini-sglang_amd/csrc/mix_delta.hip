@@ -17,7 +17,7 @@
 //                            fp32 online softmax, per-head sigmoid output gate; one workgroup per query token
 //   short_conv_kernel        causal per-channel convolution over time + SiLU, inputs before the portion from the request's
 //                            conv state; q / k heads made unit vectors (q also * d^-1/2);  conv_state_kernel shifts the state
-//   delta_rule_kernel        S <- decay S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q   per (request, head); a thread
+//   delta_rule_kernel        (decoded tokens, short portions and sizes that mix_delta_block.hip does not take:) S <- decay S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q   per (request, head); a thread
 //                            owns one value column of S in registers; scalar or per-key-channel decay; long portions as
 //                            parallel chunks: per-chunk transition (L | P), delta_scan_kernel over a request's chunks, outputs
 //   head_gated_norm_kernel   per-head rms over dv * w * (sigmoid | silu)(gate)

@@ -310,6 +310,52 @@ def test_delta_rule_state_slots_and_cuts(dev, chunk):
             assert rel(got, ref) < 1e-5, (per_channel, b)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("per_channel", [False, True], ids=["head", "channel"])
+@pytest.mark.parametrize("H,G,d,dv", [(4, 2, 128, 128), (3, 3, 64, 32), (2, 1, 128, 32), (8, 8, 64, 96)])
+def test_delta_rule_blocks(dev, H, G, d, dv, per_channel, dtype):
+    """Portions around the blocks of 16 tokens, fresh and continued, on state rows that hold garbage, with decays from nearly 1 to
+    nearly 0 (products that underflow within a block), against the token loop in float64.  Bound: some 30 fp32 roundings of 2^-24 on
+    the way of a sum of unit vectors' products, 1e-5 of the largest value with room."""
+    from mini_sglang_amd import mixops
+
+    new, old = [16, 1, 45, 100, 17, 0, 15], [0, 8, 5, 0, 16, 3, 0]
+    g = torch.Generator().manual_seed(d + dv + H)
+    B, T, n = len(new), sum(new), H * d if per_channel else H
+    rnd = lambda *x: torch.randn(*x, generator=g, dtype=torch.float64)  # noqa: E731
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)  # noqa: E731
+    q, k, v = unit(rnd(T, G, d)) * d ** -0.5, unit(rnd(T, G, d)), rnd(T, H, dv)
+    b_raw, a_raw = rnd(T, H).to(dtype).double(), (3.0 * rnd(T, n)).to(dtype).double()
+    q, k, v = (x.float().double() for x in (q, k, v))
+    rate, dt = -torch.exp(rnd(H)).float().double(), (0.5 * rnd(n)).float().double()
+    state = rnd(B + 1, H, d, dv).float()
+    got_state = state.to(dev)
+    out = torch.empty((T, H * dv), dtype=torch.float32, device=dev)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    cu = [0]
+    for x in new:
+        cu.append(cu[-1] + x)
+    assert mixops.mix_lib().msgl_mix_delta_rule_blocks_floats(T, B, H, d, dv) > 0
+    mixops.delta_rule(out, torch.cat([q.reshape(T, -1), k.reshape(T, -1), v.reshape(T, -1)], 1).float().to(dev), got_state, b_raw.to(dtype).to(dev), a_raw.to(dtype).to(dev),
+                      per_channel, rate.float().to(dev), dt.float().to(dev), i32(cu), i32([x + y for x, y in zip(new, old)]), i32(range(1, B + 1)), B, G)
+    out, got_state = out.double().cpu().view(T, H, dv), got_state.double().cpu()
+    decay = torch.exp(rate[:, None] * torch.nn.functional.softplus(a_raw + dt).view(T, H, -1))
+    for b, m in enumerate(new):
+        if m == 0:
+            assert torch.equal(got_state[b + 1], state[b + 1].double())
+            continue
+        S, ref = state[b + 1].double() * (1.0 if old[b] else 0.0), []
+        for t in range(cu[b], cu[b + 1]):
+            kk, qq = k[t].repeat_interleave(H // G, 0), q[t].repeat_interleave(H // G, 0)
+            S = S * decay[t][:, :, None]
+            u = torch.sigmoid(b_raw[t])[:, None] * (v[t] - torch.einsum("hde,hd->he", S, kk))
+            S = S + kk[:, :, None] * u[:, None, :]
+            ref.append(torch.einsum("hde,hd->he", S, qq))
+        assert rel(out[cu[b]: cu[b + 1]], torch.stack(ref)) < 1e-5, (b, m)
+        assert rel(got_state[b + 1], S) < 1e-5, (b, m)
+    assert torch.equal(got_state[0], state[0].double())  # nobody's row
+
+
 # ----------------------------------------------------------------------------------------- schedules
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, FP32_TOL), (torch.bfloat16, BF16_TOL)], ids=["fp32", "bf16"])
 def test_whole_prompt(dtype, tol):
