@@ -11,6 +11,7 @@
 //   latent_prep_kernel       latent row: rms-norm(c) | rotate(k_r) -> cache[out_loc];  rotate(q_r) -> q_abs tail
 //   latent_attn_mfma_kernel  bf16 caches: one shared (c | k_r) key row for all heads through LDS, both products on the matrix
 //                            cores, fp32 online softmax, output in latent space; key ranges + latent_attn_merge_kernel for decode
+//                            (widths 512 + 64 and 256 + 64: mix_latent.hip)
 //   latent_attn_kernel       the same in plain fp32 (fp32 caches, shapes past the matrix-core instances)
 //   lightning_kernel         S <- decay * S + k v^T, o = S^T q per (request, head), state rows indexed by slot; long portions
 //                            as parallel chunks joined by lightning_scan_kernel
@@ -910,6 +911,11 @@ __global__ __launch_bounds__(64) void latent_attn_merge_kernel(float* __restrict
 
 }  // namespace
 
+// mix_latent.hip: latent attention at the usual widths (1 launched, 0 not its sizes, < 0 error)
+extern "C" int mix_latent_attn_mfma(float* out, float* part_o, float* part_ml, const float* q_abs, const void* cache, const int* table,
+                                    int64_t table_stride, const int* req_rows, const int* seq_lens, const int* cu_q, int batch, int total_q, int H,
+                                    int dk, int dv, float scale, const float* sink, int splits, hipStream_t s);
+
 extern "C" {
 
 static thread_local char g_err[512] = "";
@@ -991,6 +997,9 @@ int msgl_mix_latent_attn(float* out, const float* q_abs, const void* cache, cons
     MIX_REQUIRE(grid.y <= 65535, "latent_attn: too many heads");
     float* part_o = workspace;
     float* part_ml = workspace ? workspace + (size_t)total_q * H * splits * dv : nullptr;
+    const int done = mix_latent_attn_mfma(out, part_o, part_ml, q_abs, cache, table, table_stride, req_rows, seq_lens, cu_q, batch, total_q, H, dk,
+                                          dv, scale, sink, splits, s);
+    if (done) return done < 0 ? done : MSGL_MIX_OK;
     const int vec = (((uintptr_t)cache & 15u) == 0 && dk % 8 == 0) ? 1 : 0;
 #define ATTN_CASE(KC, VC)                                                                                                              \
   if (dk <= KC * 32 && dv <= VC * 16) {                                                                                                \

@@ -129,6 +129,12 @@ def latent_attn(out: torch.Tensor, q_abs: torch.Tensor, cache: torch.Tensor, tab
     assert out.shape == (T, H, dv) and cache.is_contiguous() and cache.shape[1] == dk
     assert table.dtype == torch.int32 and table.stride(1) == 1
     assert req_rows.numel() >= batch and seq_lens.numel() >= batch and cu_q.numel() >= batch + 1
+    if splits == 1 and cache.dtype == torch.bfloat16 and (dk, dv) in ((576, 512), (320, 256)):
+        # Portions of few rows: 128 of them fill a CU, and with fewer than half of the CUs at work their keys are cut into ranges (of at
+        # least 128 keys, a rule of the kernel: short sequences leave the later ranges empty).  One portion, 16 heads: 32 tokens after 1000
+        # keys 85 -> 38 us, 512 fresh tokens 50 -> 46 us; 128 fresh ones (one range has keys) 21.5 -> 22 us.
+        groups = (T // max(1, 128 // min(H, 128)) + batch) * -(-H // 128)
+        splits = max(1, min(256 // max(groups, 1), table.shape[1] // 256, 8)) if T > batch * (16 // min(H, 16)) else 1
     ws = None
     if splits > 1:
         ws = torch.empty(mix_lib().msgl_mix_latent_attn_workspace_floats(T, H, dv, splits), dtype=torch.float32, device=out.device)

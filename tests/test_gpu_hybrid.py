@@ -323,6 +323,47 @@ def test_latent_attention_matrix_core_batch(dev):
             assert float((got - ref).abs().max()) < 2e-2, (b, t)
 
 
+@pytest.mark.parametrize("splits", [1, 3], ids=["one-range", "three-ranges"])
+@pytest.mark.parametrize("H,R", [(16, 512), (8, 512), (16, 256), (20, 256), (3, 512)])
+@pytest.mark.parametrize("sink", [False, True], ids=["plain", "sink"])
+def test_latent_attention_usual_widths(dev, H, R, splits, sink):
+    """The kernels of the usual widths: portions of 1 - 70 new tokens after 0 - 200 cached ones in one launch, and a launch of single
+    tokens, at the edges of their 16- and 32-key tiles and 16- and 128-row groups, scores of which some late key passes the first ones by
+    far (the reference maximum has to move).  Bound: the weights' bf16 rounding, 2^-9 of the weighted values' size, and the rounding of
+    scores' operands (2^-9 of a score of up to 30: 3 % of a weight where the top scores are close)."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(H + R)
+    r, scale = 64, (128 + 64) ** -0.5
+    sinks = torch.linspace(-3, 6, H) if sink else None
+    for new, old in (([70, 1, 33, 5, 8, 1], [0, 200, 31, 3, 64, 0]), ([1] * 6, [0, 14, 15, 16, 63, 300])):
+        B, T = len(new), sum(new)
+        slots, at = torch.randperm(1024, generator=g), 0
+        table, cache = torch.zeros((B, 320), dtype=torch.int32), torch.randn(1024, R + r, generator=g).bfloat16()
+        q = torch.randn(T, H, R + r, generator=g) * 0.8
+        refs, row, cu = [], 0, [0]
+        for b, (n, c) in enumerate(zip(new, old)):
+            mine = slots[at: at + n + c]
+            at += n + c
+            table[b, : n + c] = mine.int()
+            cache[mine[(n + c) // 2]] *= 2.5  # a loud key half way
+            keys = cache[mine].double()
+            s = torch.einsum("thk,jk->thj", q[row: row + n].double(), keys) * scale
+            s = s.masked_fill(torch.arange(n + c)[None, None, :] > (torch.arange(n) + c)[:, None, None], -torch.inf)
+            if sink:
+                s = torch.cat([s, sinks.double()[None, :, None].expand(n, H, 1)], dim=2)
+            refs.append(torch.softmax(s, -1)[..., : n + c] @ keys[:, :R])
+            row += n
+            cu.append(row)
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+        out = torch.full((T, H, R), float("nan"), device=dev)
+        mixops.latent_attn(out, q.to(dev), cache.to(dev), table.to(dev), i32(range(B)), i32([n + c for n, c in zip(new, old)]), i32(cu), B, R, scale,
+                           splits=splits, sink=None if sinks is None else sinks.to(dev))
+        ref, got = torch.cat(refs), out.double().cpu()
+        assert float((got - ref).norm() / ref.norm()) < 8e-3, new
+        assert float((got - ref).abs().max()) < 5e-2 * float(ref.abs().max()), new
+
+
 # ----------------------------------------------------------------------------------------- schedules
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, FP32_TOL), (torch.bfloat16, BF16_TOL)], ids=["fp32", "bf16"])
 def test_whole_prompt(dtype, tol):
