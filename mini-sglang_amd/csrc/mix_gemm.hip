@@ -1,0 +1,214 @@
+// Grouped / segmented / gathered C = act(A B^T), both operands bf16, all rows in 16-byte pieces: the expert layers and per-head products of
+// msgl_mix_gemm_nt.  seqmix.hip keeps the kernels for fp32 operands, unaligned rows and odd K.
+//
+// Both operands come to LDS by DMA in k steps of KS = 64 (32 where K is no multiple of 64), ST stages in a ring, one barrier a step.  A DMA
+// writes its 64 lanes' pieces one after the other, so a row's pieces change places by the row's number when they are fetched: 16 rows'
+// fragment reads then touch every bank once.  The rows of B go to the MFMA's rows in an order that leaves a lane eight neighbouring columns
+// of two tiles: 16-byte stores.
+// An output element's k order is that of the other matrix-core kernel, ascending in blocks of 32, wherever its row lies: the same bits.
+#include "mix_common.h"
+
+namespace {
+
+typedef __attribute__((address_space(1))) void glb_void_t;
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// The length of the list of row tiles, group by group.
+template <int MT>
+__device__ __forceinline__ int count_tiles(const int* __restrict__ seg, int groups, int M) {
+  if (!seg) return groups * ((M + MT - 1) / MT);
+  int n = 0;
+  for (int g = threadIdx.x & 63; g < groups; g += 64) n += (seg[g + 1] - seg[g] + MT - 1) / MT;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) n += __shfl_xor(n, o, 64);
+  return __builtin_amdgcn_readfirstlane(n);
+}
+
+// What bounds it: for long segments the rows' way to LDS (256 x 256 tiles: 64 KB for 2048 cycles of the matrix cores, at 8 TB/s in all, four
+// fifths of what a large library product draws) and tiles that the last round of CUs and the segments' ends leave empty; for short ones the
+// way of B from memory.  k steps of 64 are whole cache lines of both operands: with steps of 32 and twice the stages the same tiles are
+// a quarter slower.
+//   64 experts x 768 rows, N 1024, K 2048: 539 -> 265 us (777 TFLOP/s); 64 x 3 rows: 123 -> 100 us (268 MB of weights)
+//   MT x NT = 256 x 256, 8 waves of 64 x 128   long segments
+//             128 x 128, 4 waves of 64 x 64    middling ones: two workgroups a CU
+//              64 x 128, 4 waves of 64 x 32    short ones: the ring holds 2 x 2 x 16 KB of B per CU under way
+template <typename TC, int MT, int NT, int W, int WR, int KS, int ST>
+__global__ __launch_bounds__(64 * W, 2) void gemm_nt_dma_kernel(TC* __restrict__ C, const bf16_t* __restrict__ A, const bf16_t* __restrict__ Bm, int M,
+                                                             int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int groups, int64_t a_gs,
+                                                             int64_t b_gs, int64_t c_gs, const int* __restrict__ seg,
+                                                             const int* __restrict__ a_rows, int a_div, const int* __restrict__ c_rows, int act) {
+  constexpr int WC = W / WR, TI = MT / WR / 16, TJ = NT / WC / 16;  // waves by rows x columns; a wave's 16 x 16 tiles
+  constexpr int ROW = KS * 2, LPR = KS / 8, RPI = 64 / LPR;  // bytes of a row in LDS; lanes (pieces) of a row, rows of a DMA instruction
+  constexpr int STAGE = (MT + NT) * ROW, UA = MT / RPI / W, UB = NT / RPI / W, U = UA + UB;  // bytes; DMA instructions of a wave and step
+  static_assert((KS == 32 || KS == 64) && MT % (W * RPI) == 0 && NT % (W * RPI) == 0 && TJ % 2 == 0, "tiles");
+  extern __shared__ __attribute__((aligned(1024))) char ring[];  // [ST][MT rows of A | NT rows of B][KS]
+  const int n_cols = (N + NT - 1) / NT, total = count_tiles<MT>(seg, groups, M) * n_cols;
+  // neighbours in the list share rows of A or B: a run of them to each XCD
+  const int per = (total + 7) / 8, t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || t >= total) return;
+  const int rt = t / n_cols, n0 = (t - rt * n_cols) * NT;
+  int g, m0, row0 = 0, rows = M;
+  if (seg) {
+    g = find_group_wave(seg, groups, MT, rt, &m0);
+    row0 = seg[g];
+    rows = seg[g + 1] - row0;
+  } else {
+    const int each = (M + MT - 1) / MT;
+    g = rt / each;
+    m0 = (rt - g * each) * MT;
+  }
+  const bf16_t* Ag = A + (seg ? 0 : g * a_gs);
+  const bf16_t* Bg = Bm + g * b_gs;
+  TC* Cg = C + (seg ? 0 : g * c_gs);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lg = lane >> 4;
+  const int wm = wave / WC * (MT / WR), wn = wave % WC * (NT / WC);
+  // instruction u of this wave: LPR lanes a row; rows past the end read the last one (never stored).  A row's piece p lies at place p ^ key.
+  const auto a_key = [](int r) { return KS == 32 ? (r >> 2) & 3 : (r >> 1) & 7; };
+  const auto b_key = [](int r) { return KS == 32 ? (r >> 3) & 3 : ((r >> 1) & 1) | ((r >> 2) & 6); };
+  const char* src[U];
+#pragma unroll
+  for (int u = 0; u < UA; ++u) {
+    const int r = RPI * (wave + W * u) + lane / LPR, m = row0 + min(m0 + r, rows - 1);
+    src[u] = reinterpret_cast<const char*>(Ag + (int64_t)(a_rows ? a_rows[m] / a_div : m) * lda) + ((lane & (LPR - 1)) ^ a_key(r)) * 16;
+  }
+#pragma unroll
+  for (int u = 0; u < UB; ++u) {
+    const int r = RPI * (wave + W * u) + lane / LPR;
+    src[UA + u] = reinterpret_cast<const char*>(Bg + (int64_t)min(n0 + r, N - 1) * ldb) + ((lane & (LPR - 1)) ^ b_key(r)) * 16;
+  }
+  auto dma = [&](int stage) {
+    char* dst = ring + stage * STAGE + wave * 1024;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      __builtin_amdgcn_global_load_lds((glb_void_t*)src[u], (lds_void_t*)(dst + (u < UA ? u * W * 1024 : MT * ROW + (u - UA) * W * 1024)), 16, 0, 0);
+      src[u] += ROW;
+    }
+  };
+  f32x4_t acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const bool live = m0 + wm < rows;  // this wave has rows
+  const int n_steps = K / KS;
+#pragma unroll
+  for (int i = 0; i < ST - 1; ++i)
+    if (i < n_steps) dma(i);
+  int a_off[KS / 32], b_off[KS / 32];  // for each block of 32 of the step
+#pragma unroll
+  for (int kb = 0; kb < KS / 32; ++kb) {
+    const int bn = 8 * (lr >> 2) + (lr & 3);  // + 4: the pair's second tile (the same key)
+    a_off[kb] = (wm + lr) * ROW + ((4 * kb + lg) ^ a_key(lr)) * 16;
+    b_off[kb] = (MT + wn + bn) * ROW + ((4 * kb + lg) ^ b_key(bn)) * 16;
+  }
+  int at = 0;
+  for (int step = 0; step < n_steps; ++step) {
+    // this wave's pieces of the step have come when only those of the later ones are under way (memory counters retire in order)
+    if (step + ST - 2 < n_steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 2) * U) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // everybody's; everybody done with the stage before
+    if (step + ST - 1 < n_steps) dma(at == 0 ? ST - 1 : at - 1);
+    if (live) {
+      const char* buf = ring + at * STAGE;
+#pragma unroll
+      for (int kb = 0; kb < KS / 32; ++kb) {
+        bf16x8_t fa[TI], fb[TJ];
+#pragma unroll
+        for (int i = 0; i < TI; ++i) fa[i] = *reinterpret_cast<const bf16x8_t*>(buf + a_off[kb] + i * 16 * ROW);
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) fb[j] = *reinterpret_cast<const bf16x8_t*>(buf + b_off[kb] + (j >> 1) * 32 * ROW + (j & 1) * 4 * ROW);
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+          for (int i = 0; i < TI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+      }
+    }
+    at = at == ST - 1 ? 0 : at + 1;
+  }
+  // lane holds C[m = tile row lr][n = 32 pair + 8 lg .. + 7]
+  int at_row[TI];
+#pragma unroll
+  for (int i = 0; i < TI; ++i) {
+    const int m = row0 + min(m0 + wm + i * 16 + lr, rows - 1);
+    at_row[i] = c_rows ? c_rows[m] : m;
+  }
+#pragma unroll
+  for (int i = 0; i < TI; ++i) {
+    if (m0 + wm + i * 16 + lr >= rows) continue;
+    TC* row = Cg + (int64_t)at_row[i] * ldc;
+#pragma unroll
+    for (int p = 0; p < TJ / 2; ++p) {
+      const int n = n0 + wn + 32 * p + 8 * lg;
+      float v[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        v[c] = acc[i][2 * p + (c >> 2)][c & 3];
+        if (act == MSGL_MIX_ACT_RELU2) {
+          v[c] = fmaxf(v[c], 0.f);
+          v[c] = v[c] * v[c];
+        }
+      }
+      if (n >= N) continue;
+      if constexpr (sizeof(TC) == 2) {
+        *reinterpret_cast<Q4*>(row + n) = Q4{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
+      } else {
+        *reinterpret_cast<float4*>(row + n) = float4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<float4*>(row + n + 4) = float4{v[4], v[5], v[6], v[7]};
+      }
+    }
+  }
+}
+
+}  // namespace
+
+// 1: launched; 0: not this kernel's operands (the caller takes the other ones); < 0: an error code.
+extern "C" __attribute__((visibility("hidden"))) int mix_gemm_nt_dma(void* C, const void* A, const void* B, int M, int N, int K, int64_t lda, int64_t ldb,
+                                                                     int64_t ldc, int groups, int64_t a_gs, int64_t b_gs, int64_t c_gs, const int* seg,
+                                                                     const int* a_rows, int a_div, const int* c_rows, int act, int tc, hipStream_t s) {
+  const auto al = [](const void* p, int64_t ld, int64_t gs) { return ((uintptr_t)p & 15u) == 0 && ld % 8 == 0 && gs % 8 == 0; };
+  if (K % 32 || N % 8 || !al(A, lda, a_gs) || !al(B, ldb, b_gs) || !al(C, ldc, c_gs)) return 0;
+  const auto blocks = [&](int mt, int nt) -> int64_t {  // the most tiles there can be, in whole rounds of the XCDs
+    const int64_t list = seg ? (int64_t)M / mt + groups : (int64_t)groups * ((M + mt - 1) / mt);
+    return (list * ((N + nt - 1) / nt) + 7) / 8 * 8;
+  };
+#define GEMM_RUN(TC, MT, NT, W, WR, KS, ST)                                                                                                  \
+  {                                                                                                                                   \
+    const int64_t n = blocks(MT, NT);                                                                                                 \
+    if (n > 0x7fffffff) return 0;                                                                                                     \
+    const size_t lds = (size_t)ST * (MT + NT) * KS * 2;                                                                                   \
+    MIX_REQUIRE(ensure_lds((const void*)gemm_nt_dma_kernel<TC, MT, NT, W, WR, KS, ST>, lds) == 0, "gemm_nt: %zu bytes of LDS", lds);         \
+    hipLaunchKernelGGL((gemm_nt_dma_kernel<TC, MT, NT, W, WR, KS, ST>), dim3((unsigned)n), dim3(64 * W), lds, s, mp<TC>(C), cp<bf16_t>(A),      \
+                       cp<bf16_t>(B), M, N, K, lda, ldb, ldc, groups, a_gs, b_gs, c_gs, seg, a_rows, a_div, c_rows, act);             \
+  }
+  // Rows per group on average, and how many of the largest tiles there are.  Groups x rows, N, K (us, weights not in cache):
+  //                              64 x 128   128 x 128   256 x 256
+  //   16 x 62, 1536, 1024           24.6       26.8        34.8
+  //   64 x 64, 1024, 2048            114        105         106
+  //   16 x 188, 1536, 1024          37.9       30.9        39.9    96 large tiles: most CUs without one
+  //   32 x 188, 1024, 1024          45.2       38.5        43.7
+  //   64 x 128, 1024, 2048           134        126         117
+  //   16 x 1500, 1024, 768          93.1       72.6        63.0
+  //   64 x 768, 1024, 2048           420        304         265
+  //   64 x 256, 2048, 512            106       82.1        88.0    (the one of 19 sizes measured where the rule misses by more than 3 %)
+  const int64_t each = seg ? M / groups : M;
+  const bool large = each >= 96 && blocks(256, 256) >= 256;
+#define GEMM_SIZE(TC)                                                   \
+  {                                                                     \
+    if (K % 64) {                                                       \
+      if (each < 64) GEMM_RUN(TC, 64, 128, 4, 1, 32, 6)                 \
+      else GEMM_RUN(TC, 128, 128, 4, 2, 32, 4)                          \
+    } else if (each < 64) {                                             \
+      GEMM_RUN(TC, 64, 128, 4, 1, 64, 3)                                \
+    } else if (!large) {                                                \
+      GEMM_RUN(TC, 128, 128, 4, 2, 64, 2)                               \
+    } else {                                                            \
+      GEMM_RUN(TC, 256, 256, 8, 4, 64, 2)                               \
+    }                                                                   \
+  }
+  if (tc == MSGL_MIX_BF16) GEMM_SIZE(bf16_t)
+  else GEMM_SIZE(float)
+#undef GEMM_SIZE
+#undef GEMM_RUN
+  MIX_LAUNCHED("gemm_nt (matrix cores, DMA)");
+  return 1;
+}

@@ -19,7 +19,8 @@
 //   route_kernel             fp32 router on fp32 logits (mix_route.h): softmax or sigmoid, bias-corrected group-limited top-k, normalised weights
 //   moe_count / moe_place    (token, choice) pairs bucketed by expert -> segment offsets + permutation
 //   gemm_nt_mfma_kernel      grouped / segmented / gathered C = act(A B^T) for 16-bit weights on the matrix cores: per-head
-//                            latent products, expert layers, router logits of long batches
+//                            latent products, expert layers, router logits of long batches (bf16 x bf16 in whole 16-byte pieces:
+//                            mix_gemm.hip)
 //   gemm_nt_kernel           the same in fp32 FMA: fp32 engines, and every shape the library refuses
 #include "mix_route.h"
 
@@ -916,6 +917,11 @@ extern "C" int mix_latent_attn_mfma(float* out, float* part_o, float* part_ml, c
                                     int64_t table_stride, const int* req_rows, const int* seq_lens, const int* cu_q, int batch, int total_q, int H,
                                     int dk, int dv, float scale, const float* sink, int splits, hipStream_t s);
 
+// mix_gemm.hip: both operands bf16 in 16-byte pieces (1 launched, 0 not its operands, < 0 error)
+extern "C" int mix_gemm_nt_dma(void* C, const void* A, const void* B, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int groups,
+                               int64_t a_gs, int64_t b_gs, int64_t c_gs, const int* seg, const int* a_rows, int a_div, const int* c_rows, int act,
+                               int tc, hipStream_t s);
+
 extern "C" {
 
 static thread_local char g_err[512] = "";
@@ -1129,6 +1135,10 @@ int msgl_mix_gemm_nt(void* C, const void* A, const void* B, int M, int N, int K,
   if (tb == MSGL_MIX_BF16) {  // 16-bit weights: the matrix-core kernel
     const int row_tiles = (M + kMT - 1) / kMT;
     MIX_REQUIRE(row_tiles <= 65535, "gemm_nt: too many rows");
+    if (ta == MSGL_MIX_BF16) {
+      const int done = mix_gemm_nt_dma(C, A, B, M, N, K, lda, ldb, ldc, groups, a_gs, b_gs, c_gs, seg, a_rows, a_div, c_rows, act, tc, s);
+      if (done) return done < 0 ? done : MSGL_MIX_OK;
+    }
     const dim3 grid((N + kMT - 1) / kMT, row_tiles, groups);
     auto al = [](const void* p, int64_t ld, int64_t gs, int elems) {
       return ((uintptr_t)p & 15u) == 0 && ld % elems == 0 && gs % elems == 0;

@@ -364,6 +364,38 @@ def test_latent_attention_usual_widths(dev, H, R, splits, sink):
         assert float((got - ref).abs().max()) < 5e-2 * float(ref.abs().max()), new
 
 
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("N,K", [(256, 32), (128, 64), (264, 96), (520, 256), (72, 128)])
+@pytest.mark.parametrize("lens", [[1, 0, 63, 2, 16], [64, 65, 0, 127, 128, 129, 300], [255, 256, 257] * 30, [0, 0, 700, 17] + [1] * 70], ids=["short", "edges", "long", "many"])
+def test_segmented_product_tiles(dev, lens, N, K, out):
+    """Every tile size of the DMA kernel at the edges of its tiles, k shorter and longer than its ring, gathered and scattered rows, against
+    float64.  Bound: fp32 sums of K exact products, and the rounding of a bf16 result (2^-9 of its size)."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(N + K + len(lens))
+    E, rows = len(lens), sum(lens)
+    seg = torch.tensor([0] + lens).cumsum(0).int()
+    a = torch.randn((rows + 1) // 2, K, generator=g).bfloat16()  # two choices a token
+    b = torch.randn(E, N, K, generator=g).bfloat16()
+    perm, place = torch.randperm(rows, generator=g).int(), torch.randperm(rows, generator=g).int()
+    got = torch.full((rows, N), float("nan"), dtype=out, device=dev)
+    mixops.gemm_nt(got, a.to(dev), b.to(dev), rows, N, K, lda=K, ldb=K, ldc=N, groups=E, b_gs=N * K, seg=seg.to(dev), a_rows=perm.to(dev), a_div=2,
+                   c_rows=place.to(dev), act=mixops.ACT_RELU2)
+    ref = torch.empty(rows, N, dtype=torch.float64)
+    for e in range(E):
+        m = slice(int(seg[e]), int(seg[e + 1]))
+        ref[place[m].long()] = (a[perm[m].long() // 2].double() @ b[e].double().T).clamp_min(0).square()
+    size = (a.double().abs().max() * b.double().abs().max() * K).square()  # of a result, at most; sums are off by K 2^-24 of it and far less
+    tol = ref * (2.0 ** -8 if out == torch.bfloat16 else 2.0 ** -18) + size * K * 2.0 ** -24
+    assert ((got.double().cpu() - ref).abs() <= tol).all()
+    # groups of equal size, rows in place
+    a3 = torch.randn(3, 70, K, generator=g).bfloat16()
+    got = torch.full((3, 70, N), float("nan"), dtype=out, device=dev)
+    mixops.gemm_nt(got, a3.to(dev), b[:1].expand(3, N, K).contiguous().to(dev), 70, N, K, lda=K, ldb=K, ldc=N, groups=3, a_gs=70 * K, b_gs=N * K, c_gs=70 * N)
+    ref = a3.double() @ b[0].double().T
+    assert ((got.double().cpu() - ref).abs() <= ref.abs() * 2.0 ** -8 * (out == torch.bfloat16) + size.sqrt() * K * 2.0 ** -23).all()
+
+
 # ----------------------------------------------------------------------------------------- schedules
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, FP32_TOL), (torch.bfloat16, BF16_TOL)], ids=["fp32", "bf16"])
 def test_whole_prompt(dtype, tol):
