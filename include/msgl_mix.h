@@ -92,7 +92,7 @@ int msgl_mix_gated_norm(void* out, const float* o, const void* gate, int64_t ld_
 int msgl_mix_route(int* ids, float* wts, const float* z, const void* bias, int tokens, int E, int top, int G, int keep, int sigmoid,
                    int group_best, float scale, int dtype, void* stream);
 
-/* seg[E + 1], perm[n]: flat (token, choice) indices bucketed by expert, stable inside a bucket; counts[E] is scratch. */
+/* seg[E + 1], perm[n]: flat (token, choice) indices bucketed by expert, stable inside a bucket; counts[E]: not used (may not be null). */
 int msgl_mix_moe_sort(int* seg, int* perm, int* counts, const int* ids, int n, int E, void* stream);
 
 /* C[g] = act(A[g] B[g]^T) with fp32 accumulation; groups advance by *_gs elements.  With seg, group g owns rows

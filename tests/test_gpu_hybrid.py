@@ -396,6 +396,23 @@ def test_segmented_product_tiles(dev, lens, N, K, out):
     assert ((got.double().cpu() - ref).abs() <= ref.abs() * 2.0 ** -8 * (out == torch.bfloat16) + size.sqrt() * K * 2.0 ** -23).all()
 
 
+@pytest.mark.parametrize("n,skip", [(1, 0), (7, 1), (2047, 0), (2048, 3), (2049, 0), (8191, 0), (8193, 1), (16385, 0), (40001, 2)])
+def test_bucketing_is_a_stable_sort(dev, n, skip):
+    """Rounds of 2048 and 8192 entries, their ends, an unaligned list, experts without entries, the first and the last expert: whole numbers, equal."""
+    from mini_sglang_amd import mixops
+
+    E = 20
+    ids = torch.randint(0, E // 2, (n + skip,), generator=torch.Generator().manual_seed(n)).mul_(2)[skip:]
+    ids[-1] = E - 1
+    seg, perm = mixops.moe_sort(ids.int().to(dev), E)
+    unaligned = torch.empty(n + skip, dtype=torch.int32, device=dev)[skip:]
+    unaligned.copy_(ids)
+    seg2, perm2 = mixops.moe_sort(unaligned, E)
+    assert torch.equal(perm.cpu().long()[:n], torch.sort(ids, stable=True).indices)
+    assert seg.cpu().tolist() == [0] + torch.bincount(ids, minlength=E).cumsum(0).tolist()
+    assert torch.equal(perm[:n], perm2[:n]) and torch.equal(seg, seg2)
+
+
 # ----------------------------------------------------------------------------------------- schedules
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, FP32_TOL), (torch.bfloat16, BF16_TOL)], ids=["fp32", "bf16"])
 def test_whole_prompt(dtype, tol):
