@@ -139,6 +139,14 @@ __device__ __forceinline__ Q4 load8(const float* p, int n, bool vec) {
 }
 
 // two fp32 numbers as packed bf16 (round to nearest even), one instruction
+// the larger of this lane's number and lane ^ 32's, without LDS: a swap of halves between two copies leaves both numbers in every lane
+__device__ __forceinline__ float pair_max(float x) {
+  const uint32_t a = __builtin_bit_cast(uint32_t, x);
+  const auto y = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+  const uint32_t y0 = y[0], y1 = y[1];  // (a bit cast of the vector's element itself takes element 0 both times)
+  return fmaxf(__builtin_bit_cast(float, y0), __builtin_bit_cast(float, y1));
+}
+
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
@@ -202,6 +210,35 @@ __device__ __forceinline__ int find_group_wave(const int* __restrict__ cu_q, int
   return -1;
 }
 
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+// The two packed bf16 weights added to a sum: the sum of what the products use, so that a row's weights add up to one
+__device__ __forceinline__ float add_pair(uint32_t p, float sum) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, p), __builtin_bit_cast(bf16x2_t, 0x3f803f80u), sum, false);
+}
+
+// A wave's sum / largest number of non-negative integers in every lane's scalar, by row shifts and broadcasts of the vector unit: eight
+// instructions (a shuffle is a trip through LDS, and the bisection below needs dozens of sums before a workgroup can start).
+template <typename F>
+__device__ __forceinline__ int wave_fold(int v, F f) {
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true));   // row_shr:1
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true));   // row_shr:2
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true));   // row_shr:4
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true));   // row_shr:8
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1 and 3
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2 and 3
+  return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_total(int v) {
+  return wave_fold(v, [](int a, int b) { return a + b; });
+}
+
+// how many groups of up to QT rows the batch has
+__device__ __forceinline__ int count_groups(const int* __restrict__ cu_q, int B, int QT) {
+  int n = 0;
+  for (int b = threadIdx.x & 63; b < B; b += 64) n += (cu_q[b + 1] - cu_q[b] + QT - 1) / QT;
+  return wave_total(n);
+}
+
 // The same again with the batch's groups in the order of their last key position, farthest first (what
 // comes last in a launch should be short).  Up to 64 requests: the position x with #groups ending at or past x > index >= #groups ending past
 // x by bisection, then the rank among the groups that end at x.  More requests: last group first, in the order of the batch.
@@ -218,19 +255,11 @@ __device__ __forceinline__ int find_group_by_keys(const int* __restrict__ cu_q, 
     }
     // groups of this lane's request that end at position x or later (the end of group p is start + QT (p + 1), the last one's rounded up)
     auto past = [&](int x) { return max(0, n - max(0, (x - start + QT - 1) / QT - 1)); };
-    auto total = [&](int v) {
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-      return __builtin_amdgcn_readfirstlane(v);
-    };
-    int hi = start + n * QT;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) hi = max(hi, __shfl_xor(hi, o, 64));
-    hi = __builtin_amdgcn_readfirstlane(hi) + 1;  // nothing ends here
+    int hi = wave_fold(start + n * QT, [](int a, int b) { return max(a, b); }) + 1;  // nothing ends here
     int lo = 0, above = 0;                        // everything ends past 0
-    if (total(n) <= index) return -1;
+    if (wave_total(n) <= index) return -1;
     while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1, c = total(past(mid));
+      const int mid = (lo + hi) >> 1, c = wave_total(past(mid));
       if (c > index) {
         lo = mid;
       } else {

@@ -15,7 +15,6 @@
 
 namespace {
 
-typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(1))) void glb_void_t;
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -41,11 +40,6 @@ __device__ __forceinline__ bf16x8_t scaled8(const float* p, float f) {
 __device__ __forceinline__ float weight(float s, float sharp, float ref) { return __builtin_amdgcn_exp2f(fmaf(s, sharp, -ref)); }
 // LDS accesses of one wave go in order; this keeps the compiler's order
 __device__ __forceinline__ void wave_fence() { asm volatile("" ::: "memory"); }
-// the two packed bf16 weights added to a sum: the sum of what the products use, so that a row's weights add up to one
-__device__ __forceinline__ float add_pair(uint32_t p, float sum) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_v, p), __builtin_bit_cast(bf16x2_v, 0x3f803f80u), sum, false);
-}
-
 template <int DK>
 struct LatentRow {
   static constexpr int pieces = DK / 8 + 1;   // 16-byte pieces of a row in LDS, the last one padding
@@ -192,8 +186,7 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
     float mx = -INFINITY;
 #pragma unroll
     for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    mx *= sharp;
+    mx = pair_max(mx) * sharp;
     if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
       const float m_new = fmaxf(m, mx);
       const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
@@ -430,8 +423,7 @@ __global__ __launch_bounds__(256, 1) void latent_decode_kernel(float* __restrict
       mx = fmaxf(mx, s[c]);
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    mx *= sharp;
+    mx = pair_max(mx) * sharp;
     if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
       const float m_new = fmaxf(m, mx);
       const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - m_new);

@@ -1190,6 +1190,12 @@ int msgl_mix_selective_scan(void* out, const void* x, int64_t ld_x, const void* 
   return MSGL_MIX_EINVAL;
 }
 
+// mix_maps.hip: two maps, portions of prompts (1 launched, 0 not its sizes, < 0 error)
+extern "C" int mix_maps_prompt(void* out, int64_t ld_out, float* part_o, float* part_ml, const float* q, const void* k_cache, const void* v_cache, const int* table,
+                    int64_t table_stride, const int* req_rows, const int* seq_lens, const int* cu_q, int batch, int total_q, int H, int G, int d, int dv,
+                    float scale, int window, int keep, const float* lam, const void* gate, int64_t ld_gate, float post, float eps, int splits,
+                    hipStream_t s);
+
 // both forms of the attention: MAPS = 1 with an optional sink, MAPS = 2 the difference of two maps
 namespace {
 
@@ -1240,6 +1246,12 @@ int sink_attn_any(void* out, int64_t ld_out, const float* q, const void* k_cache
     while (HBm * 2 <= rep && HBm * 2 <= 64) HBm *= 2;
     // few rows per request (decode): 16 rows per workgroup, the tiles' keys spread over its waves
     const bool spread = HBm <= 16 && total_q <= batch * (16 / HBm);
+    if (MAPS == 2 && !spread) {
+      const int done = mix_maps_prompt(out, ld_out, part_o, part_ml, q, k_cache, v_cache, table, table_stride, req_rows, seq_lens, cu_q, batch, total_q,
+                                       H, G, d, dv, scale, window, keep, df.lam, df.gate, df.ld_gate, df.post, df.eps, splits, s);
+      if (done < 0) return done;
+      if (done) return sink_merge_launch<bf16_t, MAPS>(s, mp<bf16_t>(out), ld_out, part_o, part_ml, total_q, H, dv, splits, sink, df);
+    }
     const int QTm = (spread ? 16 : 64) / HBm, hbl = (rep + HBm - 1) / HBm;
     const int groups_m = (total_q + QTm - 1) / QTm + batch;
     MIX_REQUIRE((int64_t)G * hbl <= 65535, "sink_attn: too many heads");

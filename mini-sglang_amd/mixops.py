@@ -762,6 +762,14 @@ def diff_attn(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
     assert table.dtype == torch.int32 and table.stride(1) == 1 and _f32(lam, 1) is not None
     assert gate is None or (gate.shape == (T, H * dv) and gate.stride(1) == 1 and gate.dtype == out.dtype)
     assert req_rows.numel() >= batch and seq_lens.numel() >= batch and cu_q.numel() >= batch + 1
+    if splits == 1 and k_cache.dtype == torch.bfloat16 and (d, dv) == (64, 128):
+        # Portions of few rows: the kernel's groups of 128 rows leave most CUs idle, so their keys are cut into ranges (of at least 256 keys, a
+        # rule of the kernel).  16 heads on 4, one portion: 32 tokens after 1000 keys 51 -> 30 us, 128 after 2000 86 -> 39 us; 512 fresh ones
+        # (68 groups) 29 us in one range, 36 us in three.
+        hb = min(1 << ((H // G).bit_length() - 1), 32)
+        groups = (T // (128 // hb) + batch) * G * -(-(H // G) // hb)
+        if T > batch * (16 // min(hb, 16)) and groups <= 64:
+            splits = max(1, min(256 // groups, table.shape[1] // 256, 8))
     ws = None
     if splits > 1:
         ws = torch.empty(mix_lib().msgl_mix_sink_attn_workspace_floats(T, 2 * H, dv, splits), dtype=torch.float32, device=out.device)

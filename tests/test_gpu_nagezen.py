@@ -643,3 +643,38 @@ def test_trace_command_line(tmp_path):
     assert float((got0 - ra[[0, 29]]).abs().max()) < FP32_TOL * scale
     assert float((got1 - ra[[30]]).abs().max()) < FP32_TOL * scale
     assert float((got2[0] - ra[44]).abs().max()) < FP32_TOL * scale and float((got2[1] - rb[8]).abs().max()) < FP32_TOL * scale
+
+
+@pytest.mark.parametrize("window,keep", [(0, 0), (45, 0), (100, 13), (64, 64), (3, 200)])
+@pytest.mark.parametrize("H,G", [(16, 4), (8, 2), (4, 4), (6, 2), (40, 1)])
+def test_diff_attention_portions_of_usual_width(dev, H, G, window, keep):
+    """The kernel of prompt portions (64 / 128 wide): four requests in one launch whose portions end around its 128-row groups and 32- and
+    64-key tiles, windows and kept keys inside tiles, heads per group that are no power of two and more than 32, one range and three, with
+    and without a gate.  Bound: bf16 weights (2^-9) under a difference of maps about as large as each of them, and the bf16 result."""
+    from mini_sglang_amd import mixops
+
+    d, dv, scale, lam, eps = 64, 128, 64 ** -0.5, 0.4, 1e-5
+    new, old = [70, 33, 128, 19], [0, 95, 1, 200]
+    g = torch.Generator().manual_seed(H + window + keep)
+    lens, B = [a + b for a, b in zip(new, old)], len(new)
+    seqs = [tuple(torch.randn(n, *w, generator=g, dtype=torch.float64).bfloat16().double() for w in ((H, 2, d), (G, 2, d), (G, dv), (H, dv))) for n in lens]
+    kc, vc = (torch.zeros((1024, n), dtype=torch.bfloat16, device=dev) for n in (G * 2 * d, G * dv))
+    table, perm, at = torch.zeros((B + 1, 256), dtype=torch.int32), torch.randperm(1024, generator=g), 0
+    for b, (_, k, v, _) in enumerate(seqs):
+        sl = perm[at: at + lens[b]]
+        at += lens[b]
+        table[b + 1, : lens[b]] = sl.int()
+        kc[sl.to(dev)] = k.reshape(lens[b], -1).bfloat16().to(dev)
+        vc[sl.to(dev)] = v.reshape(lens[b], -1).bfloat16().to(dev)
+    qd, gd = (torch.cat([s[i][n - m:].reshape(m, -1) for s, n, m in zip(seqs, lens, new)]) for i in (0, 3))
+    cu = torch.tensor([0] + new).cumsum(0).int().to(dev)
+    for splits, gate in ((1, True), (1, False), (3, True)):
+        out = torch.full((sum(new), H * dv), float("nan"), dtype=torch.bfloat16, device=dev)
+        mixops.diff_attn(out, qd.float().to(dev), kc, vc, table.to(dev), torch.arange(1, B + 1, dtype=torch.int32, device=dev),
+                         torch.tensor(lens, dtype=torch.int32, device=dev), cu, B, H, G, d, dv, scale, window, keep,
+                         torch.tensor([lam], dtype=torch.float32, device=dev), 0.7, eps, gate=gd.bfloat16().to(dev) if gate else None, splits=splits)
+        got, at = out.double().cpu().view(sum(new), H, dv), 0
+        for (q, k, v, gt), n, m in zip(seqs, lens, new):
+            ref = _diff_ref(q, k, v, scale, window, keep, lam, 0.7, eps, gt if gate else torch.full_like(gt, torch.inf))[n - m:]
+            assert rel(got[at: at + m], ref) < 1e-2, (splits, gate, n)
+            at += m
