@@ -148,6 +148,20 @@ __device__ __forceinline__ uint2 tr_read_b64(const char* lds_ptr) {
   return __builtin_bit_cast(uint2, r);
 }
 
+// Two weights as a packed pair, added to the row's sum: in bf16 the rounded ones in one instruction, so that the weights that P.V uses add up
+// to one; in fp16 the fp32 ones (small weights are subnormal there, which the dot product may drop).
+template <typename T>
+__device__ __forceinline__ uint32_t weight_pair(float e0, float e1, float* sum) {
+  const uint32_t p = Elem<T>::pack(e0, e1);
+  if constexpr (std::is_same_v<T, BF16>) {
+    typedef __bf16 v2 __attribute__((ext_vector_type(2)));
+    *sum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2, p), __builtin_bit_cast(v2, 0x3f803f80u), *sum, false);
+  } else {
+    *sum += e0 + e1;
+  }
+  return p;
+}
+
 constexpr int kTileBytes = kKTile * kD * 2;  // 16 KB: one K (or V) tile image
 
 // ABL (diagnosis only, wrong results): 1 = K/V tiles loaded once (no HBM/L2 stream, no LDS writes after the first tile),
@@ -286,7 +300,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
       l_run += s[0][0] + s[1][15];
     } else {
       float tmax = kNegBigP;
-      float m_new, alpha, rsum = 0.f;
+      float m_new, alpha;
       const bool need_mask = key0 + kKTile - 1 > wave_min_qpos;
       if constexpr (!kFold) {
   #pragma unroll
@@ -311,7 +325,6 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
           for (int r = 0; r < 16; ++r) {
             const float e = __builtin_amdgcn_exp2f(s[kb][r] - m_new);
             s[kb][r] = e;
-            rsum += e;
           }
         }
       } else {
@@ -337,18 +350,20 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
           for (int r = 0; r < 16; ++r) {
             const float e = __builtin_amdgcn_exp2f(fmaf(s[kb][r], p.scale_log2, -m_new));
             s[kb][r] = e;
-            rsum += e;
           }
         }
       }
-      rsum += __shfl_xor(rsum, 32, 64);
-      l_run = fmaf(l_run, alpha, rsum);
       if (!__all(m_new == m_run)) {  // alpha == 1 on every row otherwise: the rescale would be the identity
+        l_run *= alpha;
   #pragma unroll
         for (int nb = 0; nb < 4; ++nb)
   #pragma unroll
           for (int r = 0; r < 16; ++r) o[nb][r] *= alpha;
       }
+  #pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+  #pragma unroll
+        for (int r = 0; r < 16; r += 2) (void)weight_pair<T>(s[kb][r], s[kb][r + 1], &l_run);
       m_run = m_new;
     }
 
@@ -383,6 +398,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
   }
 
   // ---- epilogue: O[q row][d] = O^T / l ---------------------------------------------------------
+  l_run += __shfl_xor(l_run, 32, 64);  // the lanes' shares of the row's sum
   if (q_valid) {
     const float inv = 1.0f / l_run;
     uint16_t* op = p.out + (int64_t)(q_begin + my_q) * p.out_stride + (int64_t)hq * kD;
@@ -416,6 +432,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) const void glb_void_t;
 
+// the larger of this lane's number and lane ^ 32's, without LDS: a swap of halves between two copies leaves both numbers in every lane
+__device__ __forceinline__ float pair_max(float x) {
+  const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  const uint32_t y0 = y[0], y1 = y[1];
+  return fmaxf(__uint_as_float(y0), __uint_as_float(y1));
+}
 template <typename T, int ABL = 0>
 __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillParams p, int total_tiles) {
   // two distinct LDS objects, not one array: the compiler then knows a tile's fragment reads cannot alias the DMA writes
@@ -548,17 +570,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
         if (ks < 4) {
           kf1[2 * ks] = *reinterpret_cast<const U4*>(buf + koff[2 * ks] + 8192);
           kf1[2 * ks + 1] = *reinterpret_cast<const U4*>(buf + koff[2 * ks + 1] + 8192);
-        } else if constexpr (!(ABL & 8)) {
-          vfa[ks - 4] = read_vf(0, 0, ks - 4);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) {
         s[1] = mfma32<T>(kf1[ks], qf[ks], s[1]);
-        if constexpr (!(ABL & 8)) {
-          if (ks < 4) vfa[4 + ks] = read_vf(0, 1, ks);
-        }
+        if constexpr (!(ABL & 8)) vfa[ks] = read_vf(0, ks >> 2, ks & 3);
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
@@ -573,9 +591,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
     }
     if constexpr (kPrioMatrix) __builtin_amdgcn_s_setprio(0);
     if constexpr (ABL & 32) __builtin_amdgcn_s_setprio(1);
+    uint32_t pw[2][8];  // the weights, packed in pairs
     if constexpr (ABL & 4) {
       m_run = 0.f;
       l_run += s[0][0] + s[1][15];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) pw[kb][r >> 1] = Elem<T>::pack(s[kb][r], s[kb][r + 1]);
     } else {
       // ---- causal mask (tiles crossing this wave's diagonal only): key0 + c + 4 hi > my_qpos  <=>  c > thr
       if (key0 + kKTile - 1 > wave_min_qpos) {
@@ -592,36 +615,32 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[kb][r]);
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * p.scale_log2;
-      const float m_new = fmaxf(m_run, tmax);
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      float rsum = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float e = __builtin_amdgcn_exp2f(fmaf(s[kb][r], p.scale_log2, -m_new));
-          s[kb][r] = e;
-          rsum += e;
-        }
-      rsum += __shfl_xor(rsum, 32, 64);
-      l_run = fmaf(l_run, alpha, rsum);
-      if (!__all(m_new == m_run)) {
+      tmax = pair_max(tmax) * p.scale_log2;
+      if (!__all(tmax <= m_run)) {
+        const float m_new = fmaxf(m_run, tmax);
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= alpha;
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) o[nb][r] *= alpha;
+        m_run = m_new;
       }
-      m_run = m_new;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2)
+          pw[kb][r >> 1] = weight_pair<T>(__builtin_amdgcn_exp2f(fmaf(s[kb][r], p.scale_log2, -m_run)),
+                                          __builtin_amdgcn_exp2f(fmaf(s[kb][r + 1], p.scale_log2, -m_run)), &l_run);
     }
     // ---- O^T += V^T . P^T: keys 0..31 on the fragments read during QK^T, the fragments of keys 32..63 read under them
     if constexpr (!(ABL & 8)) {
       auto pack_p = [&](int kb, int half) {
         U4 pf;
-        pf.x = Elem<T>::pack(s[kb][8 * half + 0], s[kb][8 * half + 1]);
-        pf.y = Elem<T>::pack(s[kb][8 * half + 2], s[kb][8 * half + 3]);
-        pf.z = Elem<T>::pack(s[kb][8 * half + 4], s[kb][8 * half + 5]);
-        pf.w = Elem<T>::pack(s[kb][8 * half + 6], s[kb][8 * half + 7]);
+        pf.x = pw[kb][4 * half];
+        pf.y = pw[kb][4 * half + 1];
+        pf.z = pw[kb][4 * half + 2];
+        pf.w = pw[kb][4 * half + 3];
         return pf;
       };
       U4 vfb[8];
@@ -657,6 +676,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
     if (kt + 1 < ntiles) tile_body(std::integral_constant<int, 1>{}, kt + 1);
   }
 
+  l_run += __shfl_xor(l_run, 32, 64);  // the lanes' shares of the row's sum
   if (q_valid) {
     const float inv = 1.0f / l_run;
     uint16_t* op = p.out + (int64_t)(q_begin + my_q) * p.out_stride + (int64_t)hq * kD;
