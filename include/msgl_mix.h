@@ -168,9 +168,9 @@ int msgl_mix_delta_rule(float* out, const float* qkv, float* state, const void* 
 
 /* The same rule in blocks of 16 tokens on the fp32 matrix instructions, for portions of tokens: everything that does not depend on the
  * state is computed for all blocks at once, then one walk per (request, head, 32 value columns).  Any batch; no chunk list.
- * msgl_mix_delta_rule_blocks_floats: floats of scratch for `total_q` new tokens of `batch` requests, 0 where these sizes have no such
- * form (d 64 or 128, dv a multiple of 32). */
-int64_t msgl_mix_delta_rule_blocks_floats(int64_t total_q, int batch, int H, int d, int dv);
+ * msgl_mix_delta_rule_block_floats: floats of a block and head, 0 where these sizes have no such form (d 64 or 128, dv a multiple of 32);
+ * scratch holds (total_q / 16 + batch) * H of them. */
+int msgl_mix_delta_rule_block_floats(int d, int dv);
 int msgl_mix_delta_rule_blocks(float* out, const float* qkv, float* state, const void* b_raw, int64_t ld_b, const void* a_raw, int64_t ld_a,
                                int per_channel, const float* rate, const float* dt_bias, const int* cu_q, const int* seq_lens,
                                const int* slots, int batch, int total_q, int H, int G, int d, int dv, int dtype, float* scratch,

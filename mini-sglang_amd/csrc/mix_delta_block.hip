@@ -441,9 +441,9 @@ __global__ __launch_bounds__(320) void delta_walk_kernel(float* __restrict__ out
 
 extern "C" {
 
-int64_t msgl_mix_delta_rule_blocks_floats(int64_t total_q, int batch, int H, int d, int dv) {
-  if ((d != 64 && d != 128) || dv < 32 || dv % 32 || total_q < 1 || batch < 1 || H < 1) return 0;
-  return (total_q / kBT + batch) * H * (int64_t)BlockPart{d, dv}.size();
+int msgl_mix_delta_rule_block_floats(int d, int dv) {
+  if ((d != 64 && d != 128) || dv < 32 || dv % 32) return 0;
+  return (int)BlockPart{d, dv}.size();
 }
 
 int msgl_mix_delta_rule_blocks(float* out, const float* qkv, float* state, const void* b_raw, int64_t ld_b, const void* a_raw, int64_t ld_a,

@@ -437,7 +437,7 @@ def delta_rule(out: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, b_raw:
     # against 89 / 93 / 98 / 237.  With many requests a block per request is work of its own, unless one of them may be long.
     many = batch * H > 256
     blocks = T >= 12 * batch or T - batch >= 256 if many else T >= 6 * batch
-    floats = mix_lib().msgl_mix_delta_rule_blocks_floats(T, batch, H, d, dv) if blocks else 0
+    floats = mix_lib().msgl_mix_delta_rule_block_floats(d, dv) * (T // 16 + batch) * H if blocks else 0
     if floats:
         scratch = torch.empty(floats, dtype=torch.float32, device=out.device)
         check_mix(mix_lib().msgl_mix_delta_rule_blocks(

@@ -335,7 +335,7 @@ def test_delta_rule_blocks(dev, H, G, d, dv, per_channel, dtype):
     cu = [0]
     for x in new:
         cu.append(cu[-1] + x)
-    assert mixops.mix_lib().msgl_mix_delta_rule_blocks_floats(T, B, H, d, dv) > 0
+    assert mixops.mix_lib().msgl_mix_delta_rule_block_floats(d, dv) > 0
     mixops.delta_rule(out, torch.cat([q.reshape(T, -1), k.reshape(T, -1), v.reshape(T, -1)], 1).float().to(dev), got_state, b_raw.to(dtype).to(dev), a_raw.to(dtype).to(dev),
                       per_channel, rate.float().to(dev), dt.float().to(dev), i32(cu), i32([x + y for x, y in zip(new, old)]), i32(range(1, B + 1)), B, G)
     out, got_state = out.double().cpu().view(T, H, dv), got_state.double().cpu()
