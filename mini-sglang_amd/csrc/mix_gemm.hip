@@ -28,7 +28,7 @@ __device__ __forceinline__ int count_tiles(const int* __restrict__ seg, int grou
 // fifths of what a large library product draws) and tiles that the last round of CUs and the segments' ends leave empty; for short ones the
 // way of B from memory.  k steps of 64 are whole cache lines of both operands: with steps of 32 and twice the stages the same tiles are
 // a quarter slower.
-//   64 experts x 768 rows, N 1024, K 2048: 539 -> 265 us (777 TFLOP/s); 64 x 3 rows: 123 -> 100 us (268 MB of weights)
+//   64 experts x 768 rows, N 1024, K 2048: 539 -> 265 us (777 TFLOP/s); 64 x 3 rows: 123 -> 96 us (268 MB of weights)
 //   MT x NT = 256 x 256, 8 waves of 64 x 128   long segments
 //             128 x 128, 4 waves of 64 x 64    middling ones: two workgroups a CU
 //              64 x 128, 4 waves of 64 x 32    short ones: the ring holds 2 x 2 x 16 KB of B per CU under way
@@ -91,9 +91,6 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_nt_dma_kernel(TC* __restrict__
     for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const bool live = m0 + wm < rows;  // this wave has rows
   const int n_steps = K / KS;
-#pragma unroll
-  for (int i = 0; i < ST - 1; ++i)
-    if (i < n_steps) dma(i);
   int a_off[KS / 32], b_off[KS / 32];  // for each block of 32 of the step
 #pragma unroll
   for (int kb = 0; kb < KS / 32; ++kb) {
@@ -102,28 +99,74 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_nt_dma_kernel(TC* __restrict__
     b_off[kb] = (MT + wn + bn) * ROW + ((4 * kb + lg) ^ b_key(bn)) * 16;
   }
   int at = 0;
-  for (int step = 0; step < n_steps; ++step) {
-    // this wave's pieces of the step have come when only those of the later ones are under way (memory counters retire in order)
-    if (step + ST - 2 < n_steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 2) * U) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();  // everybody's; everybody done with the stage before
-    if (step + ST - 1 < n_steps) dma(at == 0 ? ST - 1 : at - 1);
-    if (live) {
+  if constexpr (MT == 64 && KS == 64) {
+    // Short segments, few products: the fragments' reads are what is left to hide.  A step's two blocks of 32 take turns, each block's fragments
+    // are read before the other one's products, and the barrier lies between them: by then the step has been read by everybody, its stage takes
+    // a later one.  (64 x 3 rows, N 1024, K 2048: 100 -> 96 us, 16 x 62, N 1536, K 1024: 24.8 -> 22.8; larger tiles are 1 - 3 % slower this way.)
+    bf16x8_t fa[2][TI], fb[2][TJ];
+    auto read = [&](int kb) __attribute__((always_inline)) {
       const char* buf = ring + at * STAGE;
 #pragma unroll
-      for (int kb = 0; kb < KS / 32; ++kb) {
-        bf16x8_t fa[TI], fb[TJ];
+      for (int i = 0; i < TI; ++i) fa[kb][i] = *reinterpret_cast<const bf16x8_t*>(buf + a_off[kb] + i * 16 * ROW);
 #pragma unroll
-        for (int i = 0; i < TI; ++i) fa[i] = *reinterpret_cast<const bf16x8_t*>(buf + a_off[kb] + i * 16 * ROW);
+      for (int j = 0; j < TJ; ++j) fb[kb][j] = *reinterpret_cast<const bf16x8_t*>(buf + b_off[kb] + (j >> 1) * 32 * ROW + (j & 1) * 4 * ROW);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](int kb) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) fb[j] = *reinterpret_cast<const bf16x8_t*>(buf + b_off[kb] + (j >> 1) * 32 * ROW + (j & 1) * 4 * ROW);
+      for (int j = 0; j < TJ; ++j)
 #pragma unroll
-        for (int j = 0; j < TJ; ++j)
+        for (int i = 0; i < TI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kb][j], fa[kb][i], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
 #pragma unroll
-          for (int i = 0; i < TI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
-      }
+    for (int i = 0; i < ST; ++i)
+      if (i < n_steps) dma(i);
+    if (n_steps >= ST) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 1) * U) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    read(0);
+#pragma unroll 1
+    for (int step = 0; step < n_steps; ++step) {
+      asm volatile("" : "+s"(step));       // or the compiler makes copies of the loop for its last steps
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): block 0's fragments, before block 1's are asked for
+      read(1);
+      multiply(0);
+      if (step + ST <= n_steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 2) * U) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (step + ST < n_steps) dma(at);
+      at = at == ST - 1 ? 0 : at + 1;
+      read(0);  // past the last step: some stage, not used
+      multiply(1);
     }
-    at = at == ST - 1 ? 0 : at + 1;
+  } else {
+#pragma unroll
+    for (int i = 0; i < ST - 1; ++i)
+      if (i < n_steps) dma(i);
+    for (int step = 0; step < n_steps; ++step) {
+      // this wave's pieces of the step have come when only those of the later ones are under way (memory counters retire in order)
+      if (step + ST - 2 < n_steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 2) * U) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();  // everybody's; everybody done with the stage before
+      if (step + ST - 1 < n_steps) dma(at == 0 ? ST - 1 : at - 1);
+      if (live) {
+        const char* buf = ring + at * STAGE;
+#pragma unroll
+        for (int kb = 0; kb < KS / 32; ++kb) {
+          bf16x8_t fa[TI], fb[TJ];
+#pragma unroll
+          for (int i = 0; i < TI; ++i) fa[i] = *reinterpret_cast<const bf16x8_t*>(buf + a_off[kb] + i * 16 * ROW);
+#pragma unroll
+          for (int j = 0; j < TJ; ++j) fb[j] = *reinterpret_cast<const bf16x8_t*>(buf + b_off[kb] + (j >> 1) * 32 * ROW + (j & 1) * 4 * ROW);
+#pragma unroll
+          for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int i = 0; i < TI; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+        }
+      }
+      at = at == ST - 1 ? 0 : at + 1;
+    }
   }
   // lane holds C[m = tile row lr][n = 32 pair + 8 lg .. + 7]
   int at_row[TI];
@@ -182,7 +225,7 @@ extern "C" __attribute__((visibility("hidden"))) int mix_gemm_nt_dma(void* C, co
   }
   // Rows per group on average, and how many of the largest tiles there are.  Groups x rows, N, K (us, weights not in cache):
   //                              64 x 128   128 x 128   256 x 256
-  //   16 x 62, 1536, 1024           24.6       26.8        34.8
+  //   16 x 62, 1536, 1024           22.8       26.8        34.8
   //   64 x 64, 1024, 2048            114        105         106
   //   16 x 188, 1536, 1024          37.9       30.9        39.9    96 large tiles: most CUs without one
   //   32 x 188, 1024, 1024          45.2       38.5        43.7
