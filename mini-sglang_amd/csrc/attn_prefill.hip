@@ -148,18 +148,19 @@ __device__ __forceinline__ uint2 tr_read_b64(const char* lds_ptr) {
   return __builtin_bit_cast(uint2, r);
 }
 
-// Two weights as a packed pair, added to the row's sum: in bf16 the rounded ones in one instruction, so that the weights that P.V uses add up
-// to one; in fp16 the fp32 ones (small weights are subnormal there, which the dot product may drop).
-template <typename T>
-__device__ __forceinline__ uint32_t weight_pair(float e0, float e1, float* sum) {
-  const uint32_t p = Elem<T>::pack(e0, e1);
-  if constexpr (std::is_same_v<T, BF16>) {
-    typedef __bf16 v2 __attribute__((ext_vector_type(2)));
-    *sum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2, p), __builtin_bit_cast(v2, 0x3f803f80u), *sum, false);
-  } else {
-    *sum += e0 + e1;
-  }
-  return p;
+// This lane's number and lane ^ 32's, without LDS: a swap of halves between two copies leaves both numbers in every lane.
+__device__ __forceinline__ float2 both_halves(float x) {
+  const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  const uint32_t y0 = y[0], y1 = y[1];  // (a bit cast of the vector's element itself takes element 0 both times)
+  return float2{__uint_as_float(y0), __uint_as_float(y1)};
+}
+__device__ __forceinline__ float pair_max(float x) {
+  const float2 y = both_halves(x);
+  return fmaxf(y.x, y.y);
+}
+__device__ __forceinline__ float pair_sum(float x) {
+  const float2 y = both_halves(x);
+  return y.x + y.y;
 }
 
 constexpr int kTileBytes = kKTile * kD * 2;  // 16 KB: one K (or V) tile image
@@ -300,7 +301,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
       l_run += s[0][0] + s[1][15];
     } else {
       float tmax = kNegBigP;
-      float m_new, alpha;
+      float m_new, alpha, rsum = 0.f;
       const bool need_mask = key0 + kKTile - 1 > wave_min_qpos;
       if constexpr (!kFold) {
   #pragma unroll
@@ -325,6 +326,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
           for (int r = 0; r < 16; ++r) {
             const float e = __builtin_amdgcn_exp2f(s[kb][r] - m_new);
             s[kb][r] = e;
+            rsum += e;
           }
         }
       } else {
@@ -350,20 +352,18 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
           for (int r = 0; r < 16; ++r) {
             const float e = __builtin_amdgcn_exp2f(fmaf(s[kb][r], p.scale_log2, -m_new));
             s[kb][r] = e;
+            rsum += e;
           }
         }
       }
+      rsum += __shfl_xor(rsum, 32, 64);
+      l_run = fmaf(l_run, alpha, rsum);
       if (!__all(m_new == m_run)) {  // alpha == 1 on every row otherwise: the rescale would be the identity
-        l_run *= alpha;
   #pragma unroll
         for (int nb = 0; nb < 4; ++nb)
   #pragma unroll
           for (int r = 0; r < 16; ++r) o[nb][r] *= alpha;
       }
-  #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-  #pragma unroll
-        for (int r = 0; r < 16; r += 2) (void)weight_pair<T>(s[kb][r], s[kb][r + 1], &l_run);
       m_run = m_new;
     }
 
@@ -398,7 +398,6 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
   }
 
   // ---- epilogue: O[q row][d] = O^T / l ---------------------------------------------------------
-  l_run += __shfl_xor(l_run, 32, 64);  // the lanes' shares of the row's sum
   if (q_valid) {
     const float inv = 1.0f / l_run;
     uint16_t* op = p.out + (int64_t)(q_begin + my_q) * p.out_stride + (int64_t)hq * kD;
@@ -428,21 +427,16 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 //     everyone has just finished reading, compute tile t;
 //   * LDS reads issued >= 4 MFMAs ahead of their use (pinned with sched_barrier); beside a DMA under way the compiler waits for ALL of a
 //     wave's reads at the first use of any, so the V^T fragments are asked for after the second key block's have come;
-//   * nothing of the softmax crosses LDS: the halves' maximum by a lane swap, the row's sum stays the lane's own until the end.
+//   * nothing of the softmax crosses LDS: the halves' maximum and their shares of a tile's sum by lane swaps.
 // What bounds it: a wave's tile is 1024 cycles of the matrix cores and about as many of the vector units (32 scores a lane, the exponential
-// 16 cycles each), and two waves per SIMD overlap them only in part.  40 heads on 8, 29 requests of 100 - 1024 tokens: 239 -> 235 us with the
-// last two points; 64 heads, 8192 tokens after 16384: 5380 -> 5340 (1010 TFLOP/s).
+// 16 cycles each), and two waves per SIMD overlap them only in part.  40 heads on 8, 29 requests of 100 - 1024 tokens: 245 -> 244 us with the
+// last two points; 64 heads, 8192 tokens after 16384: 5570 -> 5490 (1000 TFLOP/s), the same bits.  (Sums of the rounded weights, one instruction
+// a pair: 242 and 5510 us, and 2^-9 of a row's weight off.)
 // ABL (diagnosis, wrong results): 1 = tiles DMA'd once, 2 = no QK^T, 4 = no softmax, 8 = no PV.
 // ------------------------------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) const void glb_void_t;
 
-// the larger of this lane's number and lane ^ 32's, without LDS: a swap of halves between two copies leaves both numbers in every lane
-__device__ __forceinline__ float pair_max(float x) {
-  const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  const uint32_t y0 = y[0], y1 = y[1];
-  return fmaxf(__uint_as_float(y0), __uint_as_float(y1));
-}
 template <typename T, int ABL = 0>
 __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillParams p, int total_tiles) {
   // two distinct LDS objects, not one array: the compiler then knows a tile's fragment reads cannot alias the DMA writes
@@ -621,22 +615,29 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
 #pragma unroll
         for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[kb][r]);
       tmax = pair_max(tmax) * p.scale_log2;
+      float alpha = 1.f;
       if (!__all(tmax <= m_run)) {
         const float m_new = fmaxf(m_run, tmax);
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        l_run *= alpha;
+        alpha = __builtin_amdgcn_exp2f(m_run - m_new);
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) o[nb][r] *= alpha;
         m_run = m_new;
       }
+      // the row's sum is of the fp32 weights, tile by tile: its order is part of the result (the other instances' bits)
+      float rsum = 0.f;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int r = 0; r < 16; r += 2)
-          pw[kb][r >> 1] = weight_pair<T>(__builtin_amdgcn_exp2f(fmaf(s[kb][r], p.scale_log2, -m_run)),
-                                          __builtin_amdgcn_exp2f(fmaf(s[kb][r + 1], p.scale_log2, -m_run)), &l_run);
+        for (int r = 0; r < 16; r += 2) {
+          const float e0 = __builtin_amdgcn_exp2f(fmaf(s[kb][r], p.scale_log2, -m_run));
+          const float e1 = __builtin_amdgcn_exp2f(fmaf(s[kb][r + 1], p.scale_log2, -m_run));
+          rsum += e0;
+          rsum += e1;
+          pw[kb][r >> 1] = Elem<T>::pack(e0, e1);
+        }
+      l_run = fmaf(l_run, alpha, pair_sum(rsum));
     }
     // ---- O^T += V^T . P^T: keys 0..31 on the fragments read during QK^T, the fragments of keys 32..63 read under them
     if constexpr (!(ABL & 8)) {
@@ -681,7 +682,6 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
     if (kt + 1 < ntiles) tile_body(std::integral_constant<int, 1>{}, kt + 1);
   }
 
-  l_run += __shfl_xor(l_run, 32, 64);  // the lanes' shares of the row's sum
   if (q_valid) {
     const float inv = 1.0f / l_run;
     uint16_t* op = p.out + (int64_t)(q_begin + my_q) * p.out_stride + (int64_t)hq * kD;

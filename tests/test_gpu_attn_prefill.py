@@ -197,3 +197,26 @@ def test_prefill_matches_decode_on_last_token(ops, dev):
                 qkv=c["qkv"][last].contiguous(), hq=hq, hkv=8, D=D)
     dec, _ = td.run_decode(ops, dev, case)
     torch.testing.assert_close(out[last].float(), dec.float(), atol=8e-3, rtol=2 ** -6)
+
+
+def test_prefill_row_sum_of_unrounded_weights(ops, dev, impl):
+    """A row's sum takes the fp32 weights, the products the bf16 ones: all weights but one are 0.25062, which bf16 makes 0.25.  Over values in
+    [1, 2) the results' own rounding (2^-9 of them, at random) averages out over 4096 of them to 2e-5; a sum of the rounded weights would
+    be 2.4e-3 off in all of them."""
+    g = torch.Generator().manual_seed(15)
+    c = build(g, [(256, 257)] * 4, 8, 8, 16)
+    D, hq = 128, 8
+    c["qkv"][:] = 0
+    c["qkv"][:, : hq * D].view(4, hq, D)[..., :2] = 1.0
+    c["v"][:] = (1.0 + torch.rand(c["v"].shape, generator=g)).to(torch.bfloat16)
+    c["k"][:] = 0
+    c["k"][..., 0], c["k"][..., 1] = -15.625, -0.03125
+    for row in c["rows"]:
+        c["k"][c["table"][row, 0].long()] = 0
+    out = run(ops, dev, c, impl).double()
+    w = math.exp(-15.65625 * D ** -0.5)
+    assert float(torch.tensor(w).bfloat16()) == 0.25
+    for b, row in enumerate(c["rows"]):
+        v = c["v"][c["table"][row, :257].long()].double()
+        ref = (v[0] + 0.25 * v[1:].sum(0)) / (1.0 + 256 * w)
+        assert abs(float(((out[b] - ref) / ref).mean())) < 3e-4
