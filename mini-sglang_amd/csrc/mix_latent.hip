@@ -7,8 +7,9 @@
 //
 // Both: S^T = K Q^T and O^T += V^T P^T, so that a lane ends the first product with scores of ONE query row and starts the second with
 // them; the rows come to LDS by DMA (no staging registers), 16 bytes of padding per row carried along as one more piece, so that 8 rows'
-// 16-byte reads and 4 rows' transposing reads both touch all banks once.  The reference maximum follows every new maximum: the largest
-// weight then is 1, exact in bf16 (letting it lag by up to 2^8 saves 2 % of the time and adds a tenth to the error).
+// 16-byte reads and 4 rows' transposing reads both touch all banks once.  A row's sum is of the fp32 weights.  The reference maximum
+// follows every new maximum: the largest weight then is 1, exact in bf16 (letting it lag by up to 2^8 saves 2 % of the time and adds a
+// tenth to the error).
 #include <algorithm>
 
 #include "mix_common.h"
@@ -55,7 +56,7 @@ struct LatentRow {
 // w + 4, and they take turns: while waves 0 - 3 turn tile t's scores into weights, waves 4 - 7 run the products of tile t - 1's values and
 // tile t's scores; after a barrier the roles change.  So the matrix cores have work in both halves, and each half's barrier serves the
 // meeting of the scores, the images' arrival and their release.
-// 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1546 -> 412 us (704 TFLOP/s), of it 115 us that the queries' and outputs' 563 MB
+// 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1535 -> 414 us (714 TFLOP/s), of it 115 us that the queries' and outputs' 563 MB
 // take to come and go at 4.9 TB/s, hardly overlapped: a workgroup fills its CU and starts and ends with them.
 template <int DK, int DV>
 __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
                                                                const float* __restrict__ sink) {
   constexpr int NKS = DK / 32, NVT = DV / 64;  // this wave's halves: 16-wide steps of the first product, 32-column tiles of the second
   constexpr int ROW = LatentRow<DK>::bytes, PCS = LatentRow<DK>::pieces, KT = 32;
-  constexpr int AHEAD = 2, VAHEAD = 3;  // fragments are read so many products before their use
+  constexpr int AHEAD = 1, VAHEAD = 3;  // fragments are read so many products before their use (2 in the first: a Q fragment spills, 423 us for 414)
   constexpr int NI = (KT * PCS + 63) / 64, IMAGE = NI * 1024, NDMA = (NI + 7) / 8;  // DMA instructions of a tile; of a wave at most
   // three objects: the compiler then knows that a tile's reads do not meet a later tile's DMA
   __shared__ __attribute__((aligned(1024))) char img0[IMAGE], img1[IMAGE], img2[IMAGE];
@@ -198,11 +199,14 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
       m = m_new;
     }
     const float ref = m == -INFINITY ? 0.f : m;  // no key yet: every weight is exp2(-inf) = 0
+    float sum = 0.f;  // of the fp32 weights
 #pragma unroll
     for (int e = 0; e < 16; e += 2) {
-      pw[e >> 1] = pack_bf16(weight(s[e], sharp, ref), weight(s[e + 1], sharp, ref));
-      lsum = add_pair(pw[e >> 1], lsum);
+      const float w0 = weight(s[e], sharp, ref), w1 = weight(s[e + 1], sharp, ref);
+      sum += w0 + w1;
+      pw[e >> 1] = pack_bf16(w0, w1);
     }
+    lsum += sum;
   };
   auto values = [&](const char* buf) __attribute__((always_inline)) {  // O^T += V^T P^T, 16 keys a step: a lane's eight of them are what its registers 8 step ... hold
     bf16x8_t vf[VAHEAD + 1];
@@ -433,9 +437,11 @@ __global__ __launch_bounds__(256, 1) void latent_decode_kernel(float* __restrict
       m = m_new;
     }
     const float ref = m == -INFINITY ? 0.f : m;
-    const uint32_t p01 = pack_bf16(weight(s[0], sharp, ref), weight(s[1], sharp, ref));
-    const uint32_t p23 = pack_bf16(weight(s[2], sharp, ref), weight(s[3], sharp, ref));
-    lsum = add_pair(p23, add_pair(p01, lsum));
+    float w[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) w[c] = weight(s[c], sharp, ref);
+    lsum += (w[0] + w[1]) + (w[2] + w[3]);
+    const uint32_t p01 = pack_bf16(w[0], w[1]), p23 = pack_bf16(w[2], w[3]);
     const s16x4_t pf = __builtin_bit_cast(s16x4_t, uint2{p01, p23});
     const char* vb = buf + (4 * lg + (lr >> 2)) * ROW + 8 * (lr & 3);
 #pragma unroll

@@ -364,6 +364,39 @@ def test_latent_attention_usual_widths(dev, H, R, splits, sink):
         assert float((got - ref).abs().max()) < 5e-2 * float(ref.abs().max()), new
 
 
+@pytest.mark.parametrize("splits", [1, 2], ids=["one-range", "two-ranges"])
+@pytest.mark.parametrize("new", [1, 20], ids=["decode", "portion"])
+@pytest.mark.parametrize("R", [512, 256])
+def test_latent_attention_row_sum_of_unrounded_weights(dev, R, new, splits):
+    """The denominator takes the fp32 weights, the products the bf16 ones: every 16th key weighs 1, the others 0.25087, which bf16 makes
+    0.25.  A sum of the rounded weights would be 3e-3 off; fp32 sums of 400 terms and the hardware's exponential are below 2e-5."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(R + new)
+    H, r, old, w = 16, 64, 400, math.exp(-1.3828125)
+    assert float(torch.tensor(w).bfloat16()) == 0.25
+    n = old + new
+    cache = torch.zeros((512, R + r))
+    cache[:, :R] = 1.0 + torch.rand((512, R), generator=g)
+    cache = cache.bfloat16()
+    q = torch.zeros((new, H, R + r))
+    q[..., R: R + 2] = 1.0
+    mine = torch.randperm(512, generator=g)[:n]
+    quiet = torch.arange(n) % 16 != 0
+    cache[mine[quiet], R], cache[mine[quiet], R + 1] = -1.375, -0.0078125
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    out = torch.empty((new, H, R), device=dev)
+    table = torch.zeros((1, 1024), dtype=torch.int32, device=dev)
+    table[0, :n] = mine.int().to(dev)
+    mixops.latent_attn(out, q.to(dev), cache.to(dev), table, i32([0]), i32([n]), i32([0, new]), 1, R, 1.0, splits=splits)
+    v, got = cache[mine, :R].double(), out.double().cpu()
+    for t in range(new):
+        k = old + t + 1
+        part = torch.where(quiet[:k], 0.25, 1.0).double()
+        ref = (part[:, None] * v[:k]).sum(0) / (quiet[:k].sum() * w + (~quiet[:k]).sum())
+        assert float(((got[t] - ref) / ref).abs().max()) < 2e-5, t
+
+
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
 @pytest.mark.parametrize("N,K", [(256, 32), (128, 64), (264, 96), (520, 256), (72, 128)])
 @pytest.mark.parametrize("lens", [[1, 0, 63, 2, 16], [64, 65, 0, 127, 128, 129, 300], [255, 256, 257] * 30, [0, 0, 700, 17] + [1] * 70], ids=["short", "edges", "long", "many"])
