@@ -210,12 +210,6 @@ __device__ __forceinline__ int find_group_wave(const int* __restrict__ cu_q, int
   return -1;
 }
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-// The two packed bf16 weights added to a sum: the sum of what the products use, so that a row's weights add up to one
-__device__ __forceinline__ float add_pair(uint32_t p, float sum) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, p), __builtin_bit_cast(bf16x2_t, 0x3f803f80u), sum, false);
-}
-
 // A wave's sum / largest number of non-negative integers in every lane's scalar, by row shifts and broadcasts of the vector unit: eight
 // instructions (a shuffle is a trip through LDS, and the bisection below needs dozens of sums before a workgroup can start).
 template <typename F>

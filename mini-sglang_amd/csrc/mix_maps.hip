@@ -181,11 +181,14 @@ __global__ __launch_bounds__(256, 2) void maps_prompt_kernel(bf16_t* __restrict_
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
       const float ref = m[a] == -INFINITY ? 0.f : m[a];  // no key yet: every weight is exp2(-inf) = 0
+      float sum = 0.f;  // of the fp32 weights
 #pragma unroll
       for (int e = 0; e < 16; e += 2) {
-        pw[a][e >> 1] = pack_bf16(__builtin_amdgcn_exp2f(s[a][e] - ref), __builtin_amdgcn_exp2f(s[a][e + 1] - ref));
-        lsum[a] = add_pair(pw[a][e >> 1], lsum[a]);
+        const float w0 = __builtin_amdgcn_exp2f(s[a][e] - ref), w1 = __builtin_amdgcn_exp2f(s[a][e + 1] - ref);
+        sum += w0 + w1;
+        pw[a][e >> 1] = pack_bf16(w0, w1);
       }
+      lsum[a] += sum;
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {

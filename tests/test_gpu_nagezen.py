@@ -11,6 +11,7 @@ their last owner's state.
 from __future__ import annotations
 
 import json
+import math
 
 import pytest
 import torch
@@ -678,3 +679,36 @@ def test_diff_attention_portions_of_usual_width(dev, H, G, window, keep):
             ref = _diff_ref(q, k, v, scale, window, keep, lam, 0.7, eps, gt if gate else torch.full_like(gt, torch.inf))[n - m:]
             assert rel(got[at: at + m], ref) < 1e-2, (splits, gate, n)
             at += m
+
+
+@pytest.mark.parametrize("splits", [1, 2], ids=["one-range", "two-ranges"])
+def test_diff_attention_row_sum_of_unrounded_weights(dev, splits):
+    """Both denominators take the fp32 weights, the products the bf16 ones: in the first map every 16th key weighs 1 and the others 0.2509,
+    which bf16 makes 0.25, in the second all weigh 1.  The maps' difference is small beside either of them (0.04 of 1.5), so a sum of the
+    rounded weights, 3e-3 off, would move it by a tenth; the bf16 result is good to 2^-9."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(5)
+    H, G, d, dv, old, new = 16, 4, 64, 128, 580, 20
+    n = old + new
+    w = 2.0 ** (-(1.375 + 0.0052490234375) * float(torch.tensor(math.log2(math.e)).bfloat16()))  # q = 1 times log2(e) is rounded with the scale
+    assert float(torch.tensor(w).bfloat16()) == 0.25
+    mine = torch.randperm(1024, generator=g)[:n]
+    quiet = torch.arange(n) % 16 != 0
+    kc, vc = torch.zeros((1024, G, 2, d)), (1.0 + torch.rand((1024, G, dv), generator=g)).bfloat16()
+    kc[mine[quiet], :, 0, 0], kc[mine[quiet], :, 0, 1] = -1.375, -0.0052490234375
+    q = torch.zeros((new, H, 2, d))
+    q[..., :2] = 1.0
+    table = torch.zeros((1, 1024), dtype=torch.int32, device=dev)
+    table[0, :n] = mine.int().to(dev)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    out = torch.empty((new, H * dv), dtype=torch.bfloat16, device=dev)
+    mixops.diff_attn(out, q.view(new, -1).to(dev), kc.view(1024, -1).bfloat16().to(dev), vc.view(1024, -1).to(dev), table, i32([0]), i32([n]), i32([0, new]), 1, H, G, d, dv,
+                     1.0, 0, 0, torch.ones(1, device=dev), 1.0, 1e-12, splits=splits)
+    got, v = out.double().cpu().view(new, H, dv), vc[mine].double().repeat_interleave(H // G, dim=1)
+    for t in range(new):
+        k = old + t + 1
+        part = torch.where(quiet[:k], 0.25, 1.0).double()
+        a1 = (part[:, None, None] * v[:k]).sum(0) / (quiet[:k].sum() * w + (~quiet[:k]).sum())
+        ref = O.rms_unit(a1 - v[:k].mean(0), 1e-12)
+        assert rel(got[t], ref) < 1e-2, t
