@@ -897,7 +897,7 @@ int msgl_mix_window_attn(void* out, const void* src, int64_t ld_src, int g_off, 
   float* part_ml = workspace ? workspace + (size_t)splits * total_q * H * dv : nullptr;
   // bf16 caches of 8 or 16 heads up to 128 wide: the matrix cores, down to one new token per request, where 15 of a group's 16 rows are
   // empty (16 heads, 2000 cached keys, this kernel -> that one: 4 requests x 1 token 102 -> 47 us, x 4 240 -> 52, x 32 581 -> 77;
-  // 32 x 1 153 -> 80; 4 requests of 1500 - 2548 new tokens 5198 -> 277).  Other sizes and fp32 stay here.
+  // 32 x 1 153 -> 80; 4 requests of 1500 - 2548 new tokens 5182 -> 294).  Other sizes and fp32 stay here.
   int done = 0;
   if (dtype == MSGL_MIX_BF16) {
     done = mix_window_attn_mfma(out, part_o, part_ml, src, ld_src, g_off, k_cache, v_cache, table, table_stride, req_rows, seq_lens, cu_q, batch,

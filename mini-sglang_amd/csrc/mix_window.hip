@@ -7,12 +7,12 @@
 // as contraction: it goes to the fp32 matrix instructions (on vector FMAs it was 256 of them a pair, and every wave read every head's
 // scores back from LDS).
 //
-// 4 requests of 1500 - 2548 new tokens, 16 heads of 128 over 4 key heads, window 2048: 5198 us on the vector units, 453 us with both
-// products on the matrix cores and the mixing on vector FMAs in step with them, 277 us as below (264 TFLOP/s of useful products; the
-// softmax and the LDS round trip of the scores are what is left).
+// 4 requests of 1500 - 2548 new tokens, 16 heads of 128 over 4 key heads, window 2048: 5182 us on the vector units, 453 us with both
+// products on the matrix cores and the mixing on vector FMAs in step with them, 294 us as below (249 TFLOP/s of useful products; the
+// softmax and the LDS round trip of the scores are what is left, and 20 us are the weights' third part: 273 us with two).
 //
 // Precision: scores are bf16 x bf16 products with fp32 sums, mixed and exponentiated in fp32; a probability enters the second product
-// as the sum of two bf16 numbers (its rounding and what the rounding left, 16 bits in all), so nothing held in 32 bits drops to 16.
+// as the sum of three bf16 numbers (its rounding, that of what is left, and the rest: 8 bits each), which is the fp32 number itself.
 #include "mix_common.h"
 
 namespace {
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) s[hh][ks] = *reinterpret_cast<const f32x4_t*>(mixed + ((h0 + hh) * 16 + lr) * kWinRow + ks * 16 + 4 * lg);
     const bool whole = nj <= k_end && nj - 1 <= all_hi && j0 >= all_lo;
-    uint2 hi[HPW][KS], lo[HPW][KS];
+    uint2 part[3][HPW][KS];  // a weight's three bf16 parts, the largest first
 #pragma unroll
     for (int hh = 0; hh < HPW; ++hh) {
       float tmax = -INFINITY;
@@ -214,9 +214,14 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
           p[c] = __builtin_amdgcn_exp2f(s[hh][ks][c] - base);
           psum += p[c];
         }
-        hi[hh][ks] = uint2{pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3])};
-        lo[hh][ks] = uint2{pack_bf16(p[0] - __uint_as_float(hi[hh][ks].x << 16), p[1] - __uint_as_float(hi[hh][ks].x & 0xffff0000u)),
-                           pack_bf16(p[2] - __uint_as_float(hi[hh][ks].y << 16), p[3] - __uint_as_float(hi[hh][ks].y & 0xffff0000u))};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const uint2 x = part[i][hh][ks] = uint2{pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3])};
+          p[0] -= __uint_as_float(x.x << 16);
+          p[1] -= __uint_as_float(x.x & 0xffff0000u);
+          p[2] -= __uint_as_float(x.y << 16);
+          p[3] -= __uint_as_float(x.y & 0xffff0000u);
+        }
       }
       lsum[hh] = fmaf(lsum[hh], alpha, psum);
       if (__builtin_amdgcn_ballot_w64(m_new > m[hh]) != 0) {
@@ -239,10 +244,11 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
         const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
         for (int hh = 0; hh < HPW; ++hh) {
-          const Q4 ph{hi[hh][2 * kp].x, hi[hh][2 * kp].y, hi[hh][2 * kp + 1].x, hi[hh][2 * kp + 1].y};
-          const Q4 pl{lo[hh][2 * kp].x, lo[hh][2 * kp].y, lo[hh][2 * kp + 1].x, lo[hh][2 * kp + 1].y};
-          o[hh][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, pl), o[hh][vt], 0, 0, 0);
-          o[hh][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, ph), o[hh][vt], 0, 0, 0);
+#pragma unroll
+          for (int i = 2; i >= 0; --i) {
+            const uint2 a = part[i][hh][2 * kp], b = part[i][hh][2 * kp + 1];
+            o[hh][vt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8_t, Q4{a.x, a.y, b.x, b.y}), o[hh][vt], 0, 0, 0);
+          }
         }
       }
     }

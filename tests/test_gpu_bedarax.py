@@ -256,6 +256,41 @@ def test_window_matrix_cores(dev, H, G, d, dv, splits):
         assert bool((diff <= 2.0 ** -8 * ref.abs() + 2.0 ** -14 * ref.abs().max()).all()), (window, float(diff.max()))
 
 
+@pytest.mark.parametrize("splits", [1, 2], ids=["one-range", "two-ranges"])
+@pytest.mark.parametrize("new", [1, 20], ids=["decode", "portion"])
+@pytest.mark.parametrize("H,G", [(16, 4), (8, 1)])
+def test_window_weights_keep_32_bits(dev, H, G, new, splits):
+    """Two keys of weight 1 whose values are the two leading bf16 parts of a third key's weight w, and that key with the value -1: the result
+    is what w has beyond 16 bits.  A weight cut to two bf16 parts gives zero.  Bound: w's last bits, the rounding of its exponent and the
+    exponential, 2^-22 of w where the part looked at is about 2^-18 of it, and the bf16 result."""
+    from mini_sglang_amd import mixops
+
+    def parts(w):
+        h = float(torch.tensor(w).bfloat16())
+        m = float(torch.tensor(w - h, dtype=torch.float64).bfloat16())
+        return h, m, w - h - m
+
+    d = dv = 64
+    at = max((-k / 128 for k in range(64, 256)), key=lambda x: abs(parts(math.exp(x))[2]))
+    w = math.exp(at)
+    h, m, rest = parts(w)
+    assert abs(rest) > 2.0 ** -19 * w
+    n = 3 + new
+    kc, vc = torch.zeros((64, G, d)), torch.zeros((64, G, dv))
+    kc[2, :, 0], kc[3:n, :, 0] = at, -256.0  # the new tokens' own keys weigh nothing
+    vc[0], vc[1], vc[2] = h, m, -1.0
+    src = torch.zeros((new, H * d + H))
+    src[:, : H * d].view(new, H, d)[..., 0] = 1.0
+    src[:, H * d:] = 40.0  # open gates
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    table = torch.arange(64, dtype=torch.int32, device=dev)[None]
+    out = torch.empty((new, H * dv), dtype=torch.bfloat16, device=dev)
+    mixops.window_attn(out, src.bfloat16().to(dev), H * d, kc.view(64, -1).bfloat16().to(dev), vc.view(64, -1).bfloat16().to(dev), table, i32([0]), i32([n]), i32([0, new]), 1,
+                       H, G, d, dv, 0, 1.0, torch.eye(H, device=dev), splits=splits)
+    ref = -rest / (2.0 + w)
+    assert float((out.double().cpu() - ref).abs().max()) < 2.0 ** -22 * w + 2.0 ** -8 * abs(ref)
+
+
 @pytest.mark.parametrize("chunk", [0, 1, 5], ids=["whole", "chunks-of-1", "chunks-of-5"])
 def test_delta_rule_state_slots_and_cuts(dev, chunk):
     """The recurrence kernel alone: two requests in one launch on state rows that hold garbage, then continued in a second
