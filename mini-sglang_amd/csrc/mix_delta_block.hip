@@ -33,7 +33,7 @@ __device__ __forceinline__ float exp_split(float y) {  // e^y: y log2(e) in two 
   const float h = y * 1.4426950408889634f;
   const float l = fmaf(y, 1.4426950408889634f, -h) + y * 1.9259629911e-8f;
   const float e = __builtin_amdgcn_exp2f(h);
-  return fmaf(e, l * 0.6931471805599453f, e);
+  return e > 0.f && e < INFINITY ? fmaf(e, l * 0.6931471805599453f, e) : e;  // past the exponents' range (an infinite gate) l is no number
 }
 __device__ __forceinline__ float decay_of(float r, float z, const float*) { return expf(r * softplusf_(z)); }
 __device__ __forceinline__ float decay_of(float r, float z, const bf16_t*) {

@@ -391,6 +391,60 @@ def test_delta_rule_blocks(dev, H, G, d, dv, per_channel, dtype):
     assert torch.equal(got_state[0], state[0].double())  # nobody's row
 
 
+def _delta_case(dev, dtype, H, G, d, dv, per_channel, new, old, change=None, seed=0):
+    """Runs mixops.delta_rule over requests of `new` tokens after `old` ones and the token loop in float64; `change` edits the inputs (dict of
+    q, k, v, b, a in float64) first -> (outputs per request, states), (the same of the token loop)."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(seed)
+    B, T, n = len(new), sum(new), H * d if per_channel else H
+    rnd = lambda *x: torch.randn(*x, generator=g, dtype=torch.float64)  # noqa: E731
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)  # noqa: E731
+    x = {"q": unit(rnd(T, G, d)) * d ** -0.5, "k": unit(rnd(T, G, d)), "v": rnd(T, H, dv), "b": rnd(T, H), "a": rnd(T, n)}
+    if change:
+        change(x)
+    x = {name: y.to(dtype if name in "ab" else torch.float32) for name, y in x.items()}
+    rate, dt, state = -torch.exp(rnd(H)).float(), (0.5 * rnd(n)).float(), rnd(B + 1, H, d, dv).float()
+    got_state, out = state.to(dev), torch.empty((T, H * dv), dtype=torch.float32, device=dev)
+    i32 = lambda y: torch.tensor(y, dtype=torch.int32, device=dev)  # noqa: E731
+    cu = [0]
+    for m in new:
+        cu.append(cu[-1] + m)
+    mixops.delta_rule(out, torch.cat([x[y].reshape(T, -1) for y in "qkv"], 1).to(dev), got_state, x["b"].to(dev), x["a"].to(dev), per_channel, rate.to(dev), dt.to(dev), i32(cu),
+                      i32([y + z for y, z in zip(new, old)]), i32(range(1, B + 1)), B, G)
+    x = {name: y.double() for name, y in x.items()}
+    decay = torch.exp(rate.double()[:, None] * torch.nn.functional.softplus(x["a"] + dt.double()).view(T, H, -1))
+    refs, states = [], []
+    for b in range(B):
+        S, ref = state[b + 1].double() * (1.0 if old[b] else 0.0), []
+        for t in range(cu[b], cu[b + 1]):
+            kk, qq = x["k"][t].repeat_interleave(H // G, 0), x["q"][t].repeat_interleave(H // G, 0)
+            S = S * decay[t][:, :, None]
+            u = torch.sigmoid(x["b"][t])[:, None] * (x["v"][t] - (S * kk[:, :, None]).sum(1))
+            S = S + kk[:, :, None] * u[:, None, :]
+            ref.append((S * qq[:, :, None]).sum(1))
+        refs.append(torch.stack(ref))
+        states.append(S)
+    got = out.double().cpu().view(T, H, dv)
+    return ([got[cu[b]: cu[b + 1]] for b in range(B)], list(got_state.double().cpu()[1:])), (refs, states)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("per_channel", [False, True], ids=["head", "channel"])
+def test_delta_rule_blocks_infinite_gates(dev, per_channel, dtype):
+    """Gates of +inf (and finite ones past what an exponent holds) forget everything, gates of -inf nothing: the blocks against the token loop."""
+    def change(x):
+        n = x["a"].shape[1]
+        x["a"][5, : n // 2] = torch.inf
+        x["a"][20, n // 2:] = 3.0e38
+        x["a"][9, : n // 2] = -torch.inf
+        x["a"][37] = torch.inf
+
+    (got, state), (ref, states) = _delta_case(dev, dtype, 4, 2, 128, 64, per_channel, [40, 13], [7, 0], change)
+    for b in range(2):
+        assert rel(got[b], ref[b]) < 1e-5 and rel(state[b], states[b]) < 1e-5, b
+
+
 # ----------------------------------------------------------------------------------------- schedules
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, FP32_TOL), (torch.bfloat16, BF16_TOL)], ids=["fp32", "bf16"])
 def test_whole_prompt(dtype, tol):
