@@ -19,6 +19,8 @@
 // 128 registers a token, in three launches.
 // 4 requests of 1500 - 2548 tokens, 16 heads, d = dv = 128, decays per channel: 4038 -> 390 us (blocks 177, walk 240); error against 64
 // bits 1.9e-7 -> 1.4e-7.
+#include <type_traits>
+
 #include "mix_common.h"
 
 namespace {
@@ -315,6 +317,7 @@ __global__ __launch_bounds__(320) void delta_walk_kernel(float* __restrict__ out
     for (int n = 0; n < nblk; ++n, orow += (size_t)kBT * H * dv) {
       __syncthreads();
       const f32x4_t qk = full_qk[n & 1][lane];
+      float zero = 0.f;
 #pragma unroll
       for (int ct = 0; ct < 2; ++ct) {
         const f32x4_t u = full_u[n & 1][ct][lane];
@@ -326,6 +329,24 @@ __global__ __launch_bounds__(320) void delta_walk_kernel(float* __restrict__ out
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           if (n * kBT + 4 * lg + e < n_new) orow[(size_t)e * H * dv + 16 * ct] = o[e];
+        zero = fmaf(o[0], 0.f, zero);
+      }
+      // Q's upper triangle is zeros, so a u that is not finite spoils its column for all tokens of the block, also those before it (zero times
+      // infinity), and one token's number shows it: then the outputs again, each token without the u behind it
+      if (__builtin_amdgcn_ballot_w64(zero != 0.f) != 0) {
+        const float* qs = reinterpret_cast<const float*>(full_qk[n & 1]);
+#pragma unroll 1
+        for (int x = 0; x < 8; ++x) {
+          const int e = x & 3, ct = x >> 2, t = 4 * lg + e;
+          const float* us = reinterpret_cast<const float*>(full_u[n & 1][ct]);
+          float o = 0.f;
+          for (int j = 0; j <= t; ++j) {
+            const int at = (j >> 2) * 64 + (j & 3);  // a lane's four numbers are tokens 4 lg ... of row or column lr
+            o = fmaf(qs[at + t * 4], us[at + lr * 4], o);
+          }
+          for (int w = 0; w < 4; ++w) o += reinterpret_cast<const float*>(share_o[n % 3][w][ct])[lane * 4 + e];
+          if (n * kBT + t < n_new) orow[(size_t)e * H * dv + 16 * ct] = o;
+        }
       }
     }
     return;
@@ -369,7 +390,7 @@ __global__ __launch_bounds__(320) void delta_walk_kernel(float* __restrict__ out
       for (int ct = 0; ct < 2; ++ct) x.u[ct][e] = (at + at_u + e * dv)[16 * ct];
     x.qk = *reinterpret_cast<const f32x4_t*>(at + at_qk);
   };
-  auto block = [&](const Ops& x, int n) {
+  auto block = [&](const Ops& x, int n, auto tail) __attribute__((always_inline)) {
     f32x4_t pu[2], po[2];
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct) pu[ct] = po[ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -397,6 +418,12 @@ __global__ __launch_bounds__(320) void delta_walk_kernel(float* __restrict__ out
 #pragma unroll
       for (int w = 0; w < 4; ++w) u[ct] -= share_u[n & 1][w][ct][lane];
     }
+    if (tail && (n + 1) * kBT > n_new) {  // rows past the portion are zero also where a value before them is infinite
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) u[ct][e] = n * kBT + 4 * lg + e < n_new ? u[ct][e] : 0.f;
+    }
     if (wave == 0) {
       full_u[n & 1][0][lane] = u[0];
       full_u[n & 1][1][lane] = u[1];
@@ -418,16 +445,20 @@ __global__ __launch_bounds__(320) void delta_walk_kernel(float* __restrict__ out
   fetch(x0, 0);
   fetch(x1, 1);
   int n = 0;
-  for (; n + 3 <= nblk; n += 3) {
+  const std::false_type within;
+  for (; n + 3 < nblk; n += 3) {
     fetch(x2, n + 2);
-    block(x0, n);
+    block(x0, n, within);
     fetch(x0, n + 3);
-    block(x1, n + 1);
+    block(x1, n + 1, within);
     fetch(x1, n + 4);
-    block(x2, n + 2);
+    block(x2, n + 2, within);
   }
-  if (n < nblk) block(x0, n);
-  if (n + 1 < nblk) block(x1, n + 1);
+  const std::true_type tail;  // the last one to three blocks: only they look for the portion's end
+  fetch(x2, n + 2);
+  block(x0, n, tail);
+  if (n + 1 < nblk) block(x1, n + 1, tail);
+  if (n + 2 < nblk) block(x2, n + 2, tail);
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NT; ++i)

@@ -445,6 +445,38 @@ def test_delta_rule_blocks_infinite_gates(dev, per_channel, dtype):
         assert rel(got[b], ref[b]) < 1e-5 and rel(state[b], states[b]) < 1e-5, b
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("per_channel", [False, True], ids=["head", "channel"])
+@pytest.mark.parametrize("at", [6, 15, 16, 39])
+def test_delta_rule_blocks_infinite_value(dev, at, per_channel, dtype):
+    """An infinite value leaves the tokens before it and the columns beside it alone, and the state as the token loop leaves it: in the middle
+    of a block, at its ends and as the portion's last token (with rows past the portion behind it)."""
+    def change(x):
+        x["v"][at, 1, 3] = torch.inf
+        x["v"][at, 1, 40] = -torch.inf
+
+    (got, state), (ref, states) = _delta_case(dev, dtype, 2, 1, 128, 64, per_channel, [40], [9], change)
+    assert rel(got[0][:at], ref[0][:at]) < 1e-5
+    hit = torch.zeros(2, 64, dtype=torch.bool)
+    hit[1, 3] = hit[1, 40] = True
+    assert rel(got[0][:, ~hit], ref[0][:, ~hit]) < 1e-5 and rel(state[0].transpose(1, 2)[~hit], states[0].transpose(1, 2)[~hit]) < 1e-5
+    assert not torch.isfinite(got[0][at:, hit]).any()
+    spoilt, want = state[0].transpose(1, 2)[hit], states[0].transpose(1, 2)[hit]
+    assert torch.equal(torch.isnan(spoilt), torch.isnan(want)) and torch.equal(torch.nan_to_num(spoilt), torch.nan_to_num(want))
+
+
+@pytest.mark.parametrize("name", ["q", "k", "b", "a"])
+@pytest.mark.parametrize("per_channel", [False, True], ids=["head", "channel"])
+def test_delta_rule_blocks_nan_token(dev, name, per_channel):
+    """A token whose query, key, strength or gate is no number leaves the tokens before it alone."""
+    def change(x):
+        x[name][21].view(-1)[0] = torch.nan
+
+    (got, state), (ref, states) = _delta_case(dev, torch.bfloat16, 2, 2, 64, 64, per_channel, [40], [9], change)
+    assert rel(got[0][:21], ref[0][:21]) < 1e-5
+    assert torch.equal(torch.isnan(got[0]), torch.isnan(ref[0])) and torch.equal(torch.isnan(state[0]), torch.isnan(states[0]))
+
+
 # ----------------------------------------------------------------------------------------- schedules
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, FP32_TOL), (torch.bfloat16, BF16_TOL)], ids=["fp32", "bf16"])
 def test_whole_prompt(dtype, tol):
