@@ -272,6 +272,11 @@ int msgl_sample_top_k_top_p(int32_t* out, const float* probs, const int32_t* top
 int msgl_sample_filtered_logits(int32_t* out, const void* logits, const float* temperatures, const int32_t* top_k,
                                 const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride, int logits_dtype,
                                 uint64_t seed, uint64_t offset, void* stream);
+/* The same, and a copy of what it drew from for another draw after the caller's buffers have moved on: kept [rows, vocab] in the
+ * logits' type, kept_temperatures [rows]. */
+int msgl_sample_filtered_logits_keep(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
+                                     const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
+                                     int logits_dtype, uint64_t seed, uint64_t offset, void* stream);
 /* Sample one token per row straight from logits: index ~ softmax(logits[r, :] / temperature[r]), no
  * top-k / top-p filter, probabilities never materialised (the fused form of the reference's
  * softmax -> sampling_from_probs pair, P/engine/sample.py:24-44).  Rows 16-byte aligned.

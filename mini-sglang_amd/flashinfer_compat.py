@@ -123,14 +123,16 @@ def gelu_and_mul(input: torch.Tensor, out: Optional[torch.Tensor] = None,
 class _DeferredProbs:
     """What `softmax(logits, T)` hands back: the reference's `sample_impl` (P/engine/sample.py:24-45) passes it
     straight to one of the sampling functions and never looks inside.  Temperature-only batches are then drawn
-    by ONE fused kernel from the logits (no [B, V] fp32 probabilities tensor), and so are the
-    top-k / top-p functions, through the exact values that the probabilities would have.  Anything else that treats the object as a
-    tensor gets the materialised tensor through `__torch_function__`-free explicit conversion (`.probs()`)."""
+    by ONE fused kernel from the logits (no [B, V] fp32 probabilities tensor), and so are the top-k / top-p functions, through the exact
+    values that the probabilities would have.  The first of those leaves a copy of the logits and temperatures it drew from, so that a
+    later draw from the same object, or `.probs()`, does not see what the caller has put into the buffers since.  Anything else that
+    treats the object as a tensor gets the materialised tensor through `__torch_function__`-free explicit conversion (`.probs()`)."""
 
-    __slots__ = ("logits", "temperature", "_probs")
+    __slots__ = ("logits", "temperature", "_probs", "_kept")
 
     def __init__(self, logits: torch.Tensor, temperature: torch.Tensor) -> None:
         self.logits, self.temperature, self._probs = logits, temperature, None
+        self._kept = None  # (logits, temperature) as the first filtered draw found them
 
     @property
     def shape(self):
@@ -146,8 +148,18 @@ class _DeferredProbs:
 
     def probs(self) -> torch.Tensor:
         if self._probs is None:
-            self._probs = ops.softmax_temperature(self.logits, self.temperature)
+            self._probs = ops.softmax_temperature(*(self._kept or (self.logits, self.temperature)))
         return self._probs
+
+    def draw(self, top_k, top_p, seed: int, offset: int) -> torch.Tensor:
+        """The filtered draw straight from the logits (nobody has asked for the probabilities)."""
+        if self._kept is not None:
+            return ops.sample_filtered_logits(*self._kept, top_k, top_p, seed, offset)
+        rows = self.logits.shape[0]
+        kept = torch.empty(self.logits.shape, dtype=self.logits.dtype, device=self.device), torch.empty(rows, dtype=torch.float32, device=self.device)
+        picks = ops.sample_filtered_logits(self.logits, self.temperature, top_k, top_p, seed, offset, keep=kept)
+        self._kept = kept
+        return picks
 
 
 def _as_probs(p) -> torch.Tensor:
@@ -180,9 +192,8 @@ class _SamplingNamespace:
         if isinstance(top_p, float):
             top_p = torch.full((probs.shape[0],), top_p, dtype=torch.float32, device=dev)
         # every TP rank seeds identically (P/engine/engine.py:37) => identical draws on all ranks
-        if isinstance(probs, _DeferredProbs) and probs._probs is None:  # nobody has asked for the probabilities: straight from the logits
-            return ops.sample_filtered_logits(probs.logits, probs.temperature, top_k, top_p, torch.initial_seed(),
-                                              self._next_offset(probs.shape[0]))
+        if isinstance(probs, _DeferredProbs) and probs._probs is None:
+            return probs.draw(top_k, top_p, torch.initial_seed(), self._next_offset(probs.shape[0]))
         probs = _as_probs(probs)
         return ops.sample_top_k_top_p(probs, top_k, top_p, torch.initial_seed(), self._next_offset(probs.shape[0]))
 

@@ -447,8 +447,9 @@ def sample_top_k_top_p(probs: torch.Tensor, top_k: Optional[torch.Tensor], top_p
 
 
 def sample_filtered_logits(logits: torch.Tensor, temperatures: torch.Tensor, top_k: Optional[torch.Tensor], top_p: Optional[torch.Tensor],
-                           seed: int, offset: int) -> torch.Tensor:
-    """sample_top_k_top_p(softmax_temperature(logits, temperatures), ...) in one launch, without the probabilities: the same picks."""
+                           seed: int, offset: int, keep: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> torch.Tensor:
+    """sample_top_k_top_p(softmax_temperature(logits, temperatures), ...) in one launch, without the probabilities: the same picks.
+    keep: contiguous (logits, temperatures) of the same shapes and types that receive a copy of what was drawn from."""
     _need_cuda(logits, temperatures)
     assert logits.dim() == 2 and logits.stride(1) == 1 and temperatures.dtype == torch.float32
     rows = logits.shape[0]
@@ -457,11 +458,15 @@ def sample_filtered_logits(logits: torch.Tensor, temperatures: torch.Tensor, top
         assert top_k.dtype == torch.int32 and top_k.is_cuda and top_k.numel() == rows
     if top_p is not None:
         assert top_p.dtype == torch.float32 and top_p.is_cuda and top_p.numel() == rows
+    if keep is not None:
+        _need_cuda(*keep)
+        assert keep[0].shape == logits.shape and keep[0].dtype == logits.dtype and keep[0].is_contiguous()
+        assert keep[1].shape == (rows,) and keep[1].dtype == torch.float32 and keep[1].is_contiguous()
     check(
-        lib().msgl_sample_filtered_logits(
-            out.data_ptr(), logits.data_ptr(), temperatures.data_ptr(), top_k.data_ptr() if top_k is not None else None,
-            top_p.data_ptr() if top_p is not None else None, rows, logits.shape[1], logits.stride(0), _logits_dt(logits),
-            seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF, _stream(),
+        lib().msgl_sample_filtered_logits_keep(
+            out.data_ptr(), None if keep is None else keep[0].data_ptr(), None if keep is None else keep[1].data_ptr(), logits.data_ptr(),
+            temperatures.data_ptr(), top_k.data_ptr() if top_k is not None else None, top_p.data_ptr() if top_p is not None else None, rows,
+            logits.shape[1], logits.stride(0), _logits_dt(logits), seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF, _stream(),
         ),
         "sample_filtered_logits",
     )

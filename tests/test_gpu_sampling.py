@@ -274,3 +274,28 @@ def test_filtered_draw_is_the_integer_rule(ops, dev, dtype, vocab):
         want = [_filtered_pick(host[r], rows[r][0], rows[r][1], 77, off + r) for r in range(len(rows))]
         assert ops.sample_top_k_top_p(probs, k, p, 77, off).cpu().tolist() == want
         assert ops.sample_filtered_logits(logits, t, k, p, 77, off).cpu().tolist() == want
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+def test_a_second_draw_takes_what_the_first_one_took(ops, dev, dtype):
+    """Several draws from one softmax() result while the logits and temperatures buffers go on to the next step: all from the first step's
+    probabilities, and so is .probs()."""
+    from mini_sglang_amd import flashinfer_compat as fi
+
+    g = torch.Generator().manual_seed(9)
+    step = [(torch.randn((5, 33333), generator=g) * 2.5).to(dtype).to(dev) for _ in range(2)]
+    buf = torch.empty((5, 33400), dtype=dtype, device=dev)[:, :33333]  # rows with a stride, as of a padded buffer
+    temp = [torch.full((5,), x, device=dev) for x in (0.7, 0.3)]
+    k, p = torch.full((5,), 40, dtype=torch.int32, device=dev), torch.full((5,), 0.9, device=dev)
+    t = temp[0].clone()
+    buf.copy_(step[0])
+    draw = type(fi.sampling)()
+    probs = draw.softmax(buf, t)
+    got = [draw.top_k_top_p_sampling_from_probs(probs, k, p)]
+    buf.copy_(step[1])
+    t.copy_(temp[1])
+    got += [draw.top_k_sampling_from_probs(probs, k), draw.top_p_sampling_from_probs(probs, p)]
+    stored = ops.softmax_temperature(step[0], temp[0])
+    want = [ops.sample_top_k_top_p(stored, a, b, torch.initial_seed(), 5 * i) for i, (a, b) in enumerate(((k, p), (k, None), (None, p)))]
+    assert torch.stack(got).tolist() == torch.stack(want).tolist()
+    assert torch.equal(probs.probs(), stored)
