@@ -388,7 +388,7 @@ def window_attn(out: torch.Tensor, src: torch.Tensor, g_off: int, k_cache: torch
         # a few short portions are some tens of 16-token groups for 256 compute units: cut their keys as well (32 portions of 8 - 32
         # tokens over 2000 keys, 16 heads: 226 -> 72 us); from static sizes only, so a captured graph keeps its grid
         groups, keys = T // 16 + batch, min(window, table.shape[1]) if window > 0 else table.shape[1]
-        if groups <= 128:
+        if 0 < groups <= 128:
             splits = max(1, min(256 // groups, keys // 256, 8))
     ws = None
     if splits > 1:
