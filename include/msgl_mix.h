@@ -137,6 +137,8 @@ int msgl_mix_kv_store(void* k_cache, void* v_cache, const int* out_loc, const vo
  * `splits` > 1 cuts every token's visible keys into that many ranges whose partial results (workspace: fp32,
  * msgl_mix_window_attn_workspace_floats) a second launch merges -- for steps with few query tokens. */
 int msgl_mix_window_attn_workspace_floats(int total_q, int H, int dv, int splits);
+/* 1 where these sizes have the matrix-core form (16 query tokens per workgroup), 0 where they have the plain one. */
+int msgl_mix_window_attn_on_matrix_cores(int H, int G, int d, int dv, int dtype);
 int msgl_mix_window_attn(void* out, const void* src, int64_t ld_src, int g_off, const void* k_cache, const void* v_cache, const int* table,
                          int64_t table_stride, const int* req_rows, const int* seq_lens, const int* cu_q, int batch, int total_q, int H,
                          int G, int d, int dv, int window, float scale, const float* talk, int dtype, int splits, float* workspace,

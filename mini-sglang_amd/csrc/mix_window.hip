@@ -293,14 +293,19 @@ size_t window_lds(int G) {
 
 }  // namespace
 
+// heads of 8 | 16 so that a wave's heads share a value head; rows that 16-byte loads and 8-byte stores may walk
+extern "C" int msgl_mix_window_attn_on_matrix_cores(int H, int G, int d, int dv, int dtype) {
+  return dtype == MSGL_MIX_BF16 && (H == 8 || H == 16) && G >= 1 && G <= H / 4 && (H / 2) % G == 0 && d >= 1 && d <= 128 && dv >= 1 && dv <= 128 &&
+         d % 8 == 0 && dv % 8 == 0;
+}
+
 // 1: launched; 0: these sizes are not this kernel's (the caller takes the other one); < 0: an error code.
 extern "C" __attribute__((visibility("hidden"))) int mix_window_attn_mfma(
     void* out, float* part_o, float* part_ml, const void* src, int64_t ld_src, int g_off, const void* k_cache, const void* v_cache, const int* table,
     int64_t table_stride, const int* req_rows, const int* seq_lens, const int* cu_q, int batch, int total_q, int H, int G, int d, int dv, int window,
     float scale, const float* talk, int splits, hipStream_t s) {
   const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  // heads of 8 | 16 so that a wave's heads share a value head; rows that 16-byte loads and 8-byte stores may walk
-  if (!(H == 8 || H == 16) || G > H / 4 || (H / 2) % G || d > 128 || dv > 128 || d % 8 || dv % 8) return 0;
+  if (!msgl_mix_window_attn_on_matrix_cores(H, G, d, dv, MSGL_MIX_BF16)) return 0;
   if (!al(k_cache) || !al(v_cache) || !al(out) || (part_o && !al(part_o))) return 0;
   const int qvec = al(src) && ld_src % 8 == 0;
   const dim3 grid(total_q / 16 + batch, splits);

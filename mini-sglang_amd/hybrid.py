@@ -1170,7 +1170,7 @@ class HybridDecoder:
         # few query rows per request (decode, short portions): cut the keys into ranges so that the launch fills the chip
         splits = mixops.latent_attn_splits(md.batch, T, H, md.max_seqlen_k) if md.max_seqlen_q <= 16 else 1
         mixops.latent_attn(o_lat, q_abs, rows, ctx.page_table, md.req_rows, md.seq_lens, md.cu_seqlens_q, md.batch, R, s.scale,
-                           splits=splits, sink=L.sink)
+                           splits=splits, sink=L.sink, max_keys=md.max_seqlen_k)
         # with an output gate the heads' values stay fp32 until the gate has multiplied them: one rounding on the way into W_o
         o = torch.empty((T, H * dv), dtype=torch.float32 if s.out_gate else self.dtype, device=h.device)
         mixops.gemm_nt(o, o_lat, L.uv, T, dv, R, lda=H * R, ldb=R, ldc=H * dv, groups=H, a_gs=R, b_gs=dv * R, c_gs=dv)
@@ -1312,7 +1312,7 @@ class HybridDecoder:
         gate = proj[:, L.w_in.shape[0] - H * dv:] if s.out_gate else None
         splits = mixops.sink_attn_splits(md.batch, T, H, G, s.window, md.max_seqlen_k, s.keep_first) if md.max_seqlen_q <= 16 else 1
         mixops.diff_attn(o, q, kc, vc, ctx.page_table, md.req_rows, md.seq_lens, md.cu_seqlens_q, md.batch, H, G, d, dv, s.scale, s.window,
-                         s.keep_first, L.lam_now, 1.0 - s.diff, eps, gate=gate, splits=splits)
+                         s.keep_first, L.lam_now, 1.0 - s.diff, eps, gate=gate, splits=splits, max_keys=md.max_seqlen_k)
         return mixops.linear(o, L.o)
 
     def _gated_ff_act(self, h: torch.Tensor, up: torch.Tensor, down: torch.Tensor, act: int) -> torch.Tensor:
@@ -1457,7 +1457,8 @@ class HybridDecoder:
             shared["v_first"] = proj[:, v_off: v_off + G * dv]
         o = torch.empty((T, H * dv), dtype=self.dtype, device=h.device)
         mixops.window_attn(o, proj, g_off, kc, vc, ctx.page_table, md.req_rows, md.seq_lens, md.cu_seqlens_q, md.batch, H, G, d, dv,
-                           s.window, s.scale, L.talk, splits=mixops.window_attn_splits(md.batch, T, s.window, md.max_seqlen_k))
+                           s.window, s.scale, L.talk, splits=mixops.window_attn_splits(md.batch, T, s.window, md.max_seqlen_k),
+                           max_keys=md.max_seqlen_k)
         return mixops.linear(o, L.o)
 
     def _delta(self, i: int, L: _Layer, h: torch.Tensor, ctx: Any, batch: Any) -> torch.Tensor:

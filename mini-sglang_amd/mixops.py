@@ -118,10 +118,21 @@ def latent_attn_splits(batch: int, total_q: int, H: int, max_keys: int) -> int:
     return max(1, min(1024 // max(blocks, 1), max_keys // 256, 64))
 
 
+def latent_portion_splits(batch: int, total_q: int, H: int, max_keys: int) -> int:
+    """Key ranges of portions with few rows at the usual widths: 128 rows fill a CU, and with fewer than half of the CUs at work their keys are
+    cut into ranges of at least 128 keys (a rule of the kernel too).  One portion, 16 heads: 32 tokens after 1000 keys 85 -> 38 us, 20 after
+    1000 in 4 / 8 ranges 33 / 26 us; 20 after 100 in one range 21 us, where seven empty ones more make it 26."""
+    if total_q <= batch * (16 // min(H, 16)):
+        return 1
+    groups = (total_q // (128 // min(H, 128)) + batch) * -(-H // 128)
+    return max(1, min(256 // max(groups, 1), -(-max_keys // 128), 8))
+
+
 def latent_attn(out: torch.Tensor, q_abs: torch.Tensor, cache: torch.Tensor, table: torch.Tensor, req_rows: torch.Tensor,
                 seq_lens: torch.Tensor, cu_q: torch.Tensor, batch: int, dv: int, scale: float, splits: int = 1,
-                sink: Optional[torch.Tensor] = None) -> None:
-    """sink (fp32 [H]): one more term exp(sink[h]) in every softmax denominator of head h, with no key and no value."""
+                sink: Optional[torch.Tensor] = None, max_keys: Optional[int] = None) -> None:
+    """sink (fp32 [H]): one more term exp(sink[h]) in every softmax denominator of head h, with no key and no value.  splits: key ranges at
+    most; with 1, portions of few rows get a number of their own, from the longest sequence `max_keys` (None: the table's width)."""
     _dev(out, q_abs, cache, table, req_rows, seq_lens, cu_q, sink)
     assert sink is None or (sink.dtype == torch.float32 and sink.is_contiguous() and sink.shape == (q_abs.shape[1],))
     T, H, dk = q_abs.shape
@@ -130,11 +141,7 @@ def latent_attn(out: torch.Tensor, q_abs: torch.Tensor, cache: torch.Tensor, tab
     assert table.dtype == torch.int32 and table.stride(1) == 1
     assert req_rows.numel() >= batch and seq_lens.numel() >= batch and cu_q.numel() >= batch + 1
     if splits == 1 and cache.dtype == torch.bfloat16 and (dk, dv) in ((576, 512), (320, 256)):
-        # Portions of few rows: 128 of them fill a CU, and with fewer than half of the CUs at work their keys are cut into ranges (of at
-        # least 128 keys, a rule of the kernel: short sequences leave the later ranges empty).  One portion, 16 heads: 32 tokens after 1000
-        # keys 85 -> 38 us, 512 fresh tokens 50 -> 46 us; 128 fresh ones (one range has keys) 21.5 -> 22 us.
-        groups = (T // max(1, 128 // min(H, 128)) + batch) * -(-H // 128)
-        splits = max(1, min(256 // max(groups, 1), table.shape[1] // 256, 8)) if T > batch * (16 // min(H, 16)) else 1
+        splits = latent_portion_splits(batch, T, H, table.shape[1] if max_keys is None else max_keys)
     ws = None
     if splits > 1:
         ws = torch.empty(mix_lib().msgl_mix_latent_attn_workspace_floats(T, H, dv, splits), dtype=torch.float32, device=out.device)
@@ -371,12 +378,23 @@ def window_attn_splits(batch: int, total_q: int, window: int, max_keys: int) -> 
     return max(1, min(512 // max(total_q, 1), keys // 128, 32))
 
 
+def window_portion_splits(batch: int, total_q: int, window: int, max_keys: int, matrix: bool) -> int:
+    """Key ranges where window_attn_splits gives one: a few short portions are some tens of token groups for 256 compute units, so their keys are
+    cut as well.  16-token groups on the matrix cores, from 128 keys a range (16 heads; 500 fresh tokens in 1 / 4 ranges 52 / 41 us, 100
+    decoded ones over 300 keys in 1 / 2 46 / 39, but 8 portions of 100 fresh ones 27 / 36); the plain kernel, whose every token walks all
+    heads, from 64 (fp32, 16 heads: 8 portions of 100 120 / 86 us, 20 tokens after 1000 862 / 128 in 8; 2 after 50 40 / 46).  A function of
+    static sizes only, so a captured graph keeps its grid."""
+    groups, keys = total_q // 16 + batch, min(window, max_keys) if window > 0 else max_keys
+    return max(1, min(256 // groups, -(-keys // (128 if matrix else 64)), 8)) if 0 < groups <= 128 else 1
+
+
 def window_attn(out: torch.Tensor, src: torch.Tensor, g_off: int, k_cache: torch.Tensor, v_cache: torch.Tensor, table: torch.Tensor,
                 req_rows: torch.Tensor, seq_lens: torch.Tensor, cu_q: torch.Tensor, batch: int, H: int, G: int, d: int, dv: int,
-                window: int, scale: float, talk: torch.Tensor, splits: int = 1) -> None:
+                window: int, scale: float, talk: torch.Tensor, splits: int = 1, max_keys: Optional[int] = None) -> None:
     """Sliding-window attention with the heads' scores mixed by `talk` (fp32 [H, H]) and a sigmoid gate per head (src[:, g_off + h]);
     q = src[:, : H * d].  out: [T, H * dv] in the model dtype.  splits > 1: the visible keys of every token in that many ranges
-    (partial results merged by a second launch), for steps with few query tokens."""
+    (partial results merged by a second launch), for steps with few query tokens; with 1, steps of few token groups get a number of their
+    own, from the longest sequence `max_keys` (None: the table's width)."""
     _dev(out, src, k_cache, v_cache, table, req_rows, seq_lens, cu_q, talk)
     T = src.shape[0]
     assert src.stride(1) == 1 and out.is_contiguous() and out.shape == (T, H * dv) and out.dtype == src.dtype
@@ -385,11 +403,8 @@ def window_attn(out: torch.Tensor, src: torch.Tensor, g_off: int, k_cache: torch
     assert table.dtype == torch.int32 and table.stride(1) == 1
     assert req_rows.numel() >= batch and seq_lens.numel() >= batch and cu_q.numel() >= batch + 1
     if splits == 1:
-        # a few short portions are some tens of 16-token groups for 256 compute units: cut their keys as well (32 portions of 8 - 32
-        # tokens over 2000 keys, 16 heads: 226 -> 72 us); from static sizes only, so a captured graph keeps its grid
-        groups, keys = T // 16 + batch, min(window, table.shape[1]) if window > 0 else table.shape[1]
-        if 0 < groups <= 128:
-            splits = max(1, min(256 // groups, keys // 256, 8))
+        splits = window_portion_splits(batch, T, window, table.shape[1] if max_keys is None else max_keys,
+                                       bool(mix_lib().msgl_mix_window_attn_on_matrix_cores(H, G, d, dv, _code(src))))
     ws = None
     if splits > 1:
         ws = torch.empty(mix_lib().msgl_mix_window_attn_workspace_floats(T, H, dv, splits), dtype=torch.float32, device=out.device)
@@ -748,12 +763,26 @@ def sink_attn(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
         int(keep), _p(sink), _code(k_cache), splits, _p(ws), _stream()), "sink_attn")
 
 
+def diff_portion_splits(batch: int, total_q: int, H: int, G: int, window: int, keep: int, max_keys: int) -> int:
+    """Key ranges of portions with few rows at the usual widths: the kernel's groups of 128 rows leave most CUs idle, so their keys are cut into
+    ranges of at least 256 keys (a rule of the kernel too).  16 heads on 4, one portion: 32 tokens after 1000 keys 51 -> 30 us, 128 after
+    2000 86 -> 39 us; 512 fresh ones (68 groups) 29 us in one range, 36 us in three; 100 fresh ones 26 us, 32 with seven empty ranges."""
+    rep = H // G
+    hb = min(1 << (rep.bit_length() - 1), 32)
+    groups = (total_q // (128 // hb) + batch) * G * -(-rep // hb)
+    if total_q <= batch * (16 // min(hb, 16)) or groups > 64:
+        return 1
+    return max(1, min(256 // max(groups, 1), (min(window + keep, max_keys) if window > 0 else max_keys) // 256, 8))
+
+
 def diff_attn(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, table: torch.Tensor, req_rows: torch.Tensor,
               seq_lens: torch.Tensor, cu_q: torch.Tensor, batch: int, H: int, G: int, d: int, dv: int, scale: float, window: int, keep: int,
-              lam: torch.Tensor, post: float, eps: float, gate: Optional[torch.Tensor] = None, splits: int = 1) -> None:
+              lam: torch.Tensor, post: float, eps: float, gate: Optional[torch.Tensor] = None, splits: int = 1,
+              max_keys: Optional[int] = None) -> None:
     """Two softmax maps over the same values (q fp32 [T, H * 2 * d], key rows [G, 2, d], visible keys as in sink_attn): with their
     outputs a1, a2 and lam (fp32 [1] on the device) out = rms_unit(a1 - lam a2) per head * post * sigmoid(gate) (gate [T, H * dv] in
-    out's dtype, a view with a row stride is fine, or None)."""
+    out's dtype, a view with a row stride is fine, or None).  splits: key ranges; with 1, portions of few rows get a number of their own,
+    from the longest sequence `max_keys` (None: the table's width)."""
     _dev(out, q, k_cache, v_cache, table, req_rows, seq_lens, cu_q, lam, gate)
     T = q.shape[0]
     assert q.dtype == torch.float32 and q.is_contiguous() and q.shape == (T, H * 2 * d)
@@ -762,14 +791,8 @@ def diff_attn(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache
     assert table.dtype == torch.int32 and table.stride(1) == 1 and _f32(lam, 1) is not None
     assert gate is None or (gate.shape == (T, H * dv) and gate.stride(1) == 1 and gate.dtype == out.dtype)
     assert req_rows.numel() >= batch and seq_lens.numel() >= batch and cu_q.numel() >= batch + 1
-    if splits == 1 and k_cache.dtype == torch.bfloat16 and (d, dv) == (64, 128):
-        # Portions of few rows: the kernel's groups of 128 rows leave most CUs idle, so their keys are cut into ranges (of at least 256 keys, a
-        # rule of the kernel).  16 heads on 4, one portion: 32 tokens after 1000 keys 51 -> 30 us, 128 after 2000 86 -> 39 us; 512 fresh ones
-        # (68 groups) 29 us in one range, 36 us in three.
-        hb = min(1 << ((H // G).bit_length() - 1), 32)
-        groups = (T // (128 // hb) + batch) * G * -(-(H // G) // hb)
-        if T > batch * (16 // min(hb, 16)) and groups <= 64:
-            splits = max(1, min(256 // groups, table.shape[1] // 256, 8))
+    if splits == 1 and k_cache.dtype == torch.bfloat16 and (d, dv) == (64, 128) and H >= G >= 1:
+        splits = diff_portion_splits(batch, T, H, G, window, keep, table.shape[1] if max_keys is None else max_keys)
     ws = None
     if splits > 1:
         ws = torch.empty(mix_lib().msgl_mix_sink_attn_workspace_floats(T, 2 * H, dv, splits), dtype=torch.float32, device=out.device)

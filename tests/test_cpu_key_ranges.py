@@ -47,3 +47,45 @@ def _window(rec, T, batch, width, dtype=torch.bfloat16, H=16, G=4, d=128, window
 def test_window_without_requests(launched):
     """A step without requests has no groups to divide by."""
     assert _window(launched, 0, 0, 4096) == 1
+
+
+def _latent(rec, T, batch, width, H=16, **kw):
+    from mini_sglang_amd import mixops
+
+    mixops.latent_attn(torch.zeros(T, H, 512), torch.zeros(T, H, 576), torch.zeros(8, 576, dtype=torch.bfloat16), torch.zeros((batch, width), dtype=torch.int32),
+                       _i32(*range(batch)), _i32(*[1] * batch), _i32(*range(batch + 1)), batch, 512, 0.1, **kw)
+    return rec.splits
+
+
+def _diff(rec, T, batch, width, H=16, G=4, window=0, keep=0, **kw):
+    from mini_sglang_amd import mixops
+
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16)  # noqa: E731
+    mixops.diff_attn(z(T, H * 128), torch.zeros(T, H * 128), z(8, G * 128), z(8, G * 128), torch.zeros((batch, width), dtype=torch.int32), _i32(*range(batch)),
+                     _i32(*[1] * batch), _i32(*range(batch + 1)), batch, H, G, 64, 128, 0.1, window, keep, torch.ones(1), 0.5, 1e-5, **kw)
+    return rec.splits
+
+
+@pytest.mark.parametrize("call", [_latent, _window, _diff], ids=["latent", "window", "maps"])
+def test_ranges_follow_the_longest_sequence_not_the_table(launched, call):
+    """An engine's table is as wide as the longest sequence it allows: the batch's longest one decides, the width only where it is not given."""
+    wide = 40960
+    assert call(launched, 100, 1, wide, max_keys=100) == 1  # a short fresh portion: one range
+    for n in (100, 300, 500, 1000, 5000):
+        assert call(launched, 20, 1, wide, max_keys=n) == call(launched, 20, 1, n), n
+    assert call(launched, 20, 1, wide, max_keys=5000) == call(launched, 20, 1, wide) == 8
+    assert call(launched, 20, 1, wide, max_keys=100, splits=3) == 3  # the caller's own number stays
+    assert call(launched, 8192, 4, wide, max_keys=4000) == 1  # groups enough
+
+
+def test_ranges_stay_inside_the_window(launched):
+    assert _window(launched, 20, 1, 40960, window=256, max_keys=9000) == 2
+    assert _diff(launched, 20, 1, 40960, window=64, keep=64, max_keys=9000) == 1
+    assert _diff(launched, 20, 1, 40960, window=1024, keep=64, max_keys=9000) == 4
+
+
+def test_window_ranges_of_the_plain_kernel(launched):
+    """fp32 engines and head counts that the matrix cores do not take: a range from 64 keys on."""
+    for kw in ({"dtype": torch.float32}, {"H": 12}, {"G": 8}, {"d": 136}):
+        assert _window(launched, 20, 1, 40960, max_keys=64, **kw) == 1 and _window(launched, 20, 1, 40960, max_keys=100, **kw) == 2
+        assert _window(launched, 20, 1, 40960, max_keys=5000, **kw) == 8
