@@ -46,6 +46,17 @@ __global__ __launch_bounds__(256, 2) void maps_prompt_kernel(bf16_t* __restrict_
   const int r_own = wave * 32 + (lane & 31);
   const int tl = tok0 + (r_own >> hb_log2), hh = h0 + (r_own & (HB - 1));
   const int limit = tl < q_len && hh < h_end ? start + tl : -1;
+  if (RANGES && k_begin >= k_end) {  // no keys left for this range: its partial outputs are not read
+    if (hi == 0 && limit >= 0) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const size_t row = (((size_t)z * total_q + first + tl) * H + hh) * 2 + a;
+        part_ml[row * 2] = -INFINITY;
+        part_ml[row * 2 + 1] = 0.f;
+      }
+    }
+    return;
+  }
   const int lo_row = window > 0 ? max(0, limit - window + 1) : 0;
   // this wave's rows: the first and the last token's position, the last one's first key
   const int w_min = start + tok0 + ((wave * 32) >> hb_log2), w_max = min(start + last_tok, w_min + ((31 + HB) >> hb_log2) - 1);

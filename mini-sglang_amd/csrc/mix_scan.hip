@@ -946,13 +946,18 @@ __global__ __launch_bounds__(64) void diff_merge_kernel(T* __restrict__ out, int
   const size_t t = blockIdx.x / H;
   const int h = blockIdx.x % H;
   float M[2] = {-INFINITY, -INFINITY}, f[2];
+  int live = 0;  // ranges behind the last one with a key of this row add nothing, and mix_maps.hip leaves partial outputs without keys unwritten
   for (int s = 0; s < splits; ++s)
 #pragma unroll
-    for (int a = 0; a < 2; ++a) M[a] = fmaxf(M[a], part_ml[((((size_t)s * total_q + t) * H + h) * 2 + a) * 2]);
+    for (int a = 0; a < 2; ++a) {
+      const float* ml = part_ml + ((((size_t)s * total_q + t) * H + h) * 2 + a) * 2;
+      M[a] = fmaxf(M[a], ml[0]);
+      live = ml[1] == 0.f ? live : s + 1;
+    }
 #pragma unroll
   for (int a = 0; a < 2; ++a) {
     float den = 0.f;
-    for (int s = 0; s < splits; ++s) {
+    for (int s = 0; s < live; ++s) {
       const float* ml = part_ml + ((((size_t)s * total_q + t) * H + h) * 2 + a) * 2;
       den += ml[1] * expf(ml[0] - M[a]);
     }
@@ -964,7 +969,7 @@ __global__ __launch_bounds__(64) void diff_merge_kernel(T* __restrict__ out, int
     const int c = threadIdx.x + 64 * i;
     o[i] = 0.f;
     if (c < dv) {
-      for (int s = 0; s < splits; ++s)
+      for (int s = 0; s < live; ++s)
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
           const size_t row = (((size_t)s * total_q + t) * H + h) * 2 + a;

@@ -681,6 +681,70 @@ def test_diff_attention_portions_of_usual_width(dev, H, G, window, keep):
             at += m
 
 
+@pytest.mark.parametrize("window,keep", [(0, 0), (700, 0), (600, 300), (300, 64)])
+@pytest.mark.parametrize("H,G", [(16, 4), (6, 2)])
+@pytest.mark.parametrize("splits,width", [(3, 1280), (5, 1280), (1, 1280)], ids=["three-ranges", "five-ranges", "own-rule"])
+def test_diff_attention_key_ranges_of_portions(dev, H, G, window, keep, splits, width):
+    """Portions in one launch whose sequences leave one, two, three and five ranges of at least 256 keys with work and the others empty; the
+    window's first key and the seam between kept and window keys lie inside ranges and on their ends; the number that the entry point chooses
+    by itself; partial results in memory that held no numbers.  Bound as for one range."""
+    from mini_sglang_amd import mixops
+
+    d, dv, scale, lam, eps = 64, 128, 64 ** -0.5, 0.4, 1e-5
+    new, old = [20, 33, 9, 40], [0, 700, 1100, 300]
+    g = torch.Generator().manual_seed(H + window + keep)
+    lens, B = [a + b for a, b in zip(new, old)], len(new)
+    if splits == 1:
+        assert (mixops.diff_portion_splits(B, sum(new), H, G, window, keep, width) > 1) == (window != 300)
+    kc, vc = (torch.zeros((2560, n), dtype=torch.bfloat16, device=dev) for n in (G * 2 * d, G * dv))
+    table, perm, at = torch.zeros((B, width), dtype=torch.int32), torch.randperm(2560, generator=g), 0
+    q, k, v = [], [], []
+    for b, (n, m) in enumerate(zip(lens, new)):
+        sl = perm[at: at + n]
+        at += n
+        table[b, :n] = sl.int()
+        q.append(torch.randn(m, H, 2, d, generator=g).bfloat16().double())
+        k.append(torch.randn(n, G, 2, d, generator=g).bfloat16().double())
+        v.append(torch.randn(n, G, dv, generator=g).bfloat16().double())
+        kc[sl.to(dev)], vc[sl.to(dev)] = k[-1].view(n, -1).bfloat16().to(dev), v[-1].view(n, -1).bfloat16().to(dev)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    out = torch.empty((sum(new), H * dv), dtype=torch.bfloat16, device=dev)
+    spoilt = torch.full((1 << 22,), float("nan"), device=dev)  # the caching allocator hands this memory out again
+    torch.cuda.synchronize()
+    del spoilt
+    mixops.diff_attn(out, torch.cat([x.reshape(x.shape[0], -1) for x in q]).float().to(dev), kc, vc, table.to(dev), i32(range(B)), i32(lens),
+                     torch.tensor([0] + new).cumsum(0).int().to(dev), B, H, G, d, dv, scale, window, keep, torch.full((1,), lam, device=dev), 0.7, eps, splits=splits)
+    at = 0
+    for x, kk, vv, n, m in zip(q, k, v, lens, new):
+        pos, key = torch.arange(n - m, n)[:, None], torch.arange(n)[None, :]
+        seen = (key <= pos) & ((pos - key < window) | (key < keep) if window else torch.ones(1, dtype=torch.bool))
+        maps = []
+        for a in range(2):
+            s = torch.stack([x[:, h, a] @ kk[:, h // (H // G), a].T for h in range(H)], 1) * scale
+            p = torch.softmax(s.masked_fill(~seen[:, None], -torch.inf), -1)
+            maps.append(torch.stack([p[:, h] @ vv[:, h // (H // G)] for h in range(H)], 1))
+        ref = O.rms_unit(maps[0] - lam * maps[1], eps) * 0.7
+        assert rel(out.double().cpu()[at: at + m].view(m, H, dv), ref) < 1e-2, n
+        at += m
+
+
+@pytest.mark.parametrize("splits", [1, 4])
+def test_diff_attention_range_of_undefined_keys(dev, splits):
+    """The last range holds nothing but keys that are no numbers: the rows that see them are none either, in one range and in four."""
+    from mini_sglang_amd import mixops
+
+    H, G, n, new = 8, 2, 773, 5  # ranges of 256 keys, the new tokens' own in the fourth
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    g = torch.Generator().manual_seed(1)
+    k, v = torch.randn(1024, G * 128, generator=g), torch.randn(1024, G * 128, generator=g)
+    k[768:773] = torch.nan
+    out = torch.zeros((new, H * 128), dtype=torch.bfloat16, device=dev)
+    mixops.diff_attn(out, torch.randn(new, H * 128, generator=g).to(dev), k.bfloat16().to(dev), v.bfloat16().to(dev), torch.arange(256, dtype=torch.int32, device=dev).repeat(4)[None] +
+                     torch.arange(4, dtype=torch.int32, device=dev).repeat_interleave(256)[None] * 256, i32([0]), i32([n]), i32([0, new]), 1, H, G, 64, 128, 0.125, 0, 0,
+                     torch.full((1,), 0.4, device=dev), 1.0, 1e-5, splits=splits)
+    assert torch.isnan(out).all()
+
+
 @pytest.mark.parametrize("splits", [1, 2], ids=["one-range", "two-ranges"])
 def test_diff_attention_row_sum_of_unrounded_weights(dev, splits):
     """Both denominators take the fp32 weights, the products the bf16 ones: in the first map every 16th key weighs 1 and the others 0.2509,
