@@ -362,7 +362,10 @@ __device__ __forceinline__ uint32_t kth_largest(uint32_t bits, int target, uint3
 
 constexpr int kList = 2048;          // candidates of a row that the short path holds (= kBins: it reuses the histograms)
 constexpr int kListTopK = 1024;      // largest top-k it is tried for: one column maximum per thread bounds the k-th largest from below
-constexpr int kListTopP = 512;       // candidates asked for when only a mass is given
+// candidates asked for when only a mass is given: a list takes time with its square (512: 120 us for any row of 32000, 62 without a list), and a
+// nucleus that does not fit pays for it on top (bf16 rows, top-p 0.9, one row of 151936: nucleus 8: 55 us with 64, 91 with 256, 157 with 512, 219
+// without; nucleus 2127: 141, 185, 225, 217)
+constexpr int kListTopP = 64;
 constexpr uint32_t kTinyWeight = 0x17800000u;  // 2^-80: below it two weights apart may be one probability (denormal)
 
 // One 1024-thread workgroup per row.
@@ -392,6 +395,7 @@ __device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64
 
   uint32_t thr_bits = 0u;  // keep set = { bits >= thr_bits, p > 0 }
   u64 kept_mass = 0;
+  bool have_mass = false;  // kept_mass is that of the whole row
   bool done = false;       // uniform: the threshold is known and every number that reaches it is in the list
   int n = 0;
 
@@ -450,6 +454,7 @@ __device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64
     }
     u64 target = 0;
     if (by_mass) {
+      have_mass = true;
       u64 loc = 0;
       walk_row(src, vocab, [&](int64_t, float x, bool in) {
         const u64 m = fixed_mass(src.prob(src.weight(x)));
@@ -528,12 +533,14 @@ __device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64
     if (v != kNoDigit) thr_bits = v;
   }
   if (pp < 1.0f) {
-    u64 loc = 0;
-    walk_row(src, vocab, [&](int64_t, float x, bool in) {
-      const float p = src.prob(src.weight(x));
-      if (in && __float_as_uint(p) >= thr_bits) loc += fixed_mass(p);
-    });
-    kept_mass = block_sum_u64(loc, lds_w);
+    if (!have_mass) {
+      u64 loc = 0;
+      walk_row(src, vocab, [&](int64_t, float x, bool in) {
+        const float p = src.prob(src.weight(x));
+        if (in && __float_as_uint(p) >= thr_bits) loc += fixed_mass(p);
+      });
+      kept_mass = block_sum_u64(loc, lds_w);
+    }
     u64 target = (u64)((double)pp * (double)kept_mass);
     if (target < 1) target = 1;
     if (target > kept_mass) target = kept_mass;

@@ -299,3 +299,24 @@ def test_a_second_draw_takes_what_the_first_one_took(ops, dev, dtype):
     want = [ops.sample_top_k_top_p(stored, a, b, torch.initial_seed(), 5 * i) for i, (a, b) in enumerate(((k, p), (k, None), (None, p)))]
     assert torch.stack(got).tolist() == torch.stack(want).tolist()
     assert torch.equal(probs.probs(), stored)
+
+
+@pytest.mark.parametrize("vocab", [2000, 33333])
+def test_nucleus_at_the_list_s_length(ops, dev, vocab):
+    """Nuclei of 1 to 130 tokens around the 64 that the candidate list is asked for, equal and unequal ones, in different columns and in one: the
+    picks of the integer rule, from the logits and from stored probabilities."""
+    g = torch.Generator().manual_seed(vocab)
+    sizes = [1, 2, 60, 63, 64, 65, 66, 70, 100, 130]
+    rows = [(m, kind) for m in sizes for kind in ("equal", "steps", "column")]
+    logits = torch.full((len(rows), vocab), -9.0) + 0.1 * torch.randn((len(rows), vocab), generator=g)
+    for r, (m, kind) in enumerate(rows):
+        at = torch.randperm(vocab, generator=g)[:m] if kind != "column" else (torch.arange(m) * 1024 + 5) % vocab
+        logits[r, at] = 8.0 if kind == "equal" else 8.0 - 0.03 * torch.arange(m)
+    logits = logits.bfloat16().to(dev)
+    t, p = torch.ones(len(rows), device=dev), torch.full((len(rows),), 0.98, device=dev)
+    probs = ops.softmax_temperature(logits, t)
+    host = probs.cpu().numpy()
+    for off in (0, 5000, 10000):
+        want = [_filtered_pick(host[r], 0, 0.98, 3, off + r) for r in range(len(rows))]
+        assert ops.sample_filtered_logits(logits, t, None, p, 3, off).cpu().tolist() == want
+        assert ops.sample_top_k_top_p(probs, None, p, 3, off).cpu().tolist() == want
