@@ -233,8 +233,11 @@ extern "C" __attribute__((visibility("hidden"))) int mix_gemm_nt_dma(void* C, co
   //   16 x 1500, 1024, 768          93.1       72.6        63.0
   //   64 x 768, 1024, 2048           420        304         265
   //   64 x 256, 2048, 512            106       82.1        88.0    (the one of 19 sizes measured where the rule misses by more than 3 %)
+  // Groups of uneven length, as a router fills them (random | log-normal, sigma 0.7), where a 256-row tile holds one short group:
+  //   64 x 96, 1024, 2048                      72.8 | 90.5   74.7 | 112    32 x 96, 2048, 1024: 29.8 | 43.0   33.8 | 56.7
+  //   64 x 112, 1024, 2048                     97.2 | 90.7   76.9 | 114    32 x 128, 2048, 1024: 46.9 | 44.6   36.1 | 57.5
   const int64_t each = seg ? M / groups : M;
-  const bool large = each >= 96 && blocks(256, 256) >= 256;
+  const bool large = each >= 112 && blocks(256, 256) >= 256;
 #define GEMM_SIZE(TC)                                                   \
   {                                                                     \
     if (K % 64) {                                                       \
