@@ -432,12 +432,28 @@ def short_conv(src: torch.Tensor, C: int, taps: torch.Tensor, state: Optional[to
     return out
 
 
+def delta_in_blocks(batch: int, total_q: int, H: int, d: int, per_channel: bool, longest: Optional[int] = None) -> bool:
+    """Blocks of 16 tokens on the matrix instructions (two launches, 14 us however short the portions are, and more for every further request
+    and head), or token by token (a token of the longest portion: 2.2 us at d = 128, 4.4 with a decay per channel, 1.0 and 1.7 at d = 64).
+    Token loop / blocks in us on both sides of the line, requests x tokens, 16 heads of d = 128: 1 x 6 26 / 14.5; 16 x 6 29 / 34, 16 x 8 34 / 33,
+    64 x 6 65 / 90, 64 x 12 99 / 93; per channel 1 x 6 38 / 15, 64 x 6 92 / 90.  d = 64 (dv 128): 1 x 8 16.0 / 17.6, 1 x 12 20.0 / 18.5, 16 x 16
+    26 / 31, 40 x 16 39 / 56, 64 x 24 89 / 89; per channel 1 x 6 17.5 / 16.2, 16 x 8 23 / 28, 16 x 16 38 / 31, 64 x 12 68 / 69.  One long portion
+    among single tokens: 16 requests, one of 80 tokens, 196 us token by token and 47 in blocks; where the longest is not known, only many
+    tokens speak for one."""
+    wide = batch * H > 128  # every further (request, head) is a walk of its own
+    need = {(128, False): (6, 8), (128, True): (6, 6), (64, False): (10, 28), (64, True): (6, 13)}.get((d, bool(per_channel)), (6, 12))[wide]
+    if total_q >= need * batch:
+        return True
+    return longest >= 40 if longest is not None else batch * H > 256 and total_q - batch >= 256
+
+
 def delta_rule(out: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, b_raw: torch.Tensor, a_raw: torch.Tensor, per_channel: bool,
                rate: torch.Tensor, dt_bias: torch.Tensor, cu_q: torch.Tensor, seq_lens: torch.Tensor, slots: torch.Tensor, batch: int,
-               G: int, chunks=None) -> None:
+               G: int, chunks=None, longest: Optional[int] = None) -> None:
     """state: fp32 [slots, H, d, dv]; qkv: fp32 rows [q G*d | k G*d | v H*dv]; b_raw [T, H], a_raw [T, H] or [T, H*d] in the model
     dtype (views with a row stride are fine); rate = -exp(A_log) and dt_bias in fp32.  chunks = (items int32 [n, 3], item_first
-    int32 [batch + 1], n) cuts long portions into pieces that run in parallel (see include/msgl_mix.h)."""
+    int32 [batch + 1], n) cuts long portions into pieces that run in parallel (see include/msgl_mix.h) where the token loop takes them:
+    other head sizes than 64 / 128 x a multiple of 32.  longest: new tokens of the longest portion, where the caller knows them."""
     _dev(out, qkv, state, b_raw, a_raw, rate, dt_bias, cu_q, seq_lens, slots)
     _, H, d, dv = state.shape
     T = qkv.shape[0]
@@ -446,12 +462,7 @@ def delta_rule(out: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, b_raw:
     assert qkv.shape == (T, 2 * G * d + H * dv) and out.dtype == torch.float32 and out.is_contiguous() and out.shape == (T, H * dv)
     assert b_raw.stride(1) == 1 and a_raw.stride(1) == 1 and b_raw.shape == (T, H) and a_raw.shape == (T, na) and a_raw.dtype == b_raw.dtype
     assert rate.dtype == torch.float32 and rate.shape == (H,) and dt_bias.dtype == torch.float32 and dt_bias.shape == (na,)
-    # Blocks of 16 tokens on the matrix instructions, or token by token.  The blocks cost 20 us however short the portions are (two
-    # launches, a block's latency), the token loop 4.4 us (decay per channel) or 1.7 us a token of the longest portion: 16 heads, one
-    # request of 4 / 6 / 16 / 500 tokens 30 / 39 / 82 / 2259 us against 21 / 20 / 21 / 67; 64 requests of 1 / 8 / 16 / 64: 40 / 114 / 199 / 714
-    # against 89 / 93 / 98 / 237.  With many requests a block per request is work of its own, unless one of them may be long.
-    many = batch * H > 256
-    blocks = T >= 12 * batch or T - batch >= 256 if many else T >= 6 * batch
+    blocks = delta_in_blocks(batch, T, H, d, per_channel, longest)
     floats = mix_lib().msgl_mix_delta_rule_block_floats(d, dv) * (T // 16 + batch) * H if blocks else 0
     if floats:
         scratch = torch.empty(floats, dtype=torch.float32, device=out.device)

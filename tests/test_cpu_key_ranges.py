@@ -89,3 +89,18 @@ def test_window_ranges_of_the_plain_kernel(launched):
     for kw in ({"dtype": torch.float32}, {"H": 12}, {"G": 8}, {"d": 136}):
         assert _window(launched, 20, 1, 40960, max_keys=64, **kw) == 1 and _window(launched, 20, 1, 40960, max_keys=100, **kw) == 2
         assert _window(launched, 20, 1, 40960, max_keys=5000, **kw) == 8
+
+
+def test_delta_rule_blocks_where_they_are_faster():
+    """Portions on both sides of the line between the token loop and blocks of 16 tokens, the measured one at each; a longest portion that the
+    caller names decides over the mean."""
+    from mini_sglang_amd.mixops import delta_in_blocks
+
+    for batch, each, H, d, channel, want in [
+            (1, 5, 16, 128, False, False), (1, 6, 16, 128, False, True), (8, 6, 16, 128, True, True), (16, 6, 16, 128, False, False), (16, 8, 16, 128, False, True),
+            (64, 6, 4, 128, True, True), (1, 9, 16, 64, False, False), (1, 10, 16, 64, False, True), (40, 16, 16, 64, False, False), (16, 28, 16, 64, False, True),
+            (1, 5, 8, 64, True, False), (4, 6, 8, 64, True, True), (16, 8, 16, 64, True, False), (64, 13, 16, 64, True, True), (32, 1, 16, 128, True, False)]:
+        assert delta_in_blocks(batch, batch * each, H, d, channel, longest=each) == want, (batch, each, H, d, channel)
+    assert delta_in_blocks(40, 640, 16, 64, False)  # many requests that may hide a long portion
+    assert delta_in_blocks(16, 95, 16, 128, False, longest=80) and not delta_in_blocks(16, 95, 16, 128, False)
+    assert not delta_in_blocks(64, 384, 16, 128, False, longest=6) and not delta_in_blocks(64, 64, 16, 64, True, longest=1)
