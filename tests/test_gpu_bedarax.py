@@ -256,6 +256,39 @@ def test_window_matrix_cores(dev, H, G, d, dv, splits):
         assert bool((diff <= 2.0 ** -8 * ref.abs() + 2.0 ** -14 * ref.abs().max()).all()), (window, float(diff.max()))
 
 
+@pytest.mark.parametrize("B", [64, 65, 150])
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("most", [1, 40], ids=["decode", "portions"])
+def test_window_many_requests(dev, B, splits, most):
+    """More requests than a wave has lanes (their groups are found another way), some of them without new tokens, each against its own
+    launch.  Bound: the bf16 results (2^-8 of the value) and fp32 sums of other ranges."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(B + most)
+    H, G, d, window = 16, 4, 64, 50
+    new = [1] * B if most == 1 else torch.randint(0, most + 1, (B,), generator=g).tolist()
+    lens = [n + c for n, c in zip(new, torch.randint(0, 90, (B,), generator=g).tolist())]
+    slots, at = torch.randperm(sum(lens), generator=g), 0
+    table = torch.zeros((B, 160), dtype=torch.int32)
+    for b, n in enumerate(lens):
+        table[b, :n] = slots[at: at + n].int()
+        at += n
+    kc, vc = (torch.randn(sum(lens), G * d, generator=g).bfloat16().to(dev) for _ in range(2))
+    src = torch.randn(sum(new), H * d + H, generator=g).bfloat16().to(dev)
+    talk = (torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)).to(dev)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    out, table = torch.full((sum(new), H * d), float("nan"), dtype=torch.bfloat16, device=dev), table.to(dev)
+    mixops.window_attn(out, src, H * d, kc, vc, table, i32(range(B)), i32(lens), torch.tensor([0] + new).cumsum(0).int().to(dev), B, H, G, d, d, window, d ** -0.5, talk, splits=splits)
+    row = 0
+    for b, (n, k) in enumerate(zip(new, lens)):
+        if n:
+            one = torch.empty((n, H * d), dtype=torch.bfloat16, device=dev)
+            mixops.window_attn(one, src[row: row + n], H * d, kc, vc, table, i32([b]), i32([k]), i32([0, n]), 1, H, G, d, d, window, d ** -0.5, talk, max_keys=k)
+            diff = (out[row: row + n].double() - one.double()).abs()
+            assert bool((diff <= 2.0 ** -7 * one.double().abs() + 2.0 ** -14 * one.double().abs().max()).all()), b
+            row += n
+
+
 @pytest.mark.parametrize("splits", [1, 2], ids=["one-range", "two-ranges"])
 @pytest.mark.parametrize("new", [1, 20], ids=["decode", "portion"])
 @pytest.mark.parametrize("H,G", [(16, 4), (8, 1)])

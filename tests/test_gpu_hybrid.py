@@ -364,6 +364,38 @@ def test_latent_attention_usual_widths(dev, H, R, splits, sink):
         assert float((got - ref).abs().max()) < 5e-2 * float(ref.abs().max()), new
 
 
+@pytest.mark.parametrize("B", [64, 65, 150])
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("most", [1, 20], ids=["decode", "portions"])
+def test_latent_attention_many_requests(dev, B, splits, most):
+    """More requests than a wave has lanes (their groups are found another way), some of them without new tokens, each against its own
+    launch.  Bound: the ranges differ, so bf16 weights under another maximum, as in the test above."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(B + most)
+    H, R, r = 16, 256, 64
+    new = [1] * B if most == 1 else torch.randint(0, most + 1, (B,), generator=g).tolist()
+    old = torch.randint(0, 90, (B,), generator=g).tolist()
+    lens = [n + c for n, c in zip(new, old)]
+    slots, at = torch.randperm(sum(lens), generator=g), 0
+    table = torch.zeros((B, 128), dtype=torch.int32)
+    for b, n in enumerate(lens):
+        table[b, :n] = slots[at: at + n].int()
+        at += n
+    cache = torch.randn(sum(lens), R + r, generator=g).bfloat16().to(dev)
+    q = (torch.randn(sum(new), H, R + r, generator=g) * 0.8).to(dev)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    out, table = torch.full((sum(new), H, R), float("nan"), device=dev), table.to(dev)
+    mixops.latent_attn(out, q, cache, table, i32(range(B)), i32(lens), torch.tensor([0] + new).cumsum(0).int().to(dev), B, R, (128 + r) ** -0.5, splits=splits)
+    row = 0
+    for b, (n, k) in enumerate(zip(new, lens)):
+        if n:
+            one = torch.empty((n, H, R), device=dev)
+            mixops.latent_attn(one, q[row: row + n].contiguous(), cache, table, i32([b]), i32([k]), i32([0, n]), 1, R, (128 + r) ** -0.5, max_keys=k)
+            assert rel(out[row: row + n].double().cpu(), one.double().cpu()) < 5e-3, b
+            row += n
+
+
 @pytest.mark.parametrize("splits", [1, 2], ids=["one-range", "two-ranges"])
 @pytest.mark.parametrize("new", [1, 20], ids=["decode", "portion"])
 @pytest.mark.parametrize("R", [512, 256])
@@ -398,11 +430,12 @@ def test_latent_attention_row_sum_of_unrounded_weights(dev, R, new, splits):
 
 
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
-@pytest.mark.parametrize("N,K", [(256, 32), (128, 64), (264, 96), (520, 256), (72, 128)])
+@pytest.mark.parametrize("N,K", [(256, 32), (128, 64), (264, 96), (520, 256), (520, 64), (72, 128), (136, 224), (264, 288)])
 @pytest.mark.parametrize("lens", [[1, 0, 63, 2, 16], [64, 65, 0, 127, 128, 129, 300], [255, 256, 257] * 30, [0, 0, 700, 17] + [1] * 70], ids=["short", "edges", "long", "many"])
 def test_segmented_product_tiles(dev, lens, N, K, out):
-    """Every tile size of the DMA kernel at the edges of its tiles, k shorter and longer than its ring, gathered and scattered rows, against
-    float64.  Bound: fp32 sums of K exact products, and the rounding of a bf16 result (2^-9 of its size)."""
+    """Every tile size of the DMA kernel at the edges of its tiles (256 x 256: the long lists with N > 256), k shorter and longer than its rings in
+    steps of 32 (up to nine of them, rings of six and four) and of 64, gathered and scattered rows, against float64.  Bound: fp32 sums of
+    K exact products, K 2^-24 of the sum of their sizes, through the square; and the rounding of a bf16 result (its unit roundoff, 2^-8)."""
     from mini_sglang_amd import mixops
 
     g = torch.Generator().manual_seed(N + K + len(lens))
@@ -414,19 +447,22 @@ def test_segmented_product_tiles(dev, lens, N, K, out):
     got = torch.full((rows, N), float("nan"), dtype=out, device=dev)
     mixops.gemm_nt(got, a.to(dev), b.to(dev), rows, N, K, lda=K, ldb=K, ldc=N, groups=E, b_gs=N * K, seg=seg.to(dev), a_rows=perm.to(dev), a_div=2,
                    c_rows=place.to(dev), act=mixops.ACT_RELU2)
-    ref = torch.empty(rows, N, dtype=torch.float64)
+    ref, off = torch.empty(rows, N, dtype=torch.float64), torch.empty(rows, N, dtype=torch.float64)
     for e in range(E):
         m = slice(int(seg[e]), int(seg[e + 1]))
-        ref[place[m].long()] = (a[perm[m].long() // 2].double() @ b[e].double().T).clamp_min(0).square()
-    size = (a.double().abs().max() * b.double().abs().max() * K).square()  # of a result, at most; sums are off by K 2^-24 of it and far less
-    tol = ref * (2.0 ** -8 if out == torch.bfloat16 else 2.0 ** -18) + size * K * 2.0 ** -24
+        x, y = a[perm[m].long() // 2].double(), b[e].double().T
+        z = (x @ y).clamp_min(0)
+        err = K * 2.0 ** -24 * (x.abs() @ y.abs())
+        ref[place[m].long()] = z.square()
+        off[place[m].long()] = 2 * z * err + err.square()
+    tol = off + (ref + off) * (2.0 ** -8 if out == torch.bfloat16 else 2.0 ** -23)
     assert ((got.double().cpu() - ref).abs() <= tol).all()
     # groups of equal size, rows in place
     a3 = torch.randn(3, 70, K, generator=g).bfloat16()
     got = torch.full((3, 70, N), float("nan"), dtype=out, device=dev)
     mixops.gemm_nt(got, a3.to(dev), b[:1].expand(3, N, K).contiguous().to(dev), 70, N, K, lda=K, ldb=K, ldc=N, groups=3, a_gs=70 * K, b_gs=N * K, c_gs=70 * N)
-    ref = a3.double() @ b[0].double().T
-    assert ((got.double().cpu() - ref).abs() <= ref.abs() * 2.0 ** -8 * (out == torch.bfloat16) + size.sqrt() * K * 2.0 ** -23).all()
+    ref, err = a3.double() @ b[0].double().T, K * 2.0 ** -24 * (a3.double().abs() @ b[0].double().abs().T)
+    assert ((got.double().cpu() - ref).abs() <= err + (ref.abs() + err) * 2.0 ** -8 * (out == torch.bfloat16)).all()
 
 
 @pytest.mark.parametrize("n,skip", [(1, 0), (7, 1), (2047, 0), (2048, 3), (2049, 0), (8191, 0), (8193, 1), (16385, 0), (40001, 2)])

@@ -650,7 +650,7 @@ def test_trace_command_line(tmp_path):
 @pytest.mark.parametrize("H,G", [(16, 4), (8, 2), (4, 4), (6, 2), (40, 1)])
 def test_diff_attention_portions_of_usual_width(dev, H, G, window, keep):
     """The kernel of prompt portions (64 / 128 wide): four requests in one launch whose portions end around its 128-row groups and 32- and
-    64-key tiles, windows and kept keys inside tiles, heads per group that are no power of two and more than 32, one range and three, with
+    64-key tiles, windows and kept keys inside tiles, heads per group that are no power of two and more than 32, one range and three (two of them empty), with
     and without a gate.  Bound: bf16 weights (2^-9) under a difference of maps about as large as each of them, and the bf16 result."""
     from mini_sglang_amd import mixops
 
@@ -726,6 +726,37 @@ def test_diff_attention_key_ranges_of_portions(dev, H, G, window, keep, splits, 
         ref = O.rms_unit(maps[0] - lam * maps[1], eps) * 0.7
         assert rel(out.double().cpu()[at: at + m].view(m, H, dv), ref) < 1e-2, n
         at += m
+
+
+@pytest.mark.parametrize("B", [64, 65, 150])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_diff_attention_many_requests(dev, B, splits):
+    """More requests than a wave has lanes (their groups are found another way), some of them without new tokens, each against its own launch.
+    Bound: bf16 weights and results."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(B)
+    H, G, d, dv, window, keep = 16, 4, 64, 128, 50, 7
+    new = torch.randint(0, 41, (B,), generator=g).tolist()
+    lens = [n + c for n, c in zip(new, torch.randint(0, 90, (B,), generator=g).tolist())]
+    slots, at = torch.randperm(sum(lens), generator=g), 0
+    table = torch.zeros((B, 160), dtype=torch.int32)
+    for b, n in enumerate(lens):
+        table[b, :n] = slots[at: at + n].int()
+        at += n
+    kc, vc = (torch.randn(sum(lens), n, generator=g).bfloat16().to(dev) for n in (G * 2 * d, G * dv))
+    q, lam = torch.randn(sum(new), H * 2 * d, generator=g).to(dev), torch.full((1,), 0.4, device=dev)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    out, table = torch.full((sum(new), H * dv), float("nan"), dtype=torch.bfloat16, device=dev), table.to(dev)
+    mixops.diff_attn(out, q, kc, vc, table, i32(range(B)), i32(lens), torch.tensor([0] + new).cumsum(0).int().to(dev), B, H, G, d, dv, d ** -0.5, window, keep, lam, 0.7, 1e-5,
+                     splits=splits)
+    row = 0
+    for b, (n, k) in enumerate(zip(new, lens)):
+        if n:
+            one = torch.empty((n, H * dv), dtype=torch.bfloat16, device=dev)
+            mixops.diff_attn(one, q[row: row + n].contiguous(), kc, vc, table, i32([b]), i32([k]), i32([0, n]), 1, H, G, d, dv, d ** -0.5, window, keep, lam, 0.7, 1e-5, max_keys=k)
+            assert rel(out[row: row + n].double().cpu(), one.double().cpu()) < 1e-2, b
+            row += n
 
 
 @pytest.mark.parametrize("splits", [1, 4])
