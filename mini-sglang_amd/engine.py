@@ -10,6 +10,7 @@ from __future__ import annotations
 import os
 
 import gc
+from contextlib import contextmanager
 from dataclasses import dataclass, field
 from typing import Any, Dict, List, NamedTuple, Optional
 
@@ -85,8 +86,7 @@ class Sampler:
     def sample(self, logits: torch.Tensor, args: SamplingPlan) -> torch.Tensor:
         if args.temperatures is None:  # greedy: first index of the row max
             return ops.argmax_rows(logits)
-        # same op sequence as sample_impl (sample.py:24-45); `softmax` is deferred, so a temperature-only batch
-        # is one fused draw from the logits and only the top-k / top-p variants materialise probabilities
+        # same op sequence as sample_impl (sample.py:24-45); `softmax` is deferred, so every variant is one fused draw from the logits
         probs = fi.sampling.softmax(logits, args.temperatures)
         draw = {
             (False, False): lambda: fi.sampling.sampling_from_probs(probs),
@@ -173,6 +173,19 @@ def determine_graph_bs(cuda_graph_bs: Optional[List[int]], cuda_graph_max_bs: Op
 
 
 # ------------------------------------------------------------------------------ graph runner
+@contextmanager
+def _no_collection():
+    """No cyclic garbage collection meanwhile.  An engine and its graph runner refer to each other, so a dropped engine's graphs go whenever the
+    collector happens to run; a graph's destruction waits for the device, which is refused while a capture is open and ends the process."""
+    was = gc.isenabled()
+    gc.disable()
+    try:
+        yield
+    finally:
+        if was:
+            gc.enable()
+
+
 class GraphRunner:
     """hipGraph capture/replay of the decode forward, P/engine/graph.py:78-171."""
 
@@ -222,7 +235,7 @@ class GraphRunner:
             # with a communicator inside the graph, RCCL's proxy thread may touch the HIP API while this
             # thread captures: only this thread's calls are held to the capture rules then
             mode = "thread_local" if engine.cfg.tp_size > 1 else "global"
-            with torch.cuda.graph(graph, pool=self._pool, stream=engine.stream, capture_error_mode=mode):
+            with _no_collection(), torch.cuda.graph(graph, pool=self._pool, stream=engine.stream, capture_error_mode=mode):
                 forward_into_static()
         if self._pool is None:
             self._pool = graph.pool()

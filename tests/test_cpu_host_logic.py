@@ -215,3 +215,52 @@ def test_ro_plan_arithmetic_matches_the_kernel_and_covers_every_unit():
             assert max(widths) - min(widths) <= 1 and 1 <= slices <= K // 64
         assert all(s == 1 for _, s in ops.ro_candidates(M, N, K, 256, silu=True))
     assert _lib.lib().msgl_ro_gemm_workspace_bytes(256, 5120, 6) == 6 * 256 * 5120 * 4
+
+
+def test_no_garbage_is_collected_inside_a_capture(monkeypatch):
+    """A dropped engine is a reference cycle that owns captured graphs; their destruction must not fall into another capture.  The collector is
+    made to run at every allocation, objects in cycles note where they end."""
+    import contextlib
+    import gc
+    import types
+
+    import torch
+
+    from mini_sglang_amd import engine as E
+
+    ended, open_ = [], [False]
+
+    class Owner:
+        def __init__(self):
+            self.me = self
+
+        def __del__(self):
+            ended.append(open_[0])
+
+    @contextlib.contextmanager
+    def capture(*_a, **_k):
+        open_[0] = True
+        yield
+        open_[0] = False
+
+    def forward(_ctx, _batch, logits_out):
+        Owner()
+        [[] for _ in range(50)]  # allocations that the collector counts
+        return logits_out
+
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: types.SimpleNamespace(pool=lambda: None))
+    monkeypatch.setattr(torch.cuda, "graph", capture)
+    logits = torch.zeros(1, 4)
+    eng = types.SimpleNamespace(attn_backend=types.SimpleNamespace(prepare_for_capture=lambda b: None), dummy_req=None, model=types.SimpleNamespace(forward=forward),
+                                ctx=types.SimpleNamespace(forward_batch=lambda b: contextlib.nullcontext()), cfg=types.SimpleNamespace(tp_size=1), stream=None)
+    runner = types.SimpleNamespace(engine=eng, input_ids=logits[0], out_loc=logits[0], positions=logits[0], logits=logits, _pool=None, graph_map={})
+    monkeypatch.setattr(E, "Batch", lambda **k: types.SimpleNamespace(**k))
+    old = gc.get_threshold()
+    gc.set_threshold(1, 1, 1)
+    try:
+        E.GraphRunner.capture(runner, 1)
+        assert gc.isenabled()
+    finally:
+        gc.set_threshold(*old)
+    gc.collect()
+    assert ended and not any(ended)
