@@ -253,7 +253,8 @@ class MixAttnBackend:
         k = np.fromiter((r.device_len for r in reqs), dtype=np.int64, count=bs)
         rows = np.fromiter((r.table_idx for r in reqs), dtype=np.int64, count=bs)
         # a long portion's recurrence runs as pieces in parallel (their states joined by a scan): RECURRENT_CHUNK tokens for the
-        # decay-only recurrence, DELTA_CHUNK for the delta rule, whose scan step is a [d, d] x [d, dv] product per piece
+        # decay-only recurrence, DELTA_CHUNK for the delta rule, whose scan step is a [d, d] x [d, dv] product per piece (head sizes that
+        # have no form in blocks; the others' long portions go without the list)
         lists = []
         if int(q.max()) >= 2 * self.RECURRENT_CHUNK and self._kinds & {"lightning"}:
             lists.append(("chunks", self.RECURRENT_CHUNK))

@@ -138,7 +138,6 @@ __device__ __forceinline__ Q4 load8(const float* p, int n, bool vec) {
             bf16_bits(f[4]) | (bf16_bits(f[5]) << 16), bf16_bits(f[6]) | (bf16_bits(f[7]) << 16)};
 }
 
-// two fp32 numbers as packed bf16 (round to nearest even), one instruction
 // the larger of this lane's number and lane ^ 32's, without LDS: a swap of halves between two copies leaves both numbers in every lane
 __device__ __forceinline__ float pair_max(float x) {
   const uint32_t a = __builtin_bit_cast(uint32_t, x);
@@ -147,6 +146,7 @@ __device__ __forceinline__ float pair_max(float x) {
   return fmaxf(__builtin_bit_cast(float, y0), __builtin_bit_cast(float, y1));
 }
 
+// two fp32 numbers as packed bf16 (round to nearest even), one instruction
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {

@@ -14,10 +14,10 @@
 // split by the highest bit in which t and j differ, and per level both factors are running products inside a half block.
 //
 // What bounds it: the walk is a serial chain of blocks per (request, head), 50 fp32 MFMAs of 32 cycles a wave and block plus the meeting in
-// LDS (1.5 us a block measured); the block kernel is bound by its instructions (5 waves per SIMD of them at a time) and by memory (49 d + 256 +
+// LDS (1.4 us a block measured); the block kernel is bound by its instructions (5 waves per SIMD of them at a time) and by memory (49 d + 256 +
 // 16 dv floats a block and head written, and read again by the walk).  The token loop was bound by one wave's serial walk: two passes over
 // 128 registers a token, in three launches.
-// 4 requests of 1500 - 2548 tokens, 16 heads, d = dv = 128, decays per channel: 4038 -> 390 us (blocks 177, walk 240); error against 64
+// 4 requests of 1500 - 2548 tokens, 16 heads, d = dv = 128, decays per channel: 4038 -> 389 us (blocks 171, walk 219); error against 64
 // bits 1.9e-7 -> 1.4e-7.
 #include <type_traits>
 
