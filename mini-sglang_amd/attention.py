@@ -238,7 +238,10 @@ class MixAttnBackend:
         self._cap: Optional[torch.Tensor] = None
         self._kinds = {getattr(s, "kind", "") for s in getattr(config, "layers", ())}
         self._decay_heads = max((s.heads for s in getattr(config, "layers", ()) if getattr(s, "kind", "") in ("retention", "gla")), default=0)
-        self._kinds |= {getattr(p, "kind", "") for s in getattr(config, "layers", ()) for p in (getattr(s, "left", None), getattr(s, "right", None)) if p}
+        parts = [p for s in getattr(config, "layers", ()) for p in (getattr(s, "left", None), getattr(s, "right", None)) if p]
+        self._kinds |= {getattr(p, "kind", "") for p in parts}
+        self._delta_pieces = any(not _lib.mix_lib().msgl_mix_delta_rule_block_floats(s.dim, s.vdim) for s in [*getattr(config, "layers", ()), *parts]
+                                 if getattr(s, "kind", "") in ("delta", "channel_delta"))
 
     @staticmethod
     def decay_chunk(tokens: int, heads: int) -> int:
@@ -254,11 +257,11 @@ class MixAttnBackend:
         rows = np.fromiter((r.table_idx for r in reqs), dtype=np.int64, count=bs)
         # a long portion's recurrence runs as pieces in parallel (their states joined by a scan): RECURRENT_CHUNK tokens for the
         # decay-only recurrence, DELTA_CHUNK for the delta rule, whose scan step is a [d, d] x [d, dv] product per piece (head sizes that
-        # have no form in blocks; the others' long portions go without the list)
+        # have no form in blocks; the others take the blocks for any portion of that length and read no list)
         lists = []
         if int(q.max()) >= 2 * self.RECURRENT_CHUNK and self._kinds & {"lightning"}:
             lists.append(("chunks", self.RECURRENT_CHUNK))
-        if int(q.max()) >= 2 * self.DELTA_CHUNK and self._kinds & {"delta", "channel_delta"}:
+        if self._delta_pieces and int(q.max()) >= 2 * self.DELTA_CHUNK:
             lists.append(("delta_chunks", self.DELTA_CHUNK))
         if int(q.max()) >= 2 * self.SSD_CHUNK and "state_space" in self._kinds:
             lists.append(("ssd_chunks", self.SSD_CHUNK))

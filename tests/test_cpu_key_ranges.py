@@ -104,3 +104,25 @@ def test_delta_rule_blocks_where_they_are_faster():
     assert delta_in_blocks(40, 640, 16, 64, False)  # many requests that may hide a long portion
     assert delta_in_blocks(16, 95, 16, 128, False, longest=80) and not delta_in_blocks(16, 95, 16, 128, False)
     assert not delta_in_blocks(64, 384, 16, 128, False, longest=6) and not delta_in_blocks(64, 64, 16, 64, True, longest=1)
+
+
+def test_delta_rule_pieces_where_the_token_loop_takes_long_portions(monkeypatch):
+    """The list of a long portion's pieces is built for head sizes that have no form in blocks, and for no other: they read none at that length."""
+    from types import SimpleNamespace as N
+
+    from mini_sglang_amd import attention, mixops
+
+    empty = torch.empty
+    monkeypatch.setattr(attention.torch, "empty", lambda *a, pin_memory=False, **kw: empty(*a, **kw))
+    ctx = N(kv_cache=N(device=torch.device("cpu")), page_table=torch.zeros((4, 2048), dtype=torch.int32))
+    n = 2 * attention.MixAttnBackend.DELTA_CHUNK
+    for dim, vdim, kind, want in [(128, 128, "delta", False), (64, 96, "channel_delta", False), (64, 80, "delta", True), (96, 96, "channel_delta", True)]:
+        layer = N(kind=kind, dim=dim, vdim=vdim)
+        for layers in ([layer], [N(kind="parallel", left=N(kind="window"), right=layer)]):
+            batch = N(padded_reqs=[N(extend_len=k, device_len=k + 5, table_idx=i) for i, k in enumerate((1, n, 7))])
+            attention.MixAttnBackend(N(layers=layers), ctx).prepare_metadata(batch)
+            md = batch.attn_metadata
+            assert (md.delta_chunks is not None) == want and (want or mixops.delta_in_blocks(3, n + 8, 16, dim, kind == "channel_delta", md.max_seqlen_q))
+            if want:
+                items, first, count = md.delta_chunks
+                assert count == 4 and items.view(-1, 3).tolist() == [[0, 0, 1], [1, 0, n // 2], [1, n // 2, n], [2, 0, 7]] and first.tolist() == [0, 1, 3, 4]
