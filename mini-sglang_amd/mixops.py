@@ -206,11 +206,12 @@ def moe_sort(ids: torch.Tensor, experts: int):
     """-> (segment offsets int32 [E + 1], permutation int32 [T * top])."""
     _dev(ids)
     n = ids.numel()
-    seg = torch.empty(2 * experts + 1, dtype=torch.int32, device=ids.device)  # offsets, then the per-expert counts (scratch)
+    seg = torch.empty(experts + 1, dtype=torch.int32, device=ids.device)
     perm = torch.empty(max(n, 1), dtype=torch.int32, device=ids.device)
-    check_mix(mix_lib().msgl_mix_moe_sort(seg.data_ptr(), perm.data_ptr(), seg[experts + 1:].data_ptr(), _i32(ids).data_ptr(), n,
-                                          experts, _stream()), "moe_sort")
-    return seg[: experts + 1], perm
+    # (the third pointer, once a place for counts, is not used)
+    check_mix(mix_lib().msgl_mix_moe_sort(seg.data_ptr(), perm.data_ptr(), seg.data_ptr(), _i32(ids).data_ptr(), n, experts, _stream()),
+              "moe_sort")
+    return seg, perm
 
 
 def gemm_nt(C: torch.Tensor, A: torch.Tensor, B: torch.Tensor, M: int, N: int, K: int, *, lda: int, ldb: int, ldc: int,
