@@ -507,6 +507,7 @@ def _refine_reference_graphs(gr: Any, model: Any) -> List[dict]:
 
     from minisgl.core import Batch, Req, get_global_ctx
 
+    from .engine import _no_collection
     from .plan_refine import refine_plans_in_graph
 
     ctx, bs = get_global_ctx(), gr.max_graph_bs
@@ -522,7 +523,7 @@ def _refine_reference_graphs(gr: Any, model: Any) -> List[dict]:
         gr.buffer.set_batch(batch)
         with ctx.forward_batch(batch):
             gr.buffer.logits[:bs] = model.forward()
-            with torch.cuda.graph(graph, pool=pool, stream=gr.stream):
+            with _no_collection(), torch.cuda.graph(graph, pool=pool, stream=gr.stream):
                 gr.buffer.logits[:bs] = model.forward()
         gr.graph_map[bs] = graph
 

@@ -264,3 +264,37 @@ def test_no_garbage_is_collected_inside_a_capture(monkeypatch):
         gc.set_threshold(*old)
     gc.collect()
     assert ended and not any(ended)
+
+
+def test_no_garbage_is_collected_while_plans_are_captured_again(monkeypatch):
+    """The same of the capture that re-ranks plans inside the reference engine's graph: the collector is off in it and on behind it."""
+    import contextlib
+    import gc
+    import sys
+    import types
+
+    import torch
+
+    from mini_sglang_amd import minisgl_plugin, plan_refine
+
+    inside = []
+
+    @contextlib.contextmanager
+    def capture(*_a, **_k):
+        inside.append(gc.isenabled())
+        yield
+
+    ctx = types.SimpleNamespace(forward_batch=lambda b: contextlib.nullcontext(), page_table=torch.zeros(1, 4), page_size=1,
+                                kv_cache=types.SimpleNamespace(k_cache=lambda i: torch.zeros(3)))
+    core = types.ModuleType("minisgl.core")
+    core.Batch, core.Req, core.get_global_ctx = lambda **k: types.SimpleNamespace(**k), None, lambda: ctx
+    monkeypatch.setitem(sys.modules, "minisgl", types.ModuleType("minisgl"))
+    monkeypatch.setitem(sys.modules, "minisgl.core", core)
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", object)
+    monkeypatch.setattr(torch.cuda, "graph", capture)
+    monkeypatch.setattr(plan_refine, "refine_plans_in_graph", lambda capture, **_k: capture())
+    backend = types.SimpleNamespace(prepare_for_capture=lambda b: None, prepare_metadata=None)
+    runner = types.SimpleNamespace(max_graph_bs=1, graph_map={1: types.SimpleNamespace(pool=lambda: None)}, dummy_req=None, attn_backend=backend, replay=None, device=None,
+                                   buffer=types.SimpleNamespace(set_batch=lambda b: None, logits=torch.zeros(1, 4)), stream=None)
+    minisgl_plugin._refine_reference_graphs(runner, types.SimpleNamespace(forward=lambda: torch.zeros(1, 4)))
+    assert inside == [False] and gc.isenabled()
