@@ -529,6 +529,7 @@ __device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64
   if (has_k) {
     // fewer than k positive probabilities (a low temperature underflows the tail to 0): top-k keeps all of them,
     // as flashinfer does -- no threshold; ties at the k-th largest value stay in the keep set
+    // (such a row comes here past its list: 64 rows x 151936 at temperature 0.02, k 1000: 100 us, 295 over stored probabilities)
     const uint32_t v = select_bits<false>(src, vocab, 0u, (u64)k, h_cnt, h_mass, lds_w, &s_digit);
     if (v != kNoDigit) thr_bits = v;
   }
