@@ -6,6 +6,7 @@ true 32-bit mode) and, for shapes the library has no solution for, the grouped k
 """
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -389,6 +390,12 @@ def window_portion_splits(batch: int, total_q: int, window: int, max_keys: int, 
     return max(1, min(256 // groups, -(-keys // (128 if matrix else 64)), 8)) if 0 < groups <= 128 else 1
 
 
+@lru_cache(maxsize=64)
+def _window_on_matrix_cores(H: int, G: int, d: int, dv: int, code: int) -> bool:
+    """The kernel library's own rule, a function of the sizes (asked once: 2 us a call, and a decode step's launch takes 15)."""
+    return bool(mix_lib().msgl_mix_window_attn_on_matrix_cores(H, G, d, dv, code))
+
+
 def window_attn(out: torch.Tensor, src: torch.Tensor, g_off: int, k_cache: torch.Tensor, v_cache: torch.Tensor, table: torch.Tensor,
                 req_rows: torch.Tensor, seq_lens: torch.Tensor, cu_q: torch.Tensor, batch: int, H: int, G: int, d: int, dv: int,
                 window: int, scale: float, talk: torch.Tensor, splits: int = 1, max_keys: Optional[int] = None) -> None:
@@ -405,7 +412,7 @@ def window_attn(out: torch.Tensor, src: torch.Tensor, g_off: int, k_cache: torch
     assert req_rows.numel() >= batch and seq_lens.numel() >= batch and cu_q.numel() >= batch + 1
     if splits == 1:
         splits = window_portion_splits(batch, T, window, table.shape[1] if max_keys is None else max_keys,
-                                       bool(mix_lib().msgl_mix_window_attn_on_matrix_cores(H, G, d, dv, _code(src))))
+                                       _window_on_matrix_cores(H, G, d, dv, _code(src)))
     ws = None
     if splits > 1:
         ws = torch.empty(mix_lib().msgl_mix_window_attn_workspace_floats(T, H, dv, splits), dtype=torch.float32, device=out.device)
@@ -433,6 +440,10 @@ def short_conv(src: torch.Tensor, C: int, taps: torch.Tensor, state: Optional[to
     return out
 
 
+# new tokens per request from which on blocks are faster, up to 128 walks and beyond, by head size and kind of decay (0 / 1: per channel)
+_DELTA_BLOCK_TOKENS = {(128, 0): (6, 8), (128, 1): (6, 6), (64, 0): (10, 28), (64, 1): (6, 13)}
+
+
 def delta_in_blocks(batch: int, total_q: int, H: int, d: int, per_channel: bool, longest: Optional[int] = None) -> bool:
     """Blocks of 16 tokens on the matrix instructions (two launches, 14 us however short the portions are, and more for every further request
     and head), or token by token (a token of the longest portion: 2.2 us at d = 128, 4.4 with a decay per channel, 1.0 and 1.7 at d = 64).
@@ -441,9 +452,7 @@ def delta_in_blocks(batch: int, total_q: int, H: int, d: int, per_channel: bool,
     26 / 31, 40 x 16 39 / 56, 64 x 24 89 / 89; per channel 1 x 6 17.5 / 16.2, 16 x 8 23 / 28, 16 x 16 38 / 31, 64 x 12 68 / 69.  One long portion
     among single tokens: 16 requests, one of 80 tokens, 196 us token by token and 47 in blocks; where the longest is not known, only many
     tokens speak for one."""
-    wide = batch * H > 128  # every further (request, head) is a walk of its own
-    need = {(128, False): (6, 8), (128, True): (6, 6), (64, False): (10, 28), (64, True): (6, 13)}.get((d, bool(per_channel)), (6, 12))[wide]
-    if total_q >= need * batch:
+    if total_q >= _DELTA_BLOCK_TOKENS.get((d, bool(per_channel)), (6, 12))[batch * H > 128] * batch:  # every further (request, head) is a walk of its own
         return True
     return longest >= 40 if longest is not None else batch * H > 256 and total_q - batch >= 256
 
