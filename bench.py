@@ -40,6 +40,19 @@ HBM_PEAK_GBPS = 8000.0  # MI355X_MICROARCH.md: 8.0 TB/s spec (6.29 TB/s measured
 METRIC = "decode tokens/s/GPU + p50 TTFT, Qwen3-14B TP=1 and Qwen3-32B TP=4"
 
 
+def result_line(result: dict) -> str:
+    """The result as one line that a reader of stdout's last 8000 characters has whole: numbers behind the first level in six digits, recorded results
+    as their files' names and headline numbers."""
+    def short(x):
+        if isinstance(x, dict):
+            return {k: short(v) for k, v in x.items()}
+        if isinstance(x, (list, tuple)):
+            return [short(v) for v in x]
+        return float(f"{x:.6g}") if isinstance(x, float) else x
+
+    return json.dumps({k: v if isinstance(v, float) else short(v) for k, v in result.items()}, separators=(",", ":"))
+
+
 def product_code_fingerprint() -> str:
     """sha256 over the product's sources (kernels, host C++, package Python, the C header): a number recorded under profiles/
     by another process (the reference-driven step time) carries the fingerprint of the code that produced it, and this file
@@ -615,18 +628,12 @@ def run_workload(args, model_name: str, rank: int, local_rank: int, world: int, 
     if primary:
         result["gemm_tune"] = {
             "mode": ecfg.gemm_tune,
-            "shapes": [dict(name=r["name"], M=r["M"], N=r["N"], K=r["K"], heuristic_us=round(r["default_us"], 1),
-                            tuned_us=round(r["best_us"], 1), candidates=r["tried"],
-                            tflops=round(2.0 * r["M"] * r["N"] * r["K"] / r["best_us"] / 1e6, 1),
-                            weight_TBps=round(2.0 * r["N"] * r["K"] / r["best_us"] / 1e6, 2),
-                            **({"hand_written": r["kernel"], "library_best_us": round(r["library_best_us"], 1)}
-                               if r.get("skinny_used") else {}),
-                            **({"fold_credit_us": r["fold_credit_us"]} if r.get("fold_credit_us") else {}),
-                            **({"projection_then_silu_us": round(r["silu_unfused_us"], 1),
-                                "fused_silu_epilogue_us": round(r["silu_fused_us"], 1), "fused_silu_used": r["silu_fused_used"]}
-                               if r.get("silu_fused_us") else {})) for r in engine.gemm_report],
+            "columns": "us: the library's heuristic, the library's best, the chosen plan; its kernel if hand-written",
+            "shapes": {f"{r['name']} {r['M']}x{r['N']}x{r['K']}": [round(r["default_us"], 1), round(r["library_best_us"] if r.get("skinny_used") else r["best_us"], 1),
+                                                                   round(r["best_us"], 1)] +
+                       ([r["kernel"].replace("msgl::", "").split("[")[0]] if r.get("skinny_used") else []) for r in engine.gemm_report},
         }
-        result["gemm_tune"]["refined_in_graph"] = getattr(engine, "refine_report", [])
+        result["gemm_tune"]["refined_in_graph"] = {f"{r['name']} {r['M']}": r["chosen"] for r in getattr(engine, "refine_report", [])}
     else:
         result["gemm_plans_at_full_batch"] = {r["name"]: dict(us=round(r["best_us"], 1), kernel=r["kernel"][:70]) for r in full}
     engine.shutdown()  # raises if a peer-to-peer barrier ever timed out (NaN-poisoned collectives)
@@ -819,20 +826,17 @@ def main() -> None:
             except Exception:
                 continue
             if "scales" in d and d.get("model"):
-                replays[d["model"]] = {"kind": "committed", "source": f"profiles/{f.name}", "cache": d.get("cache"), "tp": d.get("tp"),
-                                       "trace": d.get("trace"), "recorded_on_code": d.get("code_fingerprint"), "this_code": fp,
+                replays[d["model"]] = {"kind": "committed", "source": f"profiles/{f.name}", "recorded_on_code": d.get("code_fingerprint"),
                                        "stale": d.get("code_fingerprint") != fp,
-                                       "by_scale": {k: {"complete": v["complete"], "throughput_tok_s": v["throughput_tok_s"],
-                                                        "ttft_ms": {q: v["ttft_ms"][q] for q in ("p50", "p90", "p99")},
-                                                        "tpot_ms": {q: v["tpot_ms"][q] for q in ("p50", "p90", "p99")}}
-                                                    for k, v in d["scales"].items()}}
+                                       "throughput_tok_s_by_scale": {k: v["throughput_tok_s"] if v["complete"] else None for k, v in d["scales"].items()}}
         if replays:
             result["online_trace_replay"] = replays
         # what the GPU parity suite compared on its last committed run (tests/parity_stats.py -> profiles/r*_parity_summary.json)
         par = sorted((ROOT / "profiles").glob("r*_parity_summary.json"))
         if par:
             try:
-                result["parity"] = dict(json.loads(par[-1].read_text()), kind="committed", source=f"profiles/{par[-1].name}")
+                result["parity"] = {"bit_identical_forwards": json.loads(par[-1].read_text()).get("bit_identical_forwards"), "kind": "committed",
+                                    "source": f"profiles/{par[-1].name}"}
             except Exception as e:
                 result["parity"] = {"error": f"{type(e).__name__}: {e}"}
     if rank == 0 and world == 1 and not args.no_e2e:
@@ -840,6 +844,7 @@ def main() -> None:
         # generate() over 256 requests, in/out 100..1024, prefill included, one untimed warm-up -- BASELINE configs 1, 2
         from tools.offline_bench import run as offline_run
 
+        print("[bench] step measured", file=sys.stderr, flush=True)  # the whole runs below say nothing for two minutes
         result["e2e_offline"] = {}
         for name in (["qwen3-0.6b"] + ([args.model] if args.model != "qwen3-0.6b" else [])):
             try:
@@ -849,6 +854,7 @@ def main() -> None:
                                                                  "ttft_p50_ms")}
             except Exception as e:
                 result["e2e_offline"][name] = {"error": f"{type(e).__name__}: {e}"}
+            print(f"[bench] {name} measured", file=sys.stderr, flush=True)
         # the reference's DEFAULT page size (P/engine/config.py:25: page_size = 1; its FlashInfer backend always sees token-granular
         # tables, P/attention/fi.py:179-187): the same workload on a token-granular pool (round 6: the matrix-core decode kernel
         # gathers token rows by per-lane addresses)
@@ -882,7 +888,7 @@ def main() -> None:
             "reference_driven_ms": (result.get("reference_driven") or {}).get("decode_ms_per_step"),
             "reference_driven_stale": (result.get("reference_driven") or {}).get("stale"),
         }
-        print(json.dumps(result), flush=True)
+        print(result_line(result), flush=True)
     if world > 1:
         dist.destroy_process_group()
 

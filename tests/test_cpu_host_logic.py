@@ -298,3 +298,13 @@ def test_no_garbage_is_collected_while_plans_are_captured_again(monkeypatch):
                                    buffer=types.SimpleNamespace(set_batch=lambda b: None, logits=torch.zeros(1, 4)), stream=None)
     minisgl_plugin._refine_reference_graphs(runner, types.SimpleNamespace(forward=lambda: torch.zeros(1, 4)))
     assert inside == [False] and gc.isenabled()
+
+
+def test_benchmark_line_keeps_the_headline_numbers():
+    """The line is JSON again with the first level's numbers as they are, those behind it in six digits."""
+    import json
+
+    import bench
+
+    line = bench.result_line({"value": 14843.764966979887, "ms_per_step": 17.1, "steps": 20, "config": {"batch": 256, "x": [1.23456789, None, "t"]}})
+    assert "\n" not in line and json.loads(line) == {"value": 14843.764966979887, "ms_per_step": 17.1, "steps": 20, "config": {"batch": 256, "x": [1.23457, None, "t"]}}
