@@ -277,6 +277,14 @@ int msgl_sample_filtered_logits(int32_t* out, const void* logits, const float* t
 int msgl_sample_filtered_logits_keep(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
                                      const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
                                      int logits_dtype, uint64_t seed, uint64_t offset, void* stream);
+/* The same with a workspace of msgl_sample_workspace_bytes(rows, vocab, 1, top_k != NULL, top_p != NULL) bytes (16-byte aligned, contents arbitrary
+ * before and after; NULL: as above): several workgroups share a row, same picks.  kept may be NULL. */
+int msgl_sample_filtered_logits_ws(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
+                                   const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
+                                   int logits_dtype, uint64_t seed, uint64_t offset, void* workspace, int64_t workspace_bytes, void* stream);
+/* Bytes of the workspace above (filtered = 1) or of msgl_sample_from_logits_ws (filtered = has_k = has_p = 0);
+ * 0 where one workgroup per row is as good and none is used. */
+int64_t msgl_sample_workspace_bytes(int64_t rows, int64_t vocab, int filtered, int has_k, int has_p);
 /* Sample one token per row straight from logits: index ~ softmax(logits[r, :] / temperature[r]), no
  * top-k / top-p filter, probabilities never materialised (the fused form of the reference's
  * softmax -> sampling_from_probs pair, P/engine/sample.py:24-44).  Rows 16-byte aligned.
@@ -284,6 +292,10 @@ int msgl_sample_filtered_logits_keep(int32_t* out, void* kept, float* kept_tempe
 int msgl_sample_from_logits(int32_t* out, const void* logits, const float* temperatures, int64_t rows,
                             int64_t vocab, int64_t logits_stride, int logits_dtype, uint64_t seed,
                             uint64_t offset, void* stream);
+/* The same with a workspace of msgl_sample_workspace_bytes(rows, vocab, 0, 0, 0) bytes: several workgroups share a row, same picks. */
+int msgl_sample_from_logits_ws(int32_t* out, const void* logits, const float* temperatures, int64_t rows, int64_t vocab,
+                               int64_t logits_stride, int logits_dtype, uint64_t seed, uint64_t offset, void* workspace,
+                               int64_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
  * Weight-streaming projection GEMM for small decode batches (1 <= M <= 64):

@@ -73,7 +73,10 @@ HIP_SIGNATURES = {
     "msgl_sample_top_k_top_p": (_i, [_p, _p, _p, _p, _l, _l, _l, _u64, _u64, _p]),
     "msgl_sample_filtered_logits": (_i, [_p, _p, _p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p]),
     "msgl_sample_filtered_logits_keep": (_i, [_p, _p, _p, _p, _p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p]),
+    "msgl_sample_filtered_logits_ws": (_i, [_p, _p, _p, _p, _p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p, _l, _p]),
+    "msgl_sample_workspace_bytes": (_l, [_l, _l, _i, _i, _i]),
     "msgl_sample_from_logits": (_i, [_p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p]),
+    "msgl_sample_from_logits_ws": (_i, [_p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p, _l, _p]),
     "msgl_skinny_gemm_nt": (_i, [_p, _p, _p, _i, _i, _i, _l, _l, _l, _i, _i, _i, _p]),
     "msgl_skinny_gemm_silu_nt": (_i, [_p, _p, _p, _i, _i, _i, _l, _l, _l, _i, _i, _i, _p]),
     "msgl_rowstream_gemm_supported": (_i, [_i, _i, _i, _i, _i]),

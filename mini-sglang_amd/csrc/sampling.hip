@@ -170,14 +170,19 @@ __device__ __forceinline__ u64 block_prefix_incl(u64 v, u64* lds_w) {
   return v + base;
 }
 
-__device__ __forceinline__ u64 block_sum_u64(u64 v, u64* lds_w) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+__device__ __forceinline__ u64 wave_sum_u64(u64 v) {
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
     const uint32_t lo = __shfl_xor((uint32_t)v, d, 64);
     const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), d, 64);
     v += ((u64)hi << 32) | lo;
   }
+  return v;
+}
+
+__device__ __forceinline__ u64 block_sum_u64(u64 v, u64* lds_w) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  v = wave_sum_u64(v);
   if (lane == 0) lds_w[w] = v;
   __syncthreads();
   u64 r = 0;
@@ -212,6 +217,8 @@ struct Philox {
 
 constexpr int kBins = 2048;  // 11-bit digits; thread t owns bins 2047-2t and 2046-2t (descending)
 constexpr uint32_t kNoDigit = 0xffffffffu;
+constexpr u64 kNoMass = ~0ull;
+constexpr u64 kSure = 1ull << 63;
 constexpr int kStrip = 8;    // loads of a row in flight per thread: a pass is bound by their latency, not by bytes
 
 // What a row's probabilities come from.  raw(i): the stored number; weight(x): a number in the order of the probabilities
@@ -321,232 +328,220 @@ __device__ __forceinline__ uint32_t select_bits(const Src& src, int64_t vocab, u
   return prefix;
 }
 
-// the `target`-th largest (1-based) of the workgroup's 1024 non-negative numbers, one per thread
-__device__ __forceinline__ uint32_t kth_largest(uint32_t bits, int target, uint32_t* hist, uint32_t* s_two) {
+// A lower bound of the `target`-th largest of the workgroup's 1024 weights, one per thread: the lower end of the 16th of an octave that holds it,
+// 0 below 2^-63.  One histogram, spread over the octaves that the maxima lie in: the exact one takes four, the upper ones with all 1024 in a few bins
+// (64 rows x 151936: 5 us of a draw).
+__device__ __forceinline__ uint32_t kth_bound(uint32_t bits, int target, uint32_t* hist, uint32_t* s_one) {
+  constexpr uint32_t kLow = 64u << 23;
   const int tid = threadIdx.x;
-  uint32_t prefix = 0u, mask = 0u;
-#pragma unroll 1
-  for (int shift = 24; shift >= 0; shift -= 8) {
-    if (tid < 256) hist[tid] = 0u;
-    __syncthreads();
-    if ((bits & mask) == prefix) atomicAdd(&hist[(bits >> shift) & 255u], 1u);
-    __syncthreads();
-    if (tid < 64) {  // lane l owns the bins 255 - 4 l ... 252 - 4 l
-      int c[4], s = 0;
+  hist[tid] = 0u;
+  if (tid == 0) *s_one = 0u;
+  __syncthreads();
+  if (bits >= kLow) atomicAdd(&hist[min((bits - kLow) >> 19, 1023u)], 1u);
+  __syncthreads();
+  if (tid < 64) {  // lane l owns the bins 1023 - 16 l ... 1008 - 16 l
+    int c[16], mine = 0;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) s += c[q] = (int)hist[255 - 4 * tid - q];
-      int above = s;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int o = __shfl_up(above, d, 64);
-        if (tid >= d) above += o;
-      }
-      above -= s;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (above < target && target <= above + c[q]) {
-          s_two[0] = (uint32_t)(255 - 4 * tid - q);
-          s_two[1] = (uint32_t)above;
-        }
-        above += c[q];
-      }
+    for (int q = 0; q < 4; ++q) {
+      const uint4 h = *reinterpret_cast<const uint4*>(hist + 1020 - 16 * tid - 4 * q);
+      c[4 * q] = (int)h.w; c[4 * q + 1] = (int)h.z; c[4 * q + 2] = (int)h.y; c[4 * q + 3] = (int)h.x;
     }
-    __syncthreads();
-    prefix |= s_two[0] << shift;
-    mask |= 255u << shift;
-    target -= (int)s_two[1];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) mine += c[q];
+    int above = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_up(above, d, 64);
+      if (tid >= d) above += o;
+    }
+    above -= mine;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      if (above < target && target <= above + c[q]) *s_one = kLow + ((uint32_t)(1023 - 16 * tid - q) << 19);
+      above += c[q];
+    }
   }
   __syncthreads();
-  return prefix;
+  return *s_one;
 }
 
 constexpr int kList = 2048;          // candidates of a row that the short path holds (= kBins: it reuses the histograms)
 constexpr int kListTopK = 1024;      // largest top-k it is tried for: one column maximum per thread bounds the k-th largest from below
-// candidates asked for when only a mass is given: a list takes time with its square (512: 120 us for any row of 32000, 62 without a list), and a
-// nucleus that does not fit pays for it on top (bf16 rows, top-p 0.9, one row of 151936: nucleus 8: 55 us with 64, 91 with 256, 157 with 512, 219
-// without; nucleus 2127: 141, 185, 225, 217)
+// candidates asked for when only a mass is given: a list takes time with its square, and a nucleus that does not fit pays for it on top (bf16 rows,
+// top-p 0.9, one row of 151936, one thread a candidate: nucleus 8: 55 us with 64, 91 with 256, 157 with 512, 219 without; nucleus 2127: 141, 185,
+// 225, 217)
 constexpr int kListTopP = 64;
-constexpr uint32_t kTinyWeight = 0x17800000u;  // 2^-80: below it two weights apart may be one probability (denormal)
 
-// One 1024-thread workgroup per row.
-//
-// Short path (any top-k up to 1024, or a top-p whose nucleus is small): thread t's largest number over the columns t, t + 1024, ...
-// is known after one pass; the k-th largest of these 1024 maxima has at least k numbers at or above it, so the second pass collects
-// only what reaches it -- some k numbers out of a 152 k vocabulary -- and both thresholds and the draw are integer sums over that
-// list.  The general path finds the same thresholds by three radix levels over the whole row; it stays for wide nuclei, top-k above
-// 1024 and rows whose largest numbers share a column.
-//
-// Bound: one CU walks one row (304 KB of bf16 logits) twice, an exponential and ~10 VALU operations per element in the second pass.
-// 64 rows x 151936 bf16 logits, top-k and top-p: softmax_kernel + radix levels over the stored fp32 probabilities (ten passes, u64 LDS
-// atomics for every element of a first level) 551 us; this kernel from the logits 49 us.
+struct __attribute__((aligned(16))) RowShared {
+  uint32_t h_cnt[kBins];  // histogram | candidates' probability bits
+  u64 h_mass[kBins];      // histogram | candidates' masses
+  int s_index[kList];
+  u64 acc[kRowThreads];          // sums per candidate
+  uint32_t acc_n[kRowThreads / 2];
+  u64 lds_w[kRowThreads / 64];
+  float lds_f[kRowThreads / 64];
+  uint32_t s_digit, s_two[2];
+  int s_pick, s_n;
+};
+
+__device__ __forceinline__ u64 mass_target(float pp, u64 kept_mass) {
+  u64 target = (u64)((double)pp * (double)kept_mass);
+  if (target < 1) target = 1;
+  if (target > kept_mass) target = kept_mass;
+  return target;
+}
+
+// Philox's number of row r, scaled to [0, total): (total * x) >> 32 without 128-bit arithmetic
+__device__ __forceinline__ u64 draw_below(u64 total, u64 seed, u64 ctr) {
+  const uint32_t x = Philox::draw(seed, ctr);
+  return (total >> 32) * (u64)x + (((total & 0xffffffffull) * (u64)x) >> 32);
+}
+
+// The draw where the list (n candidates, their weights' bits in h_cnt) holds all that it needs; false where the threshold lies below the
+// list.  kept_mass: set to the whole row's mass where only a mass is given.  s_pick is -1 on entry.
 template <class Src>
-__device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64_t k, float pp, int64_t vocab, float inv_t, u64 seed, u64 offset) {
-  __shared__ uint32_t h_cnt[kBins];  // histogram | candidates' probability bits
-  __shared__ u64 h_mass[kBins];      // histogram | candidates' masses
-  __shared__ int s_index[kList];
-  __shared__ u64 lds_w[kRowThreads / 64];
-  __shared__ float lds_f[kRowThreads / 64];
-  __shared__ uint32_t s_digit, s_two[2];
-  __shared__ int s_pick, s_n;
+__device__ __forceinline__ bool draw_from_list(const Src& src, RowShared& sh, int* __restrict__ out, int n, uint32_t floor_bits, bool by_count, int64_t k,
+                                               float pp, int64_t vocab, u64 seed, u64 offset, u64& kept_mass) {
   const int tid = threadIdx.x;
-  const int64_t r = blockIdx.x;
-  const bool has_k = k >= 1 && k < vocab;
-  const bool by_count = has_k && k <= kListTopK, by_mass = !has_k && pp < 1.0f;
-
-  uint32_t thr_bits = 0u;  // keep set = { bits >= thr_bits, p > 0 }
-  u64 kept_mass = 0;
-  bool have_mass = false;  // kept_mass is that of the whole row
-  bool done = false;       // uniform: the threshold is known and every number that reaches it is in the list
-  int n = 0;
-
-  float col = Src::kSoftmax ? -INFINITY : 0.f;
-  if (Src::kSoftmax || by_count || by_mass)
-    walk_row(src, vocab, [&](int64_t, float x, bool in) { col = in ? fmaxf(col, x) : col; });
-  if constexpr (Src::kSoftmax) {
-    src.mx = block_reduce_max(col, lds_f);
-    src.k = inv_t * 1.4426950408889634f;
+  const bool by_mass = !by_count;
+  // Every candidate against every other one: `cp` candidates side by side, the others in `parts` portions whose sums meet in LDS.
+  // 64 rows, lists of some 110: two such comparisons and the rest of the draw take 24 us with one thread a candidate, 8 so.
+  constexpr int kOwn = kList / kRowThreads;
+  int cp = 64;
+  while (cp < n && cp < kRowThreads) cp *= 2;
+  const int parts = kRowThreads / cp, part = tid / cp, c0 = tid - part * cp;
+  for (int c = tid; c < n; c += kRowThreads) {
+    const float p = src.prob(__uint_as_float(sh.h_cnt[c]));
+    sh.h_mass[c] = fixed_mass(p) | (sh.h_cnt[c] >= floor_bits ? kSure : 0ull);  // kSure: not among the few below the floor, of whose equals some may be missing
+    sh.h_cnt[c] = __float_as_uint(p);
   }
-  uint32_t floor_bits = 0u, list_bits = kNoDigit;  // list_bits: what a weight has to reach to be listed
-  if (by_count || by_mass) {
-    const float w = src.weight(col);
-    const int want = (int)(by_count ? k : (int64_t)kListTopP);
-    floor_bits = kth_largest(w > 0.f ? __float_as_uint(w) : 0u, want, h_cnt, s_two);  // NaN counts as nothing here
-    // weights up to some units in the last place apart can be the same probability: the list starts a little below
-    if (floor_bits > (Src::kSoftmax ? kTinyWeight : 0u)) list_bits = floor_bits - (Src::kSoftmax ? 8u : 0u);
-  }
-  if (tid == 0) { s_n = 0; s_pick = -1; }
-  __syncthreads();
-  if (Src::kSoftmax || list_bits != kNoDigit) {
-    float sum = 0.f;
-    walk_row(src, vocab, [&](int64_t i, float x, bool in) {
-      const float w = src.weight(x);
-      if (in) sum += w;
-      const bool hit = in && w > 0.f && __float_as_uint(w) >= list_bits;
-      const u64 votes = __ballot(hit);
-      if (votes) {
-        const int lane = tid & 63;
-        int at = 0;
-        if (lane == 0) at = atomicAdd(&s_n, __popcll(votes));
-        at = __shfl(at, 0, 64) + __popcll(votes & ((1ull << lane) - 1ull));
-        if (hit && at < kList) {
-          s_index[at] = (int)i;
-          h_cnt[at] = __float_as_uint(w);
-        }
-      }
+  if (tid < kRowThreads / 2) sh.acc[tid] = sh.acc[tid + kRowThreads / 2] = sh.acc_n[tid] = 0;
+  u64 target = 0;
+  if (by_mass) {
+    u64 loc = 0;
+    walk_row(src, vocab, [&](int64_t, float x, bool in) {
+      const u64 m = fixed_mass(src.prob(src.weight(x)));
+      loc += in ? m : 0ull;
     });
-    if constexpr (Src::kSoftmax) src.inv = 1.0f / block_reduce_sum(sum, lds_f);
-    __syncthreads();
-    n = s_n;
+    kept_mass = block_sum_u64(loc, sh.lds_w);
+    target = mass_target(pp, kept_mass);
   }
-  if (list_bits != kNoDigit && n <= kList) {
-    uint32_t mine[kList / kRowThreads];
-    bool sure[kList / kRowThreads];  // not among the few below the floor, of whose equals some may be missing
+  if (tid == 0) sh.s_digit = kNoDigit;
+  __syncthreads();
+  u64 m_above[kOwn], m_same[kOwn];
+  int c_above[kOwn], c_same[kOwn];
 #pragma unroll
-    for (int e = 0; e < kList / kRowThreads; ++e) {
-      const int c = tid + e * kRowThreads;
-      sure[e] = c < n && h_cnt[c] >= floor_bits;
-      const float p = c < n ? src.prob(__uint_as_float(h_cnt[c])) : 0.f;
-      mine[e] = __float_as_uint(p);
-      if (c < n) {
-        h_cnt[c] = mine[e];
-        h_mass[c] = fixed_mass(p);
-      }
+  for (int e = 0; e < kOwn; ++e) {
+    m_above[e] = m_same[e] = 0;
+    c_above[e] = c_same[e] = 0;
+    const int c = c0 + e * kRowThreads;
+    if (c >= n || (e > 0 && cp < kRowThreads)) continue;
+    const uint32_t own = sh.h_cnt[c];
+#pragma unroll 4
+    for (int j = part; j < n; j += parts) {
+      const uint32_t b = sh.h_cnt[j];
+      const u64 m = sh.h_mass[j] & ~kSure;
+      c_above[e] += b > own;
+      c_same[e] += b == own;
+      m_above[e] += b > own ? m : 0ull;
+      m_same[e] += b == own ? m : 0ull;
     }
-    u64 target = 0;
-    if (by_mass) {
-      have_mass = true;
-      u64 loc = 0;
-      walk_row(src, vocab, [&](int64_t, float x, bool in) {
-        const u64 m = fixed_mass(src.prob(src.weight(x)));
-        loc += in ? m : 0ull;
-      });
-      kept_mass = block_sum_u64(loc, lds_w);
-      target = (u64)((double)pp * (double)kept_mass);
-      if (target < 1) target = 1;
-      if (target > kept_mass) target = kept_mass;
-    }
-    if (tid == 0) s_digit = kNoDigit;
-    __syncthreads();
-    u64 m_above[kList / kRowThreads], m_same[kList / kRowThreads];
-#pragma unroll
-    for (int e = 0; e < kList / kRowThreads; ++e) {
-      m_above[e] = m_same[e] = 0;
-      if (tid + e * kRowThreads >= n) continue;
-      int c_above = 0, c_same = 0;
-      for (int j = 0; j < n; ++j) {
-        const uint32_t b = h_cnt[j];
-        const u64 m = h_mass[j];
-        if (b > mine[e]) { ++c_above; m_above[e] += m; }
-        else if (b == mine[e]) { ++c_same; m_same[e] += m; }
-      }
-      const bool here = by_count ? c_above < k && k <= c_above + c_same : m_above[e] < target && target <= m_above[e] + m_same[e];
-      if (sure[e] && here) {  // equal candidates write equal words
-        s_digit = mine[e];
-        lds_w[0] = m_above[e] + m_same[e];
-      }
-    }
-    __syncthreads();
-    if (s_digit != kNoDigit && (by_count || kept_mass > 0)) {
-      thr_bits = s_digit;
-      kept_mass = lds_w[0];
-      done = true;
-    }
-    __syncthreads();
-    if (done && by_count && pp < 1.0f && kept_mass > 0) {
-      target = (u64)((double)pp * (double)kept_mass);
-      if (target < 1) target = 1;
-      if (target > kept_mass) target = kept_mass;
-#pragma unroll
-      for (int e = 0; e < kList / kRowThreads; ++e)
-        if (mine[e] >= thr_bits && tid + e * kRowThreads < n && m_above[e] < target && target <= m_above[e] + m_same[e]) s_digit = mine[e];
-      __syncthreads();
-      thr_bits = s_digit;
-    }
-    if (done) {  // the draw over the list, in index order
-      u64 loc = 0;
-#pragma unroll
-      for (int e = 0; e < kList / kRowThreads; ++e)
-        if (tid + e * kRowThreads < n && mine[e] >= thr_bits) loc += h_mass[tid + e * kRowThreads];
-      const u64 total = block_sum_u64(loc, lds_w);
-      const uint32_t x = Philox::draw(seed, offset + (u64)r);
-      const u64 u = (total >> 32) * (u64)x + (((total & 0xffffffffull) * (u64)x) >> 32);
-#pragma unroll
-      for (int e = 0; e < kList / kRowThreads; ++e) {
-        const int c = tid + e * kRowThreads;
-        if (c >= n || mine[e] < thr_bits) continue;
-        const int idx = s_index[c];
-        u64 before = 0;
-        for (int j = 0; j < n; ++j)
-          if (h_cnt[j] >= thr_bits && s_index[j] < idx) before += h_mass[j];
-        if (u >= before && u < before + h_mass[c]) s_pick = idx;
-      }
-      __syncthreads();
-      if (tid == 0) out[r] = s_pick < 0 ? 0 : s_pick;
-      return;
+    if (parts > 1) {
+      atomicAdd(&sh.acc[c], m_above[e]);
+      atomicAdd(&sh.acc[cp + c], m_same[e]);
+      atomicAdd(&sh.acc_n[c], (uint32_t)c_above[e] | (uint32_t)c_same[e] << 16);
     }
   }
+  if (parts > 1) {
+    __syncthreads();
+    m_above[0] = sh.acc[c0];
+    m_same[0] = sh.acc[cp + c0];
+    c_above[0] = (int)(sh.acc_n[c0] & 0xffffu);
+    c_same[0] = (int)(sh.acc_n[c0] >> 16);
+  }
+#pragma unroll
+  for (int e = 0; e < kOwn; ++e) {
+    const int c = c0 + e * kRowThreads;
+    if (c >= n || (e > 0 && cp < kRowThreads)) continue;
+    const bool here = by_count ? c_above[e] < k && k <= c_above[e] + c_same[e] : m_above[e] < target && target <= m_above[e] + m_same[e];
+    if ((sh.h_mass[c] & kSure) && here) {  // equal candidates write equal words
+      sh.s_digit = sh.h_cnt[c];
+      sh.lds_w[0] = m_above[e] + m_same[e];
+    }
+  }
+  __syncthreads();
+  const uint32_t found = sh.s_digit;
+  const u64 found_mass = sh.lds_w[0];
+  __syncthreads();
+  if (found == kNoDigit || (by_mass && kept_mass == 0)) return false;
+  uint32_t thr_bits = found;
+  if (by_count && pp < 1.0f && found_mass > 0) {
+    target = mass_target(pp, found_mass);
+#pragma unroll
+    for (int e = 0; e < kOwn; ++e) {
+      const int c = c0 + e * kRowThreads;
+      if (c < n && (e == 0 || cp == kRowThreads) && sh.h_cnt[c] >= thr_bits && m_above[e] < target && target <= m_above[e] + m_same[e])
+        sh.s_digit = sh.h_cnt[c];
+    }
+    __syncthreads();
+    thr_bits = sh.s_digit;
+  }
+  // the draw over the list, in index order
+  u64 loc = 0;
+  for (int c = tid; c < n; c += kRowThreads) {
+    const u64 m = sh.h_cnt[c] >= thr_bits ? sh.h_mass[c] & ~kSure : 0ull;  // what is left out weighs nothing from here on
+    sh.h_mass[c] = m;
+    loc += m;
+  }
+  sh.acc[tid] = 0;
+  const u64 total = block_sum_u64(loc, sh.lds_w);
+  const u64 u = draw_below(total, seed, offset + blockIdx.x);
+#pragma unroll
+  for (int e = 0; e < kOwn; ++e) {
+    const int c = c0 + e * kRowThreads;
+    if (c >= n || (e > 0 && cp < kRowThreads)) continue;
+    const int idx = sh.s_index[c];
+    u64 before = 0;
+#pragma unroll 4
+    for (int j = part; j < n; j += parts) before += sh.s_index[j] < idx ? sh.h_mass[j] : 0ull;
+    if (parts > 1) atomicAdd(&sh.acc[c], before);
+    else if (u >= before && u < before + sh.h_mass[c]) sh.s_pick = idx;
+  }
+  __syncthreads();
+  if (parts > 1) {
+    if (tid < n && u >= sh.acc[tid] && u < sh.acc[tid] + sh.h_mass[tid]) sh.s_pick = sh.s_index[tid];
+    __syncthreads();
+  }
+  if (tid == 0) out[blockIdx.x] = sh.s_pick < 0 ? 0 : sh.s_pick;
+  return true;
+}
 
+// The draw by three radix levels over the whole row and a walk in index order.  kept_mass: the whole row's, where it is known.
+template <class Src>
+__device__ __forceinline__ void draw_from_row(const Src& src, RowShared& sh, int* __restrict__ out, int64_t k, float pp, int64_t vocab, u64 seed, u64 offset,
+                                              u64 kept_mass) {
+  const int tid = threadIdx.x;
+  const bool has_k = k >= 1 && k < vocab;
+  uint32_t thr_bits = 0u;  // keep set = { bits >= thr_bits, p > 0 }
   if (has_k) {
     // fewer than k positive probabilities (a low temperature underflows the tail to 0): top-k keeps all of them,
     // as flashinfer does -- no threshold; ties at the k-th largest value stay in the keep set
     // (such a row comes here past its list: 64 rows x 151936 at temperature 0.02, k 1000: 100 us, 295 over stored probabilities)
-    const uint32_t v = select_bits<false>(src, vocab, 0u, (u64)k, h_cnt, h_mass, lds_w, &s_digit);
+    const uint32_t v = select_bits<false>(src, vocab, 0u, (u64)k, sh.h_cnt, sh.h_mass, sh.lds_w, &sh.s_digit);
     if (v != kNoDigit) thr_bits = v;
   }
   if (pp < 1.0f) {
-    if (!have_mass) {
+    if (kept_mass == kNoMass) {
       u64 loc = 0;
       walk_row(src, vocab, [&](int64_t, float x, bool in) {
         const float p = src.prob(src.weight(x));
         if (in && __float_as_uint(p) >= thr_bits) loc += fixed_mass(p);
       });
-      kept_mass = block_sum_u64(loc, lds_w);
+      kept_mass = block_sum_u64(loc, sh.lds_w);
     }
-    u64 target = (u64)((double)pp * (double)kept_mass);
-    if (target < 1) target = 1;
-    if (target > kept_mass) target = kept_mass;
+    const u64 target = mass_target(pp, kept_mass);
     if (kept_mass > 0) {
-      const uint32_t v = select_bits<true>(src, vocab, thr_bits, target, h_cnt, h_mass, lds_w, &s_digit);
+      const uint32_t v = select_bits<true>(src, vocab, thr_bits, target, sh.h_cnt, sh.h_mass, sh.lds_w, &sh.s_digit);
       if (v != kNoDigit) thr_bits = v > thr_bits ? v : thr_bits;  // (target <= kept_mass, so a value exists)
     }
   }
@@ -578,16 +573,14 @@ __device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64
     wave_mass += ((u64)h << 32) | l;
   }
   __syncthreads();
-  if (lane == 0) lds_w[w] = wave_mass;
+  if (lane == 0) sh.lds_w[w] = wave_mass;
   __syncthreads();
   u64 total = 0, before = 0;
   for (int i = 0; i < kWaves; ++i) {
-    if (i < w) before += lds_w[i];
-    total += lds_w[i];
+    if (i < w) before += sh.lds_w[i];
+    total += sh.lds_w[i];
   }
-  const uint32_t x = Philox::draw(seed, offset + (u64)r);
-  // u in [0, total): (total * x) >> 32 without 128-bit arithmetic
-  const u64 u = (total >> 32) * (u64)x + (((total & 0xffffffffull) * (u64)x) >> 32);
+  const u64 u = draw_below(total, seed, offset + blockIdx.x);
   if (total > 0 && u >= before && u < before + wave_mass) {  // exactly one wave
     u64 run = before;
     // strips of 8 x 64 indices: their sum first, the indices one by one only in the strip that holds u
@@ -617,14 +610,78 @@ __device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64
           const u64 o = shfl_up_u64(incl, d);
           if (lane >= d) incl += o;
         }
-        if (m[e] > 0 && u >= run + incl - m[e] && u < run + incl) s_pick = (int)(base + e * 64 + lane);
+        if (m[e] > 0 && u >= run + incl - m[e] && u < run + incl) sh.s_pick = (int)(base + e * 64 + lane);
         run += shfl_u64(incl, 63);
       }
       break;
     }
   }
   __syncthreads();
-  if (tid == 0) out[r] = s_pick < 0 ? 0 : s_pick;  // degenerate row (all-zero mass): fall back to the first index
+  if (tid == 0) out[blockIdx.x] = sh.s_pick < 0 ? 0 : sh.s_pick;  // degenerate row (all-zero mass): fall back to the first index
+}
+
+// One 1024-thread workgroup per row.
+//
+// Short path (any top-k up to 1024, or a top-p whose nucleus is small): thread t's largest number over the columns t, t + 1024, ...
+// is known after one pass; the k-th largest of these 1024 maxima has at least k numbers at or above it, so the second pass collects
+// only what reaches a bound just below it -- some k numbers out of a 152 k vocabulary -- and both thresholds and the draw are integer sums over that
+// list.  The general path finds the same thresholds by three radix levels over the whole row; it stays for wide nuclei, top-k above
+// 1024 and rows whose largest numbers share a column.
+//
+// Bound: one CU walks one row (304 KB of bf16 logits) twice, an exponential and ~10 VALU operations per element in the second pass.
+// 64 rows x 151936 bf16 logits, top-k and top-p: softmax_kernel + radix levels over the stored fp32 probabilities (ten passes, u64 LDS
+// atomics for every element of a first level) 551 us; this kernel from the logits 34 us (51 with an exact k-th maximum and one thread a candidate);
+// 64 x 35186 16 us.
+template <class Src>
+__device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64_t k, float pp, int64_t vocab, float inv_t, u64 seed, u64 offset) {
+  __shared__ RowShared sh;
+  const int tid = threadIdx.x;
+  const bool has_k = k >= 1 && k < vocab;
+  const bool by_count = has_k && k <= kListTopK, by_mass = !has_k && pp < 1.0f;
+  int n = 0;
+
+  float col = Src::kSoftmax ? -INFINITY : 0.f;
+  if (Src::kSoftmax || by_count || by_mass)
+    walk_row(src, vocab, [&](int64_t, float x, bool in) { col = in ? fmaxf(col, x) : col; });
+  if constexpr (Src::kSoftmax) {
+    src.mx = block_reduce_max(col, sh.lds_f);
+    src.k = inv_t * 1.4426950408889634f;
+  }
+  uint32_t floor_bits = 0u, list_bits = kNoDigit;  // list_bits: what a weight has to reach to be listed
+  if (by_count || by_mass) {
+    const float w = src.weight(col);
+    const int want = (int)(by_count ? k : (int64_t)kListTopP);
+    floor_bits = kth_bound(w > 0.f ? __float_as_uint(w) : 0u, want, sh.h_cnt, sh.s_two);  // NaN counts as nothing here
+    // weights up to some units in the last place apart can be the same probability: the list starts a little below
+    if (floor_bits) list_bits = floor_bits - 8u;
+  }
+  if (tid == 0) { sh.s_n = 0; sh.s_pick = -1; }
+  __syncthreads();
+  if (Src::kSoftmax || list_bits != kNoDigit) {
+    float sum = 0.f;
+    walk_row(src, vocab, [&](int64_t i, float x, bool in) {
+      const float w = src.weight(x);
+      if (in) sum += w;
+      const bool hit = in && w > 0.f && __float_as_uint(w) >= list_bits;
+      const u64 votes = __ballot(hit);
+      if (votes) {
+        const int lane = tid & 63;
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&sh.s_n, __popcll(votes));
+        at = __shfl(at, 0, 64) + __popcll(votes & ((1ull << lane) - 1ull));
+        if (hit && at < kList) {
+          sh.s_index[at] = (int)i;
+          sh.h_cnt[at] = __float_as_uint(w);
+        }
+      }
+    });
+    if constexpr (Src::kSoftmax) src.inv = 1.0f / block_reduce_sum(sum, sh.lds_f);
+    __syncthreads();
+    n = sh.s_n;
+  }
+  u64 kept_mass = kNoMass;
+  if (list_bits != kNoDigit && n <= kList && draw_from_list(src, sh, out, n, floor_bits, by_count, k, pp, vocab, seed, offset, kept_mass)) return;
+  draw_from_row(src, sh, out, k, pp, vocab, seed, offset, kept_mass);
 }
 
 __global__ __launch_bounds__(kRowThreads) void sample_kernel(int* __restrict__ out, const float* __restrict__ probs,
@@ -648,8 +705,19 @@ __device__ __forceinline__ void copy_numbers(E* __restrict__ dst, const E* __res
 
 constexpr int64_t kCopySlice = 1 << 15;  // numbers of a row that one workgroup copies
 
+// slice x of all rows' slices: a copy of the row and, with its first slice, its temperature
+template <int DT>
+__device__ __forceinline__ void copy_slice(int x, const char* __restrict__ logits, const float* __restrict__ temperatures, int64_t vocab,
+                                           int64_t row_stride_bytes, char* __restrict__ kept, float* __restrict__ kept_t) {
+  using E = std::conditional_t<DT == MSGL_F32, uint32_t, uint16_t>;
+  const int slices = (int)((vocab + kCopySlice - 1) / kCopySlice);
+  const int64_t r = x / slices, at = (x - r * slices) * kCopySlice;
+  copy_numbers(reinterpret_cast<E*>(kept) + r * vocab + at, reinterpret_cast<const E*>(logits + r * row_stride_bytes) + at, min(kCopySlice, vocab - at));
+  if (at == 0 && threadIdx.x == 0) kept_t[r] = temperatures[r];
+}
+
 // Workgroups 0 .. rows - 1 draw; with `kept` those behind them copy the rows in slices, on compute units that the draw leaves idle (64 rows x
-// 151936 bf16: 49.0 us without a copy, 51.5 with; the drawing threads storing it 59.3).
+// 151936 bf16: 2.5 us; the drawing threads storing it 10).
 template <int DT>
 __global__ __launch_bounds__(kRowThreads) void sample_filtered_logits_kernel(int* __restrict__ out, const char* __restrict__ logits,
                                                                              const float* __restrict__ temperatures,
@@ -657,11 +725,7 @@ __global__ __launch_bounds__(kRowThreads) void sample_filtered_logits_kernel(int
                                                                              int64_t vocab, int64_t row_stride_bytes, u64 seed, u64 offset, int rows,
                                                                              char* __restrict__ kept, float* __restrict__ kept_t) {
   if ((int)blockIdx.x >= rows) {
-    using E = std::conditional_t<DT == MSGL_F32, uint32_t, uint16_t>;
-    const int slices = (int)((vocab + kCopySlice - 1) / kCopySlice), x = (int)blockIdx.x - rows;
-    const int64_t r = x / slices, at = (x - r * slices) * kCopySlice;
-    copy_numbers(reinterpret_cast<E*>(kept) + r * vocab + at, reinterpret_cast<const E*>(logits + r * row_stride_bytes) + at, min(kCopySlice, vocab - at));
-    if (at == 0 && threadIdx.x == 0) kept_t[r] = temperatures[r];
+    copy_slice<DT>((int)blockIdx.x - rows, logits, temperatures, vocab, row_stride_bytes, kept, kept_t);
     return;
   }
   const int64_t r = blockIdx.x;
@@ -781,6 +845,566 @@ __global__ __launch_bounds__(kRowThreads) void sample_logits_kernel(int* __restr
   if (tid == 0) out[r] = s_pick < 0 ? 0 : s_pick;  // degenerate row (no mass): first index
 }
 
+// ------------------------------------------------------------------------------------------
+// The same draws with a row's work on several workgroups
+//
+// One workgroup walks a row of 151936 in two passes that wait for loads, and 64 rows leave 192 of 256 compute units idle.  Here `split`
+// workgroups share a row, one launch per point where the whole row has to be known:
+//   split_max    each takes a range of the row: 1024 maxima, each of some numbers of the row
+//   split_sum    each takes 1024 / split of the columns i mod 1024: weights, every column's sum in the order of the rows (the sum's bits are
+//                softmax_kernel's), and the candidates that reach the k-th largest maximum; or, with a mass alone, the mass per 64th of an octave
+//   split_mass   each takes some of up to 1024 chunks in index order: the chunk's mass above the 64th of an octave in which the threshold
+//                lies, and the candidates within (without a filter: the chunk's mass)
+//   split_pick   one workgroup a row: threshold among the candidates, the draw over the list or over chunks and inside one of them; beside them
+//                the copy of the rows
+// Thresholds, masses and picks are those of one workgroup (integer sums over the same numbers); a threshold that is not among the candidates
+// (ties across the bound, top-k above 1024) falls to draw_from_row, as there.
+// Bound: the launches' ends and starts and each one's chain of a few dependent loads and barriers (6, 14, 10 us of 32 at 64 x 151936 with top-k, where
+// the reads take 8 and the exponentials 2).  us a draw, one workgroup per row -> shared: see split_of.
+// ------------------------------------------------------------------------------------------
+constexpr int kMaxChunks = kRowThreads;
+constexpr int64_t kMostPerGroup = 1 << 17;       // numbers of a row to one workgroup
+constexpr int kPart = 1024;                      // candidates that one workgroup of a row lists
+constexpr int kTile = 8192;                      // numbers of a row's columns that a workgroup holds at a time
+constexpr uint32_t kMassLow = 87u << 23;         // 2^-40: a smaller weight's probability has no mass
+constexpr int kMassShift = 17;                   // 64 bins per octave
+constexpr int kMassBins = 40 * 64 + 1;           // the last one: weight 1
+constexpr int kOctaves = 41;                     // the last one: weight 1
+constexpr int kMassSlots = kOctaves * 64 + 64;   // bins (the last octave's up to its 64) and, behind them, the octaves
+
+struct SplitHead {
+  float mx;
+  uint32_t floor_bits;      // what a weight has to reach to be surely listed
+  uint32_t cut_lo, cut_hi;  // weights' bits between which the mass threshold lies
+};
+
+struct SplitScratch {
+  SplitHead* head;     // [rows]
+  float* top;          // [rows][1024] maxima
+  float* sum;          // [rows][1024] columns' sums
+  int* count;          // [rows][split] candidates found (more than kPart: not all of them are listed)
+  u64* list;           // [rows][split][kPart] candidates: weight's bits, index
+  u64* chunk;          // [rows][kMaxChunks] masses
+  u64* total;          // [rows][split] masses of all
+  float* hist;         // [rows][split][kMassSlots]: sums of weights per 64th of an octave (the last: 1 and above), per octave
+};
+
+// lays the parts out one behind the other from `base`; returns the bytes
+static inline size_t split_layout(SplitScratch* s, char* base, int64_t rows, int split, bool filtered, bool hist) {
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    char* p = base + at;
+    at += (bytes + 255) & ~(size_t)255;
+    return p;
+  };
+  s->head = reinterpret_cast<SplitHead*>(take(rows * sizeof(SplitHead)));
+  s->top = reinterpret_cast<float*>(take(rows * kRowThreads * sizeof(float)));
+  s->chunk = reinterpret_cast<u64*>(take(rows * kMaxChunks * sizeof(u64)));
+  if (filtered) {
+    s->sum = reinterpret_cast<float*>(take(rows * kRowThreads * sizeof(float)));
+    s->count = reinterpret_cast<int*>(take(rows * split * sizeof(int)));
+    s->list = reinterpret_cast<u64*>(take(rows * split * kPart * sizeof(u64)));
+  }
+  if (hist) {
+    s->total = reinterpret_cast<u64*>(take(rows * split * sizeof(u64)));
+    s->hist = reinterpret_cast<float*>(take(rows * split * kMassSlots * sizeof(float)));
+  }
+  return at;
+}
+
+static inline int64_t split_chunk(int64_t vocab) {
+  int64_t c = 512;
+  while ((vocab + c - 1) / c > kMaxChunks) c *= 2;
+  return c;
+}
+
+// the eight logits of a thread in a piece of 512 per wave: consecutive ones where rows are 16-byte aligned, 64 apart otherwise
+template <int DT, bool VEC>
+struct Piece {
+  static __device__ __forceinline__ int64_t at(int64_t base, int lane, int e) { return VEC ? base + lane * 8 + e : base + e * 64 + lane; }
+  // x[e] is defined where at(base, lane, e) < hi
+  static __device__ __forceinline__ void load(const void* row, int64_t base, int lane, int64_t hi, float (&x)[8]) {
+    if (VEC && base + lane * 8 + 8 <= hi) {
+      load_logits8<DT>(row, base + lane * 8, x);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = at(base, lane, e) < hi ? load_logit<DT>(row, at(base, lane, e)) : -INFINITY;
+    }
+  }
+};
+
+template <int DT, bool VEC>
+__global__ __launch_bounds__(kRowThreads, 8) void split_max_kernel(SplitScratch sc, const char* __restrict__ logits, int64_t vocab,
+                                                                   int64_t row_stride_bytes, int split) {
+  using E = std::conditional_t<DT == MSGL_F32, uint32_t, uint16_t>;
+  constexpr int kPer = 16 / sizeof(E);
+  const int tid = threadIdx.x;
+  const int64_t r = blockIdx.x / split;
+  const int g = (int)blockIdx.x - (int)r * split;
+  const char* row = logits + r * row_stride_bytes;
+  const int64_t per = ((vocab + split - 1) / split + 7) & ~7ll;
+  const int64_t lo = min(vocab, g * per), hi = min(vocab, lo + per);
+  float mx = -INFINITY;
+  if constexpr (VEC) {
+    constexpr int kDeep = 4;
+    const int64_t wide = lo + (hi - lo) / kPer * kPer;
+    for (int64_t base = lo + tid * kPer; base < wide; base += kDeep * kRowThreads * kPer) {
+      U4 raw[kDeep];
+#pragma unroll
+      for (int u = 0; u < kDeep; ++u) raw[u] = ldg16(reinterpret_cast<const E*>(row) + min(base + u * kRowThreads * kPer, wide - kPer));
+#pragma unroll
+      for (int u = 0; u < kDeep; ++u) {
+        const int64_t i = base + u * kRowThreads * kPer;
+        if (i >= wide) break;
+        const E* e = reinterpret_cast<const E*>(&raw[u]);
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) mx = fmaxf(mx, load_logit<DT>(e, q));
+      }
+    }
+    if (wide + tid < hi) mx = fmaxf(mx, load_logit<DT>(row, wide + tid));
+  } else {
+    constexpr int kDeep = 8;
+    for (int64_t base = lo + tid; base < hi; base += kDeep * kRowThreads) {
+      float x[kDeep];
+#pragma unroll
+      for (int u = 0; u < kDeep; ++u) x[u] = load_logit<DT>(row, min(base + u * kRowThreads, hi - 1));
+#pragma unroll
+      for (int u = 0; u < kDeep; ++u) mx = fmaxf(mx, x[u]);
+    }
+  }
+  for (int d = 1; d < split; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));  // one maximum per `split` neighbours
+  if (tid % split == 0) sc.top[r * kRowThreads + g * (kRowThreads / split) + tid / split] = mx;
+}
+
+// MASS: mass per bin of the weights; else the list of candidates
+template <int DT, bool VEC, bool MASS>
+__global__ __launch_bounds__(kRowThreads, VEC ? 8 : 4) void split_sum_kernel(SplitScratch sc, const char* __restrict__ logits, const float* __restrict__ temperatures,
+                                                                   const int* __restrict__ top_k, const float* __restrict__ top_p, int64_t vocab,
+                                                                   int64_t row_stride_bytes, int split) {
+  __shared__ __attribute__((aligned(16))) float tile[kTile];
+  __shared__ uint32_t pool[MASS ? kOctaves * 64 : 1];  // weights per bin, each to 15 bits: no more than kMostPerGroup of them go in
+  __shared__ __attribute__((aligned(16))) uint32_t hist[MASS ? 4 : kRowThreads];
+  __shared__ float lds_f[kRowThreads / 64];
+  __shared__ uint32_t s_bound;
+  __shared__ int s_n;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t r = blockIdx.x / split;
+  const int g = (int)blockIdx.x - (int)r * split;
+  const char* row = logits + r * row_stride_bytes;
+  const int cols = kRowThreads / split, high = kTile / cols;  // columns of this workgroup, rows of 1024 per tile
+  const float pp = top_p ? top_p[r] : 1.0f;
+
+  // eight numbers per thread and tile: of one row of 1024 where they can be loaded at once, else of eight rows
+  const int at_row = VEC ? tid / (cols / 8) : tid / cols, at_col = VEC ? tid % (cols / 8) * 8 : tid % cols;
+  auto slot = [&](int e) { return VEC ? at_row * cols + at_col + e : (at_row + e * (high / 8)) * cols + at_col; };
+  const uint32_t width = (uint32_t)vocab, step = kTile * split;  // (a sum of two of them fits 32 bits)
+  auto index = [&](uint32_t base, int e) { return base + (VEC ? at_row : at_row + e * (high / 8)) * kRowThreads + g * cols + at_col + (VEC ? e : 0); };
+  auto load = [&](uint32_t base, float (&x)[8]) {
+    if (VEC && index(base, 0) + 8 <= width) {
+      load_logits8<DT>(row, index(base, 0), x);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = index(base, e) < width ? load_logit<DT>(row, index(base, e)) : 0.f;
+    }
+  };
+  float x[8];
+  load(0, x);
+
+  const float top = sc.top[r * kRowThreads + tid];
+  const float mx = block_reduce_max(top, lds_f), k = 1.0f / temperatures[r] * 1.4426950408889634f;
+  const bool mass = MASS && pp < 1.0f;
+  uint32_t list_bits = kNoDigit;
+  if constexpr (MASS) {
+    if (mass)
+      for (int b = tid; b < kOctaves * 64; b += kRowThreads) pool[b] = 0u;
+  } else {
+    const int64_t kk = top_k[r];
+    const bool has_k = kk >= 1 && kk < vocab, by_count = has_k && kk <= kListTopK;
+    uint32_t floor_bits = 0u;
+    if (by_count || (!has_k && pp < 1.0f)) {
+      const float w = __builtin_amdgcn_exp2f((top - mx) * k);
+      floor_bits = kth_bound(w > 0.f ? __float_as_uint(w) : 0u, (int)(by_count ? kk : (int64_t)kListTopP), hist, &s_bound);  // NaN counts as nothing here
+    }
+    if (floor_bits) list_bits = floor_bits - 8u;  // see sample_row
+    if (tid == 0) s_n = list_bits == kNoDigit ? kList + 1 : 0;
+    if (g == 0 && tid == 0) sc.head[r].floor_bits = floor_bits;
+  }
+  if (g == 0 && tid == 0) sc.head[r].mx = mx;
+  __syncthreads();
+
+  u64* list = sc.list + (r * split + g) * kPart;
+  float sum = 0.f;
+  for (uint32_t base = 0; base < width; base += step) {
+    float w[8], most = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      w[e] = index(base, e) < width ? __builtin_amdgcn_exp2f((x[e] - mx) * k) : 0.f;  // a zero more leaves a sum as it is
+      most = fmaxf(most, w[e]);
+    }
+    if constexpr (VEC) {
+      *reinterpret_cast<float4*>(tile + slot(0)) = float4{w[0], w[1], w[2], w[3]};
+      *reinterpret_cast<float4*>(tile + slot(4)) = float4{w[4], w[5], w[6], w[7]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) tile[slot(e)] = w[e];
+    }
+    if (base + step < width) load(base + step, x);
+    if constexpr (MASS) {
+      if (mass) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t b = __float_as_uint(w[e]);
+          if (w[e] > 0.f && b >= kMassLow) atomicAdd(&pool[min((b - kMassLow) >> kMassShift, (uint32_t)kMassBins - 1u)], ((b & 0x7fffffu) + 0x800100u) >> 9);
+        }
+      }
+    } else if (__any(__float_as_uint(most) >= list_bits)) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const bool hit = w[e] > 0.f && __float_as_uint(w[e]) >= list_bits;
+        const u64 votes = __ballot(hit);
+        if (votes) {
+          int at = 0;
+          if (lane == 0) at = atomicAdd(&s_n, __popcll(votes));
+          at = __shfl(at, 0, 64) + __popcll(votes & ((1ull << lane) - 1ull));
+          if (hit && at < kPart) list[at] = (u64)__float_as_uint(w[e]) << 32 | index(base, e);
+        }
+      }
+    }
+    __syncthreads();
+    if (tid < cols) {
+#pragma unroll 16
+      for (int q = 0; q < high; ++q) sum += tile[q * cols + tid];
+    }
+    __syncthreads();
+  }
+  if (tid < cols) sc.sum[r * kRowThreads + g * cols + tid] = sum;
+  if constexpr (MASS) {
+    if (mass) {
+      float* to = sc.hist + ((int64_t)r * split + g) * kMassSlots;
+      for (int o = tid >> 6; o < kOctaves; o += kRowThreads / 64) {
+        const float m = ldexpf((float)pool[o * 64 + lane], o - 54), all = wave_sum(m);
+        to[o * 64 + lane] = m;
+        if (lane == 0) to[kOctaves * 64 + o] = all;
+      }
+    }
+  } else {
+    if (tid == 0) sc.count[r * split + g] = s_n;
+  }
+}
+
+// FILTER: a top-p per row (1 and above: every probability); else masses of the weights, as sample_logits_kernel's
+template <int DT, bool VEC, bool FILTER>
+__global__ __launch_bounds__(kRowThreads, 8) void split_mass_kernel(SplitScratch sc, const char* __restrict__ logits, const float* __restrict__ temperatures,
+                                                                    const float* __restrict__ top_p, int64_t vocab, int64_t row_stride_bytes, int split,
+                                                                    int64_t chunk) {
+  __shared__ u64 lds_w[kRowThreads / 64];
+  __shared__ float lds_f[kRowThreads / 64];
+  __shared__ int s_n, s_bin[2];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t r = blockIdx.x / split;
+  const int g = (int)blockIdx.x - (int)r * split;
+  const char* row = logits + r * row_stride_bytes;
+  const int64_t chunks = (vocab + chunk - 1) / chunk;
+  const int64_t c0 = (int64_t)(tid >> 6) * split + g;
+  float x[8];
+  if constexpr (!FILTER) Piece<DT, VEC>::load(row, c0 * chunk, lane, min(vocab, (c0 + 1) * chunk), x);
+
+  const float mx = FILTER ? sc.head[r].mx : block_reduce_max(sc.top[r * kRowThreads + tid], lds_f);
+  const float inv_t = 1.0f / temperatures[r];
+  const float k = FILTER ? inv_t * 1.4426950408889634f : 1.4426950408889634f / temperatures[r];  // each as the kernel whose picks these are
+  const float pp = FILTER && top_p ? top_p[r] : 1.0f;
+  float inv = 1.0f;
+  uint32_t cut_lo = 0u, cut_hi = 0u;  // candidates: weights in [cut_lo, cut_hi); counted: those from cut_hi on
+  if constexpr (FILTER) {
+    inv = 1.0f / block_reduce_sum(sc.sum[r * kRowThreads + tid], lds_f);
+    if (pp < 1.0f) {
+      // Mass of the weights from the top, octave by octave and then inside one (a wave, lane l the l-th from the top): the sums are off from the
+      // probabilities' by less than `off`.
+      if (tid < 64) {
+        const float* h = sc.hist + (int64_t)r * split * kMassSlots;
+        auto masses = [&](int slot, bool in) {
+          float m = 0.f;
+          if (in)
+            for (int q = 0; q < split; ++q) m += h[(int64_t)q * kMassSlots + slot];
+          return m;
+        };
+        auto prefix = [&](float v) {
+#pragma unroll
+          for (int d = 1; d < 64; d <<= 1) {
+            const float o = __shfl_up(v, d, 64);
+            if (lane >= d) v += o;
+          }
+          return v;
+        };
+        const float oct = masses(kOctaves * 64 + kOctaves - 1 - lane, lane < kOctaves), oct_incl = prefix(oct), all = __shfl(oct_incl, 63, 64);
+        const float want = pp * all, off = all * 0x1.4p-15f;
+        // the first lane whose sum reaches `at`, the last one with a mass otherwise
+        auto reach = [&](float m, float incl, float at) {
+          const u64 there = __ballot(m > 0.f && incl >= at), some = __ballot(m > 0.f);
+          return there ? __ffsll((long long)there) - 1 : some ? 63 - __clzll((long long)some) : 0;
+        };
+        int bin[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {  // the highest bin that may hold the threshold, the lowest one
+          const float at = q ? want + off : want - off;
+          const int o = reach(oct, oct_incl, at);
+          const float above = o ? __shfl(oct_incl, o - 1, 64) : 0.f;
+          const float m = masses((kOctaves - 1 - o) * 64 + 63 - lane, true);
+          bin[q] = (kOctaves - 1 - o) * 64 + 63 - reach(m, above + prefix(m), at);
+        }
+        if (lane == 0) {
+          s_bin[0] = bin[0];
+          s_bin[1] = bin[1];
+        }
+      }
+      __syncthreads();
+      cut_lo = kMassLow + ((uint32_t)s_bin[1] << kMassShift);
+      cut_hi = kMassLow + ((uint32_t)(s_bin[0] + 1) << kMassShift) + 8u;
+    }
+    if (g == 0 && tid == 0) {
+      sc.head[r].cut_lo = cut_lo;
+      sc.head[r].cut_hi = cut_hi;
+    }
+    if (cut_lo) cut_lo -= 8u;  // weights some units in the last place apart can be one probability
+    if (tid == 0) s_n = 0;
+    __syncthreads();
+  }
+
+  u64* list = FILTER ? sc.list + (r * split + g) * kPart : nullptr;
+  // fixed_mass without the conversion to 64-bit integers: whole numbers below 2^53 in 64-bit floating point
+  auto units = [](float p) { return fmaxf(__builtin_truncf(p * 1099511627776.0f), 0.f); };
+  double total = 0;
+  for (int64_t c = c0; c < chunks; c += split * (kRowThreads / 64)) {
+    const int64_t hi = min(vocab, (c + 1) * chunk);
+    double mass = 0;
+    for (int64_t base = c * chunk; base < hi; base += 512) {
+      if (FILTER || c != c0 || base != c * chunk) Piece<DT, VEC>::load(row, base, lane, hi, x);
+      float w[8], most = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        w[e] = Piece<DT, VEC>::at(base, lane, e) < hi ? __builtin_amdgcn_exp2f((x[e] - mx) * k) : 0.f;
+        if constexpr (!FILTER) {
+          mass += units(w[e]);
+        } else {
+          const float m = units(w[e] * inv);
+          const bool up = __float_as_uint(w[e]) >= cut_hi;
+          total += m;
+          mass += up ? m : 0.f;
+          most = fmaxf(most, up ? 0.f : w[e]);
+        }
+      }
+      if (FILTER && __any(__float_as_uint(most) >= cut_lo && most > 0.f)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t b = __float_as_uint(w[e]);
+          const bool hit = w[e] > 0.f && b >= cut_lo && b < cut_hi;
+          const u64 votes = __ballot(hit);
+          if (votes) {
+            int at = 0;
+            if (lane == 0) at = atomicAdd(&s_n, __popcll(votes));
+            at = __shfl(at, 0, 64) + __popcll(votes & ((1ull << lane) - 1ull));
+            if (hit && at < kPart) list[at] = (u64)b << 32 | (uint32_t)Piece<DT, VEC>::at(base, lane, e);
+          }
+        }
+      }
+    }
+    const u64 all = wave_sum_u64((u64)mass);
+    if (lane == 0) sc.chunk[r * kMaxChunks + c] = all;
+  }
+  if constexpr (FILTER) {
+    const u64 all = block_sum_u64((u64)total, lds_w);
+    if (tid == 0) {
+      sc.total[r * split + g] = all;
+      sc.count[r * split + g] = s_n;
+    }
+  }
+}
+
+// The draw over chunks (thread c: chunk c's mass) and inside the chunk that holds it.  mass_at(i): the mass of index i.
+template <class M>
+__device__ __forceinline__ void draw_from_chunks(RowShared& sh, int* __restrict__ out, u64 mine, int64_t vocab, int64_t chunk, u64 seed, u64 offset, M mass_at) {
+  const int tid = threadIdx.x;
+  const u64 incl = block_prefix_incl(mine, sh.lds_w);
+  const u64 total = block_sum_u64(mine, sh.lds_w), u = draw_below(total, seed, offset + blockIdx.x);
+  if (tid == 0) sh.s_n = -1;
+  __syncthreads();
+  if (mine && u >= incl - mine && u < incl) {
+    sh.s_n = tid;
+    sh.h_mass[0] = incl - mine;
+  }
+  __syncthreads();
+  const int c = sh.s_n;
+  if (c < 0) {  // no mass at all: the first index
+    if (tid == 0) out[blockIdx.x] = 0;
+    return;
+  }
+  u64 run = sh.h_mass[0];
+  const int64_t hi = min(vocab, (c + 1) * chunk);
+  for (int64_t base = c * chunk; base < hi; base += kRowThreads) {
+    const int64_t i = base + tid;
+    const u64 m = i < hi ? mass_at(i) : 0ull;
+    const u64 to = run + block_prefix_incl(m, sh.lds_w);
+    if (m && u >= to - m && u < to) out[blockIdx.x] = (int)i;  // exactly one index
+    if (tid == kRowThreads - 1) sh.h_mass[1] = to;
+    __syncthreads();
+    run = sh.h_mass[1];
+    __syncthreads();
+    if (u < run) break;
+  }
+}
+
+enum { kPickList = 0, kPickMass = 1, kPickAny = 2 };
+
+template <int DT, int HOW>
+__global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc, int* __restrict__ out, const char* __restrict__ logits,
+                                                                 const float* __restrict__ temperatures, const int* __restrict__ top_k,
+                                                                 const float* __restrict__ top_p, int64_t vocab, int64_t row_stride_bytes, int split,
+                                                                 int64_t chunk, u64 seed, u64 offset, int rows, char* __restrict__ kept,
+                                                                 float* __restrict__ kept_t) {
+  __shared__ RowShared sh;
+  const int tid = threadIdx.x;
+  if (HOW != kPickAny && (int)blockIdx.x >= rows) {  // the copy, on compute units that the picks leave idle (64 rows x 151936: 3.5 us in split_max)
+    copy_slice<DT>((int)blockIdx.x - rows, logits, temperatures, vocab, row_stride_bytes, kept, kept_t);
+    return;
+  }
+  const int64_t r = blockIdx.x;
+  const void* row = logits + r * row_stride_bytes;
+  if constexpr (HOW == kPickAny) {
+    const int64_t chunks = (vocab + chunk - 1) / chunk;
+    const u64 mine = tid < chunks ? sc.chunk[r * kMaxChunks + tid] : 0ull;
+    const float mx = block_reduce_max(sc.top[r * kRowThreads + tid], sh.lds_f), k = 1.4426950408889634f / temperatures[r];
+    draw_from_chunks(sh, out, mine, vocab, chunk, seed, offset, [&](int64_t i) { return exp_mass(load_logit<DT>(row, i), mx, k); });
+    return;
+  }
+  const SplitHead head = sc.head[r];
+  const int64_t kk = top_k ? (int64_t)top_k[r] : vocab;
+  const float pp = top_p ? top_p[r] : 1.0f;
+  LogitRow<DT> src{row, head.mx, 1.0f / temperatures[r] * 1.4426950408889634f, 1.0f};
+  src.inv = 1.0f / block_reduce_sum(sc.sum[r * kRowThreads + tid], sh.lds_f);
+  // the workgroups' lists one behind the other (their lengths in the lanes, the places before each in `upto`)
+  const int lane = tid & 63, count = lane < split ? sc.count[r * split + lane] : 0;
+  int upto = min(count, kPart + kList);
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) {
+    const int o = __shfl_up(upto, d, 64);
+    if (lane >= d) upto += o;
+  }
+  const bool listed = !__any(count > kPart) && __shfl(upto, split - 1, 64) <= kList;
+  const int n = listed ? __shfl(upto, split - 1, 64) : 0;
+  for (int c = tid; c < n; c += kRowThreads) {
+    int g = 0, from = 0;
+    for (int q = 0; q < split - 1; ++q) {
+      const int end = __builtin_amdgcn_readlane(upto, q);
+      if (c >= end) {
+        g = q + 1;
+        from = end;
+      }
+    }
+    const u64 e = sc.list[(r * split + g) * kPart + c - from];
+    sh.s_index[c] = (int)(uint32_t)e;
+    sh.h_cnt[c] = (uint32_t)(e >> 32);
+  }
+  if (tid == 0) sh.s_pick = -1;
+  u64 kept_mass = kNoMass;
+  if constexpr (HOW == kPickList) {
+    const bool by_count = kk >= 1 && kk < vocab;
+    __syncthreads();
+    if (listed && draw_from_list(src, sh, out, n, head.floor_bits, by_count, kk, pp, vocab, seed, offset, kept_mass)) return;
+  } else {
+    const int64_t chunks = (vocab + chunk - 1) / chunk;
+    u64 mine = tid < chunks ? sc.chunk[r * kMaxChunks + tid] : 0ull;
+    uint32_t thr_bits = 0u;
+    bool found = !(pp < 1.0f);
+    if (!found) {
+      const u64 above = block_sum_u64(mine, sh.lds_w);
+      kept_mass = 0;
+      for (int h = 0; h < split; ++h) kept_mass += sc.total[r * split + h];
+      const u64 target = mass_target(pp, kept_mass);
+      // masses by 1024 equal ranges of the candidates' probabilities, then of one range, down to one value
+      const uint32_t p_lo = __float_as_uint(src.prob(__uint_as_float(head.cut_lo - 8u)));
+      const uint32_t p_hi = __float_as_uint(src.prob(__uint_as_float(head.cut_hi)));
+      int shift = 0;
+      while (p_hi > p_lo && (p_hi - p_lo) >> shift >= (uint32_t)kRowThreads) ++shift;
+      u64 higher = above;
+      uint32_t from = p_lo, span = ~0u;  // the threshold is among [from, from + span]
+      bool in_list = listed;
+#pragma unroll 1
+      for (int step = shift; in_list; step = max(0, step - 10)) {  // by 1024 ranges of 2^step
+        sh.h_mass[tid] = 0ull;
+        if (tid == 0) sh.s_two[0] = kNoDigit;
+        __syncthreads();
+        for (int c = tid; c < n; c += kRowThreads) {
+          const float p = src.prob(__uint_as_float(sh.h_cnt[c]));
+          const uint32_t at = __float_as_uint(p) - from;
+          if (__float_as_uint(p) >= from && at <= span) atomicAdd(&sh.h_mass[min(at >> step, (uint32_t)kRowThreads - 1u)], fixed_mass(p));
+        }
+        __syncthreads();
+        const u64 m = sh.h_mass[kRowThreads - 1 - tid];  // descending
+        const u64 incl = higher + block_prefix_incl(m, sh.lds_w);
+        if (incl - m < target && target <= incl) {
+          sh.s_two[0] = kRowThreads - 1 - tid;
+          sh.h_mass[kRowThreads] = incl - m;
+        }
+        __syncthreads();
+        const uint32_t here = sh.s_two[0];
+        if (here == kNoDigit) {
+          in_list = false;
+        } else {
+          higher = sh.h_mass[kRowThreads];
+          from += here << step;
+          span = (1u << step) - 1u;
+        }
+        __syncthreads();
+        if (step == 0) break;
+      }
+      if (in_list) {
+        if (tid == 0) sh.s_digit = kNoDigit;
+        __syncthreads();
+        for (int c = tid; c < n; c += kRowThreads)  // surely all of them listed: a weight from the cut's lower end on has this probability
+          if (sh.h_cnt[c] >= head.cut_lo && __float_as_uint(src.prob(__uint_as_float(sh.h_cnt[c]))) == from) sh.s_digit = from;
+        __syncthreads();
+        found = sh.s_digit != kNoDigit && kept_mass > 0;
+        thr_bits = found ? from : 0u;
+      }
+      if (found) {  // candidates that stay, to their chunks
+        __syncthreads();
+        sh.h_mass[tid] = 0ull;
+        __syncthreads();
+        for (int c = tid; c < n; c += kRowThreads) {
+          const float p = src.prob(__uint_as_float(sh.h_cnt[c]));
+          if (__float_as_uint(p) >= thr_bits) atomicAdd(&sh.h_mass[sh.s_index[c] / chunk], fixed_mass(p));
+        }
+        __syncthreads();
+        mine += sh.h_mass[tid];
+        __syncthreads();
+      }
+    }
+    if (found) {
+      draw_from_chunks(sh, out, mine, vocab, chunk, seed, offset, [&](int64_t i) {
+        const float p = src.prob(src.weight(src.raw(i)));
+        return __float_as_uint(p) >= thr_bits ? fixed_mass(p) : 0ull;
+      });
+      return;
+    }
+    __syncthreads();
+  }
+  draw_from_row(src, sh, out, kk, pp, vocab, seed, offset, kept_mass);
+}
+
+// Workgroups per row (1: one walks the row).  One a compute unit in all: 64 rows x 151936, top-p alone, 54 us with 4 each, 58 with 8; 33 rows 51 and 54.
+// Where sharing pays, us a draw, shared / one workgroup:
+//   top-k      1 x 151936 20.5 / 25.2, 33 x 151936 29.4 / 31.4, 64 x 151936 29.1 / 34.2, but 8 x 65536 20.4 / 17.5, 100 x 151936 41 / 38
+//   top-p      2 x 32000 34 / 50, 64 x 35186 38 / 52, 256 x 50000 60 / 69, 256 x 151936 119 / 197
+//   no filter  8 x 65536 13.9 / 16.0, 100 x 151936 29 / 37, but 32 x 50000 14.8 / 14.8, 128 x 50000 18.2 / 15.3, 256 x 151936 48 / 44
+static inline int split_of(int64_t rows, int64_t vocab, bool filtered, bool has_k, bool has_p) {
+  const bool by_mass = filtered && has_p && !has_k;
+  const int64_t most = by_mass ? 256 : has_k ? 64 : 128, shortest = by_mass ? 8192 : has_k ? 98304 : 65536;
+  if (rows > most || vocab < shortest) return 1;
+  int split = 16;
+  while (split > 2 && (rows * split > 256 || vocab / split < 2048)) split /= 2;
+  return vocab / split < kMostPerGroup ? split : 1;
+}
+
 }  // namespace msgl
 
 using namespace msgl;
@@ -849,15 +1473,76 @@ extern "C" int msgl_sample_top_k_top_p(int32_t* out, const float* probs, const i
   return MSGL_OK;
 }
 
+// Bytes that the draws straight from logits take to split their rows over several workgroups; 0: one workgroup a row is as good.
+// filtered: through the probabilities; has_k, has_p: a top-k, a top-p per row is given.
+extern "C" int64_t msgl_sample_workspace_bytes(int64_t rows, int64_t vocab, int filtered, int has_k, int has_p) {
+  const int split = rows > 0 && vocab > 0 ? split_of(rows, vocab, filtered, has_k, has_p) : 1;
+  SplitScratch sc{};
+  return split > 1 ? (int64_t)split_layout(&sc, nullptr, rows, split, filtered, filtered && !has_k) : 0;
+}
+
+// One draw per row in three or four launches (see the comment above split_max_kernel).
+template <int DT, bool VEC>
+static void launch_split(const SplitScratch& sc, int32_t* out, char* kept, float* kept_t, const char* logits, const float* temperatures, const int32_t* top_k,
+                         const float* top_p, bool filtered, int64_t rows, int64_t vocab, int64_t stride_bytes, int split, u64 seed, u64 offset, hipStream_t s) {
+  const int64_t copies = kept ? rows * ((vocab + kCopySlice - 1) / kCopySlice) : 0;
+  const dim3 many((unsigned)(rows * split)), picks((unsigned)(rows + copies)), b(kRowThreads);
+  const int64_t chunk = split_chunk(vocab);
+  split_max_kernel<DT, VEC><<<many, b, 0, s>>>(sc, logits, vocab, stride_bytes, split);
+  if (!filtered) {
+    split_mass_kernel<DT, VEC, false><<<many, b, 0, s>>>(sc, logits, temperatures, top_p, vocab, stride_bytes, split, chunk);
+    split_pick_kernel<DT, kPickAny><<<picks, b, 0, s>>>(sc, out, logits, temperatures, top_k, top_p, vocab, stride_bytes, split, chunk, seed, offset,
+                                                        (int)rows, kept, kept_t);
+  } else if (top_k) {
+    split_sum_kernel<DT, VEC, false><<<many, b, 0, s>>>(sc, logits, temperatures, top_k, top_p, vocab, stride_bytes, split);
+    split_pick_kernel<DT, kPickList><<<picks, b, 0, s>>>(sc, out, logits, temperatures, top_k, top_p, vocab, stride_bytes, split, chunk, seed, offset,
+                                                         (int)rows, kept, kept_t);
+  } else {
+    split_sum_kernel<DT, VEC, true><<<many, b, 0, s>>>(sc, logits, temperatures, top_k, top_p, vocab, stride_bytes, split);
+    split_mass_kernel<DT, VEC, true><<<many, b, 0, s>>>(sc, logits, temperatures, top_p, vocab, stride_bytes, split, chunk);
+    split_pick_kernel<DT, kPickMass><<<picks, b, 0, s>>>(sc, out, logits, temperatures, top_k, top_p, vocab, stride_bytes, split, chunk, seed, offset,
+                                                         (int)rows, kept, kept_t);
+  }
+}
+
+// the workspace laid out, and one draw per row; `name` for errors
+static int sample_split(const char* name, void* workspace, int64_t workspace_bytes, int32_t* out, void* kept, float* kept_t, const void* logits,
+                        const float* temperatures, const int32_t* top_k, const float* top_p, bool filtered, int64_t rows, int64_t vocab, int64_t logits_stride,
+                        int logits_dtype, u64 seed, u64 offset, hipStream_t s) {
+  const int split = split_of(rows, vocab, filtered, top_k, top_p), esz = logits_dtype == MSGL_F32 ? 4 : 2;
+  SplitScratch sc{};
+  const int64_t need = (int64_t)split_layout(&sc, static_cast<char*>(workspace), rows, split, filtered, filtered && !top_k);
+  MSGL_REQUIRE(aligned16(workspace) && workspace_bytes >= need, "%s: a workspace of %lld bytes, 16-byte aligned, is needed", name, (long long)need);
+  const bool vec = aligned16(logits) && (logits_stride * esz) % 16 == 0;
+#define MSGL_SPLIT(DT)                                                                                                                               \
+  do {                                                                                                                                               \
+    auto* f = vec ? &launch_split<DT, true> : &launch_split<DT, false>;                                                                              \
+    f(sc, out, (char*)kept, kept_t, (const char*)logits, temperatures, top_k, top_p, filtered, rows, vocab, logits_stride * esz, split, seed, offset, s); \
+  } while (0)
+  if (logits_dtype == MSGL_F32) MSGL_SPLIT(MSGL_F32);
+  else if (logits_dtype == MSGL_BF16) MSGL_SPLIT(MSGL_BF16);
+  else if (logits_dtype == MSGL_FP16) MSGL_SPLIT(MSGL_FP16);
+  else {
+    set_error("%s: unsupported dtype code %d", name, logits_dtype);
+    return MSGL_EINVAL;
+  }
+#undef MSGL_SPLIT
+  MSGL_CHECK_LAUNCH(name);
+  return MSGL_OK;
+}
+
 // probs path's draw without the probs: same thresholds, same masses, same pick as softmax_temperature + sample_top_k_top_p
-extern "C" int msgl_sample_filtered_logits_keep(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
-                                                const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
-                                                int logits_dtype, uint64_t seed, uint64_t offset, void* stream) {
+extern "C" int msgl_sample_filtered_logits_ws(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
+                                              const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
+                                              int logits_dtype, uint64_t seed, uint64_t offset, void* workspace, int64_t workspace_bytes, void* stream) {
   MSGL_REQUIRE(rows >= 0, "sample_filtered_logits: negative rows");
   if (rows == 0) return MSGL_OK;
   MSGL_REQUIRE(out && logits && temperatures && !kept == !kept_temperatures, "sample_filtered_logits: null pointer");
   MSGL_REQUIRE(vocab >= 1 && vocab < (1ll << 31) && rows < (1ll << 31), "sample_filtered_logits: bad shape");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (workspace && split_of(rows, vocab, true, top_k, top_p) > 1)
+    return sample_split("sample_filtered_logits", workspace, workspace_bytes, out, kept, kept_temperatures, logits, temperatures, top_k, top_p, true, rows,
+                        vocab, logits_stride, logits_dtype, seed, offset, s);
   const int64_t groups = rows + (kept ? rows * ((vocab + kCopySlice - 1) / kCopySlice) : 0);
   MSGL_REQUIRE(groups < (1ll << 31), "sample_filtered_logits: too many rows");
   const dim3 g((unsigned)groups), b(kRowThreads);
@@ -876,6 +1561,13 @@ extern "C" int msgl_sample_filtered_logits_keep(int32_t* out, void* kept, float*
   return MSGL_OK;
 }
 
+extern "C" int msgl_sample_filtered_logits_keep(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
+                                                const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
+                                                int logits_dtype, uint64_t seed, uint64_t offset, void* stream) {
+  return msgl_sample_filtered_logits_ws(out, kept, kept_temperatures, logits, temperatures, top_k, top_p, rows, vocab, logits_stride, logits_dtype, seed,
+                                        offset, nullptr, 0, stream);
+}
+
 extern "C" int msgl_sample_filtered_logits(int32_t* out, const void* logits, const float* temperatures, const int32_t* top_k,
                                            const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride, int logits_dtype,
                                            uint64_t seed, uint64_t offset, void* stream) {
@@ -883,9 +1575,9 @@ extern "C" int msgl_sample_filtered_logits(int32_t* out, const void* logits, con
                                           offset, stream);
 }
 
-extern "C" int msgl_sample_from_logits(int32_t* out, const void* logits, const float* temperatures, int64_t rows,
-                                       int64_t vocab, int64_t logits_stride, int logits_dtype, uint64_t seed,
-                                       uint64_t offset, void* stream) {
+extern "C" int msgl_sample_from_logits_ws(int32_t* out, const void* logits, const float* temperatures, int64_t rows, int64_t vocab,
+                                          int64_t logits_stride, int logits_dtype, uint64_t seed, uint64_t offset, void* workspace,
+                                          int64_t workspace_bytes, void* stream) {
   MSGL_REQUIRE(rows >= 0, "sample_from_logits: negative rows");
   if (rows == 0) return MSGL_OK;
   MSGL_REQUIRE(out && logits && temperatures, "sample_from_logits: null pointer");
@@ -894,6 +1586,9 @@ extern "C" int msgl_sample_from_logits(int32_t* out, const void* logits, const f
   MSGL_REQUIRE(aligned16(logits) && (logits_stride * esz) % 16 == 0,
                "sample_from_logits: rows must be 16-byte aligned (stride %lld elements)", (long long)logits_stride);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (workspace && split_of(rows, vocab, false, false, false) > 1)
+    return sample_split("sample_from_logits", workspace, workspace_bytes, out, nullptr, nullptr, logits, temperatures, nullptr, nullptr, false, rows, vocab,
+                        logits_stride, logits_dtype, seed, offset, s);
   const dim3 g((unsigned)rows), b(kRowThreads);
   if (logits_dtype == MSGL_F32)
     sample_logits_kernel<MSGL_F32><<<g, b, 0, s>>>(out, (const char*)logits, temperatures, vocab, logits_stride * esz, (u64)seed, (u64)offset);
@@ -907,4 +1602,9 @@ extern "C" int msgl_sample_from_logits(int32_t* out, const void* logits, const f
   }
   MSGL_CHECK_LAUNCH("sample_from_logits");
   return MSGL_OK;
+}
+
+extern "C" int msgl_sample_from_logits(int32_t* out, const void* logits, const float* temperatures, int64_t rows, int64_t vocab, int64_t logits_stride,
+                                       int logits_dtype, uint64_t seed, uint64_t offset, void* stream) {
+  return msgl_sample_from_logits_ws(out, logits, temperatures, rows, vocab, logits_stride, logits_dtype, seed, offset, nullptr, 0, stream);
 }

@@ -446,9 +446,15 @@ def sample_top_k_top_p(probs: torch.Tensor, top_k: Optional[torch.Tensor], top_p
     return out
 
 
+def _sample_workspace(rows: int, vocab: int, filtered: bool, has_k: bool, has_p: bool, device: torch.device) -> Tuple[Optional[torch.Tensor], int]:
+    """Scratch of a draw whose rows several workgroups share (none where one workgroup a row is as good), from the allocator of the stream."""
+    n = lib().msgl_sample_workspace_bytes(rows, vocab, filtered, has_k, has_p)
+    return (torch.empty(n, dtype=torch.uint8, device=device) if n else None), n
+
+
 def sample_filtered_logits(logits: torch.Tensor, temperatures: torch.Tensor, top_k: Optional[torch.Tensor], top_p: Optional[torch.Tensor],
                            seed: int, offset: int, keep: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> torch.Tensor:
-    """sample_top_k_top_p(softmax_temperature(logits, temperatures), ...) in one launch, without the probabilities: the same picks.
+    """sample_top_k_top_p(softmax_temperature(logits, temperatures), ...) without the probabilities: the same picks.
     keep: contiguous (logits, temperatures) of the same shapes and types that receive a copy of what was drawn from."""
     _need_cuda(logits, temperatures)
     assert logits.dim() == 2 and logits.stride(1) == 1 and temperatures.dtype == torch.float32
@@ -462,11 +468,13 @@ def sample_filtered_logits(logits: torch.Tensor, temperatures: torch.Tensor, top
         _need_cuda(*keep)
         assert keep[0].shape == logits.shape and keep[0].dtype == logits.dtype and keep[0].is_contiguous()
         assert keep[1].shape == (rows,) and keep[1].dtype == torch.float32 and keep[1].is_contiguous()
+    ws, ws_bytes = _sample_workspace(rows, logits.shape[1], True, top_k is not None, top_p is not None, logits.device)
     check(
-        lib().msgl_sample_filtered_logits_keep(
+        lib().msgl_sample_filtered_logits_ws(
             out.data_ptr(), None if keep is None else keep[0].data_ptr(), None if keep is None else keep[1].data_ptr(), logits.data_ptr(),
             temperatures.data_ptr(), top_k.data_ptr() if top_k is not None else None, top_p.data_ptr() if top_p is not None else None, rows,
-            logits.shape[1], logits.stride(0), _logits_dt(logits), seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF, _stream(),
+            logits.shape[1], logits.stride(0), _logits_dt(logits), seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF,
+            None if ws is None else ws.data_ptr(), ws_bytes, _stream(),
         ),
         "sample_filtered_logits",
     )
@@ -479,10 +487,11 @@ def sample_from_logits(logits: torch.Tensor, temperatures: torch.Tensor, seed: i
     assert logits.dim() == 2 and logits.stride(1) == 1 and temperatures.dtype == torch.float32
     assert temperatures.numel() == logits.shape[0]
     out = torch.empty(logits.shape[0], dtype=torch.int32, device=logits.device)
+    ws, ws_bytes = _sample_workspace(logits.shape[0], logits.shape[1], False, False, False, logits.device)
     check(
-        lib().msgl_sample_from_logits(out.data_ptr(), logits.data_ptr(), temperatures.data_ptr(), logits.shape[0],
-                                      logits.shape[1], logits.stride(0), _logits_dt(logits),
-                                      seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF, _stream()),
+        lib().msgl_sample_from_logits_ws(out.data_ptr(), logits.data_ptr(), temperatures.data_ptr(), logits.shape[0],
+                                         logits.shape[1], logits.stride(0), _logits_dt(logits), seed & 0xFFFFFFFFFFFFFFFF,
+                                         offset & 0xFFFFFFFFFFFFFFFF, None if ws is None else ws.data_ptr(), ws_bytes, _stream()),
         "sample_from_logits",
     )
     return out

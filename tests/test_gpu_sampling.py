@@ -320,3 +320,35 @@ def test_nucleus_at_the_list_s_length(ops, dev, vocab):
         want = [_filtered_pick(host[r], 0, 0.98, 3, off + r) for r in range(len(rows))]
         assert ops.sample_filtered_logits(logits, t, None, p, 3, off).cpu().tolist() == want
         assert ops.sample_top_k_top_p(probs, None, p, 3, off).cpu().tolist() == want
+
+
+# rows that 16, 8, 4, 2 and 1 workgroups share, with and without a top-k; vocabularies at the shortest rows that are shared, beside whole columns and
+# chunks, and above 1024 chunks of 512; masses whose threshold lies high, in the tail, in a tie and (column) among numbers that the bound misses
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,vocab", [(3, 65536), (33, 33333), (40, 8192), (130, 8193), (257, 8200), (2, 600_003), (64, 98304), (17, 98309), (65, 98304)])
+def test_a_row_shared_by_workgroups_draws_the_same(ops, dev, dtype, rows, vocab):
+    g = torch.Generator(device=dev).manual_seed(vocab)
+    logits = torch.randn((rows, vocab), generator=g, device=dev) * 2.5
+    for r in range(rows):
+        if r % 5 == 1:
+            logits[r, 3::1024] += 9.0
+        elif r % 5 == 2:
+            logits[r] = torch.round(logits[r] * 2) / 2
+        elif r % 5 == 3:
+            logits[r, 5:] -= 300.0
+    logits = logits.to(dtype)
+    t = torch.tensor([(0.5, 0.7, 1.0, 0.02)[r % 4] for r in range(rows)], device=dev)
+    p = torch.tensor([(0.8, 0.98, 1e-6, 1.0, 0.999999, 0.5)[r % 6] for r in range(rows)], device=dev)
+    k = torch.tensor([(40, 0, 1024, 1, 1500)[r % 5] for r in range(rows)], dtype=torch.int32, device=dev)
+    probs = ops.softmax_temperature(logits, t)
+    host = probs.cpu().numpy()
+    for kk, pp in ((None, p), (k, p), (k, None), (None, None)):
+        for off in (0, 1000):
+            got = ops.sample_filtered_logits(logits, t, kk, pp, 77, off).cpu().tolist()
+            assert got == ops.sample_top_k_top_p(probs, kk, pp, 77, off).cpu().tolist()
+            if rows <= 33 and off == 0:
+                ks, ps = ([0] * rows if kk is None else kk.tolist()), ([1.0] * rows if pp is None else pp.tolist())
+                assert got == [_filtered_pick(host[r], ks[r], ps[r], 77, r) for r in range(rows)]
+    if (vocab * logits.element_size()) % 16 == 0:  # the unfiltered draw from the logits: as its own rows one by one, each with more workgroups
+        got = ops.sample_from_logits(logits, t, 5, 300).tolist()
+        assert got == [int(ops.sample_from_logits(logits[r: r + 1], t[r: r + 1], 5, 300 + r)) for r in range(rows)]
