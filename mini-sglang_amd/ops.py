@@ -690,17 +690,7 @@ def skinny_tune(x: torch.Tensor, weights, library_us: float, iters: int = 8, fol
     out = torch.empty((M, N), dtype=x.dtype, device=x.device)
 
     def time_us(sl, nt, rounds):
-        skinny_linear(x, w0, sl, out, nt)  # warm-up
-        ts = []
-        for _ in range(rounds):
-            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            e0.record()
-            for i in range(iters):
-                skinny_linear(x, weights[(i + 1) % len(weights)], sl, out, nt)
-            e1.record()
-            e1.synchronize()
-            ts.append(e0.elapsed_time(e1) * 1e3 / iters)
-        return min(ts)
+        return _time_launches_us(lambda w: skinny_linear(x, w, sl, out, nt), weights, iters, rounds, ahead=True)
 
     def credit(sl):
         folds = fold_mode is not None and sl <= 0 and rowstream_supported(M, N, K, fold_mode, -sl)
@@ -854,12 +844,17 @@ def m256_candidates(M: int, N: int, K: int, cus: int):
     return out
 
 
-def _time_launches_us(fn, weights, iters: int, rounds: int) -> float:
-    """min over `rounds` of the mean time of `iters` launches of fn(w) on rotating weights (events on this stream)."""
+def _time_launches_us(fn, weights, iters: int, rounds: int, ahead: bool = False) -> float:
+    """min over `rounds` of the mean time of `iters` launches of fn(w) on rotating weights (events on this stream).
+    ahead: the launches are queued behind a kernel that keeps the GPU busy for a while.  Issuing one from here takes the host
+    about 8 us; without that, everything that runs for less measures as 8 us and the choice between such kernels is chance
+    (a down projection of 6 MB got a plan of 9.9 us instead of 5.8, a decode step of Qwen3-0.6B 1390 us instead of 1260)."""
     fn(weights[0])  # warm-up
     ts = []
     for _ in range(rounds):
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        if ahead:
+            torch.cuda._sleep(iters * 60_000)  # about 26 us of the GPU per launch
         e0.record()
         for i in range(iters):
             fn(weights[(i + 1) % len(weights)])
@@ -919,10 +914,10 @@ def fused_silu_tune(x: torch.Tensor, weights, iters: int = 8) -> dict:
         # is planned to do for the shape + the activation kernel
         half = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         full = torch.empty((M, N), dtype=x.dtype, device=x.device)  # (no allocation inside the timed pair: it is not there under replay)
-        res["unfused_us"] = _time_launches_us(lambda w: silu_and_mul_interleaved(linear(x, w, full), half), weights, iters, 3)
-        ranked = sorted((_time_launches_us(lambda w: skinny_linear_silu(x, w, sl, half, nt), weights, iters, 1), (sl, nt))
+        res["unfused_us"] = _time_launches_us(lambda w: silu_and_mul_interleaved(linear(x, w, full), half), weights, iters, 3, ahead=True)
+        ranked = sorted((_time_launches_us(lambda w: skinny_linear_silu(x, w, sl, half, nt), weights, iters, 1, ahead=True), (sl, nt))
                         for sl, nt in skinny_silu_candidates(M, N, K))
-        best = min((_time_launches_us(lambda w: skinny_linear_silu(x, w, p[0], half, p[1]), weights, iters, 3), p)
+        best = min((_time_launches_us(lambda w: skinny_linear_silu(x, w, p[0], half, p[1]), weights, iters, 3, ahead=True), p)
                    for _, p in ranked[:4])
         res.update(fused_us=best[0], plan=best[1], kind="skinny")
         if best[0] < res["unfused_us"]:  # one launch less in front of the same consumer: no margin asked
