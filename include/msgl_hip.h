@@ -317,6 +317,17 @@ int msgl_skinny_gemm_nt(void* out, const void* x, const void* w, int M, int N, i
  * even `slices` (half of the waves stream the gate tile, half the up tile, slices / 2 k-slices each). */
 int msgl_skinny_gemm_silu_nt(void* out, const void* x, const void* w, int M, int N, int K, int64_t ldx,
                              int64_t ldw, int64_t ldo, int dtype, int slices, int row_tiles, void* stream);
+/* The same product with four weight rows per workgroup, for M <= 8 (N % 4 == 0, K % 128 == 0, slices <= K / 128): projections
+ * of so few rows that sixteen per workgroup leave most CUs without work.  Deterministic. */
+int msgl_skinny_quarter_gemm_nt(void* out, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw,
+                                int64_t ldo, int dtype, int slices, void* stream);
+/* fused_add_rmsnorm(x, res_in) -> res_out and the projection of its result (silu: then SiLU.mul, w interleaved, out [M, N / 2])
+ * in one launch, M <= 8: the bits of msgl_fused_add_rmsnorm followed by msgl_skinny_gemm[_silu]_nt with the same slices and
+ * row tiles (1 or 2).  res_out must be another buffer than res_in and x. */
+int msgl_skinny_norm_gemm_supported(int M, int N, int K, int slices, int row_tiles, int silu);
+int msgl_skinny_norm_gemm_nt(void* out, const void* x, const void* w, int M, int N, int K, int64_t ldx, int64_t ldw,
+                             int64_t ldo, int dtype, int slices, int row_tiles, int silu, const void* res_in, void* res_out,
+                             const void* gamma, float eps, int64_t ldr_in, int64_t ldr_out, void* stream);
 
 /* The same product for the smallest decode batches (1 <= M <= 8) as a pure stream of the weight matrix
  * (P/layers/linear.py:32,103,124 at batch sizes 1..8): one 8-wave workgroup per CU reads the consecutive rows

@@ -4,6 +4,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <type_traits>
+
 #include "../../include/msgl_hip.h"
 
 namespace msgl {
@@ -194,6 +196,21 @@ __device__ __forceinline__ U4 pack8(const float (&f)[8]) {
   u.x = Elem<T>::pack(f[0], f[1]); u.y = Elem<T>::pack(f[2], f[3]);
   u.z = Elem<T>::pack(f[4], f[5]); u.w = Elem<T>::pack(f[6], f[7]);
   return u;
+}
+
+// v_mfma_f32_4x4x4_16b: 16 independent blocks of D[4][4] += A[4][4] . B[4][4]; lane 4 b + i holds row i of block b's A, lane
+// 4 b + j column j of its B and of its D
+typedef short mfma_s16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 mfma_f16x4 __attribute__((ext_vector_type(4)));
+typedef float mfma_f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t mfma_u32x2 __attribute__((ext_vector_type(2)));
+template <typename T>
+__device__ __forceinline__ mfma_f32x4 mfma444(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, const mfma_f32x4& c) {
+  const mfma_u32x2 a = {a0, a1}, b = {b0, b1};
+  if constexpr (std::is_same_v<T, BF16>)
+    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(mfma_s16x4, a), __builtin_bit_cast(mfma_s16x4, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(mfma_f16x4, a), __builtin_bit_cast(mfma_f16x4, b), c, 0, 0, 0);
 }
 
 }  // namespace msgl

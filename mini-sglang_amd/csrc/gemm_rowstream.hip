@@ -261,19 +261,7 @@ __global__ __launch_bounds__(kRsThreads, 2) void rowstream_gemm_kernel(const Row
 // LDS [group][wave]; after the stream the eight wave sums are added in wave order.  x rows in LDS are K + 32 elements
 // apart: the four rows a ds_read_b128 touches then sit in different banks.  N % 4 == 0, K % 128 == 0.
 // ------------------------------------------------------------------------------------------------------------------
-typedef short RS4 __attribute__((ext_vector_type(4)));
-typedef _Float16 RH4 __attribute__((ext_vector_type(4)));
 typedef float RF4 __attribute__((ext_vector_type(4)));
-typedef uint32_t RW2 __attribute__((ext_vector_type(2)));
-
-template <typename T>
-__device__ __forceinline__ RF4 mfma444(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1, const RF4& c) {
-  const RW2 a = {a0, a1}, b = {b0, b1};
-  if constexpr (std::is_same_v<T, BF16>)
-    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(RS4, a), __builtin_bit_cast(RS4, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(RH4, a), __builtin_bit_cast(RH4, b), c, 0, 0, 0);
-}
 
 constexpr int kRs4Unit = 128;  // k per unit
 constexpr int kRs4Pad = 32;    // elements between the staged x rows beyond K (64 B: one quarter of the banks)

@@ -77,7 +77,8 @@ def tune_projection_gemms(groups: Sequence[Group], batch_sizes: Sequence[int], m
                          skinny_used=sk["used"], fold_credit_us=sk.get("fold_credit_us", 0.0))
                 if sk["used"]:
                     r["library_best_us"], r["best_us"] = r["best_us"], sk["skinny_us"]
-                    r["kernel"] = (f"msgl::rowstream{'4' if sk['slices'] else ''}_gemm_kernel[{sk['row_tiles']} loads in flight per lane]" if sk["slices"] <= 0 else
+                    r["kernel"] = (f"msgl::skinny_quarter_gemm_kernel[slices {sk['slices']}]" if sk["slices"] > 0 and sk["row_tiles"] == ops.QUARTER_TILE else
+                                   f"msgl::rowstream{'4' if sk['slices'] else ''}_gemm_kernel[{sk['row_tiles']} loads in flight per lane]" if sk["slices"] <= 0 else
                                    f"msgl::skinny_gemm_kernel[slices {sk['slices']}, row tiles {sk['row_tiles']}]")
             if 32 < bs <= ops.WSTREAM_MAX_M and name != "lm_head":  # LDS-shared weight-streaming kernel
                 wsr = ops.wstream_tune(x, ws, r["best_us"])
@@ -131,6 +132,9 @@ def tune_projection_gemms(groups: Sequence[Group], batch_sizes: Sequence[int], m
                     r["best_us"] = rs["fused_us"]  # projection AND activation
                     r["skinny_used"] = True
                     r["kernel"] = "msgl::ro_gemm_kernel<silu>[tiles %d]" % rs["plan"][0]
+            if flags.get("fold") == "norm" and bs <= ops.NORM_LINEAR_MAX_M:
+                # the add + norm in front of this projection inside its launch, against the two launches as planned so far
+                r.update(ops.norm_linear_tune(x, ws, silu=bool(flags.get("silu_interleaved"))))
             ops.register_candidates(name, x, ws[0], r)
             report.append(r)
             if log is not None:

@@ -348,12 +348,27 @@ class DenseDecoder:
         pending: Optional[torch.Tensor] = None
         spare: Optional[torch.Tensor] = None
 
+        # Where the search found it faster (small hidden sizes, batches <= 8) the matrix-core kernel takes the add + norm in front
+        # of qkv, of gate_up with its SiLU.mul (`act`: the launch returns the activated rows) and of the LM head: ops.norm_linear.
+        nl_on = _ROWSTREAM_FUSE and self.fused and self.tp_size == 1 and T <= ops.NORM_LINEAR_MAX_M
+
+        def norm_plan(w: torch.Tensor, act: bool = False):
+            """How the projection by `w` takes the add + norm in front of it: (kind, a, b), or None."""
+            if rs_on and (p := ops.rowstream_planned(T, w, ops.ROWSTREAM_ADD_NORM)):
+                return ("rowstream", *p)
+            if nl_on and (p := ops.norm_linear_planned(T, w, act)):
+                return ("act" if act else "skinny", *p)
+            return None
+
         def norm_into(w: torch.Tensor, y: torch.Tensor, norm_w: torch.Tensor, plan, out=None) -> torch.Tensor:
             nonlocal residual, spare
             if spare is None:
                 spare = torch.empty_like(residual)
-            r = ops.rowstream_linear(y, w, plan[0], out=out, mode=ops.ROWSTREAM_ADD_NORM, res_in=residual, res_out=spare,
-                                     gamma=norm_w, eps=cfg.rms_norm_eps, variant=plan[1])
+            if plan[0] == "rowstream":
+                r = ops.rowstream_linear(y, w, plan[1], out=out, mode=ops.ROWSTREAM_ADD_NORM, res_in=residual, res_out=spare,
+                                         gamma=norm_w, eps=cfg.rms_norm_eps, variant=plan[2])
+            else:
+                r = ops.norm_linear(y, w, plan[1], plan[2], residual, spare, norm_w, cfg.rms_norm_eps, silu=plan[0] == "act", out=out)
             residual, spare = spare, residual
             return r
 
@@ -364,7 +379,7 @@ class DenseDecoder:
             elif not normed_ahead:
                 fi.fused_add_rmsnorm(x, residual, lw.input_norm, cfg.rms_norm_eps)
             if pending is not None:  # the previous layer's down_proj output: add + input norm in the qkv launch
-                qkv, slabs = norm_into(lw.qkv, pending, lw.input_norm, ops.rowstream_planned(T, lw.qkv, ops.ROWSTREAM_ADD_NORM)), None
+                qkv, slabs = norm_into(lw.qkv, pending, lw.input_norm, norm_plan(lw.qkv)), None
                 pending = None
             else:
                 # a k-sliced full-batch plan leaves the qkv projection's reduce to the fused norm / RoPE / store pass
@@ -391,10 +406,10 @@ class DenseDecoder:
             # down_proj feeds the NEXT layer's input norm (or the final norm): its all-reduce / slab reduce joins that norm
             last = li + 1 == len(self.layers)
             nxt = self.final_norm if last else self.layers[li + 1].input_norm
-            d_gu = ops.rowstream_planned(T, lw.gate_up, ops.ROWSTREAM_ADD_NORM) if rs_on else None
+            d_gu = norm_plan(lw.gate_up, act=self.gate_up_ilv)
             act_mode = ops.ROWSTREAM_SILU_INTERLEAVED if self.gate_up_ilv else ops.ROWSTREAM_SILU
             # SiLU.mul in the staging pass pays at one row only (M = 4: 43 vs 39 us for the pair, profiles/r04_rowstream_bench.json)
-            d_dn = ops.rowstream_planned(T, lw.down, act_mode) if rs_on and T <= ops.ROWSTREAM_FOLD_ACT_MAX_M else None
+            d_dn = ops.rowstream_planned(T, lw.down, act_mode) if rs_on and T <= ops.ROWSTREAM_FOLD_ACT_MAX_M and not (d_gu and d_gu[0] == "act") else None
             if d_gu:  # o_proj, then post-attention add + norm inside the gate_up launch
                 gu = norm_into(lw.gate_up, ops.linear(o.view(-1, self.q_dim), lw.o), lw.post_norm, d_gu)
             else:
@@ -402,14 +417,15 @@ class DenseDecoder:
                 gu = None
             # the next consumer of the residual stream (next layer's qkv, or the LM head of a decode batch) takes down_proj's
             # add + norm into its own launch if it can
-            fold_next = (ops.rowstream_planned(T, self.lm_head if last else self.layers[li + 1].qkv, ops.ROWSTREAM_ADD_NORM)
-                         if rs_on and not (last and batch.is_prefill) else None)
+            fold_next = norm_plan(self.lm_head if last else self.layers[li + 1].qkv) if not (last and batch.is_prefill) else None
             if d_dn:  # SiLU.mul while down_proj stages its input
                 if gu is None:
                     gu = ops.linear(x, lw.gate_up)
                 x = ops.rowstream_linear(gu, lw.down, d_dn[0], mode=act_mode, variant=d_dn[1])
             else:
-                if gu is not None:
+                if d_gu and d_gu[0] == "act":
+                    y = gu
+                elif gu is not None:
                     y = ops.silu_and_mul_interleaved(gu) if self.gate_up_ilv else fi.silu_and_mul(gu)
                 elif self.gate_up_ilv:  # projection + SiLU.mul: one launch where planned (P/models/utils.py:45-51)
                     y = ops.linear_silu(x, lw.gate_up)
@@ -425,7 +441,7 @@ class DenseDecoder:
         bs = batch.size
         if pending is not None:  # decode batch: the final add + norm inside the LM head's launch
             out = logits_out if logits_out is not None and logits_out.shape == (T, self.lm_head.shape[0]) else None
-            return norm_into(self.lm_head, pending, self.final_norm, ops.rowstream_planned(T, self.lm_head, ops.ROWSTREAM_ADD_NORM), out)
+            return norm_into(self.lm_head, pending, self.final_norm, norm_plan(self.lm_head), out)
         if batch.is_prefill:
             x = x[batch.attn_metadata.get_last_indices(bs)].contiguous()
         if self.tp_size == 1:

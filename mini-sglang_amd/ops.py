@@ -601,17 +601,117 @@ def rowstream_planned(M: int, w: torch.Tensor, mode: int = 0):
 def skinny_linear(x: torch.Tensor, w: torch.Tensor, slices: int, out: Optional[torch.Tensor] = None,
                   row_tiles: int = 1) -> torch.Tensor:
     """out[M, N] = x[M, K] @ w[N, K]^T by msgl_skinny_gemm_nt (M <= 64).  A plan (0, depth) / (-1, depth) names the
-    row-streaming kernel of the same family (M <= 8, rowstream_linear, variant 0 / 1): the plan tables keep one (a, b) pair
-    per shape."""
+    row-streaming kernel of the same family (M <= 8, rowstream_linear, variant 0 / 1), a plan (slices, QUARTER_TILE) the
+    kernel with four weight rows per workgroup (M <= 8): the plan tables keep one (a, b) pair per shape."""
     if slices <= 0:
         return rowstream_linear(x, w, row_tiles, out, variant=-slices)
     out, M, N, K = _gemm_args(x, w, out)
+    if row_tiles == QUARTER_TILE:
+        check(
+            lib().msgl_skinny_quarter_gemm_nt(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0), w.stride(0),
+                                              out.stride(0), _dt(x), slices, _stream()),
+            "skinny_quarter_gemm_nt",
+        )
+        return out
     check(
         lib().msgl_skinny_gemm_nt(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0), w.stride(0),
                                   out.stride(0), _dt(x), slices, row_tiles, _stream()),
         "skinny_gemm_nt",
     )
     return out
+
+
+QUARTER_TILE = 0  # `row_tiles` of the skinny family's kernel with four weight rows per workgroup
+
+
+QUARTER_MAX_N = 8192  # beyond, sixteen rows per workgroup give every CU more than two (at 4096 rows of 1024: 3.9 us, four rows 4.4)
+
+
+def quarter_candidates(M: int, N: int, K: int):
+    """(k-slices, QUARTER_TILE) settings of the kernel with four weight rows per workgroup (csrc/gemm_skinny.hip)."""
+    if M > ROWSTREAM_MAX_M or N % 4 or K % 128 or N > QUARTER_MAX_N:
+        return []
+    return [(sl, QUARTER_TILE) for sl in (4, 8, 16) if sl <= K // 128]
+
+
+def norm_linear(x: torch.Tensor, w: torch.Tensor, slices: int, row_tiles: int, res_in: torch.Tensor, res_out: torch.Tensor,
+                gamma: torch.Tensor, eps: float, silu: bool = False, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """fused_add_rmsnorm(x, res_in) (new residual written to res_out) and its projection -- silu: and SiLU.mul, w in
+    interleave_gate_up order -- by msgl_skinny_norm_gemm_nt: one launch, the bits of the separate ones (M <= 8)."""
+    _need_cuda(x, w, res_in, res_out, gamma)
+    assert x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.stride(1) == 1 and w.stride(1) == 1
+    M, K = x.shape
+    N = w.shape[0]
+    cols = N // 2 if silu else N
+    assert res_in.shape == x.shape and res_out.shape == x.shape and res_in.stride(1) == 1 and res_out.stride(1) == 1
+    assert gamma.numel() == K and gamma.is_contiguous() and {t.dtype for t in (w, res_in, res_out, gamma)} == {x.dtype}
+    if out is None:
+        out = torch.empty((M, cols), dtype=x.dtype, device=x.device)
+    assert out.shape == (M, cols) and out.stride(1) == 1 and out.dtype == x.dtype and out.is_cuda
+    _no_pending_slabs(x.device)
+    check(
+        lib().msgl_skinny_norm_gemm_nt(out.data_ptr(), x.data_ptr(), w.data_ptr(), M, N, K, x.stride(0), w.stride(0), out.stride(0),
+                                       _dt(x), slices, row_tiles, int(silu), res_in.data_ptr(), res_out.data_ptr(), gamma.data_ptr(),
+                                       float(eps), res_in.stride(0), res_out.stride(0), _stream()),
+        "skinny_norm_gemm_nt",
+    )
+    return out
+
+
+@functools.lru_cache(maxsize=None)
+def norm_linear_supported(M: int, N: int, K: int, slices: int, row_tiles: int, silu: bool = False) -> bool:
+    return bool(lib().msgl_skinny_norm_gemm_supported(M, N, K, slices, row_tiles, int(silu)))
+
+
+# (device, M, N, K, ldx, ldw, dtype code) -> (k-slices, row tiles) of norm_linear, plain / with SiLU.mul
+_SKINNY_NORM_PLAN: dict = {}
+_SKINNY_NORM_SILU_PLAN: dict = {}
+NORM_LINEAR_MAX_M = 8
+
+
+def norm_linear_planned(M: int, w: torch.Tensor, silu: bool = False):
+    """(k-slices, row tiles) if norm_linear_tune found norm_linear faster than the norm and the projection, else None."""
+    table = _SKINNY_NORM_SILU_PLAN if silu else _SKINNY_NORM_PLAN
+    if M > NORM_LINEAR_MAX_M or not table:
+        return None
+    N, K = w.shape
+    return table.get((w.device.index or 0, M, N, K, K, w.stride(0), _dt(w)))
+
+
+def norm_linear_tune(x: torch.Tensor, weights, silu: bool = False, iters: int = 8) -> dict:
+    """Batches <= 8: time fused_add_rmsnorm followed by the projection as it is planned now (silu: `linear_silu`) against
+    norm_linear and plan the latter if it is faster.  A shape whose norm the row-streaming kernel takes stays with that."""
+    weights = list(weights)
+    w0 = weights[0]
+    M, K = x.shape
+    N = w0.shape[0]
+    res = dict(norm_unfused_us=None, norm_fused_us=None, norm_plan=None, norm_used=False)
+    table = _SKINNY_NORM_SILU_PLAN if silu else _SKINNY_NORM_PLAN
+    key = (x.device.index or 0, M, N, K, x.stride(0), w0.stride(0), _dt(x))
+    table.pop(key, None)
+    # (sixteen waves share the norm out no better than eight: 6.2 us where eight take 4.5; they are asked where eight hold too little)
+    settings = [(sl, nt) for sl in (4, 8, 16) for nt in (1, 2) if norm_linear_supported(M, N, K, sl, nt, silu)
+                and not (sl == 16 and norm_linear_supported(M, N, K, 8, nt, silu))]
+    if not settings or (M <= ROWSTREAM_FOLD_NORM_MAX_M and rowstream_planned(M, w0, ROWSTREAM_ADD_NORM)):
+        return res
+    out = torch.empty((M, N // 2 if silu else N), dtype=x.dtype, device=x.device)
+    gamma, r0, r1, y = torch.ones(K, dtype=x.dtype, device=x.device), torch.zeros_like(x), torch.empty_like(x), x.clone()
+
+    def unfused(w):
+        fused_add_rmsnorm(y, r0, gamma, 1e-6)
+        linear_silu(y, w, out) if silu else linear(y, w, out)
+
+    def time_us(p, rounds):
+        return _time_launches_us(lambda w: norm_linear(x, w, p[0], p[1], r0, r1, gamma, 1e-6, silu, out), weights, iters, rounds, ahead=True)
+
+    res["norm_unfused_us"] = _time_launches_us(unfused, weights, iters, 3, ahead=True)
+    ranked = sorted((time_us(p, 1), p) for p in settings)
+    best = min((time_us(p, 3), p) for _, p in ranked[:3])
+    res.update(norm_fused_us=best[0], norm_plan=best[1])
+    if best[0] < res["norm_unfused_us"]:
+        table[key] = best[1]
+        res["norm_used"] = True
+    return res
 
 
 _SKINNY_SILU_PLAN: dict = {}  # (device, M, N, K, ldx, ldw, dtype code), w = interleaved gate_up -> (k-slices, row tiles) of the fused launch
@@ -696,7 +796,7 @@ def skinny_tune(x: torch.Tensor, weights, library_us: float, iters: int = 8, fol
         folds = fold_mode is not None and sl <= 0 and rowstream_supported(M, N, K, fold_mode, -sl)
         return ROWSTREAM_FOLD_BONUS_US if folds else 0.0
 
-    ranked = sorted((time_us(sl, nt, 1) - credit(sl), sl, nt) for sl, nt in skinny_candidates(M, N, K))
+    ranked = sorted((time_us(sl, nt, 1) - credit(sl), sl, nt) for sl, nt in skinny_candidates(M, N, K) + quarter_candidates(M, N, K))
     timed = [(time_us(sl, nt, 3), sl, nt) for _, sl, nt in ranked[:5]]  # re-time the best few
     best = min(timed, key=lambda t: t[0] - credit(t[1]))
     # skinny_us is the MEASURED time of the chosen setting; fold_credit_us is what the ranking subtracted from it because the
@@ -1329,7 +1429,8 @@ def restore_search_pick(key, snap) -> None:
                         "gemm_select_finalist")
 
 
-_PLAN_TABLES = {"skinny": _SKINNY_PLAN, "skinny_silu": _SKINNY_SILU_PLAN, "wstream": _WSTREAM_PLAN, "m256": _M256_PLAN,
+_PLAN_TABLES = {"skinny": _SKINNY_PLAN, "skinny_silu": _SKINNY_SILU_PLAN, "skinny_norm": _SKINNY_NORM_PLAN,
+                "skinny_norm_silu": _SKINNY_NORM_SILU_PLAN, "wstream": _WSTREAM_PLAN, "m256": _M256_PLAN,
                 "fused_silu": _FUSED_SILU_PLAN, "ro": _RO_PLAN, "ro_silu": _RO_SILU_PLAN}
 
 
@@ -1377,6 +1478,8 @@ def reset_gemm_plans() -> None:
     _RO_SILU_PLAN.clear()
     _FUSED_SILU_PLAN.clear()
     _SKINNY_SILU_PLAN.clear()
+    _SKINNY_NORM_PLAN.clear()
+    _SKINNY_NORM_SILU_PLAN.clear()
     _CANDIDATES.clear()
     _PENDING_SLABS.clear()
     _PENDING_ALLREDUCE.clear()
