@@ -198,6 +198,21 @@ int msgl_attn_decode(void* out, const void* q, const void* k_cache, const void* 
                      int max_bs, int capacity, int num_q_heads, int num_kv_heads, int head_dim,
                      int64_t q_stride_tok, int64_t kv_stride_tok, int64_t kv_stride_head,
                      int64_t out_stride_tok, float sm_scale, int slot_run, int dtype, void* stream);
+
+/* Decode attention of a small batch with the new tokens' row work inside: per-head RMSNorm (both weights or nullptr) and NeoX RoPE
+ * (cos_sin [positions][head_dim] = 64 cos | 64 sin, or nullptr with positions nullptr) of the projection's q and k rows, store of k
+ * and v at out_loc, attention over the request's seq_lens[b] keys, the last of which is the new token (page_table[row][seq_lens[b] - 1]
+ * == out_loc[b]).  The stored rows are msgl_qk_norm_rope_store's bits; q, k and v stay as they are.  head_dim 128, at most 8 query
+ * heads per kv head.  `ranges` (msgl_attn_decode_small_ranges) workgroups share a (request, kv head); no plan.  Capturable. */
+int msgl_attn_decode_small_ranges(int batch, int num_kv_heads, int64_t max_seq_len);
+int64_t msgl_attn_decode_small_workspace_bytes(int batch, int ranges, int num_q_heads);
+int msgl_attn_decode_small(void* out, const void* q, const void* k, const void* v, const void* q_norm_w, const void* k_norm_w,
+                           float eps, const int32_t* positions, const float* cos_sin, void* k_cache, void* v_cache,
+                           const int32_t* out_loc, const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
+                           const int32_t* seq_lens, void* workspace, int64_t workspace_bytes, int batch, int ranges,
+                           int num_q_heads, int num_kv_heads, int head_dim, int64_t q_stride, int64_t k_stride, int64_t v_stride,
+                           int64_t kv_stride_tok, int64_t kv_stride_head, int64_t out_stride, float sm_scale, int dtype,
+                           void* stream);
 /* Which partial-attention kernel msgl_attn_decode_plan / msgl_attn_decode use from now on (process-wide; plan and
  * launch must be made under the same choice): 0 = default = the matrix-core kernel for every slot_run (round 6: token-granular
  * tables, slot_run < 16, are gathered by per-lane addresses on the same kernel; whole-line nt requests with K transposed through

@@ -63,6 +63,10 @@ HIP_SIGNATURES = {
         _i,
         [_p, _p, _p, _p, _p, _l, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _l, _l, _l, _l, _f, _i, _i, _p],
     ),
+    "msgl_attn_decode_small_ranges": (_i, [_i, _i, _l]),
+    "msgl_attn_decode_small_workspace_bytes": (_l, [_i, _i, _i]),
+    "msgl_attn_decode_small": (_i, [_p, _p, _p, _p, _p, _p, _f, _p, _p, _p, _p, _p, _p, _l, _p, _p, _p, _l, _i, _i, _i, _i, _i,
+                                    _l, _l, _l, _l, _l, _l, _f, _i, _p]),
     "msgl_attn_prefill": (
         _i,
         [_p, _p, _p, _p, _p, _l, _p, _p, _p, _p, _i, _i, _i, _i, _i, _l, _l, _l, _l, _f, _i, _p, _i, _p],

@@ -78,6 +78,9 @@ def fill_metadata_host(h: np.ndarray, seqlens_q: np.ndarray, seqlens_k: np.ndarr
         h[4 * bs + 2:] = prefill_tile_order(seqlens_q, seqlens_k, tiles, q_tile)
 
 
+SMALL_DECODE_HEADS = 32  # (request, kv head) pairs up to which decode attention takes the small-batch kernel at any length
+
+
 class HipAttnBackend:
     """Paged attention (prefill + decode) over the reference's KV pool and global page table."""
 
@@ -108,6 +111,7 @@ class HipAttnBackend:
         self._cap_rows: Optional[torch.Tensor] = None
         self._cap_plan: Optional[torch.Tensor] = None
         self._cap_cu_q: Optional[torch.Tensor] = None
+        self._cap_planned: set = set()  # captured batch sizes whose attention reads the work plan
 
     # ------------------------------------------------------------------ forward
     def _kv_tokens(self, layer_id: int):
@@ -115,8 +119,39 @@ class HipAttnBackend:
         v = self.kvcache.v_cache(layer_id)
         return k.view(-1, k.shape[-2], k.shape[-1]), v.view(-1, v.shape[-2], v.shape[-1])
 
+    def small_decode(self, batch: Any) -> bool:
+        """Whether the batch's decode attention takes the kernel that does the new tokens' row work itself
+        (csrc/attn_decode_small.hip).  It and the join of its ranges against row work, planned kernel and merge, us a layer in a
+        captured step, 8 kv heads, bf16: 1 request 9.1 / 11.8 at 533 tokens and 16.7 / 68 at 8000, 4 requests 13.7 / 14.1 and
+        34 / 66; 8 requests 15.1 / 14.7 and 60 / 53: its requests are half lines, and it loses once the stream is long.  With 1 or
+        2 kv heads it is ahead up to 64 of them as well (2 x 32 at 2000 tokens: 24 / 27)."""
+        md = batch.attn_metadata
+        if md.max_seqlen_q != 1 or self.head_dim != 128 or self.qo_heads % self.kv_heads or self.qo_heads // self.kv_heads > 8:
+            return False
+        heads = md.batch * self.kv_heads
+        return heads <= SMALL_DECODE_HEADS or (heads <= 2 * SMALL_DECODE_HEADS and (self.kv_heads <= 2 or self.ctx.page_table.shape[1] <= 4096))
+
+    def _attend_small(self, q, k, v, layer_id: int, batch: Any, **row_work) -> torch.Tensor:
+        md: HipAttnMetadata = batch.attn_metadata
+        k_tok, v_tok = self._kv_tokens(layer_id)
+        table = self.ctx.page_table
+        out = torch.empty((q.shape[0], q.shape[1]), dtype=q.dtype, device=q.device)
+        ranges = ops.attn_decode_small_ranges(md.batch, self.kv_heads, table.shape[1])
+        ops.attn_decode_small(out, q, k, v, k_tok, v_tok, batch.out_loc, table, md.req_rows, md.seq_lens, self._workspace, ranges, self.scale, **row_work)
+        return out.view(q.shape[0], self.qo_heads, self.head_dim)
+
+    def attend_new(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_w, k_norm_w, eps: float, positions: torch.Tensor,
+                   cos_sin: torch.Tensor, layer_id: int, batch: Any) -> torch.Tensor:
+        """qk-norm, RoPE, K / V store and attention of a batch that `small_decode` says yes to, from the projection's rows."""
+        return self._attend_small(q, k, v, layer_id, batch, q_norm_w=q_norm_w, k_norm_w=k_norm_w, eps=eps, positions=positions, cos_sin_cache=cos_sin)
+
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_id: int, batch: Any) -> torch.Tensor:
         """Reference contract (fa.py:48-65): persist k, v at batch.out_loc, then attend."""
+        if self.small_decode(batch):
+            q2, k2, v2 = (t.reshape(t.shape[0], -1) for t in (q, k, v))
+            if (batch.out_loc.dtype == torch.int32 and batch.out_loc.is_contiguous() and {t.dtype for t in (q, k, v)} == {self.kvcache.dtype}
+                    and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (q2, k2, v2))):
+                return self._attend_small(q2, k2, v2, layer_id, batch)
         self.kvcache.store_kv(k, v, batch.out_loc, layer_id)
         return self.attend(q, layer_id, batch)
 
@@ -133,6 +168,8 @@ class HipAttnBackend:
                 md.plan = torch.empty(self._plan_words, dtype=torch.int32, device=self.device)
                 ops.attn_decode_plan(md.plan, md.seq_lens, md.batch, self.max_bs, self.capacity, self.qo_heads,
                                      self.kv_heads)
+            elif md.plan is self._cap_plan:
+                self._cap_planned.add(md.batch)
             ops.attn_decode(out, q, k_tok, v_tok, table, md.req_rows, md.seq_lens, md.plan, self._workspace,
                             md.batch, self.max_bs, self.capacity, self.scale, slot_run=self.slot_run)
         else:
@@ -213,7 +250,8 @@ class HipAttnBackend:
         assert isinstance(md, HipAttnMetadata) and bs in self.capture_bs and self._cap_plan is not None
         self._cap_seq[:bs].copy_(md.seq_lens)
         self._cap_rows[:bs].copy_(md.req_rows)
-        ops.attn_decode_plan(self._cap_plan, self._cap_seq, bs, self.max_bs, self.capacity, self.qo_heads, self.kv_heads)
+        if bs in self._cap_planned:
+            ops.attn_decode_plan(self._cap_plan, self._cap_seq, bs, self.max_bs, self.capacity, self.qo_heads, self.kv_heads)
 
 
 class MixAttnBackend:

@@ -36,6 +36,7 @@ HIP_SOURCES = [
     "store_index.hip",
     "norm_rope_act.hip",
     "attn_decode.hip",
+    "attn_decode_small.hip",
     "attn_prefill.hip",
     "sampling.hip",
     "gemm_skinny.hip",

@@ -30,6 +30,7 @@
 
 #include <type_traits>
 
+#include "attn_decode_tile.h"
 #include "common.h"
 
 namespace msgl {
@@ -46,7 +47,6 @@ namespace msgl {
     __builtin_amdgcn_sched_barrier(0);      \
   } while (0)
 
-typedef uint32_t V4 __attribute__((ext_vector_type(4)));
 typedef int I4 __attribute__((ext_vector_type(4)));
 
 // raw buffer descriptor over "everything from base": 48-bit base, stride 0, num_records = 2^32 - 1 bytes
@@ -60,7 +60,6 @@ typedef int I16a __attribute__((ext_vector_type(16), aligned(16)));
 typedef __attribute__((address_space(4))) I16a CI16;
 
 constexpr int kPlanHdr = 4;  // [0] n_items [1] tokens per slot [2] batch [3] n_slots
-constexpr float kNegBig = -3.0e38f;
 
 // plan buffer layout (int32 words):
 //   hdr[4] | item_start[max_bs] | n_chunks[max_bs] | tile_start[max_bs] | slot_first[capacity + 1] |
@@ -557,56 +556,6 @@ attn_decode_kernel(const DecodeParams p) {
 // K/V tiles sit in a ring of kStages register sets: kStages - 1 tiles (8 KB each) in flight per wave while one
 // is consumed.  Work split (plan, slots, pieces), partial layout and merge are those of the streaming kernel.
 // ------------------------------------------------------------------------------
-typedef __attribute__((ext_vector_type(8))) __bf16 dbf16x8;
-typedef __attribute__((ext_vector_type(8))) _Float16 df16x8;
-typedef __attribute__((ext_vector_type(4))) _Float16 df16x4;
-typedef __attribute__((ext_vector_type(4))) short ds16x4;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((address_space(3))) ds16x4 lds_ds16x4;
-typedef __attribute__((address_space(3))) char dlds_char;
-
-template <typename T>
-__device__ __forceinline__ f32x4 mfma_k32(const V4& a, const V4& b, f32x4 c) {
-  if constexpr (std::is_same_v<T, BF16>)
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dbf16x8, a), __builtin_bit_cast(dbf16x8, b), c, 0,
-                                                   0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(df16x8, a), __builtin_bit_cast(df16x8, b), c, 0, 0,
-                                                  0);
-}
-template <typename T>
-__device__ __forceinline__ f32x4 mfma_k16(const uint2& a, const uint2& b, f32x4 c) {
-  if constexpr (std::is_same_v<T, BF16>)
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(ds16x4, a), __builtin_bit_cast(ds16x4, b), c, 0, 0,
-                                                     0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(df16x4, a), __builtin_bit_cast(df16x4, b), c, 0, 0, 0);
-}
-
-// max over the four 16-lane groups (every lane ends with it)
-__device__ __forceinline__ float max_over_rows(float x) {
-  const uint32_t u = __float_as_uint(x);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-  const uint32_t w = __float_as_uint(x);
-  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float sum_over_rows(float x) {
-  const uint32_t u = __float_as_uint(x);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  const uint32_t w = __float_as_uint(x);
-  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
-// V image: [16 tokens][256 B]; 64-B blocks XORed by the token's low two bits, the 32-B half by bit 2: the 32 lanes
-// of one ds_read_b64_tr_b16 pass (16 lanes x 2 groups) then cover 32 distinct 8-B bank pairs
-__device__ __forceinline__ int vimg_off(int tok, int byte_in_row) {
-  return tok * 256 + (byte_in_row ^ ((tok & 3) << 6) ^ (((tok >> 2) & 1) << 5));
-}
-
 // K image (kLines): [16 tokens][256 B], the row's sixteen 16-byte pieces XORed by the token: the 16 lanes of one ds_read_b128
 // pass (one piece index, tokens 0..15) and of one ds_write_b128 pass (one token, pieces 0..15) both cover all 64 banks
 __device__ __forceinline__ int kimg_off(int tok, int piece) { return tok * 256 + (((piece ^ tok) & 15) << 4); }

@@ -350,6 +350,9 @@ class DenseDecoder:
 
         # Where the search found it faster (small hidden sizes, batches <= 8) the matrix-core kernel takes the add + norm in front
         # of qkv, of gate_up with its SiLU.mul (`act`: the launch returns the activated rows) and of the LM head: ops.norm_linear.
+        # A small decode batch: qk-norm, RoPE, K / V store and attention in one launch (the backend says for which batches).
+        small = (self.fused and getattr(batch.attn_metadata, "max_seqlen_q", 0) == 1 and getattr(backend, "small_decode", lambda b: False)(batch)
+                 and batch.positions.dtype == batch.out_loc.dtype == torch.int32)
         nl_on = _ROWSTREAM_FUSE and self.fused and self.tp_size == 1 and T <= ops.NORM_LINEAR_MAX_M
 
         def norm_plan(w: torch.Tensor, act: bool = False):
@@ -385,7 +388,9 @@ class DenseDecoder:
                 # a k-sliced full-batch plan leaves the qkv projection's reduce to the fused norm / RoPE / store pass
                 qkv, slabs = ops.linear_slabs(x, lw.qkv) if self.fused and _SLAB_NORM else (ops.linear(x, lw.qkv), None)
             q, k, v = qkv.split([self.q_dim, self.kv_dim, self.kv_dim], dim=-1)
-            if self.fused:
+            if small and slabs is None:
+                o = backend.attend_new(q, k, v, lw.q_norm, lw.k_norm, cfg.rms_norm_eps, batch.positions, self.cos_sin, li, batch)
+            elif self.fused:
                 kc, vc = kv.k_cache(li), kv.v_cache(li)
                 if slabs is not None:
                     ops.qk_norm_rope_store_slabs(qkv, slabs, self.hq, self.hkv, lw.q_norm, lw.k_norm, cfg.rms_norm_eps,

@@ -352,6 +352,46 @@ def attn_decode(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cac
     )
 
 
+def attn_decode_small_ranges(batch: int, num_kv_heads: int, max_seq_len: int) -> int:
+    n = int(lib().msgl_attn_decode_small_ranges(batch, num_kv_heads, max_seq_len))
+    check(min(n, 0), "attn_decode_small_ranges")
+    return n
+
+
+def attn_decode_small(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                      out_loc: torch.Tensor, page_table: torch.Tensor, req_rows: Optional[torch.Tensor], seq_lens: torch.Tensor,
+                      workspace: torch.Tensor, ranges: int, sm_scale: float, q_norm_w: Optional[torch.Tensor] = None,
+                      k_norm_w: Optional[torch.Tensor] = None, eps: float = 0.0, positions: Optional[torch.Tensor] = None,
+                      cos_sin_cache: Optional[torch.Tensor] = None) -> None:
+    """Decode attention of a small batch with qk-norm, RoPE and the K / V store of the new tokens inside (see msgl_hip.h).
+    out [B, Hq * D], q / k / v [B, H * D] row views, k_cache / v_cache [slots, Hkv, D]."""
+    _need_cuda(out, q, k, v, k_cache, v_cache, out_loc, page_table, seq_lens, workspace)
+    b, hkv, d = q.shape[0], k_cache.shape[1], k_cache.shape[2]
+    assert out.dim() == q.dim() == k.dim() == v.dim() == 2 and out.shape == q.shape and q.shape[1] % d == 0
+    assert k.shape == v.shape == (b, hkv * d) and all(t.stride(1) == 1 for t in (out, q, k, v))
+    assert k_cache.dim() == 3 and k_cache.stride(2) == 1 and v_cache.shape == k_cache.shape and v_cache.stride() == k_cache.stride()
+    assert page_table.dim() == 2 and page_table.stride(1) == 1
+    assert {t.dtype for t in (out_loc, page_table, seq_lens)} == {torch.int32} and out_loc.numel() >= b and seq_lens.numel() >= b
+    assert {t.dtype for t in (out, k, v, k_cache, v_cache)} == {q.dtype}
+    if cos_sin_cache is not None:
+        assert positions is not None and positions.dtype == torch.int32 and positions.numel() >= b and cos_sin_cache.dtype == torch.float32
+        assert cos_sin_cache.is_contiguous() and cos_sin_cache.shape[1] == d
+
+    def ptr(t):
+        return t.data_ptr() if t is not None else None
+
+    check(
+        lib().msgl_attn_decode_small(
+            out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), ptr(q_norm_w), ptr(k_norm_w), float(eps),
+            ptr(positions if cos_sin_cache is not None else None), ptr(cos_sin_cache), k_cache.data_ptr(), v_cache.data_ptr(),
+            out_loc.data_ptr(), page_table.data_ptr(), page_table.stride(0), ptr(req_rows), seq_lens.data_ptr(), workspace.data_ptr(),
+            workspace.numel() * workspace.element_size(), b, ranges, q.shape[1] // d, hkv, d, q.stride(0), k.stride(0), v.stride(0),
+            k_cache.stride(0), k_cache.stride(1), out.stride(0), float(sm_scale), _dt(q), _stream(),
+        ),
+        "attn_decode_small",
+    )
+
+
 def attn_decode_select(impl: int) -> None:
     """0: default kernel choice, 1: streaming (VALU) kernel only -- msgl_attn_decode_select (A/B timing, tests)."""
     check(lib().msgl_attn_decode_select(int(impl)), "attn_decode_select")
