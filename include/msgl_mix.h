@@ -169,7 +169,7 @@ int msgl_mix_delta_rule(float* out, const float* qkv, float* state, const void* 
                         float* scratch, void* stream);
 
 /* The same rule in blocks of 16 tokens on the fp32 matrix instructions, for portions of tokens: everything that does not depend on the
- * state is computed for all blocks at once, then one walk per (request, head, 32 value columns).  Any batch; no chunk list.
+ * state is computed for all blocks at once, then one walk per (request, head, 16 value columns).  Any batch; no chunk list.
  * msgl_mix_delta_rule_block_floats: floats of a block and head, 0 where these sizes have no such form (d 64 or 128, dv a multiple of 32);
  * scratch holds (total_q / 16 + batch) * H of them. */
 int msgl_mix_delta_rule_block_floats(int d, int dv);

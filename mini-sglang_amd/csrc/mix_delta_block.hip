@@ -6,19 +6,20 @@
 //   (I + A) u = beta (v - (P k) S),  A_{tj} = beta_t sum_c k_tc R_{tj,c} k_jc  (j < t)
 //   o = (P q) S + Q u,               Q_{tj} = sum_c q_tc R_{tj,c} k_jc         (j <= t)
 //   S' = P_16 S + (R_{16,j} k_j)^T u
-// delta_block_kernel computes, for all blocks at once, W = (I + A)^-1 beta (P k), U = (I + A)^-1 beta v, P q, Q, R_{16} k, P_16;
-// delta_walk_kernel walks a request's blocks: u = U - W S, o = (P q) S + Q u, S = P_16 S + (R_{16} k)^T u.
+// delta_block_kernel computes, for all blocks at once, T = (I + A)^-1 beta, W = T (P k), P q, Q, R_{16} k, P_16;
+// delta_walk_kernel walks a request's blocks: u = T v - W S, o = (P q) S + Q u, S = P_16 S + (R_{16} k)^T u.
 //
 // Everything stays fp32: v_mfma_f32_16x16x4_f32 multiplies and adds in fp32.  Ratios of decays are products of at most 15 decays, never
 // quotients or exponentials of sums (an exponential of a sum of logarithms loses the digits that the sum's size takes): the pairs (t, j)
 // split by the highest bit in which t and j differ, and per level both factors are running products inside a half block.
 //
-// What bounds it: the walk is a serial chain of blocks per (request, head), 50 fp32 MFMAs of 32 cycles a wave and block plus the meeting in
-// LDS (1.4 us a block measured); the block kernel is bound by its instructions (5 waves per SIMD of them at a time) and by memory (49 d + 256 +
-// 16 dv floats a block and head written, and read again by the walk).  The token loop was bound by one wave's serial walk: two passes over
-// 128 registers a token, in three launches.
-// 4 requests of 1500 - 2548 tokens, 16 heads, d = dv = 128, decays per channel: 4038 -> 389 us (blocks 171, walk 219); error against 64
-// bits 1.9e-7 -> 1.4e-7.
+// What bounds it: the walk is a serial chain of blocks per (request, head), 25 fp32 MFMAs of 32 cycles a wave and block and the meeting in
+// LDS (1650 cycles a block of a chain alone, 2900 with two on a CU, whose operands, 27 KB a block and chain, come from L2 at 10 TB/s in
+// all); the block kernel by memory (49 d + 512 floats a block and head written, and read again by the walk; values are read by the walk
+// itself).  The token loop was bound by one wave's serial walk: two passes over 128 registers a token, in three launches.
+// 4 requests of 1500 - 2548 tokens, 16 heads, d = dv = 128, decays per channel, us (blocks, walk): 4038 in the token loop; 389 (171, 219) with
+// (I + A)^-1 beta v solved and stored per value column, operands in rows of d and 32 columns a workgroup; 306 (100, 207) now.  One request
+// of 900 tokens, 8 heads: 100 -> 62.  Error against 64 bits 1.9e-7 -> 1.4e-7 -> 1.1e-7.
 #include <type_traits>
 
 #include "mix_common.h"
@@ -47,16 +48,18 @@ __device__ __forceinline__ float decay_of(float r, float z, const bf16_t*) {
 
 constexpr int kBT = 16;  // tokens per block
 
-// a block's operands of one head in the scratch, in floats
+// A block's operands of one head in the scratch, in floats: 16 x 16 tiles in the order in which the walk's lanes (lr = lane & 15, lg =
+// lane >> 4) take them, 16 bytes a lane, so that a wave's load is one kilobyte in a row.  (Rows of d floats made every sixteen
+// lanes of a load touch sixteen lines, and the walk waited for the address unit.)
 struct BlockPart {
-  int d, dv;
-  __host__ __device__ int w() const { return 0; }                  // W        [16][d]
-  __host__ __device__ int q() const { return kBT * d; }            // P q      [16][d]
-  __host__ __device__ int k() const { return 2 * kBT * d; }        // R_16 k   [d][16]
-  __host__ __device__ int p() const { return 3 * kBT * d; }        // P_16     [d]
-  __host__ __device__ int qk() const { return 3 * kBT * d + d; }   // Q        [16][16]
-  __host__ __device__ int u() const { return 3 * kBT * d + d + kBT * kBT; }  // U [16][dv]
-  __host__ __device__ int size() const { return 3 * kBT * d + d + kBT * kBT + kBT * dv; }
+  int d;
+  __host__ __device__ int w() const { return 0; }                           // -W    [d / 16][lane][4]: token lr, channels 4 lg ...
+  __host__ __device__ int q() const { return kBT * d; }                     // P q   likewise
+  __host__ __device__ int k() const { return 2 * kBT * d; }                 // R_16 k [d / 16][lane][4]: channel lr, tokens 4 lg ...
+  __host__ __device__ int p() const { return 3 * kBT * d; }                 // P_16  [d]
+  __host__ __device__ int qk() const { return 3 * kBT * d + d; }            // Q     [lane][4]: token lr, tokens 4 lg ...
+  __host__ __device__ int t() const { return 3 * kBT * d + d + kBT * kBT; } // T     [4][lane]: token lr, token 4 lg + first index
+  __host__ __device__ int size() const { return 3 * kBT * d + d + 2 * kBT * kBT; }
 };
 
 // One workgroup of D threads per (block, head); thread = key channel (and value column).
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(D, 4) void delta_block_kernel(float* __restrict__ s
                                                         int dv) {
   constexpr int LD = D + 4, NWAVE = D / 64;  // rows padded so that 16 rows' 16-byte reads cover all banks
   __shared__ __attribute__((aligned(16))) float sx[48 * LD];
-  __shared__ __attribute__((aligned(16))) float sa[kBT][20], sq[kBT][kBT];
+  __shared__ __attribute__((aligned(16))) float sa[kBT][20], sq[kBT][20];
   __shared__ float sbeta[kBT], sg[kBT];
   const uint32_t c = threadIdx.x;  // unsigned: a uniform row plus a 32-bit offset is one address register
   const int lane = c & 63, wave = __builtin_amdgcn_readfirstlane((int)(c >> 6)), lr = lane & 15, lg = lane >> 4;
@@ -78,7 +81,7 @@ __global__ __launch_bounds__(D, 4) void delta_block_kernel(float* __restrict__ s
   const int t0 = __builtin_amdgcn_readfirstlane(cu_q[b]) + __builtin_amdgcn_readfirstlane(tok0);
   const int nt = min(kBT, __builtin_amdgcn_readfirstlane(cu_q[b + 1]) - t0), C = 2 * G * D + H * dv;
   auto token = [&](int t) { return (size_t)(t0 + min(t, nt - 1)); };  // rows past the portion: the last one again, selected away
-  const BlockPart part{D, dv};
+  const BlockPart part{D};
   float* dst = scratch + ((size_t)blockIdx.x * H + h) * part.size();
   const float r = rate[h];
   // tokens past the portion: nothing read, nothing added, nothing forgotten
@@ -232,9 +235,9 @@ __global__ __launch_bounds__(D, 4) void delta_block_kernel(float* __restrict__ s
     }
   }
   __syncthreads();
-  // x = (I + A)^-1 x and y = (I + A)^-1 y, row after row; every thread its own columns, A's rows the same words for all.  The fences keep
-  // the rows' reads apart: all of A read ahead is 144 registers, and half the waves.
-  auto solve = [&](float (&x)[kBT], float (&y)[kBT]) {
+  // x = (I + A)^-1 x (and y = (I + A)^-1 y), row after row; every thread its own columns, A's rows the same words for all.  The fences
+  // keep the rows' reads apart: all of A read ahead is 144 registers, and half the waves.
+  auto solve = [&](float (&x)[kBT], float (&y)[kBT], auto both) {
 #pragma unroll
     for (int t = 1; t < kBT; ++t) {
 #pragma unroll
@@ -244,60 +247,69 @@ __global__ __launch_bounds__(D, 4) void delta_block_kernel(float* __restrict__ s
         for (int i = 0; i < 4; ++i)
           if (j4 + i < t) {
             x[t] = fmaf(-a[i], x[j4 + i], x[t]);
-            y[t] = fmaf(-a[i], y[j4 + i], y[t]);
+            if constexpr (both) y[t] = fmaf(-a[i], y[j4 + i], y[t]);
           }
       }
       asm volatile("" : "+v"(x[t]), "+v"(y[t]) : : "memory");
     }
   };
 #pragma unroll
-  for (int t = 0; t < kBT; ++t) (dst + part.q() + t * D)[c] = q[t] * P[t];
+  for (int t = 0; t < kBT; ++t) sx[(16 + t) * LD + c] = q[t] * P[t];
   (dst + part.p())[c] = P[kBT - 1];
 #pragma unroll
   for (int t4 = 0; t4 < kBT; t4 += 4)
-    *reinterpret_cast<f32x4_t*>(dst + part.k() + t4 + c * kBT) = f32x4_t{k[t4] * S[t4], k[t4 + 1] * S[t4 + 1], k[t4 + 2] * S[t4 + 2], k[t4 + 3] * S[t4 + 3]};
+    *reinterpret_cast<f32x4_t*>(dst + part.k() + (c >> 4) * 256 + t4 * 16 + (c & 15) * 4) =
+        f32x4_t{k[t4] * S[t4], k[t4 + 1] * S[t4 + 1], k[t4 + 2] * S[t4 + 2], k[t4 + 3] * S[t4 + 3]};
 #pragma unroll
   for (int t = 0; t < kBT; ++t) k[t] *= sbeta[t] * P[t];
-  for (uint32_t i = c; i < (uint32_t)(kBT * kBT); i += D) (dst + part.qk())[i] = sq[i >> 4][i & 15];
+  if (wave == 0) *reinterpret_cast<f32x4_t*>(dst + part.qk() + lane * 4) = *reinterpret_cast<const f32x4_t*>(&sq[lr][4 * lg]);
   __builtin_amdgcn_sched_barrier(0);
-  // the key column goes along with the first value column (again with the others: dv > d is rare)
-#pragma unroll 1
-  for (uint32_t e = c; e < (uint32_t)max(dv, D); e += D) {
-    float v[kBT], x[kBT];
+  // the columns of T go along with the first wave's key columns
+  float y[kBT];
+  if (wave == 0) {
 #pragma unroll
-    for (int t = 0; t < kBT; ++t) {
-      v[t] = (qkv + token(t) * C + 2 * G * D + h * dv)[e < (uint32_t)dv ? e : 0u];
-      v[t] = t < nt ? sbeta[t] * v[t] : 0.f;
-      x[t] = k[t];
-    }
-    solve(x, v);
+    for (int t = 0; t < kBT; ++t) y[t] = c == (uint32_t)t ? sbeta[t] : 0.f;
+    solve(k, y, std::true_type{});
+    if (c < (uint32_t)kBT) {
 #pragma unroll
-    for (int t = 0; t < kBT; ++t) {
-      if (e < (uint32_t)dv) (dst + part.u() + t * dv)[e] = v[t];
+      for (int t = 0; t < kBT; ++t) (dst + part.t())[(c & 3) * 64 + (c >> 2) * 16 + t] = y[t];
     }
-    if (e == c) {
+  } else {
+    solve(k, k, std::false_type{});
+  }
 #pragma unroll
-      for (int t = 0; t < kBT; ++t) (dst + part.w() + t * D)[c] = x[t];
-    }
+  for (int t = 0; t < kBT; ++t) sx[t * LD + c] = -k[t];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < D / 16 / NWAVE; ++i) {
+    const int tile = wave * (D / 16 / NWAVE) + i;
+    *reinterpret_cast<f32x4_t*>(dst + part.w() + tile * 256 + lane * 4) = *reinterpret_cast<const f32x4_t*>(sx + lr * LD + 16 * tile + 4 * lg);
+    *reinterpret_cast<f32x4_t*>(dst + part.q() + tile * 256 + lane * 4) = *reinterpret_cast<const f32x4_t*>(sx + (16 + lr) * LD + 16 * tile + 4 * lg);
   }
 }
 
-// One workgroup per (request, head, 32 value columns), five waves.  Waves 0 - 3: wave w holds the state rows w D / 4 ... of the 32
-// columns as MFMA accumulators (lane: rows 4 lg + i, column lr), which are second operands as they stand: contraction index = state row,
-// the first operands' 16-byte reads follow the same order.  W S and (P q) S are sums over all rows, so the waves' shares meet in LDS
-// once a block; every wave then has u, in the layout the update takes it.  Wave 4 adds Q u and writes a block's outputs, one block
-// behind: it takes everything from LDS, so that the waves which load the next blocks' operands have no stores among their loads (with
-// them the compiler waited for every load in flight in front of each block: 338 us where the kernel now takes 240).
+// One workgroup per (request, head, 16 value columns), five waves.  Waves 0 - 3: wave w holds the state rows w D / 4 ... of the columns as
+// MFMA accumulators (lane: rows 4 lg + i, column lr), which are second operands as they stand: contraction index = state row, the first
+// operands' reads follow the same order.  u = T v - W S and (P q) S are sums over tokens and rows: wave w adds the tokens 4 g + w (one
+// product) and its own rows, and the waves' shares meet in LDS once a block, behind the products of (P q) S; every wave then has u, in the
+// layout the update takes it.  Wave 4 adds Q u and writes a block's outputs, one block behind: it takes everything from LDS, so that the waves
+// which load the next blocks' operands have no stores among their loads (with them the compiler waited for every load in flight in front of
+// each block), and no loads of its own, whose waits would be for the stores before them.
+// At most 128 registers, so that two workgroups share a CU: wave 4 goes to the SIMD of wave 0, and with more the second workgroup waited for
+// the first to end.  32 columns a workgroup read half as much and take 215 us for 207 (200 for 181 at 8 requests of 300 - 1000 tokens): one
+// chain's meeting is not hidden by another's products.
 template <int D>
-__global__ __launch_bounds__(320) void delta_walk_kernel(float* __restrict__ out, float* __restrict__ state, const float* __restrict__ scratch,
-                                                         const int* __restrict__ cu_q, const int* __restrict__ seq_lens,
-                                                         const int* __restrict__ slots, int B, int H, int dv) {
+__global__ __launch_bounds__(320, 4) void delta_walk_kernel(float* __restrict__ out, float* __restrict__ state, const float* __restrict__ scratch,
+                                                            const float* __restrict__ qkv, const int* __restrict__ cu_q,
+                                                            const int* __restrict__ seq_lens, const int* __restrict__ slots, int B, int H, int G,
+                                                            int dv) {
   constexpr int NT = D / 64;  // 16-row tiles of a wave
-  __shared__ __attribute__((aligned(16))) f32x4_t share_u[2][4][2][64], share_o[3][4][2][64];  // [image][wave][column tile][lane]
-  __shared__ __attribute__((aligned(16))) f32x4_t full_u[2][2][64], full_qk[2][64];
+  __shared__ __attribute__((aligned(16))) f32x4_t share_u[2][4][64], share_o[3][4][64];  // [image][wave][lane]
+  __shared__ __attribute__((aligned(16))) f32x4_t full_u[2][64], full_qk[3][64];
+  __shared__ __attribute__((aligned(16))) float decays[2][4][32];  // a wave's own
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lr = lane & 15, lg = lane >> 4;
   // the column blocks of a head read the same operands: neighbours in one XCD's L2 where the heads divide by the eight of them
-  const int ncb = dv / 32, groups = B * H;
+  const int ncb = dv / 16, groups = B * H;
   int g, cb;
   if (groups % 8 == 0) {
     const int rest = (int)blockIdx.x >> 3;
@@ -307,165 +319,167 @@ __global__ __launch_bounds__(320) void delta_walk_kernel(float* __restrict__ out
     g = (int)blockIdx.x / ncb;
     cb = (int)blockIdx.x % ncb;
   }
-  const int b = g / H, h = g - b * H, c0 = cb * 32;
+  const int b = g / H, h = g - b * H, c0 = cb * 16;
   const int first = cu_q[b], n_new = cu_q[b + 1] - first;
   if (n_new <= 0) return;
   const int nblk = (n_new + kBT - 1) / kBT;
-  if (wave == 4) {
-    float* orow = out + ((size_t)first + 4 * lg) * H * dv + (size_t)h * dv + c0 + lr;
-    __syncthreads();
-    for (int n = 0; n < nblk; ++n, orow += (size_t)kBT * H * dv) {
-      __syncthreads();
-      const f32x4_t qk = full_qk[n & 1][lane];
-      float zero = 0.f;
-#pragma unroll
-      for (int ct = 0; ct < 2; ++ct) {
-        const f32x4_t u = full_u[n & 1][ct][lane];
-        f32x4_t o{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(qk[e], u[e], o, 0, 0, 0);
-#pragma unroll
-        for (int w = 0; w < 4; ++w) o += share_o[n % 3][w][ct][lane];
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n * kBT + 4 * lg + e < n_new) orow[(size_t)e * H * dv + 16 * ct] = o[e];
-        zero = fmaf(o[0], 0.f, zero);
-      }
-      // Q's upper triangle is zeros, so a u that is not finite spoils its column for all tokens of the block, also those before it (zero times
-      // infinity), and one token's number shows it: then the outputs again, each token without the u behind it
-      if (__builtin_amdgcn_ballot_w64(zero != 0.f) != 0) {
-        const float* qs = reinterpret_cast<const float*>(full_qk[n & 1]);
-#pragma unroll 1
-        for (int x = 0; x < 8; ++x) {
-          const int e = x & 3, ct = x >> 2, t = 4 * lg + e;
-          const float* us = reinterpret_cast<const float*>(full_u[n & 1][ct]);
-          float o = 0.f;
-          for (int j = 0; j <= t; ++j) {
-            const int at = (j >> 2) * 64 + (j & 3);  // a lane's four numbers are tokens 4 lg ... of row or column lr
-            o = fmaf(qs[at + t * 4], us[at + lr * 4], o);
-          }
-          for (int w = 0; w < 4; ++w) o += reinterpret_cast<const float*>(share_o[n % 3][w][ct])[lane * 4 + e];
-          if (n * kBT + t < n_new) orow[(size_t)e * H * dv + 16 * ct] = o;
-        }
-      }
-    }
-    return;
-  }
   int blk = 0;  // blocks of the requests before this one
   for (int i = lane; i < b; i += 64) blk += (cu_q[i + 1] - cu_q[i] + kBT - 1) / kBT;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) blk += __shfl_xor(blk, o, 64);
   blk = __builtin_amdgcn_readfirstlane(blk);
-  const int r0 = wave * (D / 4);
-  const BlockPart part{D, dv};
-  const size_t step = (size_t)H * part.size();
+  const BlockPart part{D};
+  const uint32_t step = (uint32_t)(H * part.size());
   const float* src = scratch + ((size_t)blk * H + h) * part.size();
+  const f32x4_t none{0.f, 0.f, 0.f, 0.f};
+  if (wave == 4) {
+    float* orow = out + ((size_t)first + 4 * lg) * H * dv + (size_t)h * dv + c0 + lr;
+    __syncthreads();
+    for (int n = 0; n < nblk; ++n, orow += (size_t)kBT * H * dv) {
+      __syncthreads();
+      const f32x4_t u = full_u[n & 1][lane], qk = full_qk[n % 3][lane];
+      f32x4_t o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qk[0], u[0], none, 0, 0, 0), o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qk[1], u[1], none, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qk[2], u[2], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qk[3], u[3], o1, 0, 0, 0);
+      f32x4_t o = share_o[n % 3][0][lane];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) o += share_o[n % 3][w][lane];
+      o += o0 + o1;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n * kBT + 4 * lg + e < n_new) orow[(size_t)e * H * dv] = o[e];
+      // Q's upper triangle is zeros, so a u that is not finite spoils its column for all tokens of the block, also those before it (zero times
+      // infinity), and one token's number shows it: then the outputs again, each token without the u behind it
+      if (__builtin_amdgcn_ballot_w64(fmaf(o[0], 0.f, 0.f) != 0.f) != 0) {
+        const float* qs = reinterpret_cast<const float*>(full_qk[n % 3]);
+        const float* us = reinterpret_cast<const float*>(full_u[n & 1]);
+#pragma unroll 1
+        for (int e = 0; e < 4; ++e) {
+          const int t = 4 * lg + e;
+          float x = 0.f;
+          for (int j = 0; j <= t; ++j) {
+            const int at = (j >> 2) * 64 + (j & 3);  // a lane's four numbers are tokens 4 lg ... of row or column lr
+            x = fmaf(qs[at + t * 4], us[at + lr * 4], x);
+          }
+          for (int w = 0; w < 4; ++w) x += reinterpret_cast<const float*>(share_o[n % 3][w])[lane * 4 + e];
+          if (n * kBT + t < n_new) orow[(size_t)e * H * dv] = x;
+        }
+      }
+    }
+    return;
+  }
+  const int r0 = wave * (D / 4);
   float* Srow = state + ((size_t)slots[b] * H + h) * D * dv + c0 + lr;
   const bool fresh = seq_lens[b] == n_new;
-  f32x4_t S[NT][2];
+  f32x4_t S[NT];
 #pragma unroll
   for (int i = 0; i < NT; ++i)
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) S[i][ct][e] = fresh ? 0.f : Srow[(size_t)(r0 + 16 * i + 4 * lg + e) * dv + 16 * ct];
+    for (int e = 0; e < 4; ++e) S[i][e] = fresh ? 0.f : Srow[(size_t)(r0 + 16 * i + 4 * lg + e) * dv];
   struct Ops {
-    f32x4_t w[NT], q[NT], k[NT], p[NT], u[2], qk;
+    f32x4_t w[NT], q[NT], k[NT];
+    float t, v, p, qk;
   };
-  // this lane's places in a block's operands
-  const uint32_t at_w = part.w() + lr * D + r0 + 4 * lg, at_q = at_w + part.q(), at_k = part.k() + (r0 + lr) * kBT + 4 * lg, at_p = part.p() + r0 + 4 * lg,
-                 at_u = part.u() + 4 * lg * dv + c0 + lr, at_qk = part.qk() + lr * kBT + 4 * lg;
-  auto fetch = [&](Ops& x, int n) {
-    const float* at = src + (size_t)min(n, nblk - 1) * step;
+  // this lane's places in a block's operands; its value is of token 4 lg + wave
+  const uint32_t at_w = part.w() + wave * NT * 256 + lane * 4, at_q = at_w + part.q(), at_k = at_w + part.k(), at_t = part.t() + wave * 64 + lane,
+                 at_p = part.p() + r0 + (lane & (D / 4 - 1)), at_qk = part.qk() + lane * 4 + wave;
+  const int C = 2 * G * D + H * dv;
+  const float* vrow = qkv + (size_t)first * C + 2 * G * D + (size_t)h * dv + c0 + lr;
+  // Operands are requested two blocks ahead (a block takes less than a loaded memory system's latency), each into the registers of the
+  // block that has just used them: all at once they held the wave up for 500 cycles.
+  auto at_block = [&](int n) { return src + (uint64_t)(uint32_t)min(n, nblk - 1) * step; };
+  auto fetch_w = [&](Ops& x, int n) __attribute__((always_inline)) {
+    const float* at = at_block(n);
+    const int m = min(n, nblk - 1) * kBT;
+    x.t = at[at_t];
+    x.p = at[at_p];
+    x.qk = at[at_qk];
+    x.v = (vrow + (size_t)m * C)[(uint32_t)(min(4 * lg + wave, n_new - 1 - m) * C)];
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      x.w[i] = *reinterpret_cast<const f32x4_t*>(at + at_w + 16 * i);
-      x.q[i] = *reinterpret_cast<const f32x4_t*>(at + at_q + 16 * i);
-      x.k[i] = *reinterpret_cast<const f32x4_t*>(at + at_k + 16 * i * kBT);
-      x.p[i] = *reinterpret_cast<const f32x4_t*>(at + at_p + 16 * i);
+    for (int i = 0; i < NT; ++i) x.w[i] = *reinterpret_cast<const f32x4_t*>(at + at_w + 256 * i);
+  };
+  auto fetch_q = [&](Ops& x, int n) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) x.q[i] = *reinterpret_cast<const f32x4_t*>(at_block(n) + at_q + 256 * i);
+  };
+  auto fetch_k = [&](Ops& x, int n) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i) x.k[i] = *reinterpret_cast<const f32x4_t*>(at_block(n) + at_k + 256 * i);
+  };
+  auto block = [&](Ops& x, int n, auto tail) __attribute__((always_inline)) {
+    float v = x.v;
+    if (tail) v = n * kBT + 4 * lg + wave < n_new ? v : 0.f;
+    f32x4_t pv, pu[NT], po[NT];  // T v stays out of the sums of W S until these are whole: they are the smaller numbers
+    pv = __builtin_amdgcn_mfma_f32_16x16x4f32(x.t, v, none, 0, 0, 0);
+    auto with_state = [&](f32x4_t (&acc)[NT], const f32x4_t (&first)[NT], int e) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(first[i][e], S[i][e], e ? acc[i] : none, 0, 0, 0);
+    };
+#pragma unroll
+    for (int e = 0; e < 4; ++e) with_state(pu, x.w, e);
+    if (__builtin_amdgcn_ballot_w64(fmaf(v, 0.f, 0.f) != 0.f) != 0) {
+      // a value that is no number: the zeros of the upper triangle would carry it to the tokens before its own
+#pragma unroll 1
+      for (int e = 0; e < 4; ++e) {
+        float sum = 0.f;
+        for (int gj = 0; gj < 4; ++gj) {
+          const float vj = __shfl(v, gj * 16 + lr, 64), tj = __shfl(x.t, gj * 16 + 4 * lg + e, 64);
+          if (4 * gj + wave <= 4 * lg + e) sum = fmaf(tj, vj, sum);
+        }
+        pv[0] = e == 0 ? sum : pv[0];
+        pv[1] = e == 1 ? sum : pv[1];
+        pv[2] = e == 2 ? sum : pv[2];
+        pv[3] = e == 3 ? sum : pv[3];
+      }
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+    for (int i = 0; i < NT; ++i) pv += pu[i];
+    share_u[n & 1][wave][lane] = pv;
+    if (lane < D / 4) decays[n & 1][wave][lane] = x.p;
+    reinterpret_cast<float*>(full_qk[n % 3])[lane * 4 + wave] = x.qk;
+    fetch_w(x, n + 2);
 #pragma unroll
-      for (int ct = 0; ct < 2; ++ct) x.u[ct][e] = (at + at_u + e * dv)[16 * ct];
-    x.qk = *reinterpret_cast<const f32x4_t*>(at + at_qk);
-  };
-  auto block = [&](const Ops& x, int n, auto tail) __attribute__((always_inline)) {
-    f32x4_t pu[2], po[2];
+    for (int e = 0; e < 4; ++e) with_state(po, x.q, e);
+    fetch_q(x, n + 2);
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) pu[ct] = po[ct] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NT; ++i) S[i] *= *reinterpret_cast<const f32x4_t*>(&decays[n & 1][wave][16 * i + 4 * lg]);
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) pu[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[i][e], S[i][ct][e], pu[ct], 0, 0, 0);
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) share_u[n & 1][wave][ct][lane] = pu[ct];
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) po[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][e], S[i][ct][e], po[ct], 0, 0, 0);
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) share_o[n % 3][wave][ct][lane] = po[ct];
+    for (int i = 1; i < NT; ++i) po[0] += po[i];
+    share_o[n % 3][wave][lane] = po[0];
     __syncthreads();  // a wave is at most one block ahead of another, wave 4 one block behind: two and three images are enough
-    f32x4_t u[2];
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
-      u[ct] = x.u[ct];
-#pragma unroll
-      for (int w = 0; w < 4; ++w) u[ct] -= share_u[n & 1][w][ct][lane];
-    }
+    f32x4_t u = (pv + share_u[n & 1][wave ^ 1][lane]) + (share_u[n & 1][wave ^ 2][lane] + share_u[n & 1][wave ^ 3][lane]);
     if (tail && (n + 1) * kBT > n_new) {  // rows past the portion are zero also where a value before them is infinite
 #pragma unroll
-      for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) u[ct][e] = n * kBT + 4 * lg + e < n_new ? u[ct][e] : 0.f;
+      for (int e = 0; e < 4; ++e) u[e] = n * kBT + 4 * lg + e < n_new ? u[e] : 0.f;
     }
-    if (wave == 0) {
-      full_u[n & 1][0][lane] = u[0];
-      full_u[n & 1][1][lane] = u[1];
-      full_qk[n & 1][lane] = x.qk;
-    }
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-      for (int ct = 0; ct < 2; ++ct) S[i][ct] *= x.p[i];
+    if (wave == 0) full_u[n & 1][lane] = u;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) S[i][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][e], u[ct][e], S[i][ct], 0, 0, 0);
+      for (int i = 0; i < NT; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][e], u[e], S[i], 0, 0, 0);
+    fetch_k(x, n + 2);
   };
-  // operands are requested two blocks ahead: a block takes less than a loaded memory system's latency
-  Ops x0, x1, x2;
-  fetch(x0, 0);
-  fetch(x1, 1);
+  Ops x0, x1;
+  fetch_w(x0, 0);
+  fetch_q(x0, 0);
+  fetch_k(x0, 0);
+  fetch_w(x1, 1);
+  fetch_q(x1, 1);
+  fetch_k(x1, 1);
   int n = 0;
   const std::false_type within;
-  for (; n + 3 < nblk; n += 3) {
-    fetch(x2, n + 2);
+  for (; n + 2 < nblk; n += 2) {
     block(x0, n, within);
-    fetch(x0, n + 3);
     block(x1, n + 1, within);
-    fetch(x1, n + 4);
-    block(x2, n + 2, within);
   }
-  const std::true_type tail;  // the last one to three blocks: only they look for the portion's end
-  fetch(x2, n + 2);
+  const std::true_type tail;  // the last one or two blocks: only they look for the portion's end
   block(x0, n, tail);
   if (n + 1 < nblk) block(x1, n + 1, tail);
-  if (n + 2 < nblk) block(x2, n + 2, tail);
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NT; ++i)
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) Srow[(size_t)(r0 + 16 * i + 4 * lg + e) * dv + 16 * ct] = S[i][ct][e];
+    for (int e = 0; e < 4; ++e) Srow[(size_t)(r0 + 16 * i + 4 * lg + e) * dv] = S[i][e];
 }
 
 }  // namespace
@@ -474,7 +488,7 @@ extern "C" {
 
 int msgl_mix_delta_rule_block_floats(int d, int dv) {
   if ((d != 64 && d != 128) || dv < 32 || dv % 32) return 0;
-  return (int)BlockPart{d, dv}.size();
+  return (int)BlockPart{d}.size();
 }
 
 int msgl_mix_delta_rule_blocks(float* out, const float* qkv, float* state, const void* b_raw, int64_t ld_b, const void* a_raw, int64_t ld_a,
@@ -501,9 +515,9 @@ int msgl_mix_delta_rule_blocks(float* out, const float* qkv, float* state, const
 #undef DB_LAUNCH
   MIX_LAUNCHED("delta_rule_blocks");
   if (d == 128)
-    hipLaunchKernelGGL((delta_walk_kernel<128>), dim3(batch * H * (dv / 32)), dim3(320), 0, s, out, state, scratch, cu_q, seq_lens, slots, batch, H, dv);
+    hipLaunchKernelGGL((delta_walk_kernel<128>), dim3(batch * H * (dv / 16)), dim3(320), 0, s, out, state, scratch, qkv, cu_q, seq_lens, slots, batch, H, G, dv);
   else
-    hipLaunchKernelGGL((delta_walk_kernel<64>), dim3(batch * H * (dv / 32)), dim3(320), 0, s, out, state, scratch, cu_q, seq_lens, slots, batch, H, dv);
+    hipLaunchKernelGGL((delta_walk_kernel<64>), dim3(batch * H * (dv / 16)), dim3(320), 0, s, out, state, scratch, qkv, cu_q, seq_lens, slots, batch, H, G, dv);
   MIX_LAUNCHED("delta_rule_blocks (walk)");
   return MSGL_MIX_OK;
 }
