@@ -8,8 +8,11 @@
 // scores back from LDS).
 //
 // 4 requests of 1500 - 2548 new tokens, 16 heads of 128 over 4 key heads, window 2048: 5182 us on the vector units, 453 us with both
-// products on the matrix cores and the mixing on vector FMAs in step with them, 294 us as below (249 TFLOP/s of useful products; the
-// softmax and the LDS round trip of the scores are what is left, and 20 us are the weights' third part: 273 us with two).
+// products on the matrix cores and the mixing on vector FMAs in step with them, 294 us with all three as below, 257 us with the rows' addresses
+// known once instead of a division and four products per piece and tile, loads without conditions, the table entries a tile ahead and the raw
+// scores' writes over all banks (3 requests of 700 - 1700 tokens after 333, 8 heads, window 512: 63 -> 49; 20 decoded tokens 35 -> 33).  The
+// softmax and the LDS round trip of the scores are what is left, a wave's vector and matrix work one after the other; 20 us are the
+// weights' third part.  Sixteen waves of one head each need 23 registers more than they have.
 //
 // Precision: scores are bf16 x bf16 products with fp32 sums, mixed and exponentiated in fp32; a probability enters the second product
 // as the sum of three bf16 numbers (its rounding, that of what is left, and the rest: 8 bits each), which is the fp32 number itself.
@@ -63,10 +66,13 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
   const int all_hi = start + tok0, all_lo = window > 0 ? max(0, start + last_tok - window + 1) : 0;  // keys that every row sees
   const int h0 = wave * HPW, rep = NH / G, grp = h0 / rep;
   const float scale2 = scale * 1.4426950408889634f;
+  // A wave's raw scores go to LDS two heads a key, 16 keys apart for lane groups that are written together: with 16 heads, the pairs of four
+  // heads change places in every other four keys, which all are one wave's in phase C, and the writes cover all banks.
+  auto swap_of = [](int four_keys) { return NH == 16 ? 2 * (four_keys & 1) : 0; };
   // the table as first operand: row = head, contraction index 4 steps (NH = 16) of g = GS lg + step, which is what a lane reads at once
   float tk[GS];
 #pragma unroll
-  for (int u = 0; u < GS; ++u) tk[u] = lr < NH ? talk[lr * NH + GS * lg + u] * scale2 : 0.f;
+  for (int u = 0; u < GS; ++u) tk[u] = lr < NH ? talk[lr * NH + GS * lg + (u ^ (swap_of(wave)))] * scale2 : 0.f;
   bf16x8_t qf[HPW][KC];
   f32x4_t o[HPW][VC];
   float m[HPW], lsum[HPW];
@@ -86,34 +92,43 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
     lsum[hh] = 0.f;
   }
   const int* trow = table + (size_t)req_rows[b] * table_stride;
-  const size_t nk = (size_t)G * d, nv = (size_t)G * dv;
-  // 16-byte pieces of a tile's key and value rows (both 128 wide per head in LDS, zeros past the head); at most NH / 4 key heads
+  const uint32_t nk = (uint32_t)(G * d), nv = (uint32_t)(G * dv);
+  // 16-byte pieces of a tile's key and value rows (both 128 wide per head in LDS, zeros past the head); at most NH / 4 key heads.  A row's
+  // pieces divide the workgroup (both are powers of two), so a thread has one column of the rows key0, key0 + rows, ...: its offsets are
+  // known once (a division and four 32-bit products a piece and tile, at a quarter of the rate, were a tenth of the kernel).
   static_assert(KC * 4 == VC * 2, "keys and values share the piece map");
-  const int chunks = G * VC * 2;
-  constexpr int NP = kWinTile * (NH / 4) * VC * 2 / NT;  // pieces per thread
-  Q4 pre_k[NP], pre_v[NP];
-  // the rows of tile j0 (its slots in s_slot[buf]) into registers, and from there to LDS
-  auto request = [&](Q4 (&pre)[NP], const bf16_t* cache, size_t ld_row, int dh, int j0, int buf) {
+  const int chunks = G * VC * 2, rows = NT / chunks, key0 = (int)threadIdx.x / chunks, col = ((int)threadIdx.x - key0 * chunks) * 8;
+  const int hv = col / (VC * 16), in_head = col - hv * (VC * 16);
+  const bool has_k = in_head < d, has_v = in_head < dv;
+  const bf16_t *k_at = k_cache + (size_t)hv * d + (has_k ? in_head : 0), *v_at = v_cache + (size_t)hv * dv + (has_v ? in_head : 0);
+  constexpr int NP = kWinTile * (NH / 4) * VC * 2 / NT;  // pieces per thread; with fewer key heads rows come more than once
+  typedef uint32_t Piece __attribute__((ext_vector_type(4)));  // (as a struct the registers became memory)
+  Piece pre_k[NP], pre_v[NP];
+  // the rows of a tile (its slots in s_slot[buf]) into registers, and from there to LDS; a tile's rows past the last key are that key's again.
+  // No condition on a load or a store (columns past the head go to the row's padding): where one was skipped, the loaded registers were
+  // copied, and the wave waited for the loads at once (464 - 533 us).
+  const int to_k = has_k ? col : G * KC * 32, to_v = has_v ? col : G * VC * 16;
+  auto key_of = [&](int u) { return (key0 + u * rows) & (kWinTile - 1); };
+  auto request = [&](Piece (&pre)[NP], const bf16_t* at, uint32_t ld_row, int buf) {
 #pragma unroll
-    for (int u = 0; u < NP; ++u) {
-      const int e = u * NT + (int)threadIdx.x;
-      const int key = e / chunks, ch = e - key * chunks, hv = ch / (VC * 2), c = (ch - hv * (VC * 2)) * 8;
-      pre[u] = Q4{0u, 0u, 0u, 0u};
-      if (key < kWinTile && j0 + key < k_end && c < dh)
-        pre[u] = *reinterpret_cast<const Q4*>(cache + (size_t)s_slot[buf][key] * ld_row + (size_t)hv * dh + c);
-    }
+    for (int u = 0; u < NP; ++u) pre[u] = *reinterpret_cast<const Piece*>(at + (uint64_t)(uint32_t)s_slot[buf][key_of(u)] * ld_row);
   };
-  auto stage = [&](const Q4 (&pre)[NP], uint16_t* dst, int ld_row) {
+  auto stage = [&](const Piece (&pre)[NP], uint16_t* dst, int ld_row) {
 #pragma unroll
-    for (int u = 0; u < NP; ++u) {
-      const int e = u * NT + (int)threadIdx.x;
-      const int key = e / chunks, ch = e - key * chunks;
-      if (key < kWinTile) *reinterpret_cast<Q4*>(&dst[key * ld_row + ch * 8]) = pre[u];
+    for (int u = 0; u < NP; ++u) *reinterpret_cast<Piece*>(dst + key_of(u) * ld_row) = pre[u];
+  };
+  const int last_key = max(k_end - 1, 0);
+  const int in_tile = (int)threadIdx.x & (kWinTile - 1);
+  auto slot_at = [&](int j0) { return trow[min(j0 + in_tile, last_key)]; };
+  auto put_slot = [&](int slot, int buf) {
+    if (threadIdx.x < kWinTile) s_slot[buf][threadIdx.x] = slot;
+  };
+  if (!has_k || !has_v) {
+    for (int key = key0; key < kWinTile; key += rows) {
+      if (!has_k) *reinterpret_cast<Q4*>(sk + key * KSR + col) = Q4{0u, 0u, 0u, 0u};
+      if (!has_v) *reinterpret_cast<Q4*>(sv + key * VS + col) = Q4{0u, 0u, 0u, 0u};
     }
-  };
-  auto slots_of = [&](int j0, int buf) {
-    if (threadIdx.x < kWinTile && j0 + (int)threadIdx.x < k_end) s_slot[buf][threadIdx.x] = trow[j0 + threadIdx.x];
-  };
+  }
   f32x4_t sc[HPW][KS];
   auto scores = [&]() {  // raw scores of the tile in sk
 #pragma unroll
@@ -133,17 +148,18 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-        *reinterpret_cast<float2*>(raw + lr * RAW + (ks * 16 + 4 * lg + c) * NH + h0) = float2{sc[0][ks][c], sc[1][ks][c]};
+        *reinterpret_cast<float2*>(raw + lr * RAW + (ks * 16 + 4 * lg + c) * NH + (h0 ^ swap_of(lg))) = float2{sc[0][ks][c], sc[1][ks][c]};
   };
   constexpr int TW = kWinTile;
-  slots_of(k_begin, 0);
-  slots_of(k_begin + TW, 1);
-  slots_of(k_begin + 2 * TW, 2);
+  int next_slot = slot_at(k_begin + 3 * TW);  // asked for a tile before it goes to LDS: there the whole workgroup waited for the table
+  put_slot(slot_at(k_begin), 0);
+  put_slot(slot_at(k_begin + TW), 1);
+  put_slot(slot_at(k_begin + 2 * TW), 2);
   __syncthreads();
-  request(pre_k, k_cache, nk, d, k_begin, 0);
-  stage(pre_k, sk, KSR);
-  request(pre_v, v_cache, nv, dv, k_begin, 0);
-  request(pre_k, k_cache, nk, d, k_begin + TW, 1);
+  request(pre_k, k_at, nk, 0);
+  stage(pre_k, sk + to_k, KSR);
+  request(pre_v, v_at, nv, 0);
+  request(pre_k, k_at, nk, 1);
   __syncthreads();
   scores();
   store_raw();
@@ -171,14 +187,16 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
         }
       }
     }
-    stage(pre_v, sv, VS);
-    stage(pre_k, sk, KSR);
-    slots_of(j0 + 3 * TW, (buf + 3) & 3);
+    stage(pre_v, sv + to_v, VS);
+    stage(pre_k, sk + to_k, KSR);
+    put_slot(next_slot, (buf + 3) & 3);
     __syncthreads();
     // ---- D(t)
-    request(pre_v, v_cache, nv, dv, nj, (buf + 1) & 3);
-    request(pre_k, k_cache, nk, d, nj + TW, (buf + 2) & 3);
-    scores();  // of tile t + 1 (zeros past the last)
+    request(pre_v, v_at, nv, (buf + 1) & 3);
+    request(pre_k, k_at, nk, (buf + 2) & 3);
+    if (wave == 0) next_slot = slot_at(j0 + 4 * TW);
+    __builtin_amdgcn_sched_barrier(0);  // every load ahead of the products
+    scores();  // of tile t + 1
     f32x4_t s[HPW][KS];
 #pragma unroll
     for (int hh = 0; hh < HPW; ++hh)
