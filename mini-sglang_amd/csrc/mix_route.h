@@ -80,32 +80,47 @@ __device__ __forceinline__ void select_experts_wave(float* s, float* c, float* g
     }
   }
   float tot = 0.f;
-  for (int k = 0; k < top; ++k) {
-    float bv = -INFINITY;
-    int best = 0x7fffffff;
-    for (int e = lane; e < E; e += 64) {
-      const float v = c[e];
-      if (v > bv) {
-        bv = v;
-        best = e;
-      }
+  if (E <= 64) {
+    // one expert a lane: its place is the number of better ones (the loop below takes a chain of twelve exchanges per choice, 2 us for six)
+    const float mine = lane < E && c[lane] > -INFINITY ? c[lane] : -INFINITY;  // (what is no number counts as out: places stay different)
+    int better = 0;
+    for (int o = 0; o < E; ++o) {
+      const float other = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), o));
+      better += (other > mine) | ((other == mine) & (o < lane));
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(best, o, 64);
-      if (ov > bv || (ov == bv && oi < best)) {
-        bv = ov;
-        best = oi;
-      }
+    if (lane < E && better < top) {
+      ids[better] = lane;
+      gs[G + better] = s[lane];
     }
-    if (best == 0x7fffffff) best = 0;  // unreachable: the host checks top <= keep * (E / G) and choice scores are finite
-    const float sv = s[best];
-    tot += sv;
-    if (lane == 0) {
-      ids[k] = best;
-      gs[G + k] = sv;  // the chosen scores wait in LDS (in order within the wave) for the sum
-      c[best] = -INFINITY;
+    for (int k = 0; k < top; ++k) tot += gs[G + k];  // in order within the wave
+  } else {
+    for (int k = 0; k < top; ++k) {
+      float bv = -INFINITY;
+      int best = 0x7fffffff;
+      for (int e = lane; e < E; e += 64) {
+        const float v = c[e];
+        if (v > bv) {
+          bv = v;
+          best = e;
+        }
+      }
+  #pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) {
+        const float ov = __shfl_xor(bv, o, 64);
+        const int oi = __shfl_xor(best, o, 64);
+        if (ov > bv || (ov == bv && oi < best)) {
+          bv = ov;
+          best = oi;
+        }
+      }
+      if (best == 0x7fffffff) best = 0;  // unreachable: the host checks top <= keep * (E / G) and choice scores are finite
+      const float sv = s[best];
+      tot += sv;
+      if (lane == 0) {
+        ids[k] = best;
+        gs[G + k] = sv;  // the chosen scores wait in LDS (in order within the wave) for the sum
+        c[best] = -INFINITY;
+      }
     }
   }
   const float inv = rule.scale / (tot + 1e-20f);
