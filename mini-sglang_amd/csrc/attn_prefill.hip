@@ -67,8 +67,28 @@ struct PrefillParams {
   uint16_t* out;
   int64_t pt_stride, q_stride, kv_stride_tok, kv_stride_head, out_stride;
   int batch, hq, group;
+  int share, per;  // XCDs that share their kv heads, kv heads of each
   float scale_log2;
 };
+
+// Workgroup -> (kv head, q tile, query head).  XCD x = blockIdx % 8 keeps to `per` kv heads, so that their rows stay in its L2; the 8 / gcd(8,
+// kv heads) XCDs with the same ones take turns down one list, the tiles in the order given (most keys first) with all their heads: every XCD
+// gets long tiles and short ones, and what starts last is short.  (Cut into eight stretches instead, the first XCDs of a list had all the long
+// tiles, or one kv head's short tiles came before the next one's long ones.  8 requests of 300 - 1300 tokens, 16 heads on 2: 69 -> 47 us; 4000
+// tokens, 10 on 2: 106 -> 88; 20 requests of 100 - 1024, 9 on 3: 56 -> 47, 24 on 12: 129 -> 126, 32 on 16: 156 -> 152.  8 kv heads: as before.)
+struct PrefillJob {
+  int kvh, hq, tile;  // tile < 0: none left
+};
+__device__ __forceinline__ PrefillJob prefill_job(const PrefillParams& p, int total_tiles) {
+  const int xcd = (int)(blockIdx.x & 7), list = xcd / p.share;
+  const int u = (int)(blockIdx.x >> 3) * p.share + (xcd - list * p.share);
+  const int each = p.group * p.per, ti = u / each, r = u - ti * each, sub = r / p.group;
+  PrefillJob j;
+  j.kvh = list * p.per + sub;
+  j.hq = j.kvh * p.group + (r - sub * p.group);
+  j.tile = ti >= total_tiles ? -1 : p.tile_order ? p.tile_order[ti] : ti;
+  return j;
+}
 
 // element offset of a pool slot: slot and the token stride are both < 2^32 (checked at launch), so ONE v_mad_u64_u32
 // does it; the int64 x int64 product the types ask for costs two quarter-rate 32-bit multiplies and a carry chain more
@@ -176,16 +196,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: the diagonal tests below are scalar branches
   const int hi = lane >> 5;
 
-  // ---- block -> (kv head, q tile, head of the group): XCD-contiguous virtual index ------------------
-  const int n_per = (int)(gridDim.x >> 3);
-  const int vidx = (int)(blockIdx.x & 7) * n_per + (int)(blockIdx.x >> 3);
-  if (vidx >= total_tiles * p.hq) return;
-  const int per_kv = total_tiles * p.group;
-  const int kvh = vidx / per_kv;
-  const int rem = vidx - kvh * per_kv;
-  const int ti = rem / p.group;
-  const int hq = kvh * p.group + (rem - ti * p.group);
-  const int tile = p.tile_order ? p.tile_order[ti] : ti;
+  const PrefillJob job = prefill_job(p, total_tiles);
+  if (job.tile < 0) return;
+  const int kvh = job.kvh, hq = job.hq, tile = job.tile;
 
   int lo = 0, hi_b = p.batch;  // find b with tile_cu[b] <= tile < tile_cu[b+1]
   while (hi_b - lo > 1) {
@@ -452,15 +465,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hi = lane >> 5;
 
-  const int n_per = (int)(gridDim.x >> 3);
-  const int vidx = (int)(blockIdx.x & 7) * n_per + (int)(blockIdx.x >> 3);
-  if (vidx >= total_tiles * p.hq) return;
-  const int per_kv = total_tiles * p.group;
-  const int kvh = vidx / per_kv;
-  const int rem = vidx - kvh * per_kv;
-  const int ti = rem / p.group;
-  const int hq = kvh * p.group + (rem - ti * p.group);
-  const int tile = p.tile_order ? p.tile_order[ti] : ti;
+  const PrefillJob job = prefill_job(p, total_tiles);
+  if (job.tile < 0) return;
+  const int kvh = job.kvh, hq = job.hq, tile = job.tile;
 
   const TileRequest rq = find_request(p, tile, lane);
   const int q_begin = rq.q_begin;
@@ -754,6 +761,12 @@ extern "C" int msgl_attn_prefill(void* out, const void* q, const void* k_cache, 
   p.batch = batch;
   p.hq = num_q_heads;
   p.group = num_q_heads / num_kv_heads;
+  p.per = num_kv_heads;
+  p.share = 8;
+  while (p.share > 1 && p.per % 2 == 0) {
+    p.per /= 2;
+    p.share /= 2;
+  }
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype != MSGL_BF16 && dtype != MSGL_FP16) {
@@ -763,7 +776,7 @@ extern "C" int msgl_attn_prefill(void* out, const void* q, const void* k_cache, 
   if (impl == 0) impl = 4;  // the DMA-staged kernel; impl 2 keeps its predecessor callable (A/B timing, cross-check in tests)
   const int64_t total = (int64_t)total_tiles * num_q_heads;
   MSGL_REQUIRE(total < (1ll << 30), "attn_prefill: %lld workgroups", (long long)total);
-  const unsigned blocks = (unsigned)((total + 7) / 8) * 8;  // 8 XCDs x n_per
+  const unsigned blocks = (unsigned)(((int64_t)total_tiles * p.group * p.per + p.share - 1) / p.share) * 8;
   if (impl == 4) {
     if (dtype == MSGL_BF16) attn_prefill_dma_kernel<BF16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
     else attn_prefill_dma_kernel<FP16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
