@@ -260,6 +260,18 @@ int msgl_attn_prefill(void* out, const void* q, const void* k_cache, const void*
  * folded into the exponent's fma); 2 = the same math with register staging (the A/B partner; bit-identical results).
  * Every other value is refused.  (Rounds 1-3 also had 1, 3, 5 -- a first-generation and a counter-phase kernel -- and
  * timing-only ablation codes >= 16; the former were removed, the latter exist only in a -DMSGL_PREFILL_DIAG build.) */
+/* impl 0 with a job's (q tile's and head's) keys cut into up to `ranges` (2 .. 64) ranges of range_tiles 64-key tiles, the
+ * last one taking what is left, one workgroup each; their fp32 sums are joined by a second launch.  For launches too small
+ * to fill the compute units.  A job of one range has impl 0's bits. */
+int64_t msgl_attn_prefill_ranges_workspace_bytes(int total_tiles, int num_q_heads, int ranges);
+int msgl_attn_prefill_ranges(void* out, const void* q, const void* k_cache, const void* v_cache,
+                             const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
+                             const int32_t* seq_lens, const int32_t* cu_seqlens_q,
+                             const int32_t* tile_cu, int batch, int total_tiles, int num_q_heads,
+                             int num_kv_heads, int head_dim, int64_t q_stride_tok,
+                             int64_t kv_stride_tok, int64_t kv_stride_head, int64_t out_stride_tok,
+                             float sm_scale, int dtype, const int32_t* tile_order, int ranges, int range_tiles,
+                             void* workspace, int64_t workspace_bytes, void* stream);
 /* Rows per q tile: tile_cu, total_tiles and tile_order of msgl_attn_prefill are in units of this many query rows
  * (MSGL_PREFILL_QTILE for both kernels). */
 int msgl_attn_prefill_q_tile(int impl);

@@ -34,6 +34,7 @@ class HipAttnMetadata:
     tile_cu: Optional[torch.Tensor] = None  # [B+1] int32 (prefill only)
     total_tiles: int = 0
     tile_order: Optional[torch.Tensor] = None  # [total_tiles] int32: q tiles, most keys first (prefill only)
+    ranges: tuple = (1, 0)                  # key ranges of a q tile, 64-key tiles of each (prefill only)
     plan: Optional[torch.Tensor] = None     # decode work list (device)
     chunks: Optional[tuple] = None          # recurrent layers: (items [n, 3], item_first [B + 1], n) of long portions cut in pieces
     delta_chunks: Optional[tuple] = None    # the same list at the delta-rule layers' piece size
@@ -101,8 +102,8 @@ class HipAttnBackend:
         self.kv_heads = max(config.num_kv_heads // tp_size, 1)
         self.max_bs = int(ctx.page_table.shape[0])
         self.capacity = decode_capacity or max(4096, 4 * self.max_bs)
-        self._workspace = torch.empty(ops.attn_decode_workspace_bytes(self.capacity, self.qo_heads, self.head_dim),
-                                      dtype=torch.uint8, device=self.device)
+        self._workspace = torch.empty(max(ops.attn_decode_workspace_bytes(self.capacity, self.qo_heads, self.head_dim),
+                                          ops.prefill_ranges_workspace_bytes()), dtype=torch.uint8, device=self.device)
         self._plan_words = ops.attn_decode_plan_words(self.max_bs, self.capacity)
         # graph state
         self.capture_bs: List[int] = []
@@ -174,7 +175,8 @@ class HipAttnBackend:
                             md.batch, self.max_bs, self.capacity, self.scale, slot_run=self.slot_run)
         else:
             ops.attn_prefill(out, q, k_tok, v_tok, table, md.req_rows, md.seq_lens, md.cu_seqlens_q, md.tile_cu,
-                             md.batch, md.total_tiles, self.scale, tile_order=md.tile_order)
+                             md.batch, md.total_tiles, self.scale, tile_order=md.tile_order,
+                             ranges=md.ranges, workspace=self._workspace)
         return out
 
     # ------------------------------------------------------------------ metadata
@@ -204,6 +206,7 @@ class HipAttnBackend:
             cu_seqlens_q=dev[2 * bs: 3 * bs + 1], seq_lens=dev[:bs], req_rows=dev[bs: 2 * bs], batch=bs,
             max_seqlen_q=max_q, max_seqlen_k=max_k, tile_cu=None if decode else dev[3 * bs + 1: 4 * bs + 2],
             total_tiles=total_tiles, tile_order=None if decode else dev[4 * bs + 2:],
+            ranges=(1, 0) if decode else ops.prefill_ranges(total_tiles, self.qo_heads, max_q, max_k),
         )
         if decode and not self._replayed_from_graph(batch, bs):
             # runs eagerly: plan now (device side, no sync).  Only batches the engine will REPLAY are planned

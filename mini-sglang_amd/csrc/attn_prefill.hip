@@ -42,6 +42,7 @@ constexpr int kQTile = MSGL_PREFILL_QTILE;  // 128 query rows per workgroup
 constexpr int kKTile = 64;                  // keys per tile
 constexpr int kD = 128;
 constexpr float kNegBigP = -3.0e38f;
+typedef float f32x4p __attribute__((ext_vector_type(4)));
 
 template <typename T>
 __device__ __forceinline__ f32x16 mfma32(const U4& a, const U4& b, f32x16 c) {
@@ -68,6 +69,9 @@ struct PrefillParams {
   int64_t pt_stride, q_stride, kv_stride_tok, kv_stride_head, out_stride;
   int batch, hq, group;
   int share, per;  // XCDs that share their kv heads, kv heads of each
+  int stretch;     // workgroups of an XCD where each takes a stretch of the list, or 0
+  int ranges, run;  // key ranges, and tiles of each (the last one: what is left)
+  float *part_o, *part_ml;
   float scale_log2;
 };
 
@@ -76,12 +80,14 @@ struct PrefillParams {
 // gets long tiles and short ones, and what starts last is short.  (Cut into eight stretches instead, the first XCDs of a list had all the long
 // tiles, or one kv head's short tiles came before the next one's long ones.  8 requests of 300 - 1300 tokens, 16 heads on 2: 69 -> 47 us; 4000
 // tokens, 10 on 2: 106 -> 88; 20 requests of 100 - 1024, 9 on 3: 56 -> 47, 24 on 12: 129 -> 126, 32 on 16: 156 -> 152.  8 kv heads: as before.)
+// A launch of one workgroup per CU or less starts all of them at once: stretches of the list, which leave an XCD fewer requests' keys (6 requests of
+// 100 - 400 after 2500, 16 on 2: 63 us, in turns 65).
 struct PrefillJob {
   int kvh, hq, tile;  // tile < 0: none left
 };
 __device__ __forceinline__ PrefillJob prefill_job(const PrefillParams& p, int total_tiles) {
-  const int xcd = (int)(blockIdx.x & 7), list = xcd / p.share;
-  const int u = (int)(blockIdx.x >> 3) * p.share + (xcd - list * p.share);
+  const int xcd = (int)(blockIdx.x & 7), list = xcd / p.share, seat = xcd - list * p.share, n = (int)(blockIdx.x >> 3);
+  const int u = p.stretch ? seat * p.stretch + n : n * p.share + seat;
   const int each = p.group * p.per, ti = u / each, r = u - ti * each, sub = r / p.group;
   PrefillJob j;
   j.kvh = list * p.per + sub;
@@ -445,12 +451,16 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 // 16 cycles each), and two waves per SIMD overlap them only in part.  40 heads on 8, 29 requests of 100 - 1024 tokens: 245 -> 244 us with the
 // last two points; 64 heads, 8192 tokens after 16384: 5570 -> 5490 (1000 TFLOP/s), the same bits.  (Sums of the rounded weights, one instruction
 // a pair: 242 and 5510 us, and 2^-9 of a row's weight off.)
+// RANGES: workgroup (.., z) takes the tiles z * run .. of the job's keys; sums of more than one range go to attn_prefill_join_kernel in fp32, in
+// the order of the lanes.  For launches that leave compute units empty, where the longest chain of tiles (1.26 us each) is the time: 16 heads on
+// 8, 100 tokens after 2000: 45.1 -> 13.7 us, 1000 after 3000: 81.7 -> 53.2; 5 on 1, 2000 tokens: 43.0 -> 20.5 (both launches, in a captured chain;
+// the rule and its other side: ops.prefill_ranges)
 // ABL (diagnosis, wrong results): 1 = tiles DMA'd once, 2 = no QK^T, 4 = no softmax, 8 = no PV.
 // ------------------------------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) const void glb_void_t;
 
-template <typename T, int ABL = 0>
+template <typename T, int ABL = 0, bool RANGES = false>
 __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillParams p, int total_tiles) {
   // two distinct LDS objects, not one array: the compiler then knows a tile's fragment reads cannot alias the DMA writes
   // of the next tile (other object) and does not wait for them (vmcnt) before the reads
@@ -478,7 +488,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
   const int* pt = p.page_table + (int64_t)row * p.pt_stride;
   const int diag = k_len - q_len;
   const int kend = min(k_len, diag + min(q0 + kQTile, q_len));
-  const int ntiles = (kend + kKTile - 1) / kKTile;
+  const int all_tiles = (kend + kKTile - 1) / kKTile;
+  const int t0 = RANGES ? (int)blockIdx.y * p.run : 0;
+  const int ntiles = RANGES && blockIdx.y + 1 < gridDim.y ? min(all_tiles, t0 + p.run) : all_tiles;  // past this workgroup's last
+  if (RANGES && t0 > 0 && t0 >= ntiles) return;
 
   const int my_q = q0 + wave * 32 + (lane & 31);
   const bool q_valid = my_q < q_len;
@@ -679,16 +692,25 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
     }
   };
 
-  if (ntiles > 0) {
-    load_slots(0);
+  if (t0 < ntiles) {
+    load_slots(t0);
     issue_dma(lds_a);
-    if (ntiles > 1) load_slots(1);
+    if (t0 + 1 < ntiles) load_slots(t0 + 1);
   }
-  for (int kt = 0; kt < ntiles; kt += 2) {
+  for (int kt = t0; kt < ntiles; kt += 2) {
     tile_body(std::integral_constant<int, 0>{}, kt);
     if (kt + 1 < ntiles) tile_body(std::integral_constant<int, 1>{}, kt + 1);
   }
 
+  if (RANGES && all_tiles > p.run) {
+    const int64_t at = ((int64_t)blockIdx.y * total_tiles * p.hq + (int64_t)tile * p.hq + hq) * 4 + wave;
+    f32x4p* po = reinterpret_cast<f32x4p*>(p.part_o) + at * 1024 + lane;  // [16 pieces][64 lanes]
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      po[i * 64] = f32x4p{o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1], o[i >> 2][4 * (i & 3) + 2], o[i >> 2][4 * (i & 3) + 3]};
+    *reinterpret_cast<float2*>(p.part_ml + (at * 64 + lane) * 2) = make_float2(m_run, l_run);
+    return;
+  }
   if (q_valid) {
     const float inv = 1.0f / l_run;
     uint16_t* op = p.out + (int64_t)(q_begin + my_q) * p.out_stride + (int64_t)hq * kD;
@@ -706,6 +728,52 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
   }
 }
 
+// The ranges of a job: one wave for 32 rows and 32 columns (piece group nb) of one wave of the kernel above, all loads coalesced.
+template <typename T>
+__global__ __launch_bounds__(64) void attn_prefill_join_kernel(const PrefillParams p, int total_tiles) {
+  const int lane = threadIdx.x & 63, hi = lane >> 5;
+  const PrefillJob job = prefill_job(p, total_tiles);
+  if (job.tile < 0) return;
+  const TileRequest rq = find_request(p, job.tile, lane);
+  const int q_len = rq.q_end - rq.q_begin, q0 = (job.tile - rq.tile_first) * kQTile;
+  const int kend = min(rq.k_len, rq.k_len - q_len + min(q0 + kQTile, q_len));
+  const int n = min(((kend + kKTile - 1) / kKTile + p.run - 1) / p.run, p.ranges);
+  if (n <= 1) return;
+  const int wave = (int)blockIdx.y >> 2, nb = (int)blockIdx.y & 3;
+  const int64_t step = (int64_t)total_tiles * p.hq * 4, at0 = ((int64_t)job.tile * p.hq + job.hq) * 4 + wave;
+  float m = kNegBigP, l = 0.f;
+  f32x4p acc[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) acc[r] = f32x4p{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int z = 0; z < n; ++z) {  // a range without a visible key for the row: weight 0
+    const int64_t at = at0 + z * step;
+    const float2 st = *reinterpret_cast<const float2*>(p.part_ml + (at * 64 + lane) * 2);
+    const f32x4p* po = reinterpret_cast<const f32x4p*>(p.part_o) + at * 1024 + nb * 256 + lane;
+    f32x4p x[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = po[r * 64];
+    const float mn = fmaxf(m, st.x), w0 = __builtin_amdgcn_exp2f(m - mn), w1 = __builtin_amdgcn_exp2f(st.x - mn);
+    m = mn;
+    l = fmaf(l, w0, st.y * w1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[r][e] = fmaf(acc[r][e], w0, x[r][e] * w1);
+  }
+  const int my_q = q0 + wave * 32 + (lane & 31);
+  if (my_q >= q_len) return;
+  const float inv = 1.0f / l;
+  uint16_t* op = p.out + (int64_t)(rq.q_begin + my_q) * p.out_stride + (int64_t)job.hq * kD + nb * 32 + 4 * hi;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    uint2 w;
+    w.x = Elem<T>::pack(acc[r][0] * inv, acc[r][1] * inv);
+    w.y = Elem<T>::pack(acc[r][2] * inv, acc[r][3] * inv);
+    *reinterpret_cast<uint2*>(op + 8 * r) = w;
+  }
+}
+
 
 }  // namespace msgl
 
@@ -713,13 +781,14 @@ using namespace msgl;
 
 extern "C" int msgl_attn_prefill_q_tile(int /*impl*/) { return kQTile; }
 
-extern "C" int msgl_attn_prefill(void* out, const void* q, const void* k_cache, const void* v_cache,
+// ranges > 1: impl 0 with that many key ranges at most, `run` tiles each
+static int prefill(void* out, const void* q, const void* k_cache, const void* v_cache,
                                  const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
                                  const int32_t* seq_lens, const int32_t* cu_seqlens_q, const int32_t* tile_cu,
                                  int batch, int total_tiles, int num_q_heads, int num_kv_heads, int head_dim,
                                  int64_t q_stride_tok, int64_t kv_stride_tok, int64_t kv_stride_head,
                                  int64_t out_stride_tok, float sm_scale, int dtype, const int32_t* tile_order,
-                                 int impl, void* stream) {
+                                 int impl, int ranges, int run, float* workspace, void* stream) {
   MSGL_REQUIRE(batch >= 0 && total_tiles >= 0, "attn_prefill: negative sizes");
 #ifdef MSGL_PREFILL_DIAG
   MSGL_REQUIRE(impl == 0 || impl == 2 || impl == 4 || (impl >= 16 && impl < 48) || (impl >= 64 && impl < 128),
@@ -776,8 +845,23 @@ extern "C" int msgl_attn_prefill(void* out, const void* q, const void* k_cache, 
   if (impl == 0) impl = 4;  // the DMA-staged kernel; impl 2 keeps its predecessor callable (A/B timing, cross-check in tests)
   const int64_t total = (int64_t)total_tiles * num_q_heads;
   MSGL_REQUIRE(total < (1ll << 30), "attn_prefill: %lld workgroups", (long long)total);
-  const unsigned blocks = (unsigned)(((int64_t)total_tiles * p.group * p.per + p.share - 1) / p.share) * 8;
-  if (impl == 4) {
+  const int even = (int)(((int64_t)total_tiles * p.group * p.per + p.share - 1) / p.share);
+  p.stretch = ranges == 1 && total <= 256 ? even : 0;
+  const unsigned blocks = (unsigned)even * 8;
+  if (ranges > 1) {
+    p.ranges = ranges;
+    p.run = run;
+    p.part_o = workspace;
+    p.part_ml = workspace + total * ranges * kQTile * kD;
+    const dim3 grid(blocks, (unsigned)ranges), joins(blocks, 16);
+    if (dtype == MSGL_BF16) {
+      attn_prefill_dma_kernel<BF16, 0, true><<<grid, dim3(256), 0, s>>>(p, total_tiles);
+      attn_prefill_join_kernel<BF16><<<joins, dim3(64), 0, s>>>(p, total_tiles);
+    } else {
+      attn_prefill_dma_kernel<FP16, 0, true><<<grid, dim3(256), 0, s>>>(p, total_tiles);
+      attn_prefill_join_kernel<FP16><<<joins, dim3(64), 0, s>>>(p, total_tiles);
+    }
+  } else if (impl == 4) {
     if (dtype == MSGL_BF16) attn_prefill_dma_kernel<BF16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
     else attn_prefill_dma_kernel<FP16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
   } else if (impl == 2) {
@@ -807,4 +891,31 @@ extern "C" int msgl_attn_prefill(void* out, const void* q, const void* k_cache, 
 #endif
   MSGL_CHECK_LAUNCH("attn_prefill");
   return MSGL_OK;
+}
+
+extern "C" int msgl_attn_prefill(void* out, const void* q, const void* k_cache, const void* v_cache, const int32_t* page_table, int64_t pt_stride,
+                                       const int32_t* req_rows, const int32_t* seq_lens, const int32_t* cu_seqlens_q, const int32_t* tile_cu,
+                                       int batch, int total_tiles, int num_q_heads, int num_kv_heads, int head_dim, int64_t q_stride_tok,
+                                       int64_t kv_stride_tok, int64_t kv_stride_head, int64_t out_stride_tok, float sm_scale, int dtype,
+                                       const int32_t* tile_order, int impl, void* stream) {
+  return prefill(out, q, k_cache, v_cache, page_table, pt_stride, req_rows, seq_lens, cu_seqlens_q, tile_cu, batch, total_tiles, num_q_heads,
+                 num_kv_heads, head_dim, q_stride_tok, kv_stride_tok, kv_stride_head, out_stride_tok, sm_scale, dtype, tile_order, impl, 1, 0, nullptr, stream);
+}
+
+extern "C" int64_t msgl_attn_prefill_ranges_workspace_bytes(int total_tiles, int num_q_heads, int ranges) {
+  if (total_tiles < 0 || num_q_heads < 1 || ranges < 1) return MSGL_EINVAL;
+  return (int64_t)total_tiles * num_q_heads * ranges * kQTile * (kD + 4) * (int64_t)sizeof(float);  // sums; (m, l) of each lane of a row's pair
+}
+
+extern "C" int msgl_attn_prefill_ranges(void* out, const void* q, const void* k_cache, const void* v_cache, const int32_t* page_table, int64_t pt_stride,
+                                              const int32_t* req_rows, const int32_t* seq_lens, const int32_t* cu_seqlens_q, const int32_t* tile_cu,
+                                              int batch, int total_tiles, int num_q_heads, int num_kv_heads, int head_dim, int64_t q_stride_tok,
+                                              int64_t kv_stride_tok, int64_t kv_stride_head, int64_t out_stride_tok, float sm_scale, int dtype,
+                                              const int32_t* tile_order, int ranges, int range_tiles, void* workspace, int64_t workspace_bytes, void* stream) {
+  MSGL_REQUIRE(ranges >= 2 && ranges <= 64 && range_tiles >= 1, "attn_prefill_ranges: %d ranges of %d tiles", ranges, range_tiles);
+  MSGL_REQUIRE(num_q_heads >= 1 && total_tiles >= 0, "attn_prefill_ranges: %d tiles, %d heads", total_tiles, num_q_heads);
+  MSGL_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= msgl_attn_prefill_ranges_workspace_bytes(total_tiles, num_q_heads, ranges),
+               "attn_prefill_ranges: workspace of %lld bytes", (long long)workspace_bytes);
+  return prefill(out, q, k_cache, v_cache, page_table, pt_stride, req_rows, seq_lens, cu_seqlens_q, tile_cu, batch, total_tiles, num_q_heads,
+                 num_kv_heads, head_dim, q_stride_tok, kv_stride_tok, kv_stride_head, out_stride_tok, sm_scale, dtype, tile_order, 0, ranges, range_tiles, (float*)workspace, stream);
 }

@@ -409,13 +409,47 @@ def prefill_q_tile(impl: Optional[int] = None) -> int:
     return int(lib().msgl_attn_prefill_q_tile(PREFILL_IMPL if impl is None else int(impl)))
 
 
+PREFILL_RANGE_JOBS = 800  # workgroups that `prefill_ranges` makes of a launch at most
+
+
+def prefill_ranges(total_tiles: int, qo_heads: int, max_seqlen_q: int, max_seqlen_k: int) -> Tuple[int, int]:
+    """Key ranges of a (q tile, head) of the default prefill kernel at most, and 64-key tiles of each.
+
+    A tile is 1.26 us of a workgroup, and a launch of few workgroups takes as long as its longest chain of them; ranges shorten the chain and cost
+    a second launch and fp32 sums (5 us).  us in a captured chain, one range -> these:
+      16 heads on 8: 100 tokens after 2000   45.1 -> 13.7    1000 after 3000  81.7 -> 53.2
+       5 heads on 1: 2000                    43.0 -> 20.5    4000             80.3 -> 50.6
+      64 heads on 8: 100 after 2000          45.4 -> 21.5
+    As many as give every CU one workgroup (the queries' own keys count half, under the diagonal), three tiles or more each: 80 workgroups of up to
+    32 tiles in 2 / 4 / 8 ranges 28.7 / 20.5 / 22.2, 64 of 33 in 2 / 4 / 7 29.1 / 21.5 / 25.4.  Two still help while no more than 200 are
+    busy all the time: 384 causal ones of up to 47 tiles (192) 68.7 -> 62.4, 320 of 63 behind 3000 keys (280) 106 -> 111.  Chains under
+    32 tiles stay whole: of 16 tiles 24.7 -> 20.0, less than the host needs for the launches (34.5 -> 40.5 a call without a graph);
+    of 5 tiles 10.2 -> 11.1."""
+    jobs, longest = total_tiles * qo_heads, -(-max_seqlen_k // 64)
+    if longest < 32 or PREFILL_IMPL == 2:
+        return 1, 0
+    busy = jobs * (1.0 - max_seqlen_q / (2.0 * max_seqlen_k))
+    ranges = min(int(max(256 / busy, 2 if busy <= 200 else 1)), 64)
+    run = max(3, -(-longest // ranges))
+    ranges = -(-longest // run)
+    return (ranges, run) if ranges > 1 else (1, 0)
+
+
+def prefill_ranges_workspace_bytes(jobs: int = PREFILL_RANGE_JOBS) -> int:
+    """For any ranges of `prefill_ranges`, or for `jobs` = q tiles x heads x ranges."""
+    return int(lib().msgl_attn_prefill_ranges_workspace_bytes(jobs, 1, 1))
+
+
 def attn_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                  page_table: torch.Tensor, req_rows: Optional[torch.Tensor], seq_lens: torch.Tensor,
                  cu_seqlens_q: torch.Tensor, tile_cu: torch.Tensor, batch: int, total_tiles: int,
-                 sm_scale: float, tile_order: Optional[torch.Tensor] = None, impl: Optional[int] = None) -> None:
+                 sm_scale: float, tile_order: Optional[torch.Tensor] = None, impl: Optional[int] = None,
+                 ranges: Tuple[int, int] = (1, 0), workspace: Optional[torch.Tensor] = None) -> None:
     """tile_order: optional int32 [total_tiles] schedule of the q tiles (heaviest first); impl: None = process default
     (PREFILL_IMPL), 0 = 4 the DMA-staged kernel, 2 its register-staged predecessor (include/msgl_hip.h; anything else is
-    refused by the library).  tile_cu / total_tiles / tile_order are in units of prefill_q_tile(impl) query rows."""
+    refused by the library).  tile_cu / total_tiles / tile_order are in units of prefill_q_tile(impl) query rows.
+    ranges: (key ranges of a q tile at most, 64-key tiles of each) for the DMA-staged kernel, see `prefill_ranges`; more than one needs a
+    workspace of prefill_ranges_workspace_bytes."""
     _need_cuda(out, q, k_cache, v_cache, page_table, seq_lens, cu_seqlens_q, tile_cu)
     if impl is None:
         impl = PREFILL_IMPL
@@ -427,13 +461,18 @@ def attn_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_ca
     assert q.stride(2) == 1 and q.stride(1) == d and out.stride(2) == 1 and out.stride(1) == d
     assert k_cache.stride(2) == 1 and v_cache.stride() == k_cache.stride()
     assert page_table.dtype == torch.int32 and page_table.stride(1) == 1
+    entry, last = lib().msgl_attn_prefill, (int(impl),)
+    if ranges[0] > 1:
+        assert int(impl) in (0, 4) and workspace is not None, impl
+        _need_cuda(workspace)
+        entry, last = lib().msgl_attn_prefill_ranges, (*ranges, workspace.data_ptr(), workspace.numel() * workspace.element_size())
     check(
-        lib().msgl_attn_prefill(
+        entry(
             out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), page_table.data_ptr(),
             page_table.stride(0), req_rows.data_ptr() if req_rows is not None else None, seq_lens.data_ptr(),
             cu_seqlens_q.data_ptr(), tile_cu.data_ptr(), batch, total_tiles, hq, hkv, d, q.stride(0),
             k_cache.stride(0), k_cache.stride(1), out.stride(0), float(sm_scale), _dt(q),
-            tile_order.data_ptr() if tile_order is not None else None, int(impl), _stream(),
+            tile_order.data_ptr() if tile_order is not None else None, *last, _stream(),
         ),
         "attn_prefill",
     )

@@ -220,3 +220,34 @@ def test_prefill_row_sum_of_unrounded_weights(ops, dev, impl):
         v = c["v"][c["table"][row, :257].long()].double()
         ref = (v[0] + 0.25 * v[1:].sum(0)) / (1.0 + 256 * w)
         assert abs(float(((out[b] - ref) / ref).mean())) < 3e-4
+
+
+@pytest.mark.parametrize("hq,hkv,specs,ranges,dtype", [
+    (16, 8, [(2000, 2100)], None, torch.bfloat16),             # a short portion after a long one
+    (5, 1, [(0, 2060)], None, torch.bfloat16),                 # the first tiles' jobs have one range
+    (10, 2, [(1100, 1101), (0, 129), (2000, 2160)], None, torch.float16),  # ragged ends, jobs of every number of ranges
+    (6, 3, [(0, 5), (960, 1024)], (2, 3), torch.bfloat16),     # the last range takes what is left
+    (4, 4, [(4000, 4100)], (64, 1), torch.bfloat16),           # 65 tiles, the most ranges
+    (4, 2, [(64, 192), (0, 65)], (2, 1), torch.bfloat16),      # a wave's rows see nothing of their second range
+])
+def test_prefill_key_ranges(ops, dev, monkeypatch, hq, hkv, specs, ranges, dtype):
+    """Ranges of the keys on workgroups of their own: the oracle's results; a job of one range keeps the bits of the launch without."""
+    c = build(torch.Generator().manual_seed(16), specs, hq, hkv, 16, dtype)
+    whole = run(ops, dev, c)
+    tiles = sum(-(-n // ops.prefill_q_tile()) for n in c["q_lens"])
+    rule = ops.prefill_ranges(tiles, hq, max(c["q_lens"]), max(c["k_lens"]))
+    ranges = ranges or rule
+    assert ranges[0] > 1
+    ws = torch.empty(ops.prefill_ranges_workspace_bytes(tiles * hq * ranges[0]), dtype=torch.uint8, device=dev)
+    plain = ops.attn_prefill
+    monkeypatch.setattr(ops, "attn_prefill", lambda *a, **k: plain(*a, **k, ranges=ranges, workspace=ws))
+    out = run(ops, dev, c)
+    torch.testing.assert_close(out.double(), oracle(c), **TOL)
+    assert torch.equal(out, run(ops, dev, c, order=None))
+    at = 0
+    for n, k in zip(c["q_lens"], c["k_lens"]):
+        for t in range(0, n, 128):
+            rows = slice(at + t, at + min(t + 128, n))
+            if -(-(k - n + min(t + 128, n)) // 64) <= ranges[1]:
+                assert torch.equal(out[rows], whole[rows])
+        at += n
