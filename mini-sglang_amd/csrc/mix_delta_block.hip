@@ -288,6 +288,50 @@ __global__ __launch_bounds__(D, 4) void delta_block_kernel(float* __restrict__ s
   }
 }
 
+// The request at a place of the walks' order (`each` workgroups a request), its first token, its tokens and the blocks of the requests before it.
+// A walk takes as long as its request, 0.9 us a block alone on a CU and 1.6 beside another one.  So the longest requests come first, one round of
+// the CUs; those of the second round meet them in reverse, and where it is not full the longest ones stay alone; what does not fit two rounds
+// follows in order, the shortest last.  Walks that each are less than a place's share of more than two rounds stay as they come: no end to wait for,
+// and equal ones side by side wait for their first loads together (us of the walks, as they come -> ordered: 8 requests of 80 - 130 tokens,
+// 16 heads: 29.9 -> 31.8; 8 of 300 - 1000: 134.9 -> 138.5).  Ordered: 4 of 1500 - 2548, 16 heads: 214 -> 190; 5 of 400 - 1500, 8 heads:
+// 90 -> 80; 7 of 100 - 1100, 16 heads: 118 -> 104; 3 of 200 - 2600: 147.
+struct WalkRequest {
+  int b, first, n_new, blk;
+};
+__device__ __forceinline__ WalkRequest walk_request(const int* __restrict__ cu_q, int B, int each, int place) {
+  const int lane = threadIdx.x & 63;
+  WalkRequest r;
+  if (B > 64) {
+    r.b = place;
+    r.first = cu_q[place];
+    r.n_new = cu_q[place + 1] - r.first;
+    r.blk = 0;
+    for (int i = lane; i < place; i += 64) r.blk += (cu_q[i + 1] - cu_q[i] + kBT - 1) / kBT;
+    r.blk = wave_total(r.blk);
+    return r;
+  }
+  const int first = lane < B ? cu_q[lane] : 0, n = lane < B ? cu_q[lane + 1] - first : 0;
+  const int round = max(1, 256 / each), met = min(round, B - round);  // requests in the second round
+  const int longest = wave_fold(n, [](int x, int y) { return max(x, y); });
+  const bool ordered = B <= 2 * round || (int64_t)longest * 512 >= (int64_t)wave_total(n) * each;
+  r.b = place;
+  if (ordered) {
+    int rank = place;
+    if (met > 0 && place < round) rank = place < met ? round - met + place : place - met;
+    else if (met > 0 && place < 2 * round) rank = round + met - 1 - (place - round);
+    int longer = 0;
+    for (int i = 0; i < B; ++i) {
+      const int ni = __builtin_amdgcn_readlane(n, i);
+      longer += ni > n || (ni == n && i < lane);
+    }
+    r.b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(longer == rank && lane < B));
+  }
+  r.first = __builtin_amdgcn_readlane(first, r.b);
+  r.n_new = __builtin_amdgcn_readlane(n, r.b);
+  r.blk = wave_total(lane < r.b ? (n + kBT - 1) / kBT : 0);
+  return r;
+}
+
 // One workgroup per (request, head, 16 value columns), five waves.  Waves 0 - 3: wave w holds the state rows w D / 4 ... of the columns as
 // MFMA accumulators (lane: rows 4 lg + i, column lr), which are second operands as they stand: contraction index = state row, the first
 // operands' reads follow the same order.  u = T v - W S and (P q) S are sums over tokens and rows: wave w adds the tokens 4 g + w (one
@@ -319,15 +363,11 @@ __global__ __launch_bounds__(320, 4) void delta_walk_kernel(float* __restrict__ 
     g = (int)blockIdx.x / ncb;
     cb = (int)blockIdx.x % ncb;
   }
-  const int b = g / H, h = g - b * H, c0 = cb * 16;
-  const int first = cu_q[b], n_new = cu_q[b + 1] - first;
+  const int place = g / H, h = g - place * H, c0 = cb * 16;
+  const WalkRequest req = walk_request(cu_q, B, H * ncb, place);
+  const int b = req.b, first = req.first, n_new = req.n_new, blk = req.blk;
   if (n_new <= 0) return;
   const int nblk = (n_new + kBT - 1) / kBT;
-  int blk = 0;  // blocks of the requests before this one
-  for (int i = lane; i < b; i += 64) blk += (cu_q[i + 1] - cu_q[i] + kBT - 1) / kBT;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) blk += __shfl_xor(blk, o, 64);
-  blk = __builtin_amdgcn_readfirstlane(blk);
   const BlockPart part{D};
   const uint32_t step = (uint32_t)(H * part.size());
   const float* src = scratch + ((size_t)blk * H + h) * part.size();
