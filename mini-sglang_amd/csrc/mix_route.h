@@ -81,7 +81,7 @@ __device__ __forceinline__ void select_experts_wave(float* s, float* c, float* g
   }
   float tot = 0.f;
   if (E <= 64) {
-    // one expert a lane: its place is the number of better ones (the loop below takes a chain of twelve exchanges per choice, 2 us for six)
+    // one expert a lane: its place is the number of better ones (the loop below takes a chain of twelve exchanges per choice, 1 us for six)
     const float mine = lane < E && c[lane] > -INFINITY ? c[lane] : -INFINITY;  // (what is no number counts as out: places stay different)
     int better = 0;
     for (int o = 0; o < E; ++o) {
