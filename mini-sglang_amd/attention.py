@@ -105,6 +105,9 @@ class HipAttnBackend:
         self._workspace = torch.empty(max(ops.attn_decode_workspace_bytes(self.capacity, self.qo_heads, self.head_dim),
                                           ops.prefill_ranges_workspace_bytes()), dtype=torch.uint8, device=self.device)
         self._plan_words = ops.attn_decode_plan_words(self.max_bs, self.capacity)
+        self._small_heads = 0  # requests x kv heads of a decode batch up to which `small_decode` says yes
+        if self.head_dim == 128 and self.qo_heads % self.kv_heads == 0 and self.qo_heads // self.kv_heads <= 8:
+            self._small_heads = SMALL_DECODE_HEADS * (2 if self.kv_heads <= 2 or int(ctx.page_table.shape[1]) <= 4096 else 1)
         # graph state
         self.capture_bs: List[int] = []
         self.max_graph_bs = 0
@@ -127,10 +130,7 @@ class HipAttnBackend:
         34 / 66; 8 requests 15.1 / 14.7 and 60 / 53: its requests are half lines, and it loses once the stream is long.  With 1 or
         2 kv heads it is ahead up to 64 of them as well (2 x 32 at 2000 tokens: 24 / 27)."""
         md = batch.attn_metadata
-        if md.max_seqlen_q != 1 or self.head_dim != 128 or self.qo_heads % self.kv_heads or self.qo_heads // self.kv_heads > 8:
-            return False
-        heads = md.batch * self.kv_heads
-        return heads <= SMALL_DECODE_HEADS or (heads <= 2 * SMALL_DECODE_HEADS and (self.kv_heads <= 2 or self.ctx.page_table.shape[1] <= 4096))
+        return md.max_seqlen_q == 1 and md.batch * self.kv_heads <= self._small_heads
 
     def _attend_small(self, q, k, v, layer_id: int, batch: Any, **row_work) -> torch.Tensor:
         md: HipAttnMetadata = batch.attn_metadata
