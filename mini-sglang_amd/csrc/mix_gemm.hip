@@ -32,7 +32,10 @@ __device__ __forceinline__ int count_tiles(const int* __restrict__ seg, int grou
 //   MT x NT = 256 x 256, 8 waves of 64 x 128   long segments
 //             128 x 128, 4 waves of 64 x 64    middling ones: two workgroups a CU
 //              64 x 128, 4 waves of 64 x 32    short ones: the ring holds 2 x 2 x 16 KB of B per CU under way
-template <typename TC, int MT, int NT, int W, int WR, int KS, int ST>
+//              32 x 128, 4 waves of 32 x 32    a decode step's few rows: less of A beside B, 2 x 3 x 16 KB of B under way
+// STREAM: B passes by the caches (one row tile reads it).  64 x 3 rows, N 1024, K 2048 and N 2048, K 512: 53.6 and 25.5 us, 32-row tiles
+// 50.4 and 25.2, streaming 46.7 and 21.3 (5.7 and 6.3 TB/s); 32 x 256 tiles 56 and 24.5, a stage less 53 and 24.8, one more 55 and 30.
+template <typename TC, int MT, int NT, int W, int WR, int KS, int ST, bool STREAM = false>
 __global__ __launch_bounds__(64 * W, 2) void gemm_nt_dma_kernel(TC* __restrict__ C, const bf16_t* __restrict__ A, const bf16_t* __restrict__ Bm, int M,
                                                              int N, int K, int64_t lda, int64_t ldb, int64_t ldc, int groups, int64_t a_gs,
                                                              int64_t b_gs, int64_t c_gs, const int* __restrict__ seg,
@@ -80,7 +83,11 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_nt_dma_kernel(TC* __restrict__
     char* dst = ring + stage * STAGE + wave * 1024;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      __builtin_amdgcn_global_load_lds((glb_void_t*)src[u], (lds_void_t*)(dst + (u < UA ? u * W * 1024 : MT * ROW + (u - UA) * W * 1024)), 16, 0, 0);
+      constexpr int kNonTemporal = 2;
+      if (STREAM && u >= UA)
+        __builtin_amdgcn_global_load_lds((glb_void_t*)src[u], (lds_void_t*)(dst + MT * ROW + (u - UA) * W * 1024), 16, 0, kNonTemporal);
+      else
+        __builtin_amdgcn_global_load_lds((glb_void_t*)src[u], (lds_void_t*)(dst + (u < UA ? u * W * 1024 : MT * ROW + (u - UA) * W * 1024)), 16, 0, 0);
       src[u] += ROW;
     }
   };
@@ -99,7 +106,7 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_nt_dma_kernel(TC* __restrict__
     b_off[kb] = (MT + wn + bn) * ROW + ((4 * kb + lg) ^ b_key(bn)) * 16;
   }
   int at = 0;
-  if constexpr (MT == 64 && KS == 64) {
+  if constexpr (MT <= 64 && KS == 64) {
     // Short segments, few products: the fragments' reads are what is left to hide.  A step's two blocks of 32 take turns, each block's fragments
     // are read before the other one's products, and the barrier lies between them: by then the step has been read by everybody, its stage takes
     // a later one.  (64 x 3 rows, N 1024, K 2048: 100 -> 96 us, 16 x 62, N 1536, K 1024: 24.8 -> 22.8; larger tiles are 1 - 3 % slower this way.)
@@ -202,6 +209,11 @@ __global__ __launch_bounds__(64 * W, 2) void gemm_nt_dma_kernel(TC* __restrict__
   }
 }
 
+template <int MT, int NT, int WR, int KS, int ST, bool STREAM = false>
+constexpr size_t gemm_lds() {
+  return (size_t)ST * (MT + NT) * KS * 2;
+}
+
 }  // namespace
 
 // 1: launched; 0: not this kernel's operands (the caller takes the other ones); < 0: an error code.
@@ -214,14 +226,15 @@ extern "C" __attribute__((visibility("hidden"))) int mix_gemm_nt_dma(void* C, co
     const int64_t list = seg ? (int64_t)M / mt + groups : (int64_t)groups * ((M + mt - 1) / mt);
     return (list * ((N + nt - 1) / nt) + 7) / 8 * 8;
   };
-#define GEMM_RUN(TC, MT, NT, W, WR, KS, ST)                                                                                                  \
+#define GEMM_RUN(TC, MT, NT, W, ...)                                                                                                  \
   {                                                                                                                                   \
+    const auto kernel = gemm_nt_dma_kernel<TC, MT, NT, W, __VA_ARGS__>;                                                               \
+    constexpr size_t lds = gemm_lds<MT, NT, __VA_ARGS__>();                                                                           \
     const int64_t n = blocks(MT, NT);                                                                                                 \
     if (n > 0x7fffffff) return 0;                                                                                                     \
-    const size_t lds = (size_t)ST * (MT + NT) * KS * 2;                                                                                   \
-    MIX_REQUIRE(ensure_lds((const void*)gemm_nt_dma_kernel<TC, MT, NT, W, WR, KS, ST>, lds) == 0, "gemm_nt: %zu bytes of LDS", lds);         \
-    hipLaunchKernelGGL((gemm_nt_dma_kernel<TC, MT, NT, W, WR, KS, ST>), dim3((unsigned)n), dim3(64 * W), lds, s, mp<TC>(C), cp<bf16_t>(A),      \
-                       cp<bf16_t>(B), M, N, K, lda, ldb, ldc, groups, a_gs, b_gs, c_gs, seg, a_rows, a_div, c_rows, act);             \
+    MIX_REQUIRE(ensure_lds((const void*)kernel, lds) == 0, "gemm_nt: %zu bytes of LDS", lds);                                         \
+    hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(64 * W), lds, s, mp<TC>(C), cp<bf16_t>(A), cp<bf16_t>(B), M, N, K, lda, ldb, ldc, groups, \
+                       a_gs, b_gs, c_gs, seg, a_rows, a_div, c_rows, act);                                                            \
   }
   // Rows per group on average, and how many of the largest tiles there are.  Groups x rows, N, K (us, weights not in cache):
   //                              64 x 128   128 x 128   256 x 256
@@ -236,6 +249,10 @@ extern "C" __attribute__((visibility("hidden"))) int mix_gemm_nt_dma(void* C, co
   // Groups of uneven length, as a router fills them (random | log-normal, sigma 0.7), where a 256-row tile holds one short group:
   //   64 x 96, 1024, 2048                      72.8 | 90.5   74.7 | 112    32 x 96, 2048, 1024: 29.8 | 43.0   33.8 | 56.7
   //   64 x 112, 1024, 2048                     97.2 | 90.7   76.9 | 114    32 x 128, 2048, 1024: 46.9 | 44.6   36.1 | 57.5
+  // Few rows a group, N 1024, K 2048, 64 groups (random | log-normal 0.7 | 1.3): 64-row tiles -> 32-row, B streaming -> 64-row, B streaming
+  //   x 4: 61.3 | 53.5 | 47.1 -> 51.5 | 45.5 | 41.3     x 14: 62.8 | 72.8 | 55.5 -> 52.8 | 61.2 | 54.6
+  //   x 20: 62.8 | 71.9 | 61.0 -> -> 56.7 | 67.4 | 57.9    x 40: 63.0 | 70.1 | 70.6 -> -> 57.2 | 66.8 | 66.8
+  //   x 62: 73.2 | 70.7 | 71.6 -> -> 74.9 | 77.3 | 79.5    (second row tiles read B again; a B small enough to stay in the last cache is 5 - 10 % slower)
   const int64_t each = seg ? M / groups : M;
   const bool large = each >= 112 && blocks(256, 256) >= 256;
 #define GEMM_SIZE(TC)                                                   \
@@ -243,6 +260,10 @@ extern "C" __attribute__((visibility("hidden"))) int mix_gemm_nt_dma(void* C, co
     if (K % 64) {                                                       \
       if (each < 64) GEMM_RUN(TC, 64, 128, 4, 1, 32, 6)                 \
       else GEMM_RUN(TC, 128, 128, 4, 2, 32, 4)                          \
+    } else if (each < 16) {                                             \
+      GEMM_RUN(TC, 32, 128, 4, 1, 64, 4, true)                          \
+    } else if (each < 48) {                                             \
+      GEMM_RUN(TC, 64, 128, 4, 1, 64, 3, true)                          \
     } else if (each < 64) {                                             \
       GEMM_RUN(TC, 64, 128, 4, 1, 64, 3)                                \
     } else if (!large) {                                                \

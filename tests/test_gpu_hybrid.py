@@ -465,6 +465,20 @@ def test_segmented_product_tiles(dev, lens, N, K, out):
     assert ((got.double().cpu() - ref).abs() <= err + (ref.abs() + err) * 2.0 ** -8 * (out == torch.bfloat16)).all()
 
 
+@pytest.mark.parametrize("lens,N,K,out", [
+    ([1], 8, 64, torch.bfloat16),                               # one row, one step
+    ([0, 33, 1, 32, 5, 0, 31, 16], 136, 192, torch.bfloat16),   # under 16 rows a group: ends of 32-row tiles, three steps for a ring of four
+    ([15] * 5, 264, 320, torch.float32),                        # five steps
+    ([90, 0, 3, 0, 0, 2], 128, 1024, torch.bfloat16),           # one group with most of the rows
+    ([64, 65, 1, 30], 136, 128, torch.bfloat16),                # up to 48: 64-row tiles, two steps for a ring of three
+    ([47, 47], 8, 576, torch.float32),
+    ([63, 40], 264, 256, torch.bfloat16),
+])
+def test_segmented_product_few_rows(dev, lens, N, K, out):
+    """The tiles for few rows a group, whose B passes by the caches: same references and bounds."""
+    test_segmented_product_tiles(dev, lens, N, K, out)
+
+
 @pytest.mark.parametrize("n,skip", [(1, 0), (7, 1), (2047, 0), (2048, 3), (2049, 0), (8191, 0), (8193, 1), (16385, 0), (40001, 2)])
 def test_bucketing_is_a_stable_sort(dev, n, skip):
     """Rounds of 2048 and 8192 entries, their ends, an unaligned list, experts without entries, the first and the last expert: whole numbers, equal."""
