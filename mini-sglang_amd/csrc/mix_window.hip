@@ -104,7 +104,8 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
   constexpr int NP = kWinTile * (NH / 4) * VC * 2 / NT;  // pieces per thread; with fewer key heads rows come more than once
   typedef uint32_t Piece __attribute__((ext_vector_type(4)));  // (as a struct the registers became memory)
   Piece pre_k[NP], pre_v[NP];
-  // the rows of a tile (its slots in s_slot[buf]) into registers, and from there to LDS; a tile's rows past the last key are that key's again.
+  // the rows of a tile (its slots in s_slot[buf]) into registers, and from there to LDS; a tile's rows past the last key are that key's again
+  // (their values become zeros in LDS).
   // No condition on a load or a store (columns past the head go to the row's padding): where one was skipped, the loaded registers were
   // copied, and the wave waited for the loads at once (464 - 533 us).
   const int to_k = has_k ? col : G * KC * 32, to_v = has_v ? col : G * VC * 16;
@@ -188,6 +189,10 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
       }
     }
     stage(pre_v, sv + to_v, VS);
+    if (nj > k_end) {  // values past the last key: a row that sees an infinite last one would add zero times infinity
+      for (int key = key0; key < kWinTile; key += rows)
+        if (j0 + key >= k_end) *reinterpret_cast<Piece*>(sv + to_v + key * VS) = Piece{0u, 0u, 0u, 0u};
+    }
     stage(pre_k, sk + to_k, KSR);
     put_slot(next_slot, (buf + 3) & 3);
     __syncthreads();

@@ -72,6 +72,34 @@ def test_attention_rows_that_a_number_reaches(dev, call, group):
     assert not torch.isfinite(got[row: NEW[0], 5]).any()
 
 
+def test_window_row_that_sees_an_infinite_value_at_its_end(dev):
+    """Decoded tokens whose own value is infinite in one column: a weight enters the product in three bf16 parts, all positive for about a quarter of
+    the rows, and these have an infinite result.  Nothing that lies behind the last key in its tile turns it into a NaN."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(3)
+    lens = [5 + 29 * b for b in range(20)]
+    lens = [n + (n % 32 == 0) for n in lens]
+    table, at = torch.zeros((len(lens), 600), dtype=torch.int32), 0
+    for b, n in enumerate(lens):
+        table[b, :n] = torch.arange(at, at + n)
+        at += n
+    ends = torch.tensor(lens).cumsum(0) - 1
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    key, value = (torch.randn(at, 512, generator=g).bfloat16() for _ in range(2))
+    value[ends, 5::128] = torch.inf
+    q = torch.randn(len(lens), 16 * 129, generator=g).bfloat16().to(dev)
+    for splits in (1, 3):
+        out = torch.empty((len(lens), 16 * 128), dtype=torch.bfloat16, device=dev)
+        mixops.window_attn(out, q, 16 * 128, key.to(dev), value.to(dev), table.to(dev), i32(range(len(lens))), i32(lens), i32(range(len(lens) + 1)), len(lens),
+                           16, 4, 128, 128, 0, 0.05, torch.eye(16, device=dev) + 0.1, splits=splits, max_keys=max(lens))
+        hit = out[:, 5::128]
+        assert not torch.isfinite(hit).any() and torch.isposinf(hit).float().mean() > 0.1
+        keep = torch.ones(16 * 128, dtype=torch.bool, device=dev)
+        keep[5::128] = False
+        assert torch.isfinite(out[:, keep]).all()
+
+
 @pytest.mark.parametrize("lens,N,K", [((1, 3, 40), 72, 64), ((64, 65, 127), 264, 96), ((256, 511, 300) * 20, 520, 64)], ids=["short", "middling", "long"])
 def test_product_row_and_column_that_a_number_reaches(dev, lens, N, K):
     """Segmented products: an operand's row with a NaN or an infinity makes its row or column of the result undefined and leaves the rest its bits."""
