@@ -102,12 +102,15 @@ class HipAttnBackend:
         self.kv_heads = max(config.num_kv_heads // tp_size, 1)
         self.max_bs = int(ctx.page_table.shape[0])
         self.capacity = decode_capacity or max(4096, 4 * self.max_bs)
-        self._workspace = torch.empty(max(ops.attn_decode_workspace_bytes(self.capacity, self.qo_heads, self.head_dim),
-                                          ops.prefill_ranges_workspace_bytes()), dtype=torch.uint8, device=self.device)
         self._plan_words = ops.attn_decode_plan_words(self.max_bs, self.capacity)
         self._small_heads = 0  # requests x kv heads of a decode batch up to which `small_decode` says yes
         if self.head_dim == 128 and self.qo_heads % self.kv_heads == 0 and self.qo_heads // self.kv_heads <= 8:
             self._small_heads = SMALL_DECODE_HEADS * (2 if self.kv_heads <= 2 or int(ctx.page_table.shape[1]) <= 4096 else 1)
+        # decode steps only: one at a time per backend (prompts take scratch of their own)
+        small = (ops.attn_decode_small_workspace_bytes(b, ops.attn_decode_small_ranges(b, self.kv_heads, ctx.page_table.shape[1]), self.qo_heads)
+                 for b in range(1, self._small_heads // self.kv_heads + 1))
+        self._workspace = torch.empty(max([ops.attn_decode_workspace_bytes(self.capacity, self.qo_heads, self.head_dim), *small]),
+                                      dtype=torch.uint8, device=self.device)
         # graph state
         self.capture_bs: List[int] = []
         self.max_graph_bs = 0
@@ -174,9 +177,13 @@ class HipAttnBackend:
             ops.attn_decode(out, q, k_tok, v_tok, table, md.req_rows, md.seq_lens, md.plan, self._workspace,
                             md.batch, self.max_bs, self.capacity, self.scale, slot_run=self.slot_run)
         else:
+            # sums of key ranges: scratch of this call's stream, not the decode steps', which may run beside it on another one
+            scratch = None
+            if md.ranges[0] > 1:
+                scratch = torch.empty(ops.prefill_ranges_workspace_bytes(md.total_tiles * self.qo_heads * md.ranges[0]), dtype=torch.uint8, device=self.device)
             ops.attn_prefill(out, q, k_tok, v_tok, table, md.req_rows, md.seq_lens, md.cu_seqlens_q, md.tile_cu,
                              md.batch, md.total_tiles, self.scale, tile_order=md.tile_order,
-                             ranges=md.ranges, workspace=self._workspace)
+                             ranges=md.ranges, workspace=scratch)
         return out
 
     # ------------------------------------------------------------------ metadata

@@ -358,6 +358,12 @@ def attn_decode_small_ranges(batch: int, num_kv_heads: int, max_seq_len: int) ->
     return n
 
 
+def attn_decode_small_workspace_bytes(batch: int, ranges: int, num_q_heads: int) -> int:
+    n = int(lib().msgl_attn_decode_small_workspace_bytes(batch, ranges, num_q_heads))
+    check(min(n, 0), "attn_decode_small_workspace_bytes")
+    return n
+
+
 def attn_decode_small(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                       out_loc: torch.Tensor, page_table: torch.Tensor, req_rows: Optional[torch.Tensor], seq_lens: torch.Tensor,
                       workspace: torch.Tensor, ranges: int, sm_scale: float, q_norm_w: Optional[torch.Tensor] = None,
@@ -409,9 +415,6 @@ def prefill_q_tile(impl: Optional[int] = None) -> int:
     return int(lib().msgl_attn_prefill_q_tile(PREFILL_IMPL if impl is None else int(impl)))
 
 
-PREFILL_RANGE_JOBS = 800  # workgroups that `prefill_ranges` makes of a launch at most
-
-
 def prefill_ranges(total_tiles: int, qo_heads: int, max_seqlen_q: int, max_seqlen_k: int) -> Tuple[int, int]:
     """Key ranges of a (q tile, head) of the default prefill kernel at most, and 64-key tiles of each.
 
@@ -435,8 +438,8 @@ def prefill_ranges(total_tiles: int, qo_heads: int, max_seqlen_q: int, max_seqle
     return (ranges, run) if ranges > 1 else (1, 0)
 
 
-def prefill_ranges_workspace_bytes(jobs: int = PREFILL_RANGE_JOBS) -> int:
-    """For any ranges of `prefill_ranges`, or for `jobs` = q tiles x heads x ranges."""
+def prefill_ranges_workspace_bytes(jobs: int) -> int:
+    """`jobs`: q tiles x heads x ranges (`prefill_ranges` makes at most 800 of a launch, 54 MB)."""
     return int(lib().msgl_attn_prefill_ranges_workspace_bytes(jobs, 1, 1))
 
 

@@ -251,3 +251,47 @@ def test_prefill_key_ranges(ops, dev, monkeypatch, hq, hkv, specs, ranges, dtype
             if -(-(k - n + min(t + 128, n)) // 64) <= ranges[1]:
                 assert torch.equal(out[rows], whole[rows])
         at += n
+
+
+def test_prompt_attention_leaves_the_decode_workspace_alone(ops, dev):
+    """Prompts and decode steps of one backend on different streams share no scratch: the sums of key ranges live in memory of their own."""
+    from mini_sglang_amd.attention import HipAttnBackend
+    from mini_sglang_amd.core import Batch, Context, Req
+    from mini_sglang_amd.kvcache import create_kvcache_pool
+    from mini_sglang_amd.model import ModelConfig
+
+    old, new, hq, hkv = 2000, 100, 16, 8
+    ctx = Context(16)
+    m = ModelConfig(num_layers=1, num_qo_heads=hq, num_kv_heads=hkv, head_dim=128, hidden_size=1024, vocab_size=64, intermediate_size=64)
+    ctx.page_table = torch.arange(2 * 2112, dtype=torch.int32, device=dev).view(2, 2112) % 2112
+    ctx.kv_cache = create_kvcache_pool(m, 132, 16, torch.bfloat16, dev)
+    for t in (ctx.kv_cache.k_tokens(0), ctx.kv_cache.v_tokens(0)):
+        t.normal_()
+    backend = HipAttnBackend(m, ctx)
+    batch = Batch(reqs=[Req(input_ids=torch.zeros(old + new, dtype=torch.int32), table_idx=0, cached_len=old, output_len=1, uid=0)], phase="prefill")
+    batch.out_loc = torch.arange(old, old + new, dtype=torch.int32, device=dev)
+    batch.padded_reqs = batch.reqs
+    backend.prepare_metadata(batch)
+    assert batch.attn_metadata.ranges[0] > 1
+    backend._workspace.fill_(0x5A)
+    q, k, v = (torch.randn(new, h * 128, device=dev).bfloat16() for h in (hq, hkv, hkv))
+    out = backend.forward(q.view(new, hq, 128), k, v, 0, batch)
+    assert torch.isfinite(out).all() and bool((backend._workspace == 0x5A).all())
+
+
+def test_a_small_decode_capacity_holds_the_small_batch_kernel(ops, dev):
+    """The decode workspace is at least what small batches take, whatever number of pieces the caller asks for."""
+    from mini_sglang_amd.attention import HipAttnBackend
+    from mini_sglang_amd.core import Context
+    from mini_sglang_amd.kvcache import create_kvcache_pool
+    from mini_sglang_amd.model import ModelConfig
+
+    for hq, hkv in ((16, 8), (8, 1), (64, 8)):
+        ctx = Context(16)
+        m = ModelConfig(num_layers=1, num_qo_heads=hq, num_kv_heads=hkv, head_dim=128, hidden_size=1024, vocab_size=64, intermediate_size=64)
+        ctx.page_table = torch.zeros((70, 40960), dtype=torch.int32, device=dev)
+        ctx.kv_cache = create_kvcache_pool(m, 4, 16, torch.bfloat16, dev)
+        backend = HipAttnBackend(m, ctx, decode_capacity=70)
+        for b in range(1, backend._small_heads // hkv + 1):
+            need = ops.lib().msgl_attn_decode_small_workspace_bytes(b, ops.attn_decode_small_ranges(b, hkv, 40960), hq)
+            assert backend._workspace.numel() >= need, (hq, hkv, b)
