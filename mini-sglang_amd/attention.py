@@ -35,6 +35,7 @@ class HipAttnMetadata:
     total_tiles: int = 0
     tile_order: Optional[torch.Tensor] = None  # [total_tiles] int32: q tiles, most keys first (prefill only)
     ranges: tuple = (1, 0)                  # key ranges of a q tile, 64-key tiles of each (prefill only)
+    scratch: Optional[torch.Tensor] = None  # their partial sums, from the first layer on
     plan: Optional[torch.Tensor] = None     # decode work list (device)
     chunks: Optional[tuple] = None          # recurrent layers: (items [n, 3], item_first [B + 1], n) of long portions cut in pieces
     delta_chunks: Optional[tuple] = None    # the same list at the delta-rule layers' piece size
@@ -106,7 +107,7 @@ class HipAttnBackend:
         self._small_heads = 0  # requests x kv heads of a decode batch up to which `small_decode` says yes
         if self.head_dim == 128 and self.qo_heads % self.kv_heads == 0 and self.qo_heads // self.kv_heads <= 8:
             self._small_heads = SMALL_DECODE_HEADS * (2 if self.kv_heads <= 2 or int(ctx.page_table.shape[1]) <= 4096 else 1)
-        # decode steps only: one at a time per backend (prompts take scratch of their own)
+        # decode steps only: one at a time per backend (prompts have scratch of their own)
         small = (ops.attn_decode_small_workspace_bytes(b, ops.attn_decode_small_ranges(b, self.kv_heads, ctx.page_table.shape[1]), self.qo_heads)
                  for b in range(1, self._small_heads // self.kv_heads + 1))
         self._workspace = torch.empty(max([ops.attn_decode_workspace_bytes(self.capacity, self.qo_heads, self.head_dim), *small]),
@@ -177,13 +178,12 @@ class HipAttnBackend:
             ops.attn_decode(out, q, k_tok, v_tok, table, md.req_rows, md.seq_lens, md.plan, self._workspace,
                             md.batch, self.max_bs, self.capacity, self.scale, slot_run=self.slot_run)
         else:
-            # sums of key ranges: scratch of this call's stream, not the decode steps', which may run beside it on another one
-            scratch = None
-            if md.ranges[0] > 1:
-                scratch = torch.empty(ops.prefill_ranges_workspace_bytes(md.total_tiles * self.qo_heads * md.ranges[0]), dtype=torch.uint8, device=self.device)
+            if md.ranges[0] > 1 and md.scratch is None:
+                # this batch's own, for its layers one after the other: other batches may run beside it on other streams, decode steps among them
+                md.scratch = torch.empty(ops.prefill_ranges_workspace_bytes(md.total_tiles * self.qo_heads * md.ranges[0]), dtype=torch.uint8, device=self.device)
             ops.attn_prefill(out, q, k_tok, v_tok, table, md.req_rows, md.seq_lens, md.cu_seqlens_q, md.tile_cu,
                              md.batch, md.total_tiles, self.scale, tile_order=md.tile_order,
-                             ranges=md.ranges, workspace=scratch)
+                             ranges=md.ranges, workspace=md.scratch)
         return out
 
     # ------------------------------------------------------------------ metadata
