@@ -969,7 +969,8 @@ __global__ __launch_bounds__(kRowThreads, 8) void split_max_kernel(SplitScratch 
 #pragma unroll
       for (int u = 0; u < kDeep; ++u) x[u] = load_logit<DT>(row, min(base + u * kRowThreads, hi - 1));
 #pragma unroll
-      for (int u = 0; u < kDeep; ++u) mx = fmaxf(mx, x[u]);
+      for (int u = 0; u < kDeep; ++u)  // (a number counts once: the k-th largest of the maxima is to bound the k-th largest number)
+        if (base + u * kRowThreads < hi) mx = fmaxf(mx, x[u]);
     }
   }
   for (int d = 1; d < split; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));  // one maximum per `split` neighbours

@@ -4,6 +4,8 @@ The reference's RNG stream (flashinfer) cannot be reproduced, so non-greedy samp
 distributionally (chi-square against the exact filtered distribution of the oracle) plus exactness
 on degenerate rows (top_k = 1, top_p -> 0  =>  argmax), as SURVEY.md Appendix B prescribes.
 """
+import math
+
 import pytest
 import torch
 
@@ -352,3 +354,30 @@ def test_a_row_shared_by_workgroups_draws_the_same(ops, dev, dtype, rows, vocab)
     if (vocab * logits.element_size()) % 16 == 0:  # the unfiltered draw from the logits: as its own rows one by one, each with more workgroups
         got = ops.sample_from_logits(logits, t, 5, 300).tolist()
         assert got == [int(ops.sample_from_logits(logits[r: r + 1], t[r: r + 1], 5, 300 + r)) for r in range(rows)]
+
+
+def _draw_with_workspace(ops, dev, logits, t, k, p):
+    """A shared-row draw with a workspace to look into: its first parts are 16 bytes a row (maximum, candidates' bound, ..) and 1024 maxima a row."""
+    rows, vocab = logits.shape
+    n = ops.lib().msgl_sample_workspace_bytes(rows, vocab, 1, k is not None, p is not None)
+    assert n > 0
+    ws, out = torch.zeros(n, dtype=torch.uint8, device=dev), torch.empty(rows, dtype=torch.int32, device=dev)
+    ops.check(ops.lib().msgl_sample_filtered_logits_ws(
+        out.data_ptr(), None, None, logits.data_ptr(), t.data_ptr(), None if k is None else k.data_ptr(), None if p is None else p.data_ptr(), rows, vocab,
+        logits.stride(0), ops._logits_dt(logits), 1, 0, ws.data_ptr(), n, ops._stream()), "sample")
+    torch.cuda.synchronize()
+    at = (16 * rows + 255) // 256 * 256
+    return ws[: 16 * rows].view(torch.int32).view(rows, 4), ws[at: at + 4096 * rows].view(torch.float32).view(rows, 1024)
+
+
+@pytest.mark.parametrize("vocab", [100001, 98304, 131073])
+def test_maxima_of_a_shared_row_are_of_different_numbers(ops, dev, vocab):
+    """The k-th largest of the 1024 maxima bounds the k-th largest number from below only if no number counts twice; a row that the bound cuts short is
+    drawn by radix levels, six times as slow.  All numbers differ, and a workgroup's last one is its largest."""
+    rows = 4
+    logits = torch.arange(vocab, device=dev, dtype=torch.float32).repeat(rows, 1).mul_(1e-3)
+    t, k = torch.ones(rows, device=dev), torch.full((rows,), 20, dtype=torch.int32, device=dev)
+    head, top = _draw_with_workspace(ops, dev, logits, t, k, None)
+    for r in range(rows):
+        real = top[r][top[r] > -math.inf]
+        assert real.numel() == real.unique().numel() and real.numel() > 512
