@@ -381,3 +381,21 @@ def test_maxima_of_a_shared_row_are_of_different_numbers(ops, dev, vocab):
     for r in range(rows):
         real = top[r][top[r] > -math.inf]
         assert real.numel() == real.unique().numel() and real.numel() > 512
+
+
+@pytest.mark.parametrize("temperature", [1.0, 0.25, 0.1])
+def test_the_bound_of_candidates_reaches_low_temperatures(ops, dev, temperature):
+    """The k-th largest weight of a sharp row (2^-29, 2^-115 and, at 0.1, none above 0) is bounded from below as long as there is one."""
+    rows, vocab = 3, 131072
+    logits = torch.full((rows, vocab), -4.0, device=dev)
+    logits[:, ::1021] = 0.0
+    logits[:, 777] = 20.0
+    t, k = torch.full((rows,), temperature, device=dev), torch.full((rows,), 30, dtype=torch.int32, device=dev)
+    head, _ = _draw_with_workspace(ops, dev, logits, t, k, None)
+    weight = 2.0 ** (-20.0 / temperature * 1.4426950408889634)
+    for bits in head[:, 1].tolist():
+        if weight > 2.0 ** -126:
+            bound = torch.tensor(bits, dtype=torch.int32).view(torch.float32).item()
+            assert weight / 1.25 <= bound <= weight * 1.00001
+        else:
+            assert bits == 0
