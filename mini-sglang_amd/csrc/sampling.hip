@@ -1394,13 +1394,20 @@ __global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc
 }
 
 // Workgroups per row (1: one walks the row).  One a compute unit in all: 64 rows x 151936, top-p alone, 54 us with 4 each, 58 with 8; 33 rows 51 and 54.
-// Where sharing pays, us a draw, shared / one workgroup:
+// Where sharing pays, us a draw, shared / one workgroup, bf16:
 //   top-k      1 x 151936 20.5 / 25.2, 33 x 151936 29.4 / 31.4, 64 x 151936 29.1 / 34.2, but 8 x 65536 20.4 / 17.5, 100 x 151936 41 / 38
-//   top-p      2 x 32000 34 / 50, 64 x 35186 38 / 52, 256 x 50000 60 / 69, 256 x 151936 119 / 197
-//   no filter  8 x 65536 13.9 / 16.0, 100 x 151936 29 / 37, but 32 x 50000 14.8 / 14.8, 128 x 50000 18.2 / 15.3, 256 x 151936 48 / 44
+//   no filter  64 x 65536 16.5 / 17.7, 128 x 98304 24.4 / 25.9, 100 x 151936 29 / 37, but 128 x 65536 20.4 / 18.7, 128 x 50000 18.2 / 15.3,
+//              32 x 50000 14.8 / 14.8, 256 x 151936 48 / 44
+//   top-p      wide nuclei (logits of deviation 2.5) and, behind them, nuclei of a few tokens in every row (deviation 10), which one workgroup
+//              finds in its list of 64 candidates:
+//              1 x 32000 32 / 56, 32 / 27     8 x 50304 40 / 69, 39 / 30     64 x 16384 32 / 40, 31 / 25     64 x 50304 36 / 71, 35 / 31
+//              64 x 151936 51 / 161, 49 / 57     128 x 151936 72 / 175, 68 / 63     256 x 151936 108 / 195, 99 / 70
+//              One wide row sets the time of a batch.  The line lies where sharing saves less on wide rows than it costs on narrow ones:
+//              1 x 8200 28 / 33, 28 / 20     8 x 16384 33 / 39, 33 / 22     64 x 8200 31 / 34, 30 / 21     128 x 8200 30 / 35, 30 / 23
 static inline int split_of(int64_t rows, int64_t vocab, bool filtered, bool has_k, bool has_p) {
   const bool by_mass = filtered && has_p && !has_k;
-  const int64_t most = by_mass ? 256 : has_k ? 64 : 128, shortest = by_mass ? 8192 : has_k ? 98304 : 65536;
+  const int64_t most = by_mass ? 256 : has_k ? 64 : 128;
+  const int64_t shortest = by_mass ? (rows < 64 ? 32000 : 16384) : has_k || rows > 64 ? 98304 : 65536;
   if (rows > most || vocab < shortest) return 1;
   int split = 16;
   while (split > 2 && (rows * split > 256 || vocab / split < 2048)) split /= 2;

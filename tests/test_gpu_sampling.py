@@ -327,7 +327,8 @@ def test_nucleus_at_the_list_s_length(ops, dev, vocab):
 # rows that 16, 8, 4, 2 and 1 workgroups share, with and without a top-k; vocabularies at the shortest rows that are shared, beside whole columns and
 # chunks, and above 1024 chunks of 512; masses whose threshold lies high, in the tail, in a tie and (column) among numbers that the bound misses
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("rows,vocab", [(3, 65536), (33, 33333), (40, 8192), (130, 8193), (257, 8200), (2, 600_003), (64, 98304), (17, 98309), (65, 98304)])
+@pytest.mark.parametrize("rows,vocab", [(3, 65536), (33, 33333), (40, 8192), (130, 8193), (257, 8200), (2, 600_003), (64, 98304), (17, 98309), (65, 98304),
+                                        (130, 16391), (64, 16384), (9, 32000)])
 def test_a_row_shared_by_workgroups_draws_the_same(ops, dev, dtype, rows, vocab):
     g = torch.Generator(device=dev).manual_seed(vocab)
     logits = torch.randn((rows, vocab), generator=g, device=dev) * 2.5
@@ -399,3 +400,13 @@ def test_the_bound_of_candidates_reaches_low_temperatures(ops, dev, temperature)
             assert weight / 1.25 <= bound <= weight * 1.00001
         else:
             assert bits == 0
+
+
+# (filter, rows, vocabulary) on both sides of the lines that split_of's comment gives times for
+@pytest.mark.parametrize("how,rows,vocab,shared", [
+    ("none", 64, 65536, True), ("none", 65, 65536, False), ("none", 128, 98303, False), ("none", 128, 98304, True), ("none", 129, 98304, False),
+    ("k", 64, 98304, True), ("k", 1, 98303, False), ("k", 65, 151936, False),
+    ("p", 1, 31999, False), ("p", 1, 32000, True), ("p", 63, 31999, False), ("p", 64, 16384, True), ("p", 64, 16383, False), ("p", 256, 16384, True), ("p", 257, 32000, False),
+])
+def test_draws_that_share_their_rows(ops, how, rows, vocab, shared):
+    assert (ops.lib().msgl_sample_workspace_bytes(rows, vocab, how != "none", how == "k", how == "p") > 0) is shared
