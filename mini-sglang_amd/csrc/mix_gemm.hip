@@ -252,17 +252,24 @@ extern "C" __attribute__((visibility("hidden"))) int mix_gemm_nt_dma(void* C, co
   // Few rows a group, N 1024, K 2048, 64 groups (random | log-normal 0.7 | 1.3): 64-row tiles -> 32-row, B streaming -> 64-row, B streaming
   //   x 4: 61.3 | 53.5 | 47.1 -> 51.5 | 45.5 | 41.3     x 14: 62.8 | 72.8 | 55.5 -> 52.8 | 61.2 | 54.6
   //   x 20: 62.8 | 71.9 | 61.0 -> -> 56.7 | 67.4 | 57.9    x 40: 63.0 | 70.1 | 70.6 -> -> 57.2 | 66.8 | 66.8
-  //   x 62: 73.2 | 70.7 | 71.6 -> -> 74.9 | 77.3 | 79.5    (second row tiles read B again; a B small enough to stay in the last cache is 5 - 10 % slower)
+  //   x 62: 73.2 | 70.7 | 71.6 -> -> 74.9 | 77.3 | 79.5    (second row tiles read B again)
+  // A B that the last cache (256 MB) keeps from one pass to the next loses by streaming, and small ones belong to models that it holds.  Layers in
+  // turn that take 200 | 800 MB, us (64-row tiles, and under 16 rows a group 32-row ones; B streaming): the line lies at 64 MB
+  //   34 MB (16 x 1024 x 1024)   x 4: 9.3 | 10.5; 10.4 | 10.1     x 14: 9.6 | 11.2; 11.1 | 10.8     x 40: 10.6 | 12.7; 12.4 | 12.4
+  //   50 MB (24 x 1024 x 1024)   x 4: 10.8 | 12.3; 11.3 | 11.3    x 20: 11.7 | 13.4; 12.6 | 12.6    x 40: 12.3 | 14.0; 13.1 | 13.2
+  //   67 MB (32 x 1024 x 1024)   x 4 (64-row tiles): 13.4 | 15.5; 13.8 | 13.9    x 20: 13.8 | 15.8; 14.0 | 14.4    x 40: 14.6 | 16.3; 14.5 | 15.1
   const int64_t each = seg ? M / groups : M;
   const bool large = each >= 112 && blocks(256, 256) >= 256;
+  const bool stream = (int64_t)groups * N * K >= 32 << 20;
 #define GEMM_SIZE(TC)                                                   \
   {                                                                     \
     if (K % 64) {                                                       \
       if (each < 64) GEMM_RUN(TC, 64, 128, 4, 1, 32, 6)                 \
       else GEMM_RUN(TC, 128, 128, 4, 2, 32, 4)                          \
     } else if (each < 16) {                                             \
-      GEMM_RUN(TC, 32, 128, 4, 1, 64, 4, true)                          \
-    } else if (each < 48) {                                             \
+      if (stream) GEMM_RUN(TC, 32, 128, 4, 1, 64, 4, true)              \
+      else GEMM_RUN(TC, 32, 128, 4, 1, 64, 4)                           \
+    } else if (each < 48 && stream) {                                   \
       GEMM_RUN(TC, 64, 128, 4, 1, 64, 3, true)                          \
     } else if (each < 64) {                                             \
       GEMM_RUN(TC, 64, 128, 4, 1, 64, 3)                                \

@@ -473,9 +473,11 @@ def test_segmented_product_tiles(dev, lens, N, K, out):
     ([64, 65, 1, 30], 136, 128, torch.bfloat16),                # up to 48: 64-row tiles, two steps for a ring of three
     ([47, 47], 8, 576, torch.float32),
     ([63, 40], 264, 256, torch.bfloat16),
+    ([0, 33, 1, 32, 5, 0, 31, 16] * 4, 1032, 1088, torch.bfloat16),  # B of 72 MB, which passes by the caches
+    ([64, 65, 1, 30] * 8, 1032, 1088, torch.float32),
 ])
 def test_segmented_product_few_rows(dev, lens, N, K, out):
-    """The tiles for few rows a group, whose B passes by the caches: same references and bounds."""
+    """The tiles for few rows a group, B through the caches and past them: same references and bounds."""
     test_segmented_product_tiles(dev, lens, N, K, out)
 
 
