@@ -784,9 +784,9 @@ def norm_linear_tune(x: torch.Tensor, weights, silu: bool = False, iters: int = 
         linear_silu(y, w, out) if silu else linear(y, w, out)
 
     def time_us(p, rounds):
-        return _time_launches_us(lambda w: norm_linear(x, w, p[0], p[1], r0, r1, gamma, 1e-6, silu, out), weights, iters, rounds, ahead=True)
+        return _time_launches_us(lambda w: norm_linear(x, w, p[0], p[1], r0, r1, gamma, 1e-6, silu, out), weights, iters, rounds)
 
-    res["norm_unfused_us"] = _time_launches_us(unfused, weights, iters, 3, ahead=True)
+    res["norm_unfused_us"] = _time_launches_us(unfused, weights, iters, 3)
     ranked = sorted((time_us(p, 1), p) for p in settings)
     best = min((time_us(p, 3), p) for _, p in ranked[:3])
     res.update(norm_fused_us=best[0], norm_plan=best[1])
@@ -872,7 +872,7 @@ def skinny_tune(x: torch.Tensor, weights, library_us: float, iters: int = 8, fol
     out = torch.empty((M, N), dtype=x.dtype, device=x.device)
 
     def time_us(sl, nt, rounds):
-        return _time_launches_us(lambda w: skinny_linear(x, w, sl, out, nt), weights, iters, rounds, ahead=True)
+        return _time_launches_us(lambda w: skinny_linear(x, w, sl, out, nt), weights, iters, rounds)
 
     def credit(sl):
         folds = fold_mode is not None and sl <= 0 and rowstream_supported(M, N, K, fold_mode, -sl)
@@ -947,17 +947,7 @@ def wstream_tune(x: torch.Tensor, weights, incumbent_us: float, iters: int = 8) 
     out = torch.empty((M, N), dtype=x.dtype, device=x.device)
 
     def time_us(nt, ks, rounds):
-        wstream_linear(x, w0, nt, ks, out)  # warm-up
-        ts = []
-        for _ in range(rounds):
-            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            e0.record()
-            for i in range(iters):
-                wstream_linear(x, weights[(i + 1) % len(weights)], nt, ks, out)
-            e1.record()
-            e1.synchronize()
-            ts.append(e0.elapsed_time(e1) * 1e3 / iters)
-        return min(ts)
+        return _time_launches_us(lambda w: wstream_linear(x, w, nt, ks, out), weights, iters, rounds)
 
     cands = wstream_candidates(M, N, K)
     if not cands:
@@ -1026,17 +1016,21 @@ def m256_candidates(M: int, N: int, K: int, cus: int):
     return out
 
 
-def _time_launches_us(fn, weights, iters: int, rounds: int, ahead: bool = False) -> float:
+def _time_launches_us(fn, weights, iters: int, rounds: int) -> float:
     """min over `rounds` of the mean time of `iters` launches of fn(w) on rotating weights (events on this stream).
-    ahead: the launches are queued behind a kernel that keeps the GPU busy for a while.  Issuing one from here takes the host
+    The launches are queued behind a kernel that keeps the GPU busy for a while.  Issuing one from here takes the host
     about 8 us; without that, everything that runs for less measures as 8 us and the choice between such kernels is chance
-    (a down projection of 6 MB got a plan of 9.9 us instead of 5.8, a decode step of Qwen3-0.6B 1390 us instead of 1260)."""
+    (a down projection of 6 MB got a plan of 9.9 us instead of 5.8, a decode step of Qwen3-0.6B 1390 us instead of 1260).
+    Every time of a hand-written kernel that the plan search compares with another one is taken here.  The library's own search
+    (csrc/gemm.cpp) stays on its clock, an event before and behind every launch, some 5 us more than a launch takes among others: its
+    rivals' times contain the sum over k-slices, which a step leaves to the next kernel (linear_slabs).  Timed here as well, the
+    library won projections by which steps lost: 14B layers, 32 rows 996 -> 1048 us (6 layers), a quarter's shard, 256 rows 1985 -> 2050
+    (12 layers); Qwen3-0.6B, 24 rows 1749 -> 1802, though 128 rows 3220 -> 3060."""
     fn(weights[0])  # warm-up
     ts = []
     for _ in range(rounds):
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        if ahead:
-            torch.cuda._sleep(iters * 60_000)  # about 26 us of the GPU per launch
+        torch.cuda._sleep(iters * 60_000)  # about 26 us of the GPU per launch
         e0.record()
         for i in range(iters):
             fn(weights[(i + 1) % len(weights)])
@@ -1096,10 +1090,10 @@ def fused_silu_tune(x: torch.Tensor, weights, iters: int = 8) -> dict:
         # is planned to do for the shape + the activation kernel
         half = torch.empty((M, N // 2), dtype=x.dtype, device=x.device)
         full = torch.empty((M, N), dtype=x.dtype, device=x.device)  # (no allocation inside the timed pair: it is not there under replay)
-        res["unfused_us"] = _time_launches_us(lambda w: silu_and_mul_interleaved(linear(x, w, full), half), weights, iters, 3, ahead=True)
-        ranked = sorted((_time_launches_us(lambda w: skinny_linear_silu(x, w, sl, half, nt), weights, iters, 1, ahead=True), (sl, nt))
+        res["unfused_us"] = _time_launches_us(lambda w: silu_and_mul_interleaved(linear(x, w, full), half), weights, iters, 3)
+        ranked = sorted((_time_launches_us(lambda w: skinny_linear_silu(x, w, sl, half, nt), weights, iters, 1), (sl, nt))
                         for sl, nt in skinny_silu_candidates(M, N, K))
-        best = min((_time_launches_us(lambda w: skinny_linear_silu(x, w, p[0], half, p[1]), weights, iters, 3, ahead=True), p)
+        best = min((_time_launches_us(lambda w: skinny_linear_silu(x, w, p[0], half, p[1]), weights, iters, 3), p)
                    for _, p in ranked[:4])
         res.update(fused_us=best[0], plan=best[1], kind="skinny")
         if best[0] < res["unfused_us"]:  # one launch less in front of the same consumer: no margin asked

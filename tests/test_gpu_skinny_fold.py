@@ -69,3 +69,50 @@ def test_four_rows_per_workgroup_is_the_product(ops, dev, dtype, M, N, K):
         err = (got.double() - want).abs()
         assert bool((err <= want.abs() * eps / 2 + K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())).all()), (sl, err.max())
         assert bool((out[M:] == 7).all()) and bool((out[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("M", [4, 48, 200])
+def test_plan_search_times_every_family_behind_a_busy_gpu(ops, dev, monkeypatch, M):
+    """The hand-written kernels' times are all taken the same way: issued from the host, every launch below 8 us measures as 8 us."""
+    from mini_sglang_amd.gemm_plan import tune_projection_gemms
+
+    clock, sleep, inside, outside = ops._time_launches_us, torch.cuda._sleep, [False], []
+    timed, slept = set(), [0]
+
+    def sleeping(cycles):
+        slept[0] += 1
+        return sleep(cycles)
+
+    def recording(fn, weights, iters, rounds, *a, **k):
+        inside[0], slept[0] = True, 0
+        try:
+            return clock(fn, weights, iters, rounds, *a, **k)
+        finally:
+            inside[0] = False
+            assert slept[0] == rounds
+
+    def watch(name):
+        plain = getattr(ops, name)
+
+        def call(*a, **k):
+            (timed.add if inside[0] else outside.append)(name)
+            return plain(*a, **k)
+
+        monkeypatch.setattr(ops, name, call)
+
+    families = ["skinny_linear", "skinny_linear_silu", "norm_linear", "wstream_linear", "full_batch_linear", "g3_linear", "ro_linear"]
+    for name in families:
+        watch(name)
+    monkeypatch.setattr(ops, "_time_launches_us", recording)
+    monkeypatch.setattr(torch.cuda, "_sleep", sleeping)
+    g = torch.Generator(device=dev).manual_seed(M)
+    N, K = 2048, 1024
+    ws = [ops.interleave_gate_up(_rnd(g, N, K, dtype=torch.bfloat16, std=K ** -0.5)) for _ in range(3)]
+    try:
+        tune_projection_gemms([("gate_up", ws, K, {"silu_interleaved": True, "fold": "norm"})], [M], "heuristic", torch.bfloat16, dev)
+        want = {4: {"skinny_linear", "skinny_linear_silu", "norm_linear", "ro_linear"},
+                48: {"skinny_linear", "skinny_linear_silu", "wstream_linear", "ro_linear"},
+                200: {"wstream_linear", "full_batch_linear", "g3_linear", "ro_linear"}}[M]
+        assert want <= timed and not outside
+    finally:
+        ops.reset_gemm_plans()
