@@ -134,7 +134,13 @@ def tune_projection_gemms(groups: Sequence[Group], batch_sizes: Sequence[int], m
                     r["kernel"] = "msgl::ro_gemm_kernel<silu>[tiles %d]" % rs["plan"][0]
             if flags.get("fold") == "norm" and bs <= ops.NORM_LINEAR_MAX_M:
                 # the add + norm in front of this projection inside its launch, against the two launches as planned so far
-                r.update(ops.norm_linear_tune(x, ws, silu=bool(flags.get("silu_interleaved"))))
+                nr = ops.norm_linear_tune(x, ws, silu=bool(flags.get("silu_interleaved")))
+                r.update(nr)
+                if nr["norm_used"]:
+                    r.setdefault("library_best_us", r["best_us"])
+                    r["best_us"] = nr["norm_fused_us"]  # the norm, the projection and, if interleaved, the activation
+                    r["skinny_used"] = True
+                    r["kernel"] = "msgl::skinny_gemm_kernel<norm%s>[slices %d, row tiles %d]" % ((", silu" if flags.get("silu_interleaved") else "",) + tuple(nr["norm_plan"]))
             ops.register_candidates(name, x, ws[0], r)
             report.append(r)
             if log is not None:

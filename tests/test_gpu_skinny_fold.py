@@ -109,10 +109,13 @@ def test_plan_search_times_every_family_behind_a_busy_gpu(ops, dev, monkeypatch,
     N, K = 2048, 1024
     ws = [ops.interleave_gate_up(_rnd(g, N, K, dtype=torch.bfloat16, std=K ** -0.5)) for _ in range(3)]
     try:
-        tune_projection_gemms([("gate_up", ws, K, {"silu_interleaved": True, "fold": "norm"})], [M], "heuristic", torch.bfloat16, dev)
+        rep = tune_projection_gemms([("gate_up", ws, K, {"silu_interleaved": True, "fold": "norm"})], [M], "heuristic", torch.bfloat16, dev)
         want = {4: {"skinny_linear", "skinny_linear_silu", "norm_linear", "ro_linear"},
                 48: {"skinny_linear", "skinny_linear_silu", "wstream_linear", "ro_linear"},
                 200: {"wstream_linear", "full_batch_linear", "g3_linear", "ro_linear"}}[M]
         assert want <= timed and not outside
+        r = rep[0]
+        if r.get("norm_used"):  # the plan that runs is the one that is reported
+            assert "norm" in r["kernel"] and r["best_us"] == r["norm_fused_us"] and r["skinny_used"]
     finally:
         ops.reset_gemm_plans()
