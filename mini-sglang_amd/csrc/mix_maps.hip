@@ -33,10 +33,14 @@ __global__ __launch_bounds__(256, 2) void maps_prompt_kernel(bf16_t* __restrict_
   int tok0 = 0;
   // The longest groups first, all of a group's heads before the next group: what starts last is short.  (A head's groups after another's: the
   // last head's longest groups start when half the work is done, and end long after the rest.  182 -> 151 us; window 1024,
-  // 8 heads on 4: 84 -> 78; 3 portions of 130 after 1000, 16 heads on 8: 56.7 -> 53.9.)
-  const int rep = H / G, hblocks = (rep + HB - 1) >> hb_log2, n_heads = G * hblocks;
-  const int index = (int)blockIdx.x / n_heads, hy = (int)blockIdx.x - index * n_heads;
-  const int b = find_group_by_keys(cu_q, seq_lens, B, QT, index, (int)gridDim.x / n_heads, &tok0);
+  // 8 heads on 4: 84 -> 78; 3 portions of 1500, 16 heads on 4: 100 -> 83.  Of 408 sizes of 1 - 8 portions, 8 and 16 heads on 2 and 4, 65 to 1000
+  // workgroups, 5 % faster on average; eight are 4 - 13 % slower, of 513 - 780 workgroups behind long prefixes, mostly with two heads' groups to an
+  // index: 5 of 850 after 650, 16 on 2: 109 -> 126.)  With key ranges, a few tens of groups and no rest to wait for, it is the other way round: 1
+  // portion of 300 after 2000, 8 heads on 4: 39.1 us, a group's heads together 42.3; 2 of 300 after 650 37.0 and 40.8.
+  const int rep = H / G, hblocks = (rep + HB - 1) >> hb_log2, n_heads = G * hblocks, n_groups = (int)gridDim.x / n_heads;
+  const int index = RANGES ? (int)blockIdx.x % n_groups : (int)blockIdx.x / n_heads;
+  const int hy = RANGES ? (int)blockIdx.x / n_groups : (int)blockIdx.x - index * n_heads;
+  const int b = find_group_by_keys(cu_q, seq_lens, B, QT, index, n_groups, &tok0);
   if (b < 0) return;
   const int kvh = hy / hblocks, h0 = kvh * rep + (hy - kvh * hblocks) * HB, h_end = (kvh + 1) * rep, z = blockIdx.z;
   const int first = cu_q[b], q_len = cu_q[b + 1] - first, start = seq_lens[b] - q_len;
