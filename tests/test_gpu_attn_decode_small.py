@@ -110,6 +110,27 @@ def test_small_decode_refusals(ops, dev):
                                   torch.empty(floats, dtype=torch.float32, device=dev), ranges, 1.0)
 
 
+@pytest.mark.parametrize("hq,hkv,d,width,most", [(16, 8, 128, 4096, 8), (16, 8, 128, 4128, 4), (40, 8, 128, 40960, 4), (10, 2, 128, 40960, 32), (5, 1, 128, 40960, 64),
+                                                 (32, 32, 128, 40960, 1), (18, 2, 128, 512, 0), (16, 8, 64, 512, 0)])
+def test_batches_that_take_the_small_kernel(dev, hq, hkv, d, width, most):
+    """The rule by requests x kv heads on both sides of its lines: a table of up to 4096 tokens, one or two kv heads, other heads than the kernel's."""
+    from types import SimpleNamespace
+
+    from mini_sglang_amd.attention import HipAttnBackend
+    from mini_sglang_amd.core import Context
+    from mini_sglang_amd.kvcache import create_kvcache_pool
+    from mini_sglang_amd.model import ModelConfig
+
+    m = ModelConfig(num_layers=1, num_qo_heads=hq, num_kv_heads=hkv, head_dim=d, hidden_size=256, vocab_size=64, intermediate_size=64)
+    ctx = Context(16)
+    ctx.page_table = torch.zeros((80, width), dtype=torch.int32, device=dev)
+    ctx.kv_cache = create_kvcache_pool(m, 2, 16, torch.bfloat16, dev)
+    backend = HipAttnBackend(m, ctx)
+    says = [b for b in range(1, 80) if backend.small_decode(SimpleNamespace(attn_metadata=SimpleNamespace(max_seqlen_q=1, batch=b)))]
+    assert says == list(range(1, most + 1))
+    assert not backend.small_decode(SimpleNamespace(attn_metadata=SimpleNamespace(max_seqlen_q=2, batch=1)))
+
+
 def test_replayed_batches_of_both_kernels_keep_their_plan(dev, monkeypatch):
     """An engine whose captured batch sizes lie on both sides of the rule: replays of either after the other, against eager runs."""
     from mini_sglang_amd import ops

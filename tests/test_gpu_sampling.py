@@ -410,3 +410,18 @@ def test_the_bound_of_candidates_reaches_low_temperatures(ops, dev, temperature)
 ])
 def test_draws_that_share_their_rows(ops, how, rows, vocab, shared):
     assert (ops.lib().msgl_sample_workspace_bytes(rows, vocab, how != "none", how == "k", how == "p") > 0) is shared
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,vocab", [(3, 65536), (64, 98304), (40, 151936), (1, 600_008), (70, 131080)])
+def test_unfiltered_draws_of_shared_rows_are_those_of_one_workgroup(ops, dev, dtype, rows, vocab):
+    """Rows that 16 to 2 workgroups share, more than 1024 chunks of 512 numbers among them, against the kernel with one workgroup a row (no workspace)."""
+    g = torch.Generator(device=dev).manual_seed(rows + vocab)
+    logits = (torch.randn((rows, vocab), generator=g, device=dev) * 2.5).to(dtype)
+    t = torch.tensor([(0.5, 1.0, 3.0, 0.02)[r % 4] for r in range(rows)], device=dev)
+    assert ops.lib().msgl_sample_workspace_bytes(rows, vocab, 0, 0, 0) > 0
+    want = torch.empty(rows, dtype=torch.int32, device=dev)
+    for off in range(0, 4000, 500):
+        ops.check(ops.lib().msgl_sample_from_logits(want.data_ptr(), logits.data_ptr(), t.data_ptr(), rows, vocab, logits.stride(0), ops._logits_dt(logits), 9, off,
+                                                    ops._stream()), "sample")
+        assert torch.equal(ops.sample_from_logits(logits, t, 9, off), want)
