@@ -80,7 +80,7 @@ def fill_metadata_host(h: np.ndarray, seqlens_q: np.ndarray, seqlens_k: np.ndarr
         h[4 * bs + 2:] = prefill_tile_order(seqlens_q, seqlens_k, tiles, q_tile)
 
 
-SMALL_DECODE_HEADS = 32  # (request, kv head) pairs up to which decode attention takes the small-batch kernel at any length
+SMALL_DECODE_HEADS = 32  # (request, kv head) pairs up to which decode attention takes the small-batch kernel whatever the table's width
 
 
 class HipAttnBackend:
@@ -129,10 +129,16 @@ class HipAttnBackend:
 
     def small_decode(self, batch: Any) -> bool:
         """Whether the batch's decode attention takes the kernel that does the new tokens' row work itself
-        (csrc/attn_decode_small.hip).  It and the join of its ranges against row work, planned kernel and merge, us a layer in a
-        captured step, 8 kv heads, bf16: 1 request 9.1 / 11.8 at 533 tokens and 16.7 / 68 at 8000, 4 requests 13.7 / 14.1 and
-        34 / 66; 8 requests 15.1 / 14.7 and 60 / 53: its requests are half lines, and it loses once the stream is long.  With 1 or
-        2 kv heads it is ahead up to 64 of them as well (2 x 32 at 2000 tokens: 24 / 27)."""
+        (csrc/attn_decode_small.hip), in place of row work, planned kernel and merge.  us of a step saved by it per layer, inside
+        captured steps of Qwen3-0.6B (28 layers, 16 heads on 8) | of six layers of a 14B model (40 on 8), bf16:
+          table of 40960 tokens   1 request of 533 4.8 | 8.8     4 of 533 2.0 | 5.2     8 of 533 1.8 | 4.7     5 of 8000 - | 1.1
+          just wide enough        4 of 533 6.6 | 9.9             8 of 533 2.5 | 5.7     8 of 2000 2.4 | 4.4    8 of 4000 1.5 | 1.3
+        Its requests are half lines, and it loses once the stream is long: 8 of 8000 - | -0.8, 8 of 16000 - | -23.  A captured step does
+        not know its lengths, so more than 32 (request, kv head) pairs take it only where the table ends at 4096 tokens.  At 4
+        requests it is ahead up to 12000 tokens (8000 - | 5.8, 12000 - | 2.3) and loses from 14000 on with three and more heads a kv
+        head (16000 30 | -1.7, 32000 - | -13.6, of some 250), which the shorter ones are worth.  With 1 or 2 kv heads it is ahead
+        up to 64 pairs at all lengths (a chain of attention alone, 10 on 2, 32 requests: 533 tokens 20.1 / 16.7, 16000 105.4 / 104.6;
+        5 on 1, 64: 533 20.1 / 16.6, 16000 107.0 / 101.6)."""
         md = batch.attn_metadata
         return md.max_seqlen_q == 1 and md.batch * self.kv_heads <= self._small_heads
 
@@ -151,7 +157,8 @@ class HipAttnBackend:
         return self._attend_small(q, k, v, layer_id, batch, q_norm_w=q_norm_w, k_norm_w=k_norm_w, eps=eps, positions=positions, cos_sin_cache=cos_sin)
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_id: int, batch: Any) -> torch.Tensor:
-        """Reference contract (fa.py:48-65): persist k, v at batch.out_loc, then attend."""
+        """Reference contract (fa.py:48-65): persist k, v at batch.out_loc, then attend.  A decode batch's out_loc is where its requests'
+        last table entries point, as the scheduler allocates them."""
         if self.small_decode(batch):
             q2, k2, v2 = (t.reshape(t.shape[0], -1) for t in (q, k, v))
             if (batch.out_loc.dtype == torch.int32 and batch.out_loc.is_contiguous() and {t.dtype for t in (q, k, v)} == {self.kvcache.dtype}

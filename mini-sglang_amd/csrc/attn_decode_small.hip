@@ -13,7 +13,9 @@
 //     LDS image and transposing reads, as in attn_decode.hip; the next tile is requested before the present one is used;
 //   * the queries are the second operand: column j < G is query head j, and column G carries the NEW KEY through the same norm and
 //     rotation.  The wave that owns the last tile puts that key into the tile's operand, reads the new value row where the
-//     projection left it, and stores both in the cache: nobody reads the cache row that is being written;
+//     projection left it, and stores both in the cache.  Nobody uses what the cache row holds that is being written: its value is
+//     never read, its key is by the owner (put aside for the new one), by lanes past the end of the last tile (their scores are
+//     masked) and by waves without a tile (which multiply nothing);
 //   * the eight waves' sums meet in LDS; a request of one range is finished there.
 // Same arithmetic as msgl_qk_norm_rope_store for the stored rows (same bits); fp32 partial sums as before.
 #include "attn_decode_tile.h"

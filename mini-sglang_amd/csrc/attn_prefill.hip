@@ -79,7 +79,9 @@ struct PrefillParams {
 // kv heads) XCDs with the same ones take turns down one list, the tiles in the order given (most keys first) with all their heads: every XCD
 // gets long tiles and short ones, and what starts last is short.  (Cut into eight stretches instead, the first XCDs of a list had all the long
 // tiles, or one kv head's short tiles came before the next one's long ones.  8 requests of 300 - 1300 tokens, 16 heads on 2: 69 -> 47 us; 4000
-// tokens, 10 on 2: 106 -> 88; 20 requests of 100 - 1024, 9 on 3: 56 -> 47, 24 on 12: 129 -> 126, 32 on 16: 156 -> 152.  8 kv heads: as before.)
+// tokens, 10 on 2: 106 -> 88; 20 requests of 100 - 1024, 9 on 3: 56 -> 47, 24 on 12: 129 -> 126, 32 on 16: 156 -> 152.  8 kv heads: as before.
+// Many requests of like length lose where an XCD's list has several kv heads, whose rows then pass through its L2 together: 20 of 90 - 170 tokens,
+// 24 on 12: 28 -> 30, after 3000 200 -> 213; 9 on 3: 14.8 -> 16.0.)
 // A launch of one workgroup per CU or less starts all of them at once: stretches of the list, which leave an XCD fewer requests' keys (6 requests of
 // 100 - 400 after 2500, 16 on 2: 63 us, in turns 65).
 struct PrefillJob {

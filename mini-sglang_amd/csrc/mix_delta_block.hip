@@ -18,8 +18,8 @@
 // all); the block kernel by memory (49 d + 512 floats a block and head written, and read again by the walk; values are read by the walk
 // itself).  The token loop was bound by one wave's serial walk: two passes over 128 registers a token, in three launches.
 // 4 requests of 1500 - 2548 tokens, 16 heads, d = dv = 128, decays per channel, us (blocks, walk): 4038 in the token loop; 389 (171, 219) with
-// (I + A)^-1 beta v solved and stored per value column, operands in rows of d and 32 columns a workgroup; 306 (100, 207) now.  One request
-// of 900 tokens, 8 heads: 100 -> 62.  Error against 64 bits 1.9e-7 -> 1.4e-7 -> 1.1e-7.
+// (I + A)^-1 beta v solved and stored per value column, operands in rows of d and 32 columns a workgroup; 306 (100, 207) as below, 277 (99,
+// 178) with the walks in order of length.  One request of 900 tokens, 8 heads: 100 -> 62.  Error against 64 bits 1.9e-7 -> 1.4e-7 -> 1.1e-7.
 #include <type_traits>
 
 #include "mix_common.h"
@@ -340,8 +340,8 @@ __device__ __forceinline__ WalkRequest walk_request(const int* __restrict__ cu_q
 // which load the next blocks' operands have no stores among their loads (with them the compiler waited for every load in flight in front of
 // each block), and no loads of its own, whose waits would be for the stores before them.
 // At most 128 registers, so that two workgroups share a CU: wave 4 goes to the SIMD of wave 0, and with more the second workgroup waited for
-// the first to end.  32 columns a workgroup read half as much and take 215 us for 207 (200 for 181 at 8 requests of 300 - 1000 tokens): one
-// chain's meeting is not hidden by another's products.
+// the first to end.  32 columns a workgroup read half as much and took 215 us for 207 (200 for 181 at 8 requests of 300 - 1000 tokens), both
+// without the order of the walks: one chain's meeting is not hidden by another's products.
 template <int D>
 __global__ __launch_bounds__(320, 4) void delta_walk_kernel(float* __restrict__ out, float* __restrict__ state, const float* __restrict__ scratch,
                                                             const float* __restrict__ qkv, const int* __restrict__ cu_q,

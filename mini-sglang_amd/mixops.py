@@ -382,9 +382,9 @@ def window_attn_splits(batch: int, total_q: int, window: int, max_keys: int) -> 
 
 def window_portion_splits(batch: int, total_q: int, window: int, max_keys: int, matrix: bool) -> int:
     """Key ranges where window_attn_splits gives one: a few short portions are some tens of token groups for 256 compute units, so their keys are
-    cut as well.  16-token groups on the matrix cores, from 128 keys a range (16 heads; 500 fresh tokens in 1 / 4 ranges 52 / 41 us, 100
-    decoded ones over 300 keys in 1 / 2 46 / 39, but 8 portions of 100 fresh ones 27 / 36); the plain kernel, whose every token walks all
-    heads, from 64 (fp32, 16 heads: 8 portions of 100 120 / 86 us, 20 tokens after 1000 862 / 128 in 8; 2 after 50 40 / 46).  A function of
+    cut as well.  16-token groups on the matrix cores, from 128 keys a range (16 heads on 4; 500 fresh tokens in 1 / 4 ranges 61 / 35 us, 1000
+    110 / 49, 20 after 1000 in 1 / 8 112 / 34, 100 decoded ones over 300 keys in 1 / 2 41 / 34, but 8 portions of 100 fresh ones 21 / 31); the
+    plain kernel, whose every token walks all heads, from 64 (fp32, 16 heads: 8 portions of 100 120 / 86 us, 20 tokens after 1000 862 / 128 in 8; 2 after 50 40 / 46).  A function of
     static sizes only, so a captured graph keeps its grid."""
     groups, keys = total_q // 16 + batch, min(window, max_keys) if window > 0 else max_keys
     return max(1, min(256 // groups, -(-keys // (128 if matrix else 64)), 8)) if 0 < groups <= 128 else 1
@@ -445,13 +445,15 @@ _DELTA_BLOCK_TOKENS = {(128, 0): (6, 8), (128, 1): (6, 6), (64, 0): (10, 28), (6
 
 
 def delta_in_blocks(batch: int, total_q: int, H: int, d: int, per_channel: bool, longest: Optional[int] = None) -> bool:
-    """Blocks of 16 tokens on the matrix instructions (two launches, 14 us however short the portions are, and more for every further request
-    and head), or token by token (a token of the longest portion: 2.2 us at d = 128, 4.4 with a decay per channel, 1.0 and 1.7 at d = 64).
-    Token loop / blocks in us on both sides of the line, requests x tokens, 16 heads of d = 128: 1 x 6 26 / 14.5; 16 x 6 29 / 34, 16 x 8 34 / 33,
-    64 x 6 65 / 90, 64 x 12 99 / 93; per channel 1 x 6 38 / 15, 64 x 6 92 / 90.  d = 64 (dv 128): 1 x 8 16.0 / 17.6, 1 x 12 20.0 / 18.5, 16 x 16
-    26 / 31, 40 x 16 39 / 56, 64 x 24 89 / 89; per channel 1 x 6 17.5 / 16.2, 16 x 8 23 / 28, 16 x 16 38 / 31, 64 x 12 68 / 69.  One long portion
-    among single tokens: 16 requests, one of 80 tokens, 196 us token by token and 47 in blocks; where the longest is not known, only many
-    tokens speak for one."""
+    """Blocks of 16 tokens on the matrix instructions (two launches, 12.5 us however short the portions are, and more for every further
+    request and head), or token by token (a token of the longest portion: 2.2 us at d = 128, 4.4 with a decay per channel, 1.0 and 1.7 at d = 64).
+    Token loop / blocks in us on both sides of the line, requests x tokens, 16 heads of d = 128: 1 x 4 20.6 / 12.5, 1 x 6 24.9 / 12.4; 16 x 6
+    27.9 / 29.4, 16 x 8 32.3 / 29.5; 64 x 6 60 / 78, 64 x 8 72 / 78, 64 x 12 95 / 78; per channel 1 x 4 28.7 / 12.7; 16 x 4 31.7 / 30.3, 16 x 6
+    41.4 / 30.4; 64 x 4 66 / 80, 64 x 6 88 / 80.  d = 64 (dv 128): 1 x 8 15.0 / 13.7, 1 x 12 19.0 / 13.8; 16 x 24 33.7 / 31.7, 16 x 48 62 / 38;
+    40 x 24 46 / 58, 40 x 48 83 / 68; per channel 1 x 4 13.1 / 12.3, 1 x 6 16.7 / 12.5; 16 x 12 29.8 / 24.9, 16 x 16 36.8 / 25.1; 40 x 16 46.0 / 46.5.
+    (The line was set by slower blocks: single requests of 2 - 4 tokens and some decoded batches of few would gain from a lower one.)  One long
+    portion among single tokens: 16 requests, one of 80 tokens, 196 us token by token and 47 in blocks before these got faster; where the
+    longest is not known, only many tokens speak for one."""
     if total_q >= _DELTA_BLOCK_TOKENS.get((d, bool(per_channel)), (6, 12))[batch * H > 128] * batch:  # every further (request, head) is a walk of its own
         return True
     return longest >= 40 if longest is not None else batch * H > 256 and total_q - batch >= 256
