@@ -68,7 +68,7 @@ struct PrefillParams {
   uint16_t* out;
   int64_t pt_stride, q_stride, kv_stride_tok, kv_stride_head, out_stride;
   int batch, hq, group;
-  int share, per;  // XCDs that share their kv heads, kv heads of each
+  int share_log2, per;  // XCDs that share their kv heads, kv heads of each
   int stretch;     // workgroups of an XCD where each takes a stretch of the list, or 0
   int ranges, run;  // key ranges, and tiles of each (the last one: what is left)
   float *part_o, *part_ml;
@@ -88,8 +88,8 @@ struct PrefillJob {
   int kvh, hq, tile;  // tile < 0: none left
 };
 __device__ __forceinline__ PrefillJob prefill_job(const PrefillParams& p, int total_tiles) {
-  const int xcd = (int)(blockIdx.x & 7), list = xcd / p.share, seat = xcd - list * p.share, n = (int)(blockIdx.x >> 3);
-  const int u = p.stretch ? seat * p.stretch + n : n * p.share + seat;
+  const int xcd = (int)(blockIdx.x & 7), list = xcd >> p.share_log2, seat = xcd - (list << p.share_log2), n = (int)(blockIdx.x >> 3);
+  const int u = p.stretch ? seat * p.stretch + n : (n << p.share_log2) + seat;
   const int each = p.group * p.per, ti = u / each, r = u - ti * each, sub = r / p.group;
   PrefillJob j;
   j.kvh = list * p.per + sub;
@@ -833,10 +833,10 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   p.hq = num_q_heads;
   p.group = num_q_heads / num_kv_heads;
   p.per = num_kv_heads;
-  p.share = 8;
-  while (p.share > 1 && p.per % 2 == 0) {
+  p.share_log2 = 3;
+  while (p.share_log2 > 0 && p.per % 2 == 0) {
     p.per /= 2;
-    p.share /= 2;
+    --p.share_log2;
   }
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -847,7 +847,7 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   if (impl == 0) impl = 4;  // the DMA-staged kernel; impl 2 keeps its predecessor callable (A/B timing, cross-check in tests)
   const int64_t total = (int64_t)total_tiles * num_q_heads;
   MSGL_REQUIRE(total < (1ll << 30), "attn_prefill: %lld workgroups", (long long)total);
-  const int even = (int)(((int64_t)total_tiles * p.group * p.per + p.share - 1) / p.share);
+  const int even = (int)(((int64_t)total_tiles * p.group * p.per + (1 << p.share_log2) - 1) >> p.share_log2);
   p.stretch = ranges == 1 && total <= 256 ? even : 0;
   const unsigned blocks = (unsigned)even * 8;
   if (ranges > 1) {
