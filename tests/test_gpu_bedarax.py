@@ -256,6 +256,36 @@ def test_window_matrix_cores(dev, H, G, d, dv, splits):
         assert bool((diff <= 2.0 ** -8 * ref.abs() + 2.0 ** -14 * ref.abs().max()).all()), (window, float(diff.max()))
 
 
+@pytest.mark.parametrize("splits", [1, 2], ids=["one-range", "two-ranges"])
+@pytest.mark.parametrize("step", [0.02, 0.3, 3.0])
+@pytest.mark.parametrize("H,G,shift", [(16, 4, 0), (16, 4, 3), (8, 2, 0)], ids=["16", "16-unaligned", "8"])
+def test_window_rising_scores(dev, H, G, shift, step, splits):
+    """Scores that rise by `step` a key, so that every key is a new maximum and the kernel's reference lags behind by less and by more than
+    it may; queries at an address that 16-byte loads may not read.  Against float64; bound as in test_window_matrix_cores."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(H)
+    d, c, n = 128, 61, 40
+    k, v = torch.randn(n + c, G, d, generator=g) * 0.1, torch.randn(n + c, G, d, generator=g).bfloat16()
+    k[..., 0] = torch.arange(n + c)[:, None] * step
+    k = k.bfloat16()
+    src = torch.randn(n, H * d + H, generator=g)
+    src[:, : H * d].view(n, H, d)[..., 0] = 1.0
+    src, talk = src.bfloat16(), torch.eye(H)
+    q = torch.cat([torch.zeros(c, H, d, dtype=torch.float64), src[:, : H * d].double().view(n, H, d)])
+    gate = torch.cat([torch.zeros(c, H, dtype=torch.float64), src[:, H * d:].double()])
+    ref = _window_reference(q, k.double(), v.double(), gate, talk.double(), 1.0, 0, H // G)[c:].reshape(n, -1)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    room = torch.empty(src.numel() + shift, dtype=torch.bfloat16, device=dev)
+    q_dev = room[shift:].view(src.shape)
+    q_dev.copy_(src)
+    out = torch.empty((n, H * d), dtype=torch.bfloat16, device=dev)
+    mixops.window_attn(out, q_dev, H * d, k.view(n + c, -1).to(dev), v.view(n + c, -1).to(dev), torch.arange(n + c, dtype=torch.int32, device=dev)[None], i32([0]),
+                       i32([n + c]), i32([0, n]), 1, H, G, d, d, 0, 1.0, talk.to(dev), splits=splits)
+    diff = (out.double().cpu() - ref).abs()
+    assert bool((diff <= 2.0 ** -8 * ref.abs() + 2.0 ** -14 * ref.abs().max()).all()), float(diff.max())
+
+
 @pytest.mark.parametrize("B", [64, 65, 150])
 @pytest.mark.parametrize("splits", [1, 3])
 @pytest.mark.parametrize("most", [1, 40], ids=["decode", "portions"])
