@@ -860,8 +860,9 @@ __global__ __launch_bounds__(kRowThreads) void sample_logits_kernel(int* __restr
 //                the copy of the rows
 // Thresholds, masses and picks are those of one workgroup (integer sums over the same numbers); a threshold that is not among the candidates
 // (ties across the bound, top-k above 1024) falls to draw_from_row, as there.
-// Bound: the launches' ends and starts and each one's chain of a few dependent loads and barriers (6, 14, 10 us of 32 at 64 x 151936 with top-k, where
-// the reads take 8 and the exponentials 2).  us a draw, one workgroup per row -> shared: see split_of.
+// Bound: the launches' ends and starts and each one's chain of a few dependent loads and barriers (5.5, 12, 10 us of 27 at 64 x 151936 with top-k, where
+// the reads take 8 and the exponentials 2; it was 31 with a tile of split_sum asked for at a time, divisions and dependent scalar loads in front of the first
+// load and a barrier more a tile).  us a draw, one workgroup per row -> shared: see split_of.
 // ------------------------------------------------------------------------------------------
 constexpr int kMaxChunks = kRowThreads;
 constexpr int64_t kMostPerGroup = 1 << 17;       // numbers of a row to one workgroup
@@ -940,10 +941,11 @@ __global__ __launch_bounds__(kRowThreads, 8) void split_max_kernel(SplitScratch 
   using E = std::conditional_t<DT == MSGL_F32, uint32_t, uint16_t>;
   constexpr int kPer = 16 / sizeof(E);
   const int tid = threadIdx.x;
-  const int64_t r = blockIdx.x / split;
+  const int log_split = __builtin_ctz(split);  // a power of two; divisions in front of the first load are time
+  const int64_t r = blockIdx.x >> log_split;
   const int g = (int)blockIdx.x - (int)r * split;
   const char* row = logits + r * row_stride_bytes;
-  const int64_t per = ((vocab + split - 1) / split + 7) & ~7ll;
+  const int64_t per = (((vocab + split - 1) >> log_split) + 7) & ~7ll;
   const int64_t lo = min(vocab, g * per), hi = min(vocab, lo + per);
   float mx = -INFINITY;
   if constexpr (VEC) {
@@ -975,52 +977,64 @@ __global__ __launch_bounds__(kRowThreads, 8) void split_max_kernel(SplitScratch 
     }
   }
   for (int d = 1; d < split; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));  // one maximum per `split` neighbours
-  if (tid % split == 0) sc.top[r * kRowThreads + g * (kRowThreads / split) + tid / split] = mx;
+  if ((tid & (split - 1)) == 0) sc.top[r * kRowThreads + g * (kRowThreads >> log_split) + (tid >> log_split)] = mx;
 }
 
 // MASS: mass per bin of the weights; else the list of candidates
 template <int DT, bool VEC, bool MASS>
-__global__ __launch_bounds__(kRowThreads, VEC ? 8 : 4) void split_sum_kernel(SplitScratch sc, const char* __restrict__ logits, const float* __restrict__ temperatures,
+__global__ __launch_bounds__(kRowThreads, VEC && MASS ? 8 : 4) void split_sum_kernel(SplitScratch sc, const char* __restrict__ logits, const float* __restrict__ temperatures,
                                                                    const int* __restrict__ top_k, const float* __restrict__ top_p, int64_t vocab,
-                                                                   int64_t row_stride_bytes, int split) {
-  __shared__ __attribute__((aligned(16))) float tile[kTile];
+                                                                   int64_t row_stride_bytes, int split, char* __restrict__ kept, float* __restrict__ kept_t) {
+  using E = std::conditional_t<DT == MSGL_F32, float, uint16_t>;
+  __shared__ __attribute__((aligned(16))) float tiles[2][kTile];  // one is summed while the next is filled
   __shared__ uint32_t pool[MASS ? kOctaves * 64 : 1];  // weights per bin, each to 15 bits: no more than kMostPerGroup of them go in
   __shared__ __attribute__((aligned(16))) uint32_t hist[MASS ? 4 : kRowThreads];
   __shared__ float lds_f[kRowThreads / 64];
   __shared__ uint32_t s_bound;
   __shared__ int s_n;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int64_t r = blockIdx.x / split;
+  const int log_split = __builtin_ctz(split);  // a power of two; divisions in front of the first load are time
+  const int64_t r = blockIdx.x >> log_split;
   const int g = (int)blockIdx.x - (int)r * split;
   const char* row = logits + r * row_stride_bytes;
-  const int cols = kRowThreads / split, high = kTile / cols;  // columns of this workgroup, rows of 1024 per tile
-  const float pp = top_p ? top_p[r] : 1.0f;
+  const int cols = kRowThreads >> log_split, high = kTile / kRowThreads << log_split;  // columns of this workgroup, rows of 1024 per tile
+  const float top = sc.top[r * kRowThreads + tid];  // in front of the numbers: they come back in the order of the requests
 
   // eight numbers per thread and tile: of one row of 1024 where they can be loaded at once, else of eight rows
-  const int at_row = VEC ? tid / (cols / 8) : tid / cols, at_col = VEC ? tid % (cols / 8) * 8 : tid % cols;
+  const int log_cols = 10 - log_split;
+  static_assert(kRowThreads == 1 << 10, "columns");
+  const int at_row = tid >> (VEC ? log_cols - 3 : log_cols), at_col = VEC ? (tid & ((cols >> 3) - 1)) * 8 : tid & (cols - 1);
   auto slot = [&](int e) { return VEC ? at_row * cols + at_col + e : (at_row + e * (high / 8)) * cols + at_col; };
   const uint32_t width = (uint32_t)vocab, step = kTile * split;  // (a sum of two of them fits 32 bits)
   auto index = [&](uint32_t base, int e) { return base + (VEC ? at_row : at_row + e * (high / 8)) * kRowThreads + g * cols + at_col + (VEC ? e : 0); };
-  auto load = [&](uint32_t base, float (&x)[8]) {
-    if (VEC && index(base, 0) + 8 <= width) {
-      load_logits8<DT>(row, index(base, 0), x);
+  // Several tiles are asked for ahead, all that a row of 151936 has on four workgroups: with one, a tile took a loaded memory's latency.
+  constexpr int kDeep = !VEC ? 1 : MASS ? 2 : DT == MSGL_F32 ? 3 : 5;
+  struct alignas(16) Eight {
+    E e[8];
+  };
+  Eight raw[kDeep];
+  auto load = [&](uint32_t base, Eight& x) __attribute__((always_inline)) {
+    if (VEC && (base + step <= width || index(base, 0) + 8 <= width)) {
+#pragma unroll
+      for (int h = 0; h < (int)sizeof(Eight) / 16; ++h) reinterpret_cast<U4*>(&x)[h] = ldg16(reinterpret_cast<const char*>(reinterpret_cast<const E*>(row) + index(base, 0)) + 16 * h);
     } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = index(base, e) < width ? load_logit<DT>(row, index(base, e)) : 0.f;
+      for (int e = 0; e < 8; ++e) x.e[e] = index(base, e) < width ? reinterpret_cast<const E*>(row)[index(base, e)] : (E)0;
     }
   };
-  float x[8];
-  load(0, x);
+#pragma unroll
+  for (int u = 0; u < kDeep; ++u)
+    if (u == 0 || u * step < width) load(u * step, raw[u]);
+  const float pp = top_p ? top_p[r] : 1.0f, temperature = temperatures[r];
+  const int64_t kk = !MASS && top_k ? (int64_t)top_k[r] : 0;
 
-  const float top = sc.top[r * kRowThreads + tid];
-  const float mx = block_reduce_max(top, lds_f), k = 1.0f / temperatures[r] * 1.4426950408889634f;
+  const float mx = block_reduce_max(top, lds_f), k = 1.0f / temperature * 1.4426950408889634f;
   const bool mass = MASS && pp < 1.0f;
   uint32_t list_bits = kNoDigit;
   if constexpr (MASS) {
     if (mass)
       for (int b = tid; b < kOctaves * 64; b += kRowThreads) pool[b] = 0u;
   } else {
-    const int64_t kk = top_k[r];
     const bool has_k = kk >= 1 && kk < vocab, by_count = has_k && kk <= kListTopK;
     uint32_t floor_bits = 0u;
     if (by_count || (!has_k && pp < 1.0f)) {
@@ -1031,18 +1045,32 @@ __global__ __launch_bounds__(kRowThreads, VEC ? 8 : 4) void split_sum_kernel(Spl
     if (tid == 0) s_n = list_bits == kNoDigit ? kList + 1 : 0;
     if (g == 0 && tid == 0) sc.head[r].floor_bits = floor_bits;
   }
-  if (g == 0 && tid == 0) sc.head[r].mx = mx;
+  if (g == 0 && tid == 0) {
+    sc.head[r].mx = mx;
+    if (MASS && kept) kept_t[r] = temperature;
+  }
   __syncthreads();
 
   u64* list = sc.list + (r * split + g) * kPart;
   float sum = 0.f;
-  for (uint32_t base = 0; base < width; base += step) {
+  int image = 0;
+  auto one_tile = [&](uint32_t base, Eight& held) __attribute__((always_inline)) {
+    float* tile = tiles[image];
+    image ^= 1;
     float w[8], most = 0.f;
+    if (MASS && kept && index(base, 0) + 8 <= width) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      w[e] = index(base, e) < width ? __builtin_amdgcn_exp2f((x[e] - mx) * k) : 0.f;  // a zero more leaves a sum as it is
-      most = fmaxf(most, w[e]);
+      for (int h = 0; h < (int)sizeof(Eight) / 16; ++h)
+        reinterpret_cast<U4*>(kept + ((int64_t)r * vocab + index(base, 0)) * sizeof(E))[h] = reinterpret_cast<const U4*>(&held)[h];
     }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = __builtin_amdgcn_exp2f((load_logit<DT>(held.e, e) - mx) * k);
+    if (base + step > width) {  // (the row's last tile)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w[e] = index(base, e) < width ? w[e] : 0.f;  // a zero more leaves a sum as it is
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) most = fmaxf(most, w[e]);
     if constexpr (VEC) {
       *reinterpret_cast<float4*>(tile + slot(0)) = float4{w[0], w[1], w[2], w[3]};
       *reinterpret_cast<float4*>(tile + slot(4)) = float4{w[4], w[5], w[6], w[7]};
@@ -1050,7 +1078,7 @@ __global__ __launch_bounds__(kRowThreads, VEC ? 8 : 4) void split_sum_kernel(Spl
 #pragma unroll
       for (int e = 0; e < 8; ++e) tile[slot(e)] = w[e];
     }
-    if (base + step < width) load(base + step, x);
+    if (base + kDeep * step < width) load(base + kDeep * step, held);
     if constexpr (MASS) {
       if (mass) {
 #pragma unroll
@@ -1077,7 +1105,11 @@ __global__ __launch_bounds__(kRowThreads, VEC ? 8 : 4) void split_sum_kernel(Spl
 #pragma unroll 16
       for (int q = 0; q < high; ++q) sum += tile[q * cols + tid];
     }
-    __syncthreads();
+  };
+  for (uint32_t base = 0; base < width; base += kDeep * step) {
+#pragma unroll
+    for (int u = 0; u < kDeep; ++u)
+      if (base + u * step < width) one_tile(base + u * step, raw[u]);
   }
   if (tid < cols) sc.sum[r * kRowThreads + g * cols + tid] = sum;
   if constexpr (MASS) {
@@ -1103,10 +1135,11 @@ __global__ __launch_bounds__(kRowThreads, 8) void split_mass_kernel(SplitScratch
   __shared__ float lds_f[kRowThreads / 64];
   __shared__ int s_n, s_bin[2];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int64_t r = blockIdx.x / split;
+  const int log_split = __builtin_ctz(split);  // a power of two; divisions in front of the first load are time
+  const int64_t r = blockIdx.x >> log_split;
   const int g = (int)blockIdx.x - (int)r * split;
   const char* row = logits + r * row_stride_bytes;
-  const int64_t chunks = (vocab + chunk - 1) / chunk;
+  const int64_t chunks = (vocab + chunk - 1) >> __builtin_ctzll(chunk);  // a power of two
   const int64_t c0 = (int64_t)(tid >> 6) * split + g;
   float x[8];
   if constexpr (!FILTER) Piece<DT, VEC>::load(row, c0 * chunk, lane, min(vocab, (c0 + 1) * chunk), x);
@@ -1272,19 +1305,19 @@ __global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc
   const int64_t r = blockIdx.x;
   const void* row = logits + r * row_stride_bytes;
   if constexpr (HOW == kPickAny) {
-    const int64_t chunks = (vocab + chunk - 1) / chunk;
+    const int64_t chunks = (vocab + chunk - 1) >> __builtin_ctzll(chunk);  // a power of two
     const u64 mine = tid < chunks ? sc.chunk[r * kMaxChunks + tid] : 0ull;
     const float mx = block_reduce_max(sc.top[r * kRowThreads + tid], sh.lds_f), k = 1.4426950408889634f / temperatures[r];
     draw_from_chunks(sh, out, mine, vocab, chunk, seed, offset, [&](int64_t i) { return exp_mass(load_logit<DT>(row, i), mx, k); });
     return;
   }
+  // everything that is asked for by the row alone at once, then the list, then the sums' meeting
+  const int lane = tid & 63, count = lane < split ? sc.count[r * split + lane] : 0;
   const SplitHead head = sc.head[r];
+  const float sum = sc.sum[r * kRowThreads + tid], temperature = temperatures[r];
   const int64_t kk = top_k ? (int64_t)top_k[r] : vocab;
   const float pp = top_p ? top_p[r] : 1.0f;
-  LogitRow<DT> src{row, head.mx, 1.0f / temperatures[r] * 1.4426950408889634f, 1.0f};
-  src.inv = 1.0f / block_reduce_sum(sc.sum[r * kRowThreads + tid], sh.lds_f);
   // the workgroups' lists one behind the other (their lengths in the lanes, the places before each in `upto`)
-  const int lane = tid & 63, count = lane < split ? sc.count[r * split + lane] : 0;
   int upto = min(count, kPart + kList);
 #pragma unroll
   for (int d = 1; d < 16; d <<= 1) {
@@ -1306,6 +1339,8 @@ __global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc
     sh.s_index[c] = (int)(uint32_t)e;
     sh.h_cnt[c] = (uint32_t)(e >> 32);
   }
+  LogitRow<DT> src{row, head.mx, 1.0f / temperature * 1.4426950408889634f, 1.0f};
+  src.inv = 1.0f / block_reduce_sum(sum, sh.lds_f);
   if (tid == 0) sh.s_pick = -1;
   u64 kept_mass = kNoMass;
   if constexpr (HOW == kPickList) {
@@ -1313,7 +1348,7 @@ __global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc
     __syncthreads();
     if (listed && draw_from_list(src, sh, out, n, head.floor_bits, by_count, kk, pp, vocab, seed, offset, kept_mass)) return;
   } else {
-    const int64_t chunks = (vocab + chunk - 1) / chunk;
+    const int64_t chunks = (vocab + chunk - 1) >> __builtin_ctzll(chunk);  // a power of two
     u64 mine = tid < chunks ? sc.chunk[r * kMaxChunks + tid] : 0ull;
     uint32_t thr_bits = 0u;
     bool found = !(pp < 1.0f);
@@ -1374,7 +1409,7 @@ __global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc
         __syncthreads();
         for (int c = tid; c < n; c += kRowThreads) {
           const float p = src.prob(__uint_as_float(sh.h_cnt[c]));
-          if (__float_as_uint(p) >= thr_bits) atomicAdd(&sh.h_mass[sh.s_index[c] / chunk], fixed_mass(p));
+          if (__float_as_uint(p) >= thr_bits) atomicAdd(&sh.h_mass[sh.s_index[c] >> __builtin_ctzll(chunk)], fixed_mass(p));
         }
         __syncthreads();
         mine += sh.h_mass[tid];
@@ -1494,6 +1529,11 @@ extern "C" int64_t msgl_sample_workspace_bytes(int64_t rows, int64_t vocab, int 
 template <int DT, bool VEC>
 static void launch_split(const SplitScratch& sc, int32_t* out, char* kept, float* kept_t, const char* logits, const float* temperatures, const int32_t* top_k,
                          const float* top_p, bool filtered, int64_t rows, int64_t vocab, int64_t stride_bytes, int split, u64 seed, u64 offset, hipStream_t s) {
+  // The copy of the rows: beside the picks, on the compute units that these leave idle; where they leave few, by the sums' kernel, which has the
+  // rows in registers (us: 202 x 151936, top-p alone 101 beside the picks, 92 with the sums; 105 x 120687 the same; 64 x 151936 with top-k 28, 29)
+  const bool here = VEC && filtered && !top_k && kept && rows > 128 && vocab % 8 == 0 && aligned16(kept);
+  char* const kept_sum = here ? kept : nullptr;
+  if (here) kept = nullptr;
   const int64_t copies = kept ? rows * ((vocab + kCopySlice - 1) / kCopySlice) : 0;
   const dim3 many((unsigned)(rows * split)), picks((unsigned)(rows + copies)), b(kRowThreads);
   const int64_t chunk = split_chunk(vocab);
@@ -1503,11 +1543,11 @@ static void launch_split(const SplitScratch& sc, int32_t* out, char* kept, float
     split_pick_kernel<DT, kPickAny><<<picks, b, 0, s>>>(sc, out, logits, temperatures, top_k, top_p, vocab, stride_bytes, split, chunk, seed, offset,
                                                         (int)rows, kept, kept_t);
   } else if (top_k) {
-    split_sum_kernel<DT, VEC, false><<<many, b, 0, s>>>(sc, logits, temperatures, top_k, top_p, vocab, stride_bytes, split);
+    split_sum_kernel<DT, VEC, false><<<many, b, 0, s>>>(sc, logits, temperatures, top_k, top_p, vocab, stride_bytes, split, kept_sum, kept_t);
     split_pick_kernel<DT, kPickList><<<picks, b, 0, s>>>(sc, out, logits, temperatures, top_k, top_p, vocab, stride_bytes, split, chunk, seed, offset,
                                                          (int)rows, kept, kept_t);
   } else {
-    split_sum_kernel<DT, VEC, true><<<many, b, 0, s>>>(sc, logits, temperatures, top_k, top_p, vocab, stride_bytes, split);
+    split_sum_kernel<DT, VEC, true><<<many, b, 0, s>>>(sc, logits, temperatures, top_k, top_p, vocab, stride_bytes, split, kept_sum, kept_t);
     split_mass_kernel<DT, VEC, true><<<many, b, 0, s>>>(sc, logits, temperatures, top_p, vocab, stride_bytes, split, chunk);
     split_pick_kernel<DT, kPickMass><<<picks, b, 0, s>>>(sc, out, logits, temperatures, top_k, top_p, vocab, stride_bytes, split, chunk, seed, offset,
                                                          (int)rows, kept, kept_t);
