@@ -357,6 +357,28 @@ def test_a_row_shared_by_workgroups_draws_the_same(ops, dev, dtype, rows, vocab)
         assert got == [int(ops.sample_from_logits(logits[r: r + 1], t[r: r + 1], 5, 300 + r)) for r in range(rows)]
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,vocab,gap", [(129, 32000, 0), (129, 32004, 4), (128, 32000, 0), (130, 40961, 7), (20, 163848, 0)])
+def test_copies_of_shared_rows(ops, dev, dtype, rows, vocab, gap):
+    """The rows and temperatures that a draw leaves for later ones are its inputs, bit for bit: above 128 rows from the kernel that sums them, else (and where
+    16 bytes cannot be stored) beside the picks; rows of more tiles than are asked for ahead."""
+    g = torch.Generator(device=dev).manual_seed(rows)
+    logits = (torch.randn((rows, vocab + gap), generator=g, device=dev) * 2.5).to(dtype)[:, :vocab]
+    t = torch.rand(rows, generator=g, device=dev) + 0.5
+    p = torch.full((rows,), 0.9, device=dev)
+    k = torch.full((rows,), 30, dtype=torch.int32, device=dev)
+    for kk, pp in ((None, p), (k, p)):
+        n = ops.lib().msgl_sample_workspace_bytes(rows, vocab, 1, kk is not None, 1)
+        ws = torch.empty(max(n, 16), dtype=torch.uint8, device=dev)
+        out = torch.empty(rows, dtype=torch.int32, device=dev)
+        kept, kept_t = torch.full((rows * vocab + 64,), 7.0, dtype=dtype, device=dev), torch.zeros(rows, device=dev)
+        ops.check(ops.lib().msgl_sample_filtered_logits_ws(
+            out.data_ptr(), kept.data_ptr(), kept_t.data_ptr(), logits.data_ptr(), t.data_ptr(), None if kk is None else kk.data_ptr(), pp.data_ptr(), rows, vocab,
+            logits.stride(0), ops._logits_dt(logits), 3, 0, ws.data_ptr() if n else None, n, ops._stream()), "sample")
+        assert bool((kept[: rows * vocab].view(rows, vocab) == logits).all()) and bool((kept[rows * vocab:] == 7).all()) and bool((kept_t == t).all())
+        assert out.tolist() == ops.sample_top_k_top_p(ops.softmax_temperature(logits, t), kk, pp, 3, 0).tolist()
+
+
 def _draw_with_workspace(ops, dev, logits, t, k, p):
     """A shared-row draw with a workspace to look into: its first parts are 16 bytes a row (maximum, candidates' bound, ..) and 1024 maxima a row."""
     rows, vocab = logits.shape
