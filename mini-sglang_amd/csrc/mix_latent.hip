@@ -6,11 +6,12 @@
 //   latent_join_kernel    adds up the key ranges of either
 //
 // Both: S^T = K Q^T and O^T += V^T P^T, so that a lane ends the first product with scores of ONE query row and starts the second with
-// them; the rows come to LDS by DMA (no staging registers), 16 bytes of padding per row carried along as one more piece, so that 8 rows'
+// them; the rows come to LDS by DMA (no staging registers), padded (decode: 16 bytes carried along as one more piece) so that 8 rows'
 // 16-byte reads and 4 rows' transposing reads both touch all banks once.  A row's sum is of the fp32 weights.  The reference maximum
 // follows every new maximum: the largest weight then is 1, exact in bf16 (letting it lag by up to 2^8 saves 2 % of the time and adds a
 // tenth to the error).
 #include <algorithm>
+#include <type_traits>
 
 #include "mix_common.h"
 
@@ -48,16 +49,18 @@ struct LatentRow {
 };
 
 // ---------------------------------------------------------------------------------------------------------------- portions
-// What bounds it: both products on the matrix cores (2 (DK + DV) flops a pair and head) and, equally, the LDS reads that feed them: a
-// 32 x 32 x 16 product of 32 cycles takes 1 KB, four SIMDs 128 B a cycle, all that LDS gives.  So a row set has to be 32 rows (with 16
-// the same reads feed half the products), and 32 rows x (DK of Q + DV of O) are 400 registers: two waves share a row set.  Each holds
-// half of Q's columns and half of O's, and their partial scores meet in LDS once a tile (a sixth of the LDS traffic).  (One wave per row set:
-// the scores and O together pass the 256 accumulators.)  8 waves, 128 rows, 32-key tiles in three LDS images.  A SIMD has two waves, w and
-// w + 4, and they take turns: while waves 0 - 3 turn tile t's scores into weights, waves 4 - 7 run the products of tile t - 1's values and
-// tile t's scores; after a barrier the roles change.  So the matrix cores have work in both halves, and each half's barrier serves the
-// meeting of the scores, the images' arrival and their release.
-// 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1535 -> 414 us (714 TFLOP/s), of it 115 us that the queries' and outputs' 563 MB
-// take to come and go at 4.9 TB/s, hardly overlapped: a workgroup fills its CU and starts and ends with them.
+// What bounds it: both products on the matrix cores (2 (DK + DV) flops a pair and head, 2176 cycles a SIMD and tile at 512 + 64), the vector work
+// beside them (O's rescaling when a maximum moves is half of it; a product of 32 cycles keeps the vector unit for 8) and the LDS reads that feed
+// them: a 32 x 32 x 16 product takes 1 KB.  So a row set has to be 32 rows (with 16 the same reads feed half the products), and 32 rows x (DK of Q +
+// DV of O) are 400 registers: two waves share a row set, on one SIMD.  The score wave holds Q and a quarter of O: it makes a tile's scores and weights and
+// adds its quarter; the value wave, one tile behind, holds three quarters of O and takes the weights and the factor of the maximum's move from LDS.
+// Each thus has registers for fragments read three products ahead, the scores meet nowhere and a weight is made once; one barrier a tile.
+// (Both holding half of Q and half of O, scores meeting in LDS, two barriers a tile: fragments one product ahead, 5150 cycles a tile of 32 keys, now 3900.
+// Twelve waves, one of scores and two of values a row set: 168 registers do not hold a third of O's accumulators and a second place where ways meet.)
+// Value waves fetch the rows: a DMA without addresses of its own in a lane's registers, and the score waves' reads wait for nothing but themselves.
+// 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1535 us -> 408 -> 351 us (840 TFLOP/s), of it some 60 us that a workgroup's start and end
+// take (queries and outputs, 563 MB at 4.9 TB/s; a workgroup fills its CU), 50 us the rows' way to LDS, 30 us the rescaling.  2 of 2253 tokens, 8 heads
+// 178 -> 139; 6 of 50 - 353 38 -> 33; 4 of 470, 256 + 64: 35 -> 32; 5 of 23 - 225, 8 heads 29.0 -> 29.4, the largest loss seen.
 template <int DK, int DV>
 __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
                                                                const float* __restrict__ q_abs, const bf16_t* __restrict__ cache,
@@ -65,209 +68,124 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
                                                                const int* __restrict__ req_rows, const int* __restrict__ seq_lens,
                                                                const int* __restrict__ cu_q, int B, int H, float scale, int QT, int HB, int splits,
                                                                const float* __restrict__ sink) {
-  constexpr int NKS = DK / 32, NVT = DV / 64;  // this wave's halves: 16-wide steps of the first product, 32-column tiles of the second
-  constexpr int ROW = LatentRow<DK>::bytes, PCS = LatentRow<DK>::pieces, KT = 32;
-  constexpr int AHEAD = 1, VAHEAD = 3;  // fragments are read so many products before their use (2 in the first: a Q fragment spills, 423 us for 414)
-  constexpr int NI = (KT * PCS + 63) / 64, IMAGE = NI * 1024, NDMA = (NI + 7) / 8;  // DMA instructions of a tile; of a wave at most
-  // three objects: the compiler then knows that a tile's reads do not meet a later tile's DMA
+  static_assert(DK - DV == 64, "the rotated entries' image");
+  constexpr int NKS = DK / 16, NA = DV / 16, KT = 32;       // 16-wide steps of the first product, those over the latent entries
+  constexpr int NVS = DV / 128, NVV = 3 * NVS;               // 32-column tiles of O in a score wave (the last ones), in a value wave
+  // A tile's rows in LDS: the latent entries with 48 bytes of padding (16 rows' 16-byte reads touch all banks once, and so do the 4 x 32 bytes of a
+  // transposing read), and behind them the rotated entries, 128 bytes a row, a row's pieces in places changed by its number.
+  constexpr int ROW = DV * 2 + 48, TAIL = KT * ROW, IMAGE = TAIL + KT * 128;
+  constexpr int NL = DV == 512 ? 7 : 0, NQ = NKS - NL;  // query fragments in LDS, in registers
+  // objects of their own: the compiler then knows that a tile's reads do not meet a later tile's DMA
   __shared__ __attribute__((aligned(1024))) char img0[IMAGE], img1[IMAGE], img2[IMAGE];
-  __shared__ __attribute__((aligned(16))) f32x4_t meet[8][4][64];  // [wave][four scores][lane]
-  __shared__ int s_slot[4][KT];
+  __shared__ __attribute__((aligned(16))) f32x4_t s_p[2][4][2][64];  // weights [tile & 1][row set][16 keys][lane]
+  __shared__ __attribute__((aligned(16))) f32x4_t s_q[4][NL ? NL : 1][64];
+  __shared__ float s_alpha[2][4][32];
+  __shared__ float2 s_ml[4][32];
+  __shared__ __attribute__((aligned(16))) int s_slot[4][KT];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), hi = lane >> 5;
-  const int rows0 = (wave >> 1) * 32, half = wave & 1;
+  const int set = wave & 3, role = wave >> 2, rows0 = set * 32;
   int tok0 = 0;
   const int b = find_group_by_keys(cu_q, seq_lens, B, QT, (int)blockIdx.x, (int)gridDim.x, &tok0);
   if (b < 0) return;
   const int h0 = blockIdx.y * HB, z = blockIdx.z;
   const int first = cu_q[b], q_len = cu_q[b + 1] - first, start = seq_lens[b] - q_len;
-  int limit;  // the last key position that this lane's row sees, -1: no row
   const int last_tok = min(tok0 + QT, q_len) - 1;
   const int set_lo = start + tok0 + rows0 / HB;  // keys up to here are seen by every row of the set
   const int n_keys = start + last_tok + 1;
   const int per = max(((n_keys + splits - 1) / splits + KT - 1) / KT * KT, kLeastRange);
   const int k_begin = z * per, k_end = min(n_keys, k_begin + per);
+  const int n_tiles = k_begin < k_end ? (k_end - k_begin + KT - 1) / KT : 0;
   const float sharp = fmaxf(fabsf(scale) * 1.4426950408889634f, 1e-30f);  // scores to log2 (times a scale's sign, which Q takes: exact)
-  // Q comes in whole cache lines, 8 lanes for a row's 32 columns, and takes its fragments' order in LDS (fragments straight from memory
-  // touch 64 rows' lines with every load: 60 us of 460 at 8096 tokens and 16 heads)
-  bf16x8_t qf[NKS];
-  {
-    char* turn = reinterpret_cast<char*>(&meet[wave][0][0]);  // this wave's own until the first scores
-    constexpr int QROW = 80;                                  // 32 columns and 16 bytes of padding
-    const int rr = rows0 + (lane >> 3);
-    const float sign = scale < 0.f ? -1.f : 1.f;
-    float4 x[NKS / 2][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = rr + 8 * i, tl = tok0 + r / HB, hh = h0 + r % HB;
-      const bool valid = r < QT * HB && tl < q_len && hh < H;
-      const float* qrow = q_abs + (((size_t)first + (valid ? tl : tok0)) * H + (valid ? hh : h0)) * DK + half * (DK / 2) + 4 * (lane & 7);
-#pragma unroll
-      for (int c = 0; c < NKS / 2; ++c) x[c][i] = *reinterpret_cast<const float4*>(qrow + 32 * c);
-    }
-#pragma unroll
-    for (int c = 0; c < NKS / 2; ++c) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<uint2*>(turn + ((lane >> 3) + 8 * i) * QROW + 8 * (lane & 7)) =
-            uint2{pack_bf16(x[c][i].x * sign, x[c][i].y * sign), pack_bf16(x[c][i].z * sign, x[c][i].w * sign)};
-      wave_fence();
-#pragma unroll
-      for (int k = 0; k < 2; ++k) qf[2 * c + k] = *reinterpret_cast<const bf16x8_t*>(turn + (lane & 31) * QROW + 32 * k + 16 * hi);
-      wave_fence();
-    }
-    const int r = rows0 + (lane & 31), tl = tok0 + r / HB;
-    limit = r < QT * HB && tl < q_len && h0 + r % HB < H ? start + tl : -1;
-  }
-  f32x16_t o[NVT];
-#pragma unroll
-  for (int vt = 0; vt < NVT; ++vt)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) o[vt][e] = 0.f;
-  float m = -INFINITY, lsum = 0.f;  // reference maximum (log2), this lane's share of the row's sum
   const int* trow = table + (size_t)req_rows[b] * table_stride;
   const char* base = reinterpret_cast<const char*>(cache);
   auto slot_at = [&](int j0) { return trow[min(j0 + (lane & 31), n_keys - 1)]; };  // past the range: some row of the sequence, weight zero
-  // instruction i = 8 j + wave of a tile: 64 pieces of two or three rows
-  auto dma = [&](char* dst, int t) {
-    int l = lane, w = wave;
-    asm volatile("" : "+v"(l), "+s"(w));  // the places are worked out anew each tile: kept over the loop they would spill
+  // Value waves fetch.  Rows 8 v ... + 7: a row's latent entries are one instruction with one slot for the wave, the eight rows' rotated entries another.
+  // (Rows of 73 pieces over instructions of 64 took 20 vector operations and an LDS read in front of each.)
+  auto dma = [&](char* dst, int slot) __attribute__((always_inline)) {  // slot: of row 8 v + lane / 8
+    int l = lane, v = wave - 4;
+    asm volatile("" : "+v"(l), "+s"(v));  // the places are worked out anew each tile: kept over the loop they would spill
 #pragma unroll
-    for (int j = 0; j < NDMA; ++j) {
-      const int i = 8 * j + w;
-      if (i < NI) {
-        const int key = i * 64 / PCS, at = i * 64 - key * PCS + l;
-        const int next = (at >= PCS) + (at >= 2 * PCS);
-        const int ch = min(at - next * PCS, PCS - 2);
-        const size_t slot = (size_t)s_slot[t & 3][min(key + next, KT - 1)];
-        __builtin_amdgcn_global_load_lds((glb_void_t*)(base + slot * (DK * 2) + ch * 16), (lds_void_t*)(dst + i * 1024), 16, 0, 0);
+    for (int j = 0; j < 8; ++j) {
+      const char* row = base + (uint64_t)(uint32_t)__builtin_amdgcn_readlane(slot, 8 * j) * (DK * 2);
+      if (DV == 512 || lane < 32) __builtin_amdgcn_global_load_lds((glb_void_t*)(row + l * 16), (lds_void_t*)(dst + (8 * v + j) * ROW), 16, 0, 0);
+    }
+    const int r = 8 * v + (l >> 3);
+    __builtin_amdgcn_global_load_lds((glb_void_t*)(base + (uint64_t)(uint32_t)slot * (DK * 2) + DV * 2 + ((l ^ (r >> 1)) & 7) * 16),
+                                     (lds_void_t*)(dst + TAIL + v * 1024), 16, 0, 0);
+  };
+
+  // ---- queries: in whole cache lines, 8 lanes for a row's 32 columns, and by way of LDS into their fragments' order (fragments straight from memory
+  // touch 64 rows' lines with every load: 60 us of 460 at 8096 tokens and 16 heads).  The two waves of a row set take 32-column pieces in turn, the
+  // score wave keeps them: its own through LDS of its own, the other one's by way of two images, all at once.  (The whole way of a role, these loads
+  // included, lies behind one branch: what one role alone needs must not live beside the other's.)
+  constexpr int NU = DK / 64;  // a wave's pieces
+  auto queries = [&](auto fetch, auto keep) __attribute__((always_inline)) {
+    // slots in front of the queries: the value waves' of the first tile, the next two tiles' by way of LDS
+    const int slot = fetch ? trow[min(k_begin + 8 * (wave - 4) + (lane >> 3), n_keys - 1)] : slot_at(k_begin + wave * KT);
+    float4 x[NU][4];
+    const float sign = scale < 0.f ? -1.f : 1.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = rows0 + (lane >> 3) + 8 * i, tl = tok0 + r / HB, hh = h0 + r % HB;
+      const bool valid = r < QT * HB && tl < q_len && hh < H;
+      const float* qrow = q_abs + (((size_t)first + (valid ? tl : tok0)) * H + (valid ? hh : h0)) * DK + role * 32 + 4 * (lane & 7);
+#pragma unroll
+      for (int u = 0; u < NU; ++u) x[u][i] = *reinterpret_cast<const float4*>(qrow + 64 * u);
+    }
+    if (fetch) dma(img0, slot);
+    else if (wave < 3 && lane < KT) s_slot[wave][lane] = slot;
+    char* other = (set < 2 ? img1 : img2) + (set & 1) * (2 * NU * 1024);
+    static_assert(IMAGE >= 4 * NU * 1024, "two row sets' fragments");
+    if (fetch) {
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)  // fragment 2 u + (column of 32) / 16: [column / 8 & 1][row][8 columns]
+          *reinterpret_cast<uint2*>(other + (2 * u + ((lane & 7) >> 2)) * 1024 + ((lane >> 1) & 1) * 512 + ((lane >> 3) + 8 * i) * 16 + (lane & 1) * 8) =
+              uint2{pack_bf16(x[u][i].x * sign, x[u][i].y * sign), pack_bf16(x[u][i].z * sign, x[u][i].w * sign)};
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of the first tile
+    } else {
+      char* turn = reinterpret_cast<char*>(s_p) + set * 4096;
+      constexpr int QROW = 80;  // 32 columns and 16 bytes of padding
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *reinterpret_cast<uint2*>(turn + ((lane >> 3) + 8 * i) * QROW + 8 * (lane & 7)) =
+              uint2{pack_bf16(x[u][i].x * sign, x[u][i].y * sign), pack_bf16(x[u][i].z * sign, x[u][i].w * sign)};
+        wave_fence();
+#pragma unroll
+        for (int k = 0; k < 2; ++k) keep(4 * u + k, turn + (lane & 31) * QROW + 32 * k + 16 * hi);
+        wave_fence();
       }
     }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2 * NU; ++k) keep(k / 2 * 4 + 2 + (k & 1), other + k * 1024 + lane * 16);
+    __syncthreads();
   };
-  const int k_off = (lane & 31) * ROW + half * DK + hi * 16;
-  // transposing read: a 16-lane group reads 4 keys x 16 columns and hands lane j its column's four keys
-  const int v_off = (4 * hi + ((lane & 15) >> 2)) * ROW + half * DV + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
-  auto vfrag = [&](const char* buf, int i) {  // tile i % NVT of step i / NVT
-    const char* p = buf + v_off + i / NVT * 16 * ROW + i % NVT * 64;
+
+  // transposing read of values: a 16-lane group reads 4 keys x 16 columns and hands lane j its column's four keys
+  const int v_off = (4 * hi + ((lane & 15) >> 2)) * ROW + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+  auto vfrag = [&](const char* p) __attribute__((always_inline)) {  // 32 columns of 16 keys
     const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)p);
     const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(p + 8 * ROW));
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  f32x16_t s;
-  uint32_t pw[8];
-  auto scores = [&](const char* buf) __attribute__((always_inline)) {  // this wave's half of S^T, to `meet`
-    bf16x8_t kf[AHEAD + 1];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) s[e] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < AHEAD; ++ks) kf[ks] = *reinterpret_cast<const bf16x8_t*>(buf + k_off + ks * 32);
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      if (ks + AHEAD < NKS) kf[(ks + AHEAD) % (AHEAD + 1)] = *reinterpret_cast<const bf16x8_t*>(buf + k_off + (ks + AHEAD) * 32);
-      __builtin_amdgcn_sched_barrier(0);
-      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks % (AHEAD + 1)], qf[ks], s, 0, 0, 0);
-    }
-#pragma unroll
-    for (int g = 0; g < 4; ++g) meet[wave][g][lane] = f32x4_t{s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]};
-  };
-  auto weights = [&](int t) __attribute__((always_inline)) {
-    const int j0 = k_begin + t * KT;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const f32x4_t x = meet[wave & 6][g][lane] + meet[wave | 1][g][lane];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s[4 * g + e] = x[e];
-    }
-    // a lane's keys: j0 + (e & 3) + 8 (e >> 2) + 4 hi
-    if (j0 + KT - 1 > set_lo || j0 + KT > k_end) {
-      const int last = min(limit, k_end - 1) - j0 - 4 * hi;
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        if ((e & 3) + 8 * (e >> 2) > last) s[e] = -INFINITY;
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
-    mx = pair_max(mx) * sharp;
-    if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
-      const float m_new = fmaxf(m, mx);
-      const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
-#pragma unroll
-      for (int vt = 0; vt < NVT; ++vt)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) o[vt][e] *= alpha;
-      lsum *= alpha;
-      m = m_new;
-    }
-    const float ref = m == -INFINITY ? 0.f : m;  // no key yet: every weight is exp2(-inf) = 0
-    float sum = 0.f;  // of the fp32 weights
-#pragma unroll
-    for (int e = 0; e < 16; e += 2) {
-      const float w0 = weight(s[e], sharp, ref), w1 = weight(s[e + 1], sharp, ref);
-      sum += w0 + w1;
-      pw[e >> 1] = pack_bf16(w0, w1);
-    }
-    lsum += sum;
-  };
-  auto values = [&](const char* buf) __attribute__((always_inline)) {  // O^T += V^T P^T, 16 keys a step: a lane's eight of them are what its registers 8 step ... hold
-    bf16x8_t vf[VAHEAD + 1];
-#pragma unroll
-    for (int i = 0; i < VAHEAD; ++i) vf[i] = vfrag(buf, i);
-#pragma unroll
-    for (int i = 0; i < 2 * NVT; ++i) {
-      if (i + VAHEAD < 2 * NVT) vf[(i + VAHEAD) % (VAHEAD + 1)] = vfrag(buf, i + VAHEAD);
-      __builtin_amdgcn_sched_barrier(0);
-      const int w = i / NVT * 4;
-      const Q4 pq{pw[w], pw[w + 1], pw[w + 2], pw[w + 3]};
-      o[i % NVT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i % (VAHEAD + 1)], __builtin_bit_cast(bf16x8_t, pq), o[i % NVT], 0, 0, 0);
-    }
-  };
-  const int n_tiles = k_begin < k_end ? (k_end - k_begin + KT - 1) / KT : 0;
-  // between the halves of a stage: tile t + 1 is there, nobody reads tile t - 1 any more, whose image takes tile t + 2
-  auto turn = [&](char* before, int t) __attribute__((always_inline)) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of tile t + 1
-    __syncthreads();
-    int slot = 0;
-    if (t + 2 < n_tiles) {
-      if (wave == 7) slot = slot_at(k_begin + (t + 3) * KT);  // in front of the DMA: waiting for it does not wait for the DMA
-      dma(before, t + 2);
-    }
-    return slot;
-  };
-  auto early = [&](char* before, char* cur, char* next, int t) __attribute__((always_inline)) {
-    weights(t);
-    turn(before, t);
-    values(cur);
-    if (t + 1 < n_tiles) scores(next);
-    __syncthreads();
-    return t + 1 < n_tiles;
-  };
-  auto late = [&](char* before, char* cur, int t) __attribute__((always_inline)) {
-    scores(cur);
-    const int slot = turn(before, t);
-    weights(t);
-    if (t + 2 < n_tiles && wave == 7 && lane < KT) s_slot[(t + 3) & 3][lane] = slot;
-    __syncthreads();
-    values(cur);
-    return t + 1 < n_tiles;
-  };
-  auto finish = [&]() __attribute__((always_inline)) {
-    lsum += __shfl_xor(lsum, 32, 64);
-    m *= kLn2;
+  // a row set's outputs times f, 32 columns at a time by way of LDS, so that a row's are stored as one cache line (lanes' own 16 bytes of 64 rows'
+  // lines: 60 us of 460 at 8096 tokens and 16 heads); a row's 16-byte pieces change places by its number, against bank conflicts
+  auto finish = [&](const f32x16_t* o, int nvt, int col0) __attribute__((always_inline)) {
     int l = lane;
     asm volatile("" : "+v"(l));  // the rows are worked out anew: no registers for them meanwhile
-    const int hh = min(h0 + (rows0 + (l & 31)) % HB, H - 1);
     float f = 1.f;
     if (splits == 1) {
-      const float sf = sink_factor(sink, hh, m);
-      f = sf / (sf * lsum + sink_weight(sink, hh, m));
-    } else if (limit >= 0 && hi == 0 && half == 0) {
-      const size_t row = ((size_t)first + tok0 + (rows0 + (l & 31)) / HB) * H + hh;
-      part_ml[(row * splits + z) * 2] = m;
-      part_ml[(row * splits + z) * 2 + 1] = lsum;
+      const int hh = min(h0 + (rows0 + (l & 31)) % HB, H - 1);
+      const float2 ml = s_ml[set][l & 31];
+      const float sf = sink_factor(sink, hh, ml.x);
+      f = sf / (sf * ml.y + sink_weight(sink, hh, ml.x));
     }
-    // 32 columns at a time by way of LDS, so that a row's are stored as one cache line (lanes' own 16 bytes of 64 rows' lines: 60 us of
-    // 460 at 8096 tokens and 16 heads); a row's 16-byte pieces change places by its number, against bank conflicts
-    char* turn = reinterpret_cast<char*>(&meet[wave][0][0]);
+    char* turn = (wave < 4 ? img0 : img1) + (wave & 3) * 4096;
+    static_assert(IMAGE >= 4 * 4096, "four waves' turns");
     float* dst[4];
     bool valid[4];
 #pragma unroll
@@ -275,10 +193,10 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
       const int r = rows0 + (l >> 3) + 8 * i, tl = tok0 + r / HB, h = h0 + r % HB;
       valid[i] = r < QT * HB && tl < q_len && h < H && (n_tiles > 0 || splits == 1);  // without keys the partial output is not read
       const size_t row = ((size_t)first + tl) * H + h;
-      dst[i] = (splits == 1 ? out + row * DV : part_o + (row * splits + z) * DV) + half * (DV / 2) + 4 * (l & 7);
+      dst[i] = (splits == 1 ? out + row * DV : part_o + (row * splits + z) * DV) + col0 + 4 * (l & 7);
     }
 #pragma unroll
-    for (int vt = 0; vt < NVT; ++vt) {
+    for (int vt = 0; vt < nvt; ++vt) {
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         *reinterpret_cast<float4*>(turn + (l & 31) * 128 + (((2 * g + hi) ^ l) & 7) * 16) =
@@ -291,39 +209,182 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
       wave_fence();
     }
   };
-  if (n_tiles > 0) {
-    if (wave < 3 && lane < KT) s_slot[wave][lane] = slot_at(k_begin + wave * KT);
-    __syncthreads();
-    dma(img0, 0);
-    if (n_tiles > 1) dma(img1, 1);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-  }
-  // Both ways pass the same barriers: one, and two a tile.  They stay apart to the end (the marks keep the compiler from joining the
-  // equal tails): where they met, all accumulators would have to lie in the same registers, and hundreds were spilled.
-  if (wave < 4) {
-    if (n_tiles > 0) {
-      scores(img0);
+
+  // ---- Iteration t: the score waves turn tile t into weights and add their columns' values, the value waves add tile t - 1's to theirs and fetch
+  // tile t + 1 into the image of tile t - 2.  Both ways pass the same barriers: n_tiles + 1.
+  if (role == 0) {
+    const int r = rows0 + (lane & 31), tl = tok0 + r / HB;
+    const int limit = r < QT * HB && tl < q_len && h0 + r % HB < H ? start + tl : -1;  // the last key position that this lane's row sees, -1: no row
+    const int k_off = (lane & 31) * ROW + hi * 16;
+    bf16x8_t qf[NQ];
+    if (n_tiles > 0)
+      queries(std::false_type{}, [&](int ks, const char* at) __attribute__((always_inline)) {
+        const bf16x8_t f = *reinterpret_cast<const bf16x8_t*>(at);
+        if (ks < NQ) qf[ks < NQ ? ks : 0] = f;
+        else s_q[set][ks < NQ ? 0 : ks - NQ][lane] = __builtin_bit_cast(f32x4_t, f);
+      });
+    float m = -INFINITY, lsum = 0.f;  // reference maximum (log2), this lane's share of the row's sum
+    f32x16_t o[NVS];
+#pragma unroll
+    for (int vt = 0; vt < NVS; ++vt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[vt][e] = 0.f;
+    auto scores = [&](const char* buf, int t) __attribute__((always_inline)) {
+      constexpr int AHEAD = 3;  // fragments are read so many products before their use
+      int l = lane;
+      asm volatile("" : "+v"(l));
+      auto kfrag = [&](int ks) __attribute__((always_inline)) {
+        if (ks < NA) return *reinterpret_cast<const bf16x8_t*>(buf + k_off + ks * 32);
+        return *reinterpret_cast<const bf16x8_t*>(buf + TAIL + (l & 31) * 128 + (((2 * (ks - NA) + (l >> 5)) ^ ((l & 31) >> 1)) & 7) * 16);
+      };
+      f32x16_t s;
+      bf16x8_t kf[AHEAD + 1], ql[2];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[e] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < AHEAD; ++ks) kf[ks] = kfrag(ks);
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+        if (ks + AHEAD < NKS) kf[(ks + AHEAD) % (AHEAD + 1)] = kfrag(ks + AHEAD);
+        if (ks + 1 >= NQ && ks + 1 < NKS) ql[(ks + 1) & 1] = __builtin_bit_cast(bf16x8_t, s_q[set][ks + 1 >= NQ ? (ks + 1 - NQ) % (NL ? NL : 1) : 0][lane]);
+        __builtin_amdgcn_sched_barrier(0);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks % (AHEAD + 1)], ks < NQ ? qf[ks < NQ ? ks : 0] : ql[ks & 1], s, 0, 0, 0);
+      }
+      // a lane's keys: j0 + (e & 3) + 8 (e >> 2) + 4 hi
+      const int j0 = k_begin + t * KT;
+      if (j0 + KT - 1 > set_lo || j0 + KT > k_end) {
+        const int last = min(limit, k_end - 1) - j0 - 4 * hi;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if ((e & 3) + 8 * (e >> 2) > last) s[e] = -INFINITY;
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
+      mx = pair_max(mx) * sharp;
+      const float m_new = fmaxf(m, mx);
+      const float alpha = m_new == m ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
+      if (hi == 0) s_alpha[t & 1][set][lane] = alpha;
+      if (__builtin_amdgcn_ballot_w64(m_new != m) != 0) {
+#pragma unroll
+        for (int vt = 0; vt < NVS; ++vt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) o[vt][e] *= alpha;
+        lsum *= alpha;
+        m = m_new;
+      }
+      const char* vp = buf + v_off + NVV * 64;
+      bf16x8_t vf[3];
+      vf[0] = vfrag(vp);
+      vf[1] = vfrag(vp + 64);
+      const float ref = m == -INFINITY ? 0.f : m;  // no key yet: every weight is exp2(-inf) = 0
+      float sum = 0.f;  // of the fp32 weights
+      uint32_t pw[8];
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) {
+        const float w0 = weight(s[e], sharp, ref), w1 = weight(s[e + 1], sharp, ref);
+        sum += w0 + w1;
+        pw[e >> 1] = pack_bf16(w0, w1);
+      }
+      lsum += sum;
+#pragma unroll
+      for (int w = 0; w < 2; ++w)
+        *reinterpret_cast<Q4*>(&s_p[t & 1][set][w][lane]) = Q4{pw[4 * w], pw[4 * w + 1], pw[4 * w + 2], pw[4 * w + 3]};
+#pragma unroll
+      for (int i = 0; i < 2 * NVS; ++i) {  // O^T += V^T P^T, 16 keys a step: a lane's eight of them are what its registers 8 step ... hold
+        if (i + 2 < 2 * NVS) vf[(i + 2) % 3] = vfrag(vp + (i + 2) / NVS * 16 * ROW + (i + 2) % NVS * 64);
+        __builtin_amdgcn_sched_barrier(0);
+        const int w = i / NVS * 4;
+        const Q4 pq{pw[w], pw[w + 1], pw[w + 2], pw[w + 3]};
+        o[i % NVS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i % 3], __builtin_bit_cast(bf16x8_t, pq), o[i % NVS], 0, 0, 0);
+      }
       __syncthreads();
-      for (int t = 0;; t += 3) {
-        if (!early(img2, img0, img1, t)) break;
-        if (!early(img0, img1, img2, t + 1)) break;
-        if (!early(img1, img2, img0, t + 2)) break;
+    };
+    for (int t = 0; t < n_tiles; t += 3) {
+      scores(img0, t);
+      if (t + 1 < n_tiles) scores(img1, t + 1);
+      if (t + 2 < n_tiles) scores(img2, t + 2);
+    }
+    lsum += __shfl_xor(lsum, 32, 64);
+    m *= kLn2;
+    if (hi == 0) {
+      s_ml[set][lane] = float2{m, lsum};
+      if (splits > 1 && limit >= 0) {
+        const size_t row = ((size_t)first + tl) * H + h0 + r % HB;
+        part_ml[(row * splits + z) * 2] = m;
+        part_ml[(row * splits + z) * 2 + 1] = lsum;
       }
     }
-    finish();
-    asm volatile("; waves 0 - 3");
+    __syncthreads();
+    finish(o, NVS, NVV * 32);
+    asm volatile("; score waves");
   } else {
-    if (n_tiles > 0) {
+    if (n_tiles > 0) queries(std::true_type{}, [](int, const char*) {});
+    f32x16_t o[NVV];
+#pragma unroll
+    for (int vt = 0; vt < NVV; ++vt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[vt][e] = 0.f;
+    auto values = [&](const char* buf, int t) __attribute__((always_inline)) {
+      constexpr int SOME = 2;  // fragments are read so many at a time, a set ahead
+      const char* vp = buf + v_off;
+      const float alpha = s_alpha[t & 1][set][lane & 31];
+      Q4 p[2];
+#pragma unroll
+      for (int w = 0; w < 2; ++w) p[w] = *reinterpret_cast<const Q4*>(&s_p[t & 1][set][w][lane]);
+      bf16x8_t vf[2][SOME];
+#pragma unroll
+      for (int n = 0; n < SOME; ++n) vf[0][n] = vfrag(vp + n * 64);
+      __builtin_amdgcn_sched_barrier(0);
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+        for (int vt = 0; vt < NVV; ++vt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) o[vt][e] *= alpha;
+      }
+#pragma unroll
+      for (int i = 0; i < 2 * NVV; i += SOME) {
+        if (i + SOME < 2 * NVV) {
+#pragma unroll
+          for (int n = 0; n < SOME; ++n) vf[(i / SOME & 1) ^ 1][n] = vfrag(vp + (i + SOME + n) / NVV * 16 * ROW + (i + SOME + n) % NVV * 64);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < SOME; ++n)
+          o[(i + n) % NVV] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i / SOME & 1][n], __builtin_bit_cast(bf16x8_t, p[(i + n) / NVV]), o[(i + n) % NVV], 0, 0, 0);
+      }
+    };
+    auto fetch = [&](char* next, int t) __attribute__((always_inline)) {
+      int slot = 0;
+      if (wave == 7 && t + 3 < n_tiles) slot = slot_at(k_begin + (t + 3) * KT);  // in front of the DMA: waiting for it does not wait for the DMA
+      if (t + 1 < n_tiles) dma(next, s_slot[(t + 1) & 3][8 * (wave - 4) + (lane >> 3)]);
+      return slot;
+    };
+    auto arrived = [&](int slot, int t) __attribute__((always_inline)) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of tile t + 1
+      if (wave == 7 && lane < KT) s_slot[(t + 3) & 3][lane] = slot;
       __syncthreads();
-      for (int t = 0;; t += 3) {
-        if (!late(img2, img0, t)) break;
-        if (!late(img0, img1, t + 1)) break;
-        if (!late(img1, img2, t + 2)) break;
+    };
+    auto step = [&](const char* before, char* next, int t) __attribute__((always_inline)) {
+      const int slot = fetch(next, t);
+      values(before, t - 1);
+      arrived(slot, t);
+    };
+    arrived(fetch(img1, 0), 0);
+    if (n_tiles > 0) {
+      int t = 1;  // (no step of the loop is conditional: where ways met, the accumulators had two places, and hundreds were spilled)
+      for (; t + 2 <= n_tiles; t += 3) {
+        step(img0, img2, t);
+        step(img1, img0, t + 1);
+        step(img2, img1, t + 2);
+      }
+      if (t <= n_tiles) {
+        step(img0, img2, t);
+        if (t + 1 <= n_tiles) step(img1, img0, t + 1);
       }
     }
-    finish();
-    asm volatile("; waves 4 - 7");
+    finish(o, NVV, 0);
+    asm volatile("; value waves");
   }
 }
 

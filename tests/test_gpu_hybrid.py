@@ -364,6 +364,29 @@ def test_latent_attention_usual_widths(dev, H, R, splits, sink):
         assert float((got - ref).abs().max()) < 5e-2 * float(ref.abs().max()), new
 
 
+@pytest.mark.parametrize("scale", [0.08, -0.08])
+@pytest.mark.parametrize("H,R", [(16, 512), (12, 512), (16, 256)])
+def test_latent_portion_tiles(dev, H, R, scale):
+    """One portion behind so many keys that its 32-key tiles are 1 ... 8 (the ways through images that follow each other in threes), whole or with a key
+    more, in one range and in ranges some of which have no keys.  Bound as in test_latent_attention_usual_widths."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(H + R)
+    r, n = 64, 13
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    for keys in (n, 32, 33, 64, 65, 96, 97, 128, 129, 160, 192, 193, 224, 256):
+        slots = torch.randperm(keys, generator=g)
+        cache, q = torch.randn(keys, R + r, generator=g).bfloat16(), torch.randn(n, H, R + r, generator=g) * 0.8
+        rows = cache[slots].double()
+        s = torch.einsum("thk,jk->thj", q.double(), rows) * scale
+        s = s.masked_fill(torch.arange(keys)[None, None, :] > (torch.arange(n) + keys - n)[:, None, None], -torch.inf)
+        ref = torch.softmax(s, -1) @ rows[:, :R]
+        for splits in (1, 3):
+            out = torch.full((n, H, R), float("nan"), device=dev)
+            mixops.latent_attn(out, q.to(dev), cache.to(dev), slots.int()[None].to(dev), i32(0), i32(keys), i32(0, n), 1, R, scale, splits=splits)
+            assert float((out.double().cpu() - ref).norm() / ref.norm()) < 8e-3, (keys, splits)
+
+
 @pytest.mark.parametrize("B", [64, 65, 150])
 @pytest.mark.parametrize("splits", [1, 3])
 @pytest.mark.parametrize("most", [1, 20], ids=["decode", "portions"])
