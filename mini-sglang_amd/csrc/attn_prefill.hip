@@ -462,6 +462,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) const void glb_void_t;
 
+// lane I's number of every 16 lanes
+template <int I>
+__device__ __forceinline__ uint64_t row_lane(uint64_t x) {
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, 0x150 + I, 0xf, 0xf, true);  // row_newbcast
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), 0x150 + I, 0xf, 0xf, true);
+  return (uint64_t)hi << 32 | lo;
+}
+
 template <typename T, int ABL = 0, bool RANGES = false>
 __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillParams p, int total_tiles) {
   // two distinct LDS objects, not one array: the compiler then knows a tile's fragment reads cannot alias the DMA writes
@@ -517,21 +525,26 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
   // ---- staging: DMA instruction i of this wave fills rows 16 i + 4 wave .. + 3 (chunk 4 i + wave of the image);
   //      lane -> row st_row + 16 i, 16-byte slot (lane & 15)
   const int st_row = tid >> 4;
-  const int64_t k_lane = (int64_t)kvh * p.kv_stride_head + (((lane & 15) ^ (st_row & 15)) << 3);
-  const int64_t v_lane = (int64_t)kvh * p.kv_stride_head + (((lane & 15) ^ ((st_row & 3) << 2)) << 3);
-  int sl[4];
-  auto load_slots = [&](int kt) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sl[i] = pt[min(kt * kKTile + st_row + 16 * i, k_len - 1)];
-  };
+  const char* k_lane = reinterpret_cast<const char*>(p.k + (int64_t)kvh * p.kv_stride_head + (((lane & 15) ^ (st_row & 15)) << 3));
+  const char* v_lane = reinterpret_cast<const char*>(p.v + (int64_t)kvh * p.kv_stride_head + (((lane & 15) ^ ((st_row & 3) << 2)) << 3));
+  // A row's slot and offset are found once: lane i of the 16 that copy rows st_row, + 16, + 32, + 48 has row st_row + 16 i's, and the sixteen
+  // take it from there as the address is added up (every lane for its own four rows: three more quarter-rate multiplies and three more
+  // loads a tile; 64 heads, 8192 tokens after 16384: 5285 -> 5210 us, 29 requests of 100 - 1024, 40 heads on 8: 236 -> 234)
+  const uint32_t row_of = st_row + 16 * (lane & 3);
+  int sl;
+  auto load_slots = [&](int kt) { sl = pt[min((uint32_t)(kt * kKTile) + row_of, (uint32_t)(k_len - 1))]; };
   auto issue_dma = [&](char* buf) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t off = slot_offset(sl[i], p.kv_stride_tok);
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(p.k + off + k_lane), (lds_void_t*)(buf + (4 * i + wave) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(p.v + off + v_lane),
-                                       (lds_void_t*)(buf + kTileBytes + (4 * i + wave) * 1024), 16, 0, 0);
-    }
+    const uint64_t off = (uint64_t)slot_offset(sl, p.kv_stride_tok) * 2;
+    auto four_rows = [&](auto I) __attribute__((always_inline)) {
+      constexpr int i = decltype(I)::value;
+      const uint64_t o = row_lane<i>(off);
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(k_lane + o), (lds_void_t*)(buf + (4 * i + wave) * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(v_lane + o), (lds_void_t*)(buf + kTileBytes + (4 * i + wave) * 1024), 16, 0, 0);
+    };
+    four_rows(std::integral_constant<int, 0>{});
+    four_rows(std::integral_constant<int, 1>{});
+    four_rows(std::integral_constant<int, 2>{});
+    four_rows(std::integral_constant<int, 3>{});
   };
   // per-lane LDS addresses (buffer 0): K fragment of k-step ks, V^T fragment of d block nb
   int koff[8], voff[4];
