@@ -36,6 +36,7 @@ class HipAttnMetadata:
     tile_order: Optional[torch.Tensor] = None  # [total_tiles] int32: q tiles, most keys first (prefill only)
     ranges: tuple = (1, 0)                  # key ranges of a q tile, 64-key tiles of each (prefill only)
     scratch: Optional[torch.Tensor] = None  # their partial sums, from the first layer on
+    pairs: bool = False                     # two heads a workgroup (prefill only)
     plan: Optional[torch.Tensor] = None     # decode work list (device)
     chunks: Optional[tuple] = None          # recurrent layers: (items [n, 3], item_first [B + 1], n) of long portions cut in pieces
     delta_chunks: Optional[tuple] = None    # the same list at the delta-rule layers' piece size
@@ -190,7 +191,7 @@ class HipAttnBackend:
                 md.scratch = torch.empty(ops.prefill_ranges_workspace_bytes(md.total_tiles * self.qo_heads * md.ranges[0]), dtype=torch.uint8, device=self.device)
             ops.attn_prefill(out, q, k_tok, v_tok, table, md.req_rows, md.seq_lens, md.cu_seqlens_q, md.tile_cu,
                              md.batch, md.total_tiles, self.scale, tile_order=md.tile_order,
-                             ranges=md.ranges, workspace=md.scratch)
+                             ranges=md.ranges, workspace=md.scratch, pairs=md.pairs)
         return out
 
     # ------------------------------------------------------------------ metadata
@@ -221,6 +222,7 @@ class HipAttnBackend:
             max_seqlen_q=max_q, max_seqlen_k=max_k, tile_cu=None if decode else dev[3 * bs + 1: 4 * bs + 2],
             total_tiles=total_tiles, tile_order=None if decode else dev[4 * bs + 2:],
             ranges=(1, 0) if decode else ops.prefill_ranges(total_tiles, self.qo_heads, max_q, max_k),
+            pairs=not decode and ops.prefill_pairs(total_tiles, self.qo_heads, self.kv_heads, seqlens_q, seqlens_k),
         )
         if decode and not self._replayed_from_graph(batch, bs):
             # runs eagerly: plan now (device side, no sync).  Only batches the engine will REPLAY are planned

@@ -449,10 +449,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 //   * LDS reads issued >= 4 MFMAs ahead of their use (pinned with sched_barrier); beside a DMA under way the compiler waits for ALL of a
 //     wave's reads at the first use of any, so the V^T fragments are asked for after the second key block's have come;
 //   * nothing of the softmax crosses LDS: the halves' maximum and their shares of a tile's sum by lane swaps.
-// What bounds it: a wave's tile is 1024 cycles of the matrix cores and about as many of the vector units (32 scores a lane, the exponential
-// 16 cycles each), and two waves per SIMD overlap them only in part.  40 heads on 8, 29 requests of 100 - 1024 tokens: 245 -> 244 us with the
-// last two points; 64 heads, 8192 tokens after 16384: 5570 -> 5490 (1000 TFLOP/s), the same bits.  (Sums of the rounded weights, one instruction
-// a pair: 242 and 5510 us, and 2^-9 of a row's weight off.)
+// What bounds it: power, where the launch is long (1.8 GHz; inputs of zeros 5330 -> 4020 us), and the copies.  64 heads, 8192 tokens after 16384, us
+// with a part left out: all copies but the first 4330, no exponentials 5025, no rescale 5200, none of exponentials, rescale and mask 4930; the scores
+// of the next tile in the same wave beside a tile's weights: 5290.  A wave's tile is 1024 cycles of the matrix cores and about as many of the vector
+// units (32 scores a lane, the exponential 16 cycles each).  5240 us with one head a workgroup, 4940 with two (1110 TFLOP/s); 40 heads on 8, 29 requests
+// of 100 - 1024 tokens: 234.  (Sums of the rounded weights, one instruction a pair: 0.5 % faster, and 2^-9 of a row's weight off.)
+// HEADS = 2: eight waves, two heads of a kv head beside each other over the same tiles: half the copies.  One workgroup a CU then, so nothing runs
+// under its start, and the last round is coarser: for many long chains of tiles (the rule and its other side: ops.prefill_pairs).
 // RANGES: workgroup (.., z) takes the tiles z * run .. of the job's keys; sums of more than one range go to attn_prefill_join_kernel in fp32, in
 // the order of the lanes.  For launches that leave compute units empty, where the longest chain of tiles (1.26 us each) is the time: 16 heads on
 // 8, 100 tokens after 2000: 45.1 -> 13.7 us, 1000 after 3000: 81.7 -> 53.2; 5 on 1, 2000 tokens: 43.0 -> 20.5 (both launches, in a captured chain;
@@ -470,8 +473,8 @@ __device__ __forceinline__ uint64_t row_lane(uint64_t x) {
   return (uint64_t)hi << 32 | lo;
 }
 
-template <typename T, int ABL = 0, bool RANGES = false>
-__global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillParams p, int total_tiles) {
+template <typename T, int ABL = 0, bool RANGES = false, int HEADS = 1>
+__global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const PrefillParams p, int total_tiles) {
   // two distinct LDS objects, not one array: the compiler then knows a tile's fragment reads cannot alias the DMA writes
   // of the next tile (other object) and does not wait for them (vmcnt) before the reads
   __shared__ __attribute__((aligned(1024))) char lds_a[2 * kTileBytes];  // tiles 0, 2, ..: [K | V]
@@ -482,20 +485,19 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
   constexpr bool kPrioMatrix = (ABL & 16) != 0;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), rows = wave & 3;  // rows 32 rows .. + 31 of the q tile
   const int hi = lane >> 5;
 
   const PrefillJob job = prefill_job(p, total_tiles);
   if (job.tile < 0) return;
-  const int kvh = job.kvh, hq = job.hq, tile = job.tile;
+  const int kvh = job.kvh, hq = job.hq * HEADS + (wave >> 2), tile = job.tile;
 
   const TileRequest rq = find_request(p, tile, lane);
   const int q_begin = rq.q_begin;
   const int q_len = rq.q_end - q_begin;
   const int k_len = rq.k_len;
   const int q0 = (tile - rq.tile_first) * kQTile;
-  const int row = rq.row;
-  const int* pt = p.page_table + (int64_t)row * p.pt_stride;
+  const int* pt = p.page_table + (int64_t)rq.row * p.pt_stride;
   const int diag = k_len - q_len;
   const int kend = min(k_len, diag + min(q0 + kQTile, q_len));
   const int all_tiles = (kend + kKTile - 1) / kKTile;
@@ -503,7 +505,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
   const int ntiles = RANGES && blockIdx.y + 1 < gridDim.y ? min(all_tiles, t0 + p.run) : all_tiles;  // past this workgroup's last
   if (RANGES && t0 > 0 && t0 >= ntiles) return;
 
-  const int my_q = q0 + wave * 32 + (lane & 31);
+  const int my_q = q0 + rows * 32 + (lane & 31);
   const bool q_valid = my_q < q_len;
   const int64_t q_tok = q_begin + (q_valid ? my_q : q_len - 1);
   U4 qf[8];
@@ -513,7 +515,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
     for (int ks = 0; ks < 8; ++ks) qf[ks] = ldg16(qp + ks * 16);
   }
   const int my_qpos = diag + my_q;
-  const int wave_min_qpos = diag + q0 + wave * 32;  // scalar
+  const int wave_min_qpos = diag + q0 + rows * 32;  // scalar
 
   f32x16 o[4];
 #pragma unroll
@@ -522,15 +524,16 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
     for (int r = 0; r < 16; ++r) o[nb][r] = 0.f;
   float m_run = kNegBigP, l_run = 0.f;
 
-  // ---- staging: DMA instruction i of this wave fills rows 16 i + 4 wave .. + 3 (chunk 4 i + wave of the image);
-  //      lane -> row st_row + 16 i, 16-byte slot (lane & 15)
+  // ---- staging: DMA instruction i of this wave fills rows kApart i + 4 wave .. + 3 of the image; lane -> row st_row + kApart i,
+  //      16-byte slot (lane & 15)
+  constexpr int kApart = 16 * HEADS, kTurns = 4 / HEADS;
   const int st_row = tid >> 4;
   const char* k_lane = reinterpret_cast<const char*>(p.k + (int64_t)kvh * p.kv_stride_head + (((lane & 15) ^ (st_row & 15)) << 3));
   const char* v_lane = reinterpret_cast<const char*>(p.v + (int64_t)kvh * p.kv_stride_head + (((lane & 15) ^ ((st_row & 3) << 2)) << 3));
-  // A row's slot and offset are found once: lane i of the 16 that copy rows st_row, + 16, + 32, + 48 has row st_row + 16 i's, and the sixteen
-  // take it from there as the address is added up (every lane for its own four rows: three more quarter-rate multiplies and three more
+  // A row's slot and offset are found once: lane i of the 16 that copy rows st_row, st_row + kApart, .. has row st_row + kApart i's, and the sixteen
+  // take it from there as the address is added up (every lane for its own four rows, HEADS = 1: three more quarter-rate multiplies and three more
   // loads a tile; 64 heads, 8192 tokens after 16384: 5285 -> 5210 us, 29 requests of 100 - 1024, 40 heads on 8: 236 -> 234)
-  const uint32_t row_of = st_row + 16 * (lane & 3);
+  const uint32_t row_of = st_row + kApart * (lane & (kTurns - 1));
   int sl;
   auto load_slots = [&](int kt) { sl = pt[min((uint32_t)(kt * kKTile) + row_of, (uint32_t)(k_len - 1))]; };
   auto issue_dma = [&](char* buf) {
@@ -538,13 +541,15 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
     auto four_rows = [&](auto I) __attribute__((always_inline)) {
       constexpr int i = decltype(I)::value;
       const uint64_t o = row_lane<i>(off);
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(k_lane + o), (lds_void_t*)(buf + (4 * i + wave) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(v_lane + o), (lds_void_t*)(buf + kTileBytes + (4 * i + wave) * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(k_lane + o), (lds_void_t*)(buf + (kApart / 4 * i + wave) * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(v_lane + o), (lds_void_t*)(buf + kTileBytes + (kApart / 4 * i + wave) * 1024), 16, 0, 0);
     };
     four_rows(std::integral_constant<int, 0>{});
     four_rows(std::integral_constant<int, 1>{});
-    four_rows(std::integral_constant<int, 2>{});
-    four_rows(std::integral_constant<int, 3>{});
+    if constexpr (kTurns == 4) {
+      four_rows(std::integral_constant<int, 2>{});
+      four_rows(std::integral_constant<int, 3>{});
+    }
   };
   // per-lane LDS addresses (buffer 0): K fragment of k-step ks, V^T fragment of d block nb
   int koff[8], voff[4];
@@ -718,7 +723,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_dma_kernel(const PrefillP
   }
 
   if (RANGES && all_tiles > p.run) {
-    const int64_t at = ((int64_t)blockIdx.y * total_tiles * p.hq + (int64_t)tile * p.hq + hq) * 4 + wave;
+    const int64_t at = ((int64_t)blockIdx.y * total_tiles * p.hq + (int64_t)tile * p.hq + hq) * 4 + rows;
     f32x4p* po = reinterpret_cast<f32x4p*>(p.part_o) + at * 1024 + lane;  // [16 pieces][64 lanes]
 #pragma unroll
     for (int i = 0; i < 16; ++i)
@@ -806,11 +811,11 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
                                  int impl, int ranges, int run, float* workspace, void* stream) {
   MSGL_REQUIRE(batch >= 0 && total_tiles >= 0, "attn_prefill: negative sizes");
 #ifdef MSGL_PREFILL_DIAG
-  MSGL_REQUIRE(impl == 0 || impl == 2 || impl == 4 || (impl >= 16 && impl < 48) || (impl >= 64 && impl < 128),
+  MSGL_REQUIRE(impl == 0 || impl == 2 || impl == 4 || impl == 6 || (impl >= 16 && impl < 48) || (impl >= 64 && impl < 128),
                "attn_prefill: impl %d (0 = 4 DMA-staged, 2 register-staged; diagnostic build: 16 + bits / 64 + bits = ablations)", impl);
 #else
-  MSGL_REQUIRE(impl == 0 || impl == 2 || impl == 4,
-               "attn_prefill: impl %d (0 = 4 the DMA-staged kernel, 2 the register-staged kernel; ablation codes need a "
+  MSGL_REQUIRE(impl == 0 || impl == 2 || impl == 4 || impl == 6,
+               "attn_prefill: impl %d (0 = 4 the DMA-staged kernel, 6 with two heads a workgroup, 2 the register-staged kernel; ablation codes need a "
                "-DMSGL_PREFILL_DIAG build)", impl);
 #endif
   if (batch == 0 || total_tiles == 0) return MSGL_OK;
@@ -819,6 +824,7 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   MSGL_REQUIRE(head_dim == 128, "attn_prefill: head_dim %d unsupported (128 only)", head_dim);
   MSGL_REQUIRE(num_kv_heads >= 1 && num_q_heads % num_kv_heads == 0 && num_q_heads <= 65535,
                "attn_prefill: %d q heads / %d kv heads", num_q_heads, num_kv_heads);
+  MSGL_REQUIRE(impl != 6 || num_q_heads / num_kv_heads % 2 == 0, "attn_prefill: heads in pairs, %d q heads / %d kv heads", num_q_heads, num_kv_heads);
   MSGL_REQUIRE(kv_stride_tok > 0 && kv_stride_tok < (1ll << 32), "attn_prefill: kv token stride %lld", (long long)kv_stride_tok);
   MSGL_REQUIRE(q_stride_tok % 8 == 0 && kv_stride_tok % 8 == 0 && kv_stride_head % 8 == 0 &&
                    out_stride_tok % 4 == 0,
@@ -844,7 +850,8 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   p.out_stride = out_stride_tok;
   p.batch = batch;
   p.hq = num_q_heads;
-  p.group = num_q_heads / num_kv_heads;
+  const int heads = impl == 6 ? 2 : 1;  // of a workgroup
+  p.group = num_q_heads / num_kv_heads / heads;
   p.per = num_kv_heads;
   p.share_log2 = 3;
   while (p.share_log2 > 0 && p.per % 2 == 0) {
@@ -858,7 +865,7 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
     return MSGL_EINVAL;
   }
   if (impl == 0) impl = 4;  // the DMA-staged kernel; impl 2 keeps its predecessor callable (A/B timing, cross-check in tests)
-  const int64_t total = (int64_t)total_tiles * num_q_heads;
+  const int64_t total = (int64_t)total_tiles * (num_q_heads / heads);
   MSGL_REQUIRE(total < (1ll << 30), "attn_prefill: %lld workgroups", (long long)total);
   const int even = (int)(((int64_t)total_tiles * p.group * p.per + (1 << p.share_log2) - 1) >> p.share_log2);
   p.stretch = ranges == 1 && total <= 256 ? even : 0;
@@ -879,6 +886,9 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   } else if (impl == 4) {
     if (dtype == MSGL_BF16) attn_prefill_dma_kernel<BF16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
     else attn_prefill_dma_kernel<FP16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
+  } else if (impl == 6) {
+    if (dtype == MSGL_BF16) attn_prefill_dma_kernel<BF16, 0, false, 2><<<dim3(blocks), dim3(512), 0, s>>>(p, total_tiles);
+    else attn_prefill_dma_kernel<FP16, 0, false, 2><<<dim3(blocks), dim3(512), 0, s>>>(p, total_tiles);
   } else if (impl == 2) {
     if (dtype == MSGL_BF16) attn_prefill_tr_kernel<BF16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
     else attn_prefill_tr_kernel<FP16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);

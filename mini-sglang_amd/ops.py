@@ -11,6 +11,7 @@ import functools
 import os
 from typing import Optional, Tuple
 
+import numpy as np
 import torch
 
 from . import _lib
@@ -438,6 +439,23 @@ def prefill_ranges(total_tiles: int, qo_heads: int, max_seqlen_q: int, max_seqle
     return (ranges, run) if ranges > 1 else (1, 0)
 
 
+def prefill_pairs(total_tiles: int, qo_heads: int, kv_heads: int, seqlens_q: np.ndarray, seqlens_k: np.ndarray) -> bool:
+    """Whether a launch without key ranges takes two heads of a kv head a workgroup: half the copies, and one workgroup a CU.
+
+    The copies are what this saves, 6 % of a long tile chain; a workgroup's start is no longer under another one's tiles, and the last round of
+    workgroups is a coarser one.  us, one head -> two (q tiles x heads; mean 64-key tiles of each):
+      4096 of 324  5240 -> 4940    4224 of 26  525 -> 512    3072 of 15.8  226 -> 223    4096 of 12.9  271 -> 264    4096 of 11  232 -> 235
+      3904 of 8.6  185 -> 190      4096 of 3   110 -> 119
+    Fewer than six rounds of the 512 places win or lose by how full the last one is (2688 of 26 340 -> 342, 1408 of 26 177 -> 169, 1088 of
+    26 149 -> 166, 640 of 26 100 -> 112, 512 of 33 108 -> 121), but two rounds nearly full win: 896 of 26 120 -> 111, 1024 of 65 315 -> 282,
+    960 of 24 121 -> 116, 928 of 15.6 81 -> 76, 1024 of 16 84 -> 82, of 10 58 -> 60."""
+    jobs = total_tiles * qo_heads
+    if (jobs < 3072 and not 896 <= jobs <= 1024) or qo_heads // kv_heads % 2:
+        return False
+    tiles = float(((seqlens_q + 127) // 128 * (seqlens_k - 0.5 * seqlens_q + 64)).sum()) / 64  # of keys, over the q tiles
+    return tiles >= 15 * total_tiles
+
+
 def prefill_ranges_workspace_bytes(jobs: int) -> int:
     """`jobs`: q tiles x heads x ranges (`prefill_ranges` makes at most 800 of a launch, 54 MB)."""
     return int(lib().msgl_attn_prefill_ranges_workspace_bytes(jobs, 1, 1))
@@ -447,15 +465,17 @@ def attn_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_ca
                  page_table: torch.Tensor, req_rows: Optional[torch.Tensor], seq_lens: torch.Tensor,
                  cu_seqlens_q: torch.Tensor, tile_cu: torch.Tensor, batch: int, total_tiles: int,
                  sm_scale: float, tile_order: Optional[torch.Tensor] = None, impl: Optional[int] = None,
-                 ranges: Tuple[int, int] = (1, 0), workspace: Optional[torch.Tensor] = None) -> None:
+                 ranges: Tuple[int, int] = (1, 0), workspace: Optional[torch.Tensor] = None, pairs: bool = False) -> None:
     """tile_order: optional int32 [total_tiles] schedule of the q tiles (heaviest first); impl: None = process default
     (PREFILL_IMPL), 0 = 4 the DMA-staged kernel, 2 its register-staged predecessor (include/msgl_hip.h; anything else is
     refused by the library).  tile_cu / total_tiles / tile_order are in units of prefill_q_tile(impl) query rows.
     ranges: (key ranges of a q tile at most, 64-key tiles of each) for the DMA-staged kernel, see `prefill_ranges`; more than one needs a
-    workspace of prefill_ranges_workspace_bytes."""
+    workspace of prefill_ranges_workspace_bytes.  pairs: two heads a workgroup where that kernel runs without ranges, see `prefill_pairs`."""
     _need_cuda(out, q, k_cache, v_cache, page_table, seq_lens, cu_seqlens_q, tile_cu)
     if impl is None:
         impl = PREFILL_IMPL
+    if pairs and ranges[0] == 1 and int(impl) in (0, 4):
+        impl = 6
     if tile_order is not None:
         _need_cuda(tile_order)
         assert tile_order.dtype == torch.int32 and tile_order.is_contiguous() and tile_order.numel() == total_tiles

@@ -253,6 +253,24 @@ def test_prefill_key_ranges(ops, dev, monkeypatch, hq, hkv, specs, ranges, dtype
         at += n
 
 
+@pytest.mark.parametrize("hq,hkv,specs,dtype", [
+    (2, 1, [(0, 1)], torch.bfloat16),                                          # one row, one pair
+    (16, 8, [(0, n) for n in (5, 31, 33, 64, 127, 129, 300)], torch.bfloat16),  # one tile, odd and even chains, waves without rows
+    (6, 1, [(0, 129), (700, 701), (63, 192)], torch.float16),                  # three pairs of a kv head, a short portion after a long one
+    (64, 8, [(1000, 1600)], torch.bfloat16),                                   # more workgroups than compute units
+])
+def test_prefill_heads_in_pairs(ops, dev, monkeypatch, hq, hkv, specs, dtype):
+    """Two heads a workgroup: the bits of one head a workgroup, which the oracle's tests pin; an odd group is refused."""
+    c = build(torch.Generator().manual_seed(17), specs, hq, hkv, 16, dtype)
+    whole = run(ops, dev, c)
+    plain = ops.attn_prefill
+    monkeypatch.setattr(ops, "attn_prefill", lambda *a, **k: plain(*a, **k, pairs=True))
+    for order in ("heavy", "reversed", None):
+        assert torch.equal(run(ops, dev, c, order=order), whole)
+    with pytest.raises(RuntimeError, match="pairs"):
+        run(ops, dev, build(torch.Generator().manual_seed(18), [(0, 5)], 5, 1, 16, dtype))
+
+
 def test_prompt_attention_leaves_the_decode_workspace_alone(ops, dev):
     """Prompts and decode steps of one backend on different streams share no scratch: the sums of key ranges live in memory of their own."""
     from mini_sglang_amd.attention import HipAttnBackend
