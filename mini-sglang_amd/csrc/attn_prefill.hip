@@ -453,7 +453,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 // with a part left out: all copies but the first 4330, no exponentials 5025, no rescale 5200, none of exponentials, rescale and mask 4930; the scores
 // of the next tile in the same wave beside a tile's weights: 5290.  A wave's tile is 1024 cycles of the matrix cores and about as many of the vector
 // units (32 scores a lane, the exponential 16 cycles each).  5240 us with one head a workgroup, 4940 with two (1110 TFLOP/s); 40 heads on 8, 29 requests
-// of 100 - 1024 tokens: 234.  (Sums of the rounded weights, one instruction a pair: 0.5 % faster, and 2^-9 of a row's weight off.)
+// of 100 - 1024 tokens: 234, and with Q and the outputs in whole rows by way of LDS (one head a workgroup; on a slower card 249 -> 240, 60 requests of
+// 128 - 256 tokens 129 -> 122): starts and outputs are half of such a launch (empty workgroups 14 us, requests and outputs 41, the first tile 48).  (Sums of the rounded weights, one instruction a pair: 0.5 % faster, and 2^-9 of a row's weight off.)
 // HEADS = 2: eight waves, two heads of a kv head beside each other over the same tiles: half the copies.  One workgroup a CU then, so nothing runs
 // under its start, and the last round is coarser: for many long chains of tiles (the rule and its other side: ops.prefill_pairs).
 // RANGES: workgroup (.., z) takes the tiles z * run .. of the job's keys; sums of more than one range go to attn_prefill_join_kernel in fp32, in
@@ -507,10 +508,9 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
 
   const int my_q = q0 + rows * 32 + (lane & 31);
   const bool q_valid = my_q < q_len;
-  const int64_t q_tok = q_begin + (q_valid ? my_q : q_len - 1);
   U4 qf[8];
-  {
-    const uint16_t* qp = p.q + q_tok * p.q_stride + (int64_t)hq * kD + hi * 8;
+  if constexpr (HEADS == 2) {
+    const uint16_t* qp = p.q + (int64_t)(q_begin + (q_valid ? my_q : q_len - 1)) * p.q_stride + (int64_t)hq * kD + hi * 8;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) qf[ks] = ldg16(qp + ks * 16);
   }
@@ -715,7 +715,22 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
   if (t0 < ntiles) {
     load_slots(t0);
     issue_dma(lds_a);
+    if (HEADS == 2 && t0 + 1 < ntiles) load_slots(t0 + 1);
+  }
+  if constexpr (HEADS == 1) {
+    // Q's rows by the DMA path too, into the image that is free until the first tile's barrier, a wave's own 32: whole rows, where a load of a
+    // lane's own pieces touches 32 rows.  (With two heads the image would hold half of them.)
+    char* mine = lds_b + wave * 8192;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 4 * i + (lane >> 4), q_row = min(q0 + rows * 32 + r, q_len - 1);
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(p.q + (int64_t)(q_begin + q_row) * p.q_stride + (int64_t)hq * kD + (((lane & 15) ^ (r & 15)) << 3)),
+                                       (lds_void_t*)(mine + i * 1024), 16, 0, 0);
+    }
     if (t0 + 1 < ntiles) load_slots(t0 + 1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const U4*>(mine + (lane & 31) * 256 + (((2 * ks + hi) ^ (lane & 15)) << 4));
   }
   for (int kt = t0; kt < ntiles; kt += 2) {
     tile_body(std::integral_constant<int, 0>{}, kt);
@@ -731,20 +746,34 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
     *reinterpret_cast<float2*>(p.part_ml + (at * 64 + lane) * 2) = make_float2(m_run, l_run);
     return;
   }
-  if (q_valid) {
-    const float inv = 1.0f / l_run;
+  const float inv = 1.0f / l_run;
+  auto piece = [&](int nb, int rg) __attribute__((always_inline)) {  // columns 32 nb + 8 rg + 4 hi .. + 3 of the lane's row
+    return uint2{Elem<T>::pack(o[nb][4 * rg] * inv, o[nb][4 * rg + 1] * inv), Elem<T>::pack(o[nb][4 * rg + 2] * inv, o[nb][4 * rg + 3] * inv)};
+  };
+  if constexpr (HEADS == 1) {
+    // Outputs by way of the image that does not hold the last tile (everyone is done with it), a wave's rows in its own part: whole rows of 256
+    // bytes leave it, where a lane's own pieces are 16 bytes of 32 rows a store.  16-byte pieces change places by the row's number.
+    char* turn = (((ntiles - t0) & 1) ? lds_b : lds_a) + wave * 8192;
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg)
+        *reinterpret_cast<uint2*>(turn + (lane & 31) * 256 + (((nb * 4 + rg) ^ (lane & 15)) << 4) + 8 * hi) = piece(nb, rg);
+    asm volatile("" ::: "memory");  // a wave's own part: its LDS operations keep their order
+    const int first = q0 + rows * 32, left = q_len - first;
+    uint16_t* op = p.out + (int64_t)(q_begin + first) * p.out_stride + (int64_t)hq * kD + (lane & 31) * 4;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = 2 * i + hi;
+      const uint2 w = *reinterpret_cast<const uint2*>(turn + r * 256 + ((((lane & 31) >> 1) ^ (r & 15)) << 4) + 8 * (lane & 1));
+      if (r < left) *reinterpret_cast<uint2*>(op + (int64_t)r * p.out_stride) = w;
+    }
+  } else if (q_valid) {
     uint16_t* op = p.out + (int64_t)(q_begin + my_q) * p.out_stride + (int64_t)hq * kD;
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
+    for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const int d = nb * 32 + 8 * rg + 4 * hi;
-        uint2 w;
-        w.x = Elem<T>::pack(o[nb][4 * rg + 0] * inv, o[nb][4 * rg + 1] * inv);
-        w.y = Elem<T>::pack(o[nb][4 * rg + 2] * inv, o[nb][4 * rg + 3] * inv);
-        *reinterpret_cast<uint2*>(op + d) = w;
-      }
-    }
+      for (int rg = 0; rg < 4; ++rg) *reinterpret_cast<uint2*>(op + nb * 32 + 8 * rg + 4 * hi) = piece(nb, rg);
   }
 }
 
