@@ -453,8 +453,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 // with a part left out: all copies but the first 4330, no exponentials 5025, no rescale 5200, none of exponentials, rescale and mask 4930; the scores
 // of the next tile in the same wave beside a tile's weights: 5290.  A wave's tile is 1024 cycles of the matrix cores and about as many of the vector
 // units (32 scores a lane, the exponential 16 cycles each).  5240 us with one head a workgroup, 4940 with two (1110 TFLOP/s); 40 heads on 8, 29 requests
-// of 100 - 1024 tokens: 234, and with Q and the outputs in whole rows by way of LDS (one head a workgroup; on a slower card 249 -> 240, 60 requests of
-// 128 - 256 tokens 129 -> 122): starts and outputs are half of such a launch (empty workgroups 14 us, requests and outputs 41, the first tile 48).  (Sums of the rounded weights, one instruction a pair: 0.5 % faster, and 2^-9 of a row's weight off.)
+// of 100 - 1024 tokens: 234, and with Q and the outputs in whole rows by way of LDS (one head a workgroup; on a slower card 249 -> 240, 60 requests
+// of 128 - 256 tokens 129 -> 122): starts and outputs are half of such a launch (empty workgroups 14 us, requests and outputs 41, the first tile
+// 48).  (Sums of the rounded weights, one instruction a pair: 0.5 % faster, and 2^-9 of a row's weight off.)
 // HEADS = 2: eight waves, two heads of a kv head beside each other over the same tiles: half the copies.  One workgroup a CU then, so nothing runs
 // under its start, and the last round is coarser: for many long chains of tiles (the rule and its other side: ops.prefill_pairs).
 // RANGES: workgroup (.., z) takes the tiles z * run .. of the job's keys; sums of more than one range go to attn_prefill_join_kernel in fp32, in
