@@ -297,6 +297,31 @@ def test_prompt_attention_leaves_the_decode_workspace_alone(ops, dev):
     assert torch.isfinite(out).all() and bool((backend._workspace == 0x5A).all())
 
 
+@pytest.mark.parametrize("hq,hkv,new,pairs", [(64, 8, 2048, True), (64, 8, 1900, True), (64, 8, 1700, False), (40, 8, 3072, False)])
+def test_backend_pairs_heads_by_its_rule(ops, dev, hq, hkv, new, pairs):
+    """Heads go in pairs where a launch has 896 to 1024 chains of 15 tiles and more on average and a kv head an even number of heads; the bits are the other launch's."""
+    from mini_sglang_amd.attention import HipAttnBackend
+    from mini_sglang_amd.core import Batch, Context, Req
+    from mini_sglang_amd.kvcache import create_kvcache_pool
+    from mini_sglang_amd.model import ModelConfig
+
+    ctx = Context(16)
+    m = ModelConfig(num_layers=1, num_qo_heads=hq, num_kv_heads=hkv, head_dim=128, hidden_size=1024, vocab_size=64, intermediate_size=64)
+    ctx.page_table = torch.arange(3328, dtype=torch.int32, device=dev).view(1, 3328)
+    ctx.kv_cache = create_kvcache_pool(m, 208, 16, torch.bfloat16, dev)
+    backend = HipAttnBackend(m, ctx)
+    batch = Batch(reqs=[Req(input_ids=torch.zeros(new, dtype=torch.int32), table_idx=0, cached_len=0, output_len=1, uid=0)], phase="prefill")
+    batch.out_loc = torch.arange(new, dtype=torch.int32, device=dev)
+    batch.padded_reqs = batch.reqs
+    backend.prepare_metadata(batch)
+    md = batch.attn_metadata
+    assert md.pairs == pairs and md.ranges[0] == 1
+    q, k, v = (torch.randn(new, h * 128, device=dev).bfloat16() for h in (hq, hkv, hkv))
+    out = backend.forward(q.view(new, hq, 128), k, v, 0, batch)
+    md.pairs = False
+    assert torch.equal(out, backend.forward(q.view(new, hq, 128), k, v, 0, batch))
+
+
 def test_a_small_decode_capacity_holds_the_small_batch_kernel(ops, dev):
     """The decode workspace is at least what small batches take, whatever number of pieces the caller asks for."""
     from mini_sglang_amd.attention import HipAttnBackend
