@@ -96,7 +96,7 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
       for (int kc = 0; kc < KC; ++kc) {
         const int k = kc * 32 + lg * 8;
         Q4 f{0u, 0u, 0u, 0u};
-        if (FULL) f = *reinterpret_cast<const Q4*>(qrow + 4 * j * d + k);  // a row that is none sees no key
+        if (FULL) f = *reinterpret_cast<const Q4*>(qrow + 4 * j * d + k);  // a row that is none takes the first one's queries; its sums go nowhere
         else if (there && k < d) f = load8(qrow + 4 * j * d + k, d - k, qvec != 0);
         qf[j][kc] = __builtin_bit_cast(bf16x8_t, f);
       }
@@ -246,10 +246,10 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
     tmax = pair_max(tmax);
     request_keys(2);
     // The reference maximum may lag by 2^8: the weights' three parts have their 24 bits wherever these lie (rescaling O at every new maximum was
-    // a quarter of the vector work)
+    // a quarter of the vector work).  A row's moves for its own scores only: its bits do not depend on the wave's other rows.
     if (__builtin_amdgcn_ballot_w64(tmax > m + 8.f) != 0) {
-      const float m_new = fmaxf(m, tmax);
-      const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
+      const float m_new = tmax > m + 8.f ? tmax : m;
+      const float alpha = m_new == m ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
 #pragma unroll
       for (int nb = 0; nb < VC / 2; ++nb)
 #pragma unroll

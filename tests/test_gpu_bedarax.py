@@ -286,6 +286,36 @@ def test_window_rising_scores(dev, H, G, shift, step, splits):
     assert bool((diff <= 2.0 ** -8 * ref.abs() + 2.0 ** -14 * ref.abs().max()).all()), float(diff.max())
 
 
+@pytest.mark.parametrize("splits", [1, 2], ids=["one-range", "two-ranges"])
+@pytest.mark.parametrize("H,G,d", [(16, 4, 128), (16, 1, 64), (8, 2, 128)])
+def test_window_rows_keep_to_themselves(dev, H, G, d, splits):
+    """Scores that rise slowly, so that a row's reference lags behind its maximum: neither a neighbouring head's nor a neighbouring token's scores, rising fast,
+    change a bit of the other rows."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(H + d)
+    c, n = 61, 512
+    k, v = torch.randn(n + c, G, d, generator=g) * 0.1, torch.randn(n + c, G, d, generator=g).bfloat16()
+    k[..., 0] = torch.arange(n + c)[:, None] * 0.02
+    src = torch.randn(n, H * d + H, generator=g)
+    src[:, : H * d].view(n, H, d)[..., 0] = 1.0
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    caches, table = (k.bfloat16().view(n + c, -1).to(dev), v.view(n + c, -1).to(dev)), torch.arange(n + c, dtype=torch.int32, device=dev)[None]
+
+    def attend(heads, tokens):
+        x = src.clone()
+        x[:, : H * d].view(n, H, d)[tokens, heads, 0] = 15.0
+        out = torch.empty((n, H * d), dtype=torch.bfloat16, device=dev)
+        mixops.window_attn(out, x.bfloat16().to(dev), H * d, *caches, table, i32([0]), i32([n + c]), i32([0, n]), 1, H, G, d, d, 0, 1.0, torch.eye(H, device=dev), splits=splits)
+        return out.view(n, H, d)
+
+    everyone, quiet = slice(None), attend(slice(0), slice(None))
+    by_head, by_token = attend(slice(0, None, 2), everyone), attend(everyone, slice(0, None, 3))
+    assert torch.equal(by_head[:, 1::2], quiet[:, 1::2]) and not torch.equal(by_head[:, ::2], quiet[:, ::2])
+    others = [t for t in range(n) if t % 3]
+    assert torch.equal(by_token[others], quiet[others])
+
+
 @pytest.mark.parametrize("B", [64, 65, 150])
 @pytest.mark.parametrize("splits", [1, 3])
 @pytest.mark.parametrize("most", [1, 40], ids=["decode", "portions"])
