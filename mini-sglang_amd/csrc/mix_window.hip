@@ -37,7 +37,7 @@ constexpr int kWinHead = 16 * kWinRow + 4;  // floats of a head: four of them ap
 //   Q K^T with rows (head of four, query of four), mixed scores as their product with the table over the heads
 //   mixed scores to LDS; the waves share the heads, 32 rows (two heads of 16 queries): mask, online softmax, O^T += V^T P^T (a lane reads
 //   four consecutive keys of its row, the layout the product takes; V through transposing LDS reads).  Meanwhile the next rows arrive.
-// FULL: heads of 128 and queries that 16-byte loads may read
+// FULL: heads of 128
 template <int NH, int G, bool FULL>
 __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
                                                                   const bf16_t* __restrict__ src, int64_t ld_src, int g_off,
@@ -45,7 +45,7 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
                                                                   const int* __restrict__ table, int64_t table_stride,
                                                                   const int* __restrict__ req_rows, const int* __restrict__ seq_lens,
                                                                   const int* __restrict__ cu_q, int B, int total_q, int d, int dv,
-                                                                  int window, float scale, const float* __restrict__ talk, int splits, int qvec) {
+                                                                  int window, float scale, const float* __restrict__ talk, int splits) {
   constexpr int HPW = 2, NT = NH * 32, NW = NH / 2, KC = kWinKC, VC = kWinVC, NJ = NH / 4, KSW = 8 / NW;
   constexpr int RS = G * KC * 32;  // a row of keys or values in LDS
   // objects of their own: the compiler then knows which reads do not meet a DMA under way
@@ -85,21 +85,21 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
   float tk[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) tk[j] = lr < NH ? talk[lr * NH + 4 * j + lg] * scale2 : 0.f;
-  bf16x8_t qf[NJ][KC];  // row 4 (head of four) + (query of four)
+  bf16x8_t qf[NJ][KC];  // row 4 (head of four) + (query of four); a row that is none takes the first one's queries, its sums go nowhere
   {
     const int t = tok0 + 4 * quad + (lr & 3);
-    const bool there = t < q_len;
-    const bf16_t* qrow = src + (size_t)(cu_q[b] + (there ? t : tok0)) * (size_t)ld_src + (size_t)(lr >> 2) * d;
+    const bf16_t* qrow = src + (size_t)(cu_q[b] + (t < q_len ? t : tok0)) * (size_t)ld_src + (size_t)(lr >> 2) * d;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j)
+    for (int kc = 0; kc < KC; ++kc) {
+      const int k = kc * 32 + lg * 8;
+      // 16 bytes from where they lie, whatever the rows' stride: global memory takes any alignment (12 tokens, unaligned: 16.6 us, number by number
+      // 31.5).  Past the head its last piece for now: a lane's condition on a load would be a wait for it.
 #pragma unroll
-      for (int kc = 0; kc < KC; ++kc) {
-        const int k = kc * 32 + lg * 8;
-        Q4 f{0u, 0u, 0u, 0u};
-        if (FULL) f = *reinterpret_cast<const Q4*>(qrow + 4 * j * d + k);  // a row that is none takes the first one's queries; its sums go nowhere
-        else if (there && k < d) f = load8(qrow + 4 * j * d + k, d - k, qvec != 0);
-        qf[j][kc] = __builtin_bit_cast(bf16x8_t, f);
+      for (int j = 0; j < NJ; ++j) {
+        qf[j][kc] = bf16x8_t{};
+        if (FULL || kc * 32 < d) __builtin_memcpy(&qf[j][kc], qrow + 4 * j * d + (FULL ? k : min(k, d - 8)), 16);
       }
+    }
   }
   // this lane's row of the second product: head h0 + (lane >> 4 & 1), query lr
   f32x16_t o[VC / 2];
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
     for (int e = 0; e < 16; ++e) o[nb][e] = 0.f;
   float m = -INFINITY, lsum = 0.f;
   const uint32_t nk = (uint32_t)(G * d), nv = (uint32_t)(G * dv);
-  // 16-byte pieces of a tile's key and value rows (both 128 wide per head in LDS, zeros past the head).  A row's pieces divide the workgroup
+  // 16-byte pieces of a tile's key and value rows (both 128 wide per head in LDS).  A row's pieces divide the workgroup
   // (both are powers of two), so a thread has one column of the rows key0, key0 + ROWS, ...: its offsets are known once (a division and four
   // 32-bit products a piece and tile, at a quarter of the rate, were a tenth of the kernel).
   static_assert(KC * 4 == VC * 2, "keys and values share the piece map");
@@ -154,14 +154,14 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
         if (j0 + key >= k_end) *reinterpret_cast<Q4*>(img + (key * PCS + (int)threadIdx.x % PCS) * 8) = Q4{0u, 0u, 0u, 0u};
     }
   };
-  // zeros past the heads, where no DMA goes
-  auto clear = [&](uint16_t* img, bool keys) __attribute__((always_inline)) {
-    for (int key = key0; !FULL && key < kWinTile; key += ROWS)
-      if (keys ? 8 * ((piece ^ key) & 15) >= d : 8 * cv >= dv) *reinterpret_cast<Q4*>(img + (key * PCS + (int)threadIdx.x % PCS) * 8) = Q4{0u, 0u, 0u, 0u};
-  };
-  clear(sk, true);
-  clear(sv1, true);
-  clear(sv0, false);
+  // Zeros past the heads of keys, where no DMA goes.  (Values there are whatever LDS holds: their columns of O are not stored.)
+  if (!FULL) {
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int at = (u * NT + (int)threadIdx.x) * 8;
+      if (8 * (u & 1 ? ck1 : ck0) >= d) *reinterpret_cast<Q4*>(sk + at) = *reinterpret_cast<Q4*>(sv1 + at) = Q4{0u, 0u, 0u, 0u};
+    }
+  }
   // mixed scores of an image's tile
   f32x4_t mx[KSW][4];
   auto scores = [&](const uint16_t* img) __attribute__((always_inline)) {
@@ -205,11 +205,18 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
 #pragma unroll
   for (int u = 0; u < NP; ++u) request_v(sv0, slots_v, u);
   arrived(sv0, k_begin);
+  if (!FULL) {  // zeros past the head
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc)
+      if (kc * 32 + lg * 8 >= d) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) qf[j][kc] = bf16x8_t{};
+      }
+  }
   __syncthreads();
   scores(sv1);
   put_scores();
   __syncthreads();
-  clear(sv1, false);
   // tile t: the next one's keys are there, its values and the keys of the one after it are asked for
   auto tile = [&](uint16_t* cur, uint16_t* next, int t) __attribute__((always_inline)) {
     const int j0 = k_begin + t * TW, nj = j0 + TW, buf = t & 3;
@@ -371,13 +378,12 @@ extern "C" __attribute__((visibility("hidden"))) int mix_window_attn_mfma(
   const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   if (!msgl_mix_window_attn_on_matrix_cores(H, G, d, dv, MSGL_MIX_BF16)) return 0;
   if (!al(k_cache) || !al(v_cache) || !al(out) || (part_o && !al(part_o))) return 0;
-  const int qvec = al(src) && ld_src % 8 == 0;
   const dim3 grid(total_q / 16 + batch, splits);
-#define WIN_KERNEL(NH, G) (d == 128 && dv == 128 && qvec ? window_attn_mfma_kernel<NH, G, true> : window_attn_mfma_kernel<NH, G, false>)
+#define WIN_KERNEL(NH, G) (d == 128 && dv == 128 ? window_attn_mfma_kernel<NH, G, true> : window_attn_mfma_kernel<NH, G, false>)
   const auto kernel = H == 16 ? (G == 4 ? WIN_KERNEL(16, 4) : G == 2 ? WIN_KERNEL(16, 2) : WIN_KERNEL(16, 1)) : G == 2 ? WIN_KERNEL(8, 2) : WIN_KERNEL(8, 1);
 #undef WIN_KERNEL
   hipLaunchKernelGGL(kernel, grid, dim3(H * 32), 0, s, mp<bf16_t>(out), part_o, part_ml, cp<bf16_t>(src), ld_src, g_off, cp<bf16_t>(k_cache),
-                     cp<bf16_t>(v_cache), table, table_stride, req_rows, seq_lens, cu_q, batch, total_q, d, dv, window, scale, talk, splits, qvec);
+                     cp<bf16_t>(v_cache), table, table_stride, req_rows, seq_lens, cu_q, batch, total_q, d, dv, window, scale, talk, splits);
   MIX_LAUNCHED("window_attn");
   return 1;
 }

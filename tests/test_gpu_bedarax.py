@@ -316,6 +316,33 @@ def test_window_rows_keep_to_themselves(dev, H, G, d, splits):
     assert torch.equal(by_token[others], quiet[others])
 
 
+@pytest.mark.parametrize("shift,gap", [(1, 0), (4, 1), (0, 6)])
+@pytest.mark.parametrize("H,G,d,dv", [(16, 4, 128, 128), (16, 2, 64, 128), (8, 1, 40, 16), (8, 2, 8, 8)])
+def test_window_queries_at_any_address(dev, H, G, d, dv, shift, gap):
+    """Queries at addresses and row strides of no alignment: the bits of aligned ones, which test_window_matrix_cores pins.  Neither what lies behind a head's
+    columns nor the rows' gap is looked at."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(H + d)
+    new, old = [1, 19, 32], [40, 0, 7]
+    T, L, width = sum(new), [a + b for a, b in zip(new, old)], H * d + H
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    k, v = torch.randn(sum(L), G * d, generator=g).bfloat16().to(dev), torch.randn(sum(L), G * dv, generator=g).bfloat16().to(dev)
+    table = torch.zeros(3, max(L), dtype=torch.int32)
+    for b, n in enumerate(L):
+        table[b, :n] = torch.arange(sum(L[:b]), sum(L[:b]) + n)
+    src = torch.randn(T, width, generator=g).bfloat16()
+    outs = []
+    for at, stride in ((0, -(-width // 8) * 8), (shift, -(-width // 8) * 8 + gap)):
+        room = torch.full((at + T * stride,), float("nan"), dtype=torch.bfloat16, device=dev)
+        rows = room[at:].view(T, stride)[:, :width]
+        rows.copy_(src)
+        out = torch.empty((T, H * dv), dtype=torch.bfloat16, device=dev)
+        mixops.window_attn(out, rows, H * d, k, v, table.to(dev), i32([0, 1, 2]), i32(L), i32([0, 1, 20, 52]), 3, H, G, d, dv, 24, d ** -0.5, torch.eye(H, device=dev) + 0.1)
+        outs.append(out)
+    assert bool(torch.isfinite(outs[0]).all()) and torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("B", [64, 65, 150])
 @pytest.mark.parametrize("splits", [1, 3])
 @pytest.mark.parametrize("most", [1, 40], ids=["decode", "portions"])
