@@ -70,6 +70,7 @@ struct PrefillParams {
   int batch, hq, group;
   int share_log2, per;  // XCDs that share their kv heads, kv heads of each
   int stretch;     // workgroups of an XCD where each takes a stretch of the list, or 0
+  int few;         // q tiles of fewer rows load and store by lanes' own pieces
   int ranges, run;  // key ranges, and tiles of each (the last one: what is left)
   float *part_o, *part_ml;
   float scale_log2;
@@ -510,13 +511,15 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
   const int my_q = q0 + rows * 32 + (lane & 31);
   const bool q_valid = my_q < q_len;
   U4 qf[8];
-  if constexpr (HEADS == 2) {
+  const bool own_pieces = HEADS == 2 || q_len - q0 < p.few;  // a lane loads and stores its own pieces of its row
+  if (own_pieces) {
     const uint16_t* qp = p.q + (int64_t)(q_begin + (q_valid ? my_q : q_len - 1)) * p.q_stride + (int64_t)hq * kD + hi * 8;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) qf[ks] = ldg16(qp + ks * 16);
   }
   const int my_qpos = diag + my_q;
-  const int wave_min_qpos = diag + q0 + rows * 32;  // scalar
+  const int left = q_len - (q0 + rows * 32);  // this wave's rows, 32 of them at most
+  const int wave_min_qpos = left > 0 ? diag + q0 + rows * 32 : -kKTile;  // scalar; no row: no tile
 
   f32x16 o[4];
 #pragma unroll
@@ -716,17 +719,20 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
   if (t0 < ntiles) {
     load_slots(t0);
     issue_dma(lds_a);
-    if (HEADS == 2 && t0 + 1 < ntiles) load_slots(t0 + 1);
+    if (own_pieces && t0 + 1 < ntiles) load_slots(t0 + 1);
   }
-  if constexpr (HEADS == 1) {
+  if (!own_pieces) {
     // Q's rows by the DMA path too, into the image that is free until the first tile's barrier, a wave's own 32: whole rows, where a load of a
-    // lane's own pieces touches 32 rows.  (With two heads the image would hold half of them.)
+    // lane's own pieces touches 32 rows.  (With two heads the image would hold half of them.)  Tiles of few rows have few to touch, and the way
+    // through LDS and back is 0.4 us of a workgroup: not where it is all of a launch's time.
     char* mine = lds_b + wave * 8192;
+    if (left > 0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int r = 4 * i + (lane >> 4), q_row = min(q0 + rows * 32 + r, q_len - 1);
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(p.q + (int64_t)(q_begin + q_row) * p.q_stride + (int64_t)hq * kD + (((lane & 15) ^ (r & 15)) << 3)),
-                                       (lds_void_t*)(mine + i * 1024), 16, 0, 0);
+      for (int i = 0; i < 8; ++i) {
+        const int r = 4 * i + (lane >> 4), q_row = min(q0 + rows * 32 + r, q_len - 1);
+        __builtin_amdgcn_global_load_lds((glb_void_t*)(p.q + (int64_t)(q_begin + q_row) * p.q_stride + (int64_t)hq * kD + (((lane & 15) ^ (r & 15)) << 3)),
+                                         (lds_void_t*)(mine + i * 1024), 16, 0, 0);
+      }
     }
     if (t0 + 1 < ntiles) load_slots(t0 + 1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -751,7 +757,8 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
   auto piece = [&](int nb, int rg) __attribute__((always_inline)) {  // columns 32 nb + 8 rg + 4 hi .. + 3 of the lane's row
     return uint2{Elem<T>::pack(o[nb][4 * rg] * inv, o[nb][4 * rg + 1] * inv), Elem<T>::pack(o[nb][4 * rg + 2] * inv, o[nb][4 * rg + 3] * inv)};
   };
-  if constexpr (HEADS == 1) {
+  if (left <= 0) return;
+  if (!own_pieces) {
     // Outputs by way of the image that does not hold the last tile (everyone is done with it), a wave's rows in its own part: whole rows of 256
     // bytes leave it, where a lane's own pieces are 16 bytes of 32 rows a store.  16-byte pieces change places by the row's number.
     char* turn = (((ntiles - t0) & 1) ? lds_b : lds_a) + wave * 8192;
@@ -761,8 +768,7 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
       for (int rg = 0; rg < 4; ++rg)
         *reinterpret_cast<uint2*>(turn + (lane & 31) * 256 + (((nb * 4 + rg) ^ (lane & 15)) << 4) + 8 * hi) = piece(nb, rg);
     asm volatile("" ::: "memory");  // a wave's own part: its LDS operations keep their order
-    const int first = q0 + rows * 32, left = q_len - first;
-    uint16_t* op = p.out + (int64_t)(q_begin + first) * p.out_stride + (int64_t)hq * kD + (lane & 31) * 4;
+    uint16_t* op = p.out + (int64_t)(q_begin + q0 + rows * 32) * p.out_stride + (int64_t)hq * kD + (lane & 31) * 4;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int r = 2 * i + hi;
@@ -899,6 +905,10 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   MSGL_REQUIRE(total < (1ll << 30), "attn_prefill: %lld workgroups", (long long)total);
   const int even = (int)(((int64_t)total_tiles * p.group * p.per + (1 << p.share_log2) - 1) >> p.share_log2);
   p.stretch = ranges == 1 && total <= 256 ? even : 0;
+  // Where all workgroups start at once the time is one workgroup's, and only full tiles go in whole rows by way of LDS; else from half a tile on.
+  // us, 8 requests of n tokens, own pieces / whole rows: 16 heads on 8 (128 workgroups) of 32 7.5 / 8.3, 64 8.8 / 9.0, 100 10.9 / 11.4, 128 11.8 /
+  // 11.9; 40 requests, 40 on 8 (1600): of 20 20.5 / 22.5, 40 26.4 / 27.4, 64 30.8 / 29.9, 100 42.3 / 40.3, 128 48.8 / 43.7
+  p.few = total * ranges <= 512 ? kQTile : kQTile / 2;
   const unsigned blocks = (unsigned)even * 8;
   if (ranges > 1) {
     p.ranges = ranges;
