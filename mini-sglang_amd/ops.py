@@ -442,18 +442,22 @@ def prefill_ranges(total_tiles: int, qo_heads: int, max_seqlen_q: int, max_seqle
 def prefill_pairs(total_tiles: int, qo_heads: int, kv_heads: int, seqlens_q: np.ndarray, seqlens_k: np.ndarray) -> bool:
     """Whether a launch without key ranges takes two heads of a kv head a workgroup: half the copies, and one workgroup a CU.
 
-    The copies are what this saves, 6 % of a long tile chain; a workgroup's start is no longer under another one's tiles, and the last round of
-    workgroups is a coarser one.  us, one head -> two (q tiles x heads; mean 64-key tiles of each):
-      4096 of 324  5240 -> 4940    4224 of 26  525 -> 512    3072 of 15.8  226 -> 223    4096 of 12.9  271 -> 264    4096 of 11  232 -> 235
-      3904 of 8.6  185 -> 190      4096 of 3   110 -> 119
-    Fewer than six rounds of the 512 places win or lose by how full the last one is (2688 of 26 340 -> 342, 1408 of 26 177 -> 169, 1088 of
-    26 149 -> 166, 640 of 26 100 -> 112, 512 of 33 108 -> 121), but two rounds nearly full win: 896 of 26 120 -> 111, 1024 of 65 315 -> 282,
-    960 of 24 121 -> 116, 928 of 15.6 81 -> 76, 1024 of 16 84 -> 82, of 10 58 -> 60."""
+    The copies are what this saves, 6 % of a long tile chain; a workgroup's start is no longer under another one's tiles, and there are 256 places of
+    double work instead of 512.  us, one head -> two (q tiles x heads; mean 64-key tiles of each):
+      six rounds of 512 and more, from 36 tiles on: 4992 of 241 5181 -> 4889    4128 of 45 852 -> 835    3520 of 45 751 -> 724    3072 of 38 541 -> 532
+        3648 of 38 663 -> 666; below, the starts decide: 4032 of 33 619 -> 625    3840 of 25 471 -> 477    6144 of 16 476 -> 511    4704 of 14 349 -> 383
+      two rounds nearly full, from 15 tiles on: 1024 of 169 746 -> 702    896 of 29 141 -> 127    1024 of 17 94 -> 87    960 of 15 82 -> 75
+        960 of 9 59 -> 64; the longest chain (tiles) within 1.25 of what a place has on average: 912 of 20 (46) 106 -> 102, but 912 of 43 (106) 195 -> 211,
+        968 of 29 (75) 152 -> 157, 920 of 15 (40) 83 -> 86
+      between them it goes either way with the last round and the mix of chains, by up to 7 %: 1408 of 170 1020 -> 956, 1920 of 31 282 -> 270, 1216 of 76
+        424 -> 442, 2208 of 22 251 -> 261"""
     jobs = total_tiles * qo_heads
     if (jobs < 3072 and not 896 <= jobs <= 1024) or qo_heads // kv_heads % 2:
         return False
     tiles = float(((seqlens_q + 127) // 128 * (seqlens_k - 0.5 * seqlens_q + 64)).sum()) / 64  # of keys, over the q tiles
-    return tiles >= 15 * total_tiles
+    if jobs >= 3072:
+        return tiles >= 36 * total_tiles
+    return tiles >= 15 * total_tiles and -(-int(seqlens_k.max()) // 64) <= 1.25 * tiles * qo_heads / 512
 
 
 def prefill_ranges_workspace_bytes(jobs: int) -> int:

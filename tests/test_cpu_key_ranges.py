@@ -126,3 +126,26 @@ def test_delta_rule_pieces_where_the_token_loop_takes_long_portions(monkeypatch)
             if want:
                 items, first, count = md.delta_chunks
                 assert count == 4 and items.view(-1, 3).tolist() == [[0, 0, 1], [1, 0, n // 2], [1, n // 2, n], [2, 0, 7]] and first.tolist() == [0, 1, 3, 4]
+
+
+def test_prefill_heads_go_in_pairs_by_length_of_chains():
+    """Two heads a workgroup: the rule's both bands, their lines in number of chains, mean length, longest one and group."""
+    import numpy as np
+
+    from mini_sglang_amd import ops
+
+    def pairs(hq, hkv, *portions):  # portions: (requests, new tokens, tokens before them)
+        q = np.array([n for c, n, _ in portions for _ in range(c)], dtype=np.int64)
+        k = np.array([n + o for c, n, o in portions for _ in range(c)], dtype=np.int64)
+        return ops.prefill_pairs(int(((q + 127) // 128).sum()), hq, hkv, q, k)
+
+    # from 3072 chains on, 36 tiles on average
+    assert pairs(64, 8, (1, 8192, 16384)) and pairs(64, 8, (1, 6144, 0)) and pairs(32, 16, (3, 4300, 2000)) and pairs(8, 1, (12, 4096, 1000))
+    assert not pairs(64, 8, (1, 6016, 9000))                                                   # 3008 chains
+    assert not pairs(128, 8, (8, 1910, 0)) and not pairs(64, 8, (4, 2030, 500)) and not pairs(24, 4, (42, 340, 1000))  # 16 - 24 tiles
+    assert not pairs(40, 8, (1, 16384, 8192)) and not pairs(12, 4, (1, 65536, 0))              # odd groups
+    # two rounds nearly full, 15 tiles on average, none much longer than an even share
+    assert pairs(64, 8, (1, 2048, 0)) and pairs(64, 8, (1, 1792, 0)) and pairs(8, 1, (9, 1700, 6000)) and pairs(16, 8, (3, 2400, 0))
+    assert not pairs(64, 8, (1, 2176, 0)) and not pairs(64, 8, (1, 1664, 0))                   # 1088, 832 chains
+    assert not pairs(24, 4, (5, 1000, 0))                                                      # 8 tiles
+    assert not pairs(8, 1, (1, 6784, 0), (3, 2500, 0)) and pairs(8, 1, (4, 3600, 0))           # one chain of 106 tiles, even ones
