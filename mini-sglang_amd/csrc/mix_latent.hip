@@ -58,9 +58,12 @@ struct LatentRow {
 // (Both holding half of Q and half of O, scores meeting in LDS, two barriers a tile: fragments one product ahead, 5150 cycles a tile of 32 keys, now 3900.
 // Twelve waves, one of scores and two of values a row set: 168 registers do not hold a third of O's accumulators and a second place where ways meet.)
 // Value waves fetch the rows: a DMA without addresses of its own in a lane's registers, and the score waves' reads wait for nothing but themselves.
-// 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1535 us -> 408 -> 351 us (840 TFLOP/s), of it some 60 us that a workgroup's start and end
-// take (queries and outputs, 563 MB at 4.9 TB/s; a workgroup fills its CU), 50 us the rows' way to LDS, 30 us the rescaling.  2 of 2253 tokens, 8 heads
-// 178 -> 139; 6 of 50 - 353 38 -> 33; 4 of 470, 256 + 64: 35 -> 32; 5 of 23 - 225, 8 heads 29.0 -> 29.4, the largest loss seen.
+// 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1535 us -> 408 -> 340 us (867 TFLOP/s; 350 on a slower card), 50 us of it the rows' way to LDS, 30
+// us the rescaling, some 60 us workgroups' starts and ends: four follow each other on a CU, which each fills, and the queries' and outputs' 563 MB
+// (115 us at 4.9 TB/s by themselves) come and go partly beside other workgroups' tiles.  2 of 2253 tokens, 8 heads 178 -> 140; 6 of 50 - 353 38 -> 32; 4 of
+// 470, 256 + 64: 35 -> 31.5; 5 of 23 - 225, 8 heads 29.0 -> 28.1.  One tile and full sets cost the two roles' one after the other: 8 portions of 8 tokens, 16
+// heads 12.5 -> 12.7, 40 of 17 15.9 -> 16.4, the largest loss seen.  (Two pieces of queries an LDS turn without bank conflicts, outputs several turns at a
+// time, no barrier behind the last weights, sets without rows only at the barriers: 13.7, 17.2 without them; 8 of 2 tokens 13.2 -> 10.1.)
 template <int DK, int DV>
 __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
                                                                const float* __restrict__ q_abs, const bf16_t* __restrict__ cache,
@@ -79,6 +82,7 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
   __shared__ __attribute__((aligned(1024))) char img0[IMAGE], img1[IMAGE], img2[IMAGE];
   __shared__ __attribute__((aligned(16))) f32x4_t s_p[2][4][2][64];  // weights [tile & 1][row set][16 keys][lane]
   __shared__ __attribute__((aligned(16))) f32x4_t s_q[4][NL ? NL : 1][64];
+  __shared__ __attribute__((aligned(16))) char s_turn[NL ? 16 : 4 * 4096];
   __shared__ float s_alpha[2][4][32];
   __shared__ float2 s_ml[4][32];
   __shared__ __attribute__((aligned(16))) int s_slot[4][KT];
@@ -119,9 +123,10 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
   // score wave keeps them: its own through LDS of its own, the other one's by way of two images, all at once.  (The whole way of a role, these loads
   // included, lies behind one branch: what one role alone needs must not live beside the other's.)
   constexpr int NU = DK / 64;  // a wave's pieces
+  auto first_slot = [&]() { return role ? trow[min(k_begin + 8 * (wave - 4) + (lane >> 3), n_keys - 1)] : slot_at(k_begin + wave * KT); };
   auto queries = [&](auto fetch, auto keep) __attribute__((always_inline)) {
     // slots in front of the queries: the value waves' of the first tile, the next two tiles' by way of LDS
-    const int slot = fetch ? trow[min(k_begin + 8 * (wave - 4) + (lane >> 3), n_keys - 1)] : slot_at(k_begin + wave * KT);
+    const int slot = first_slot();
     float4 x[NU][4];
     const float sign = scale < 0.f ? -1.f : 1.f;
 #pragma unroll
@@ -136,32 +141,35 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
     else if (wave < 3 && lane < KT) s_slot[wave][lane] = slot;
     char* other = (set < 2 ? img1 : img2) + (set & 1) * (2 * NU * 1024);
     static_assert(IMAGE >= 4 * NU * 1024, "two row sets' fragments");
+    // a piece to two fragments: [column / 16][column / 8 & 1][row][8 columns], four rows' places changed by the columns' number against bank conflicts
+    auto put = [&](char* at, const float4(&y)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<uint2*>(at + ((lane & 7) >> 2) * 1024 + ((((lane >> 1) & 1) * 32 + (lane >> 3) + 8 * i) ^ ((lane >> 1) & 3) * 4) * 16 + (lane & 1) * 8) =
+            uint2{pack_bf16(y[i].x * sign, y[i].y * sign), pack_bf16(y[i].z * sign, y[i].w * sign)};
+    };
+    auto place = [&](int k) { return k * 1024 + (lane ^ (2 * (k & 1) + hi) * 4) * 16; };
     if (fetch) {
 #pragma unroll
-      for (int u = 0; u < NU; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)  // fragment 2 u + (column of 32) / 16: [column / 8 & 1][row][8 columns]
-          *reinterpret_cast<uint2*>(other + (2 * u + ((lane & 7) >> 2)) * 1024 + ((lane >> 1) & 1) * 512 + ((lane >> 3) + 8 * i) * 16 + (lane & 1) * 8) =
-              uint2{pack_bf16(x[u][i].x * sign, x[u][i].y * sign), pack_bf16(x[u][i].z * sign, x[u][i].w * sign)};
+      for (int u = 0; u < NU; ++u) put(other + u * 2048, x[u]);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of the first tile
     } else {
-      char* turn = reinterpret_cast<char*>(s_p) + set * 4096;
-      constexpr int QROW = 80;  // 32 columns and 16 bytes of padding
+      char* turn = reinterpret_cast<char*>(s_p) + set * 4096;  // two pieces at a time
 #pragma unroll
-      for (int u = 0; u < NU; ++u) {
+      for (int u0 = 0; u0 < NU; u0 += 2) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          *reinterpret_cast<uint2*>(turn + ((lane >> 3) + 8 * i) * QROW + 8 * (lane & 7)) =
-              uint2{pack_bf16(x[u][i].x * sign, x[u][i].y * sign), pack_bf16(x[u][i].z * sign, x[u][i].w * sign)};
+        for (int u = u0; u < u0 + 2 && u < NU; ++u) put(turn + (u - u0) * 2048, x[u]);
         wave_fence();
 #pragma unroll
-        for (int k = 0; k < 2; ++k) keep(4 * u + k, turn + (lane & 31) * QROW + 32 * k + 16 * hi);
+        for (int u = u0; u < u0 + 2 && u < NU; ++u)
+#pragma unroll
+          for (int k = 0; k < 2; ++k) keep(4 * u + k, turn + place(2 * (u - u0) + k));
         wave_fence();
       }
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 2 * NU; ++k) keep(k / 2 * 4 + 2 + (k & 1), other + k * 1024 + lane * 16);
+    for (int k = 0; k < 2 * NU; ++k) keep(k / 2 * 4 + 2 + (k & 1), other + place(k));
     __syncthreads();
   };
 
@@ -172,9 +180,9 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
     const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(p + 8 * ROW));
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  // a row set's outputs times f, 32 columns at a time by way of LDS, so that a row's are stored as one cache line (lanes' own 16 bytes of 64 rows'
-  // lines: 60 us of 460 at 8096 tokens and 16 heads); a row's 16-byte pieces change places by its number, against bank conflicts
-  auto finish = [&](const f32x16_t* o, int nvt, int col0) __attribute__((always_inline)) {
+  // a row set's outputs times f by way of LDS, `some` times 32 columns at a time, so that a row's are stored as cache lines (lanes' own 16 bytes of 64
+  // rows' lines: 60 us of 460 at 8096 tokens and 16 heads); a row's 16-byte pieces change places by its number, against bank conflicts
+  auto finish = [&](const f32x16_t* o, auto nvt, auto some, char* turn, int col0) __attribute__((always_inline)) {
     int l = lane;
     asm volatile("" : "+v"(l));  // the rows are worked out anew: no registers for them meanwhile
     float f = 1.f;
@@ -184,8 +192,6 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
       const float sf = sink_factor(sink, hh, ml.x);
       f = sf / (sf * ml.y + sink_weight(sink, hh, ml.x));
     }
-    char* turn = (wave < 4 ? img0 : img1) + (wave & 3) * 4096;
-    static_assert(IMAGE >= 4 * 4096, "four waves' turns");
     float* dst[4];
     bool valid[4];
 #pragma unroll
@@ -196,22 +202,62 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
       dst[i] = (splits == 1 ? out + row * DV : part_o + (row * splits + z) * DV) + col0 + 4 * (l & 7);
     }
 #pragma unroll
-    for (int vt = 0; vt < nvt; ++vt) {
+    for (int vt0 = 0; vt0 < nvt; vt0 += some) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<float4*>(turn + (l & 31) * 128 + (((2 * g + hi) ^ l) & 7) * 16) =
-            float4{o[vt][4 * g] * f, o[vt][4 * g + 1] * f, o[vt][4 * g + 2] * f, o[vt][4 * g + 3] * f};
+      for (int n = 0; n < some; ++n)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x16_t& x = o[vt0 + n];
+          *reinterpret_cast<float4*>(turn + n * 4096 + (l & 31) * 128 + (((2 * g + hi) ^ l) & 7) * 16) =
+              float4{x[4 * g] * f, x[4 * g + 1] * f, x[4 * g + 2] * f, x[4 * g + 3] * f};
+        }
       wave_fence();
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (valid[i])
-          *reinterpret_cast<float4*>(dst[i] + vt * 32) = *reinterpret_cast<const float4*>(turn + ((l >> 3) + 8 * i) * 128 + (((l & 7) ^ (l >> 3)) & 7) * 16);
+      for (int i = 0; i < 4; ++i) {
+        if (valid[i]) {
+#pragma unroll
+          for (int n = 0; n < some; ++n)
+            *reinterpret_cast<float4*>(dst[i] + (vt0 + n) * 32) =
+                *reinterpret_cast<const float4*>(turn + n * 4096 + ((l >> 3) + 8 * i) * 128 + (((l & 7) ^ (l >> 3)) & 7) * 16);
+        }
+      }
       wave_fence();
     }
   };
 
+  auto fetch = [&](char* next, int t) __attribute__((always_inline)) {
+    int slot = 0;
+    if (wave == 7 && t + 3 < n_tiles) slot = slot_at(k_begin + (t + 3) * KT);  // in front of the DMA: waiting for it does not wait for the DMA
+    if (t + 1 < n_tiles) dma(next, s_slot[(t + 1) & 3][8 * (wave - 4) + (lane >> 3)]);
+    return slot;
+  };
+  auto arrived = [&](int slot, int t) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of tile t + 1
+    if (wave == 7 && lane < KT) s_slot[(t + 3) & 3][lane] = slot;
+    __syncthreads();
+  };
+
   // ---- Iteration t: the score waves turn tile t into weights and add their columns' values, the value waves add tile t - 1's to theirs and fetch
-  // tile t + 1 into the image of tile t - 2.  Both ways pass the same barriers: n_tiles + 1.
+  // tile t + 1 into the image of tile t - 2.  Both ways pass the same barriers, n_tiles of them: nothing is waited for after the last weights.
+  // A set without rows: its share of the rows' way to LDS and the barriers (a scalar branch, which a wave takes or not), nothing of the LDS reads
+  if (__builtin_amdgcn_readfirstlane(rows0 >= QT * HB || tok0 + rows0 / HB >= q_len) != 0) {
+    if (n_tiles > 0) {
+      const int slot = first_slot();
+      if (role == 0) {
+        if (wave < 3 && lane < KT) s_slot[wave][lane] = slot;
+      } else {
+        dma(img0, slot);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      __syncthreads();
+      __syncthreads();
+    }
+    for (int t = 0; t < n_tiles; ++t) {
+      if (role == 1) arrived(fetch(t % 3 == 0 ? img1 : t % 3 == 1 ? img2 : img0, t), t);
+      else __syncthreads();
+    }
+    return;
+  }
   if (role == 0) {
     const int r = rows0 + (lane & 31), tl = tok0 + r / HB;
     const int limit = r < QT * HB && tl < q_len && h0 + r % HB < H ? start + tl : -1;  // the last key position that this lane's row sees, -1: no row
@@ -287,9 +333,14 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
         pw[e >> 1] = pack_bf16(w0, w1);
       }
       lsum += sum;
+      if (t + 1 == n_tiles) {
+        lsum += __shfl_xor(lsum, 32, 64);
+        if (hi == 0) s_ml[set][lane] = float2{m * kLn2, lsum};
+      }
 #pragma unroll
       for (int w = 0; w < 2; ++w)
         *reinterpret_cast<Q4*>(&s_p[t & 1][set][w][lane]) = Q4{pw[4 * w], pw[4 * w + 1], pw[4 * w + 2], pw[4 * w + 3]};
+      __syncthreads();
 #pragma unroll
       for (int i = 0; i < 2 * NVS; ++i) {  // O^T += V^T P^T, 16 keys a step: a lane's eight of them are what its registers 8 step ... hold
         if (i + 2 < 2 * NVS) vf[(i + 2) % 3] = vfrag(vp + (i + 2) / NVS * 16 * ROW + (i + 2) % NVS * 64);
@@ -298,25 +349,18 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
         const Q4 pq{pw[w], pw[w + 1], pw[w + 2], pw[w + 3]};
         o[i % NVS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i % 3], __builtin_bit_cast(bf16x8_t, pq), o[i % NVS], 0, 0, 0);
       }
-      __syncthreads();
     };
     for (int t = 0; t < n_tiles; t += 3) {
       scores(img0, t);
       if (t + 1 < n_tiles) scores(img1, t + 1);
       if (t + 2 < n_tiles) scores(img2, t + 2);
     }
-    lsum += __shfl_xor(lsum, 32, 64);
-    m *= kLn2;
-    if (hi == 0) {
-      s_ml[set][lane] = float2{m, lsum};
-      if (splits > 1 && limit >= 0) {
-        const size_t row = ((size_t)first + tl) * H + h0 + r % HB;
-        part_ml[(row * splits + z) * 2] = m;
-        part_ml[(row * splits + z) * 2 + 1] = lsum;
-      }
+    if (hi == 0 && splits > 1 && limit >= 0) {
+      const size_t row = ((size_t)first + tl) * H + h0 + r % HB;
+      part_ml[(row * splits + z) * 2] = m * kLn2;
+      part_ml[(row * splits + z) * 2 + 1] = lsum;
     }
-    __syncthreads();
-    finish(o, NVS, NVV * 32);
+    finish(o, std::integral_constant<int, NVS>{}, std::integral_constant<int, 1>{}, NL ? reinterpret_cast<char*>(s_q[set]) : s_turn + set * 4096, NVV * 32);
     asm volatile("; score waves");
   } else {
     if (n_tiles > 0) queries(std::true_type{}, [](int, const char*) {});
@@ -354,24 +398,13 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
           o[(i + n) % NVV] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i / SOME & 1][n], __builtin_bit_cast(bf16x8_t, p[(i + n) / NVV]), o[(i + n) % NVV], 0, 0, 0);
       }
     };
-    auto fetch = [&](char* next, int t) __attribute__((always_inline)) {
-      int slot = 0;
-      if (wave == 7 && t + 3 < n_tiles) slot = slot_at(k_begin + (t + 3) * KT);  // in front of the DMA: waiting for it does not wait for the DMA
-      if (t + 1 < n_tiles) dma(next, s_slot[(t + 1) & 3][8 * (wave - 4) + (lane >> 3)]);
-      return slot;
-    };
-    auto arrived = [&](int slot, int t) __attribute__((always_inline)) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of tile t + 1
-      if (wave == 7 && lane < KT) s_slot[(t + 3) & 3][lane] = slot;
-      __syncthreads();
-    };
     auto step = [&](const char* before, char* next, int t) __attribute__((always_inline)) {
       const int slot = fetch(next, t);
       values(before, t - 1);
-      arrived(slot, t);
+      if (t < n_tiles) arrived(slot, t);
     };
-    arrived(fetch(img1, 0), 0);
     if (n_tiles > 0) {
+      arrived(fetch(img1, 0), 0);
       int t = 1;  // (no step of the loop is conditional: where ways met, the accumulators had two places, and hundreds were spilled)
       for (; t + 2 <= n_tiles; t += 3) {
         step(img0, img2, t);
@@ -383,7 +416,10 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
         if (t + 1 <= n_tiles) step(img1, img0, t + 1);
       }
     }
-    finish(o, NVV, 0);
+    // by way of the two images that do not hold the last tile
+    static_assert(IMAGE >= 2 * NVS * 4096, "two waves' turns");
+    const int free_one = (n_tiles + (set >> 1)) % 3;
+    finish(o, std::integral_constant<int, NVV>{}, std::integral_constant<int, NVS>{}, (free_one == 0 ? img0 : free_one == 1 ? img1 : img2) + (set & 1) * (NVS * 4096), 0);
     asm volatile("; value waves");
   }
 }

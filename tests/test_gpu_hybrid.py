@@ -387,6 +387,40 @@ def test_latent_portion_tiles(dev, H, R, scale):
             assert float((out.double().cpu() - ref).norm() / ref.norm()) < 8e-3, (keys, splits)
 
 
+@pytest.mark.parametrize("R", [512, 256])
+@pytest.mark.parametrize("H", [4, 16, 32])
+def test_latent_portions_of_few_rows(dev, H, R):
+    """Portions that leave some of a workgroup's four sets of 32 rows empty, or one row in one, over one to four tiles.  Bound as in
+    test_latent_attention_usual_widths."""
+    from mini_sglang_amd import mixops
+
+    g = torch.Generator().manual_seed(H + R)
+    r, scale = 64, 0.08
+    new = sorted({n for rows in (32, 36, 64, 68, 96, 100, 128, 132) for n in (max(1, rows // H), rows // H + 1)})
+    old = [0, 20, 40, 70, 100]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    keys = [n + old[i % 5] for i, n in enumerate(new)]
+    slots = torch.randperm(sum(keys), generator=g)
+    cache, q = torch.randn(sum(keys), R + r, generator=g).bfloat16(), torch.randn(sum(new), H, R + r, generator=g) * 0.8
+    table, ref, at, row = torch.zeros(len(new), max(keys), dtype=torch.int32), [], 0, 0
+    for b, (n, m) in enumerate(zip(new, keys)):
+        table[b, :m] = slots[at: at + m].int()
+        rows = cache[slots[at: at + m]].double()
+        s = torch.einsum("thk,jk->thj", q[row: row + n].double(), rows) * scale
+        s = s.masked_fill(torch.arange(m)[None, None, :] > (torch.arange(n) + m - n)[:, None, None], -torch.inf)
+        ref.append(torch.softmax(s, -1) @ rows[:, :R])
+        at, row = at + m, row + n
+    cu = i32([0] + new).cumsum(0).int()
+    for splits in (1, 2):
+        out = torch.full((sum(new) + 1, H, R), float("nan"), device=dev)
+        mixops.latent_attn(out[:-1], q.to(dev), cache.to(dev), table.to(dev), i32(list(range(len(new)))), i32(keys), cu, len(new), R, scale, splits=splits)
+        got = out.double().cpu()
+        assert bool(got[-1].isnan().all())
+        for b, want in enumerate(ref):
+            have = got[sum(new[:b]): sum(new[: b + 1])]
+            assert float((have - want).norm() / want.norm()) < 8e-3, (new[b], keys[b], splits)
+
+
 @pytest.mark.parametrize("B", [64, 65, 150])
 @pytest.mark.parametrize("splits", [1, 3])
 @pytest.mark.parametrize("most", [1, 20], ids=["decode", "portions"])
