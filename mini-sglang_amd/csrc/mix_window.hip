@@ -37,7 +37,7 @@ constexpr int kWinHead = 16 * kWinRow + 4;  // floats of a head: four of them ap
 //   Q K^T with rows (head of four, query of four), mixed scores as their product with the table over the heads
 //   mixed scores to LDS; the waves share the heads, 32 rows (two heads of 16 queries): mask, online softmax, O^T += V^T P^T (a lane reads
 //   four consecutive keys of its row, the layout the product takes; V through transposing LDS reads).  Meanwhile the next rows arrive.
-// FULL: heads of 128
+// FULL: key heads of 128
 template <int NH, int G, bool FULL>
 __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
                                                                   const bf16_t* __restrict__ src, int64_t ld_src, int g_off,
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
   // banks once.  (Rows 8 apart: odd ones' keys the other half.)
   constexpr int FLIP = ROWS & 8;
   const int ck0 = (piece ^ key0) & 15, ck1 = ck0 ^ FLIP, cv = piece ^ ((key0 & 3) << 2);
-  const uint32_t k_at0 = hv * d + 8 * ck0, k_at1 = hv * d + 8 * ck1, v_at = hv * dv + 8 * cv;
+  const uint32_t k_at0 = hv * d + 8 * ck0, k_at1 = hv * d + 8 * ck1, v_at = hv * dv + min(8 * cv, dv - 8);
   // a tile's slots of this thread's rows, read together ahead of their use: a read in front of each request waited for all LDS reads before it
   struct Slots {
     int of[NP];
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
     __builtin_amdgcn_sched_barrier(kAllButLoads);
   };
   auto request_v = [&](uint16_t* img, const Slots& slots, int u) __attribute__((always_inline)) {
-    if (u < NP && (FULL || 8 * cv < dv))
+    if (u < NP)
       __builtin_amdgcn_global_load_lds((glb_void_t*)(row_at(v_cache, slots.of[u < NP ? u : 0], nv) + v_at),
                                        (lds_void_t*)(img + (u * NT + wave * 64) * 8), 16, 0, 0);
     __builtin_amdgcn_sched_barrier(kAllButLoads);
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
         if (j0 + key >= k_end) *reinterpret_cast<Q4*>(img + (key * PCS + (int)threadIdx.x % PCS) * 8) = Q4{0u, 0u, 0u, 0u};
     }
   };
-  // Zeros past the heads of keys, where no DMA goes.  (Values there are whatever LDS holds: their columns of O are not stored.)
+  // Zeros past the heads of keys, where no DMA goes.  (Past the values' heads lies their last piece again: those columns of O are not stored.)
   if (!FULL) {
 #pragma unroll
     for (int u = 0; u < NP; ++u) {
@@ -379,7 +379,7 @@ extern "C" __attribute__((visibility("hidden"))) int mix_window_attn_mfma(
   if (!msgl_mix_window_attn_on_matrix_cores(H, G, d, dv, MSGL_MIX_BF16)) return 0;
   if (!al(k_cache) || !al(v_cache) || !al(out) || (part_o && !al(part_o))) return 0;
   const dim3 grid(total_q / 16 + batch, splits);
-#define WIN_KERNEL(NH, G) (d == 128 && dv == 128 ? window_attn_mfma_kernel<NH, G, true> : window_attn_mfma_kernel<NH, G, false>)
+#define WIN_KERNEL(NH, G) (d == 128 ? window_attn_mfma_kernel<NH, G, true> : window_attn_mfma_kernel<NH, G, false>)
   const auto kernel = H == 16 ? (G == 4 ? WIN_KERNEL(16, 4) : G == 2 ? WIN_KERNEL(16, 2) : WIN_KERNEL(16, 1)) : G == 2 ? WIN_KERNEL(8, 2) : WIN_KERNEL(8, 1);
 #undef WIN_KERNEL
   hipLaunchKernelGGL(kernel, grid, dim3(H * 32), 0, s, mp<bf16_t>(out), part_o, part_ml, cp<bf16_t>(src), ld_src, g_off, cp<bf16_t>(k_cache),
