@@ -254,10 +254,10 @@ def test_prefill_key_ranges(ops, dev, monkeypatch, hq, hkv, specs, ranges, dtype
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("more", [0, 5])
+@pytest.mark.parametrize("more", [0, 5, 12])
 def test_prefill_short_tiles(ops, dev, more, dtype):
-    """q tiles around the numbers of rows from which they are loaded and stored in whole rows, waves without rows among them, in launches of 400 and of 600
-    workgroups: the bits of the register-staged kernel, which has one way only."""
+    """q tiles around the numbers of rows from which they are loaded and stored in whole rows, waves without rows among them, in launches of 400, 600 and 880
+    workgroups (one round; one and a half, where such waves stay; more): the bits of the register-staged kernel, which has one way only."""
     new = [1, 31, 32, 33, 63, 64, 65, 127, 128, 96] + [129] * (more // 2) + [70] * (more % 2)
     c = build(torch.Generator().manual_seed(23), [(70, 70 + n) for n in new], 40, 8, 16, dtype)
     assert torch.equal(run(ops, dev, c, impl=4), run(ops, dev, c, impl=2))
