@@ -71,7 +71,7 @@ struct PrefillParams {
   int share_log2, per;  // XCDs that share their kv heads, kv heads of each
   int stretch;     // workgroups of an XCD where each takes a stretch of the list, or 0
   int few;         // q tiles of fewer rows load and store by lanes' own pieces
-  int idle;        // waves without rows make no products
+  int idle;        // waves without rows make no products (one head a workgroup)
   int ranges, run;  // key ranges, and tiles of each (the last one: what is left)
   float *part_o, *part_ml;
   float scale_log2;
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
   }
   const int my_qpos = diag + my_q;
   const int left = q_len - (q0 + rows * 32);  // this wave's rows, 32 of them at most
-  const int wave_min_qpos = left > 0 || !p.idle ? diag + q0 + rows * 32 : -kKTile;  // scalar; no row: no tile
+  const int wave_min_qpos = HEADS == 2 || left > 0 || !p.idle ? diag + q0 + rows * 32 : -kKTile;  // scalar; no row: no tile
 
   f32x16 o[4];
 #pragma unroll
@@ -758,7 +758,7 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
   auto piece = [&](int nb, int rg) __attribute__((always_inline)) {  // columns 32 nb + 8 rg + 4 hi .. + 3 of the lane's row
     return uint2{Elem<T>::pack(o[nb][4 * rg] * inv, o[nb][4 * rg + 1] * inv), Elem<T>::pack(o[nb][4 * rg + 2] * inv, o[nb][4 * rg + 3] * inv)};
   };
-  if (left <= 0) return;
+  if (HEADS == 1 && left <= 0) return;
   if (!own_pieces) {
     // Outputs by way of the image that does not hold the last tile (everyone is done with it), a wave's rows in its own part: whole rows of 256
     // bytes leave it, where a lane's own pieces are 16 bytes of 32 rows a store.  16-byte pieces change places by the row's number.
@@ -909,13 +909,13 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   // Waves without rows leave the matrix cores to the others (40 heads on 8, 14 requests of 14 - 41 tokens after 300: 25.7 -> 23.7 us; 64 on 8, 20 of 65 -
   // 187 after 2000 287 -> 259; 29 of 100 - 1024 on 40 heads 229 -> 225).  Not in one and a half rounds: who then ends early takes two of the last
   // workgroups onto one CU (768: 8 of 93 - 218 after 2000 120 -> 132; 740: 83 -> 90; from 768 on none of 100 sizes more than 2 % slower).
-  const int64_t places = 512 / heads, wanted = total * ranges;
-  p.idle = wanted <= places || wanted > places * 3 / 2;
+  const int64_t wanted = total * ranges;
+  p.idle = wanted <= 512 || wanted > 768;
   // Where all workgroups start at once the time is one workgroup's, and only full tiles go in whole rows by way of LDS; else from about half a tile on.
   // us, 8 requests of n tokens, own pieces / whole rows: 16 heads on 8 (128 workgroups) of 32 7.5 / 8.3, 64 8.8 / 9.0, 100 10.9 / 11.4, 128 11.8 /
   // 11.9; 40 requests, 40 on 8 (1600): of 20 20.5 / 22.5, 40 26.4 / 27.4, 64 30.8 / 29.9, 100 42.3 / 40.3, 128 48.8 / 43.7; where all four waves stay, 61
   // rows behind full tiles (640) 23.1 / 22.1
-  p.few = wanted <= places ? kQTile : p.idle ? kQTile / 2 : 48;
+  p.few = wanted <= 512 ? kQTile : p.idle ? kQTile / 2 : 48;
   const unsigned blocks = (unsigned)even * 8;
   if (ranges > 1) {
     p.ranges = ranges;

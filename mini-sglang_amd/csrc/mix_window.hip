@@ -89,17 +89,16 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
   {
     const int t = tok0 + 4 * quad + (lr & 3);
     const bf16_t* qrow = src + (size_t)(cu_q[b] + (t < q_len ? t : tok0)) * (size_t)ld_src + (size_t)(lr >> 2) * d;
+    // 16 bytes from where they lie, whatever the rows' stride: global memory takes any alignment (12 tokens, unaligned: 16.6 us, number by number
+    // 31.5).  Past the head its last piece for now: a lane's condition on a load would be a wait for it.
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc) {
-      const int k = kc * 32 + lg * 8;
-      // 16 bytes from where they lie, whatever the rows' stride: global memory takes any alignment (12 tokens, unaligned: 16.6 us, number by number
-      // 31.5).  Past the head its last piece for now: a lane's condition on a load would be a wait for it.
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
+      for (int kc = 0; kc < KC; ++kc) {
+        const int k = kc * 32 + lg * 8;
         qf[j][kc] = bf16x8_t{};
         if (FULL || kc * 32 < d) __builtin_memcpy(&qf[j][kc], qrow + 4 * j * d + (FULL ? k : min(k, d - 8)), 16);
       }
-    }
   }
   // this lane's row of the second product: head h0 + (lane >> 4 & 1), query lr
   f32x16_t o[VC / 2];

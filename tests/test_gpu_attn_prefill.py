@@ -267,7 +267,11 @@ def test_prefill_short_tiles(ops, dev, more, dtype):
     (2, 1, [(0, 1)], torch.bfloat16),                                          # one row, one pair
     (16, 8, [(0, n) for n in (5, 31, 33, 64, 127, 129, 300)], torch.bfloat16),  # one tile, odd and even chains, waves without rows
     (6, 1, [(0, 129), (700, 701), (63, 192)], torch.float16),                  # three pairs of a kv head, a short portion after a long one
-    (64, 8, [(1000, 1600)], torch.bfloat16),                                   # more workgroups than compute units
+    (64, 8, [(1000, 1600)], torch.bfloat16),                                   # several pairs of a kv head, keys before the portion
+    # more workgroups than compute units, whose lists go in turns: one XCD's kv heads shared by four, by two XCDs and one of its own several of them
+    (16, 2, [(0, 900), (100, 1500), (0, 130), (0, 1000), (50, 650), (0, 300)], torch.bfloat16),
+    (24, 6, [(0, 700), (300, 1100), (0, 129), (64, 650), (0, 1), (500, 1300)], torch.float16),
+    (64, 16, [(0, 1), (700, 1000), (0, 520)], torch.float16),
 ])
 def test_prefill_heads_in_pairs(ops, dev, monkeypatch, hq, hkv, specs, dtype):
     """Two heads a workgroup: the bits of one head a workgroup, which the oracle's tests pin; an odd group is refused."""
@@ -307,18 +311,20 @@ def test_prompt_attention_leaves_the_decode_workspace_alone(ops, dev):
     assert torch.isfinite(out).all() and bool((backend._workspace == 0x5A).all())
 
 
-@pytest.mark.parametrize("hq,hkv,new,pairs", [(64, 8, 2048, True), (64, 8, 1900, True), (64, 8, 1700, False), (40, 8, 3072, False)])
-def test_backend_pairs_heads_by_its_rule(ops, dev, hq, hkv, new, pairs):
-    """Heads go in pairs where a launch has 896 to 1024 chains of 15 tiles and more on average and a kv head an even number of heads; the bits are the other launch's."""
+@pytest.mark.parametrize("hq,hkv,new,pairs", [(64, 8, 2048, True), (64, 8, 1900, True), (64, 8, 1700, False), (40, 8, 3072, False), (64, 8, 6144, True), (64, 8, 3328, False)])
+def test_backend_pairs_heads_by_its_rule(ops, dev, monkeypatch, hq, hkv, new, pairs):
+    """Heads go in pairs where a launch has 896 to 1024 chains of 15 tiles and more on average, or from 3072 of 36 on, and a kv head an even number of heads: the
+    launch that the library gets is that one, and the bits are the other one's."""
     from mini_sglang_amd.attention import HipAttnBackend
     from mini_sglang_amd.core import Batch, Context, Req
     from mini_sglang_amd.kvcache import create_kvcache_pool
     from mini_sglang_amd.model import ModelConfig
 
     ctx = Context(16)
+    width = max(3328, new)
     m = ModelConfig(num_layers=1, num_qo_heads=hq, num_kv_heads=hkv, head_dim=128, hidden_size=1024, vocab_size=64, intermediate_size=64)
-    ctx.page_table = torch.arange(3328, dtype=torch.int32, device=dev).view(1, 3328)
-    ctx.kv_cache = create_kvcache_pool(m, 208, 16, torch.bfloat16, dev)
+    ctx.page_table = torch.arange(width, dtype=torch.int32, device=dev).view(1, width)
+    ctx.kv_cache = create_kvcache_pool(m, width // 16, 16, torch.bfloat16, dev)
     backend = HipAttnBackend(m, ctx)
     batch = Batch(reqs=[Req(input_ids=torch.zeros(new, dtype=torch.int32), table_idx=0, cached_len=0, output_len=1, uid=0)], phase="prefill")
     batch.out_loc = torch.arange(new, dtype=torch.int32, device=dev)
@@ -326,10 +332,19 @@ def test_backend_pairs_heads_by_its_rule(ops, dev, hq, hkv, new, pairs):
     backend.prepare_metadata(batch)
     md = batch.attn_metadata
     assert md.pairs == pairs and md.ranges[0] == 1
+    real, impls = ops.lib(), []
+
+    class Recorder:
+        def __getattr__(self, name):
+            call = getattr(real, name)
+            return call if name != "msgl_attn_prefill" else lambda *a: (impls.append(int(a[-2])), call(*a))[1]
+
+    monkeypatch.setattr(ops, "lib", lambda: Recorder())
     q, k, v = (torch.randn(new, h * 128, device=dev).bfloat16() for h in (hq, hkv, hkv))
     out = backend.forward(q.view(new, hq, 128), k, v, 0, batch)
-    md.pairs = False
+    md.pairs = not pairs and hq // hkv % 2 == 0  # the other launch, where there is one
     assert torch.equal(out, backend.forward(q.view(new, hq, 128), k, v, 0, batch))
+    assert impls == [6 if pairs else 0, 6 if md.pairs else 0]
 
 
 def test_a_small_decode_capacity_holds_the_small_batch_kernel(ops, dev):
