@@ -259,8 +259,7 @@ int msgl_attn_prefill(void* out, const void* q, const void* k_cache, const void*
  * (global_load_lds_dwordx4, ds_read_b64_tr_b16 V fragments, double-buffered LDS, XCD-contiguous kv heads, softmax scale
  * folded into the exponent's fma); 6 = the same with two heads of a kv head a workgroup (an even number of heads each; for many
  * long tile chains; bit-identical); 2 = the same math with register staging (the A/B partner; bit-identical results).
- * Every other value is refused.  (Rounds 1-3 also had 1, 3, 5 -- a first-generation and a counter-phase kernel -- and
- * timing-only ablation codes >= 16; the former were removed, the latter exist only in a -DMSGL_PREFILL_DIAG build.) */
+ * Every other value is refused (timing-only ablation codes >= 16 exist in a -DMSGL_PREFILL_DIAG build alone). */
 /* impl 0 with a job's (q tile's and head's) keys cut into up to `ranges` (2 .. 64) ranges of range_tiles 64-key tiles, the
  * last one taking what is left, one workgroup each; their fp32 sums are joined by a second launch.  For launches too small
  * to fill the compute units.  A job of one range has impl 0's bits. */

@@ -1,16 +1,12 @@
 // Paged varlen causal prefill attention for gfx950 (MFMA 32x32x16, fp32 accumulate).
 //
-// Two kernels with the same math per query row, bit-identical to each other (impl codes in include/msgl_hip.h): the
-// default DMA-staged one (attn_prefill_dma_kernel, impl 4 = 0) and its register-staged predecessor
-// (attn_prefill_tr_kernel, impl 2), kept as the A/B partner and cross-check.  One workgroup = 4 waves = one 128-row
-// query tile of one (request, q head); each wave owns 32 query rows.  K/V are gathered through the reference's
-// token-granular page table in 64-key tiles one tile ahead of the MFMAs: global -> registers -> LDS (impl 2), global ->
-// LDS by DMA (global_load_lds_dwordx4; impl 4).  Rounds 1-3 also carried a first-generation kernel (V transposed by
-// 2-byte LDS stores) and a counter-phase kernel (two wave groups of a 256-row tile, matrix segment beside softmax
-// segment: bit-identical, 43 % VALU/MFMA co-execution, NOT faster -- DESIGN.md section 8); both were removed in round 4,
-// their measurements stay under profiles/r03_prefill_*.  Ablation variants (ABL != 0: timing only, WRONG results) are
-// compiled only with -DMSGL_PREFILL_DIAG (MSGL_PREFILL_DIAG=1 python mini-sglang_amd/build.py): a stray impl code
-// cannot select one in a production build.
+// Two kernels with the same math per query row, bit-identical to each other (impl codes in include/msgl_hip.h): the default DMA-staged one
+// (attn_prefill_dma_kernel, impl 4 = 0; 6 = two heads a workgroup) and its register-staged predecessor (attn_prefill_tr_kernel, impl 2), kept as the A/B
+// partner and cross-check.  One workgroup = 4 waves = one 128-row query tile of one (request, q head), with impl 6 8 waves = the same tile of two heads of a
+// kv head; each wave owns 32 query rows of a head.  K/V are gathered through the reference's token-granular page table in 64-key tiles one tile ahead of
+// the MFMAs: global -> registers -> LDS (impl 2), global -> LDS by DMA (global_load_lds_dwordx4; impl 4, 6).  Launches that leave compute units empty cut a
+// job's keys into ranges, whose sums attn_prefill_join_kernel puts together.  Ablation variants (ABL != 0: timing only, WRONG results) are compiled only with
+// -DMSGL_PREFILL_DIAG (MSGL_PREFILL_DIAG=1 python mini-sglang_amd/build.py): a stray impl code cannot select one in a production build.
 //
 // Data flow per 64-key tile and wave (all in registers except the K/V tile):
 //   S^T = K . Q^T   ("swapped" QK^T: A = K rows from LDS (XOR-swizzled, conflict-free
@@ -452,12 +448,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 //     wave's reads at the first use of any, so the V^T fragments are asked for after the second key block's have come;
 //   * nothing of the softmax crosses LDS: the halves' maximum and their shares of a tile's sum by lane swaps.
 // What bounds it: power, where the launch is long (1.8 GHz; inputs of zeros 5330 -> 4020 us), and the copies.  64 heads, 8192 tokens after 16384, us
-// with a part left out: all copies but the first 4330, no exponentials 5025, no rescale 5200, none of exponentials, rescale and mask 4930; the scores
-// of the next tile in the same wave beside a tile's weights: 5290.  A wave's tile is 1024 cycles of the matrix cores and about as many of the vector
-// units (32 scores a lane, the exponential 16 cycles each).  5240 us with one head a workgroup, 4940 with two (1110 TFLOP/s); 40 heads on 8, 29 requests
-// of 100 - 1024 tokens: 234, and with Q and the outputs in whole rows by way of LDS (one head a workgroup; on a slower card 249 -> 240, 60 requests
-// of 128 - 256 tokens 129 -> 122): starts and outputs are half of such a launch (empty workgroups 14 us, requests and outputs 41, the first tile
-// 48).  (Sums of the rounded weights, one instruction a pair: 0.5 % faster, and 2^-9 of a row's weight off.)
+// with a part left out (one head a workgroup, 5290 with all): all copies but the first 4330, no exponentials 5025, no rescale 5200, none of exponentials,
+// rescale and mask 4930; the scores of the next tile in the same wave beside a tile's weights: 5290.  A wave's tile is 1024 cycles of the matrix cores and
+// about as many of the vector units (32 scores a lane, the exponential 16 cycles each).  5240 us with a row's offset found once, 4960 with two heads a
+// workgroup (1110 TFLOP/s).  40 heads on 8, 29 requests of 100 - 1024 tokens, with store_kv_kernel (23): 238 -> 234 us with a row's offset found once, 226
+// with Q and the outputs in whole rows by way of LDS, 220 without products for rows that are none; starts and outputs are half of such a launch (in us
+// before those two: empty workgroups 14, requests and outputs 41, the first tile 48, the second 17, each of the others 19).  60 requests of 128 - 256
+// tokens 125 -> 109.  (Sums of the rounded weights, one instruction a pair: 0.5 % faster, and 2^-9 of a row's weight off.)
 // HEADS = 2: eight waves, two heads of a kv head beside each other over the same tiles: half the copies.  One workgroup a CU then, so nothing runs
 // under its start, and the last round is coarser: for many long chains of tiles (the rule and its other side: ops.prefill_pairs).
 // RANGES: workgroup (.., z) takes the tiles z * run .. of the job's keys; sums of more than one range go to attn_prefill_join_kernel in fp32, in
@@ -849,7 +846,7 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   MSGL_REQUIRE(batch >= 0 && total_tiles >= 0, "attn_prefill: negative sizes");
 #ifdef MSGL_PREFILL_DIAG
   MSGL_REQUIRE(impl == 0 || impl == 2 || impl == 4 || impl == 6 || (impl >= 16 && impl < 48) || (impl >= 64 && impl < 128),
-               "attn_prefill: impl %d (0 = 4 DMA-staged, 2 register-staged; diagnostic build: 16 + bits / 64 + bits = ablations)", impl);
+               "attn_prefill: impl %d (0 = 4 DMA-staged, 6 with two heads a workgroup, 2 register-staged; diagnostic build: 16 + bits / 64 + bits = ablations)", impl);
 #else
   MSGL_REQUIRE(impl == 0 || impl == 2 || impl == 4 || impl == 6,
                "attn_prefill: impl %d (0 = 4 the DMA-staged kernel, 6 with two heads a workgroup, 2 the register-staged kernel; ablation codes need a "

@@ -58,7 +58,7 @@ struct LatentRow {
 // (Both holding half of Q and half of O, scores meeting in LDS, two barriers a tile: fragments one product ahead, 5150 cycles a tile of 32 keys, now 3900.
 // Twelve waves, one of scores and two of values a row set: 168 registers do not hold a third of O's accumulators and a second place where ways meet.)
 // Value waves fetch the rows: a DMA without addresses of its own in a lane's registers, and the score waves' reads wait for nothing but themselves.
-// 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1535 us -> 408 -> 340 us (867 TFLOP/s; 350 on a slower card), 50 us of it the rows' way to LDS, 30
+// 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1535 us -> 408 -> 340 us (870 TFLOP/s), 50 us of it the rows' way to LDS, 30
 // us the rescaling, some 60 us workgroups' starts and ends: four follow each other on a CU, which each fills, and the queries' and outputs' 563 MB
 // (115 us at 4.9 TB/s by themselves) come and go partly beside other workgroups' tiles.  2 of 2253 tokens, 8 heads 178 -> 140; 6 of 50 - 353 38 -> 32; 4 of
 // 470, 256 + 64: 35 -> 31.5; 5 of 23 - 225, 8 heads 29.0 -> 28.1.  One tile and full sets cost the two roles' one after the other: 8 portions of 8 tokens, 16

@@ -857,7 +857,7 @@ __global__ __launch_bounds__(kRowThreads) void sample_logits_kernel(int* __restr
 //   split_mass   each takes some of up to 1024 chunks in index order: the chunk's mass above the 64th of an octave in which the threshold
 //                lies, and the candidates within (without a filter: the chunk's mass)
 //   split_pick   one workgroup a row: threshold among the candidates, the draw over the list or over chunks and inside one of them; beside them
-//                the copy of the rows
+//                the copy of the rows, but for draws by a mass alone of more than 128 rows, where split_sum writes it (launch_split)
 // Thresholds, masses and picks are those of one workgroup (integer sums over the same numbers); a threshold that is not among the candidates
 // (ties across the bound, top-k above 1024) falls to draw_from_row, as there.
 // Bound: the launches' ends and starts and each one's chain of a few dependent loads and barriers (5.5, 12, 10 us of 27 at 64 x 151936 with top-k, where
@@ -1005,7 +1005,8 @@ __global__ __launch_bounds__(kRowThreads, VEC && MASS ? 8 : 4) void split_sum_ke
   static_assert(kRowThreads == 1 << 10, "columns");
   const int at_row = tid >> (VEC ? log_cols - 3 : log_cols), at_col = VEC ? (tid & ((cols >> 3) - 1)) * 8 : tid & (cols - 1);
   auto slot = [&](int e) { return VEC ? at_row * cols + at_col + e : (at_row + e * (high / 8)) * cols + at_col; };
-  const uint32_t width = (uint32_t)vocab, step = kTile * split;  // (a sum of two of them fits 32 bits)
+  // (a row has fewer than split x kMostPerGroup = 2^21 numbers at most, a step is 2^17 at most: their sums, six steps past the row included, fit 32 bits)
+  const uint32_t width = (uint32_t)vocab, step = kTile * split;
   auto index = [&](uint32_t base, int e) { return base + (VEC ? at_row : at_row + e * (high / 8)) * kRowThreads + g * cols + at_col + (VEC ? e : 0); };
   // Several tiles are asked for ahead, all that a row of 151936 has on four workgroups: with one, a tile took a loaded memory's latency.
   constexpr int kDeep = !VEC ? 1 : MASS ? 2 : DT == MSGL_F32 ? 3 : 5;

@@ -471,10 +471,11 @@ def attn_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_ca
                  sm_scale: float, tile_order: Optional[torch.Tensor] = None, impl: Optional[int] = None,
                  ranges: Tuple[int, int] = (1, 0), workspace: Optional[torch.Tensor] = None, pairs: bool = False) -> None:
     """tile_order: optional int32 [total_tiles] schedule of the q tiles (heaviest first); impl: None = process default
-    (PREFILL_IMPL), 0 = 4 the DMA-staged kernel, 2 its register-staged predecessor (include/msgl_hip.h; anything else is
-    refused by the library).  tile_cu / total_tiles / tile_order are in units of prefill_q_tile(impl) query rows.
+    (PREFILL_IMPL), 0 = 4 the DMA-staged kernel, 6 the same with two heads of a kv head a workgroup (an even number of heads each), 2 its register-staged
+    predecessor (include/msgl_hip.h; anything else is refused by the library).  tile_cu / total_tiles / tile_order are in units of prefill_q_tile(impl) query rows.
     ranges: (key ranges of a q tile at most, 64-key tiles of each) for the DMA-staged kernel, see `prefill_ranges`; more than one needs a
-    workspace of prefill_ranges_workspace_bytes.  pairs: two heads a workgroup where that kernel runs without ranges, see `prefill_pairs`."""
+    workspace of prefill_ranges_workspace_bytes.  pairs: where impl (or the default) is 0 or 4 and there are no ranges, 6 in its
+    place, see `prefill_pairs`."""
     _need_cuda(out, q, k_cache, v_cache, page_table, seq_lens, cu_seqlens_q, tile_cu)
     if impl is None:
         impl = PREFILL_IMPL
