@@ -5,8 +5,7 @@
     python -m torch.distributed.run --nnodes=1 --nproc-per-node N --master-addr 127.0.0.1 \
         --master-port P bench.py --gpus N --steps K --warmup W        (N > 1: TP = N, one rank per GPU)
 
-Workload (metric quoted on Qwen3-14B TP=1; fits one GPU => configs[2]'s model on
-configs[1]'s request shape): Qwen3-14B bf16, 256 sequences, context lengths drawn from the
+Workload: Qwen3-14B bf16 on one GPU, 256 sequences, context lengths drawn from the
 token-weighted context distribution of the reference's offline benchmark
 (benchmark/offline/bench.py:11-31: in/out 100..1024, mean context per decoded token 902.8),
 page_size 256, temperature 0.6, seeded N(0, 0.02^2) weights (no checkpoints offline), synthetic
@@ -83,7 +82,7 @@ def bench_contexts(num_seqs: int, seed: int = 0):
 def cpu_baseline(cfg, contexts, rounds: int = 3):
     """Oracle (oracle/ref_model.py, torch eager fp32) timed on the host cores ON THE GPU WORKLOAD'S SHAPE: ONE decoder
     layer of the same dims at the full batch (256 requests, the bench's own contexts, K/V gathered through a page
-    table) + embedding, final norm and LM head, x num_layers (BASELINE.md section 4).  A reported baseline, not a target."""
+    table) + embedding, final norm and LM head, x num_layers.  A reported baseline, not a target."""
     from oracle import ref_model
 
     avail = len(os.sched_getaffinity(0))
@@ -96,7 +95,7 @@ def cpu_baseline(cfg, contexts, rounds: int = 3):
     w = ref_model.random_weights(
         type("C", (), dict(cfg.__dict__, vocab_size=small_vocab, tie_word_embeddings=True))(), torch.float32, num_layers=L)
     w.lm_head = torch.randn((cfg.vocab_size, cfg.hidden_size), generator=g) * 0.02
-    # bf16 weights, fp32 accumulation (BASELINE.md section 4): every weight rounded to bf16, held and multiplied as fp32
+    # bf16 weights, fp32 accumulation: every weight rounded to bf16, held and multiplied as fp32
     # (torch's CPU bf16 matmul is several times slower than its fp32 one on these hosts and would flatter the GPU)
     bf = lambda t: t.to(torch.bfloat16).float()  # noqa: E731
     w.embed, w.final_norm, w.lm_head = bf(w.embed), bf(w.final_norm), bf(w.lm_head)
@@ -119,9 +118,9 @@ def cpu_baseline(cfg, contexts, rounds: int = 3):
         return time.perf_counter() - t0
 
     # thread count: torch-eager on a many-core host is not monotone in threads (the per-request attention loop and the
-    # M = 256 GEMMs want different counts; 64 threads measured 3.5x SLOWER per layer than 8 on one box): one layer at each
+    # M = 256 GEMMs want different counts; 64 threads measured 3.5x SLOWER per layer than 8 on one host): one layer at each
     # of a few counts, the fastest is the baseline's (and is what `cores` reports)
-    # (all 256 cores of a GPU box took 287 s for ONE layer in round 6 -- oversubscribed per-request attention loop: never probed)
+    # (all 256 cores of a host took 287 s for ONE layer -- oversubscribed per-request attention loop: never probed)
     counts = [int(forced)] if forced else sorted({c for c in (8, 16, 32, 64) if c <= avail} or {avail})
     torch.set_num_threads(counts[0])
     run(no_head, lens)  # warm-up (thread pool, allocator)
@@ -194,7 +193,7 @@ def gemm_traffic_over_algorithmic():
     except Exception:
         return None, None
     man = f["manifest"]
-    if "path_ops" in man:  # round 5 on: the manifest names the launches of the step's path and their algorithmic bytes
+    if "path_ops" in man:  # the manifest names the launches of the step's path and their algorithmic bytes
         ops_, algo = man["path_ops"], man["path_algorithmic_bytes"]
     else:
         ops_ = [k for k in f["per_launch"] if not k.startswith("gate_up g3") and not k.startswith("tail reduce")]
@@ -205,7 +204,7 @@ def gemm_traffic_over_algorithmic():
 
 def measure_prefill_attention(device, hq: int, hkv: int, budget: int = 16384):
     """MFMA roofline of the prefill attention kernel on ONE chunk of the bench's own prompts (the first
-    `budget` prompt tokens, no cache hit), one layer: causal flops (SURVEY.md 8d) / HIP-event time."""
+    `budget` prompt tokens, no cache hit), one layer: causal flops / HIP-event time."""
     from tools.microbench import MFMA_PEAK_TFLOPS, prefill_case, prefill_chunk_lens, time_us
     from mini_sglang_amd import ops
 
@@ -284,13 +283,13 @@ def _known_answers(f_all_reduce, f_all_gather, rank: int, world: int, device, nu
 
 
 def check_collectives(comm, rank: int, world: int, device) -> dict:
-    """PREFLIGHT on the links the run is about to use (VERDICT r5 item 7), printed to stderr by rank 0 BEFORE the workload
+    """PREFLIGHT on the links the run is about to use, printed to stderr by rank 0 BEFORE the workload
     starts and carried in the final line, so that a multi-GPU run that dies later still says how far the links got:
       * `ncclCommCount` / the device every RCCL rank bound (`rccl_ranks_seen`, `rccl_devices`);
       * the reference's known answers (tests/kernel/test_comm.py:96-149) through RCCL and through the peer-to-peer kernels,
         each at the three message sizes of the path -- 256 KB (one-shot range), 2.6 MB ([256, hidden] decode all-reduce),
         84 MB ([8192, hidden] prefill chunk; RCCL only unless the mapped buffers were sized for it);
-      * all-reduce time and bus bandwidth per path and size: busbw = 2 (n - 1) / n x bytes / t (SURVEY 8d), to be read
+      * all-reduce time and bus bandwidth per path and size: busbw = 2 (n - 1) / n x bytes / t, to be read
         against one xGMI link (153 GB/s, ring) and all seven (peer-to-peer kernels)."""
     import torch.distributed as dist
 
@@ -502,10 +501,10 @@ def run_workload(args, model_name: str, rank: int, local_rank: int, world: int, 
     #  * `us_per_launch` (what `achieved` / `frac` use): ONE event pair around 40 launches queued back to back, divided by
     #    40 -- covers both kernels and the gaps between them, the stream never idles (as inside the captured step); this is
     #    the figure rocprofv3 --kernel-trace reproduces as (attention + merge) average duration (+ ~0.3 us of gaps);
-    #  * `us_per_launch_event_gap_median` (round 5's headline, kept for comparison): an event after every launch, median
+    #  * `us_per_launch_event_gap_median` (kept for comparison): an event after every launch, median
     #    distance of consecutive events -- reads ~3 % LOW (an event's stamp is taken before the merge kernel has drained);
-    #  * `us_per_launch_idle_stream` (rounds 1-4): one synchronised event pair per launch -- adds the host-to-idle-GPU
-    #    launch latency to every sample (5-8 % high, box dependent).
+    #  * `us_per_launch_idle_stream`: one synchronised event pair per launch -- adds the host-to-idle-GPU
+    #    launch latency to every sample (5-8 % high, depending on the machine).
     reps, tot = 30, 0.0
     for _ in range(reps):
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -538,7 +537,7 @@ def run_workload(args, model_name: str, rank: int, local_rank: int, world: int, 
         pair.append(e0.elapsed_time(e1) * 1e3 / pair_reps)
     attn_us = sorted(pair)[1]  # partial + merge kernels of one layer, median of three runs of 40
     S = sum(lens_now)
-    attn_bytes = S * 2 * hkv * D * it + 2 * B * hq * D * it + S * 4 + 2 * B * 4  # SURVEY.md section 8d
+    attn_bytes = S * 2 * hkv * D * it + 2 * B * hq * D * it + S * 4 + 2 * B * 4
     achieved = attn_bytes / attn_us / 1e3
     # whole-step algorithmic bytes per rank: streamed weights + KV read/write + logits
     kv_tok = 2 * mcfg.num_layers * hkv * D * it
@@ -598,7 +597,7 @@ def run_workload(args, model_name: str, rank: int, local_rank: int, world: int, 
             "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBPS, "traffic": traffic,
             "traffic_source": traffic_src, "traffic_over_algorithmic": traffic_ratio, "us_per_launch": attn_us,
             "us_per_launch_event_gap_median": attn_us_gap, "us_per_launch_idle_stream": attn_us_idle,
-            "timing": "us_per_launch = one HIP-event pair around 40 launches (attention + merge each) queued back to back / 40, median of 3: covers both kernels; event_gap_median = round 5's method (reads ~3 % low); idle_stream = one synchronised pair per launch (rounds 1-4, reads 5-8 % high)",
+            "timing": "us_per_launch = one HIP-event pair around 40 launches (attention + merge each) queued back to back / 40, median of 3: covers both kernels; event_gap_median = an event after every launch (reads ~3 % low); idle_stream = one synchronised pair per launch (rounds 1-4, reads 5-8 % high)",
             "algorithmic_bytes": attn_bytes, "launch_shape": shape,
         },
         "prefill_roofline": prefill_roofline,
@@ -747,7 +746,7 @@ def main() -> None:
     assert world == args.gpus, f"--gpus {args.gpus} but WORLD_SIZE={world}"
     assert torch.cuda.is_available(), "bench.py needs MI355X GPUs (there is no CPU fallback)"
     # MSGL_BENCH_SHARE_GPU=1: every rank on cuda:0 with the peer-to-peer communicator only (RCCL refuses two ranks per
-    # device) -- exercises the whole N > 1 code path of this file on a 1-GPU box; not a measurement
+    # device) -- exercises the whole N > 1 code path of this file on one GPU; not a measurement
     share_gpu = os.environ.get("MSGL_BENCH_SHARE_GPU") == "1"
     if not share_gpu and torch.cuda.device_count() < world:
         raise SystemExit(f"bench.py --gpus {world}: only {torch.cuda.device_count()} GPU(s) visible "
@@ -761,7 +760,7 @@ def main() -> None:
 
     if world > 1:
         os.environ.setdefault("MASTER_ADDR", "127.0.0.1")
-        # one node: rendezvous and the RCCL bootstrap over loopback (the box's hostname may not resolve);
+        # one node: rendezvous and the RCCL bootstrap over loopback (the hostname may not resolve);
         # the data path is xGMI peer-to-peer either way
         os.environ.setdefault("GLOO_SOCKET_IFNAME", "lo")
         os.environ.setdefault("NCCL_SOCKET_IFNAME", "lo")
@@ -784,9 +783,9 @@ def main() -> None:
     mcfg = PRESETS[args.model]
     contexts = bench_contexts(args.batch)
     ms_per_step = result["ms_per_step"]
-    # the metric's second configuration ("Qwen3-32B TP=4"): at --gpus 4 the same request set on Qwen3-32B.
+    # the metric's second configuration, Qwen3-32B TP=4: at --gpus 4 the same request set on Qwen3-32B.
     # $MSGL_BENCH_SECOND_MODEL runs a second workload at any N (how the two-workloads-in-one-process path -- communicators
-    # torn down and rebuilt, a second engine in the freed memory -- is exercised on a 1-GPU box with a small model)
+    # torn down and rebuilt, a second engine in the freed memory -- is exercised on one GPU with a small model)
     second = os.environ.get("MSGL_BENCH_SECOND_MODEL") or ("qwen3-32b" if world == 4 and args.model == "qwen3-14b" else None)
     if second and not args.no_second_config:
         key = "qwen3_32b_tp4" if (second == "qwen3-32b" and world == 4) else f"second_config_{second}_tp{world}"
@@ -802,10 +801,10 @@ def main() -> None:
     if ref_runs and args.model == "qwen3-14b" and world == 1:
         try:
             d = json.loads(ref_runs[-1].read_text())
-            # "committed": recorded by the GPU test suite on a box of the same kind and kept under profiles/; this file may
+            # "committed": recorded by the GPU test suite on a machine of the same kind and kept under profiles/; this file may
             # not import oracle/_ref (the reference), so it cannot re-measure it
             # stale = the sources have changed since that run was recorded (fingerprint stored by the test that wrote the file;
-            # files from before round 5 carry none): the number then describes an EARLIER state of the kernels
+            # older files carry none): the number then describes an EARLIER state of the kernels
             fp = product_code_fingerprint()
             result["reference_driven"] = {"kind": "committed", "decode_ms_per_step": d["decode_ms_per_step_median"], "tokens_per_s": d["tokens_per_s"],
                                           "vs_this_run_ms_per_step": d["decode_ms_per_step_median"] / ms_per_step,
@@ -814,7 +813,7 @@ def main() -> None:
                                           "stale": d.get("code_fingerprint") != fp}
         except Exception as e:
             result["reference_driven"] = {"error": f"{type(e).__name__}: {e}"}
-    # the ONLINE half of the metric (BASELINE config 4's protocol): the reference's Scheduler fed a synthetic Qwen-like trace at
+    # the ONLINE half of the metric: the reference's Scheduler fed a synthetic Qwen-like trace at
     # the reference's scale list through the plugin -- recorded by tools/trace_replay.py (it imports oracle/_ref, this file may
     # not) and committed under profiles/; stale when the product sources have changed since
     if world == 1:
@@ -841,7 +840,7 @@ def main() -> None:
                 result["parity"] = {"error": f"{type(e).__name__}: {e}"}
     if rank == 0 and world == 1 and not args.no_e2e:
         # the reference's own throughput definition (benchmark/offline/bench.py:32-38): sum(max_tokens) / wall of one
-        # generate() over 256 requests, in/out 100..1024, prefill included, one untimed warm-up -- BASELINE configs 1, 2
+        # generate() over 256 requests, in/out 100..1024, prefill included, one untimed warm-up
         from tools.offline_bench import run as offline_run
 
         print("[bench] step measured", file=sys.stderr, flush=True)  # the whole runs below say nothing for two minutes
@@ -856,7 +855,7 @@ def main() -> None:
                 result["e2e_offline"][name] = {"error": f"{type(e).__name__}: {e}"}
             print(f"[bench] {name} measured", file=sys.stderr, flush=True)
         # the reference's DEFAULT page size (P/engine/config.py:25: page_size = 1; its FlashInfer backend always sees token-granular
-        # tables, P/attention/fi.py:179-187): the same workload on a token-granular pool (round 6: the matrix-core decode kernel
+        # tables, P/attention/fi.py:179-187): the same workload on a token-granular pool (the matrix-core decode kernel
         # gathers token rows by per-lane addresses)
         try:
             r = offline_run(args.model, 256, 0.6, 1, os.environ.get("MSGL_GEMM_TUNE", "full"), device)

@@ -8,7 +8,7 @@
  * are relative to the reference root, `P/` = python/minisgl/, `C/` =
  * python/minisgl/kernel/csrc/.
  *
- * Conventions (mirrors the reference FFI contract, SURVEY.md section 8b):
+ * Conventions (mirrors the reference FFI contract):
  *   - plain pointers + sizes + explicit strides, no torch / DLPack types;
  *   - all device pointers are raw HIP device addresses; `stream` is a
  *     hipStream_t passed as void* (the caller's current stream, cf.
@@ -117,7 +117,7 @@ int msgl_rope_neox_inplace(void* q, void* k, const void* positions, int position
                            int dtype, void* stream);
 
 /* ------------------------------------------------------------------------
- * Fused per-token pass over the qkv row (SURVEY.md section 8f rank 1):
+ * Fused per-token pass over the qkv row:
  *   [q-norm, k-norm (optional)] -> NeoX RoPE (in place on q,k) -> scatter k,v
  * rows to the KV pool at out_loc.  Equivalent to the op sequence of
  * P/layers/attention.py:47-56 + P/kvcache/mha_pool.py:45-56.
@@ -214,11 +214,11 @@ int msgl_attn_decode_small(void* out, const void* q, const void* k, const void* 
                            int64_t kv_stride_tok, int64_t kv_stride_head, int64_t out_stride, float sm_scale, int dtype,
                            void* stream);
 /* Which partial-attention kernel msgl_attn_decode_plan / msgl_attn_decode use from now on (process-wide; plan and
- * launch must be made under the same choice): 0 = default = the matrix-core kernel for every slot_run (round 6: token-granular
+ * launch must be made under the same choice): 0 = default = the matrix-core kernel for every slot_run (token-granular
  * tables, slot_run < 16, are gathered by per-lane addresses on the same kernel; whole-line nt requests with K transposed through
- * LDS where a token row is >= 1 KB, round 5's 16-row x 64-B direct-to-operand requests below), 1 = the round-1 streaming kernel
+ * LDS where a token row is >= 1 KB, 16-row x 64-B direct-to-operand requests below), 1 = the streaming kernel
  * only; for timing and diagnosis also 22 / 32 = matrix-core kernel held to 2 / 3 waves per SIMD (two-stage request ring), 60 / 61 =
- * the default variant with the round-5 / the whole-line request shape forced (same bits either way), 72 = variant 22 with the
+ * the default variant with the direct-to-operand / the whole-line request shape forced (same bits either way), 72 = variant 22 with the
  * in-kernel combine instead of the merge kernel, 71 = the default variant by number (72's A/B partner), 92 = variant 22 with the
  * products left out (what the request pattern alone costs), 93 = variant 22 leaving clock stamps (msgl_attn_decode_trace), 94 =
  * variant 22 without the per-piece record prefetch.  Also settable by MSGL_DECODE_IMPL before the first call.  Both kernels meet
@@ -462,8 +462,8 @@ int msgl_ro_gemm_nt(void* out, const void* x, const void* w, int M, int N, int K
  * Native radix prefix tree (libmsgl_hip.so, csrc/radix.cpp; host code, no device work).
  * Replaces: the tree walk of RadixPrefixCache -- _tree_walk, RadixTreeNode.split_at / get_match_len, lock_handle,
  * evict, _collect_leave_nodes_for_evict (python/minisgl/kvcache/radix_cache.py:65-77, 111-130, 147-175, 189-230),
- * which the reference runs in Python with one dict lookup, one tensor slice and one tvm-ffi call per node
- * (SURVEY.md section 8f rank 4).  The tree owns keys (token ids), reference counts, timestamps and the two size counters;
+ * which the reference runs in Python with one dict lookup, one tensor slice and one tvm-ffi call per node.
+ * The tree owns keys (token ids), reference counts, timestamps and the two size counters;
  * the VALUE tensors (pool slots, device memory) and the clock stay with the caller (mini-sglang_amd/radix.py), which
  * mirrors each reported split / eviction on them.  Nodes are named by int64 ids (the root is id 0).
  * Children are an insertion-ordered map and eviction is CPython's heapq over timestamps, so that every observable

@@ -1,6 +1,6 @@
 """MI355X-native paged-attention serving core behind mini-sglang's operator API.
 
-Layout (only what the hot path needs, SURVEY.md section 8):
+Layout (only what the hot path needs):
   csrc/              hand-written HIP kernels for gfx950 + the C-ABI (include/msgl_hip.h)
   _lib.py, ops.py    ctypes binding and torch-facing wrappers (pointers + strides + stream)
   kernel.py          mirror of minisgl.kernel   (store_cache, indexing, fast_compare_key, init_pynccl: peer-to-peer +

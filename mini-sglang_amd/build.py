@@ -3,7 +3,7 @@
     python mini-sglang_amd/build.py            # build what is stale
     python mini-sglang_amd/build.py --force
 
-Outputs (git-ignored, shipped to the GPU box by gpurun because they are in-tree):
+Outputs (git-ignored, in-tree):
     mini-sglang_amd/lib/libmsgl_hip.so    every kernel + host helpers   (include/msgl_hip.h)
     mini-sglang_amd/lib/libmsgl_comm.so   RCCL communicator             (links librccl)
     mini-sglang_amd/lib/libmsgl_gemm.so   projection GEMMs + tuner      (links libhipblaslt)
@@ -106,7 +106,7 @@ def build_all(force: bool = False, verbose: bool = True, only=None) -> dict[str,
     # (a checkout that ships built libraries does not ship the objects)
     link = [HIPCC, "-shared", "-fPIC"]
     libs = {
-        # --no-undefined: a kernel whose host-side launch stub went missing must fail HERE, not at dlopen on the GPU box
+        # --no-undefined: a kernel whose host-side launch stub went missing must fail HERE, not at dlopen
         "hip": (HIP_SOURCES, [*link, f"--offload-arch={ARCH}", "-Wl,--no-undefined"], []),
         "mix": (MIX_SOURCES, [*link, f"--offload-arch={ARCH}", "-Wl,--no-undefined"], []),
         "comm": (COMM_SOURCES, link, ["-L", str(ROCM / "lib"), "-lrccl", f"-Wl,-rpath,{ROCM / 'lib'}"]),

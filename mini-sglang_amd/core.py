@@ -1,9 +1,9 @@
-"""Attribute holders for the standalone driver (engine.py / offline.py / bench.py on the GPU box).
+"""Attribute holders for the standalone driver (engine.py / offline.py / bench.py).
 
 When the reference is installed, its own `minisgl.core` objects (P/core.py:16-136) are what reach the
 attention backend and the KV pool; this module is NOT a replacement for them.  The backend only reads
 attributes -- `Batch.{reqs, padded_reqs, phase, positions, out_loc, input_ids, attn_metadata}` and
-`Req.{table_idx, cached_len, device_len, extend_len}` (SURVEY.md section 8b) -- so the standalone driver hands
+`Req.{table_idx, cached_len, device_len, extend_len}` -- so the standalone driver hands
 it these minimal holders carrying the same attribute names and nothing else of the reference's class bodies.
 """
 from __future__ import annotations

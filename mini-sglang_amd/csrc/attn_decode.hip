@@ -598,7 +598,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, kMinW) void attn_decode_mfma_kerne
   dlds_char* img = (dlds_char*)lds + wv * (kLines ? 8192 : 4096);
   // kLines: request j of a tile covers token rows 4 j + qd, lane piece `tok` (16 B) of the head's 256-B row -- whole 128-B
   // lines per request, which is what lets the nt policy pay (see the banner above the kernel)
-  // !kRun (token-granular page tables, round 6): lane group qd owns the tile's tokens 4 qd .. 4 qd + 3 -- ONE 16-byte table
+  // !kRun (token-granular page tables): lane group qd owns the tile's tokens 4 qd .. 4 qd + 3 -- ONE 16-byte table
   // read per tile gives it their four pool slots -- and request kk fetches token 4 qd + kk's row by a per-lane address
   int wr_off[4], rd_off[8], kwr_off[4], krd_off[4];
 #pragma unroll
@@ -1084,7 +1084,7 @@ static int decode_impl() {
   return g_decode_impl;
 }
 // matrix-core kernel variants: code = 10 * (waves per SIMD) + ring stages.  Two stages (deeper rings measured the same or
-// slower in rounds 2-3: profiles/r02d_decode_ab.txt, and again in round 6 on the whole-line request shape -- 3 / 4 stages at
+// slower: profiles/r02d_decode_ab.txt, and again on the whole-line request shape -- 3 / 4 stages at
 // two waves per SIMD and 3 / 4 / 6 stages at one: 146.5 ... 151.8 us against 147.6 at Qwen3-14B TP1, profiles/
 // r06h_decode_ab_ring_depth_and_residency.txt; their instantiations are not kept) at the residency the plan is made
 // for -- three waves per SIMD where the streaming kernel also has three (G <= 2), two otherwise.  92 = variant 22 without the
@@ -1103,23 +1103,23 @@ static int launch_decode_mfma(const DecodeParams& p, int batch, int capacity, hi
   const int64_t waves = (int64_t)decode_target_slots(G, p.hv, capacity, p.max_bs) * p.hv;
   // select code 72: the last-arriving piece of a request combines the partial sums inside the kernel instead of the merge
   // launch (needs the arrival counters to cover the kv heads and 32-bit offsets into the partial sums).  Bit-identical
-  // to the merge kernel.  NOT the default: round 4 measured it INSIDE the captured 256-sequence Qwen3-14B step (tools/
-  // step_ab.py) at -45 / -25 / +-0 us per step on three boxes (one launch boundary per layer less), but stand-alone on the
+  // to the merge kernel.  NOT the default: measured INSIDE the captured 256-sequence Qwen3-14B step (tools/
+  // step_ab.py) it is -45 / -25 / +-0 us per step on three machines (one launch boundary per layer less), but stand-alone on the
   // TP-shard shapes it LOSES 3-6 us per layer (14B TP4 49.1 vs 45.8 us, 70B TP8 35.4 vs 29.6, Qwen3-0.6B 174.3 vs 171.8:
   // the combiner's dependent sc1 round trips at the very end of a short kernel; profiles/r04_decode_ab_with_combine_as_impl0.txt, r04_decode_ab_final.txt) and 8 us at
   // B = 32.  Select code 71 = the default variant by its number (A/B partner of 72).
-  // Request shape.  Round 6 (tools/kv_stream_probe.hip, profiles/r06a_kv_stream_probe.txt): whole-line requests (4 token rows x
-  // 256 B) under the nt policy stream the paged pool at 6.8 TB/s where round 5's 16 rows x 64 B reach 5.9 (and LOSE with nt:
+  // Request shape (tools/kv_stream_probe.hip, profiles/r06a_kv_stream_probe.txt): whole-line requests (4 token rows x
+  // 256 B) under the nt policy stream the paged pool at 6.8 TB/s where 16 rows x 64 B reach 5.9 (and LOSE with nt:
   // nt lines bypass the L1, so the second 64-B half of a line is fetched again).  The price is K's trip through the wave's
   // LDS image; it pays where the stream is long -- token rows of >= 1 KB (>= 4 local kv heads): 14B TP1 171.7 -> 153.6 us,
   // Qwen3-0.6B 165.6 -> 145.1 -- and is neutral to -3 % on the short TP-shard launches (profiles/r06b_decode_ab.txt), which keep
-  // the direct-to-operand shape.  Select 60 / 61 force the round-5 / the whole-line shape (A/B; same bits either way).
+  // the direct-to-operand shape.  Select 60 / 61 force the direct-to-operand / the whole-line shape (A/B; same bits either way).
   const bool lines = decode_impl() == 61 || (decode_impl() != 60 && p.kv_stride_tok * 2 >= 1024);
   const bool combine = decode_impl() == 72 && p.hv <= kTicketHeads &&
                        (int64_t)capacity * p.hq * 128 * (int64_t)sizeof(float) < (1ll << 31);
-  // token-granular page tables (slot_run < 16; the reference's default page_size = 1, P/engine/config.py:25): round 6 gives
-  // them the matrix-core kernel too -- whole-line requests by per-lane addresses, one 16-byte table read per lane group and
-  // tile -- instead of the round-1 streaming kernel
+  // token-granular page tables (slot_run < 16; the reference's default page_size = 1, P/engine/config.py:25) take
+  // the matrix-core kernel too -- whole-line requests by per-lane addresses, one 16-byte table read per lane group and
+  // tile -- instead of the streaming kernel
   const bool run = p.slot_run >= 16;
 #define MSGL_MFMA_LAUNCH(STAGES, WAVES, MINW, ...)                                                    \
   attn_decode_mfma_kernel<T, STAGES, WAVES, MINW, __VA_ARGS__>                                        \
@@ -1196,7 +1196,7 @@ extern "C" int msgl_attn_decode_select(int impl) {
   MSGL_REQUIRE(impl == 0 || impl == 1 || impl == 22 || impl == 32 || impl == 71 || impl == 72 || impl == 92 || impl == 93 || impl == 94 || impl == 60 || impl == 61,
                "attn_decode_select: impl %d (0 = default, 1 = streaming kernel only, 22 / 32 = matrix-core kernel with "
                "2 / 3 waves per SIMD (a two-stage request ring), 71 / 72 = the default variant with the merge kernel forced / with the "
-               "in-kernel combine forced, 60 / 61 = the default variant with round 5's 16-row x 64-B requests / with whole-line nt requests forced)", impl);
+               "in-kernel combine forced, 60 / 61 = the default variant with 16-row x 64-B requests / with whole-line nt requests forced)", impl);
   g_decode_impl = impl;
   return MSGL_OK;
 }

@@ -8,7 +8,7 @@
 // (pynccl.cu:81-90, 105-123).  Here the default is the direct in-place collective on the
 // caller's tensor (no extra HBM round trip); staging through a buffer registered with
 // ncclCommRegister is kept as an opt-in (MSGL_COMM_STAGE=1) until it can be measured on an
-// 8-GPU xGMI node -- this round only had 1-GPU boxes.
+// 8-GPU xGMI node.
 #include <hip/hip_runtime.h>
 #include <rccl/rccl.h>
 #include <stdarg.h>
@@ -65,7 +65,7 @@ struct msgl_comm {
   void* reg_handle = nullptr;  // ncclCommRegister handle, may stay null
   bool stage = false;          // MSGL_COMM_STAGE=1
   bool shortcut1 = true;       // world == 1: skip the library call (MSGL_COMM_NO_SHORTCUT=1 keeps it, so that
-                               // a 1-GPU box can exercise RCCL's enqueue path, e.g. under hipGraph capture)
+                               // one GPU can exercise RCCL's enqueue path, e.g. under hipGraph capture)
 };
 
 extern "C" {

@@ -1,4 +1,4 @@
-// Peer-to-peer collectives over xGMI for decode-size messages (SURVEY.md section 8f rank 3).
+// Peer-to-peer collectives over xGMI for decode-size messages.
 //
 // The reference stages messages <= max_bytes through a symmetric buffer (ncclMemAlloc +
 // ncclCommWindowRegister(NCCL_WIN_COLL_SYMMETRIC), C/src/pynccl.cu:81-90, 105-123) so that NCCL's symmetric

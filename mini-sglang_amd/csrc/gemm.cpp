@@ -1,4 +1,4 @@
-// Decode/prefill projection GEMMs (SURVEY.md section 8f rank 2): a thin C-ABI over the
+// Decode/prefill projection GEMMs: a thin C-ABI over the
 // hipBLASLt *library* kernels with a per-shape solution search.
 //
 // The reference leaves these to `F.linear` (P/layers/linear.py:32,103,124, embedding.py:98), i.e.

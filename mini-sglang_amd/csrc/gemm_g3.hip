@@ -1,7 +1,7 @@
 // Full-batch decode projection GEMM, generation 3 (128 < M <= 256): loader waves + matrix waves.
 //     out[M, N] = x[M, K] . w[N, K]^T        (torch F.linear layout, bf16 / fp16, fp32 accumulate)
 //
-// What round 2 measured on the register-staged kernel (gemm_m256.hip, profiles/r02b_m256_gemm_ablation.txt): weight
+// Measured on the register-staged kernel (gemm_m256.hip, profiles/r02b_m256_gemm_ablation.txt): weight
 // stream alone 62 us, activation re-reads through L2 alone 29 us, both 89 us, both + MFMA 110 us -- the three are
 // ADDITIVE because every wave issues its own loads: a vector-memory instruction that meets a full request queue
 // blocks the in-order wave that issued it, and with it that wave's ds_reads and MFMAs.  This kernel separates the roles:
@@ -18,7 +18,7 @@
 //     stream the next segment's first two steps.
 //   * work split as in gemm_m256.hip: `full` tiles whole, the rest cut into `tail_split` k-slices spread over all
 //     workgroups (fp32 slabs, added in slice order by a second kernel or by the consumer of the projection).
-//   * tried in round 4 and dropped (profiles/r04a_g3_store_policy_and_loader_roles.json, same-box, bit-identical outputs):
+//   * tried and dropped (profiles/r04a_g3_store_policy_and_loader_roles.json, one machine, bit-identical outputs):
 //     sc1 (write-through) or nt slab stores -- 32.1 -> 38.8 / 36.6 us (qkv), 25.2 -> 34.7 / 31.9 (o), and the pair with the
 //     slab-consuming norm loses as much; two loaders issuing only x pieces and two only w pieces instead of a quarter of both
 //     each -- within 0.5 us everywhere (the x and w terms add per CU whichever wave issues them).

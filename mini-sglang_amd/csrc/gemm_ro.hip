@@ -1,7 +1,7 @@
-// Decode projection GEMM, "row-owner" generation (round 5), planned for 3 <= M <= 256 (takes M >= 1):
+// Decode projection GEMM, "row-owner" generation, planned for 3 <= M <= 256 (takes M >= 1):
 //     out[M, N] = x[M, K] . w[N, K]^T        (torch F.linear layout, bf16 / fp16, fp32 accumulate)
 //
-// What gemm_g3.hip left on the table ("What bounds the full-batch projections"):
+// What gemm_g3.hip left on the table:
 //   * its tiles are 128 weight rows wide whatever N is, so gate_up (N = 34816 = 272 tiles on 256 CUs) runs a second round
 //     for 6 % of its work (a 20-us tail + a reduce launch), qkv / o / down fill 224 / 240 / 240 of 256 CUs, and at batches
 //     <= 128 the accumulator budget is half empty;
@@ -19,7 +19,7 @@
 //     tile's units: MTW = 2 up to M = 256 (<= 9 units per tile), MTW = 1 up to M = 128 (<= 18 units per tile: half the x
 //     bytes per weight byte).  Token tiles past M are neither loaded nor multiplied: the x traffic follows M in steps of 8 rows.
 //   * the k loop body is compiled per tile width (switch on the width, uniform): straight-line MFMA blocks, no guards inside.
-// By the per-CU law of DESIGN section 3 (t = w_cu / 27.6 B/ns + x_cu / 100 B/ns) gate_up at M = 256 costs 50 + 26 us against
+// By the per-CU law (t = w_cu / 27.6 B/ns + x_cu / 100 B/ns) gate_up at M = 256 costs 50 + 26 us against
 // g3's 88 + tail and the library's 104 + 7 (activation launch); at M = 128: 50 + 13.
 //
 // LDS image as g3: 128-B rows (64 k), 16-B chunk c of row r at slot c ^ ((r >> 1) & 7), applied on the SOURCE address of the

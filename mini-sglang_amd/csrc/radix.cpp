@@ -1,7 +1,7 @@
 // Native radix prefix tree (host code): the structure walk of the reference's RadixPrefixCache
 // (P/kvcache/radix_cache.py:17-236) -- child lookup by first page, first-difference compare, page-aligned split,
 // reference counts, LRU eviction over unreferenced leaves -- behind the C ABI (include/msgl_hip.h, msgl_radix_*).
-// the reference walks the tree in Python, one dict lookup, one tensor slice and one
+// The reference walks the tree in Python, one dict lookup, one tensor slice and one
 // tvm-ffi call (fast_compare_key) per node.
 //
 // What stays in Python (mini-sglang_amd/radix.py): the per-node VALUE tensors (KV pool slots, device memory) and

@@ -2,8 +2,8 @@
 
 Host-side mirror of the reference's L4 (P/engine/engine.py:29-211, graph.py:21-171,
 sample.py:24-75) restricted to what drives the hot path.  The reference's own Engine runs
-unchanged on the plugin when `minisgl` is installed; this one exists for the
-GPU box, where only this repository is present.
+unchanged on the plugin when `minisgl` is installed; this one exists for
+machines where only this repository is present.
 """
 from __future__ import annotations
 

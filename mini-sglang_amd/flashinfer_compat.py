@@ -3,7 +3,7 @@
 The reference reaches flashinfer through attributes bound in constructors
 (P/layers/norm.py:10-30, P/layers/rotary.py:35-37) and lazy imports
 (P/layers/activation.py:10,16, P/engine/sample.py:30); a module exposing the same names
-with the same argument meaning is a drop-in (SURVEY.md section 8b).  Everything forwards to
+with the same argument meaning is a drop-in.  Everything forwards to
 the hand-written gfx950 kernels via ops.py.
 """
 from __future__ import annotations

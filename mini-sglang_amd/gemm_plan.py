@@ -1,4 +1,4 @@
-"""Per-shape kernel choice for the projection GEMMs of a decode step (SURVEY.md section 8f rank 2).
+"""Per-shape kernel choice for the projection GEMMs of a decode step.
 
 `F.linear` of the reference (P/layers/linear.py:32,103,124, P/layers/embedding.py:98) is one library call
 with the library's heuristic; here each (M, N, K) a captured decode graph will launch is timed once, before

@@ -96,7 +96,7 @@ class P2PCommunicator:
     """Peer-to-peer collectives over mapped buffers (csrc/comm_p2p.hip): the symmetric-buffer path of the reference's
     NCCLWrapper (C/src/pynccl.cu:81-90, 105-123) for messages <= max_bytes.  Same surface as PyNCCLCommunicator.
     Needs only a CPU group for the one-time exchange of IPC handles, so -- unlike RCCL -- two ranks may also share
-    one device (how the N > 1 path is exercised on a 1-GPU box)."""
+    one device (how the N > 1 path is exercised on one GPU)."""
 
     def __init__(self, rank: int, world_size: int, cpu_group, max_bytes: int, *, one_shot_max_bytes: int = 256 << 10,
                  blocks: int = 32) -> None:

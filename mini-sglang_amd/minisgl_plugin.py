@@ -1,14 +1,14 @@
 """Registers the MI355X core into an installed `minisgl` (the reference), without touching its
 source: after `install()` the reference's scheduler, radix cache, engine, models and server run
-unchanged with `--attn hip` (see INTEGRATION.md for the two-line bootstrap).
+unchanged with `--attn hip`.
 
-Seams filled (SURVEY.md section 8b):
+Seams filled:
   attention backend   SUPPORTED_ATTENTION_BACKENDS.register("hip")        P/attention/__init__.py:19-40
   minisgl.kernel      store_cache / indexing / fast_compare_key / init_pynccl   P/kernel/__init__.py
   flashinfer names    rmsnorm, fused_add_rmsnorm, apply_rope_with_cos_sin_cache_inplace,
                       silu_and_mul, gelu_and_mul, sampling.*              P/layers/norm.py:10-30 ...
 
-and, so that the path the reference drives is the path bench.py measures (SURVEY.md section 8f):
+and, so that the path the reference drives is the path bench.py measures:
   F.linear            the name `F` of P/layers/linear.py:32,103,124 and P/layers/embedding.py:98 resolves to a
                       proxy of torch.nn.functional whose `linear` is ops.linear (bias / CPU / odd dtypes fall
                       back to torch)
@@ -601,7 +601,7 @@ def _install_deterministic_decode_order(only_under_tp: bool = False) -> None:
     """`DecodeManager.running_reqs` is a `set` of eq=False dataclasses (P/scheduler/decode.py:12,35, P/core.py:28): the
     decode batch order -- and with it the order `allocate_paged` hands out free pages (P/scheduler/cache.py:42-53) -- is
     the set's iteration order, i.e. object addresses.  Opt-in: schedule decode batches in uid order, so that two runs
-    of the same request stream produce the same batches and KV block indices (SURVEY.md section 8f rank 4)."""
+    of the same request stream produce the same batches and KV block indices."""
     from minisgl.core import Batch
     from minisgl.scheduler.decode import DecodeManager
 
@@ -634,7 +634,7 @@ def _install_deterministic_decode_order(only_under_tp: bool = False) -> None:
 def _install_native_radix(replace_radix: bool) -> None:
     """Cache type "hip_radix" in the reference's registry (P/kvcache/__init__.py:23,59-64): RadixPrefixCache with the
     tree walk in native code (radix.py, csrc/radix.cpp).  replace_radix=True also points the name "radix" (the
-    scheduler's default, BASELINE configs 2-3) at it."""
+    scheduler's default) at it."""
     import minisgl.kvcache as kvc
     from minisgl.core import get_global_ctx
     from minisgl.kvcache.base import BaseCacheHandle, BasePrefixCache, InsertResult, MatchResult, SizeInfo

@@ -2,8 +2,8 @@
 
 This is the caller of the path, restated compactly from the reference's composition
 (P/models/qwen3.py:18-81, P/models/llama.py, P/models/utils.py:25-123, P/layers/*): the
-reference's own model classes run unchanged on top of the plugin (INTEGRATION.md); this copy
-exists because /root/reference is not present on the GPU box and bench.py / smoke need a
+reference's own model classes run unchanged on top of the plugin; this copy
+exists because the reference need not be installed and bench.py / smoke need a
 driver.  GEMMs are the library's (hipBLASLt) as in the reference (P/layers/linear.py:32), reached through
 msgl_gemm_nt so that the per-shape solution search of csrc/gemm.cpp applies (`tune_gemms`); everything
 else goes through the hand-written gfx950 kernels.
@@ -33,7 +33,7 @@ _FUSE_SILU = os.environ.get("MSGL_DISABLE_FUSED_SILU") != "1"
 # projection that consumes them is the row-streaming kernel (A/B switch; the results are bit-identical either way)
 _ROWSTREAM_FUSE = os.environ.get("MSGL_DISABLE_ROWSTREAM_FUSE") != "1"
 # all-reduce + residual add + RMSNorm as one peer-to-peer launch (csrc/comm_p2p.hip): OPT-IN.  The only measurement
-# available without a multi-GPU box -- one rank's shard with looped-back collectives, bench.py --rank-shard 4 -- has it
+# available on one GPU -- one rank's shard with looped-back collectives, bench.py --rank-shard 4 -- has it
 # SLOWER than the two launches (10.24 vs 9.07 ms per step): the kernel keeps the few dozen blocks its flag barriers want,
 # and those cannot move the 10 MB of local x / residual traffic of a 256-row batch as fast as the 256-block norm kernel.
 _FUSE_AR_NORM = os.environ.get("MSGL_FUSED_ALLREDUCE_NORM") == "1"
@@ -59,7 +59,7 @@ class ModelConfig:
 
 
 PRESETS: Dict[str, ModelConfig] = {
-    # public HF config.json values (SURVEY.md section 8 table)
+    # public HF config.json values
     "qwen3-0.6b": ModelConfig(28, 16, 8, 128, 1024, 151936, 3072, tie_word_embeddings=True, name="Qwen3-0.6B"),
     "qwen3-14b": ModelConfig(40, 40, 8, 128, 5120, 151936, 17408, name="Qwen3-14B"),
     "qwen3-32b": ModelConfig(64, 64, 8, 128, 5120, 151936, 25600, name="Qwen3-32B"),

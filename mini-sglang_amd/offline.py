@@ -2,11 +2,11 @@
 continuous decode with graph padding), producing the (Batch, positions, out_loc, page table)
 inputs the hot path consumes.
 
-It plays the part of the reference's scheduler for benchmarks on the GPU box, where the
+It plays the part of the reference's scheduler for benchmarks where the
 reference itself is absent.  Only the tensor glue of P/scheduler/scheduler.py:204-267,
 P/scheduler/cache.py:42-53,127-146 and P/scheduler/table.py:4-12 is restated (page-aligned slot
 allocation, `out_loc = page_table[(table_idx, position)]`, device-side token feedback through
-`token_pool`); admission policy, radix reuse and I/O are out of scope (SURVEY.md section 8).
+`token_pool`); admission policy, radix reuse and I/O are out of scope.
 Host work per step is vectorised (numpy), and nothing synchronises with the device: step N+1 is
 prepared while step N runs, like the reference's overlap loop.
 """

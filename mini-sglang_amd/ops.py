@@ -692,14 +692,14 @@ def rowstream_linear(x: torch.Tensor, w: torch.Tensor, depth: int = 16, out: Opt
 def rowstream_planned(M: int, w: torch.Tensor, mode: int = 0):
     """(ring depth, variant) if the plan of `linear(x [M, K], w)` is the row-streaming kernel and that kernel also takes
     the shape with staging `mode`, else None: the decoder layer folds a neighbouring row kernel into the projection only
-    where the projection already is this kernel (the folded launch then costs what the plain one does, DESIGN.md section 3)."""
+    where the projection already is this kernel (the folded launch then costs what the plain one does)."""
     if M > ROWSTREAM_MAX_M or not _SKINNY_PLAN:
         return None
     N, K = w.shape
     key = (w.device.index or 0, M, N, K, K, w.stride(0), _dt(w))
     plan = _SKINNY_PLAN.get(key)
     # (a shape whose plan is the row-owner kernel is NOT this kernel's, whatever the skinny table still holds: linear() looks at
-    # _RO_PLAN first, and the fold must take the same kernel as the plain launch -- ADVICE r5)
+    # _RO_PLAN first, and the fold must take the same kernel as the plain launch)
     if not plan or plan[0] > 0 or _WSTREAM_PLAN.get(key) or _RO_PLAN.get(key) or not rowstream_supported(M, N, K, mode, -plan[0]):
         return None
     return plan[1], -plan[0]
@@ -1479,7 +1479,7 @@ def apply_candidate(key, spec) -> None:
     dev, M, N, K, ldx, ldw, dt = key
     if kind in ("lib", "hand", "ro", "fused", "ro_silu"):
         # linear() / linear_silu() consult the skinny / weight-streaming tables BEFORE these: a candidate timed under its own
-        # label must be the kernel that runs (ADVICE r5; the re-ranking runs at the largest graph batch, where they are empty)
+        # label must be the kernel that runs (the re-ranking runs at the largest graph batch, where they are empty)
         _SKINNY_SILU_PLAN.pop(key, None)
         _SKINNY_PLAN.pop(key, None)
         if kind != "hand":

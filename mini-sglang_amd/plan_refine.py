@@ -9,7 +9,7 @@ by 0.14 ms per step.  Which candidate the back-to-back search ranks first also v
 are re-ranked WHERE THEY RUN: for each projection of the largest graph batch in turn (biggest first) each candidate is
 made the plan, the graph is re-captured and a synthetic full batch replayed (median of 20 individually timed replays).
 A challenger replaces the search's pick only if it is faster by `margin` (0.5 %) AND wins a confirmation round against a
-fresh measurement of the incumbent by the same margin (round 3 ranked on the mean of 6 replays with a 0.2 % threshold:
+fresh measurement of the incumbent by the same margin (the mean of 6 replays with a 0.2 % threshold lay
 inside run-to-run noise, plans flipped between runs).
 
 Used by this repository's engine (engine.Engine.refine_plans_in_graph) and, through `minisgl_plugin.install()`, by the

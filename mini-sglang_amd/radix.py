@@ -3,7 +3,7 @@
 Mirrors `RadixPrefixCache` / `RadixCacheHandle` (python/minisgl/kvcache/radix_cache.py:80-203): same methods, same
 arguments, same results for the same calls -- the structure (keys, reference counts, timestamps, LRU order) lives in
 the native tree, the per-node value tensors (KV pool slots, device memory) stay here and follow every split and
-eviction the tree reports.  SURVEY.md section 8(f) rank 4.
+eviction the tree reports.
 
 `NativeRadixTree` has no dependency on the reference; `make_prefix_cache_class()` binds the cache to the reference's
 abstract base classes when it is plugged in (minisgl_plugin registers it as cache type "hip_radix").

@@ -1,4 +1,4 @@
-"""Vectorised versions of the per-step tensor glue of the reference's scheduler (SURVEY.md section 8(f) rank 4):
+"""Vectorised versions of the per-step tensor glue of the reference's scheduler:
 `_make_positions`, `_make_input_tuple`, `_make_write_tuple` (python/minisgl/scheduler/scheduler.py:236-267) build
 their index tensors with one Python-level tensor operation PER REQUEST (256 `torch.arange(out=...)` / `fill_` calls for
 a full decode batch); here each is a handful of numpy operations over the whole batch.  Same signatures, same
