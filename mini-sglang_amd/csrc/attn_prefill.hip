@@ -905,7 +905,7 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   p.stretch = ranges == 1 && total <= 256 ? even : 0;
   // Waves without rows leave the matrix cores to the others (40 heads on 8, 14 requests of 14 - 41 tokens after 300: 25.7 -> 23.7 us; 64 on 8, 20 of 65 -
   // 187 after 2000 287 -> 259; 29 of 100 - 1024 on 40 heads 229 -> 225).  Not in one and a half rounds: who then ends early takes two of the last
-  // workgroups onto one CU (768: 8 of 93 - 218 after 2000 120 -> 132; 740: 83 -> 90; from 768 on none of 100 sizes more than 2 % slower).
+  // workgroups onto one CU (768: 8 of 93 - 218 after 2000 120 -> 132; 740: 83 -> 90; above, none of 100 sizes more than 2.5 % slower).
   const int64_t wanted = total * ranges;
   p.idle = wanted <= 512 || wanted > 768;
   // Where all workgroups start at once the time is one workgroup's, and only full tiles go in whole rows by way of LDS; else from about half a tile on.
