@@ -213,6 +213,25 @@ int msgl_attn_decode_small(void* out, const void* q, const void* k, const void* 
                            int num_q_heads, int num_kv_heads, int head_dim, int64_t q_stride, int64_t k_stride, int64_t v_stride,
                            int64_t kv_stride_tok, int64_t kv_stride_head, int64_t out_stride, float sm_scale, int dtype,
                            void* stream);
+/* All decoder layers of a small decode batch (csrc/decode_layers.hip): for each layer add + RMSNorm, qkv projection, per-head RMSNorm (both weights or
+ * nullptr) and NeoX RoPE, K / V store at out_loc, attention over seq_lens[b] keys (the last one is the new token, as in msgl_attn_decode_small), o projection,
+ * add + RMSNorm, gate and up projection with SiLU.mul, down projection.  x [batch, hidden] is the residual stream in front of the first layer; the
+ * last down projection's rows go to y_out and the residual stream without them to res_out (both [batch, hidden] contiguous, x may be neither).
+ * Weights are contiguous [rows, columns]; gate_up_interleaved: gate_up rows in blocks of 32 gate, 32 up.  head_dim 128, batch 1 .. 8, hidden and
+ * intermediate size multiples of 256; _supported says whether a CU's share of a layer fits its LDS.
+ * `workspace` is zero before its first launch and belongs to these launches, one at a time.  The launch has one workgroup per CU, which wait for
+ * each other, and none for one that is not running: a launch that finds CUs taken goes on without them.  Capturable. */
+typedef struct {
+  const void *input_norm, *qkv, *q_norm, *k_norm, *o, *post_norm, *gate_up, *down;
+  void *k_cache, *v_cache;
+} msgl_decode_layer_t;
+int msgl_decode_layers_supported(int batch, int hidden, int num_q_heads, int num_kv_heads, int intermediate);
+int64_t msgl_decode_layers_workspace_bytes(int batch, int layers, int hidden, int num_q_heads, int num_kv_heads, int intermediate);
+int msgl_decode_layers(void* y_out, void* res_out, const void* x, const msgl_decode_layer_t* layer, int layers, const int32_t* positions,
+                       const float* cos_sin, const int32_t* out_loc, const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
+                       const int32_t* seq_lens, void* workspace, int64_t workspace_bytes, int batch, int hidden, int num_q_heads,
+                       int num_kv_heads, int head_dim, int intermediate, int gate_up_interleaved, int64_t kv_stride_tok,
+                       int64_t kv_stride_head, float eps, float sm_scale, int dtype, void* stream);
 /* Which partial-attention kernel msgl_attn_decode_plan / msgl_attn_decode use from now on (process-wide; plan and
  * launch must be made under the same choice): 0 = default = the matrix-core kernel for every slot_run (token-granular
  * tables, slot_run < 16, are gathered by per-lane addresses on the same kernel; whole-line nt requests with K transposed through

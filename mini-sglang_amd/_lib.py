@@ -31,6 +31,10 @@ ABI_VERSION = 5
 _p, _i, _l, _f = C.c_void_p, C.c_int, C.c_int64, C.c_float
 _u64, _sz = C.c_uint64, C.c_size_t
 
+class DecodeLayer(C.Structure):  # msgl_decode_layer_t
+    _fields_ = [(n, _p) for n in ("input_norm", "qkv", "q_norm", "k_norm", "o", "post_norm", "gate_up", "down", "k_cache", "v_cache")]
+
+
 # name -> (restype, argtypes); mirrors include/msgl_hip.h one to one
 HIP_SIGNATURES = {
     "msgl_last_error": (C.c_char_p, []),
@@ -67,6 +71,9 @@ HIP_SIGNATURES = {
     "msgl_attn_decode_small_workspace_bytes": (_l, [_i, _i, _i]),
     "msgl_attn_decode_small": (_i, [_p, _p, _p, _p, _p, _p, _f, _p, _p, _p, _p, _p, _p, _l, _p, _p, _p, _l, _i, _i, _i, _i, _i,
                                     _l, _l, _l, _l, _l, _l, _f, _i, _p]),
+    "msgl_decode_layers_supported": (_i, [_i, _i, _i, _i, _i]),
+    "msgl_decode_layers_workspace_bytes": (_l, [_i, _i, _i, _i, _i, _i]),
+    "msgl_decode_layers": (_i, [_p, _p, _p, _p, _i, _p, _p, _p, _p, _l, _p, _p, _p, _l, _i, _i, _i, _i, _i, _i, _i, _l, _l, _f, _f, _i, _p]),
     "msgl_attn_prefill": (
         _i,
         [_p, _p, _p, _p, _p, _l, _p, _p, _p, _p, _i, _i, _i, _i, _i, _l, _l, _l, _l, _f, _i, _p, _i, _p],

@@ -113,6 +113,7 @@ class HipAttnBackend:
                  for b in range(1, self._small_heads // self.kv_heads + 1))
         self._workspace = torch.empty(max([ops.attn_decode_workspace_bytes(self.capacity, self.qo_heads, self.head_dim), *small]),
                                       dtype=torch.uint8, device=self.device)
+        self._layers_workspace: Optional[torch.Tensor] = None
         # graph state
         self.capture_bs: List[int] = []
         self.max_graph_bs = 0
@@ -156,6 +157,24 @@ class HipAttnBackend:
                    cos_sin: torch.Tensor, layer_id: int, batch: Any) -> torch.Tensor:
         """qk-norm, RoPE, K / V store and attention of a batch that `small_decode` says yes to, from the projection's rows."""
         return self._attend_small(q, k, v, layer_id, batch, q_norm_w=q_norm_w, k_norm_w=k_norm_w, eps=eps, positions=positions, cos_sin_cache=cos_sin)
+
+    def takes_layers(self, batch: Any, hidden: int, intermediate: int) -> bool:
+        """Whether all layers of the batch's decode step go in one launch (csrc/decode_layers.hip): a batch of `small_decode`, of a model whose layer fits the
+        compute units' LDS and gives every other one of them, at least, rows of every product."""
+        return (batch.positions.dtype == batch.out_loc.dtype == torch.int32 and hidden // 2 >= int(_lib.lib().msgl_device_cu_count()) and self.small_decode(batch)
+                and ops.decode_layers_supported(batch.attn_metadata.batch, hidden, self.qo_heads, self.kv_heads, intermediate))
+
+    def decode_layers(self, x: torch.Tensor, layers: Any, interleaved: bool, eps: float, positions: torch.Tensor, cos_sin: torch.Tensor, batch: Any):
+        """Every layer of a batch that `takes_layers` says yes to: the last down projection's rows and the residual stream without them."""
+        md: HipAttnMetadata = batch.attn_metadata
+        if self._layers_workspace is None:  # like the decode workspace: one step at a time
+            inter, (hidden, most) = layers[0].down.shape[1], (x.shape[1], self._small_heads // self.kv_heads)
+            need = max(ops.decode_layers_workspace_bytes(b, len(layers), hidden, self.qo_heads, self.kv_heads, inter) for b in range(1, most + 1)
+                       if ops.decode_layers_supported(b, hidden, self.qo_heads, self.kv_heads, inter))
+            self._layers_workspace = torch.zeros(need, dtype=torch.uint8, device=self.device)
+        tokens = [self._kv_tokens(i) for i in range(len(layers))]
+        return ops.decode_layers(x, layers, [k for k, _ in tokens], [v for _, v in tokens], positions, cos_sin, batch.out_loc, self.ctx.page_table, md.req_rows,
+                                 md.seq_lens, self._layers_workspace, self.qo_heads, interleaved, eps, self.scale)
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_id: int, batch: Any) -> torch.Tensor:
         """Reference contract (fa.py:48-65): persist k, v at batch.out_loc, then attend.  A decode batch's out_loc is where its requests'

@@ -37,6 +37,7 @@ HIP_SOURCES = [
     "norm_rope_act.hip",
     "attn_decode.hip",
     "attn_decode_small.hip",
+    "decode_layers.hip",
     "attn_prefill.hip",
     "sampling.hip",
     "gemm_skinny.hip",

@@ -8,7 +8,8 @@ driver.  GEMMs are the library's (hipBLASLt) as in the reference (P/layers/linea
 msgl_gemm_nt so that the per-shape solution search of csrc/gemm.cpp applies (`tune_gemms`); everything
 else goes through the hand-written gfx950 kernels.
 
-Two execution modes, bit-identical by construction (tests/test_gpu_model.py):
+Two execution modes, bit-identical by construction (tests/test_gpu_model.py) but for small models' small decode batches, whose layers
+go in one launch with `fused` (another order of the products' sums, csrc/decode_layers.hip):
   fused=False  the reference's op order through its seams: q_norm, k_norm, rope (flashinfer
                names), attn_backend.forward (store_kv + attention)   [P/layers/attention.py:47-57]
   fused=True   one qk_norm_rope_store kernel + attn_backend.attend
@@ -375,7 +376,16 @@ class DenseDecoder:
             residual, spare = spare, residual
             return r
 
-        for li, lw in enumerate(self.layers):
+        layers = self.layers
+        if small and self.tp_size == 1 and x.dtype == kv.dtype and getattr(backend, "takes_layers", lambda *a: False)(batch, cfg.hidden_size, self.inter):
+            # a small model's small batch: all layers in one launch, which leaves the last down_proj's rows for the final norm
+            x, residual = backend.decode_layers(x, layers, self.gate_up_ilv, cfg.rms_norm_eps, batch.positions, self.cos_sin, batch)
+            layers = ()
+            if not batch.is_prefill and norm_plan(self.lm_head):
+                pending = x
+            else:
+                fi.fused_add_rmsnorm(x, residual, self.final_norm, cfg.rms_norm_eps)
+        for li, lw in enumerate(layers):
             if residual is None:  # P/layers/norm.py:35-36
                 residual = x
                 x = fi.rmsnorm(x, lw.input_norm, cfg.rms_norm_eps)

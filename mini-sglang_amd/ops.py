@@ -7,6 +7,7 @@ function does (e.g. `indexing` output), none synchronises.
 """
 from __future__ import annotations
 
+import ctypes as C
 import functools
 import os
 from typing import Optional, Tuple
@@ -397,6 +398,55 @@ def attn_decode_small(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
         ),
         "attn_decode_small",
     )
+
+
+def decode_layers_supported(batch: int, hidden: int, num_q_heads: int, num_kv_heads: int, intermediate: int) -> bool:
+    """Whether a CU's share of such a layer fits its LDS (decode_layers)."""
+    return bool(lib().msgl_decode_layers_supported(batch, hidden, num_q_heads, num_kv_heads, intermediate))
+
+
+def decode_layers_workspace_bytes(batch: int, layers: int, hidden: int, num_q_heads: int, num_kv_heads: int, intermediate: int) -> int:
+    n = int(lib().msgl_decode_layers_workspace_bytes(batch, layers, hidden, num_q_heads, num_kv_heads, intermediate))
+    check(min(n, 0), "decode_layers_workspace_bytes")
+    return n
+
+
+def decode_layers(x: torch.Tensor, layers, k_caches, v_caches, positions: torch.Tensor, cos_sin_cache: torch.Tensor, out_loc: torch.Tensor,
+                  page_table: torch.Tensor, req_rows: Optional[torch.Tensor], seq_lens: torch.Tensor, workspace: torch.Tensor, num_q_heads: int,
+                  gate_up_interleaved: bool, eps: float, sm_scale: float) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Every decoder layer of a small decode batch in one launch (see msgl_hip.h): x [B, hidden] = the residual stream in front of the first of `layers`
+    (model.LayerWeights); k_caches / v_caches: [slots, Hkv, D] of each.  Returns the last down projection's rows and the residual stream without them."""
+    _need_cuda(x, positions, cos_sin_cache, out_loc, page_table, seq_lens, workspace)
+    layers, k_caches, v_caches = list(layers), list(k_caches), list(v_caches)
+    B, H = x.shape
+    hkv, D = k_caches[0].shape[1:]
+    inter = layers[0].down.shape[1]
+    assert x.is_contiguous() and len(k_caches) == len(v_caches) == len(layers)
+    for t in (*k_caches, *v_caches):
+        assert t.is_cuda and t.dtype == x.dtype and t.shape == k_caches[0].shape and t.stride() == k_caches[0].stride() and t.stride(2) == 1
+    shapes = {"input_norm": (H,), "qkv": ((num_q_heads + 2 * hkv) * D, H), "q_norm": (D,), "k_norm": (D,), "o": (H, num_q_heads * D), "post_norm": (H,),
+              "gate_up": (2 * inter, H), "down": (H, inter)}
+    table = (_lib.DecodeLayer * len(layers))()
+    for entry, lw, kc, vc in zip(table, layers, k_caches, v_caches):
+        for name, shape in shapes.items():
+            w = getattr(lw, name)
+            assert (w is None and name in ("q_norm", "k_norm")) or (w.is_cuda and w.dtype == x.dtype and tuple(w.shape) == shape and w.is_contiguous()), name
+            setattr(entry, name, None if w is None else w.data_ptr())
+        entry.k_cache, entry.v_cache = kc.data_ptr(), vc.data_ptr()
+    assert {t.dtype for t in (positions, out_loc, page_table, seq_lens)} == {torch.int32} and page_table.dim() == 2 and page_table.stride(1) == 1
+    assert min(t.numel() for t in (positions, out_loc, seq_lens)) >= B and all(t.is_contiguous() for t in (positions, out_loc, seq_lens))
+    assert cos_sin_cache.dtype == torch.float32 and cos_sin_cache.is_contiguous() and cos_sin_cache.shape[1] == D
+    y, res = torch.empty_like(x), torch.empty_like(x)
+    check(
+        lib().msgl_decode_layers(
+            y.data_ptr(), res.data_ptr(), x.data_ptr(), C.cast(table, C.c_void_p), len(layers), positions.data_ptr(), cos_sin_cache.data_ptr(),
+            out_loc.data_ptr(), page_table.data_ptr(), page_table.stride(0), req_rows.data_ptr() if req_rows is not None else None, seq_lens.data_ptr(),
+            workspace.data_ptr(), workspace.numel() * workspace.element_size(), B, H, num_q_heads, hkv, D, inter, int(gate_up_interleaved),
+            k_caches[0].stride(0), k_caches[0].stride(1), float(eps), float(sm_scale), _dt(x), _stream(),
+        ),
+        "decode_layers",
+    )
+    return y, res
 
 
 def attn_decode_select(impl: int) -> None:
