@@ -328,6 +328,14 @@ int msgl_sample_filtered_logits_keep(int32_t* out, void* kept, float* kept_tempe
 int msgl_sample_filtered_logits_ws(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
                                    const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
                                    int logits_dtype, uint64_t seed, uint64_t offset, void* workspace, int64_t workspace_bytes, void* stream);
+/* The same with a team of msgl_sample_team_bytes() bytes (16-byte aligned, zero before its first launch, left zero; one launch at a time): draws with a
+ * top-k whose rows' shares fit the workgroups' registers go in one launch.  A workgroup that has waited wait_us for another one's maxima looks them
+ * up itself.  NULL: as above. */
+int64_t msgl_sample_team_bytes(void);
+int msgl_sample_filtered_logits_team(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
+                                     const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
+                                     int logits_dtype, uint64_t seed, uint64_t offset, void* workspace, int64_t workspace_bytes, void* team,
+                                     int64_t team_bytes, int wait_us, void* stream);
 /* Bytes of the workspace above (filtered = 1) or of msgl_sample_from_logits_ws (filtered = has_k = has_p = 0);
  * 0 where one workgroup per row is as good and none is used. */
 int64_t msgl_sample_workspace_bytes(int64_t rows, int64_t vocab, int filtered, int has_k, int has_p);

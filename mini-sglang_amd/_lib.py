@@ -90,6 +90,8 @@ HIP_SIGNATURES = {
     "msgl_sample_filtered_logits": (_i, [_p, _p, _p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p]),
     "msgl_sample_filtered_logits_keep": (_i, [_p, _p, _p, _p, _p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p]),
     "msgl_sample_filtered_logits_ws": (_i, [_p, _p, _p, _p, _p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p, _l, _p]),
+    "msgl_sample_filtered_logits_team": (_i, [_p, _p, _p, _p, _p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p, _l, _p, _l, _i, _p]),
+    "msgl_sample_team_bytes": (_l, []),
     "msgl_sample_workspace_bytes": (_l, [_l, _l, _i, _i, _i]),
     "msgl_sample_from_logits": (_i, [_p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p]),
     "msgl_sample_from_logits_ws": (_i, [_p, _p, _p, _l, _l, _l, _i, _u64, _u64, _p, _l, _p]),

@@ -170,14 +170,22 @@ __device__ __forceinline__ u64 block_prefix_incl(u64 v, u64* lds_w) {
   return v + base;
 }
 
+template <int kCtrl>
+__device__ __forceinline__ u64 add_dpp_u64(u64 v) {
+  const uint32_t lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)v, kCtrl, 0xf, 0xf, true), hi = __builtin_amdgcn_mov_dpp((int)(uint32_t)(v >> 32), kCtrl, 0xf, 0xf, true);
+  return v + ((u64)hi << 32 | lo);
+}
 __device__ __forceinline__ u64 wave_sum_u64(u64 v) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    const uint32_t lo = __shfl_xor((uint32_t)v, d, 64);
-    const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), d, 64);
-    v += ((u64)hi << 32) | lo;
-  }
-  return v;
+  v = add_dpp_u64<kDppXor1>(v);
+  v = add_dpp_u64<kDppXor2>(v);
+  v = add_dpp_u64<kDppHalfMirror>(v);
+  v = add_dpp_u64<kDppRowMirror>(v);
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false), hi = __builtin_amdgcn_permlane16_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
+  const uint32_t l0 = lo[0], l1 = lo[1], h0 = hi[0], h1 = hi[1];
+  v = ((u64)h0 << 32 | l0) + ((u64)h1 << 32 | l1);
+  const auto lo2 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false), hi2 = __builtin_amdgcn_permlane32_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
+  const uint32_t m0 = lo2[0], m1 = lo2[1], i0 = hi2[0], i1 = hi2[1];
+  return ((u64)i0 << 32 | m0) + ((u64)i1 << 32 | m1);
 }
 
 __device__ __forceinline__ u64 block_sum_u64(u64 v, u64* lds_w) {
@@ -328,16 +336,24 @@ __device__ __forceinline__ uint32_t select_bits(const Src& src, int64_t vocab, u
   return prefix;
 }
 
+// inclusive prefix sum over a wave's lanes: within rows of 16, then row by row
+__device__ __forceinline__ int wave_prefix_incl(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2 and 3
+  return x;
+}
+
 // A lower bound of the `target`-th largest of the workgroup's 1024 weights, one per thread: the lower end of the 8th of an octave that holds it,
 // 0 below 2^-126.  One histogram, spread over all octaves up to weight 1: the exact one takes four, the upper ones with all 1024 in a few bins
 // (64 rows x 151936: 5 us of a draw).  (With 16ths down to 2^-63 only, rows whose k-th largest number lies below went to the radix levels: at
 // temperatures under 0.5 that is a distance of 20 between the logits.  256 x 151936 of deviation 10 at temperatures of 0.4 - 1: 109 us, now 42.)
-__device__ __forceinline__ uint32_t kth_bound(uint32_t bits, int target, uint32_t* hist, uint32_t* s_one) {
+__device__ __forceinline__ uint32_t kth_bound_in(uint32_t bits, int target, uint32_t* hist, uint32_t* s_one) {  // hist and *s_one are zero
   constexpr int kShift = 20;  // bins of a weight's bits; weight 1 is bin 1016
   const int tid = threadIdx.x;
-  hist[tid] = 0u;
-  if (tid == 0) *s_one = 0u;
-  __syncthreads();
   if (bits >> kShift) atomicAdd(&hist[min(bits >> kShift, 1023u)], 1u);
   __syncthreads();
   if (tid < 64) {  // lane l owns the bins 1023 - 16 l ... 1008 - 16 l
@@ -349,12 +365,7 @@ __device__ __forceinline__ uint32_t kth_bound(uint32_t bits, int target, uint32_
     }
 #pragma unroll
     for (int q = 0; q < 16; ++q) mine += c[q];
-    int above = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int o = __shfl_up(above, d, 64);
-      if (tid >= d) above += o;
-    }
+    int above = wave_prefix_incl(mine);
     above -= mine;
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
@@ -364,6 +375,13 @@ __device__ __forceinline__ uint32_t kth_bound(uint32_t bits, int target, uint32_
   }
   __syncthreads();
   return *s_one;
+}
+
+__device__ __forceinline__ uint32_t kth_bound(uint32_t bits, int target, uint32_t* hist, uint32_t* s_one) {
+  hist[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) *s_one = 0u;
+  __syncthreads();
+  return kth_bound_in(bits, target, hist, s_one);
 }
 
 constexpr int kList = 2048;          // candidates of a row that the short path holds (= kBins: it reuses the histograms)
@@ -392,9 +410,8 @@ __device__ __forceinline__ u64 mass_target(float pp, u64 kept_mass) {
   return target;
 }
 
-// Philox's number of row r, scaled to [0, total): (total * x) >> 32 without 128-bit arithmetic
-__device__ __forceinline__ u64 draw_below(u64 total, u64 seed, u64 ctr) {
-  const uint32_t x = Philox::draw(seed, ctr);
+// Philox's number x, scaled to [0, total): (total * x) >> 32 without 128-bit arithmetic
+__device__ __forceinline__ u64 draw_below(u64 total, uint32_t x) {
   return (total >> 32) * (u64)x + (((total & 0xffffffffull) * (u64)x) >> 32);
 }
 
@@ -402,9 +419,10 @@ __device__ __forceinline__ u64 draw_below(u64 total, u64 seed, u64 ctr) {
 // list.  kept_mass: set to the whole row's mass where only a mass is given.  s_pick is -1 on entry.
 template <class Src>
 __device__ __forceinline__ bool draw_from_list(const Src& src, RowShared& sh, int* __restrict__ out, int n, uint32_t floor_bits, bool by_count, int64_t k,
-                                               float pp, int64_t vocab, u64 seed, u64 offset, u64& kept_mass) {
+                                               float pp, int64_t vocab, u64 seed, u64 offset, int64_t r, u64& kept_mass) {
   const int tid = threadIdx.x;
   const bool by_mass = !by_count;
+  const uint32_t number = Philox::draw(seed, offset + r);  // (beside the first barrier's wait)
   // Every candidate against every other one: `cp` candidates side by side, the others in `parts` portions whose sums meet in LDS.
   // 64 rows, lists of some 110: two such comparisons and the rest of the draw take 24 us with one thread a candidate, 8 so.
   constexpr int kOwn = kList / kRowThreads;
@@ -496,7 +514,7 @@ __device__ __forceinline__ bool draw_from_list(const Src& src, RowShared& sh, in
   }
   sh.acc[tid] = 0;
   const u64 total = block_sum_u64(loc, sh.lds_w);
-  const u64 u = draw_below(total, seed, offset + blockIdx.x);
+  const u64 u = draw_below(total, number);
 #pragma unroll
   for (int e = 0; e < kOwn; ++e) {
     const int c = c0 + e * kRowThreads;
@@ -513,14 +531,14 @@ __device__ __forceinline__ bool draw_from_list(const Src& src, RowShared& sh, in
     if (tid < n && u >= sh.acc[tid] && u < sh.acc[tid] + sh.h_mass[tid]) sh.s_pick = sh.s_index[tid];
     __syncthreads();
   }
-  if (tid == 0) out[blockIdx.x] = sh.s_pick < 0 ? 0 : sh.s_pick;
+  if (tid == 0) out[r] = sh.s_pick < 0 ? 0 : sh.s_pick;
   return true;
 }
 
 // The draw by three radix levels over the whole row and a walk in index order.  kept_mass: the whole row's, where it is known.
 template <class Src>
 __device__ __forceinline__ void draw_from_row(const Src& src, RowShared& sh, int* __restrict__ out, int64_t k, float pp, int64_t vocab, u64 seed, u64 offset,
-                                              u64 kept_mass) {
+                                              int64_t r, u64 kept_mass) {
   const int tid = threadIdx.x;
   const bool has_k = k >= 1 && k < vocab;
   uint32_t thr_bits = 0u;  // keep set = { bits >= thr_bits, p > 0 }
@@ -581,7 +599,7 @@ __device__ __forceinline__ void draw_from_row(const Src& src, RowShared& sh, int
     if (i < w) before += sh.lds_w[i];
     total += sh.lds_w[i];
   }
-  const u64 u = draw_below(total, seed, offset + blockIdx.x);
+  const u64 u = draw_below(total, Philox::draw(seed, offset + r));
   if (total > 0 && u >= before && u < before + wave_mass) {  // exactly one wave
     u64 run = before;
     // strips of 8 x 64 indices: their sum first, the indices one by one only in the strip that holds u
@@ -618,7 +636,7 @@ __device__ __forceinline__ void draw_from_row(const Src& src, RowShared& sh, int
     }
   }
   __syncthreads();
-  if (tid == 0) out[blockIdx.x] = sh.s_pick < 0 ? 0 : sh.s_pick;  // degenerate row (all-zero mass): fall back to the first index
+  if (tid == 0) out[r] = sh.s_pick < 0 ? 0 : sh.s_pick;  // degenerate row (all-zero mass): fall back to the first index
 }
 
 // One 1024-thread workgroup per row.
@@ -681,8 +699,8 @@ __device__ __forceinline__ void sample_row(Src src, int* __restrict__ out, int64
     n = sh.s_n;
   }
   u64 kept_mass = kNoMass;
-  if (list_bits != kNoDigit && n <= kList && draw_from_list(src, sh, out, n, floor_bits, by_count, k, pp, vocab, seed, offset, kept_mass)) return;
-  draw_from_row(src, sh, out, k, pp, vocab, seed, offset, kept_mass);
+  if (list_bits != kNoDigit && n <= kList && draw_from_list(src, sh, out, n, floor_bits, by_count, k, pp, vocab, seed, offset, blockIdx.x, kept_mass)) return;
+  draw_from_row(src, sh, out, k, pp, vocab, seed, offset, blockIdx.x, kept_mass);
 }
 
 __global__ __launch_bounds__(kRowThreads) void sample_kernel(int* __restrict__ out, const float* __restrict__ probs,
@@ -860,6 +878,7 @@ __global__ __launch_bounds__(kRowThreads) void sample_logits_kernel(int* __restr
 //                the copy of the rows, but for draws by a mass alone of more than 128 rows, where split_sum writes it (launch_split)
 // Thresholds, masses and picks are those of one workgroup (integer sums over the same numbers); a threshold that is not among the candidates
 // (ties across the bound, top-k above 1024) falls to draw_from_row, as there.
+// Draws with a top-k take sample_team_kernel where a row's share fits its registers.
 // Bound: the launches' ends and starts and each one's chain of a few dependent loads and barriers (5.5, 12, 10 us of 27 at 64 x 151936 with top-k, where
 // the reads take 8 and the exponentials 2; it was 31 with a tile of split_sum asked for at a time, divisions and dependent scalar loads in front of the first
 // load and a barrier more a tile).  us a draw, one workgroup per row -> shared: see split_of.
@@ -1261,7 +1280,7 @@ template <class M>
 __device__ __forceinline__ void draw_from_chunks(RowShared& sh, int* __restrict__ out, u64 mine, int64_t vocab, int64_t chunk, u64 seed, u64 offset, M mass_at) {
   const int tid = threadIdx.x;
   const u64 incl = block_prefix_incl(mine, sh.lds_w);
-  const u64 total = block_sum_u64(mine, sh.lds_w), u = draw_below(total, seed, offset + blockIdx.x);
+  const u64 total = block_sum_u64(mine, sh.lds_w), u = draw_below(total, Philox::draw(seed, offset + blockIdx.x));
   if (tid == 0) sh.s_n = -1;
   __syncthreads();
   if (mine && u >= incl - mine && u < incl) {
@@ -1287,6 +1306,33 @@ __device__ __forceinline__ void draw_from_chunks(RowShared& sh, int* __restrict_
     __syncthreads();
     if (u < run) break;
   }
+}
+
+// The lists of a row's workgroups one behind the other, in sh's indices and bits; lane g of each wave has list g's length.  false: not all candidates are listed
+__device__ __forceinline__ bool gather_lists(RowShared& sh, const u64* __restrict__ list, int count, int split, int& n) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  int upto = min(count, kPart + kList);  // (their lengths in the lanes, the places before each in `upto`)
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) {
+    const int o = __shfl_up(upto, d, 64);
+    if (lane >= d) upto += o;
+  }
+  const bool listed = !__any(count > kPart) && __shfl(upto, split - 1, 64) <= kList;
+  n = listed ? __shfl(upto, split - 1, 64) : 0;
+  for (int c = tid; c < n; c += kRowThreads) {
+    int g = 0, from = 0;
+    for (int q = 0; q < split - 1; ++q) {
+      const int end = __builtin_amdgcn_readlane(upto, q);
+      if (c >= end) {
+        g = q + 1;
+        from = end;
+      }
+    }
+    const u64 e = __hip_atomic_load(list + g * kPart + c - from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // (sample_team_kernel's are of this launch)
+    sh.s_index[c] = (int)(uint32_t)e;
+    sh.h_cnt[c] = (uint32_t)(e >> 32);
+  }
+  return listed;
 }
 
 enum { kPickList = 0, kPickMass = 1, kPickAny = 2 };
@@ -1318,28 +1364,8 @@ __global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc
   const float sum = sc.sum[r * kRowThreads + tid], temperature = temperatures[r];
   const int64_t kk = top_k ? (int64_t)top_k[r] : vocab;
   const float pp = top_p ? top_p[r] : 1.0f;
-  // the workgroups' lists one behind the other (their lengths in the lanes, the places before each in `upto`)
-  int upto = min(count, kPart + kList);
-#pragma unroll
-  for (int d = 1; d < 16; d <<= 1) {
-    const int o = __shfl_up(upto, d, 64);
-    if (lane >= d) upto += o;
-  }
-  const bool listed = !__any(count > kPart) && __shfl(upto, split - 1, 64) <= kList;
-  const int n = listed ? __shfl(upto, split - 1, 64) : 0;
-  for (int c = tid; c < n; c += kRowThreads) {
-    int g = 0, from = 0;
-    for (int q = 0; q < split - 1; ++q) {
-      const int end = __builtin_amdgcn_readlane(upto, q);
-      if (c >= end) {
-        g = q + 1;
-        from = end;
-      }
-    }
-    const u64 e = sc.list[(r * split + g) * kPart + c - from];
-    sh.s_index[c] = (int)(uint32_t)e;
-    sh.h_cnt[c] = (uint32_t)(e >> 32);
-  }
+  int n;
+  const bool listed = gather_lists(sh, sc.list + r * split * kPart, count, split, n);
   LogitRow<DT> src{row, head.mx, 1.0f / temperature * 1.4426950408889634f, 1.0f};
   src.inv = 1.0f / block_reduce_sum(sum, sh.lds_f);
   if (tid == 0) sh.s_pick = -1;
@@ -1347,7 +1373,7 @@ __global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc
   if constexpr (HOW == kPickList) {
     const bool by_count = kk >= 1 && kk < vocab;
     __syncthreads();
-    if (listed && draw_from_list(src, sh, out, n, head.floor_bits, by_count, kk, pp, vocab, seed, offset, kept_mass)) return;
+    if (listed && draw_from_list(src, sh, out, n, head.floor_bits, by_count, kk, pp, vocab, seed, offset, r, kept_mass)) return;
   } else {
     const int64_t chunks = (vocab + chunk - 1) >> __builtin_ctzll(chunk);  // a power of two
     u64 mine = tid < chunks ? sc.chunk[r * kMaxChunks + tid] : 0ull;
@@ -1426,11 +1452,203 @@ __global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc
     }
     __syncthreads();
   }
-  draw_from_row(src, sh, out, kk, pp, vocab, seed, offset, kept_mass);
+  draw_from_row(src, sh, out, kk, pp, vocab, seed, offset, r, kept_mass);
+}
+
+// ------------------------------------------------------------------------------------------
+// Draws with a top-k in one launch
+//
+// split_max, split_sum and split_pick's work where a row's share fits a workgroup's registers: the numbers are read once, each by the thread that adds
+// it to its column's sum, and the row's workgroups tell each other
+//   * their maxima, as packets {value, 1}.  Whoever has waited wait_ticks for one (a workgroup that finds no place on the device beside other work)
+//     looks the numbers up itself, so that no workgroup depends on another one's being resident;
+//   * their columns' sums and candidates, by a count of those that are done.  Nobody waits: the last one draws, the others copy the row.
+// Both are written and read at agent scope (past the L2s); the last one leaves packets and count zero, as it found them, for the next launch.
+// Bound: a chain of launch, first read, packets' way, bound, weights, count's way, draw.
+// 64 rows x 151936 bf16: 3.3 us to the maxima, 0.7 for the packets, 3.3 to the bound (1.5 of it the slowest wave's reads: 64 addresses of 2 bytes each), 3.4 for
+// weights, candidates and sums, 0.8 for the count, 2.9 for lists and sums, 3.7 for the draw.  us a draw with its copy, three launches -> one: 64 x 151936
+// 25.4 -> 19.9, 33 x 151936 23.0 -> 17.9, 8 x 151936 19.4 -> 15.6, 1 x 151936 19.0 -> 15.2, 64 x 98304 21.6 -> 17.0, 64 x 98305 (unaligned rows) 22.9 -> 17.7.
+// Measured on the way (64 x 151936): columns by way of LDS tiles as in split_sum 24.5; the copy from the registers in front of the bound 23.7, by way of LDS
+// 23.5, by the workgroups that do not draw 22.0.
+// ------------------------------------------------------------------------------------------
+constexpr int kTeamDeep = 40;  // numbers of a row that a thread holds,
+constexpr int kTeamParts = 4;  // which are one column's in a quarter of the rows of 1024
+constexpr int kTeamRows = 64;
+constexpr int64_t kTeamBytes = kTeamRows * (kRowThreads * 8 + 64);  // packets, counts 64 bytes apart
+
+// LDS is complete, stores stay under way
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int DT>
+__global__ __launch_bounds__(kRowThreads, 4) void sample_team_kernel(SplitScratch sc, char* __restrict__ team, int* __restrict__ out, const char* __restrict__ logits,
+                                                                     const float* __restrict__ temperatures, const int* __restrict__ top_k,
+                                                                     const float* __restrict__ top_p, int64_t vocab, int64_t row_stride_bytes, int split, u64 seed,
+                                                                     u64 offset, char* __restrict__ kept, float* __restrict__ kept_t, int wait_ticks) {
+  using E = std::conditional_t<DT == MSGL_F32, float, uint16_t>;
+  constexpr int kStep = 8;  // numbers that are looked at together
+  __shared__ RowShared sh;
+  __shared__ __attribute__((aligned(16))) uint32_t hist[kRowThreads];
+  __shared__ float s_sum[kRowThreads / kTeamParts], s_max[kRowThreads / 64];
+  __shared__ uint32_t s_bound;
+  __shared__ int s_n, s_place;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int log_split = __builtin_ctz(split), log_cols = 10 - log_split, cols = 1 << log_cols;  // columns (i mod 1024) of this workgroup: 64, 128 or 256
+  const int64_t r = blockIdx.x >> log_split;
+  const int g = (int)blockIdx.x - (int)r * split;
+  const char* row = logits + r * row_stride_bytes;
+  u64* packets = reinterpret_cast<u64*>(team) + r * kRowThreads;
+  uint32_t* left = reinterpret_cast<uint32_t*>(team + (int64_t)kTeamRows * kRowThreads * 8) + r * 16;
+
+  // part q's rows of 1024 from first on, `here` of them; a wave is in one part (kTeamParts and more: without numbers)
+  const uint32_t width = (uint32_t)vocab;
+  const int rows = (int)((width + kRowThreads - 1) / kRowThreads), per = (rows + kTeamParts - 1) / kTeamParts;
+  const int q = __builtin_amdgcn_readfirstlane(tid >> log_cols), first = q * per, here = q < kTeamParts ? max(0, min(per, rows - first)) : 0;
+  const uint32_t column = g * cols + (tid & (cols - 1)), at0 = (uint32_t)first * kRowThreads + column;
+  uint32_t bits[kTeamDeep];
+#pragma unroll
+  for (int i0 = 0; i0 < kTeamDeep; i0 += kStep) {
+    if (i0 < here) {
+#pragma unroll
+      for (int i = i0; i < i0 + kStep; ++i) bits[i] = __builtin_bit_cast(std::conditional_t<DT == MSGL_F32, uint32_t, uint16_t>, reinterpret_cast<const E*>(row)[min(at0 + i * kRowThreads, width - 1)]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kTeamDeep; ++i) asm volatile("" : "+v"(bits[i]));  // all are asked for before one is used (converted eight at a time: 1.5 us more)
+  auto number = [&](int i) {
+    if constexpr (DT == MSGL_F32) return __uint_as_float(bits[i]);
+    else if constexpr (DT == MSGL_BF16) return __uint_as_float(bits[i] << 16);
+    else return (float)__builtin_bit_cast(_Float16, (uint16_t)bits[i]);
+  };
+  auto in_row = [&](int i) { return i < here && at0 + i * kRowThreads < width; };
+  const float pp = top_p ? top_p[r] : 1.0f, temperature = temperatures[r];
+  const int64_t kk = (int64_t)top_k[r];
+  hist[tid] = 0u;
+  if (tid == 0) s_bound = 0u;
+
+  // ---- the row's 1024 maxima: of four columns' parts each ----
+  float own = -INFINITY;
+#pragma unroll
+  for (int i0 = 0; i0 < kTeamDeep; i0 += kStep) {
+    if (i0 < here) {
+#pragma unroll
+      for (int i = i0; i < i0 + kStep; ++i) own = fmaxf(own, in_row(i) ? number(i) : -INFINITY);
+    }
+  }
+  own = fmaxf(own, dpp_get<kDppXor1>(own));
+  own = fmaxf(own, dpp_get<kDppXor2>(own));
+  if (q < kTeamParts && (tid & 3) == 0)
+    __hip_atomic_store(packets + g * cols + (tid >> 2), 1ull << 32 | __float_as_uint(own), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  u64 packet = 0;
+  const u64 t0 = __builtin_amdgcn_s_memrealtime();
+  for (bool more = true; more;) {
+    packet = __hip_atomic_load(packets + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    more = packet >> 32 == 0 && (int64_t)(__builtin_amdgcn_s_memrealtime() - t0) < wait_ticks;
+  }
+  float top = __uint_as_float((uint32_t)packet);
+  if (packet >> 32 == 0) {
+    const int from = (tid & (cols - 1)) * 4;  // the first thread of these four, in workgroup tid >> log_cols
+    const uint32_t at = (uint32_t)(from >> log_cols) * per * kRowThreads + (tid >> log_cols) * cols + (from & (cols - 1));
+    top = -INFINITY;
+    for (int i = 0; i < min(per, rows - (from >> log_cols) * per); ++i)
+      for (int c = 0; c < 4; ++c)
+        if (at + i * kRowThreads + c < width) top = fmaxf(top, load_logit<DT>(row, at + i * kRowThreads + c));
+  }
+  {
+    const float m = wave_max(top);
+    if (lane == 0) s_max[tid >> 6] = m;
+  }
+  lds_barrier();
+  float mx = s_max[0];
+#pragma unroll
+  for (int w = 1; w < kRowThreads / 64; ++w) mx = fmaxf(mx, s_max[w]);
+  const float k = 1.0f / temperature * 1.4426950408889634f;
+  const bool has_k = kk >= 1 && kk < vocab, by_count = has_k && kk <= kListTopK;
+  uint32_t floor_bits = 0u, list_bits = kNoDigit;
+  if (by_count || (!has_k && pp < 1.0f)) {
+    const float w = __builtin_amdgcn_exp2f((top - mx) * k);
+    floor_bits = kth_bound_in(w > 0.f ? __float_as_uint(w) : 0u, (int)(by_count ? kk : (int64_t)kListTopP), hist, &s_bound);  // NaN counts as nothing here
+  }
+  if (floor_bits) list_bits = floor_bits - 8u;  // see sample_row
+  if (tid == 0) s_n = list_bits == kNoDigit ? kList + 1 : 0;
+  __syncthreads();
+
+  // ---- weights, candidates ----
+  u64* list = sc.list + (r * split + g) * kPart;
+  float w[kTeamDeep];
+#pragma unroll
+  for (int i0 = 0; i0 < kTeamDeep; i0 += kStep) {
+    if (i0 < here) {
+      float most = 0.f;
+#pragma unroll
+      for (int i = i0; i < i0 + kStep; ++i) {
+        w[i] = __builtin_amdgcn_exp2f((number(i) - mx) * k);
+        w[i] = in_row(i) ? w[i] : 0.f;
+        most = fmaxf(most, w[i]);
+      }
+      if (__any(__float_as_uint(most) >= list_bits)) {
+#pragma unroll
+        for (int i = i0; i < i0 + kStep; ++i)
+          if (w[i] > 0.f && __float_as_uint(w[i]) >= list_bits) {
+            const int at = atomicAdd(&s_n, 1);
+            if (at < kPart) __hip_atomic_store(list + at, (u64)__float_as_uint(w[i]) << 32 | (at0 + i * kRowThreads), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+      }
+    }
+  }
+  // ---- the columns' sums, in the order of the rows: part after part ----
+#pragma unroll
+  for (int part = 0; part < kTeamParts; ++part) {
+    if (q == part) {
+      float sum = part ? s_sum[tid & (cols - 1)] : 0.f;
+#pragma unroll
+      for (int i0 = 0; i0 < kTeamDeep; i0 += kStep) {
+        if (i0 < here) {
+#pragma unroll
+          for (int i = i0; i < i0 + kStep; ++i) sum += w[i];  // a zero more leaves a sum as it is
+        }
+      }
+      if (part + 1 < kTeamParts) s_sum[tid & (cols - 1)] = sum;
+      else __hip_atomic_store(sc.sum + r * kRowThreads + column, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (part + 1 < kTeamParts) lds_barrier();
+  }
+  if (tid == 0) __hip_atomic_store(sc.count + r * split + g, s_n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // what the last one reads is out
+  __syncthreads();
+  if (tid == 0) s_place = (int)__hip_atomic_fetch_add(left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const int place = __builtin_amdgcn_readfirstlane(s_place);
+  if (place < split - 1) {  // the others copy the row while the last one draws
+    if (kept) {
+      const int64_t share = ((vocab + split - 2) / (split - 1) + 7) & ~7ll, lo = min(vocab, place * share), hi = min(vocab, lo + share);
+      copy_numbers(reinterpret_cast<E*>(kept) + r * vocab + lo, reinterpret_cast<const E*>(row) + lo, hi - lo);
+      if (place == 0 && tid == 0) kept_t[r] = temperature;
+    }
+    return;
+  }
+
+  // ---- the draw ----
+  const int count = lane < split ? __hip_atomic_load(sc.count + r * split + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+  const float whole = __hip_atomic_load(sc.sum + r * kRowThreads + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(packets + tid, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) __hip_atomic_store(left, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  int n;
+  const bool listed = gather_lists(sh, sc.list + r * split * kPart, count, split, n);
+  LogitRow<DT> src{row, mx, k, 1.0f};
+  src.inv = 1.0f / block_reduce_sum(whole, sh.lds_f);
+  if (tid == 0) sh.s_pick = -1;
+  u64 kept_mass = kNoMass;
+  __syncthreads();
+  if (listed && draw_from_list(src, sh, out, n, floor_bits, has_k, kk, pp, vocab, seed, offset, r, kept_mass)) return;
+  draw_from_row(src, sh, out, kk, pp, vocab, seed, offset, r, kept_mass);
 }
 
 // Workgroups per row (1: one walks the row).  One a compute unit in all: 64 rows x 151936, top-p alone, 54 us with 4 each, 58 with 8; 33 rows 51 and 54.
-// Where sharing pays, us a draw, shared / one workgroup, bf16:
+// Where sharing pays, us a draw, shared / one workgroup, bf16 (top-k: in three launches; sample_team_kernel is ahead of them wherever it can be taken):
 //   top-k      1 x 151936 20.5 / 25.2, 33 x 151936 29.4 / 31.4, 64 x 151936 29.1 / 34.2, but 8 x 65536 20.4 / 17.5, 100 x 151936 41 / 38
 //   no filter  64 x 65536 16.5 / 17.7, 128 x 98304 24.4 / 25.9, 100 x 151936 29 / 37, but 128 x 65536 20.4 / 18.7, 128 x 50000 18.2 / 15.3,
 //              32 x 50000 14.8 / 14.8, 256 x 151936 48 / 44
@@ -1529,9 +1747,15 @@ extern "C" int64_t msgl_sample_workspace_bytes(int64_t rows, int64_t vocab, int 
 // One draw per row in three or four launches (see the comment above split_max_kernel).
 template <int DT, bool VEC>
 static void launch_split(const SplitScratch& sc, int32_t* out, char* kept, float* kept_t, const char* logits, const float* temperatures, const int32_t* top_k,
-                         const float* top_p, bool filtered, int64_t rows, int64_t vocab, int64_t stride_bytes, int split, u64 seed, u64 offset, hipStream_t s) {
+                         const float* top_p, bool filtered, int64_t rows, int64_t vocab, int64_t stride_bytes, int split, u64 seed, u64 offset, char* team, int wait_ticks,
+                         hipStream_t s) {
   // The copy of the rows: beside the picks, on the compute units that these leave idle; where they leave few, by the sums' kernel, which has the
   // rows in registers (us: 202 x 151936, top-p alone 101 beside the picks, 92 with the sums; 105 x 120687 the same; 64 x 151936 with top-k 28, 29)
+  if (team && filtered && top_k && rows <= kTeamRows && split >= kTeamParts && vocab <= (int64_t)kTeamDeep * kTeamParts * kRowThreads) {
+    sample_team_kernel<DT><<<dim3((unsigned)(rows * split)), dim3(kRowThreads), 0, s>>>(sc, team, out, logits, temperatures, top_k, top_p, vocab, stride_bytes, split, seed,
+                                                                                        offset, kept, kept_t, wait_ticks);
+    return;
+  }
   const bool here = VEC && filtered && !top_k && kept && rows > 128 && vocab % 8 == 0 && aligned16(kept);
   char* const kept_sum = here ? kept : nullptr;
   if (here) kept = nullptr;
@@ -1558,7 +1782,7 @@ static void launch_split(const SplitScratch& sc, int32_t* out, char* kept, float
 // the workspace laid out, and one draw per row; `name` for errors
 static int sample_split(const char* name, void* workspace, int64_t workspace_bytes, int32_t* out, void* kept, float* kept_t, const void* logits,
                         const float* temperatures, const int32_t* top_k, const float* top_p, bool filtered, int64_t rows, int64_t vocab, int64_t logits_stride,
-                        int logits_dtype, u64 seed, u64 offset, hipStream_t s) {
+                        int logits_dtype, u64 seed, u64 offset, char* team, int wait_ticks, hipStream_t s) {
   const int split = split_of(rows, vocab, filtered, top_k, top_p), esz = logits_dtype == MSGL_F32 ? 4 : 2;
   SplitScratch sc{};
   const int64_t need = (int64_t)split_layout(&sc, static_cast<char*>(workspace), rows, split, filtered, filtered && !top_k);
@@ -1567,7 +1791,7 @@ static int sample_split(const char* name, void* workspace, int64_t workspace_byt
 #define MSGL_SPLIT(DT)                                                                                                                               \
   do {                                                                                                                                               \
     auto* f = vec ? &launch_split<DT, true> : &launch_split<DT, false>;                                                                              \
-    f(sc, out, (char*)kept, kept_t, (const char*)logits, temperatures, top_k, top_p, filtered, rows, vocab, logits_stride * esz, split, seed, offset, s); \
+    f(sc, out, (char*)kept, kept_t, (const char*)logits, temperatures, top_k, top_p, filtered, rows, vocab, logits_stride * esz, split, seed, offset, team, wait_ticks, s); \
   } while (0)
   if (logits_dtype == MSGL_F32) MSGL_SPLIT(MSGL_F32);
   else if (logits_dtype == MSGL_BF16) MSGL_SPLIT(MSGL_BF16);
@@ -1582,17 +1806,20 @@ static int sample_split(const char* name, void* workspace, int64_t workspace_byt
 }
 
 // probs path's draw without the probs: same thresholds, same masses, same pick as softmax_temperature + sample_top_k_top_p
-extern "C" int msgl_sample_filtered_logits_ws(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
-                                              const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
-                                              int logits_dtype, uint64_t seed, uint64_t offset, void* workspace, int64_t workspace_bytes, void* stream) {
+extern "C" int msgl_sample_filtered_logits_team(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
+                                                const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
+                                                int logits_dtype, uint64_t seed, uint64_t offset, void* workspace, int64_t workspace_bytes, void* team,
+                                                int64_t team_bytes, int wait_us, void* stream) {
   MSGL_REQUIRE(rows >= 0, "sample_filtered_logits: negative rows");
   if (rows == 0) return MSGL_OK;
   MSGL_REQUIRE(out && logits && temperatures && !kept == !kept_temperatures, "sample_filtered_logits: null pointer");
   MSGL_REQUIRE(vocab >= 1 && vocab < (1ll << 31) && rows < (1ll << 31), "sample_filtered_logits: bad shape");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  MSGL_REQUIRE(!team || (aligned16(team) && team_bytes >= kTeamBytes && wait_us >= 0 && wait_us <= 1000000), "sample_filtered_logits: a team of %lld bytes, 16-byte aligned, is needed",
+               (long long)kTeamBytes);
   if (workspace && split_of(rows, vocab, true, top_k, top_p) > 1)
     return sample_split("sample_filtered_logits", workspace, workspace_bytes, out, kept, kept_temperatures, logits, temperatures, top_k, top_p, true, rows,
-                        vocab, logits_stride, logits_dtype, seed, offset, s);
+                        vocab, logits_stride, logits_dtype, seed, offset, static_cast<char*>(team), wait_us * 100, s);
   const int64_t groups = rows + (kept ? rows * ((vocab + kCopySlice - 1) / kCopySlice) : 0);
   MSGL_REQUIRE(groups < (1ll << 31), "sample_filtered_logits: too many rows");
   const dim3 g((unsigned)groups), b(kRowThreads);
@@ -1609,6 +1836,15 @@ extern "C" int msgl_sample_filtered_logits_ws(int32_t* out, void* kept, float* k
 #undef MSGL_SAMPLE
   MSGL_CHECK_LAUNCH("sample_filtered_logits");
   return MSGL_OK;
+}
+
+extern "C" int64_t msgl_sample_team_bytes(void) { return kTeamBytes; }
+
+extern "C" int msgl_sample_filtered_logits_ws(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
+                                              const int32_t* top_k, const float* top_p, int64_t rows, int64_t vocab, int64_t logits_stride,
+                                              int logits_dtype, uint64_t seed, uint64_t offset, void* workspace, int64_t workspace_bytes, void* stream) {
+  return msgl_sample_filtered_logits_team(out, kept, kept_temperatures, logits, temperatures, top_k, top_p, rows, vocab, logits_stride, logits_dtype, seed,
+                                          offset, workspace, workspace_bytes, nullptr, 0, 0, stream);
 }
 
 extern "C" int msgl_sample_filtered_logits_keep(int32_t* out, void* kept, float* kept_temperatures, const void* logits, const float* temperatures,
@@ -1638,7 +1874,7 @@ extern "C" int msgl_sample_from_logits_ws(int32_t* out, const void* logits, cons
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (workspace && split_of(rows, vocab, false, false, false) > 1)
     return sample_split("sample_from_logits", workspace, workspace_bytes, out, nullptr, nullptr, logits, temperatures, nullptr, nullptr, false, rows, vocab,
-                        logits_stride, logits_dtype, seed, offset, s);
+                        logits_stride, logits_dtype, seed, offset, nullptr, 0, s);
   const dim3 g((unsigned)rows), b(kRowThreads);
   if (logits_dtype == MSGL_F32)
     sample_logits_kernel<MSGL_F32><<<g, b, 0, s>>>(out, (const char*)logits, temperatures, vocab, logits_stride * esz, (u64)seed, (u64)offset);

@@ -7,6 +7,7 @@ function does (e.g. `indexing` output), none synchronises.
 """
 from __future__ import annotations
 
+import collections
 import ctypes as C
 import functools
 import os
@@ -609,10 +610,34 @@ def _sample_workspace(rows: int, vocab: int, filtered: bool, has_k: bool, has_p:
     return (torch.empty(n, dtype=torch.uint8, device=device) if n else None), n
 
 
+_SAMPLE_TEAMS: "collections.OrderedDict" = collections.OrderedDict()  # (device index, stream) -> zeros that a draw's workgroups meet in
+_SAMPLE_TEAMS_MAX = 16
+
+
+def _sample_team(device: torch.device, stream: int) -> torch.Tensor:
+    """Memory in which the workgroups of a top-k draw meet: every launch finds and leaves zeros, so one stream's launches, which follow each other, share it.  A
+    captured draw clears its own: its replays may run beside the stream's other draws."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.zeros(_sample_team_bytes(), dtype=torch.uint8, device=device)
+    at = (device.index, stream)
+    team = _SAMPLE_TEAMS.get(at)
+    if team is None:
+        team = _SAMPLE_TEAMS[at] = torch.zeros(_sample_team_bytes(), dtype=torch.uint8, device=device)
+        while len(_SAMPLE_TEAMS) > _SAMPLE_TEAMS_MAX:  # back to its stream's allocator
+            _SAMPLE_TEAMS.popitem(last=False)
+    return team
+
+
+@functools.lru_cache(maxsize=None)
+def _sample_team_bytes() -> int:
+    return int(lib().msgl_sample_team_bytes())
+
+
 def sample_filtered_logits(logits: torch.Tensor, temperatures: torch.Tensor, top_k: Optional[torch.Tensor], top_p: Optional[torch.Tensor],
-                           seed: int, offset: int, keep: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> torch.Tensor:
+                           seed: int, offset: int, keep: Optional[Tuple[torch.Tensor, torch.Tensor]] = None, wait_us: int = 20) -> torch.Tensor:
     """sample_top_k_top_p(softmax_temperature(logits, temperatures), ...) without the probabilities: the same picks.
-    keep: contiguous (logits, temperatures) of the same shapes and types that receive a copy of what was drawn from."""
+    keep: contiguous (logits, temperatures) of the same shapes and types that receive a copy of what was drawn from.
+    wait_us: how long a workgroup of a shared row waits for another one's maxima before it looks them up itself."""
     _need_cuda(logits, temperatures)
     assert logits.dim() == 2 and logits.stride(1) == 1 and temperatures.dtype == torch.float32
     rows = logits.shape[0]
@@ -626,12 +651,14 @@ def sample_filtered_logits(logits: torch.Tensor, temperatures: torch.Tensor, top
         assert keep[0].shape == logits.shape and keep[0].dtype == logits.dtype and keep[0].is_contiguous()
         assert keep[1].shape == (rows,) and keep[1].dtype == torch.float32 and keep[1].is_contiguous()
     ws, ws_bytes = _sample_workspace(rows, logits.shape[1], True, top_k is not None, top_p is not None, logits.device)
+    stream = _stream()
+    team = _sample_team(logits.device, stream) if ws is not None and top_k is not None else None
     check(
-        lib().msgl_sample_filtered_logits_ws(
+        lib().msgl_sample_filtered_logits_team(
             out.data_ptr(), None if keep is None else keep[0].data_ptr(), None if keep is None else keep[1].data_ptr(), logits.data_ptr(),
             temperatures.data_ptr(), top_k.data_ptr() if top_k is not None else None, top_p.data_ptr() if top_p is not None else None, rows,
             logits.shape[1], logits.stride(0), _logits_dt(logits), seed & 0xFFFFFFFFFFFFFFFF, offset & 0xFFFFFFFFFFFFFFFF,
-            None if ws is None else ws.data_ptr(), ws_bytes, _stream(),
+            None if ws is None else ws.data_ptr(), ws_bytes, None if team is None else team.data_ptr(), 0 if team is None else team.numel(), wait_us, stream,
         ),
         "sample_filtered_logits",
     )

@@ -447,3 +447,65 @@ def test_unfiltered_draws_of_shared_rows_are_those_of_one_workgroup(ops, dev, dt
         ops.check(ops.lib().msgl_sample_from_logits(want.data_ptr(), logits.data_ptr(), t.data_ptr(), rows, vocab, logits.stride(0), ops._logits_dt(logits), 9, off,
                                                     ops._stream()), "sample")
         assert torch.equal(ops.sample_from_logits(logits, t, 9, off), want)
+
+
+# one launch for draws with a top-k: 4, 8 and 16 workgroups a row, unaligned rows, the largest share that fits the registers and one that does not
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,vocab", [(64, 98304), (64, 151936), (33, 163840), (33, 163848), (20, 98305), (5, 131071), (1, 151936)])
+def test_draws_in_one_launch(ops, dev, dtype, rows, vocab):
+    """The picks of stored probabilities, whether the workgroups wait for each other's maxima or (wait_us 0) look them up; copies bit for bit; the zeros that
+    the next launch starts from are left."""
+    g = torch.Generator(device=dev).manual_seed(rows + vocab)
+    logits = torch.randn((rows, vocab), generator=g, device=dev) * 2.5
+    for r in range(rows):
+        if r % 5 == 1:
+            logits[r, 3::1024] += 9.0  # the largest numbers in one column: more candidates than a list holds
+        elif r % 5 == 2:
+            logits[r] = torch.round(logits[r] * 2) / 2
+        elif r % 5 == 3:
+            logits[r, 5:] -= 300.0
+    logits = logits.to(dtype)
+    t = torch.tensor([(0.5, 0.7, 1.0, 0.02)[r % 4] for r in range(rows)], device=dev)
+    p = torch.tensor([(0.8, 0.98, 1e-6, 1.0, 0.999999, 0.5)[r % 6] for r in range(rows)], device=dev)
+    k = torch.tensor([(40, 0, 1024, 1, 1500, vocab)[r % 6] for r in range(rows)], dtype=torch.int32, device=dev)
+    probs = ops.softmax_temperature(logits, t)
+    kept = torch.empty_like(logits), torch.empty_like(t)
+    for pp in (p, None):
+        for off in (0, 1000):
+            want = ops.sample_top_k_top_p(probs, k, pp, 77, off)
+            for wait_us in (20, 0, 20):
+                kept[0].zero_()
+                got = ops.sample_filtered_logits(logits, t, k, pp, 77, off, keep=kept, wait_us=wait_us)
+                assert torch.equal(got, want)
+                assert torch.equal(kept[0].view(torch.uint8), logits.view(torch.uint8)) and torch.equal(kept[1], t)
+    assert not any(bool(z.any()) for z in ops._SAMPLE_TEAMS.values())
+
+
+def test_draws_in_one_launch_beside_others(ops, dev):
+    """Workgroups without a place on the device are not waited for; streams do not share what the workgroups meet in; a captured draw has its own."""
+    logits = (torch.randn((64, 151936), generator=torch.Generator(device=dev).manual_seed(1), device=dev) * 2.5).bfloat16()
+    t, k, p = torch.ones(64, device=dev), torch.full((64,), 50, dtype=torch.int32, device=dev), torch.full((64,), 0.9, device=dev)
+    want = ops.sample_top_k_top_p(ops.softmax_temperature(logits, t), k, p, 9, 0)
+    graph = torch.cuda.CUDAGraph()
+    ops.sample_filtered_logits(logits, t, k, p, 9, 0)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        captured = ops.sample_filtered_logits(logits, t, k, p, 9, 0)
+    a = torch.randn((8192, 8192), device=dev, dtype=torch.bfloat16)
+    sides = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for i in range(10):
+        captured.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(sides[0]):
+            a @ a
+            other = ops.sample_filtered_logits(logits, t, k, p, 9, 0)
+        if i % 2:
+            with torch.cuda.stream(sides[1]):
+                graph.replay()
+        else:
+            graph.replay()
+        got = ops.sample_filtered_logits(logits, t, k, p, 9, 0)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(other, want) and torch.equal(captured, want)
+    assert len(ops._SAMPLE_TEAMS) <= ops._SAMPLE_TEAMS_MAX
