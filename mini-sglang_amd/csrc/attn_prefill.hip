@@ -758,7 +758,9 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
   if (HEADS == 1 && left <= 0) return;
   if (!own_pieces) {
     // Outputs by way of the image that does not hold the last tile (everyone is done with it), a wave's rows in its own part: whole rows of 256
-    // bytes leave it, where a lane's own pieces are 16 bytes of 32 rows a store.  16-byte pieces change places by the row's number.
+    // bytes leave it, where a lane's own pieces are 16 bytes of 32 rows a store.  16-byte pieces change places by the row's number.  Nobody reads them in this
+    // launch: past the L2, which keeps keys and values (40 heads on 8, with store_kv_kernel: 29 requests of 100 - 1024 217 -> 214 us, 60 of 128 - 256
+    // 111 -> 99; 64 on 8 332 -> 328 and 160 -> 155; one of 8192 the same.  Q's copies past it too: 99 -> 105).
     char* turn = (((ntiles - t0) & 1) ? lds_b : lds_a) + wave * 8192;
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb)
@@ -771,7 +773,7 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
     for (int i = 0; i < 16; ++i) {
       const int r = 2 * i + hi;
       const uint2 w = *reinterpret_cast<const uint2*>(turn + r * 256 + ((((lane & 31) >> 1) ^ (r & 15)) << 4) + 8 * (lane & 1));
-      if (r < left) *reinterpret_cast<uint2*>(op + (int64_t)r * p.out_stride) = w;
+      if (r < left) __builtin_nontemporal_store(__builtin_bit_cast(uint64_t, w), reinterpret_cast<uint64_t*>(op + (int64_t)r * p.out_stride));
     }
   } else if (q_valid) {
     uint16_t* op = p.out + (int64_t)(q_begin + my_q) * p.out_stride + (int64_t)hq * kD;
