@@ -291,6 +291,13 @@ int msgl_attn_prefill_ranges(void* out, const void* q, const void* k_cache, cons
                              int64_t kv_stride_tok, int64_t kv_stride_head, int64_t out_stride_tok,
                              float sm_scale, int dtype, const int32_t* tile_order, int ranges, int range_tiles,
                              void* workspace, int64_t workspace_bytes, void* stream);
+/* Prefill of requests that have nothing in the pool (seq_lens = their new tokens), and the store of their keys and values, in one launch: row t of k and v
+ * ([tokens, kv heads, head_dim] at kv_stride_new elements a token, 16-byte aligned rows) goes to slot out_loc[t] of the pool as msgl_store_kv
+ * stores it, and the rows are attended to as they come; the same bits as the two launches (impl 4). */
+int msgl_attn_prefill_fresh(void* out, const void* q, const void* k, const void* v, int64_t kv_stride_new, void* k_cache, void* v_cache,
+                            const int32_t* out_loc, const int32_t* seq_lens, const int32_t* cu_seqlens_q, const int32_t* tile_cu, int batch,
+                            int total_tiles, int num_q_heads, int num_kv_heads, int head_dim, int64_t q_stride_tok, int64_t kv_stride_tok,
+                            int64_t kv_stride_head, int64_t out_stride_tok, float sm_scale, int dtype, const int32_t* tile_order, void* stream);
 /* Rows per q tile: tile_cu, total_tiles and tile_order of msgl_attn_prefill are in units of this many query rows
  * (MSGL_PREFILL_QTILE for both kernels). */
 int msgl_attn_prefill_q_tile(int impl);

@@ -82,6 +82,10 @@ HIP_SIGNATURES = {
         _i,
         [_p, _p, _p, _p, _p, _l, _p, _p, _p, _p, _i, _i, _i, _i, _i, _l, _l, _l, _l, _f, _i, _p, _i, _i, _p, _l, _p],
     ),
+    "msgl_attn_prefill_fresh": (
+        _i,
+        [_p, _p, _p, _p, _l, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _l, _l, _l, _l, _f, _i, _p, _p],
+    ),
     "msgl_attn_prefill_ranges_workspace_bytes": (_l, [_i, _i, _i]),
     "msgl_attn_prefill_q_tile": (_i, [_i]),
     "msgl_argmax_rows": (_i, [_p, _p, _l, _l, _l, _i, _p]),

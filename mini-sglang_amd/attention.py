@@ -37,6 +37,7 @@ class HipAttnMetadata:
     ranges: tuple = (1, 0)                  # key ranges of a q tile, 64-key tiles of each (prefill only)
     scratch: Optional[torch.Tensor] = None  # their partial sums, from the first layer on
     pairs: bool = False                     # two heads a workgroup (prefill only)
+    fresh: bool = False                     # short prompts that have nothing in the pool (prefill only)
     plan: Optional[torch.Tensor] = None     # decode work list (device)
     chunks: Optional[tuple] = None          # recurrent layers: (items [n, 3], item_first [B + 1], n) of long portions cut in pieces
     delta_chunks: Optional[tuple] = None    # the same list at the delta-rule layers' piece size
@@ -184,8 +185,29 @@ class HipAttnBackend:
             if (batch.out_loc.dtype == torch.int32 and batch.out_loc.is_contiguous() and {t.dtype for t in (q, k, v)} == {self.kvcache.dtype}
                     and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (q2, k2, v2))):
                 return self._attend_small(q2, k2, v2, layer_id, batch)
+        if batch.attn_metadata.fresh and self._takes_fresh(q, k, v, batch):
+            return self._attend_fresh(q, k, v, layer_id, batch)
         self.kvcache.store_kv(k, v, batch.out_loc, layer_id)
         return self.attend(q, layer_id, batch)
+
+    def _takes_fresh(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, batch: Any) -> bool:
+        """Whether a batch of short prompts with nothing cached goes from its rows as they come, and into the pool, in one launch (one stride, 16-byte pieces, no key
+        ranges or pairs of heads; the default kernel).  Its page table then says of the new tokens what out_loc says, as the scheduler allocates them."""
+        md, loc = batch.attn_metadata, batch.out_loc
+        if md.ranges[0] > 1 or md.pairs or ops.PREFILL_IMPL not in (0, 4) or self.head_dim != 128 or loc.dtype != torch.int32 or not loc.is_contiguous():
+            return False
+        k2, v2 = (t.view(t.shape[0], -1) for t in (k, v))
+        return (q.shape[0] == k2.shape[0] == loc.numel() and {q.dtype, k.dtype, v.dtype} == {self.kvcache.dtype} and k2.shape[1] == self.kv_heads * self.head_dim
+                and k2.shape == v2.shape and k2.stride() == v2.stride() and k2.stride(1) == 1 and k2.stride(0) % 8 == 0
+                and k2.data_ptr() % 16 == 0 and v2.data_ptr() % 16 == 0)
+
+    def _attend_fresh(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_id: int, batch: Any) -> torch.Tensor:
+        md: HipAttnMetadata = batch.attn_metadata
+        q = q.view(-1, self.qo_heads, self.head_dim)
+        out = torch.empty((q.shape[0], self.qo_heads, self.head_dim), dtype=q.dtype, device=q.device)
+        ops.attn_prefill_fresh(out, q, k.view(k.shape[0], -1), v.view(v.shape[0], -1), *self._kv_tokens(layer_id), batch.out_loc, md.seq_lens, md.cu_seqlens_q,
+                               md.tile_cu, md.batch, md.total_tiles, self.scale, tile_order=md.tile_order)
+        return out
 
     def attend(self, q: torch.Tensor, layer_id: int, batch: Any) -> torch.Tensor:
         """Attention only (K/V for this batch already in the pool, e.g. via the fused
@@ -242,6 +264,7 @@ class HipAttnBackend:
             total_tiles=total_tiles, tile_order=None if decode else dev[4 * bs + 2:],
             ranges=(1, 0) if decode else ops.prefill_ranges(total_tiles, self.qo_heads, max_q, max_k),
             pairs=not decode and ops.prefill_pairs(total_tiles, self.qo_heads, self.kv_heads, seqlens_q, seqlens_k),
+            fresh=not decode and max_q <= ops.FRESH_TOKENS and bool((seqlens_q == seqlens_k).all()),
         )
         if decode and not self._replayed_from_graph(batch, bs):
             # runs eagerly: plan now (device side, no sync).  Only batches the engine will REPLAY are planned

@@ -69,6 +69,10 @@ struct PrefillParams {
   int few;         // q tiles of fewer rows load and store by lanes' own pieces
   int idle;        // waves without rows make no products (one head a workgroup)
   int ranges, run;  // key ranges, and tiles of each (the last one: what is left)
+  const uint16_t *k_new, *v_new;  // FRESH: the rows of all requests' keys and values as they come, and where they are to be stored
+  uint16_t *k_pool, *v_pool;
+  const int* out_loc;
+  int64_t new_stride;
   float *part_o, *part_ml;
   float scale_log2;
 };
@@ -187,6 +191,12 @@ __device__ __forceinline__ float pair_max(float x) {
 __device__ __forceinline__ float pair_sum(float x) {
   const float2 y = both_halves(x);
   return y.x + y.y;
+}
+
+// 16 bytes that nobody reads in this launch
+__device__ __forceinline__ void store_past(uint16_t* to, const char* from) {
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  __builtin_nontemporal_store(*reinterpret_cast<const u32x4_t*>(from), reinterpret_cast<u32x4_t*>(to));
 }
 
 constexpr int kTileBytes = kKTile * kD * 2;  // 16 KB: one K (or V) tile image
@@ -461,6 +471,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 // the order of the lanes.  For launches that leave compute units empty, where the longest chain of tiles (1.26 us each) is the time: 16 heads on
 // 8, 100 tokens after 2000: 45.1 -> 13.7 us, 1000 after 3000: 81.7 -> 53.2; 5 on 1, 2000 tokens: 43.0 -> 20.5 (both launches, in a captured chain;
 // the rule and its other side: ops.prefill_ranges)
+// FRESH: nothing is cached, so keys and values are read from the rows as they come, without the page table, and stored to the pool from the two tiles that a
+// workgroup's query rows are the keys of, which lie in LDS at its end (by the first head of a kv head).  Longer chains than
+// ops.FRESH_TOKENS' are not measured with pairs of heads, and take the store and the other launch.  us, store_kv_kernel and launch -> this, 40 heads on 8: 29
+// requests of 100 - 1024 tokens 214 -> 192, 60 of 128 - 256 99 -> 85, 8 of 600 - 1000 91 -> 85, 6 of 1500 184 -> 176; 16 on 8: 60 of 128 - 256 54.5 -> 43.9; 64 on
+// 8 155 -> 140.  Beyond, 40 on 8: 4 of 2048 210 -> 202, one of 8192 706 -> 692.  (The pool's rows by way of the L2 212 where 206; each of a kv head's heads a
+// share of them: slower, each waits for its slots.)
 // ABL (diagnosis, wrong results): 1 = tiles DMA'd once, 2 = no QK^T, 4 = no softmax, 8 = no PV.
 // ------------------------------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -474,7 +490,7 @@ __device__ __forceinline__ uint64_t row_lane(uint64_t x) {
   return (uint64_t)hi << 32 | lo;
 }
 
-template <typename T, int ABL = 0, bool RANGES = false, int HEADS = 1>
+template <typename T, int ABL = 0, bool RANGES = false, int HEADS = 1, bool FRESH = false>
 __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const PrefillParams p, int total_tiles) {
   // two distinct LDS objects, not one array: the compiler then knows a tile's fragment reads cannot alias the DMA writes
   // of the next tile (other object) and does not wait for them (vmcnt) before the reads
@@ -530,16 +546,20 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
   //      16-byte slot (lane & 15)
   constexpr int kApart = 16 * HEADS, kTurns = 4 / HEADS;
   const int st_row = tid >> 4;
-  const char* k_lane = reinterpret_cast<const char*>(p.k + (int64_t)kvh * p.kv_stride_head + (((lane & 15) ^ (st_row & 15)) << 3));
-  const char* v_lane = reinterpret_cast<const char*>(p.v + (int64_t)kvh * p.kv_stride_head + (((lane & 15) ^ ((st_row & 3) << 2)) << 3));
+  const int64_t head_at = FRESH ? (int64_t)q_begin * p.new_stride + kvh * kD : (int64_t)kvh * p.kv_stride_head;
+  const char* k_lane = reinterpret_cast<const char*>((FRESH ? p.k_new : p.k) + head_at + (((lane & 15) ^ (st_row & 15)) << 3));
+  const char* v_lane = reinterpret_cast<const char*>((FRESH ? p.v_new : p.v) + head_at + (((lane & 15) ^ ((st_row & 3) << 2)) << 3));
   // A row's slot and offset are found once: lane i of the 16 that copy rows st_row, st_row + kApart, .. has row st_row + kApart i's, and the sixteen
   // take it from there as the address is added up (every lane for its own four rows, HEADS = 1: three more quarter-rate multiplies and three more
   // loads a tile; 64 heads, 8192 tokens after 16384: 5285 -> 5210 us, 29 requests of 100 - 1024, 40 heads on 8: 236 -> 234)
   const uint32_t row_of = st_row + kApart * (lane & (kTurns - 1));
   int sl;
-  auto load_slots = [&](int kt) { sl = pt[min((uint32_t)(kt * kKTile) + row_of, (uint32_t)(k_len - 1))]; };
+  auto load_slots = [&](int kt) {
+    const uint32_t key = min((uint32_t)(kt * kKTile) + row_of, (uint32_t)(k_len - 1));
+    sl = FRESH ? (int)key : pt[key];
+  };
   auto issue_dma = [&](char* buf) {
-    const uint64_t off = (uint64_t)slot_offset(sl, p.kv_stride_tok) * 2;
+    const uint64_t off = (uint64_t)slot_offset(sl, FRESH ? p.new_stride : p.kv_stride_tok) * 2;
     auto four_rows = [&](auto I) __attribute__((always_inline)) {
       constexpr int i = decltype(I)::value;
       const uint64_t o = row_lane<i>(off);
@@ -737,11 +757,32 @@ __global__ __launch_bounds__(256 * HEADS, 2) void attn_prefill_dma_kernel(const 
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const U4*>(mine + (lane & 31) * 256 + (((2 * ks + hi) ^ (lane & 15)) << 4));
   }
+  constexpr int kSlots = FRESH ? kQTile / kApart : 1;
+  const bool stores = FRESH && job.hq % p.group == 0;  // a kv head's first head
+  int slot[kSlots];
+  if (stores) {
+#pragma unroll
+    for (int i = 0; i < kSlots; ++i) slot[i] = p.out_loc[q_begin + min(q0 + st_row + kApart * i, q_len - 1)];
+  }
   for (int kt = t0; kt < ntiles; kt += 2) {
     tile_body(std::integral_constant<int, 0>{}, kt);
     if (kt + 1 < ntiles) tile_body(std::integral_constant<int, 1>{}, kt + 1);
   }
 
+  if (stores) {  // q0 is a multiple of two tiles: its first one is in lds_a
+    uint16_t *k_to = p.k_pool + (int64_t)kvh * p.kv_stride_head + (lane & 15) * 8, *v_to = p.v_pool + (int64_t)kvh * p.kv_stride_head + (lane & 15) * 8;
+#pragma unroll
+    for (int i = 0; i < kSlots; ++i) {
+      const int r = st_row + kApart * (i & (kTurns - 1));  // of the image
+      const char* img = (i < kTurns ? lds_a : lds_b) + r * 256;
+      if (q0 + st_row + kApart * i < q_len) {
+        const int64_t at = slot_offset(slot[i], p.kv_stride_tok);
+        store_past(k_to + at, img + (((lane & 15) ^ (r & 15)) << 4));
+        store_past(v_to + at, img + kTileBytes + (((lane & 15) ^ ((r & 3) << 2)) << 4));
+      }
+    }
+    __syncthreads();  // the images are read
+  }
   if (RANGES && all_tiles > p.run) {
     const int64_t at = ((int64_t)blockIdx.y * total_tiles * p.hq + (int64_t)tile * p.hq + hq) * 4 + rows;
     f32x4p* po = reinterpret_cast<f32x4p*>(p.part_o) + at * 1024 + lane;  // [16 pieces][64 lanes]
@@ -837,14 +878,21 @@ using namespace msgl;
 
 extern "C" int msgl_attn_prefill_q_tile(int /*impl*/) { return kQTile; }
 
-// ranges > 1: impl 0 with that many key ranges at most, `run` tiles each
+// the new rows of a launch that stores them (FRESH)
+struct PrefillFresh {
+  const void *k, *v;
+  int64_t stride;
+  const int32_t* out_loc;
+};
+
+// ranges > 1: impl 0 with that many key ranges at most, `run` tiles each; fresh: not with ranges
 static int prefill(void* out, const void* q, const void* k_cache, const void* v_cache,
                                  const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
                                  const int32_t* seq_lens, const int32_t* cu_seqlens_q, const int32_t* tile_cu,
                                  int batch, int total_tiles, int num_q_heads, int num_kv_heads, int head_dim,
                                  int64_t q_stride_tok, int64_t kv_stride_tok, int64_t kv_stride_head,
                                  int64_t out_stride_tok, float sm_scale, int dtype, const int32_t* tile_order,
-                                 int impl, int ranges, int run, float* workspace, void* stream) {
+                                 int impl, int ranges, int run, float* workspace, const PrefillFresh* fresh, void* stream) {
   MSGL_REQUIRE(batch >= 0 && total_tiles >= 0, "attn_prefill: negative sizes");
 #ifdef MSGL_PREFILL_DIAG
   MSGL_REQUIRE(impl == 0 || impl == 2 || impl == 4 || impl == 6 || (impl >= 16 && impl < 48) || (impl >= 64 && impl < 128),
@@ -868,7 +916,7 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   MSGL_REQUIRE(aligned16(q) && aligned16(k_cache) && aligned16(v_cache) &&
                    (reinterpret_cast<uintptr_t>(out) & 7u) == 0,
                "attn_prefill: pointers must be 16-byte aligned");
-  PrefillParams p;
+  PrefillParams p{};
   p.q = (const uint16_t*)q;
   p.k = (const uint16_t*)k_cache;
   p.v = (const uint16_t*)v_cache;
@@ -884,6 +932,16 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
   p.kv_stride_tok = kv_stride_tok;
   p.kv_stride_head = kv_stride_head;
   p.out_stride = out_stride_tok;
+  if (fresh) {
+    MSGL_REQUIRE(fresh->k && fresh->v && fresh->out_loc && aligned16(fresh->k) && aligned16(fresh->v) && fresh->stride > 0 && fresh->stride < (1ll << 32) && fresh->stride % 8 == 0,
+                 "attn_prefill_fresh: new rows must be 16-byte aligned, stride %lld", (long long)fresh->stride);
+    p.k_new = (const uint16_t*)fresh->k;
+    p.v_new = (const uint16_t*)fresh->v;
+    p.k_pool = (uint16_t*)const_cast<void*>(k_cache);
+    p.v_pool = (uint16_t*)const_cast<void*>(v_cache);
+    p.out_loc = fresh->out_loc;
+    p.new_stride = fresh->stride;
+  }
   p.batch = batch;
   p.hq = num_q_heads;
   const int heads = impl == 6 ? 2 : 1;  // of a workgroup
@@ -929,6 +987,9 @@ static int prefill(void* out, const void* q, const void* k_cache, const void* v_
       attn_prefill_dma_kernel<FP16, 0, true><<<grid, dim3(256), 0, s>>>(p, total_tiles);
       attn_prefill_join_kernel<FP16><<<joins, dim3(64), 0, s>>>(p, total_tiles);
     }
+  } else if (fresh) {
+    if (dtype == MSGL_BF16) attn_prefill_dma_kernel<BF16, 0, false, 1, true><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
+    else attn_prefill_dma_kernel<FP16, 0, false, 1, true><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
   } else if (impl == 4) {
     if (dtype == MSGL_BF16) attn_prefill_dma_kernel<BF16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
     else attn_prefill_dma_kernel<FP16><<<dim3(blocks), dim3(256), 0, s>>>(p, total_tiles);
@@ -970,7 +1031,7 @@ extern "C" int msgl_attn_prefill(void* out, const void* q, const void* k_cache, 
                                        int64_t kv_stride_tok, int64_t kv_stride_head, int64_t out_stride_tok, float sm_scale, int dtype,
                                        const int32_t* tile_order, int impl, void* stream) {
   return prefill(out, q, k_cache, v_cache, page_table, pt_stride, req_rows, seq_lens, cu_seqlens_q, tile_cu, batch, total_tiles, num_q_heads,
-                 num_kv_heads, head_dim, q_stride_tok, kv_stride_tok, kv_stride_head, out_stride_tok, sm_scale, dtype, tile_order, impl, 1, 0, nullptr, stream);
+                 num_kv_heads, head_dim, q_stride_tok, kv_stride_tok, kv_stride_head, out_stride_tok, sm_scale, dtype, tile_order, impl, 1, 0, nullptr, nullptr, stream);
 }
 
 extern "C" int64_t msgl_attn_prefill_ranges_workspace_bytes(int total_tiles, int num_q_heads, int ranges) {
@@ -988,5 +1049,14 @@ extern "C" int msgl_attn_prefill_ranges(void* out, const void* q, const void* k_
   MSGL_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= msgl_attn_prefill_ranges_workspace_bytes(total_tiles, num_q_heads, ranges),
                "attn_prefill_ranges: workspace of %lld bytes", (long long)workspace_bytes);
   return prefill(out, q, k_cache, v_cache, page_table, pt_stride, req_rows, seq_lens, cu_seqlens_q, tile_cu, batch, total_tiles, num_q_heads,
-                 num_kv_heads, head_dim, q_stride_tok, kv_stride_tok, kv_stride_head, out_stride_tok, sm_scale, dtype, tile_order, 0, ranges, range_tiles, (float*)workspace, stream);
+                 num_kv_heads, head_dim, q_stride_tok, kv_stride_tok, kv_stride_head, out_stride_tok, sm_scale, dtype, tile_order, 0, ranges, range_tiles, (float*)workspace, nullptr, stream);
+}
+
+extern "C" int msgl_attn_prefill_fresh(void* out, const void* q, const void* k, const void* v, int64_t kv_stride_new, void* k_cache, void* v_cache,
+                                       const int32_t* out_loc, const int32_t* seq_lens, const int32_t* cu_seqlens_q, const int32_t* tile_cu, int batch,
+                                       int total_tiles, int num_q_heads, int num_kv_heads, int head_dim, int64_t q_stride_tok, int64_t kv_stride_tok,
+                                       int64_t kv_stride_head, int64_t out_stride_tok, float sm_scale, int dtype, const int32_t* tile_order, void* stream) {
+  const PrefillFresh fresh{k, v, kv_stride_new, out_loc};
+  return prefill(out, q, k_cache, v_cache, out_loc, 0, nullptr, seq_lens, cu_seqlens_q, tile_cu, batch, total_tiles, num_q_heads, num_kv_heads, head_dim,
+                 q_stride_tok, kv_stride_tok, kv_stride_head, out_stride_tok, sm_scale, dtype, tile_order, 4, 1, 0, nullptr, &fresh, stream);
 }

@@ -557,6 +557,37 @@ def attn_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_ca
     )
 
 
+# Longest prompt of a batch with nothing cached whose store and attention go in one launch: chains short enough that heads do not go in pairs (prefill_pairs: 15
+# tiles on average).  What it saves, % of both launches, heads on kv heads: up to here 60 requests of 128 - 256 tokens 17 (40 on 8), 24 (16 on 8), 11 (64 on 8); 8 of 600 -
+# 1000 7, 20, 3; 6 of 1500 4, 13, 2.  Beyond, where the store is a small share: 4 of 2048 5, 10, 2, one of 8192 2, 4, 1.
+FRESH_TOKENS = 1536
+
+
+def attn_prefill_fresh(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, out_loc: torch.Tensor,
+                       seq_lens: torch.Tensor, cu_seqlens_q: torch.Tensor, tile_cu: torch.Tensor, batch: int, total_tiles: int, sm_scale: float,
+                       tile_order: Optional[torch.Tensor] = None) -> None:
+    """store_kv(k, v at out_loc) and attn_prefill of requests whose keys all are new, in one launch: the same bits.  k, v: [tokens, kv heads * head_dim] of one row
+    stride, rows 16-byte aligned; out_loc int32."""
+    _need_cuda(out, q, k, v, k_cache, v_cache, out_loc, seq_lens, cu_seqlens_q, tile_cu)
+    hq, d = q.shape[1], q.shape[2]
+    hkv = k_cache.shape[1]
+    assert q.stride(2) == 1 and q.stride(1) == d and out.stride(2) == 1 and out.stride(1) == d
+    assert k_cache.stride(2) == 1 and v_cache.stride() == k_cache.stride() and k.dtype == v.dtype == q.dtype == k_cache.dtype == v_cache.dtype
+    assert k.shape == v.shape == (q.shape[0], hkv * d) and k.stride() == v.stride() and k.stride(1) == 1
+    assert out_loc.dtype == torch.int32 and out_loc.is_contiguous() and out_loc.numel() >= q.shape[0]
+    if tile_order is not None:
+        _need_cuda(tile_order)
+        assert tile_order.dtype == torch.int32 and tile_order.is_contiguous() and tile_order.numel() == total_tiles
+    check(
+        lib().msgl_attn_prefill_fresh(
+            out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), k.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), out_loc.data_ptr(),
+            seq_lens.data_ptr(), cu_seqlens_q.data_ptr(), tile_cu.data_ptr(), batch, total_tiles, hq, hkv, d, q.stride(0), k_cache.stride(0),
+            k_cache.stride(1), out.stride(0), float(sm_scale), _dt(q), tile_order.data_ptr() if tile_order is not None else None, _stream(),
+        ),
+        "attn_prefill_fresh",
+    )
+
+
 # ---------------------------------------------------------------------------- sampling
 def argmax_rows(logits: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     _need_cuda(logits)

@@ -363,3 +363,59 @@ def test_a_small_decode_capacity_holds_the_small_batch_kernel(ops, dev):
         for b in range(1, backend._small_heads // hkv + 1):
             need = ops.lib().msgl_attn_decode_small_workspace_bytes(b, ops.attn_decode_small_ranges(b, hkv, 40960), hq)
             assert backend._workspace.numel() >= need, (hq, hkv, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("hq,hkv", [(5, 1), (16, 8), (6, 3), (40, 8)])
+@pytest.mark.parametrize("lens", [[1, 63, 64, 65, 127, 128, 129, 192, 2], [700], [257, 1000, 3] * 3, [1536]], ids=str)
+def test_fresh_prompts_store_and_attend_in_one_launch(dev, dtype, hq, hkv, lens):
+    """Requests with nothing cached: outputs and pool of the store and the attention one after the other, bit for bit; other slots stay; rows
+    of two strides and key ranges take the two launches."""
+    from mini_sglang_amd import attention, ops
+    from mini_sglang_amd.core import Batch, Context, Req
+    from mini_sglang_amd.kvcache import create_kvcache_pool
+    from mini_sglang_amd.model import ModelConfig
+
+    T, D, page = sum(lens), 128, 16
+    g = torch.Generator(device=dev).manual_seed(T)
+    pages = [-(-n // page) for n in lens]
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(T)).to(dev)
+    ctx = Context(page)
+    ctx.page_table = torch.zeros((len(lens) + 1, (max(lens) + 31) // 32 * 32), dtype=torch.int32, device=dev)
+    m = ModelConfig(1, hq, hkv, D, hq * D, 1024, 1024)
+    ctx.kv_cache = create_kvcache_pool(m, sum(pages) + 1, page, dtype, dev)
+    at, slots = 0, []
+    for i, (n, c) in enumerate(zip(lens, pages)):
+        s = (order[at: at + c, None] * page + torch.arange(page, device=dev)).reshape(-1)[:n]
+        ctx.page_table[i, :n] = s.int()
+        slots.append(s)
+        at += c
+    backend = attention.HipAttnBackend(m, ctx)
+    qkv = torch.randn((T, (hq + 2 * hkv) * D), generator=g, device=dev).to(dtype)
+    q, k, v = qkv.split([hq * D, hkv * D, hkv * D], dim=1)
+    calls, real = [], attention.ops.attn_prefill_fresh
+
+    def run(fresh, k, v, cached=0):
+        batch = Batch(reqs=[Req(input_ids=torch.zeros(n, dtype=torch.int32), table_idx=i, cached_len=cached, output_len=8, uid=i) for i, n in enumerate(lens)], phase="prefill")
+        batch.out_loc = torch.cat([s[cached:] for s in slots]).int()
+        backend.prepare_metadata(batch)
+        md = batch.attn_metadata
+        assert md.fresh is (cached == 0)
+        md.ranges, md.pairs, md.fresh = (1, 0), False, md.fresh and fresh
+        ctx.kv_cache.pool.fill_(3.0)
+        return backend.forward(q.view(T, hq, D), k, v, 0, batch), ctx.kv_cache.pool.clone(), batch
+
+    try:
+        attention.ops.attn_prefill_fresh = lambda *a, **kw: calls.append(1) or real(*a, **kw)
+        want, pool, batch = run(False, k, v)
+        assert not calls
+        got, pool2, _ = run(True, k, v)
+        assert len(calls) == 1
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and torch.equal(pool.view(torch.int16), pool2.view(torch.int16))
+        got, pool2, _ = run(True, k, v.contiguous())  # rows of two strides
+        assert len(calls) == 1 and torch.equal(got, want) and torch.equal(pool, pool2)
+        batch.attn_metadata.ranges, batch.attn_metadata.fresh = (2, 1), True
+        backend.forward(q.view(T, hq, D), k, v, 0, batch)
+        assert len(calls) == 1
+    finally:
+        attention.ops.attn_prefill_fresh = real
