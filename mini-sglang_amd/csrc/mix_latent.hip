@@ -60,7 +60,8 @@ struct LatentRow {
 // Value waves fetch the rows: a DMA without addresses of its own in a lane's registers, and the score waves' reads wait for nothing but themselves.
 // 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1535 us -> 408 -> 340 us (870 TFLOP/s), 50 us of it the rows' way to LDS, 30
 // us the rescaling, some 60 us workgroups' starts and ends: four follow each other on a CU, which each fills, and the queries' and outputs' 563 MB
-// (115 us at 4.9 TB/s by themselves) come and go partly beside other workgroups' tiles.  2 of 2253 tokens, 8 heads 178 -> 140; 6 of 50 - 353 38 -> 32; 4 of
+// (115 us at 4.9 TB/s by themselves) come and go partly beside other workgroups' tiles, past the L2 (344.4 -> 340.6 on one card, inputs partly in cache 348 ->
+// 339, with the outputs alone 342; outputs of ranges, which the join reads, stay).  2 of 2253 tokens, 8 heads 178 -> 140; 6 of 50 - 353 38 -> 32; 4 of
 // 470, 256 + 64: 35 -> 31.5; 5 of 23 - 225, 8 heads 29.0 -> 28.1.  One tile and full sets cost the two roles' one after the other: 8 portions of 8 tokens, 16
 // heads 12.5 -> 12.7, 40 of 17 15.9 -> 16.4, the largest loss seen.  (Two pieces of queries an LDS turn without bank conflicts, outputs several turns at a
 // time, no barrier behind the last weights, sets without rows only at the barriers: 13.7, 17.2 without them; 8 of 2 tokens 13.2 -> 10.1.)
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
       const bool valid = r < QT * HB && tl < q_len && hh < H;
       const float* qrow = q_abs + (((size_t)first + (valid ? tl : tok0)) * H + (valid ? hh : h0)) * DK + role * 32 + 4 * (lane & 7);
 #pragma unroll
-      for (int u = 0; u < NU; ++u) x[u][i] = *reinterpret_cast<const float4*>(qrow + 64 * u);
+      for (int u = 0; u < NU; ++u) x[u][i] = __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(qrow + 64 * u)));
     }
     if (fetch) dma(img0, slot);
     else if (wave < 3 && lane < KT) s_slot[wave][lane] = slot;
@@ -216,9 +217,12 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
       for (int i = 0; i < 4; ++i) {
         if (valid[i]) {
 #pragma unroll
-          for (int n = 0; n < some; ++n)
-            *reinterpret_cast<float4*>(dst[i] + (vt0 + n) * 32) =
-                *reinterpret_cast<const float4*>(turn + n * 4096 + ((l >> 3) + 8 * i) * 128 + (((l & 7) ^ (l >> 3)) & 7) * 16);
+          for (int n = 0; n < some; ++n) {
+            const f32x4_t x = *reinterpret_cast<const f32x4_t*>(turn + n * 4096 + ((l >> 3) + 8 * i) * 128 + (((l & 7) ^ (l >> 3)) & 7) * 16);
+            f32x4_t* to = reinterpret_cast<f32x4_t*>(dst[i] + (vt0 + n) * 32);
+            if (splits == 1) __builtin_nontemporal_store(x, to);
+            else *to = x;
+          }
         }
       }
       wave_fence();

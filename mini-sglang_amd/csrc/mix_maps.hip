@@ -288,8 +288,9 @@ __global__ __launch_bounds__(256, 2) void maps_prompt_kernel(bf16_t* __restrict_
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] *= 1.0f / (1.0f + __expf(-__builtin_bit_cast(float, e & 1 ? gw[e >> 1] & 0xffff0000u : gw[e >> 1] << 16)));
       }
-      *reinterpret_cast<Q4*>(out + tok * ld_out + (size_t)head * DV + c) =
-          Q4{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
+      // past the L2 (4 portions of 1500 - 2548 tokens, 16 heads on 4: 149.5 -> 146.5 us; the queries' loads too: 148.3)
+      const Q4 packed{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])};
+      __builtin_nontemporal_store(__builtin_bit_cast(f32x4_t, packed), reinterpret_cast<f32x4_t*>(out + tok * ld_out + (size_t)head * DV + c));
     }
     return;
   }

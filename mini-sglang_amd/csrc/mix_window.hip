@@ -341,7 +341,8 @@ __global__ __launch_bounds__(NH * 32, 2) void window_attn_mfma_kernel(bf16_t* __
       for (int i = 0; i < 4; ++i) {
         const int row = 8 * i + (lane >> 3), query = tok0 + (row & 15), col = 64 * half + 8 * (lane & 7);
         const Q4 x = *reinterpret_cast<const Q4*>(turn + row * 128 + (((lane ^ row) & 7) << 4));
-        if (query < q_len && col < dv) *reinterpret_cast<Q4*>(out + ((size_t)(cu_q[b] + query) * NH + h0 + (row >> 4)) * dv + col) = x;
+        if (query < q_len && col < dv)  // past the L2 (4 portions of 1500 - 2548 tokens, 16 heads: 205.5 -> 203.8 us)
+          __builtin_nontemporal_store(__builtin_bit_cast(f32x4_t, x), reinterpret_cast<f32x4_t*>(out + ((size_t)(cu_q[b] + query) * NH + h0 + (row >> 4)) * dv + col));
       }
       asm volatile("" ::: "memory");
     }
