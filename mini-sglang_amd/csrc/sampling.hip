@@ -1634,10 +1634,21 @@ __global__ __launch_bounds__(kRowThreads, 4) void sample_team_kernel(SplitScratc
   // ---- the draw ----
   const int count = lane < split ? __hip_atomic_load(sc.count + r * split + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
   const float whole = __hip_atomic_load(sc.sum + r * kRowThreads + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const u64 ahead = __hip_atomic_load(sc.list + (r * split + q) * kPart + (tid & (cols - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // list q's: most are no longer
   __hip_atomic_store(packets + tid, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (tid == 0) __hip_atomic_store(left, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   int n;
-  const bool listed = gather_lists(sh, sc.list + r * split * kPart, count, split, n);
+  bool listed = true;
+  if (!__any(count > cols)) {
+    const int upto = wave_prefix_incl(count), mine = __builtin_amdgcn_readlane(count, q), before = __builtin_amdgcn_readlane(upto, q) - mine;
+    n = __builtin_amdgcn_readlane(upto, 63);
+    if ((tid & (cols - 1)) < mine) {
+      sh.s_index[before + (tid & (cols - 1))] = (int)(uint32_t)ahead;
+      sh.h_cnt[before + (tid & (cols - 1))] = (uint32_t)(ahead >> 32);
+    }
+  } else {
+    listed = gather_lists(sh, sc.list + r * split * kPart, count, split, n);
+  }
   LogitRow<DT> src{row, mx, k, 1.0f};
   src.inv = 1.0f / block_reduce_sum(whole, sh.lds_f);
   if (tid == 0) sh.s_pick = -1;
