@@ -60,12 +60,14 @@ struct LatentRow {
 // Value waves fetch the rows: a DMA without addresses of its own in a lane's registers, and the score waves' reads wait for nothing but themselves.
 // 4 portions of 1500 - 2548 tokens, 16 heads, 512 + 64: 1535 us -> 408 -> 340 us (870 TFLOP/s), 50 us of it the rows' way to LDS, 30
 // us the rescaling, some 60 us workgroups' starts and ends: four follow each other on a CU, which each fills, and the queries' and outputs' 563 MB
-// (115 us at 4.9 TB/s by themselves) come and go partly beside other workgroups' tiles, past the L2 (344.4 -> 340.6 on one card, inputs partly in cache 348 ->
-// 339, with the outputs alone 342; outputs of ranges, which the join reads, stay).  2 of 2253 tokens, 8 heads 178 -> 140; 6 of 50 - 353 38 -> 32; 4 of
+// (115 us at 4.9 TB/s by themselves) come and go partly beside other workgroups' tiles; the outputs
+// past the L2, but for those of ranges, which the join reads (348 -> 342 on one card; 5 of 114 - 142, 256 + 64: 24.7 -> 23.1; 3 of 1720 206 -> 199; ranges' 35.4 ->
+// 36.5, not so.  The queries past it: 339, but 3 of 17 - 26 13.5 -> 15.3).  2 of 2253 tokens, 8 heads 178 -> 140; 6 of 50 - 353 38 -> 32; 4 of
 // 470, 256 + 64: 35 -> 31.5; 5 of 23 - 225, 8 heads 29.0 -> 28.1.  One tile and full sets cost the two roles' one after the other: 8 portions of 8 tokens, 16
 // heads 12.5 -> 12.7, 40 of 17 15.9 -> 16.4, the largest loss seen.  (Two pieces of queries an LDS turn without bank conflicts, outputs several turns at a
 // time, no barrier behind the last weights, sets without rows only at the barriers: 13.7, 17.2 without them; 8 of 2 tokens 13.2 -> 10.1.)
-template <int DK, int DV>
+// RANGES: splits > 1 (the outputs are partial ones then)
+template <int DK, int DV, bool RANGES>
 __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
                                                                const float* __restrict__ q_abs, const bf16_t* __restrict__ cache,
                                                                const int* __restrict__ table, int64_t table_stride,
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
       const bool valid = r < QT * HB && tl < q_len && hh < H;
       const float* qrow = q_abs + (((size_t)first + (valid ? tl : tok0)) * H + (valid ? hh : h0)) * DK + role * 32 + 4 * (lane & 7);
 #pragma unroll
-      for (int u = 0; u < NU; ++u) x[u][i] = __builtin_bit_cast(float4, __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(qrow + 64 * u)));
+      for (int u = 0; u < NU; ++u) x[u][i] = *reinterpret_cast<const float4*>(qrow + 64 * u);
     }
     if (fetch) dma(img0, slot);
     else if (wave < 3 && lane < KT) s_slot[wave][lane] = slot;
@@ -220,8 +222,8 @@ __global__ __launch_bounds__(512, 2) void latent_prompt_kernel(float* __restrict
           for (int n = 0; n < some; ++n) {
             const f32x4_t x = *reinterpret_cast<const f32x4_t*>(turn + n * 4096 + ((l >> 3) + 8 * i) * 128 + (((l & 7) ^ (l >> 3)) & 7) * 16);
             f32x4_t* to = reinterpret_cast<f32x4_t*>(dst[i] + (vt0 + n) * 32);
-            if (splits == 1) __builtin_nontemporal_store(x, to);
-            else *to = x;
+            if constexpr (RANGES) *to = x;
+            else __builtin_nontemporal_store(x, to);
           }
         }
       }
@@ -677,8 +679,10 @@ extern "C" __attribute__((visibility("hidden"))) int mix_latent_attn_mfma(float*
     const size_t lds = 8 * image > join ? 8 * image : join;                                                                         \
     MIX_REQUIRE(ensure_lds((const void*)latent_decode_kernel<DK, DV>, lds) == 0, "latent_attn: %zu bytes of LDS", lds);             \
     hipLaunchKernelGGL((latent_decode_kernel<DK, DV>), grid, dim3(256), lds, s, LAT_ARGS);                                          \
+  } else if (splits > 1) {                                                                                                          \
+    hipLaunchKernelGGL((latent_prompt_kernel<DK, DV, true>), grid, dim3(512), 0, s, LAT_ARGS);                                      \
   } else {                                                                                                                          \
-    hipLaunchKernelGGL((latent_prompt_kernel<DK, DV>), grid, dim3(512), 0, s, LAT_ARGS);                                            \
+    hipLaunchKernelGGL((latent_prompt_kernel<DK, DV, false>), grid, dim3(512), 0, s, LAT_ARGS);                                     \
   }
   if (dk == 576) {
     LAT_LAUNCH(576, 512)
