@@ -1466,8 +1466,9 @@ __global__ __launch_bounds__(kRowThreads) void split_pick_kernel(SplitScratch sc
 // Both are written and read at agent scope (past the L2s); the last one leaves packets and count zero, as it found them, for the next launch.
 // Bound: a chain of launch, first read, packets' way, bound, weights, count's way, draw.
 // 64 rows x 151936 bf16: 3.3 us to the maxima, 0.7 for the packets, 3.3 to the bound (1.5 of it the slowest wave's reads: 64 addresses of 2 bytes each), 3.4 for
-// weights, candidates and sums, 0.8 for the count, 2.9 for lists and sums, 3.7 for the draw.  us a draw with its copy, three launches -> one: 64 x 151936
-// 25.4 -> 19.9, 33 x 151936 23.0 -> 17.9, 8 x 151936 19.4 -> 15.6, 1 x 151936 19.0 -> 15.2, 64 x 98304 21.6 -> 17.0, 64 x 98305 (unaligned rows) 22.9 -> 17.7.
+// weights, candidates and sums, 0.8 for the count, 2 for lists and sums (2.9 with the lists behind their lengths), 3.7 for the draw.  us a draw with its copy, three
+// launches -> one: 64 x 151936 25.4 -> 19.2, 33 x 151936 23.0 -> 17.7, 8 x 151936 19.4 -> 14.9, 1 x 151936 19.0 -> 14.3, 64 x 98304 21.6 -> 16.7, 64 x 98305
+// (unaligned rows) 22.9 -> 17.3.
 // Measured on the way (64 x 151936): columns by way of LDS tiles as in split_sum 24.5; the copy from the registers in front of the bound 23.7, by way of LDS
 // 23.5, by the workgroups that do not draw 22.0.
 // ------------------------------------------------------------------------------------------
