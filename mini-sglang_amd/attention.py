@@ -161,8 +161,10 @@ class HipAttnBackend:
 
     def takes_layers(self, batch: Any, hidden: int, intermediate: int) -> bool:
         """Whether all layers of the batch's decode step go in one launch (csrc/decode_layers.hip): a batch of `small_decode`, of a model whose layer fits the
-        compute units' LDS and gives every other one of them, at least, rows of every product."""
-        return (batch.positions.dtype == batch.out_loc.dtype == torch.int32 and hidden // 2 >= int(_lib.lib().msgl_device_cu_count()) and self.small_decode(batch)
+        compute units' LDS and gives every other one of them, at least, rows of every product.  Not prompts that extend by one token: what the launch's
+        workgroups meet in is one for all decode steps, which may run beside a prompt."""
+        return (self._decode_phase(batch) and batch.positions.dtype == batch.out_loc.dtype == torch.int32
+                and hidden // 2 >= int(_lib.lib().msgl_device_cu_count()) and self.small_decode(batch)
                 and ops.decode_layers_supported(batch.attn_metadata.batch, hidden, self.qo_heads, self.kv_heads, intermediate))
 
     def decode_layers(self, x: torch.Tensor, layers: Any, interleaved: bool, eps: float, positions: torch.Tensor, cos_sin: torch.Tensor, batch: Any):
@@ -276,10 +278,13 @@ class HipAttnBackend:
             ops.attn_decode_plan(md.plan, md.seq_lens, bs, self.max_bs, self.capacity, self.qo_heads, self.kv_heads)
         batch.attn_metadata = md
 
-    def _replayed_from_graph(self, batch: Any, padded_bs: int) -> bool:
+    @staticmethod
+    def _decode_phase(batch: Any) -> bool:
         phase = getattr(batch, "phase", None)
-        is_decode = (phase == "decode") if phase is not None else True
-        return bool(is_decode and self._cap_plan is not None and padded_bs in self.capture_bs
+        return phase == "decode" if phase is not None else True
+
+    def _replayed_from_graph(self, batch: Any, padded_bs: int) -> bool:
+        return bool(self._decode_phase(batch) and self._cap_plan is not None and padded_bs in self.capture_bs
                     and len(batch.reqs) <= self.max_graph_bs)
 
     # ------------------------------------------------------------------ graph hooks
