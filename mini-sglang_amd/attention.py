@@ -35,7 +35,7 @@ class HipAttnMetadata:
     total_tiles: int = 0
     tile_order: Optional[torch.Tensor] = None  # [total_tiles] int32: q tiles, most keys first (prefill only)
     ranges: tuple = (1, 0)                  # key ranges of a q tile, 64-key tiles of each (prefill only)
-    scratch: Optional[torch.Tensor] = None  # their partial sums, from the first layer on
+    scratch: Optional[torch.Tensor] = None  # their partial sums, or those of one-token prompts, from the first layer on
     pairs: bool = False                     # two heads a workgroup (prefill only)
     fresh: bool = False                     # short prompts that have nothing in the pool (prefill only)
     plan: Optional[torch.Tensor] = None     # decode work list (device)
@@ -145,13 +145,23 @@ class HipAttnBackend:
         md = batch.attn_metadata
         return md.max_seqlen_q == 1 and md.batch * self.kv_heads <= self._small_heads
 
+    def _decode_scratch(self, batch: Any) -> torch.Tensor:
+        """The decode kernels' partial sums: decode steps share the backend's; a prompt that extends by one token a request, which may run beside a
+        step on another stream, has its own for its layers one after the other."""
+        if self._decode_phase(batch):
+            return self._workspace
+        md: HipAttnMetadata = batch.attn_metadata
+        if md.scratch is None:
+            md.scratch = torch.empty_like(self._workspace)
+        return md.scratch
+
     def _attend_small(self, q, k, v, layer_id: int, batch: Any, **row_work) -> torch.Tensor:
         md: HipAttnMetadata = batch.attn_metadata
         k_tok, v_tok = self._kv_tokens(layer_id)
         table = self.ctx.page_table
         out = torch.empty((q.shape[0], q.shape[1]), dtype=q.dtype, device=q.device)
         ranges = ops.attn_decode_small_ranges(md.batch, self.kv_heads, table.shape[1])
-        ops.attn_decode_small(out, q, k, v, k_tok, v_tok, batch.out_loc, table, md.req_rows, md.seq_lens, self._workspace, ranges, self.scale, **row_work)
+        ops.attn_decode_small(out, q, k, v, k_tok, v_tok, batch.out_loc, table, md.req_rows, md.seq_lens, self._decode_scratch(batch), ranges, self.scale, **row_work)
         return out.view(q.shape[0], self.qo_heads, self.head_dim)
 
     def attend_new(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_w, k_norm_w, eps: float, positions: torch.Tensor,
@@ -226,7 +236,7 @@ class HipAttnBackend:
                                      self.kv_heads)
             elif md.plan is self._cap_plan:
                 self._cap_planned.add(md.batch)
-            ops.attn_decode(out, q, k_tok, v_tok, table, md.req_rows, md.seq_lens, md.plan, self._workspace,
+            ops.attn_decode(out, q, k_tok, v_tok, table, md.req_rows, md.seq_lens, md.plan, self._decode_scratch(batch),
                             md.batch, self.max_bs, self.capacity, self.scale, slot_run=self.slot_run)
         else:
             if md.ranges[0] > 1 and md.scratch is None:

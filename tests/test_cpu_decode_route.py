@@ -30,3 +30,31 @@ def test_one_token_prompts_take_no_part_in_the_decode_steps_launch(backend):
     stream, and that step's launch has its workgroups meet in memory that the backend has once."""
     assert backend.takes_layers(_batch("decode"), 1024, 3072)
     assert not backend.takes_layers(_batch("prefill"), 1024, 3072)
+
+
+@pytest.mark.parametrize("small", [True, False], ids=["small batch", "planned"])
+def test_one_token_prompts_have_partial_sums_of_their_own(backend, monkeypatch, small):
+    """Decode steps share the backend's scratch; a one-token prompt keeps its own with its batch, the same for all its layers."""
+    from mini_sglang_amd import attention
+
+    seen = []
+    if small:
+        monkeypatch.setattr(attention.ops, "attn_decode_small_ranges", lambda *a: 1)
+        monkeypatch.setattr(attention.ops, "attn_decode_small", lambda *a, **k: seen.append(a[10]))
+    else:
+        backend._small_heads = 0
+        monkeypatch.setattr(attention.ops, "attn_decode", lambda *a, **k: seen.append(a[8]))
+    pool = torch.zeros(16, 8, 128)
+    backend.scale, backend.max_bs, backend.capacity, backend.slot_run, backend.device = 1.0, 4, 64, 1, torch.device("cpu")
+    backend._cap_plan, backend.ctx = None, SimpleNamespace(page_table=torch.zeros(4, 32, dtype=torch.int32))
+    backend.kvcache = SimpleNamespace(k_cache=lambda i: pool, v_cache=lambda i: pool, store_kv=lambda *a: None, dtype=torch.float32)
+    backend._workspace = torch.empty(4096, dtype=torch.uint8)
+    q, k = torch.zeros(3, 16, 128), torch.zeros(3, 8, 128)
+    for phase in ("decode", "prefill", "prefill"):
+        batch = _batch(phase)
+        batch.attn_metadata.plan = torch.zeros(1, dtype=torch.int32)
+        for layer in range(2):
+            backend.forward(q, k, k, layer, batch)
+    assert len(seen) == 6 and seen[0] is seen[1] is backend._workspace
+    assert seen[2] is seen[3] and seen[4] is seen[5] and len({id(t) for t in seen}) == 3
+    assert seen[2].numel() == backend._workspace.numel()
