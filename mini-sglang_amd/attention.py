@@ -14,7 +14,7 @@ kernels.  Differences from the reference backends that matter for speed, none fo
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import Any, List, Optional
+from typing import Any, Dict, List, Optional
 
 import numpy as np
 import torch
@@ -114,7 +114,7 @@ class HipAttnBackend:
                  for b in range(1, self._small_heads // self.kv_heads + 1))
         self._workspace = torch.empty(max([ops.attn_decode_workspace_bytes(self.capacity, self.qo_heads, self.head_dim), *small]),
                                       dtype=torch.uint8, device=self.device)
-        self._layers_workspace: Optional[torch.Tensor] = None
+        self._layers_workspaces: Dict[tuple, torch.Tensor] = {}  # (layers, hidden size, intermediate size) -> what decode_layers' workgroups meet in
         # graph state
         self.capture_bs: List[int] = []
         self.max_graph_bs = 0
@@ -169,25 +169,32 @@ class HipAttnBackend:
         """qk-norm, RoPE, K / V store and attention of a batch that `small_decode` says yes to, from the projection's rows."""
         return self._attend_small(q, k, v, layer_id, batch, q_norm_w=q_norm_w, k_norm_w=k_norm_w, eps=eps, positions=positions, cos_sin_cache=cos_sin)
 
-    def takes_layers(self, batch: Any, hidden: int, intermediate: int) -> bool:
+    def takes_layers(self, batch: Any, hidden: int, intermediate: int, layers: int) -> bool:
         """Whether all layers of the batch's decode step go in one launch (csrc/decode_layers.hip): a batch of `small_decode`, of a model whose layer fits the
         compute units' LDS and gives every other one of them, at least, rows of every product.  Not prompts that extend by one token: what the launch's
-        workgroups meet in is one for all decode steps, which may run beside a prompt."""
+        workgroups meet in is one for all decode steps, which may run beside a prompt.  Nor a capture that no step of the model came before: the zeros that the
+        first launch starts from would be written when the graph is replayed, and by every replay."""
         return (self._decode_phase(batch) and batch.positions.dtype == batch.out_loc.dtype == torch.int32
                 and hidden // 2 >= int(_lib.lib().msgl_device_cu_count()) and self.small_decode(batch)
-                and ops.decode_layers_supported(batch.attn_metadata.batch, hidden, self.qo_heads, self.kv_heads, intermediate))
+                and ops.decode_layers_supported(batch.attn_metadata.batch, hidden, self.qo_heads, self.kv_heads, intermediate)
+                and ((layers, hidden, intermediate) in self._layers_workspaces or not torch.cuda.is_current_stream_capturing()))
+
+    def _layers_workspace(self, layers: int, hidden: int, intermediate: int) -> torch.Tensor:
+        """Zeros for a model's decode steps of all batches; like the decode workspace: one step at a time."""
+        at = (layers, hidden, intermediate)
+        if at not in self._layers_workspaces:
+            need = max(ops.decode_layers_workspace_bytes(b, layers, hidden, self.qo_heads, self.kv_heads, intermediate)
+                       for b in range(1, self._small_heads // self.kv_heads + 1)
+                       if ops.decode_layers_supported(b, hidden, self.qo_heads, self.kv_heads, intermediate))
+            self._layers_workspaces[at] = torch.zeros(need, dtype=torch.uint8, device=self.device)
+        return self._layers_workspaces[at]
 
     def decode_layers(self, x: torch.Tensor, layers: Any, interleaved: bool, eps: float, positions: torch.Tensor, cos_sin: torch.Tensor, batch: Any):
         """Every layer of a batch that `takes_layers` says yes to: the last down projection's rows and the residual stream without them."""
         md: HipAttnMetadata = batch.attn_metadata
-        if self._layers_workspace is None:  # like the decode workspace: one step at a time
-            inter, (hidden, most) = layers[0].down.shape[1], (x.shape[1], self._small_heads // self.kv_heads)
-            need = max(ops.decode_layers_workspace_bytes(b, len(layers), hidden, self.qo_heads, self.kv_heads, inter) for b in range(1, most + 1)
-                       if ops.decode_layers_supported(b, hidden, self.qo_heads, self.kv_heads, inter))
-            self._layers_workspace = torch.zeros(need, dtype=torch.uint8, device=self.device)
         tokens = [self._kv_tokens(i) for i in range(len(layers))]
         return ops.decode_layers(x, layers, [k for k, _ in tokens], [v for _, v in tokens], positions, cos_sin, batch.out_loc, self.ctx.page_table, md.req_rows,
-                                 md.seq_lens, self._layers_workspace, self.qo_heads, interleaved, eps, self.scale)
+                                 md.seq_lens, self._layers_workspace(len(layers), x.shape[1], layers[0].down.shape[1]), self.qo_heads, interleaved, eps, self.scale)
 
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_id: int, batch: Any) -> torch.Tensor:
         """Reference contract (fa.py:48-65): persist k, v at batch.out_loc, then attend.  A decode batch's out_loc is where its requests'

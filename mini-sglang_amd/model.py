@@ -377,7 +377,7 @@ class DenseDecoder:
             return r
 
         layers = self.layers
-        if small and self.tp_size == 1 and x.dtype == kv.dtype and getattr(backend, "takes_layers", lambda *a: False)(batch, cfg.hidden_size, self.inter):
+        if small and self.tp_size == 1 and x.dtype == kv.dtype and getattr(backend, "takes_layers", lambda *a: False)(batch, cfg.hidden_size, self.inter, len(layers)):
             # a small model's small batch: all layers in one launch, which leaves the last down_proj's rows for the final norm
             x, residual = backend.decode_layers(x, layers, self.gate_up_ilv, cfg.rms_norm_eps, batch.positions, self.cos_sin, batch)
             layers = ()

@@ -11,9 +11,11 @@ def backend(monkeypatch):
     from mini_sglang_amd import attention
 
     b = object.__new__(attention.HipAttnBackend)
-    b.qo_heads, b.kv_heads, b.head_dim, b._small_heads = 16, 8, 128, 64
+    b.qo_heads, b.kv_heads, b.head_dim, b._small_heads, b.device = 16, 8, 128, 64, torch.device("cpu")
+    b._layers_workspaces = {}
     monkeypatch.setattr(attention._lib, "lib", lambda: SimpleNamespace(msgl_device_cu_count=lambda: 256))
     monkeypatch.setattr(attention.ops, "decode_layers_supported", lambda *a: True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     return b
 
 
@@ -28,8 +30,28 @@ def _batch(phase, n=3):
 def test_one_token_prompts_take_no_part_in_the_decode_steps_launch(backend):
     """A prompt whose requests all extend by one token (a full hit of the prefix cache, a remainder of one token) may run beside a decode step on another
     stream, and that step's launch has its workgroups meet in memory that the backend has once."""
-    assert backend.takes_layers(_batch("decode"), 1024, 3072)
-    assert not backend.takes_layers(_batch("prefill"), 1024, 3072)
+    assert backend.takes_layers(_batch("decode"), 1024, 3072, 28)
+    assert not backend.takes_layers(_batch("prefill"), 1024, 3072, 28)
+
+
+def test_the_first_step_of_a_model_is_not_captured_as_one_launch(backend, monkeypatch):
+    """The launch's workgroups start from zeros that are written once, eagerly: a capture in front of every step takes the separate launches, one after a
+    step of the same model does not; models of other sizes have memory of their own."""
+    from mini_sglang_amd import attention
+
+    monkeypatch.setattr(attention.ops, "decode_layers_workspace_bytes", lambda b, layers, hidden, hq, hkv, inter: b * layers * (hidden + inter))
+    capturing = [True]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    assert not backend.takes_layers(_batch("decode"), 1024, 3072, 28)
+    capturing[0] = False
+    assert backend.takes_layers(_batch("decode"), 1024, 3072, 28)
+    first = backend._layers_workspace(28, 1024, 3072)
+    assert first.numel() == 8 * 28 * 4096 and not first.any()
+    capturing[0] = True
+    assert backend.takes_layers(_batch("decode"), 1024, 3072, 28) and backend._layers_workspace(28, 1024, 3072) is first
+    assert not backend.takes_layers(_batch("decode"), 1024, 3072, 40)
+    capturing[0] = False
+    assert backend._layers_workspace(40, 1024, 3072).numel() == 8 * 40 * 4096 and backend._layers_workspace(28, 1024, 3072) is first
 
 
 @pytest.mark.parametrize("small", [True, False], ids=["small batch", "planned"])
