@@ -115,6 +115,8 @@ class HipAttnBackend:
         self._workspace = torch.empty(max([ops.attn_decode_workspace_bytes(self.capacity, self.qo_heads, self.head_dim), *small]),
                                       dtype=torch.uint8, device=self.device)
         self._layers_workspaces: Dict[tuple, torch.Tensor] = {}  # (layers, hidden size, intermediate size) -> what decode_layers' workgroups meet in
+        self._layers_failed: Dict[tuple, tuple] = {}  # likewise: (pinned copy of its error word, event behind the copy)
+        self._md_calls = 0
         # graph state
         self.capture_bs: List[int] = []
         self.max_graph_bs = 0
@@ -189,6 +191,22 @@ class HipAttnBackend:
             self._layers_workspaces[at] = torch.zeros(need, dtype=torch.uint8, device=self.device)
         return self._layers_workspaces[at]
 
+    def poll_errors(self) -> None:
+        """Raise if a workgroup of a one-launch step ever gave up waiting for another one's rows (the step's logits were NaN then, not a partial result).  One
+        4-byte asynchronous copy: it looks at the word that the previous poll asked for, complete by now in any loop that synchronises once per step."""
+        for at, workspace in self._layers_workspaces.items():
+            word, done = self._layers_failed.get(at, (None, None))
+            if word is None:
+                word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            elif not done.query():
+                continue
+            if int(word[0]):
+                raise _lib.MsglError(f"decode_layers: a workgroup gave up waiting in launch {int(word[0]) & 0xffffffff}; its step's logits are NaN")
+            word.copy_(ops.decode_layers_failed(workspace), non_blocking=True)
+            done = torch.cuda.Event()
+            done.record()
+            self._layers_failed[at] = word, done
+
     def decode_layers(self, x: torch.Tensor, layers: Any, interleaved: bool, eps: float, positions: torch.Tensor, cos_sin: torch.Tensor, batch: Any):
         """Every layer of a batch that `takes_layers` says yes to: the last down projection's rows and the residual stream without them."""
         md: HipAttnMetadata = batch.attn_metadata
@@ -256,14 +274,16 @@ class HipAttnBackend:
 
     # ------------------------------------------------------------------ metadata
     def prepare_metadata(self, batch: Any) -> None:
+        self._md_calls += 1
         if self.tp_size > 1:
             # driven by the reference's scheduler nobody else sees the communicator once decode runs from captured
             # graphs: every 16th step look at the peer-to-peer error word (one 4-byte async copy; raises on a timeout)
-            self._md_calls = getattr(self, "_md_calls", 0) + 1
             if self._md_calls % 16 == 0:
                 from .kernel import poll_communicator_errors
 
                 poll_communicator_errors(sync=False)
+        if self._layers_workspaces and self._md_calls % 64 == 0:  # captured one-launch steps likewise
+            self.poll_errors()
         reqs = batch.padded_reqs
         bs = len(reqs)
         seqlens_q = np.fromiter((r.extend_len for r in reqs), dtype=np.int64, count=bs)

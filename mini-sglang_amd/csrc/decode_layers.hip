@@ -43,11 +43,15 @@ constexpr int kDlMaxLayers = 40;     // their addresses travel as kernel argumen
 constexpr int kDlLds = 159 * 1024;   // (and the kernel's own few hundred bytes)
 constexpr int kDlPart = 130;         // packets of a (task, head)'s partial sums: 128 values, reference, sum
 constexpr u64_t kGatherTicks = 5000;       // 50 us (100 MHz)
-constexpr u64_t kGiveUpTicks = 400000000;  // 4 s: no packet takes that long; what is left of the launch gives NaN
+// Looks of a wait at its packets, a microsecond or more each, until it gives up: seconds of the workgroup's own running time (a queue that is set aside
+// meanwhile does not count).  What did not come is NaN then, as is everything made of it: whoever reads it, the rows of the results and the new keys and
+// values among them; and the team's block keeps the launch's number for the host.
+constexpr int kLooks = 4000000, kLooksPause = 256;
+constexpr uint32_t kNaNs = 0x7fff7fffu;  // two of either type, or one of 32 bits
 constexpr uint32_t kClosed = 0x80000000u;
 
-// words of the team's block, 64 bytes apart: counted in, left, launch number, {launch number, size}
-enum { kTeamCount = 0, kTeamLeft = 16, kTeamEpoch = 32, kTeamSize = 48, kTeamWords = 64 };
+// words of the team's block, 64 bytes apart: counted in, left, launch number, {launch number, size}, number of the last launch in which someone gave up
+enum { kTeamCount = 0, kTeamLeft = 16, kTeamEpoch = 32, kTeamSize = 48, kTeamFailed = 64, kTeamWords = 96 };
 
 struct DlLayer {  // device addresses
   u64_t norm[2], w[4], q_norm, k_norm, k_cache, v_cache;  // w: qkv, o, gate_up, down
@@ -66,8 +70,9 @@ struct DlParams {
   int lds_images, lds_sums, lds_norms, lds_new;
   int cap[4];                         // units (groups of four rows, gate_up: of four activated columns) that a weight region holds
   int K[4];
-  int alias;                          // qkv's and gate_up's regions are also the rows' of o and down
+  int looks;                          // of a wait until it ends
   DlLayer layer[kDlMaxLayers];
+  int absent;                         // workgroup that leaves (-1: none)
 };
 static_assert(sizeof(DlParams) <= 4096, "kernel arguments");
 
@@ -101,15 +106,14 @@ __device__ __forceinline__ void dl_barrier() {
 }
 
 struct DlWait {
-  u64_t t0;
   int* dead;  // LDS: someone of this workgroup gave up
   uint32_t epoch;
 
   // false once the wait has to end
   __device__ __forceinline__ bool again(int& spins) const {
-    if ((++spins & 255) == 0) {
+    if ((++spins & (kLooksPause - 1)) == 0) {
       if (*(volatile int*)dead) return false;
-      if (__builtin_amdgcn_s_memrealtime() - t0 > kGiveUpTicks) {
+      if (spins >= dl_args()->looks) {
         *(volatile int*)dead = 1;
         return false;
       }
@@ -134,6 +138,10 @@ struct DlWait {
     for (int i = 0; i < N; ++i) {
       v[2 * i] = q[i][0];
       v[2 * i + 1] = q[i][2];
+    }
+    if (!ok) {
+#pragma unroll
+      for (int i = 0; i < 2 * N; ++i) v[i] = kNaNs;
     }
   }
 };
@@ -236,12 +244,14 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
       dl_put(size, (uint32_t)n, epoch);
     } else if (rank > 0) {  // (the first one is resident, and its wait has a limit)
       u64_t v;
+      int left = kLooks;
       do v = dl_get(size);
-      while ((uint32_t)(v >> 32) != epoch && __builtin_amdgcn_s_memrealtime() - t0 < kGiveUpTicks);
+      while ((uint32_t)(v >> 32) != epoch && --left > 0);
       n = (uint32_t)(v >> 32) == epoch ? (int)(uint32_t)v : 0;
+      if (n == 0) s_dead = 1;
       if (rank >= n) rank = -1;
     }
-    s_rank = rank;
+    s_rank = rank >= 0 && rank == dl_args()->absent ? -1 : rank;
     s_size = n;
     s_epoch = epoch;
   }
@@ -250,7 +260,7 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
   const uint32_t epoch = (uint32_t)sgpr((int)s_epoch);
 
   if (rank >= 0) {
-    const DlWait wait{t0, &s_dead, epoch};
+    const DlWait wait{&s_dead, epoch};
     const int M = dl_args()->M, layers = dl_args()->layers;
     const int f = wv - kDlFetch;  // fetching waves: 0 .. 3
     // my units (groups of four rows, gate_up: of four activated columns) of the products: qkv, o and down, gate_up
@@ -861,8 +871,7 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
               if (S < 3 || more) {
                 dl_put2(pk, out_at, (m * N + 4 * unit) * 4, lo, hi, epoch);
               } else {
-                const bool dead = *(volatile int*)&s_dead;
-                *reinterpret_cast<uint2*>(dl_ptr<uint16_t>(y_out) + (int64_t)m * N + 4 * unit) = make_uint2(dead ? 0x7fff7fffu : lo, dead ? 0x7fff7fffu : hi);
+                *reinterpret_cast<uint2*>(dl_ptr<uint16_t>(y_out) + (int64_t)m * N + 4 * unit) = make_uint2(lo, hi);
               }
             }
           }
@@ -894,6 +903,7 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
   // ---- the last one to leave opens the count for the next launch ----
   if (threadIdx.x == 0) {
     uint32_t* team = dl_ptr<uint32_t>(dl_args()->team);
+    if (*(volatile int*)&s_dead) __hip_atomic_store(team + kTeamFailed, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     s_last = __hip_atomic_fetch_add(team + kTeamLeft, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     if (s_last) {
       __hip_atomic_store(team + kTeamCount, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1000,11 +1010,14 @@ static int dl_launch(const DlParams& p, const DlLayout& a, hipStream_t s) {
   return MSGL_OK;
 }
 
-extern "C" int msgl_decode_layers(void* y_out, void* res_out, const void* x, const msgl_decode_layer_t* layer, int layers, const int32_t* positions,
-                                  const float* cos_sin, const int32_t* out_loc, const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
-                                  const int32_t* seq_lens, void* workspace, int64_t workspace_bytes, int batch, int hidden, int num_q_heads,
-                                  int num_kv_heads, int head_dim, int intermediate, int gate_up_interleaved, int64_t kv_stride_tok,
-                                  int64_t kv_stride_head, float eps, float sm_scale, int dtype, void* stream) {
+extern "C" int64_t msgl_decode_layers_failed_at(void) { return kTeamFailed * 4; }
+
+extern "C" int msgl_decode_layers_bounded(void* y_out, void* res_out, const void* x, const msgl_decode_layer_t* layer, int layers, const int32_t* positions,
+                                          const float* cos_sin, const int32_t* out_loc, const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
+                                          const int32_t* seq_lens, void* workspace, int64_t workspace_bytes, int batch, int hidden, int num_q_heads,
+                                          int num_kv_heads, int head_dim, int intermediate, int gate_up_interleaved, int64_t kv_stride_tok,
+                                          int64_t kv_stride_head, float eps, float sm_scale, int dtype, int looks, int absent, void* stream) {
+  MSGL_REQUIRE(looks >= 0, "decode_layers: %d looks", looks);
   MSGL_REQUIRE(y_out && res_out && x && layer && positions && cos_sin && out_loc && page_table && seq_lens && workspace, "decode_layers: null pointer");
   MSGL_REQUIRE(layers >= 1, "decode_layers: %d layers", layers);
   MSGL_REQUIRE(head_dim == 128, "decode_layers: head_dim %d unsupported (128 only)", head_dim);
@@ -1035,11 +1048,12 @@ extern "C" int msgl_decode_layers(void* y_out, void* res_out, const void* x, con
   p.pt_stride = pt_stride; p.kv_stride_tok = kv_stride_tok; p.kv_stride_head = kv_stride_head;
   p.M = batch; p.H = hidden; p.hq = num_q_heads; p.hkv = num_kv_heads; p.inter = intermediate;
   p.ranges = a.ranges; p.interleaved = gate_up_interleaved;
+  p.looks = looks > 0 ? looks : kLooks;
+  p.absent = absent;
   p.eps = eps;
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   p.layer_packets = (int)a.layer_packets; p.at_part = a.at_part;
   p.lds_images = a.lds_images; p.lds_sums = a.lds_sums; p.lds_norms = a.lds_norms; p.lds_new = a.lds_new;
-  p.alias = a.alias;
   const int K[4] = {hidden, num_q_heads * 128, hidden, intermediate};
   for (int i = 0; i < 4; ++i) {
     p.lds_w[i] = a.lds_w[i];
@@ -1064,4 +1078,14 @@ extern "C" int msgl_decode_layers(void* y_out, void* res_out, const void* x, con
     p.y_in = p.y_out;
   }
   return MSGL_OK;
+}
+
+extern "C" int msgl_decode_layers(void* y_out, void* res_out, const void* x, const msgl_decode_layer_t* layer, int layers, const int32_t* positions,
+                                  const float* cos_sin, const int32_t* out_loc, const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
+                                  const int32_t* seq_lens, void* workspace, int64_t workspace_bytes, int batch, int hidden, int num_q_heads,
+                                  int num_kv_heads, int head_dim, int intermediate, int gate_up_interleaved, int64_t kv_stride_tok,
+                                  int64_t kv_stride_head, float eps, float sm_scale, int dtype, void* stream) {
+  return msgl_decode_layers_bounded(y_out, res_out, x, layer, layers, positions, cos_sin, out_loc, page_table, pt_stride, req_rows, seq_lens, workspace,
+                                    workspace_bytes, batch, hidden, num_q_heads, num_kv_heads, head_dim, intermediate, gate_up_interleaved, kv_stride_tok,
+                                    kv_stride_head, eps, sm_scale, dtype, 0, -1, stream);
 }

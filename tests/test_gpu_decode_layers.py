@@ -95,8 +95,8 @@ def _case(ops, dev, dtype, H, hq, hkv, inter, lens, layers=3, page=16, norm=True
     if ws is None:
         ws = torch.zeros(ops.decode_layers_workspace_bytes(B, layers, H, hq, hkv, inter), dtype=torch.uint8, device=dev)
 
-    def launch():
-        return ops.decode_layers(*args, ws, hq, ilv, EPS, 128 ** -0.5)
+    def launch(**kw):
+        return ops.decode_layers(*args, ws, hq, ilv, EPS, 128 ** -0.5, **kw)
 
     y, res = launch()
     torch.cuda.synchronize()
@@ -125,6 +125,7 @@ def _case(ops, dev, dtype, H, hq, hkv, inter, lens, layers=3, page=16, norm=True
     for _ in range(3):  # again over the rows that it stored
         y2, res2 = launch()
         assert torch.equal(y, y2) and torch.equal(res, res2) and all(torch.equal(a[loc.long()], b[loc.long()]) for a, b in zip(caches, stored))
+    launch.ws, launch.before, launch.stored, launch.caches, launch.loc = ws, before, stored, caches, loc.long()
     return launch, y, res
 
 
@@ -168,6 +169,26 @@ def test_beside_other_work_on_the_device(ops, dev, H, hq, hkv, inter, lens):
         assert torch.equal(y, y2) and torch.equal(res, res2)
 
 
+@pytest.mark.parametrize("H,hq,hkv,inter,lens", [(1024, 16, 8, 3072, [700, 90]), (1024, 16, 8, 3072, [300] * 7), (512, 8, 1, 768, [40, 3])])
+def test_waits_that_end_are_not_silent(ops, dev, H, hq, hkv, inter, lens):
+    """A workgroup leaves without a word and the others give up waiting for it: every row has NaN, no wrong key or value is stored, the error word stays; the
+    next launch is a launch like any other."""
+    launch, y, res = _case(ops, dev, torch.bfloat16, H, hq, hkv, inter, lens)
+    assert not ops.decode_layers_failed(launch.ws).any()
+    for absent in (0, 1, 17):
+        for c, c0 in zip(launch.caches, launch.before):
+            c.copy_(c0)
+        bad = sum(launch(looks=256, absent=absent))
+        assert bad.isnan().any(dim=1).all()
+        for c, c0, c1 in zip(launch.caches, launch.before, launch.stored):
+            rows, old, new = (t[launch.loc] for t in (c, c0, c1))
+            assert (rows.isnan() | (rows.view(torch.int16) == old.view(torch.int16)) | (rows == new)).all()
+        for _ in range(2):
+            y2, res2 = launch()
+            assert torch.equal(y, y2) and torch.equal(res, res2) and all(torch.equal(a[launch.loc], b[launch.loc]) for a, b in zip(launch.caches, launch.stored))
+        assert ops.decode_layers_failed(launch.ws).all()
+
+
 @pytest.mark.parametrize("batch", [1, 3, 8])
 def test_captured_steps_of_an_engine(dev, batch):
     """An engine whose steps take the launch: every replay gives the eager step's bits."""
@@ -200,6 +221,14 @@ def test_captured_steps_of_an_engine(dev, batch):
             assert torch.equal(got, want)
         assert len(calls) == 4  # (the eager ones; the captured one was made by the engine)
         assert o.decode_layers_supported(batch, 1024, 16, 8, 3072)
+        for _ in range(130):  # the error word reaches the host
+            eng.attn_backend.prepare_metadata(step)
+            torch.cuda.synchronize()
+        o.decode_layers_failed(next(iter(eng.attn_backend._layers_workspaces.values()))).fill_(7)
+        with pytest.raises(Exception, match="gave up"):
+            for _ in range(130):
+                eng.attn_backend.prepare_metadata(step)
+                torch.cuda.synchronize()
     finally:
         attention.HipAttnBackend.decode_layers = real
         eng.shutdown()
