@@ -72,7 +72,7 @@ struct DlParams {
   int K[4];
   int looks;                          // of a wait until it ends
   DlLayer layer[kDlMaxLayers];
-  int absent;                         // workgroup that leaves (-1: none)
+  int absent, most;                   // workgroup that leaves (-1: none), and size of the team at most
 };
 static_assert(sizeof(DlParams) <= 4096, "kernel arguments");
 
@@ -238,9 +238,10 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
     int rank = mine & kClosed ? -1 : (int)mine, n = 0;
     if (rank == 0) {
       uint32_t have = 1;
-      while (have < gridDim.x && __builtin_amdgcn_s_memrealtime() - t0 < kGatherTicks)
+      const uint32_t most = min(gridDim.x, (uint32_t)dl_args()->most);
+      while (have < most && __builtin_amdgcn_s_memrealtime() - t0 < kGatherTicks)
         have = __hip_atomic_load(team + kTeamCount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      n = (int)__hip_atomic_fetch_or(team + kTeamCount, kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      n = (int)min(most, __hip_atomic_fetch_or(team + kTeamCount, kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
       dl_put(size, (uint32_t)n, epoch);
     } else if (rank > 0) {  // (the first one is resident, and its wait has a limit)
       u64_t v;
@@ -1016,8 +1017,8 @@ extern "C" int msgl_decode_layers_bounded(void* y_out, void* res_out, const void
                                           const float* cos_sin, const int32_t* out_loc, const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
                                           const int32_t* seq_lens, void* workspace, int64_t workspace_bytes, int batch, int hidden, int num_q_heads,
                                           int num_kv_heads, int head_dim, int intermediate, int gate_up_interleaved, int64_t kv_stride_tok,
-                                          int64_t kv_stride_head, float eps, float sm_scale, int dtype, int looks, int absent, void* stream) {
-  MSGL_REQUIRE(looks >= 0, "decode_layers: %d looks", looks);
+                                          int64_t kv_stride_head, float eps, float sm_scale, int dtype, int looks, int absent, int most, void* stream) {
+  MSGL_REQUIRE(looks >= 0 && most >= 0, "decode_layers: %d looks, a team of %d", looks, most);
   MSGL_REQUIRE(y_out && res_out && x && layer && positions && cos_sin && out_loc && page_table && seq_lens && workspace, "decode_layers: null pointer");
   MSGL_REQUIRE(layers >= 1, "decode_layers: %d layers", layers);
   MSGL_REQUIRE(head_dim == 128, "decode_layers: head_dim %d unsupported (128 only)", head_dim);
@@ -1050,6 +1051,7 @@ extern "C" int msgl_decode_layers_bounded(void* y_out, void* res_out, const void
   p.ranges = a.ranges; p.interleaved = gate_up_interleaved;
   p.looks = looks > 0 ? looks : kLooks;
   p.absent = absent;
+  p.most = most > 0 ? most : a.cus;
   p.eps = eps;
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   p.layer_packets = (int)a.layer_packets; p.at_part = a.at_part;
@@ -1087,5 +1089,5 @@ extern "C" int msgl_decode_layers(void* y_out, void* res_out, const void* x, con
                                   int64_t kv_stride_head, float eps, float sm_scale, int dtype, void* stream) {
   return msgl_decode_layers_bounded(y_out, res_out, x, layer, layers, positions, cos_sin, out_loc, page_table, pt_stride, req_rows, seq_lens, workspace,
                                     workspace_bytes, batch, hidden, num_q_heads, num_kv_heads, head_dim, intermediate, gate_up_interleaved, kv_stride_tok,
-                                    kv_stride_head, eps, sm_scale, dtype, 0, -1, stream);
+                                    kv_stride_head, eps, sm_scale, dtype, 0, -1, 0, stream);
 }

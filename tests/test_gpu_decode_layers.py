@@ -155,7 +155,8 @@ def test_batches_share_a_workspace(ops, dev):
 
 @pytest.mark.parametrize("H,hq,hkv,inter,lens", [(1024, 16, 8, 3072, [700, 90]), (1024, 16, 8, 3072, [300] * 7), (1024, 24, 4, 768, [40])])
 def test_beside_other_work_on_the_device(ops, dev, H, hq, hkv, inter, lens):
-    """Workgroups that find their CU taken are not waited for (seen: teams of 64 to 254 of 256): the others do their share, with the same bits."""
+    """Workgroups that find their CU taken are not waited for: the others do their share, with the same bits (of teams of a given size:
+    test_small_teams)."""
     launch, y, res = _case(ops, dev, torch.bfloat16, H, hq, hkv, inter, lens)
     a = torch.randn((8192, 8192), device=dev, dtype=torch.bfloat16)
     side = torch.cuda.Stream()
@@ -167,6 +168,33 @@ def test_beside_other_work_on_the_device(ops, dev, H, hq, hkv, inter, lens):
         y2, res2 = launch()
         torch.cuda.synchronize()
         assert torch.equal(y, y2) and torch.equal(res, res2)
+
+
+@pytest.mark.parametrize("H,hq,hkv,inter,lens", [(1024, 16, 8, 3072, [700, 90]), (1024, 16, 8, 3072, [2100, 300, 5, 17, 64, 129, 1, 40]), (1024, 24, 4, 768, [40]),
+                                                 (512, 8, 1, 768, [1300, 3])])
+def test_small_teams(ops, dev, H, hq, hkv, inter, lens):
+    """Teams down to one workgroup: shares in several turns, weights fetched behind the rows, several (request, kv head, range) tasks each; the full team's bits."""
+    launch, y, res = _case(ops, dev, torch.bfloat16, H, hq, hkv, inter, lens)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    for most in (1, 2, 3, 31, 64, 130, cus - 1, cus):
+        for c, c0 in zip(launch.caches, launch.before):
+            c.copy_(c0)
+        y2, res2 = launch(most=most)
+        torch.cuda.synchronize()
+        size = int(launch.ws[192:196].view(torch.int32)[0])  # what the launch's first workgroup told the others
+        assert size == most or most > 130 and 130 < size <= most
+        assert torch.equal(y, y2) and torch.equal(res, res2) and all(torch.equal(a[launch.loc], b[launch.loc]) for a, b in zip(launch.caches, launch.stored)), most
+
+
+def test_launch_numbers_start_again(ops, dev):
+    """The last number's launch clears the packets: none of an earlier launch could pass for one of a later launch with the same number."""
+    launch, y, res = _case(ops, dev, torch.bfloat16, 1024, 16, 8, 3072, [700, 90])
+    number, packets = launch.ws[128:132].view(torch.int32), launch.ws[384:].view(torch.int64)
+    number.fill_(-3)
+    for want in (-2, -1, 1, 2):
+        y2, res2 = launch()
+        assert int(number[0]) == want and torch.equal(y, y2) and torch.equal(res, res2)
+        assert bool(packets.any()) == (want != -1)
 
 
 @pytest.mark.parametrize("H,hq,hkv,inter,lens", [(1024, 16, 8, 3072, [700, 90]), (1024, 16, 8, 3072, [300] * 7), (512, 8, 1, 768, [40, 3])])
