@@ -220,10 +220,11 @@ int msgl_attn_decode_small(void* out, const void* q, const void* k, const void* 
  * Weights are contiguous [rows, columns]; gate_up_interleaved: gate_up rows in blocks of 32 gate, 32 up.  head_dim 128, batch 1 .. 8, hidden and
  * intermediate size multiples of 256; _supported says whether a CU's share of a layer fits its LDS.
  * `workspace` is zero before its first launch and belongs to these launches, one at a time.  The launch has one workgroup per CU, which wait for
- * each other, and none for one that is not running: a launch that finds CUs taken goes on without them.  Capturable.
+ * each other, and none for one that is not running: a launch that finds CUs taken goes on without them until, layer by layer, they are there.  Capturable.
  * A wait ends after `looks` looks at memory all the same (_bounded; counted in 256s; 0: 4 million, seconds).  What did not come is NaN then, and so is what is
  * made of it, results and the pool's new rows (those of a workgroup that is not there stay as they were); the 32-bit word at _failed_at() bytes of the workspace is not zero from then on.
- * What nothing but a test wants: absent, a workgroup of the team (by its number, -1: none) that leaves without a word; most, workgroups of the team (0: all). */
+ * What nothing but a test wants: absent, a workgroup of the team (by its number, -1: none) that leaves without a word; most, workgroups of the team
+ * (0: all) in the layers before `until`. */
 typedef struct {
   const void *input_norm, *qkv, *q_norm, *k_norm, *o, *post_norm, *gate_up, *down;
   void *k_cache, *v_cache;
@@ -240,7 +241,7 @@ int msgl_decode_layers_bounded(void* y_out, void* res_out, const void* x, const 
                                const float* cos_sin, const int32_t* out_loc, const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
                                const int32_t* seq_lens, void* workspace, int64_t workspace_bytes, int batch, int hidden, int num_q_heads,
                                int num_kv_heads, int head_dim, int intermediate, int gate_up_interleaved, int64_t kv_stride_tok,
-                               int64_t kv_stride_head, float eps, float sm_scale, int dtype, int looks, int absent, int most, void* stream);
+                               int64_t kv_stride_head, float eps, float sm_scale, int dtype, int looks, int absent, int most, int until, void* stream);
 /* Which partial-attention kernel msgl_attn_decode_plan / msgl_attn_decode use from now on (process-wide; plan and
  * launch must be made under the same choice): 0 = default = the matrix-core kernel for every slot_run (token-granular
  * tables, slot_run < 16, are gathered by per-lane addresses on the same kernel; whole-line nt requests with K transposed through

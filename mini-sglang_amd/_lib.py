@@ -74,7 +74,7 @@ HIP_SIGNATURES = {
     "msgl_decode_layers_supported": (_i, [_i, _i, _i, _i, _i]),
     "msgl_decode_layers_workspace_bytes": (_l, [_i, _i, _i, _i, _i, _i]),
     "msgl_decode_layers": (_i, [_p, _p, _p, _p, _i, _p, _p, _p, _p, _l, _p, _p, _p, _l, _i, _i, _i, _i, _i, _i, _i, _l, _l, _f, _f, _i, _p]),
-    "msgl_decode_layers_bounded": (_i, [_p, _p, _p, _p, _i, _p, _p, _p, _p, _l, _p, _p, _p, _l, _i, _i, _i, _i, _i, _i, _i, _l, _l, _f, _f, _i, _i, _i, _i, _p]),
+    "msgl_decode_layers_bounded": (_i, [_p, _p, _p, _p, _i, _p, _p, _p, _p, _l, _p, _p, _p, _l, _i, _i, _i, _i, _i, _i, _i, _l, _l, _f, _f, _i, _i, _i, _i, _i, _p]),
     "msgl_decode_layers_failed_at": (_l, []),
     "msgl_attn_prefill": (
         _i,

@@ -12,8 +12,9 @@
 //     has them knows its own waves done with the stages before: LDS regions need no barriers of their own against being overwritten;
 //   * four waves fetch rows (and norm, rotate, stage them), four fetch weights, multiply and attend: a row's request never stands behind a weight's in
 //     its own wave.
-// The TEAM is who is there: a workgroup counts itself in, the first one closes the count when all have come or after kGatherTicks, and latecomers leave.  All
-// work is dealt out by the team's size, so that no workgroup ever waits for one that is not resident, whatever else runs on the device.
+// The TEAM is who is there: a workgroup counts itself in, and the first one says how many they are, when all have come or after kGatherTicks, and for each
+// layer after that until all have: latecomers join at the next layer.  All work is dealt out by the team's size, so that no workgroup ever waits for one
+// that is not resident, whatever else runs on the device.
 // Rounding points are those of the separate launches (msgl_fused_add_rmsnorm, the projections, msgl_qk_norm_rope_store, msgl_silu_and_mul_interleaved).
 //
 // Bound: latency.  A hop between 256 workgroups is 1.3 us by itself, there are five in a layer (six where a request's keys are cut into ranges), and 0.6 - 0.8 us of
@@ -48,10 +49,10 @@ constexpr u64_t kGatherTicks = 5000;       // 50 us (100 MHz)
 // values among them; and the team's block keeps the launch's number for the host.
 constexpr int kLooks = 4000000, kLooksPause = 256;
 constexpr uint32_t kNaNs = 0x7fff7fffu;  // two of either type, or one of 32 bits
-constexpr uint32_t kClosed = 0x80000000u;
 
-// words of the team's block, 64 bytes apart: counted in, left, launch number, {launch number, size}, number of the last launch in which someone gave up
-enum { kTeamCount = 0, kTeamLeft = 16, kTeamEpoch = 32, kTeamSize = 48, kTeamFailed = 64, kTeamWords = 96 };
+// words of the team's block, 64 bytes apart: counted in, left, launch number, number of the last launch in which someone gave up, and from kTeamSizes on
+// {launch number, size * 2, + 1 where it stays so} of each layer
+enum { kTeamCount = 0, kTeamLeft = 16, kTeamEpoch = 32, kTeamFailed = 48, kTeamSizes = 64, kTeamWords = kTeamSizes + 2 * kDlMaxLayers };
 
 struct DlLayer {  // device addresses
   u64_t norm[2], w[4], q_norm, k_norm, k_cache, v_cache;  // w: qkv, o, gate_up, down
@@ -72,7 +73,7 @@ struct DlParams {
   int K[4];
   int looks;                          // of a wait until it ends
   DlLayer layer[kDlMaxLayers];
-  int absent, most;                   // workgroup that leaves (-1: none), and size of the team at most
+  int absent, most, until;            // workgroup that leaves (-1: none), and size of the team at most in the layers before `until`
 };
 static_assert(sizeof(DlParams) <= 4096, "kernel arguments");
 
@@ -214,13 +215,20 @@ __device__ __forceinline__ f32x4 dl_over_blocks(const f32x4& v0, const f32x4& v1
 }
 __device__ __forceinline__ float dl_wave_sum(float x) { return sum_over_rows(row16_sum(x)); }
 
+// the team of layer l at most, and its size (* 2, + 1 where it stays so) if `have` have come
+__device__ __forceinline__ uint32_t dl_most(int l) { return l < dl_args()->until ? min(gridDim.x, (uint32_t)dl_args()->most) : gridDim.x; }
+__device__ __forceinline__ int dl_size(uint32_t have, int l) {
+  const uint32_t size = min(have, dl_most(l));
+  return (int)(2 * size + (size == gridDim.x || l + 1 == dl_args()->layers));
+}
+
 template <typename T, int MQ>
 __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlParams) {
   constexpr int D = 128;
   constexpr int kRow = kDlRow / 256;         // pieces of a row of the residual stream: MQ rows a fetching wave
   constexpr int kDlAhead = 2;                // 16-token tiles of a wave in registers, asked for a layer ahead
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  __shared__ int s_dead, s_rank, s_size, s_last;
+  __shared__ int s_dead, s_rank, s_size, s_from, s_last;
   __shared__ uint32_t s_epoch;
   __shared__ float2 s_stat[4][8];
   const int lane = threadIdx.x & 63;
@@ -233,31 +241,38 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
     s_dead = 0;
     const uint32_t before = __hip_atomic_load(team + kTeamEpoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t epoch = before == 0xffffffffu ? 1 : before + 1;
-    u64_t* size = reinterpret_cast<u64_t*>(team + kTeamSize);
-    const uint32_t mine = __hip_atomic_fetch_add(team + kTeamCount, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    int rank = mine & kClosed ? -1 : (int)mine, n = 0;
+    u64_t* sizes = reinterpret_cast<u64_t*>(team + kTeamSizes);
+    int rank = (int)__hip_atomic_fetch_add(team + kTeamCount, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), size = 0, from = 0;
     if (rank == 0) {
+      const uint32_t most = dl_most(0);
       uint32_t have = 1;
-      const uint32_t most = min(gridDim.x, (uint32_t)dl_args()->most);
       while (have < most && __builtin_amdgcn_s_memrealtime() - t0 < kGatherTicks)
         have = __hip_atomic_load(team + kTeamCount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      n = (int)min(most, __hip_atomic_fetch_or(team + kTeamCount, kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-      dl_put(size, (uint32_t)n, epoch);
-    } else if (rank > 0) {  // (the first one is resident, and its wait has a limit)
-      u64_t v;
-      int left = kLooks;
-      do v = dl_get(size);
-      while ((uint32_t)(v >> 32) != epoch && --left > 0);
-      n = (uint32_t)(v >> 32) == epoch ? (int)(uint32_t)v : 0;
-      if (n == 0) s_dead = 1;
-      if (rank >= n) rank = -1;
+      size = dl_size(have, 0);
+      dl_put(sizes, (uint32_t)size, epoch);
+    } else {  // until there is a layer that I am in (the first one is resident)
+      int left = dl_args()->looks;
+      for (;;) {
+        const u64_t v = dl_get(sizes + from);
+        if ((uint32_t)(v >> 32) == epoch) {
+          size = (int)(uint32_t)v;
+          if (rank < size >> 1) break;
+          if (size & 1) rank = -1;
+          else ++from;
+        } else if (--left <= 0) {
+          s_dead = 1;
+          rank = -1;
+        }
+        if (rank < 0) break;
+      }
     }
     s_rank = rank >= 0 && rank == dl_args()->absent ? -1 : rank;
-    s_size = n;
+    s_size = size;
+    s_from = from;
     s_epoch = epoch;
   }
   __syncthreads();
-  const int rank = sgpr(s_rank), n = sgpr(s_size);
+  const int rank = sgpr(s_rank), from = sgpr(s_from);
   const uint32_t epoch = (uint32_t)sgpr((int)s_epoch);
 
   if (rank >= 0) {
@@ -266,16 +281,32 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
     const int f = wv - kDlFetch;  // fetching waves: 0 .. 3
     // my units (groups of four rows, gate_up: of four activated columns) of the products: qkv, o and down, gate_up
     const int qkv_rows = (dl_args()->hq + 2 * dl_args()->hkv) * D;
-    auto bound = [&](int rows, int r) { return (int)((uint32_t)(rows >> 2) * (uint32_t)r / (uint32_t)n); };
-    const int first_qkv = bound(qkv_rows, rank), count_qkv = bound(qkv_rows, rank + 1) - first_qkv;
-    const int first_hid = bound(dl_args()->H, rank), count_hid = bound(dl_args()->H, rank + 1) - first_hid;
-    const int first_act = bound(dl_args()->inter, rank), count_act = bound(dl_args()->inter, rank + 1) - first_act;
+    int n, first_qkv, count_qkv, first_hid, count_hid, first_act, count_act;
+    bool open, ahead;  // the team may grow; all units have a place, and what comes next is asked for ahead, else (a small team) they take turns
     auto first_of = [&](int s) { return s == 0 ? first_qkv : s == 2 ? first_act : first_hid; };
     auto count_of = [&](int s) { return s == 0 ? count_qkv : s == 2 ? count_act : count_hid; };
     auto cap_of = [&](int s) { return dl_args()->cap[s]; };
-    // all units have a place, and what comes next is asked for ahead; else (a small team) they take turns
-    const bool ahead = count_qkv <= cap_of(0) && count_hid <= cap_of(1) && count_act <= cap_of(2);
     auto passes_of = [&](int s) { return ahead ? 1 : max(1, (count_of(s) + cap_of(s) - 1) / cap_of(s)); };
+    auto deal = [&](int size) {
+      n = size >> 1;
+      open = !(size & 1);
+      auto bound = [&](int rows, int r) { return (int)((uint32_t)(rows >> 2) * (uint32_t)r / (uint32_t)n); };
+      first_qkv = bound(qkv_rows, rank);
+      count_qkv = bound(qkv_rows, rank + 1) - first_qkv;
+      first_hid = bound(dl_args()->H, rank);
+      count_hid = bound(dl_args()->H, rank + 1) - first_hid;
+      first_act = bound(dl_args()->inter, rank);
+      count_act = bound(dl_args()->inter, rank + 1) - first_act;
+      ahead = count_qkv <= cap_of(0) && count_hid <= cap_of(1) && count_act <= cap_of(2);
+    };
+    deal(sgpr(s_size));
+    // between two layers, in front of layer l: true if the team has another size than in the one before, during which a fetching wave has looked
+    auto grown = [&](int l) {
+      if (!open || l <= from) return false;
+      const int size = sgpr(*(volatile int*)&s_size), before = n;
+      deal(size);
+      return n != before;
+    };
 
     // ---- weights: a wave fetches, keeps and multiplies 128 columns of every 512 of all units ----
     // One 1-KB piece is 128 columns of a group of four rows: 16-byte piece (column c, row r) at (4 c + r) * 16, so that a DMA reads 256 contiguous bytes of
@@ -670,8 +701,13 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
       // ---- fetching waves: stage rows, meet the multiplying waves at a barrier ----
       f32x4 cosv = {0.f, 0.f, 0.f, 0.f}, sinv = cosv;
       if (works) angles_of(mine, cosv, sinv);
-      const int heads = M * dl_args()->hq, first_join = f == 0 && dl_args()->ranges > 1 ? n - 1 - rank : heads;
-      const int active0 = first_join < heads ? sgpr(active_of(first_join)) : 0;
+      const int heads = M * dl_args()->hq;
+      int first_join, active0;
+      auto join_of = [&] {
+        first_join = f == 0 && dl_args()->ranges > 1 ? n - 1 - rank : heads;
+        active0 = first_join < heads ? sgpr(active_of(first_join)) : 0;
+      };
+      join_of();
       {
         const dl_args_t p = dl_args();
         const int H = p->H, per_row = H >> 8;
@@ -698,35 +734,53 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
       };
       for (int l = 0; l < layers; ++l) {
         const __amdgpu_buffer_rsrc_t pk = packets_of(l);
+        if (grown(l)) join_of();
+        // While the team may grow, the last of these waves of the first workgroup says which size the next layer's has, and everyone's looks for it
+        const bool asks = open && f == kDlFetch - 1 && l >= from && l + 1 < layers;
+        uint32_t* team = dl_ptr<uint32_t>(dl_args()->team);
+        u64_t* next = reinterpret_cast<u64_t*>(team + kTeamSizes) + l + 1;
+        uint32_t have = 0;
+        if (asks && rank == 0) have = __hip_atomic_load(team + kTeamCount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         {
           const dl_args_t p = dl_args();
           add_norm(l ? 2 : p->y_in ? 1 : 0, packets_of(max(l - 1, 0)), p->at[3] * 8, 0);
         }
-        dl_barrier();  // qkv's rows are there
-        sums_of(0);
+        if (asks && rank == 0) dl_put(next, (uint32_t)dl_size(have, l + 1), epoch);
+        if (l >= from) {  // (a latecomer follows the residual stream to the layer that it joins at)
+          dl_barrier();  // qkv's rows are there
+          sums_of(0);
 #pragma unroll 1
-        for (int id = rank; id < tasks; id += n) {
-          Task t = mine;
-          f32x4 cv = cosv, sv = sinv;
-          if (id != rank) {
-            t = task_of(id);
-            angles_of(t, cv, sv);
+          for (int id = rank; id < tasks; id += n) {
+            Task t = mine;
+            f32x4 cv = cosv, sv = sinv;
+            if (id != rank) {
+              t = task_of(id);
+              angles_of(t, cv, sv);
+            }
+            if (t.r < t.active) attend_rows(t, l, pk, cv, sv);
           }
-          if (t.r < t.active) attend_rows(t, l, pk, cv, sv);
-        }
 #pragma unroll 1
-        for (int id = first_join; id < heads; id += n) {
-          const int active = id == first_join ? active0 : active_of(id);
-          if (active > 1) join(id, active, pk);
+          for (int id = first_join; id < heads; id += n) {
+            const int active = id == first_join ? active0 : active_of(id);
+            if (active > 1) join(id, active, pk);
+          }
+          take_rows(pk, dl_args()->at[4] * 8, dl_args()->K[1], dl_args()->lds_rows[1]);
+          dl_barrier();  // o's rows are there
+          sums_of(1);
         }
-        take_rows(pk, dl_args()->at[4] * 8, dl_args()->K[1], dl_args()->lds_rows[1]);
-        dl_barrier();  // o's rows are there
-        sums_of(1);
         add_norm(2, pk, dl_args()->at[1] * 8, 1);
+        if (l < from) continue;
         dl_barrier();  // gate_up's rows are there
         sums_of(2);
+        u64_t seen = 0;
+        if (asks) seen = dl_get(next);
         take_rows(pk, dl_args()->at[2] * 8, dl_args()->K[3], dl_args()->lds_rows[3]);
-        dl_barrier();  // down's rows are there
+        if (asks) {
+          int spins = 0;
+          while ((uint32_t)(seen >> 32) != epoch && wait.again(spins)) seen = dl_get(next);
+          if ((uint32_t)(seen >> 32) == epoch) *(volatile int*)&s_size = (int)(uint32_t)seen;
+        }
+        dl_barrier();  // down's rows, and the team's next size, are there
         sums_of(3);
       }
       if (rank == 0) {
@@ -745,14 +799,17 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
       int slots[kDlAhead];  // of my first task's first tiles, the same in every layer
       if (works) {
         slots_of(mine, slots);
-        load_ahead(pre, mine, 0, slots);
+        load_ahead(pre, mine, from, slots);
       }
       if (wv == 1) {
-        fetch_norms(0, 0);
-        fetch_norms(0, 1);
+        fetch_norms(from, 0);
+        fetch_norms(from, 1);
       }
-      if (ahead)
-        for (int s = 0; s < 4; ++s) fetch(s, 0, first_of(s), count_of(s));
+      auto fetch_first = [&](int l) {  // a layer's products that nothing before has asked for
+        fetch(0, l, first_qkv, count_qkv);
+        fetch(1, l, first_hid, count_hid);
+      };
+      if (ahead) fetch_first(from);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       dl_barrier();  // the first norm weights are there
 
@@ -782,8 +839,8 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (asked for two stages ago)
         if (ahead) {
           read_weights();
-          if (S == 0 && l > 0) fetch(2, l, first_act, count_act);
-          if (S == 1 && l > 0) fetch(3, l, first_hid, count_hid);
+          if (S == 0) fetch(2, l, first_act, count_act);
+          if (S == 1) fetch(3, l, first_hid, count_hid);
           if (S == 2 && more) fetch(0, l + 1, first_qkv, count_qkv);
           if (S == 3 && more) fetch(1, l + 1, first_hid, count_hid);
         }
@@ -881,7 +938,7 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
           dl_barrier();  // the sums are read
         }
       };
-      for (int l = 0; l < layers; ++l) {
+      for (int l = from; l < layers; ++l) {
         stage(std::integral_constant<int, 0>{}, l);
 #pragma unroll 1
         for (int id = rank; id < tasks; id += n) {
@@ -897,6 +954,10 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
         stage(std::integral_constant<int, 1>{}, l);
         stage(std::integral_constant<int, 2>{}, l);
         stage(std::integral_constant<int, 3>{}, l);
+        if (open && l + 1 < layers && grown(l + 1) && ahead) {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (what was asked for of other shares)
+          fetch_first(l + 1);
+        }
       }
     }
   }
@@ -912,11 +973,11 @@ __global__ __launch_bounds__(kDlThreads, 2) void decode_layers_kernel(const DlPa
       __hip_atomic_store(team + kTeamEpoch, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
-  if (epoch == 0xffffffffu) {  // the numbers start again: no packet of any earlier launch stays
+  if (epoch == 0xffffffffu) {  // the numbers start again: no packet of any earlier launch stays, and no size
     __syncthreads();
     if (s_last) {
-      u64_t* packets = dl_ptr<u64_t>(dl_args()->packets);
-      const int64_t all = dl_args()->packets_all;
+      u64_t* packets = dl_ptr<u64_t>(dl_args()->packets) - kDlMaxLayers;
+      const int64_t all = dl_args()->packets_all + kDlMaxLayers;
       for (int64_t i = threadIdx.x; i < all; i += kDlThreads) packets[i] = 0;
     }
   }
@@ -1017,8 +1078,8 @@ extern "C" int msgl_decode_layers_bounded(void* y_out, void* res_out, const void
                                           const float* cos_sin, const int32_t* out_loc, const int32_t* page_table, int64_t pt_stride, const int32_t* req_rows,
                                           const int32_t* seq_lens, void* workspace, int64_t workspace_bytes, int batch, int hidden, int num_q_heads,
                                           int num_kv_heads, int head_dim, int intermediate, int gate_up_interleaved, int64_t kv_stride_tok,
-                                          int64_t kv_stride_head, float eps, float sm_scale, int dtype, int looks, int absent, int most, void* stream) {
-  MSGL_REQUIRE(looks >= 0 && most >= 0, "decode_layers: %d looks, a team of %d", looks, most);
+                                          int64_t kv_stride_head, float eps, float sm_scale, int dtype, int looks, int absent, int most, int until, void* stream) {
+  MSGL_REQUIRE(looks >= 0 && most >= 0 && until >= 0, "decode_layers: %d looks, a team of %d before layer %d", looks, most, until);
   MSGL_REQUIRE(y_out && res_out && x && layer && positions && cos_sin && out_loc && page_table && seq_lens && workspace, "decode_layers: null pointer");
   MSGL_REQUIRE(layers >= 1, "decode_layers: %d layers", layers);
   MSGL_REQUIRE(head_dim == 128, "decode_layers: head_dim %d unsupported (128 only)", head_dim);
@@ -1051,7 +1112,8 @@ extern "C" int msgl_decode_layers_bounded(void* y_out, void* res_out, const void
   p.ranges = a.ranges; p.interleaved = gate_up_interleaved;
   p.looks = looks > 0 ? looks : kLooks;
   p.absent = absent;
-  p.most = most > 0 ? most : a.cus;
+  p.most = most;
+  p.until = most > 0 ? until : 0;
   p.eps = eps;
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   p.layer_packets = (int)a.layer_packets; p.at_part = a.at_part;
@@ -1089,5 +1151,5 @@ extern "C" int msgl_decode_layers(void* y_out, void* res_out, const void* x, con
                                   int64_t kv_stride_head, float eps, float sm_scale, int dtype, void* stream) {
   return msgl_decode_layers_bounded(y_out, res_out, x, layer, layers, positions, cos_sin, out_loc, page_table, pt_stride, req_rows, seq_lens, workspace,
                                     workspace_bytes, batch, hidden, num_q_heads, num_kv_heads, head_dim, intermediate, gate_up_interleaved, kv_stride_tok,
-                                    kv_stride_head, eps, sm_scale, dtype, 0, -1, 0, stream);
+                                    kv_stride_head, eps, sm_scale, dtype, 0, -1, 0, 0, stream);
 }

@@ -414,11 +414,13 @@ def decode_layers_workspace_bytes(batch: int, layers: int, hidden: int, num_q_he
 
 def decode_layers(x: torch.Tensor, layers, k_caches, v_caches, positions: torch.Tensor, cos_sin_cache: torch.Tensor, out_loc: torch.Tensor,
                   page_table: torch.Tensor, req_rows: Optional[torch.Tensor], seq_lens: torch.Tensor, workspace: torch.Tensor, num_q_heads: int,
-                  gate_up_interleaved: bool, eps: float, sm_scale: float, looks: int = 0, absent: int = -1, most: int = 0) -> Tuple[torch.Tensor, torch.Tensor]:
+                  gate_up_interleaved: bool, eps: float, sm_scale: float, looks: int = 0, absent: int = -1, most: int = 0,
+                  until: int = 1 << 30) -> Tuple[torch.Tensor, torch.Tensor]:
     """Every decoder layer of a small decode batch in one launch (see msgl_hip.h): x [B, hidden] = the residual stream in front of the first of `layers`
     (model.LayerWeights); k_caches / v_caches: [slots, Hkv, D] of each.  Returns the last down projection's rows and the residual stream without them.
     looks: how often a workgroup looks for another one's rows before it gives up (0: the library's limit); see decode_layers_failed.
-    Tests: absent, a workgroup that leaves without a word; most, workgroups that take part (0: as many as find a place)."""
+    Tests: absent, a workgroup that leaves without a word; most, workgroups that take part in the layers before `until` (0: as
+    many as find a place)."""
     _need_cuda(x, positions, cos_sin_cache, out_loc, page_table, seq_lens, workspace)
     layers, k_caches, v_caches = list(layers), list(k_caches), list(v_caches)
     B, H = x.shape
@@ -445,7 +447,7 @@ def decode_layers(x: torch.Tensor, layers, k_caches, v_caches, positions: torch.
             y.data_ptr(), res.data_ptr(), x.data_ptr(), C.cast(table, C.c_void_p), len(layers), positions.data_ptr(), cos_sin_cache.data_ptr(),
             out_loc.data_ptr(), page_table.data_ptr(), page_table.stride(0), req_rows.data_ptr() if req_rows is not None else None, seq_lens.data_ptr(),
             workspace.data_ptr(), workspace.numel() * workspace.element_size(), B, H, num_q_heads, hkv, D, inter, int(gate_up_interleaved),
-            k_caches[0].stride(0), k_caches[0].stride(1), float(eps), float(sm_scale), _dt(x), int(looks), int(absent), int(most), _stream(),
+            k_caches[0].stride(0), k_caches[0].stride(1), float(eps), float(sm_scale), _dt(x), int(looks), int(absent), int(most), int(until), _stream(),
         ),
         "decode_layers",
     )

@@ -181,15 +181,41 @@ def test_small_teams(ops, dev, H, hq, hkv, inter, lens):
             c.copy_(c0)
         y2, res2 = launch(most=most)
         torch.cuda.synchronize()
-        size = int(launch.ws[192:196].view(torch.int32)[0])  # what the launch's first workgroup told the others
-        assert size == most or most > 130 and 130 < size <= most
+        first, *_, last = _team_sizes(launch.ws)
+        assert last == most if most < cus - 1 else 130 < first <= last <= most
         assert torch.equal(y, y2) and torch.equal(res, res2) and all(torch.equal(a[launch.loc], b[launch.loc]) for a, b in zip(launch.caches, launch.stored)), most
 
 
+def _team_sizes(ws, layers=3):
+    """What the last launch's first workgroup told the others, by layer: from the word that says that the team stays as it is on, that size."""
+    sizes = []
+    for word, _ in ws[256: 256 + 8 * layers].view(torch.int32).view(-1, 2).tolist():
+        sizes.append(word >> 1)
+        if word & 1:
+            return sizes + [word >> 1] * (layers - len(sizes))
+    raise AssertionError("a team that never stays")
+
+
+@pytest.mark.parametrize("H,hq,hkv,inter,lens", [(1024, 16, 8, 3072, [700, 90]), (1024, 16, 8, 3072, [2100, 300, 5, 17, 64, 129, 1, 40]), (1024, 24, 4, 768, [40]),
+                                                 (256, 2, 2, 512, [1300, 3, 5])])
+def test_latecomers_join(ops, dev, H, hq, hkv, inter, lens):
+    """Workgroups that come late take part from a later layer on (here: from the second or the third of three), with the bits of a team that was there at once."""
+    launch, y, res = _case(ops, dev, torch.bfloat16, H, hq, hkv, inter, lens)
+    for most, until in ((1, 1), (1, 2), (3, 1), (64, 2), (130, 1), (200, 2)):
+        for c, c0 in zip(launch.caches, launch.before):
+            c.copy_(c0)
+        y2, res2 = launch(most=most, until=until)
+        torch.cuda.synchronize()
+        sizes = _team_sizes(launch.ws)
+        assert sizes[:until] == [most] * until and sizes[-1] > 200, sizes
+        assert torch.equal(y, y2) and torch.equal(res, res2) and all(torch.equal(a[launch.loc], b[launch.loc]) for a, b in zip(launch.caches, launch.stored)), most
+    assert not ops.decode_layers_failed(launch.ws).any()
+
+
 def test_launch_numbers_start_again(ops, dev):
-    """The last number's launch clears the packets: none of an earlier launch could pass for one of a later launch with the same number."""
+    """The last number's launch clears packets and teams' sizes: none of an earlier launch could pass for one of a later launch with the same number."""
     launch, y, res = _case(ops, dev, torch.bfloat16, 1024, 16, 8, 3072, [700, 90])
-    number, packets = launch.ws[128:132].view(torch.int32), launch.ws[384:].view(torch.int64)
+    number, packets = launch.ws[128:132].view(torch.int32), launch.ws[256:].view(torch.int64)
     number.fill_(-3)
     for want in (-2, -1, 1, 2):
         y2, res2 = launch()
