@@ -126,23 +126,24 @@ struct DlWait {
   __device__ __forceinline__ void get(const __amdgpu_buffer_rsrc_t& pk, int from, uint32_t (&v)[2 * N], AT&& at) const {
     V4 q[N];
     int spins = 0;
-    bool ok;
-    do {
+    for (;;) {
       asm volatile("" ::: "memory");  // read again
 #pragma unroll
       for (int i = 0; i < N; ++i) q[i] = __builtin_bit_cast(V4, __builtin_amdgcn_raw_buffer_load_b128(pk, at(i), from, 16));  // sc1: agent scope
-      ok = true;
+      bool ok = true;
 #pragma unroll
       for (int i = 0; i < N; ++i) ok &= q[i][1] == epoch && q[i][3] == epoch;
-    } while (!ok && again(spins));
+      if (ok) break;
+      if (!again(spins)) {  // (in the loop: a step of eight requests of 2000 1230 us with the NaN behind it, 1214 so)
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = V4{kNaNs, 0, kNaNs, 0};
+        break;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       v[2 * i] = q[i][0];
       v[2 * i + 1] = q[i][2];
-    }
-    if (!ok) {
-#pragma unroll
-      for (int i = 0; i < 2 * N; ++i) v[i] = kNaNs;
     }
   }
 };
