@@ -172,12 +172,21 @@ class HipAttnBackend:
         return self._attend_small(q, k, v, layer_id, batch, q_norm_w=q_norm_w, k_norm_w=k_norm_w, eps=eps, positions=positions, cos_sin_cache=cos_sin)
 
     def takes_layers(self, batch: Any, hidden: int, intermediate: int, layers: int) -> bool:
-        """Whether all layers of the batch's decode step go in one launch (csrc/decode_layers.hip): a batch of `small_decode`, of a model whose layer fits the
-        compute units' LDS and gives every other one of them, at least, rows of every product.  Not prompts that extend by one token: what the launch's
-        workgroups meet in is one for all decode steps, which may run beside a prompt.  Nor a capture that no step of the model came before: the zeros that the
-        first launch starts from would be written when the graph is replayed, and by every replay."""
+        """Whether all layers of the batch's decode step go in one launch (csrc/decode_layers.hip): a batch of `small_decode` whose layer fits the compute units'
+        LDS, where that launch was ahead at every length.  Separate launches against it, % of a step in an engine as wide as its requests, or wider than 4096
+        tokens for longer ones (hidden size, heads on kv heads; 12 - 28 layers, bf16):
+          8 and more kv heads: 1 - 8 requests of 16 - 40000 tokens, 1024 and 768 columns, 16 on 8, 8 on 8, 10 on 10: -26 .. -1 (8 x 4000 -3 .. -1, 1 x 32000 -14 .. -2)
+          3 - 5: up to 4 requests in up to 4096 tokens -24 .. -3 (12, 16, 24 on 4, 10 on 5, 6 on 3), 6 x 1000 -5, but 8 x 533 -3 .. 0 and 8 x 1000 on 16 on 4 +4; longer
+            ones 1 x 8000 +8 .. +10, 1 x 32000 +5 .. +9
+          1, 2: up to 3 in up to 4096 -29 .. 0, but 4 x 4080 -5 .. +3, 8 x 2000 -1 .. +6, 8 x 4000 up to +12, 1 x 8000 0 .. +5
+          512 columns (half of the compute units have rows of a product): 1 x 533 -16 .. -14, but 1 x 4000 -2 .. +2, 8 requests -6 .. +15, 1 x 32000 +6 .. +9
+        A captured step does not know its lengths.  Not prompts that extend by one token: what the launch's workgroups meet in is one for all decode steps, which may
+        run beside a prompt.  Nor a capture that no step of the model came before: the zeros that the first launch starts from would be written when the graph is
+        replayed, and by every replay."""
+        few = 4 if self.kv_heads >= 3 else 3
         return (self._decode_phase(batch) and batch.positions.dtype == batch.out_loc.dtype == torch.int32
-                and hidden // 2 >= int(_lib.lib().msgl_device_cu_count()) and self.small_decode(batch)
+                and hidden >= 3 * int(_lib.lib().msgl_device_cu_count()) and self.small_decode(batch)
+                and (self.kv_heads >= 8 or batch.attn_metadata.batch <= few and int(self.ctx.page_table.shape[1]) <= 4096)
                 and ops.decode_layers_supported(batch.attn_metadata.batch, hidden, self.qo_heads, self.kv_heads, intermediate)
                 and ((layers, hidden, intermediate) in self._layers_workspaces or not torch.cuda.is_current_stream_capturing()))
 

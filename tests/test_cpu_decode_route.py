@@ -12,7 +12,7 @@ def backend(monkeypatch):
 
     b = object.__new__(attention.HipAttnBackend)
     b.qo_heads, b.kv_heads, b.head_dim, b._small_heads, b.device = 16, 8, 128, 64, torch.device("cpu")
-    b._layers_workspaces = {}
+    b._layers_workspaces, b.ctx = {}, SimpleNamespace(page_table=torch.zeros(4, 32, dtype=torch.int32))
     monkeypatch.setattr(attention._lib, "lib", lambda: SimpleNamespace(msgl_device_cu_count=lambda: 256))
     monkeypatch.setattr(attention.ops, "decode_layers_supported", lambda *a: True)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
@@ -54,6 +54,18 @@ def test_the_first_step_of_a_model_is_not_captured_as_one_launch(backend, monkey
     assert backend._layers_workspace(40, 1024, 3072).numel() == 8 * 40 * 4096 and backend._layers_workspace(28, 1024, 3072) is first
 
 
+@pytest.mark.parametrize("hidden,heads,kv_heads,width,most", [(1024, 16, 8, 4096, 8), (1024, 16, 8, 40960, 4), (768, 16, 8, 4096, 8), (512, 8, 8, 4096, 0),
+                                                              (1024, 16, 4, 4096, 4), (768, 24, 4, 4128, 0), (1024, 6, 3, 64, 4), (1024, 16, 2, 4096, 3),
+                                                              (1024, 8, 1, 4096, 3), (1024, 8, 1, 8192, 0), (512, 8, 1, 4096, 0)])
+def test_where_one_launch_is_ahead(backend, hidden, heads, kv_heads, width, most):
+    """Steps take the one launch only where it was measured ahead at every length that the engine's page table admits: up to `most` requests."""
+    from mini_sglang_amd.attention import SMALL_DECODE_HEADS
+
+    backend.qo_heads, backend.kv_heads, backend.ctx.page_table = heads, kv_heads, torch.zeros(2, width, dtype=torch.int32)
+    backend._small_heads = SMALL_DECODE_HEADS * (2 if kv_heads <= 2 or width <= 4096 else 1)
+    assert [n for n in range(1, 9) if backend.takes_layers(_batch("decode", n), hidden, 3072, 28)] == list(range(1, most + 1))
+
+
 @pytest.mark.parametrize("small", [True, False], ids=["small batch", "planned"])
 def test_one_token_prompts_have_partial_sums_of_their_own(backend, monkeypatch, small):
     """Decode steps share the backend's scratch; a one-token prompt keeps its own with its batch, the same for all its layers."""
@@ -68,7 +80,7 @@ def test_one_token_prompts_have_partial_sums_of_their_own(backend, monkeypatch, 
         monkeypatch.setattr(attention.ops, "attn_decode", lambda *a, **k: seen.append(a[8]))
     pool = torch.zeros(16, 8, 128)
     backend.scale, backend.max_bs, backend.capacity, backend.slot_run, backend.device = 1.0, 4, 64, 1, torch.device("cpu")
-    backend._cap_plan, backend.ctx = None, SimpleNamespace(page_table=torch.zeros(4, 32, dtype=torch.int32))
+    backend._cap_plan = None
     backend.kvcache = SimpleNamespace(k_cache=lambda i: pool, v_cache=lambda i: pool, store_kv=lambda *a: None, dtype=torch.float32)
     backend._workspace = torch.empty(4096, dtype=torch.uint8)
     q, k = torch.zeros(3, 16, 128), torch.zeros(3, 8, 128)
