@@ -473,7 +473,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tr_kernel(const PrefillPa
 // the rule and its other side: ops.prefill_ranges)
 // FRESH: nothing is cached, so keys and values are read from the rows as they come, without the page table, and stored to the pool from the two tiles that a
 // workgroup's query rows are the keys of, which lie in LDS at its end (by the first head of a kv head).  Prompts longer than
-// ops.FRESH_TOKENS, whose heads may go in pairs, take the store and the other launch.  us, store_kv_kernel and launch -> this, inputs in cache, 40 heads on 8: 29
+// ops.FRESH_TOKENS take the store and the other launch.  us, store_kv_kernel and launch -> this, inputs in cache, 40 heads on 8: 29
 // requests of 100 - 1024 tokens 214 -> 192 (not in cache 221 -> 208), 60 of 128 - 256 99 -> 85, 8 of 600 - 1000 91 -> 85, 6 of 1500 184 -> 176; 16 on 8: 60 of 128 -
 // 256 54.5 -> 43.9; 64 on 8 155 -> 140.  Beyond, 40 on 8: 4 of 2048 210 -> 202, one of 8192 706 -> 692.  (The pool's rows by way of the L2 212 where 206; each of a kv head's heads a
 // share of them: slower, each waits for its slots.)

@@ -7,7 +7,11 @@
 //   * WEIGHTS do not wait for rows: a workgroup's share of each of the four products has a region of LDS (123 KB at hidden size 1024), which is refilled
 //     by DMA two stages ahead, and goes to registers in front of the wait for the rows; the cache's rows of earlier tokens are there a layer ahead;
 //   * ROWS go from everyone to everyone as 8-byte packets {two 16-bit values (or one fp32), number of this launch}: written and read at agent scope
-//     (past the L2s, of which each XCD has its own), the number says by itself that the values have arrived: no fence, no flag, no counter;
+//     (past the L2s, of which each XCD has its own), the number says by itself that the values have arrived: no fence, no flag, no counter.
+//     Two packets travel in one aligned 16-byte access, which is no atomic operation of the memory model: what this rests on is that each 8-byte half of it
+//     arrives whole, as a lane's aligned 16 bytes are one piece of one request to one line on this device (whether the halves arrive together does not
+//     matter: each has its number).  As 8-byte accesses, which are atomic by the model, a step takes 8 % more (1 request of 533 tokens 676 -> 733 us, 8 of 2000
+//     1229 -> 1320);
 //   * every layer has packets of its own, so none is overwritten before all have read it; and as each stage needs rows of all workgroups, a workgroup that
 //     has them knows its own waves done with the stages before: LDS regions need no barriers of their own against being overwritten;
 //   * four waves fetch rows (and norm, rotate, stage them), four fetch weights, multiply and attend: a row's request never stands behind a weight's in
@@ -19,11 +23,15 @@
 //
 // Bound: latency.  A hop between 256 workgroups is 1.3 us by itself, there are five in a layer (six where a request's keys are cut into ranges), and 0.6 - 0.8 us of
 // dependent instructions in each; the weights' DMAs share the way with the packets and cost 4 us a layer beside them (417 of 521 us for 28 layers
-// of Qwen3-0.6B without them).  A decode step of that model, launches -> this: one request of 533 tokens 851 -> 672 us, four 997 -> 761, eight of 2000 1305 -> 1205;
-// in an engine of 40960 tokens one of 32000 1508 -> 1453, four of 16000 2242 -> 2181: it is ahead wherever msgl_attn_decode_small is taken.
-// Measured on the way (28 layers, one request of 16 tokens): a product's columns dealt out to four waves instead of its groups 545 -> 535; weights without nt
-// 535 -> 521; DMAs with 256 cycles between them 521 -> 508; sleeping between two looks at the packets +6; all of a layer's DMAs in the attention's
-// shadow +-0; without arguments read ahead, per-stage code and one barrier less 626.
+// of Qwen3-0.6B without them).  A decode step of that model, launches -> this: one request of 533 tokens 850 -> 675 us, four 882 -> 765, eight of 2000 1305 -> 1214;
+// with a vocabulary of 32768, in an engine of 40960 tokens, one of 32000 1472 -> 1424, four of 16000 2263 -> 2144 (other models: HipAttnBackend.takes_layers).
+// A team that misses workgroups has no weights ahead and several turns a product: the launch alone, one request of 533 tokens, takes 602 us with 256, 776 with
+// 255, 1028 with 128, 1757 with 64, 18800 with 4, hence the latecomers: a step begun beside a prompt's attention (8192 tokens after 16384, 64 heads on 8, 5.0 ms)
+// takes 2.0 ms (2.4 at most) where the team stayed as it began 3.2 (19.9), four requests 2.2 (2.7), 3.6 (25.9).  As launches it ends 0.8 ms behind the prompt's
+// kernel, wherever it began; that kernel takes 5.7 - 6.0 ms beside this launch, which holds the compute units' LDS, and 5.0 - 5.3 beside those.
+// Measured on the way (28 layers, one request of 16 tokens): a product's columns dealt out to four waves instead of its groups 545 -> 535; DMAs with 256
+// cycles between them 521 -> 508; sleeping between two looks at the packets +6; all of a layer's DMAs in the attention's shadow +-0; without arguments
+// read ahead, per-stage code and one barrier less 626.  Weights without nt: a step of one request of 533 tokens 676 -> 683, of four 778 -> 793, eight +-0.
 #include "attn_decode_tile.h"
 
 namespace msgl {

@@ -1660,8 +1660,11 @@ __global__ __launch_bounds__(kRowThreads, 4) void sample_team_kernel(SplitScratc
 }
 
 // Workgroups per row (1: one walks the row).  One a compute unit in all: 64 rows x 151936, top-p alone, 54 us with 4 each, 58 with 8; 33 rows 51 and 54.
-// Where sharing pays, us a draw, shared / one workgroup, bf16 (top-k: in three launches; sample_team_kernel is ahead of them wherever it can be taken):
-//   top-k      1 x 151936 20.5 / 25.2, 33 x 151936 29.4 / 31.4, 64 x 151936 29.1 / 34.2, but 8 x 65536 20.4 / 17.5, 100 x 151936 41 / 38
+// Where sharing pays, us a draw, shared / one workgroup, bf16:
+//   top-k      in three launches (callers without a team's memory), whose line this is: 1 x 151936 20.5 / 25.2, 33 x 151936 29.4 / 31.4, 64 x 151936 29.1 / 34.2,
+//              but 8 x 65536 20.4 / 17.5, 100 x 151936 41 / 38.  sample_team_kernel is ahead of these three wherever it can be taken, and of one workgroup already
+//              below the line (with top-p, in a graph): 1, 8, 64 x 80000 15.7 / 19.6, 16.3 / 20.4, 20.2 / 24.4, x 65536 15.0 / 16.5, 15.4 / 17.1, 18.7 / 19.8, but x 50304
+//              14.8 / 15.3, 15.3 / 15.9, 18.3 / 17.7, x 32000 14.1 / 14.3, 14.9 / 14.9, 16.5 / 15.8, x 16384 14.4 / 10.6, 14.9 / 11.6, 16.0 / 12.0
 //   no filter  64 x 65536 16.5 / 17.7, 128 x 98304 24.4 / 25.9, 100 x 151936 29 / 37, but 128 x 65536 20.4 / 18.7, 128 x 50000 18.2 / 15.3,
 //              32 x 50000 14.8 / 14.8, 256 x 151936 48 / 44
 //   top-p      wide nuclei (logits of deviation 2.5) and, behind them, nuclei of a few tokens in every row (deviation 10), which one workgroup

@@ -567,9 +567,10 @@ def attn_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_ca
     )
 
 
-# Longest prompt of a batch with nothing cached whose store and attention go in one launch: chains short enough that heads do not go in pairs (prefill_pairs: 15
-# tiles on average).  What it saves, % of both launches, heads on kv heads: up to here 60 requests of 128 - 256 tokens 17 (40 on 8), 24 (16 on 8), 11 (64 on 8); 8 of 600 -
-# 1000 7, 20, 3; 6 of 1500 4, 13, 2.  Beyond, where the store is a small share: 4 of 2048 5, 10, 2, one of 8192 2, 4, 1.
+# Longest prompt of a batch with nothing cached whose store and attention go in one launch (where heads do not go in pairs and keys not in ranges).  What it
+# saves, % of both launches, heads on kv heads: up to here 60 requests of 128 - 256 tokens 17 (40 on 8), 24 (16 on 8), 11 (64 on 8); 8 of 600 - 1000 7, 20, 3; 6 of 1500 6, 15, 2.
+# Beyond, the store is a smaller share and the launch ahead by less: 6 of 1900 - 2000 5, 10, 1; 3 of 4000 2, 6, 1; one of 8192 1 (40 on 8), 3 (10 on 2), of 12000 1, 3 (16 on 8).
+# A pass alone: 29 of 100 - 1024 tokens, 40 on 8, 239 -> 231 us, 8 of 600 - 1000 125 -> 117, 60 of 128 - 256, 16 on 8, 85 -> 83.
 FRESH_TOKENS = 1536
 
 
