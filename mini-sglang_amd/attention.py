@@ -291,7 +291,7 @@ class HipAttnBackend:
                 from .kernel import poll_communicator_errors
 
                 poll_communicator_errors(sync=False)
-        if self._layers_workspaces and self._md_calls % 64 == 0:  # captured one-launch steps likewise
+        if self._layers_workspaces and self._md_calls % 64 == 0 and not torch.cuda.is_current_stream_capturing():  # captured one-launch steps likewise
             self.poll_errors()
         reqs = batch.padded_reqs
         bs = len(reqs)

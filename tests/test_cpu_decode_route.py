@@ -54,6 +54,20 @@ def test_the_first_step_of_a_model_is_not_captured_as_one_launch(backend, monkey
     assert backend._layers_workspace(40, 1024, 3072).numel() == 8 * 40 * 4096 and backend._layers_workspace(28, 1024, 3072) is first
 
 
+def test_the_error_word_is_not_asked_for_inside_a_capture(backend, monkeypatch):
+    """Every 64th batch's metadata asks for the one-launch steps' error word: a copy and an event, which have no place in somebody's graph."""
+    polls, capturing = [], [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(type(backend), "poll_errors", lambda self: polls.append(1))
+    backend.tp_size, backend._md_calls, backend._layers_workspaces = 1, 0, {(28, 1024, 3072): torch.zeros(1)}
+    batch = SimpleNamespace(padded_reqs=None)  # (what follows is not looked at)
+    for i in range(4 * 64):
+        capturing[0] = i >= 2 * 64
+        with pytest.raises(TypeError):
+            backend.prepare_metadata(batch)
+    assert len(polls) == 2
+
+
 @pytest.mark.parametrize("hidden,heads,kv_heads,width,most", [(1024, 16, 8, 4096, 8), (1024, 16, 8, 40960, 4), (768, 16, 8, 4096, 8), (512, 8, 8, 4096, 0),
                                                               (1024, 16, 4, 4096, 4), (768, 24, 4, 4128, 0), (1024, 6, 3, 64, 4), (1024, 16, 2, 4096, 3),
                                                               (1024, 8, 1, 4096, 3), (1024, 8, 1, 8192, 0), (512, 8, 1, 4096, 0)])
